@@ -27,6 +27,8 @@
 //                  MFMAs of the matrix phase (the vector phase was the longer of the two).
 #include "mhip_common.hpp"
 
+#include <math.h>
+
 namespace mhip {
 namespace {
 
@@ -36,7 +38,8 @@ constexpr int kBM = kWaves * 32;   // Q rows per workgroup
 constexpr int kBN = 64;            // keys per main-loop tile
 constexpr int kTileBytes = kBN * kD * 2;   // 16384: one K or V tile in LDS, 64 rows of 256 bytes
 constexpr int kStages = 4;                 // K(t+1) .. K(t+4) and V(t) .. V(t+3) live while tile t is processed
-constexpr int kVBase = kStages * kTileBytes;
+constexpr int kVBase = kStages * kTileBytes;   // K rings of all key groups first, then the V rings
+constexpr int kNoTile = 0x7fff0000;    // scalar offset that puts every lane of a copy out of range
 constexpr int kOStride = kD + 8;   // epilogue staging of O, bf16 elements per row
 constexpr int kNoColumn = 0x7fff0000;  // vector offset that is out of every descriptor's range (spans stay below 2^31,
                                        // and so does the scalar tile offset added to it: no 32-bit wrap)
@@ -59,13 +62,30 @@ struct FwdParams {
 
 // KK = k-steps of 16 head-dim values in S^T: 8 computes on all 128 on-chip columns; 4 is the instantiation for head
 // dimensions up to 64, which leaves out the MFMAs that would only see the zero columns (half of both products).
-template <bool CAUSAL, int KK = 8>
+//
+// KS = key groups of a workgroup.  With one group the eight wavefronts hold 8 x 32 Q rows and all visit every key
+// tile.  A launch of few (batch, head, 256-row) items leaves most CUs without a workgroup then, and its time is the
+// length of one workgroup's serial chain of tiles.  With KS = 2 (4) the workgroup holds 128 (64) rows instead; wavefront
+// w works for row group w % (8 / KS) and key group w / (8 / KS), whose tiles are every KS-th one, and the groups' partial
+// (O, sum) of a row meet in LDS at the end.  Twice (four times) as many workgroups, each with half (a quarter) of the
+// serial chain; the price is as many times the L2 -> LDS traffic per row.  A key group has rings of two stages instead
+// of four, of 64-key tiles (KS = 2) or 32-key tiles (KS = 4): 128 KB of LDS in all three cases.
+template <bool CAUSAL, int KK = 8, int KS = 1>
 __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdParams p) {
   static_assert(KK == 8 || KK == 4, "128 or 64 on-chip head-dim columns");
+  static_assert(KS == 1 || KS == 2 || KS == 4, "key groups");
   constexpr int DB = KK / 2;        // blocks of 32 head-dim values in O^T
-  constexpr int kSlotsS = 2 * KK;   // matrix-phase slots of S^T (two 32-key blocks per k-step)
-  constexpr int kSlotsO = 4 * DB;   // and of O^T (four k-steps of 16 keys per block)
-  __shared__ __attribute__((aligned(16))) unsigned char smem[2 * kStages * kTileBytes];
+  constexpr int RG = kWaves / KS;   // row groups of 32
+  constexpr int kRows = 32 * RG;    // Q rows of the workgroup
+  constexpr int BN = KS == 4 ? 32 : kBN;             // keys per tile
+  constexpr int MB = BN / 32;                        // 32-key blocks per tile
+  constexpr int kTile = BN * kD * 2;                 // bytes of a tile
+  constexpr int kGroupStages = KS == 1 ? kStages : 2;
+  constexpr int kSlotsS = MB * KK;      // matrix-phase slots of S^T
+  constexpr int kSlotsO = 2 * MB * DB;  // and of O^T (k-steps of 16 keys)
+  static_assert(KS * kGroupStages * kTile == kStages * kTileBytes, "the K rings take 64 KB, and so do the V rings");
+  constexpr int kQBase = 2 * kStages * kTileBytes;   // KS > 1: Q rows, later the O rows on their way out
+  __shared__ __attribute__((aligned(16))) unsigned char smem[2 * kStages * kTileBytes + (KS > 1 ? kRows * kD * 2 : 0)];
 
   // Workgroup i runs on XCD i % 8.  Give every XCD a contiguous range of the (batch, head, q-tile)
   // order so that the workgroups sharing one K/V head also share one L2.
@@ -91,7 +111,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
   const int hq = bh % p.Hq;
   const int b = bh / p.Hq;
   const int hk = hq / p.group;
-  const int q0 = qt * kBM;
+  const int q0 = qt * kRows;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // scalar: role branches stay uniform
@@ -99,18 +119,20 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
   const int ln = lane & 31;
   const int hf = lane >> 5;
   const bool group_b = wave >= 4;                 // second ping-pong group
+  const int kg = KS == 1 ? 0 : wave / RG;         // key group
+  const int rg = KS == 1 ? wave : wave % RG;      // row group
 
   // ---- number of key tiles this Q tile has to visit -------------------------------------------
   int kv_end = p.Sc;
   if (CAUSAL) {
-    const int lim = q0 + kBM + (p.Sc - p.Sq);     // one past the last key visible to the last row
+    const int lim = q0 + kRows + (p.Sc - p.Sq);   // one past the last key visible to the last row
     kv_end = lim < kv_end ? lim : kv_end;
     if (kv_end < 0) kv_end = 0;
   }
-  const int ntiles = (kv_end + kBN - 1) / kBN;
+  const int ntiles = (kv_end + BN * KS - 1) / (BN * KS);   // of each key group; tiles past the end are hidden whole
 
   // ---- Q fragment: B operand of S^T = K Q^T, lane (ln, hf) holds Q[row][16 ks + 8 hf .. +7] -----
-  const int my_q = q0 + wave * 32 + ln;
+  const int my_q = q0 + rg * 32 + ln;
   bf16x8 qf[KK];  // loaded in the prologue, after the first tile copies are under way
 
   // ---- global -> LDS copies of the K and V tiles ---------------------------------------------------
@@ -125,38 +147,51 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
   auto swz = [](int row) { return lds_row_swizzle(row); };
   const u32x4 krs = rsrc_words(p.k + b * p.k_sb + hk * p.k_sh, (uint32_t)(((int64_t)(p.Sc - 1) * p.k_ss + p.D) * 2));
   const u32x4 vrs = rsrc_words(p.v + b * p.v_sb + hk * p.v_sh, (uint32_t)(((int64_t)(p.Sc - 1) * p.v_ss + p.D) * 2));
-  int kvoff[2], vvoff[2];
+  constexpr int kCpy = BN / RG / 4;                  // copy instructions per wavefront, tile and tensor (4 rows each)
+  int kvoff[kCpy], vvoff[kCpy];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int row = 8 * wave + 4 * u + (lane >> 4);
+  for (int u = 0; u < kCpy; ++u) {
+    const int row = 4 * kCpy * rg + 4 * u + (lane >> 4);
     const int chunk = (lane & 15) ^ swz(row);
     const bool real = chunk * 8 < p.D;
     kvoff[u] = real ? (int)(row * p.k_ss * 2) + chunk * 16 : kNoColumn;
     vvoff[u] = real ? (int)(row * p.v_ss * 2) + chunk * 16 : kNoColumn;
   }
-  const int k_tile_bytes = (int)(kBN * p.k_ss * 2);
-  const int v_tile_bytes = (int)(kBN * p.v_ss * 2);
-  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem + wave * 2048;
+  const int k_tile_bytes = (int)(BN * p.k_ss * 2);
+  const int v_tile_bytes = (int)(BN * p.v_ss * 2);
+  const uint32_t lds_smem = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+  const uint32_t lds_ring = lds_smem + kg * (kGroupStages * kTile);  // this key group's K ring; its V ring is kVBase on
+  const uint32_t lds_base = lds_ring + rg * (kCpy * 1024);
+  // tile t of this wavefront's key group; with several groups a tile past the last key is put out of range as a whole
+  auto tile_offset = [&](int t, int tile_bytes) {
+    if (KS == 1) return t * tile_bytes;
+    const int tile = t * KS + kg;
+    return tile * BN < p.Sc ? tile * tile_bytes : kNoTile;
+  };
   auto copy_k = [&](int t, int stage) {
+    const int soff = tile_offset(t, k_tile_bytes);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) copy16_to_lds(krs, lds_base + stage * kTileBytes + u * 1024, kvoff[u], t * k_tile_bytes);
+    for (int u = 0; u < kCpy; ++u) copy16_to_lds(krs, lds_base + stage * kTile + u * 1024, kvoff[u], soff);
   };
   auto copy_v = [&](int t, int stage) {
+    const int soff = tile_offset(t, v_tile_bytes);
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
-      copy16_to_lds(vrs, lds_base + kVBase + stage * kTileBytes + u * 1024, vvoff[u], t * v_tile_bytes);
+    for (int u = 0; u < kCpy; ++u)
+      copy16_to_lds(vrs, lds_base + kVBase + stage * kTile + u * 1024, vvoff[u], soff);
   };
 
   // K operand of S^T (A, 32 keys x 16 head-dim values): lane (ln, hf) reads chunk 2 kk + hf of row
   // 32 mb + ln.
-  int k_rd[KK];                                       // + mb * 8192
+  // k_a and v_a hold the LDS addresses inside the stage that is read next and move on in place, each at a point of the
+  // slot sequence where no read of its kind is due; everything else about an address is an immediate offset.
+  int k_a[KK];                                        // + mb * 8192
 #pragma unroll
-  for (int kk = 0; kk < KK; ++kk) k_rd[kk] = ln * 256 + (((2 * kk + hf) ^ swz(ln)) << 4);
+  for (int kk = 0; kk < KK; ++kk) k_a[kk] = (int)lds_ring + ln * 256 + (((2 * kk + hf) ^ swz(ln)) << 4);
   // V^T operand of O^T (A, 32 head-dim values x 16 keys) for head-dim block db and k-step (mb, j2): the
   // lane's 8 keys are rows R + {0..3} and R + 8 + {0..3}, R = 32 mb + 16 j2 + 4 hf -- the keys its P
   // registers hold.  One ds_read_b64_tr_b16 per group of 4 rows: within 16 lanes, lane s supplies the
   // address of row R + s/4, head-dim values 4 (s%4) .. +3 of the 16-column strip, and receives column s.
-  int v_rd[DB][2];                                    // [db][second four rows]  + mb * 8192 + j2 * 4096
+  int v_a[DB][2];                                     // [db][second four rows]  + mb * 8192 + j2 * 4096
   {
     const int s16 = lane & 15, strip = (lane >> 4) & 1;
     const int cl = 2 * strip + ((s16 & 3) >> 1);
@@ -165,19 +200,20 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int row = 8 * h + 4 * hf + (s16 >> 2);
-        v_rd[db][h] = row * 256 + (((4 * db + cl) ^ swz(row)) << 4) + (s16 & 1) * 8;
+        v_a[db][h] = (int)lds_ring + kVBase + row * 256 + (((4 * db + cl) ^ swz(row)) << 4) + (s16 & 1) * 8;
       }
   }
   typedef __attribute__((address_space(3))) bf16x4* lds_bf16x4;
-  auto read_k = [&](const unsigned char* ks, int mb, int kk) -> bf16x8 {
-    return *reinterpret_cast<const bf16x8*>(ks + k_rd[kk] + mb * 8192);
-  };
-  auto read_v = [&](const unsigned char* vs, int db, int kstep) -> bf16x8 {
-    const unsigned char* base = vs + (kstep >> 1) * 8192 + (kstep & 1) * 4096;
-    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(base + v_rd[db][0]));
-    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(base + v_rd[db][1]));
+  typedef __attribute__((address_space(3))) const bf16x8* lds_bf16x8;
+  auto read_k = [&](int mb, int kk) -> bf16x8 { return *(lds_bf16x8)(uintptr_t)(uint32_t)(k_a[kk] + mb * 8192); };
+  auto read_v = [&](int db, int kstep) -> bf16x8 {
+    const int off = (kstep >> 1) * 8192 + (kstep & 1) * 4096;
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(v_a[db][0] + off));
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(v_a[db][1] + off));
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
+  // byte distance from the stage of tile t to the stage of tile t + 1
+  auto stage_step = [](int t) { return (t + 1) % kGroupStages == 0 ? -(kGroupStages - 1) * kTile : kTile; };
   const int causal_shift = p.Sc - p.Sq;
 
   // ---- accumulators -----------------------------------------------------------------------------
@@ -195,28 +231,27 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
   constexpr float kTrigger = 1048576.f;   // a lane's 32 exponentials of one tile sum to less than this, or
   constexpr float kSlack = 14.f;          // rows whose maximum exceeds the reference by 2^kSlack move it
   const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  f32x16 s[2];               // S^T tile: 64 keys x 32 q rows per wave
-  u32x4 pw[4];               // P^T of the current tile as packed bf16 B operands, one per k-step
+  f32x16 s[MB];              // S^T tile: BN keys x 32 q rows per wave
+  u32x4 pw[2 * MB];          // P^T of the current tile as packed bf16 B operands, one per k-step
 
-  auto qk = [&](int stage) {
-    const unsigned char* ks = smem + stage * kTileBytes;
+  auto qk = [&]() {                   // S^T(0); leaves k_a at K(1)
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb) {
-        const bf16x8 kf = read_k(ks, mb, kk);
+      for (int mb = 0; mb < MB; ++mb) {
+        const bf16x8 kf = read_k(mb, kk);
         s[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[kk], kk == 0 ? zero : s[mb], 0, 0, 0);
       }
+      k_a[kk] += kTile;
     }
   };
 
-  auto pv = [&](int stage) {
-    const unsigned char* vs = smem + kVBase + stage * kTileBytes;
+  auto pv = [&]() {
 #pragma unroll
-    for (int kstep = 0; kstep < 4; ++kstep) {
+    for (int kstep = 0; kstep < 2 * MB; ++kstep) {
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
-        const bf16x8 vf = read_v(vs, db, kstep);
+        const bf16x8 vf = read_v(db, kstep);
         o_acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, __builtin_bit_cast(bf16x8, pw[kstep]), o_acc[db], 0, 0, 0);
       }
     }
@@ -224,14 +259,14 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
 
   // keys past the chunk end and the causal diagonal -> -inf
   auto sm_mask = [&](int t) {
-    const int kv0 = t * kBN;
-    bool need_mask = kv0 + kBN > p.Sc;
-    if (CAUSAL) need_mask = need_mask || (kv0 + kBN - 1 > q0 + causal_shift);
+    const int kv0 = (t * KS + kg) * BN;
+    bool need_mask = kv0 + BN > p.Sc;
+    if (CAUSAL) need_mask = need_mask || (kv0 + BN - 1 > q0 + causal_shift);
     if (need_mask) {
       int lim = p.Sc - 1;                                   // last visible key of this lane's row
       if (CAUSAL) { const int c = my_q + causal_shift; lim = c < lim ? c : lim; }
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
+      for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
           const int key = kv0 + mb * 32 + (j >> 2) * 8 + hf * 4 + (j & 3);
@@ -258,14 +293,14 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
   };
   auto sm_exps = [&]() {
 #pragma unroll
-    for (int idx = 0; idx < 16; ++idx) sm_pair(idx);
+    for (int idx = 0; idx < 8 * MB; ++idx) sm_pair(idx);
   };
   // Move the reference of the rows whose scores outgrew it (first tile: set it to the row maximum) and
   // rescale O and the running sum accordingly.
   auto sm_fix = [&](bool first) {
     float mx = s[0][0];
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[mb][j]);
     mx = pair_max(mx);
@@ -284,14 +319,13 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
   };
   // slot of the matrix phase after which early pair idx runs: k-step idx / 4 of the tile before is read by the
   // O^T slots kSlotsS + DB (idx / 4) .. + DB - 1, and the pairs are spread two slots apart behind that
-  auto early_slot = [](int idx) {
-    return idx < 4 ? kSlotsS + DB + kEarlyStep * idx : kSlotsS + 3 * DB + (idx - 4);
-  };
-  static_assert(kEarlyPairs <= 4 && kSlotsS + DB + kEarlyStep * (kEarlyPairs - 1) < kSlotsS + kSlotsO,
+  constexpr int kEarlyGap = MB * DB >= 4 ? kEarlyStep : 1;
+  auto early_slot = [](int idx) { return kSlotsS + DB + kEarlyGap * idx; };
+  static_assert(kEarlyPairs <= 4 && DB + kEarlyGap * (kEarlyPairs - 1) < kSlotsO,
                 "the early pairs have to fit behind the O^T slots of k-step 0");
   auto sm_tile = [&]() {
 #pragma unroll
-    for (int idx = kEarlyPairs; idx < 16; ++idx) sm_pair(idx);
+    for (int idx = kEarlyPairs; idx < 8 * MB; ++idx) sm_pair(idx);
     if (__builtin_amdgcn_ballot_w64(!(rs < kTrigger)) != 0) {
       sm_fix(false);
       sm_exps();
@@ -299,36 +333,44 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
     l_run += rs;
   };
 
-  // Matrix phase of tile t: S^T(t+1) from K stage `ks_stage` and O^T += V^T(t) P^T(t) from V stage
-  // `vs_stage`, kSlotsS + kSlotsO MFMAs (32 on 128 columns) fed by as many LDS reads.  The reads run kFragDepth
-  // operands ahead of the MFMAs through a ring of registers, so the LDS latency is covered by the MFMAs in between.
-  auto read_frag = [&](int i, const unsigned char* ks, const unsigned char* vs) -> bf16x8 {
-    if (i < kSlotsS) return read_k(ks, i & 1, i >> 1);
-    return read_v(vs, (i - kSlotsS) % DB, (i - kSlotsS) / DB);
+  // Matrix phase of tile t: S^T(t+1) and O^T += V^T(t) P^T(t), kSlotsS + kSlotsO MFMAs (32 on 128 columns and
+  // 64 keys) fed by as many LDS reads.  The reads run kFragDepth operands ahead of the MFMAs through a ring of registers, so the LDS latency is covered by the MFMAs in between.
+  auto read_frag = [&](int i) -> bf16x8 {
+    if (i < kSlotsS) return read_k(i % MB, i / MB);
+    return read_v((i - kSlotsS) % DB, (i - kSlotsS) / DB);
   };
   // The first kFragDepth operands (all of K) are read before the barrier that opens the phase, by
   // first_frags, so the matrix pipe starts without waiting for LDS.
   bf16x8 frag[kFragDepth];
-  auto first_frags = [&](int ks_stage) {
-    const unsigned char* ks = smem + ks_stage * kTileBytes;
+  auto first_frags = [&]() {
 #pragma unroll
-    for (int i = 0; i < kFragDepth; ++i) frag[i] = read_frag(i, ks, ks);
+    for (int i = 0; i < kFragDepth; ++i) frag[i] = read_frag(i);
   };
-  auto matrix_phase = [&](int t_next, int ks_stage, int vs_stage) {
-    const unsigned char* ks = smem + ks_stage * kTileBytes;
-    const unsigned char* vs = smem + kVBase + vs_stage * kTileBytes;
+  static_assert(kSlotsO >= KK / 2 && kFragDepth * 2 >= 2 * DB, "slots in which the operand addresses move on");
+  auto matrix_phase = [&](int t) {
+    const int k_step = stage_step(t + 1), v_step = stage_step(t);
 #pragma unroll
     for (int i = 0; i < kSlotsS + kSlotsO; ++i) {
       if (i < kSlotsS) {
-        const int mb = i & 1, kk = i >> 1;
+        const int mb = i % MB, kk = i / MB;
         s[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag[i % kFragDepth], qf[kk], kk == 0 ? zero : s[mb], 0, 0, 0);
       } else {
         const int db = (i - kSlotsS) % DB, kstep = (i - kSlotsS) / DB;
         o_acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag[i % kFragDepth], __builtin_bit_cast(bf16x8, pw[kstep]), o_acc[db], 0, 0, 0);
       }
-      if (i + kFragDepth < kSlotsS + kSlotsO) frag[i % kFragDepth] = read_frag(i + kFragDepth, ks, vs);
-      // S^T(t_next) is complete after its last slot; its softmax starts here, in the shadow of the O^T MFMAs
-      if (i == kSlotsS) sm_mask(t_next);
+      if (i + kFragDepth < kSlotsS + kSlotsO) frag[i % kFragDepth] = read_frag(i + kFragDepth);
+      // the last K read went out in slot kSlotsS - kFragDepth - 1, the last V read kFragDepth slots before the end
+      if (i >= kSlotsS && i < kSlotsS + KK / 2) {
+        k_a[2 * (i - kSlotsS)] += k_step;
+        k_a[2 * (i - kSlotsS) + 1] += k_step;
+      }
+      if (i >= kSlotsS + kSlotsO - DB) {
+        const int db = i - (kSlotsS + kSlotsO - DB);
+        v_a[db][0] += v_step;
+        v_a[db][1] += v_step;
+      }
+      // S^T(t+1) is complete after its last slot; its softmax starts here, in the shadow of the O^T MFMAs
+      if (i == kSlotsS) sm_mask(t + 1);
 #pragma unroll
       for (int idx = 0; idx < kEarlyPairs; ++idx)
         if (early_slot(idx) == i) sm_pair(idx);
@@ -336,96 +378,295 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
     }
   };
 
-  // ---- prologue: the first tiles into LDS, softmax of tile 0 -------------------------------------------
-  // Barriers inside the loop are bare s_barrier instructions: a fence would wait for every copy in flight.
-  if (ntiles > 0) {
+  if constexpr (KS == 1) {
+    // ---- prologue: the first tiles into LDS, softmax of tile 0 -------------------------------------------
+    // Barriers inside the loop are bare s_barrier instructions: a fence would wait for every copy in flight.
+    if (ntiles > 0) {
 #pragma unroll
-    for (int i = 0; i < kStages; ++i) copy_k(i, i);          // tiles past the chunk arrive as zeros
+      for (int i = 0; i < kStages; ++i) copy_k(i, i);          // tiles past the chunk arrive as zeros
 #pragma unroll
-    for (int i = 0; i < kStages - 1; ++i) copy_v(i, i);
-  }
-  {
-    // The Q loads go out behind the copies, so that one wait covers both latencies.  The fragment is
-    // pinned here: otherwise its first use sits inside the main loop and so does the wait for it.
-    const int row = my_q < p.Sq ? my_q : p.Sq - 1;
-    const uint16_t* qp = p.q + b * p.q_sb + (int64_t)row * p.q_ss + hq * p.q_sh + hf * 8;
-#pragma unroll
-    for (int ks = 0; ks < KK; ++ks) {
-      if (ks * 16 + hf * 8 < p.D) qf[ks] = *reinterpret_cast<const bf16x8*>(qp + ks * 16);
-      else qf[ks] = bf16x8{};                       // columns past the head dimension
+      for (int i = 0; i < kStages - 1; ++i) copy_v(i, i);
     }
+    {
+      // The Q loads go out behind the copies, so that one wait covers both latencies.  The fragment is
+      // pinned here: otherwise its first use sits inside the main loop and so does the wait for it.
+      const int row = my_q < p.Sq ? my_q : p.Sq - 1;
+      const uint16_t* qp = p.q + b * p.q_sb + (int64_t)row * p.q_ss + hq * p.q_sh + hf * 8;
 #pragma unroll
-    for (int ks = 0; ks < KK; ++ks) asm volatile("" : "+v"(qf[ks]));
-  }
-  if (ntiles > 0) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      for (int ks = 0; ks < KK; ++ks) {
+        if (ks * 16 + hf * 8 < p.D) qf[ks] = *reinterpret_cast<const bf16x8*>(qp + ks * 16);
+        else qf[ks] = bf16x8{};                       // columns past the head dimension
+      }
+#pragma unroll
+      for (int ks = 0; ks < KK; ++ks) asm volatile("" : "+v"(qf[ks]));
+    }
+    if (ntiles > 0) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      qk();
+      sm_mask(0);
+      sm_fix(true);
+      sm_exps();
+      l_run = rs;
+      if (ntiles > 1) first_frags();
+    }
+    // Phase p of the main loop: group A (waves 0-3) runs the matrix phase of tile p/2 on even p and its
+    // vector phase on odd p; group B does the same one phase later.  K(t) and V(t) live in stage t % 4 of
+    // their rings.  In the vector phase of tile t every wavefront starts its share of the copies of K(t+4)
+    // (over K(t), last read in the matrix phase of tile t-1) and V(t+3) (over V(t-1)), and before the
+    // barrier that ends the phase waits for the copies it started one tile earlier: those are then visible
+    // to every wavefront two barriers later, in time for first_frags of K(t+3) and the matrix phase of V(t+2).
+    if (group_b) __builtin_amdgcn_s_barrier();
+    for (int t = 0; t + 1 < ntiles; ++t) {
+      // ---- matrix phase: S^T(t+1) = K(t+1) Q^T and O^T += V^T(t) P^T(t), first part of softmax(t+1) ------
+      __builtin_amdgcn_s_setprio(2);
+      matrix_phase(t);
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_s_barrier();
+      // ---- vector phase: softmax(t+1), copies of the tiles ahead ---------------------------------------------
+      asm volatile("" : "+v"(s[0]), "+v"(s[MB - 1]));   // keeps the exponentials behind the barrier
+      sm_tile();
+      copy_k(t + 4, t & 3);
+      copy_v(t + 3, (t + 3) & 3);
+      if (t + 2 < ntiles) first_frags();                        // K(t+2), for the next matrix phase
+      asm volatile("s_waitcnt vmcnt(4)" ::: "memory");          // the four copies of one tile ago are done
+      __builtin_amdgcn_s_barrier();
+    }
+    if (ntiles > 0) pv();                             // last tile: nothing left to prefetch or exponentiate
+    if (!group_b) __builtin_amdgcn_s_barrier();
+
+    // ---- epilogue -----------------------------------------------------------------------------------
+    const float l_tot = pair_sum(l_run);
+    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    if (hf == 0 && my_q < p.Sq) {
+      const float lse = l_tot > 0.f ? m_ref * p.scale + fast_log2(l_tot) * kLn2 : -INFINITY;
+      p.lse[((int64_t)b * p.Hq + hq) * p.Sq + my_q] = lse;
+    }
+
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // zero-filled copies of tiles past the end included
+    __syncthreads();   // every wave is done with the K/V tiles: reuse LDS to transpose O
+    unsigned char* os = smem + wave * (32 * kOStride * 2);
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        u32x2 w;
+        w[0] = pack_bf16(o_acc[db][4 * g] * inv, o_acc[db][4 * g + 1] * inv);
+        w[1] = pack_bf16(o_acc[db][4 * g + 2] * inv, o_acc[db][4 * g + 3] * inv);
+        *reinterpret_cast<u32x2*>(os + ln * (kOStride * 2) + (db * 32 + g * 8 + hf * 4) * 2) = w;
+      }
     __syncthreads();
-    qk(0);
-    sm_mask(0);
-    sm_fix(true);
-    sm_exps();
-    l_run = rs;
-    if (ntiles > 1) first_frags(1);
-  }
-  // Phase p of the main loop: group A (waves 0-3) runs the matrix phase of tile p/2 on even p and its
-  // vector phase on odd p; group B does the same one phase later.  K(t) and V(t) live in stage t % 4 of
-  // their rings.  In the vector phase of tile t every wavefront starts its share of the copies of K(t+4)
-  // (over K(t), last read in the matrix phase of tile t-1) and V(t+3) (over V(t-1)), and before the
-  // barrier that ends the phase waits for the copies it started one tile earlier: those are then visible
-  // to every wavefront two barriers later, in time for first_frags of K(t+3) and the matrix phase of V(t+2).
-  if (group_b) __builtin_amdgcn_s_barrier();
-  for (int t = 0; t + 1 < ntiles; ++t) {
-    // ---- matrix phase: S^T(t+1) = K(t+1) Q^T and O^T += V^T(t) P^T(t), first part of softmax(t+1) ------
-    __builtin_amdgcn_s_setprio(2);
-    matrix_phase(t + 1, (t + 1) & 3, t & 3);
-    __builtin_amdgcn_s_setprio(0);
-    __builtin_amdgcn_s_barrier();
-    // ---- vector phase: softmax(t+1), copies of the tiles ahead ---------------------------------------------
-    asm volatile("" : "+v"(s[0]), "+v"(s[1]));      // keeps the exponentials behind the barrier
-    sm_tile();
-    copy_k(t + 4, t & 3);
-    copy_v(t + 3, (t + 3) & 3);
-    if (t + 2 < ntiles) first_frags((t + 2) & 3);             // K(t+2), for the next matrix phase
-    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");          // the four copies of one tile ago are done
-    __builtin_amdgcn_s_barrier();
-  }
-  if (ntiles > 0) pv((ntiles - 1) & 3);             // last tile: nothing left to prefetch or exponentiate
-  if (!group_b) __builtin_amdgcn_s_barrier();
-
-  // ---- epilogue -----------------------------------------------------------------------------------
-  const float l_tot = pair_sum(l_run);
-  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  if (hf == 0 && my_q < p.Sq) {
-    const float lse = l_tot > 0.f ? m_ref * p.scale + fast_log2(l_tot) * kLn2 : -INFINITY;
-    p.lse[((int64_t)b * p.Hq + hq) * p.Sq + my_q] = lse;
-  }
-
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // zero-filled copies of tiles past the end included
-  __syncthreads();   // every wave is done with the K/V tiles: reuse LDS to transpose O
-  unsigned char* os = smem + wave * (32 * kOStride * 2);
+    {
+      const int chunk = lane & 15;
+      uint16_t* op = p.out + b * p.o_sb + hq * p.o_sh + chunk * 8;
 #pragma unroll
-  for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      u32x2 w;
-      w[0] = pack_bf16(o_acc[db][4 * g] * inv, o_acc[db][4 * g + 1] * inv);
-      w[1] = pack_bf16(o_acc[db][4 * g + 2] * inv, o_acc[db][4 * g + 3] * inv);
-      *reinterpret_cast<u32x2*>(os + ln * (kOStride * 2) + (db * 32 + g * 8 + hf * 4) * 2) = w;
+      for (int it = 0; it < 8; ++it) {
+        const int r = (lane >> 4) + 4 * it;
+        const int row = q0 + wave * 32 + r;
+        if (row < p.Sq && chunk * 8 < p.D) {
+          const u32x4 w = *reinterpret_cast<const u32x4*>(os + r * (kOStride * 2) + chunk * 16);
+          *reinterpret_cast<u32x4*>(op + (int64_t)row * p.o_ss) = w;
+        }
+      }
     }
-  __syncthreads();
-  {
-    const int chunk = lane & 15;
-    uint16_t* op = p.out + b * p.o_sb + hq * p.o_sh + chunk * 8;
+  } else {
+    // ---- several key groups -----------------------------------------------------------------------------------
+    // Q comes through LDS here (every row is needed by KS wavefronts, and the copies can be waited for one by one):
+    // the first S^T starts when the first K tile and Q are there, not when everything requested before has arrived.
+    if (ntiles > 0) {
+      constexpr int kQCpy = kRows / kWaves / 4;
+      const int q_rows = p.Sq - q0 < kRows ? p.Sq - q0 : kRows;
+      const u32x4 qrs = rsrc_words(p.q + b * p.q_sb + (int64_t)q0 * p.q_ss + hq * p.q_sh,
+                                   (uint32_t)(((q_rows - 1) * p.q_ss + p.D) * 2));
+      const uint32_t q_lds = lds_smem + kQBase + wave * (kQCpy * 1024);
+      copy_k(0, 0);
 #pragma unroll
-    for (int it = 0; it < 8; ++it) {
-      const int r = (lane >> 4) + 4 * it;
-      const int row = q0 + wave * 32 + r;
-      if (row < p.Sq && chunk * 8 < p.D) {
-        const u32x4 w = *reinterpret_cast<const u32x4*>(os + r * (kOStride * 2) + chunk * 16);
-        *reinterpret_cast<u32x4*>(op + (int64_t)row * p.o_ss) = w;
+      for (int u = 0; u < kQCpy; ++u) {
+        const int row = 4 * kQCpy * wave + 4 * u + (lane >> 4);
+        const int chunk = (lane & 15) ^ swz(row);
+        copy16_to_lds(qrs, q_lds + u * 1024, chunk * 8 < p.D ? (int)(row * p.q_ss * 2) + chunk * 16 : kNoColumn, 0);
+      }
+      copy_v(0, 0);
+      copy_k(1, 1);
+      copy_v(1, 1);
+      asm volatile("s_waitcnt vmcnt(%0)" :: "n"(3 * kCpy) : "memory");     // K(0) and Q
+      __builtin_amdgcn_s_barrier();
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk)                  // a Q row is read like a K row of the same index
+        qf[kk] = *(lds_bf16x8)(uintptr_t)(uint32_t)(k_a[kk] - (int)lds_ring + (int)lds_smem + kQBase + rg * (32 * kD * 2));
+      qk();
+      sm_mask(0);
+      sm_fix(true);
+      sm_exps();
+      l_run = rs;
+      asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kCpy) : "memory");         // V(0) and K(1)
+      __builtin_amdgcn_s_barrier();
+      copy_k(2, 0);
+      if (ntiles > 1) first_frags();
+    }
+    // The same two phases per tile as above, with two stages per ring: K(t+2) and V(t+1), requested in the vector phase
+    // before, are waited for behind the matrix phase of tile t, and the barrier there makes them visible to the group
+    // and says that K(t+1) and V(t) have been read by all of it, whose stages then take K(t+3) and V(t+2).
+    if (group_b) __builtin_amdgcn_s_barrier();
+    for (int t = 0; t + 1 < ntiles; ++t) {
+      __builtin_amdgcn_s_setprio(2);
+      matrix_phase(t);
+      __builtin_amdgcn_s_setprio(0);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" : "+v"(s[0]), "+v"(s[MB - 1]));
+      copy_k(t + 3, (t + 1) & 1);
+      copy_v(t + 2, t & 1);
+      sm_tile();
+      if (t + 2 < ntiles) first_frags();
+      __builtin_amdgcn_s_barrier();
+    }
+    if (ntiles > 0) pv();
+    if (!group_b) __builtin_amdgcn_s_barrier();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // copies of tiles past the end
+    __syncthreads();                                   // nobody reads Q, K or V any more
+
+    // ---- the key groups' partial results meet ------------------------------------------------------------------
+    // Each group leaves its reference score and sum per row, scales its O by its weight in the row's result, and hands
+    // the head-dim columns it does not finish itself to the group that does (group g: chunks g * kShare .. of 8 columns).
+    constexpr int kShare = DB * 4 / KS;                // chunks of 8 columns (4 registers of each lane half) per group
+    f32x2* stats = reinterpret_cast<f32x2*>(smem + kQBase);              // [key group][row]
+    const float l_own = pair_sum(l_run);
+    if (hf == 0) stats[kg * kRows + rg * 32 + ln] = f32x2{m_ref, l_own};
+    __syncthreads();
+    float m_all = -INFINITY;
+    f32x2 st[KS];
+#pragma unroll
+    for (int g = 0; g < KS; ++g) {
+      st[g] = stats[g * kRows + rg * 32 + ln];
+      if (st[g][1] > 0.f) m_all = fmaxf(m_all, st[g][0]);
+    }
+    float l_tot = 0.f;
+#pragma unroll
+    for (int g = 0; g < KS; ++g)
+      if (st[g][1] > 0.f) l_tot += st[g][1] * fast_exp2((st[g][0] - m_all) * p.scale_log2);
+    const float weight = l_own > 0.f ? fast_exp2((m_ref - m_all) * p.scale_log2) / l_tot : 0.f;
+    if (kg == 0 && hf == 0 && my_q < p.Sq)
+      p.lse[((int64_t)b * p.Hq + hq) * p.Sq + my_q] =
+          l_tot > 0.f ? m_all * p.scale + fast_log2(l_tot) * kLn2 : -INFINITY;
+    // slot (row group, finishing group, giving group): kShare vectors of 64 lanes x 16 bytes
+    auto slot = [&](int to, int from) {
+      return reinterpret_cast<f32x4*>(smem) + ((rg * KS + to) * KS + from) * (kShare * 64) + lane;
+    };
+    f32x4 keep[kShare];
+#pragma unroll
+    for (int to = 0; to < KS; ++to) {
+      f32x4* dst = slot(to, kg);
+#pragma unroll
+      for (int c = 0; c < kShare; ++c) {
+        const int unit = to * kShare + c;
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = o_acc[unit >> 2][(unit & 3) * 4 + e] * weight;
+        if (to == kg) keep[c] = v;
+        else dst[c * 64] = v;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int o = 1; o < KS; ++o) {
+      const f32x4* src = slot(kg, (kg + o) % KS);
+#pragma unroll
+      for (int c = 0; c < kShare; ++c) keep[c] += src[c * 64];
+    }
+    // rows of 256 bytes, chunks swizzled like the K rows
+    unsigned char* os = smem + kQBase + rg * (32 * kD * 2);
+#pragma unroll
+    for (int c = 0; c < kShare; ++c) {
+      u32x2 w;
+      w[0] = pack_bf16(keep[c][0], keep[c][1]);
+      w[1] = pack_bf16(keep[c][2], keep[c][3]);
+      *reinterpret_cast<u32x2*>(os + ln * 256 + (((kg * kShare + c) ^ swz(ln)) << 4) + hf * 8) = w;
+    }
+    __syncthreads();
+    {
+      constexpr int kRowsPerWave = kRows / kWaves;
+      const int chunk = lane & 15;
+      uint16_t* op = p.out + b * p.o_sb + hq * p.o_sh + chunk * 8;
+#pragma unroll
+      for (int it = 0; it < kRowsPerWave / 4; ++it) {
+        const int r = wave * kRowsPerWave + (lane >> 4) + 4 * it;
+        if (q0 + r < p.Sq && chunk * 8 < p.D) {
+          const u32x4 w = *reinterpret_cast<const u32x4*>(smem + kQBase + r * 256 + ((chunk ^ swz(r)) << 4));
+          *reinterpret_cast<u32x4*>(op + (int64_t)(q0 + r) * p.o_ss) = w;
+        }
       }
     }
   }
+}
+
+template <bool CAUSAL, int KK, int KS>
+void launch_one(FwdParams& p, hipStream_t stream) {
+  const int rows = kBM / KS;
+  p.nq_tiles = (p.Sq + rows - 1) / rows;
+  p.total = p.B * p.Hq * p.nq_tiles;
+  p.per_xcd = (p.total + 7) / 8;
+  p.heads_per_xcd = (p.B * p.Hq) % 8 == 0 ? (p.B * p.Hq) / 8 : 0;
+  hipLaunchKernelGGL((attn_fwd_bf16_d128<CAUSAL, KK, KS>), dim3(p.per_xcd * 8), dim3(kWaves * 64), 0, stream, p);
+}
+template <int KK>
+void launch_fwd(FwdParams& p, bool causal, int groups, hipStream_t stream) {
+  if (causal) {
+    if (groups == 4) launch_one<true, KK, 4>(p, stream);
+    else if (groups == 2) launch_one<true, KK, 2>(p, stream);
+    else launch_one<true, KK, 1>(p, stream);
+  } else {
+    if (groups == 4) launch_one<false, KK, 4>(p, stream);
+    else if (groups == 2) launch_one<false, KK, 2>(p, stream);
+    else launch_one<false, KK, 1>(p, stream);
+  }
+}
+
+// Key groups per workgroup (1, 2 or 4): the count with the least estimated time.  A launch is rounds of up to 256
+// workgroups (one per CU); a workgroup costs `fixed` us (Q in, O out, the groups' meeting) and per tile of a group
+// `step` us, plus `busy` us times the share of the CUs at work (clock and L2).  Fitted to launches of 4 .. 2048
+// workgroups over 64 .. 4096 keys, which it gives to within 15 %; measured (us, groups 1 / 2 / 4):
+//     B1 H4  256 x 256      11.2 /  9.2 /  7.8      B4 H5   512 x 512     16.1 / 12.5 / 10.7
+//     B1 H32 1024 x 1024    28.8 / 22.6 / 29.6      B2 H16 1237 x 1237    33.2 / 41.8 / 46.6  (D 80)
+//     B1 H1  4096 x 4096    70.3 / 45.6 / 33.8      B1 H20 4096 x 4096     187 /  176 /  200
+//     B1 H32 4096 x 4096     228 /  255 /  357      B2 H12 1500 x 1500    36.8 / 21.8 / 29.0  (D 64, causal)
+// The split kernel fetches Q and puts whole tiles out of range through 32-bit offsets, which asks for row strides and
+// spans that only views of unheard-of strides exceed.
+int key_groups(const FwdParams& p, bool causal) {
+  if (p.q_ss >= (1 << 22) || (int64_t)p.Sc * p.k_ss >= (1 << 29) || (int64_t)p.Sc * p.v_ss >= (1 << 29)) return 1;
+  struct Cost { float fixed, step, busy; };
+  static constexpr Cost kCost128[3] = {{7.0f, 1.10f, 0.80f}, {6.5f, 1.19f, 0.90f}, {5.2f, 0.81f, 0.49f}};
+  static constexpr Cost kCost64[3] = {{6.0f, 1.05f, 0.17f}, {6.0f, 0.98f, 0.27f}, {4.7f, 0.72f, 0.12f}};
+  const Cost* cost = p.D <= 64 ? kCost64 : kCost128;
+  int best = 1;
+  float best_time = 0.f;
+  for (int i = 0; i < 3; ++i) {
+    const int groups = 1 << i;
+    const int rows = kBM / groups, tile = groups == 4 ? 32 : kBN;
+    const int64_t q_tiles = (p.Sq + rows - 1) / rows;
+    const float n = (float)((int64_t)p.B * p.Hq * q_tiles);
+    auto steps = [&](int64_t keys) { return (float)((keys + tile * groups - 1) / (tile * groups)); };
+    float time;
+    if (!causal) {
+      const float full = floorf(n / 256.f), part = n / 256.f - full, t = steps(p.Sc);
+      time = full * (cost[i].fixed + t * (cost[i].step + cost[i].busy));
+      if (part > 0.f) time += cost[i].fixed + t * (cost[i].step + part * cost[i].busy);
+    } else {
+      // longest tiles first: the longest workgroup, or all of the work spread over the CUs
+      const int64_t shift = (int64_t)p.Sc - p.Sq;
+      auto seen = [&](int64_t row_end) {
+        const int64_t k = row_end + shift < p.Sc ? row_end + shift : p.Sc;
+        return k > 0 ? k : 0;
+      };
+      const float first = steps(seen(rows)), last = steps(seen(q_tiles * rows));
+      const float share = n < 256.f ? n / 256.f : 1.f;
+      const float longest = cost[i].fixed + last * (cost[i].step + 0.5f * share * cost[i].busy);
+      const float spread = n / 256.f * (cost[i].fixed + 0.5f * (first + last) * (cost[i].step + cost[i].busy));
+      time = longest > spread ? longest : spread;
+    }
+    if (i == 0 || time < best_time) { best = groups; best_time = time; }
+  }
+  return best;
 }
 
 }  // namespace
@@ -447,19 +688,10 @@ int attn_fwd_bf16(const void* q, const void* k, const void* v, void* out, float*
   p.o_sb = st[9]; p.o_ss = st[10]; p.o_sh = st[11];
   p.scale = scale;
   p.scale_log2 = scale * kLog2e;
-  p.nq_tiles = (Sq + kBM - 1) / kBM;
-  p.total = B * Hq * p.nq_tiles;
-  p.per_xcd = (p.total + 7) / 8;
-  p.heads_per_xcd = (B * Hq) % 8 == 0 ? (B * Hq) / 8 : 0;
-  const dim3 grid(p.per_xcd * 8), block(kWaves * 64);
   const bool causal = mask == MHIP_MASK_CAUSAL;
-  if (D <= 64) {        // half the on-chip columns, half the MFMAs
-    if (causal) hipLaunchKernelGGL((attn_fwd_bf16_d128<true, 4>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((attn_fwd_bf16_d128<false, 4>), grid, block, 0, stream, p);
-  } else {
-    if (causal) hipLaunchKernelGGL((attn_fwd_bf16_d128<true, 8>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((attn_fwd_bf16_d128<false, 8>), grid, block, 0, stream, p);
-  }
+  const int groups = key_groups(p, causal);
+  if (D <= 64) launch_fwd<4>(p, causal, groups, stream);        // half the on-chip columns, half the MFMAs
+  else launch_fwd<8>(p, causal, groups, stream);
   return launch_status();
 }
 
