@@ -89,6 +89,12 @@ __device__ __forceinline__ void copy4_to_lds(u32x4 rsrc, uint32_t lds_addr, int 
                   "s"(__builtin_amdgcn_readfirstlane(soffset)) : "memory");
 }
 
+// The same with a 64-bit address per lane and no range check: every address has to be readable.
+__device__ __forceinline__ void copy16_to_lds(const void* src, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :: "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(src) : "memory");
+}
+
 // Tiles copied that way are rows of 256 bytes (128 bf16) without padding; chunk c (16 bytes) of row r is
 // kept at chunk position c ^ lds_row_swizzle(r).  With this map both access patterns of the MFMA operand
 // reads are free of bank conflicts: 32 consecutive rows x one chunk (ds_read_b128 of a row-major operand)
