@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/mercury_hip.h"
 
 namespace mhip {
@@ -51,6 +53,18 @@ __device__ __forceinline__ float pair_sum(float x) {
   float a, b;
   pair_exchange(x, a, b);
   return a + b;
+}
+
+// sum of x over the lane's group of 16, in all of its lanes
+__device__ __forceinline__ float row16_sum(float x) {
+  auto rotated = [](float v, auto n) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + decltype(n)::value, 0xf, 0xf, false));
+  };
+  x += rotated(x, std::integral_constant<int, 8>{});
+  x += rotated(x, std::integral_constant<int, 4>{});
+  x += rotated(x, std::integral_constant<int, 2>{});
+  x += rotated(x, std::integral_constant<int, 1>{});
+  return x;
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
