@@ -47,7 +47,7 @@ extern "C" {
 
 /* Bumped whenever an entry point's argument list changes (a caller built against another value must not call).
  * 3: the three descales of mhip_attn_fwd_block are device pointers; mhip_attn_bwd_block takes five stride triples. */
-#define MHIP_ABI_VERSION 3
+#define MHIP_ABI_VERSION 4
 int         mhip_abi_version(void);   /* the MHIP_ABI_VERSION the library was built with */
 int         mhip_version(void);
 /* Optional: per-device set-up the entry points otherwise do on their first call on a device (today: the address
@@ -132,6 +132,27 @@ int mhip_attn_bwd_block_noalloc(const void* dout, const void* q, const void* k, 
                                 int64_t dq_sb, int64_t dq_ss, int64_t dq_sh,  /* dq       */
                                 int64_t o_sb, int64_t o_ss, int64_t o_sh,     /* out      */
                                 float softmax_scale, int mask, int deterministic, void* stream);
+
+/*
+ * The block backward of one chunk of a ring step, with the sums around it (utils/attn_bwd_dsl.py:117-134: dq is summed
+ * in fp32 over the chunks, reduce(op=torch.add), and stored in q's type after the last one; a chunk's dk, dv travel
+ * on in fp32).  With T = the sum over the chunks before this one plus this chunk's dQ, T starting at 0 if `first`:
+ *   not last:  dq_acc = T                 (dq is not used)
+ *   last:      dq = bf16(T)               (dq_acc is read unless first, not written)
+ * dk / dv receive the chunk's gradients in bf16 and dk32 / dv32 (fp32, (B, Sc, Hkv, D) contiguous) the same values in
+ * fp32; either pair may be NULL, not both.  Everything else as in mhip_attn_bwd_block (the same workspace).
+ */
+int mhip_attn_bwd_chunk(const void* dout, const void* q, const void* k, const void* v,
+                        const void* out, const float* lse,
+                        void* dq, float* dq_acc, int first, int last,
+                        void* dk, void* dv, float* dk32, float* dv32,
+                        int B, int Sq, int Sc, int Hq, int Hkv, int D,
+                        int64_t q_sb, int64_t q_ss, int64_t q_sh,     /* q, dout  */
+                        int64_t k_sb, int64_t k_ss, int64_t k_sh,     /* k, v     */
+                        int64_t dk_sb, int64_t dk_ss, int64_t dk_sh,  /* dk, dv   */
+                        int64_t dq_sb, int64_t dq_ss, int64_t dq_sh,  /* dq       */
+                        int64_t o_sb, int64_t o_ss, int64_t o_sh,     /* out      */
+                        float softmax_scale, int mask, void* workspace, void* stream);
 
 /*
  * LSE-rescale merge.  Replaces the TorchScript `_update_out_and_lse`

@@ -42,12 +42,18 @@ constexpr int kNoTile = 0x7fff0000;   // scalar offset that puts every lane of a
 constexpr int kNoColumn = 0x7fff0000; // vector offset with the same effect for one lane (the sum of the two is
                                       // below 2^32: no wrap)
 
+// dq_acc += dQ and dq = dQ; or one chunk of a ring: dq_acc = dQ, dq_acc += dQ, dq = dq_acc + dQ
+enum { kDqAdd = 0, kDqFirst = 1, kDqMiddle = 2, kDqLast = 3 };
+
 struct BwdParams {
   const uint16_t* q; const uint16_t* k; const uint16_t* v; const uint16_t* dout;
   const uint16_t* out; const float* lse;   // saved output and log-sum-exp of the forward
   float* lse2; float* delta;               // both (B, Hq, Sq) fp32: written by the dQ pass, read by the dK / dV pass
   float* softmax_d;                        // rowsum(dout * out) itself for the caller, or null
-  uint16_t* dq; uint16_t* dk; uint16_t* dv; float* dq_acc;
+  uint16_t* dq; uint16_t* dk; uint16_t* dv; float* dq_acc;     // dq may be null next to dq_acc
+  float* dk32; float* dv32;                // the same bf16 values in fp32, (B, Sc, Hkv, D) contiguous, or null; dk / dv
+                                           // may be null then
+  int dq_mode;                             // what dq_acc is for: kDq*
   int B, Sq, Sc, Hq, Hkv, group;
   int D;            // head dimension of the tensors, a multiple of 8 up to kD; columns D .. kD-1 are zeros on chip
   int64_t q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, dk_sb, dk_ss, dk_sh, dq_sb, dq_ss, dq_sh, o_sb, o_ss, o_sh;
@@ -597,27 +603,67 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
       }
     }
   };
-  if (DQ) {
-    write_out(acc1, p.scale, p.dq, p.dq_sb, p.dq_ss, p.dq_sh, hs);
-    if (p.dq_acc != nullptr && my_r < n_st) {
-      // fp32 accumulator (B, Sq, Hq, D) contiguous; every element belongs to exactly one lane
-      float* ap = p.dq_acc + (((int64_t)b * p.Sq + my_r) * p.Hq + hs) * p.D;
+  // The same with fp32 rows on the way (512 bytes, the 32 chunks of 4 columns swizzled by the row): `finish` gets the
+  // lane's 8 columns of a row, whole rows per instruction.  A lane's own accumulator columns are 16 bytes of 32
+  // different rows, which is what reading and writing dq_acc from the accumulators cost.
+  auto write_out32 = [&](const f32x16 (&acc)[4], float mul, auto&& finish) {
+    __syncthreads();
+    unsigned char* os = smem + wave * (32 * kD * 4);
 #pragma unroll
-      for (int db = 0; db < 4; ++db)
+    for (int db = 0; db < 4; ++db)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          if (db * 32 + g * 8 + hf * 4 < p.D) {
-            f32x4* a4 = reinterpret_cast<f32x4*>(ap + db * 32 + g * 8 + hf * 4);
-            f32x4 v = *a4;
+      for (int g = 0; g < 4; ++g) {
+        f32x4 v;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] += acc1[db][4 * g + e] * p.scale;
-            *a4 = v;
-          }
-        }
+        for (int e = 0; e < 4; ++e) v[e] = acc[db][4 * g + e] * mul;
+        *reinterpret_cast<f32x4*>(os + ln * 512 + (((db * 8 + g * 2 + hf) ^ ln) << 4)) = v;
+      }
+    __syncthreads();
+    const int chunk = lane & 15;
+#pragma unroll
+    for (int it = 0; it < 8; ++it) {
+      const int r = (lane >> 4) + 4 * it;
+      const int row = r0 + wave * 32 + r;
+      if (row < n_st && chunk * 8 < p.D) {
+        f32x4 v[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) v[h] = *reinterpret_cast<const f32x4*>(os + r * 512 + (((2 * chunk + h) ^ r) << 4));
+        finish(v, row, chunk * 8);
+      }
     }
-  } else {
+  };
+  auto pack8 = [](const f32x4 (&v)[2]) {
+    return u32x4{pack_bf16(v[0][0], v[0][1]), pack_bf16(v[0][2], v[0][3]), pack_bf16(v[1][0], v[1][1]), pack_bf16(v[1][2], v[1][3])};
+  };
+  if (DQ) {
+    if (p.dq_acc == nullptr) {
+      write_out(acc1, p.scale, p.dq, p.dq_sb, p.dq_ss, p.dq_sh, hs);
+    } else {
+      uint16_t* dq = p.dq ? p.dq + b * p.dq_sb + hs * p.dq_sh : nullptr;
+      write_out32(acc1, p.scale, [&](f32x4 (&v)[2], int row, int col) {
+        f32x4* ap = reinterpret_cast<f32x4*>(p.dq_acc + (((int64_t)b * p.Sq + row) * p.Hq + hs) * p.D + col);
+        u32x4* qp = reinterpret_cast<u32x4*>(dq + (int64_t)row * p.dq_ss + col);
+        if (p.dq_mode == kDqAdd && dq) *qp = pack8(v);
+        if (p.dq_mode != kDqFirst) { v[0] += ap[0]; v[1] += ap[1]; }
+        if (p.dq_mode != kDqLast) { ap[0] = v[0]; ap[1] = v[1]; }
+        else *qp = pack8(v);
+      });
+    }
+  } else if (p.dk32 == nullptr) {
     write_out(acc1, p.scale, p.dk, p.dk_sb, p.dk_ss, p.dk_sh, hs);
     write_out(acc2, 1.f, p.dv, p.dk_sb, p.dk_ss, p.dk_sh, hs);
+  } else {
+    auto store = [&](float* out32, uint16_t* out16) {
+      return [=](f32x4 (&v)[2], int row, int col) {
+        f32x4* op = reinterpret_cast<f32x4*>(out32 + (((int64_t)b * p.Sc + row) * p.Hkv + hs) * p.D + col);
+        const u32x4 w = pack8(v);
+        op[0] = f32x4{bf16_lo(w[0]), bf16_hi(w[0]), bf16_lo(w[1]), bf16_hi(w[1])};
+        op[1] = f32x4{bf16_lo(w[2]), bf16_hi(w[2]), bf16_lo(w[3]), bf16_hi(w[3])};
+        if (out16) *reinterpret_cast<u32x4*>(out16 + b * p.dk_sb + (int64_t)row * p.dk_ss + hs * p.dk_sh + col) = w;
+      };
+    };
+    write_out32(acc1, p.scale, store(p.dk32, p.dk));
+    write_out32(acc2, 1.f, store(p.dv32, p.dv));
   }
 }
 
@@ -664,7 +710,7 @@ int scratch_address(void** ptr) {
 // own_scratch: take the workspace from `scratch` (resolved after the arguments have been checked)
 int bwd_block(const void* dout, const void* q, const void* k, const void* v,
               const void* out, const float* lse,
-              void* dq, void* dk, void* dv, float* dq_acc,
+              void* dq, void* dk, void* dv, float* dq_acc, int dq_mode, float* dk32, float* dv32,
               int B, int Sq, int Sc, int Hq, int Hkv, int D,
               int64_t q_sb, int64_t q_ss, int64_t q_sh,
               int64_t k_sb, int64_t k_ss, int64_t k_sh,
@@ -677,9 +723,11 @@ int bwd_block(const void* dout, const void* q, const void* k, const void* v,
   if (mask != MHIP_MASK_NONE && mask != MHIP_MASK_CAUSAL) return MHIP_EINVAL;
   if (D < 8 || D > kD || (D & 7) != 0) return MHIP_EHEADDIM;     // below 128 the missing columns are zeros on chip
   if (B == 0) return MHIP_OK;
-  if (Sq > 0 && (!dout || !q || !out || !lse || !dq || (!workspace && !own_scratch))) return MHIP_EINVAL;
-  if (Sc > 0 && (!k || !v || !dk || !dv)) return MHIP_EINVAL;
-  const void* ptrs[] = {dout, q, k, v, out, dq, dk, dv, workspace, dq_acc};
+  if (Sq > 0 && (!dout || !q || !out || !lse || (!workspace && !own_scratch))) return MHIP_EINVAL;
+  const bool dq_needed = dq_mode == kDqAdd || dq_mode == kDqLast, acc_needed = dq_mode == kDqFirst || dq_mode == kDqMiddle;
+  if (Sq > 0 && ((dq_needed && !dq) || (acc_needed && !dq_acc))) return MHIP_EINVAL;
+  if (Sc > 0 && (!k || !v || !dk32 != !dv32 || (!dk32 && (!dk || !dv)) || !dk != !dv)) return MHIP_EINVAL;
+  const void* ptrs[] = {dout, q, k, v, out, dq, dk, dv, workspace, dq_acc, dk32, dv32};
   for (const void* ptr : ptrs)
     if (ptr && !aligned16(ptr)) return MHIP_EALIGN;
   const int64_t strides[] = {q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, dk_sb, dk_ss, dk_sh, dq_sb, dq_ss, dq_sh,
@@ -709,7 +757,8 @@ int bwd_block(const void* dout, const void* q, const void* k, const void* v,
   p.lse2 = lse2_buf; p.delta = delta_buf; p.softmax_d = softmax_d;
   p.out = static_cast<const uint16_t*>(out); p.lse = lse;
   p.dq = static_cast<uint16_t*>(dq); p.dk = static_cast<uint16_t*>(dk); p.dv = static_cast<uint16_t*>(dv);
-  p.dq_acc = dq_acc;
+  p.dq_acc = dq_acc; p.dq_mode = dq_mode;
+  p.dk32 = dk32; p.dv32 = dv32;
   p.B = B; p.Sq = Sq; p.Sc = Sc; p.Hq = Hq; p.Hkv = Hkv; p.group = Hq / Hkv;
   p.D = D;
   p.q_sb = q_sb; p.q_ss = q_ss; p.q_sh = q_sh;
@@ -762,7 +811,7 @@ extern "C" int mhip_attn_bwd_block(const void* dout, const void* q, const void* 
                                    float softmax_scale, int mask, int deterministic,
                                    void* workspace, void* stream) {
   (void)deterministic;   // there are no atomics: every run is deterministic
-  return bwd_block(dout, q, k, v, out, lse, dq, dk, dv, dq_acc, B, Sq, Sc, Hq, Hkv, D, q_sb, q_ss, q_sh,
+  return bwd_block(dout, q, k, v, out, lse, dq, dk, dv, dq_acc, kDqAdd, nullptr, nullptr, B, Sq, Sc, Hq, Hkv, D, q_sb, q_ss, q_sh,
                    k_sb, k_ss, k_sh, dk_sb, dk_ss, dk_sh, dq_sb, dq_ss, dq_sh, o_sb, o_ss, o_sh, softmax_scale, mask,
                    workspace, false,
                    static_cast<hipStream_t>(stream));
@@ -780,8 +829,27 @@ extern "C" int mhip_attn_bwd_block_noalloc(const void* dout, const void* q, cons
                                            float softmax_scale, int mask, int deterministic, void* stream) {
   (void)deterministic;
   // the dQ pass overwrites the part of the scratch the dK / dV pass reads, so nothing has to be cleared
-  return bwd_block(dout, q, k, v, out, lse, dq, dk, dv, dq_acc, B, Sq, Sc, Hq, Hkv, D, q_sb, q_ss, q_sh,
+  return bwd_block(dout, q, k, v, out, lse, dq, dk, dv, dq_acc, kDqAdd, nullptr, nullptr, B, Sq, Sc, Hq, Hkv, D, q_sb, q_ss, q_sh,
                    k_sb, k_ss, k_sh, dk_sb, dk_ss, dk_sh, dq_sb, dq_ss, dq_sh, o_sb, o_ss, o_sh, softmax_scale, mask,
                    nullptr, true,
                    static_cast<hipStream_t>(stream));
+}
+
+extern "C" int mhip_attn_bwd_chunk(const void* dout, const void* q, const void* k, const void* v,
+                                   const void* out, const float* lse,
+                                   void* dq, float* dq_acc, int first, int last,
+                                   void* dk, void* dv, float* dk32, float* dv32,
+                                   int B, int Sq, int Sc, int Hq, int Hkv, int D,
+                                   int64_t q_sb, int64_t q_ss, int64_t q_sh,
+                                   int64_t k_sb, int64_t k_ss, int64_t k_sh,
+                                   int64_t dk_sb, int64_t dk_ss, int64_t dk_sh,
+                                   int64_t dq_sb, int64_t dq_ss, int64_t dq_sh,
+                                   int64_t o_sb, int64_t o_ss, int64_t o_sh,
+                                   float softmax_scale, int mask, void* workspace, void* stream) {
+  const bool only = first && last;      // the only chunk: nothing to carry
+  if (!first && !dq_acc) return MHIP_EINVAL;
+  return bwd_block(dout, q, k, v, out, lse, dq, dk, dv, only ? nullptr : dq_acc,
+                   only ? kDqAdd : first ? kDqFirst : last ? kDqLast : kDqMiddle, dk32, dv32,
+                   B, Sq, Sc, Hq, Hkv, D, q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, dk_sb, dk_ss, dk_sh, dq_sb, dq_ss, dq_sh,
+                   o_sb, o_ss, o_sh, softmax_scale, mask, workspace, false, static_cast<hipStream_t>(stream));
 }

@@ -203,6 +203,48 @@ def attn_bwd_block(dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_scale, c
     return ws.view(torch.float32)[2 * slot: 2 * slot + rows].view(B, Hq, Sq)
 
 
+def attn_bwd_chunk(dout, q, k, v, out, softmax_lse, dq: Optional[torch.Tensor], dq_acc: Optional[torch.Tensor],
+                   first: bool, last: bool, dkv: Optional[torch.Tensor], dkv32: Optional[torch.Tensor],
+                   softmax_scale) -> None:
+    """One chunk of a ring step's backward through mhip_attn_bwd_chunk: ``dq_acc`` (fp32, contiguous, q's shape) carries
+    the sum of the chunks' dq from the ``first`` to the ``last`` one, which writes it to ``dq`` (bf16) instead;
+    ``dkv`` (2, B, Sc, Hkv, D) receives the chunk's dk and dv in bf16 and ``dkv32`` (contiguous) the same values in fp32;
+    either may be None.  All operands are taken as they are: 16-byte aligned rows, q and dout of one layout."""
+    _check_block_inputs(q, k, v, 0, -1, -1, 0.0, None)
+    N.require_cuda(dout, out, softmax_lse, dq, dq_acc, dkv, dkv32)
+    B, Sq, Hq, D = q.shape
+    _, Sc, Hkv, _ = k.shape
+    for name, t, like in (("dout", dout, q), ("k", k, k), ("out", out, q), ("dq", dq, q)):
+        if t is not None and (t.shape != like.shape or t.dtype != torch.bfloat16):
+            raise RuntimeError(f"{name} must be bfloat16 with shape {tuple(like.shape)}")
+    if softmax_lse.shape != (B, Hq, Sq) or softmax_lse.dtype != torch.float32 or not softmax_lse.is_contiguous():
+        raise RuntimeError("softmax_lse must be contiguous float32 (B, Hq, Sq)")
+    for name, t, shape in (("dq_acc", dq_acc, q.shape), ("dkv32", dkv32, (2, *k.shape))):
+        if t is not None and (t.shape != shape or t.dtype != torch.float32 or not t.is_contiguous()):
+            raise RuntimeError(f"{name} must be contiguous float32 of shape {tuple(shape)}")
+    if dkv is not None and (dkv.shape != (2, *k.shape) or dkv.dtype != torch.bfloat16):
+        raise RuntimeError(f"dkv must be bfloat16 of shape {(2, *k.shape)}")
+    lib = N.lib()
+    ws = torch.empty((int(lib.mhip_attn_bwd_workspace_bytes(B, Sq, Sc, Hq, Hkv, D)),), dtype=torch.uint8,
+                     device=q.device)
+    z3 = (0, 0, 0)
+    with torch.cuda.device(q.device):
+        code = lib.mhip_attn_bwd_chunk(
+            N.ptr(dout), N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(out), N.ptr(softmax_lse), N.ptr(dq), N.ptr(dq_acc),
+            int(first), int(last), *((None, None) if dkv is None else (N.ptr(dkv[0]), N.ptr(dkv[1]))),
+            *((None, None) if dkv32 is None else (N.ptr(dkv32[0]), N.ptr(dkv32[1]))),
+            B, Sq, Sc, Hq, Hkv, D, *_strides3(q), *_strides3(k), *(z3 if dkv is None else _strides3(dkv[0])),
+            *(z3 if dq is None else _strides3(dq)), *_strides3(out),
+            float(softmax_scale), N.MASK_NONE, N.ptr(ws), N.stream_of(q))
+    N.check(code, "mhip_attn_bwd_chunk")
+
+
+def aligned_rows(*ts: torch.Tensor) -> bool:
+    """Whether the backward kernels take the tensors as they are: bf16, one layout, 16-byte aligned rows."""
+    return all(t.dtype == torch.bfloat16 and t.stride() == ts[0].stride() and t.stride(-1) == 1 and t.data_ptr() % 16 == 0
+               and all(st % 8 == 0 for st in t.stride()[:-1]) for t in ts)
+
+
 @torch.library.custom_op("mercury_amd::_flash_attn_backward", mutates_args=("dq", "dk", "dv"),
                          device_types="cuda")
 def _flash_attn_backward(

@@ -25,7 +25,8 @@ from typing import Optional
 import torch
 
 from . import _native as N
-from .flash_attn_interface import _flash_attn_backward, _flash_attn_forward, attn_bwd_block
+from .flash_attn_interface import (_flash_attn_backward, _flash_attn_forward, aligned_rows, attn_bwd_block,
+                                   attn_bwd_chunk)
 from .merge import (MAX_MERGE_MANY, get_default_args, grad_accumulate, merge_into, merge_many, pack_block,
                     unpack_into, update_out_and_lse)
 from .schedule import (LocalRing, n_dim_to_one_dim, one_dim_to_n_dim, reduce_buffer_route, shift_tuple_element,
@@ -386,13 +387,21 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
     real ring has exactly one contribution per rank, so here each chunk's block gradient is kept in
     ``dkv_chunks[chunk id]`` (fp32) and the rank's own chunk is stored to ``dkv``.
 
-    ``fused_accumulate=True`` (default) lets the block kernel add its fp32 dq straight into the accumulator
-    (one pass fewer over it per chunk, and the sum sees the unrounded block gradient) and casts a chunk's
-    dK/dV to fp32 only when ``dkv_chunks`` asks for it; ``False`` is the literal sequence: block backward
+    ``fused_accumulate=True`` (default) lets the block kernels do the sums: dq's carries over from chunk to chunk in
+    fp32 (the sum sees the unrounded block gradients) and is written in q's type by the last one, and a chunk's dK/dV
+    are written in fp32 where ``dkv_chunks`` asks for them: no pass over the gradients besides.  ``False`` is the literal sequence: block backward
     through ``_flash_attn_backward(**params)``, then ``torch.add`` on the bf16 block gradients."""
     if dropout_p != 0 or alibi_slopes is not None or tuple(window_size) != (-1, -1):
         fused_accumulate = False                # let the operator report what it does not support
-    reduce_dq = torch.zeros(q.shape, dtype=torch.float32, device=q.device) if fused_accumulate else None
+    # operands of other layouts go through the block operator, which copies them where it has to
+    carried = (fused_accumulate and aligned_rows(q, dout) and aligned_rows(o) and lse.is_contiguous()
+               and q.shape == o.shape == dout.shape)
+    write_dq = carried and aligned_rows(dq) and dq.shape == q.shape
+    reduce_dq = None
+    if not carried and fused_accumulate:
+        reduce_dq = torch.zeros(q.shape, dtype=torch.float32, device=q.device)
+    elif carried and not (write_dq and ring.world == 1):
+        reduce_dq = torch.empty(q.shape, dtype=torch.float32, device=q.device)
     _kv = _next_kv = None
     own = ring.current
     for step, hop in enumerate(_hops(ring)):
@@ -406,6 +415,22 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
             send_to, recv_from = _neighbours(ring, hop)
             _next_kv = ring.send_recv(send_to, recv_from, _kv)
             ring.commit()
+        if carried:
+            mine = chunk_id == own
+            direct = mine and dkv.shape == _kv.shape and aligned_rows(dkv[0], dkv[1])
+            block_dkv = chunk_grad = None
+            if direct:
+                block_dkv = dkv
+            elif mine or dkv_chunks is None:
+                block_dkv = torch.empty(_kv.shape, dtype=_kv.dtype, device=_kv.device)
+            if dkv_chunks is not None:
+                chunk_grad = dkv_chunks[chunk_id] = torch.empty(_kv.shape, dtype=torch.float32, device=_kv.device)
+            kv_rows = _kv if aligned_rows(_kv[0], _kv[1]) else _kv.contiguous()
+            attn_bwd_chunk(dout, q, kv_rows[0], kv_rows[1], o, lse, dq if write_dq else None, reduce_dq, step == 0,
+                           write_dq and hop is None, block_dkv, chunk_grad, softmax_scale)
+            if mine and not direct:
+                dkv[...] = block_dkv
+            continue
         block_dq = torch.empty(q.shape, dtype=q.dtype, device=q.device)
         block_dkv = torch.empty(_kv.shape, dtype=kv.dtype, device=kv.device)
         if fused_accumulate:
@@ -434,4 +459,5 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
             dkv_chunks[chunk_id] = red
         if chunk_id == own:
             dkv[...] = red.to(dkv.dtype)
-    dq[...] = reduce_dq.to(dq.dtype)
+    if not write_dq:
+        dq[...] = reduce_dq.to(dq.dtype)

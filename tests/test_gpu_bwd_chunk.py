@@ -1,0 +1,48 @@
+"""The carried sums of the backward ring step (mhip_attn_bwd_chunk): first, middle and last chunk, fp32 dK / dV, bf16
+ones for the rank's own chunk, at ragged rows and head dimensions.
+
+The kernels round P and dS to bf16 (relative 2^-9 each, random): rel-L2 of a gradient within 2^-8; the largest element
+within 2^-8 of the sum of the magnitudes that enter it, for which 12 root mean squares are allowed here; bf16 results
+add 2^-9."""
+import pytest
+import torch
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(name, got, ref):
+    got, ref = got.float().cpu(), ref.float()
+    rms = ref.square().mean().sqrt()
+    assert (got - ref).norm() <= 2 ** -8 * 1.5 * ref.norm() + 1e-6, (name, ((got - ref).norm() / ref.norm()).item())
+    assert (got - ref).abs().max() <= 12 * 2 ** -8 * rms + 2 ** -8 * ref.abs().max(), name
+
+
+@pytest.mark.parametrize("W,S,Hq,Hkv,D", [(1, 300, 2, 2, 128), (2, 129, 4, 2, 64), (3, 257, 3, 1, 40), (4, 64, 2, 2, 128)])
+@pytest.mark.parametrize("dq_dtype,keep", [(torch.bfloat16, True), (torch.float32, True), (torch.bfloat16, False)])
+def test_backward_step_carries_the_sums(W, S, Hq, Hkv, D, dq_dtype, keep):
+    import mercury_artifact_amd as M
+
+    print(f"W{W} S{S} Hq{Hq} Hkv{Hkv} D{D} {dq_dtype} keep={keep}", flush=True)
+    B, rank, scale = 2, W - 1, D ** -0.5
+    g = torch.Generator().manual_seed(W * 1000 + S)
+    q, dout = (torch.randn(B, S, Hq, D, generator=g).bfloat16() for _ in range(2))
+    kvs = [torch.randn(2, B, S, Hkv, D, generator=g).bfloat16() for _ in range(W)]
+    order = O.single_ring_order(rank, W)
+    o, lse = O.ring_forward(q.float(), [c.float() for c in kvs], order, scale)
+    rdq, rdkv = O.ring_backward(q.float(), [c.float() for c in kvs], order, o.bfloat16().float(), lse, dout.float(), scale)
+    dev = [c.cuda() for c in kvs]
+    dq = torch.full(q.shape, float("nan"), dtype=dq_dtype, device="cuda")
+    dkv = torch.full_like(dev[rank], float("nan"))
+    got = {} if keep else None
+    M.flash_attn_backward(q.cuda(), dev[rank], o.bfloat16().cuda(), lse.cuda(), dout.cuda(), dq, dkv, scale,
+                          ring=M.LocalRing((W,), rank, dev), dkv_chunks=got)
+    torch.cuda.synchronize()
+    _close("dq", dq, rdq)
+    _close("own dkv", dkv, torch.stack(tuple(rdkv[rank])))
+    if keep:
+        assert torch.equal(got[rank], dkv.float())
+    for c in range(W) if keep else ():
+        assert got[c].dtype == torch.float32
+        _close(f"dkv {c}", got[c], torch.stack(tuple(rdkv[c])))
