@@ -1,7 +1,10 @@
-"""ctypes binding of libmercury_hip.so (the C ABI declared in include/mercury_hip.h).
+"""Binding of libmercury_hip.so (the C ABI declared in include/mercury_hip.h).
+
+Two ways in: ``lib()`` through ctypes, and ``host``, the compiled module (csrc/host_ops.cpp) whose functions check the
+arguments, allocate and call the same entry points in one step, or return None for a call they leave to Python.
 
 The library is the only implementation: there is no CPU or eager-PyTorch fallback, and a
-missing library is an error, not a reason to take another path.
+missing library or host module is an error, not a reason to take another path.
 """
 from __future__ import annotations
 
@@ -11,6 +14,18 @@ from ctypes import c_float, c_int, c_int64, c_void_p
 from typing import Optional
 
 import torch
+
+try:
+    from .csrc import _mercury_host as host
+except ImportError as _e:               # reported by lib(), the first thing every operator asks for
+
+    class _NoHost:
+        reason = str(_e)
+
+        def __getattr__(self, name):
+            return lambda *args: None
+
+    host = _NoHost()
 
 # MERCURY_HIP_LIB is a deployment option: the path of the built library when it is not kept next to the package.
 LIB_PATH = os.environ.get("MERCURY_HIP_LIB") or os.path.join(
@@ -65,6 +80,9 @@ def lib() -> ctypes.CDLL:
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
+        if host.bind({name: ctypes.cast(getattr(handle, name), c_void_p).value for name in _SIGNATURES}) is not True:
+            raise RuntimeError("the host module _mercury_host is missing or stale: build it with "
+                               f"`python -m mercury_artifact_amd.csrc.build` ({getattr(host, 'reason', 'entry points')})")
         _lib = handle
     return _lib
 

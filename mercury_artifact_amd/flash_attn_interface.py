@@ -76,6 +76,9 @@ def attn_fwd_block(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, softmax_sc
     bfloat16: any head dimension that is a multiple of 8 up to 128 (the kernels work on 128 columns and fill the
     missing ones with zeros on chip, which changes neither the scores nor the columns that exist);
     float8_e4m3fn: any multiple of 16 up to 128, in the same way."""
+    done = N.host.fwd_block(q, k, v, softmax_scale, causal, q_descale, k_descale, v_descale, out, lse)
+    if done is not None:
+        return done
     _check_block_inputs(q, k, v, 0, -1, -1, 0.0, None)
     N.require_cuda(out, lse)
     B, Sq, Hq, D = q.shape
@@ -136,6 +139,35 @@ def _flash_attn_forward(
     return out, lse, empty, rng
 
 
+def _forward_now(q, k, v, dropout_p, softmax_scale, causal, window_size_left, window_size_right, softcap, alibi_slopes,
+                 return_softmax, q_descale=None, k_descale=None, v_descale=None):
+    """What the operator returns, without the dispatcher, where that would do nothing but call the kernel; else None."""
+    if (dropout_p or softcap or alibi_slopes is not None or window_size_left not in (-1, None)
+            or window_size_right not in (-1, None) or not N.host.undispatched(q, k, v, q_descale, k_descale, v_descale)):
+        return None
+    if k.dtype != q.dtype or k.dim() != 4 or q.dim() != 4:      # for the operator to report
+        return None
+    out, lse = attn_fwd_block(q, k, v, softmax_scale, bool(causal), q_descale, k_descale, v_descale)
+    return (out, lse, *N.host.no_dropout(q))
+
+
+class _ForwardOp(type(_flash_attn_forward)):
+    """The registered operator; a plain eager call of it goes straight to the kernel."""
+
+    def __call__(self, *args, **kwargs):
+        if not torch.compiler.is_compiling():
+            try:
+                done = _forward_now(*args, **kwargs)
+            except (TypeError, AttributeError):         # no list of tensors: the operator says so
+                done = None
+            if done is not None:
+                return done
+        return self._opoverload(*args, **kwargs)
+
+
+_flash_attn_forward.__class__ = _ForwardOp
+
+
 @_flash_attn_forward.register_fake
 def _(q, k, v, dropout_p, softmax_scale, causal, window_size_left, window_size_right, softcap,
       alibi_slopes, return_softmax, q_descale=None, k_descale=None, v_descale=None):
@@ -150,6 +182,9 @@ def attn_bwd_block(dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_scale, c
     """Block backward through mhip_attn_bwd_block; writes every element of dq, dk, dv in place and, if
     ``dq_acc`` (fp32, contiguous, q's shape) is given, also adds the block's dq into it.  Returns
     delta = rowsum(dout * out) as the kernel computed it, (B, Hq, Sq) fp32."""
+    delta = N.host.bwd_block(dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_scale, causal, deterministic, dq_acc)
+    if delta is not None:
+        return delta
     _check_block_inputs(q, k, v, 0, -1, -1, 0.0, None)
     N.require_cuda(dout, out, softmax_lse, dq, dk, dv, dq_acc)
     B, Sq, Hq, D = q.shape
@@ -210,6 +245,8 @@ def attn_bwd_chunk(dout, q, k, v, out, softmax_lse, dq: Optional[torch.Tensor], 
     the sum of the chunks' dq from the ``first`` to the ``last`` one, which writes it to ``dq`` (bf16) instead;
     ``dkv`` (2, B, Sc, Hkv, D) receives the chunk's dk and dv in bf16 and ``dkv32`` (contiguous) the same values in fp32;
     either may be None.  All operands are taken as they are: 16-byte aligned rows, q and dout of one layout."""
+    if N.host.bwd_chunk(dout, q, k, v, out, softmax_lse, dq, dq_acc, first, last, dkv, dkv32, softmax_scale):
+        return
     _check_block_inputs(q, k, v, 0, -1, -1, 0.0, None)
     N.require_cuda(dout, out, softmax_lse, dq, dq_acc, dkv, dkv32)
     B, Sq, Hq, D = q.shape
@@ -273,3 +310,29 @@ def _flash_attn_backward(
     _check_block_inputs(q, k, v, dropout_p, window_size_left, window_size_right, softcap, alibi_slopes, causal)
     return attn_bwd_block(dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_scale, bool(causal),
                           bool(deterministic))
+
+
+def _backward_now(dout, q, k, v, out, softmax_lse, dq, dk, dv, dropout_p, softmax_scale, causal, window_size_left,
+                  window_size_right, softcap, alibi_slopes, deterministic, rng_state=None):
+    if (dropout_p or softcap or alibi_slopes is not None or window_size_left not in (-1, None)
+            or window_size_right not in (-1, None)
+            or not N.host.undispatched(dout, q, k, v, out, softmax_lse, dq, dk, dv)):
+        return None
+    return attn_bwd_block(dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_scale, bool(causal), bool(deterministic))
+
+
+class _BackwardOp(type(_flash_attn_backward)):
+    """The registered operator; a plain eager call of it goes straight to the kernels."""
+
+    def __call__(self, *args, **kwargs):
+        if not torch.compiler.is_compiling():
+            try:
+                done = _backward_now(*args, **kwargs)
+            except (TypeError, AttributeError):
+                done = None
+            if done is not None:
+                return done
+        return self._opoverload(*args, **kwargs)
+
+
+_flash_attn_backward.__class__ = _BackwardOp

@@ -53,6 +53,8 @@ def merge_into(acc_out: Optional[torch.Tensor], acc_lse: Optional[torch.Tensor],
     """One call of mhip_lse_merge.  acc (B,Sq,Hq,D)/(B,Sq,Hq,1) fp32 or None for the first block,
     block_out (B,Sq,Hq,D) bf16, block_lse (B,Hq,Sq) fp32, dst like acc (may be acc itself),
     final_out (B,Sq,Hq,D) bf16 contiguous and final_lse (B,Hq,Sq) fp32 contiguous or None."""
+    if N.host.merge_into(acc_out, acc_lse, block_out, block_lse, dst_out, dst_lse, final_out, final_lse):
+        return
     N.require_cuda(acc_out, acc_lse, block_out, block_lse, dst_out, dst_lse, final_out, final_lse)
     B, Sq, Hq, D = block_out.shape
     if block_out.dtype != torch.bfloat16 or block_out.stride(-1) != 1:
@@ -99,6 +101,8 @@ def merge_many(block_outs: Sequence[torch.Tensor], block_lses: Sequence[torch.Te
     start of their row range): block_outs[i] (B, Sq - row_begin[i], Hq, D) bf16 with contiguous heads,
     block_lses[i] (B, Hq, Sq - row_begin[i]) fp32 contiguous, at most ``MAX_MERGE_MANY`` blocks;
     final_out (B,Sq,Hq,D) bf16 and final_lse (B,Hq,Sq) fp32, both contiguous, are written."""
+    if N.host.merge_many(block_outs, block_lses, final_out, final_lse, row_begin):
+        return
     import ctypes
 
     n = len(block_outs)
@@ -248,6 +252,9 @@ def pack_block(block_out: torch.Tensor, block_lse: torch.Tensor,
     """``torch.cat([block_out.float(), block_lse.transpose(-2,-1).unsqueeze(-1)], -1)``
     (utils/flash_attn_dsl.py:396) in one pass; with ``reduce_into`` the result is
     ``flash_reduce(reduce_into, pack)`` without materialising the pack."""
+    packed = N.host.pack_block(block_out, block_lse, reduce_into)
+    if packed is not None:
+        return packed
     N.require_cuda(block_out, block_lse, reduce_into)
     B, Sq, Hq, D = block_out.shape
     block_out, block_lse = block_out.contiguous(), block_lse.contiguous()
@@ -266,6 +273,8 @@ def unpack_into(buf: torch.Tensor, out: torch.Tensor, lse: torch.Tensor) -> None
     """``out[...] = buf[..., :-1].to(out.dtype)``, ``lse[...] = buf[..., -1].transpose(1, 2)`` (the stores after
     the managed reduction, utils/flash_attn_dsl.py:406-407) in one pass: buf (B,Sq,Hq,D+1) fp32, out
     (B,Sq,Hq,D) bf16 contiguous, lse (B,Hq,Sq) fp32 contiguous."""
+    if N.host.unpack_into(buf, out, lse):
+        return
     N.require_cuda(buf, out, lse)
     B, Sq, Hq, W = buf.shape
     D = W - 1

@@ -20,6 +20,7 @@ sequence: ``update_out_and_lse`` per chunk, then ``o[...] = _out.to(o.dtype)``,
 from __future__ import annotations
 
 import warnings
+from functools import lru_cache
 from typing import Optional
 
 import torch
@@ -29,57 +30,61 @@ from .flash_attn_interface import (_flash_attn_backward, _flash_attn_forward, al
                                    attn_bwd_chunk)
 from .merge import (MAX_MERGE_MANY, get_default_args, grad_accumulate, merge_into, merge_many, pack_block,
                     unpack_into, update_out_and_lse)
-from .schedule import (LocalRing, n_dim_to_one_dim, one_dim_to_n_dim, reduce_buffer_route, shift_tuple_element,
-                       zigzag_step)
+from .schedule import (LocalRing, n_dim_to_one_dim, n_ranks, one_dim_to_n_dim, reduce_buffer_route,
+                       shift_tuple_element, zigzag_step)
 
 __all__ = ["flash_attn_pack_kv", "gqa_pack_kv", "flash_attn_pack_split_kv", "flash_attn_expose_reduce",
            "flash_attn_expose_reduce_q_ring",
            "flash_attn_backward", "zigzag_causal_pack_kv", "fp8_pack_split_kv", "quantize_e4m3"]
 
 
-def _hops(ring: LocalRing):
-    """(dim, is_last) per step in generated-loop order: innermost mesh dimension first, a hop on
-    the next dimension when the inner loop wraps, nothing after the very last step."""
-    shape = ring.mesh_shape
-    total = ring.world
-    idx = [0] * len(shape)
-    for step in range(total):
-        hop = None
-        for d in range(len(shape)):
-            if idx[d] + 1 != shape[d]:
-                hop = d
-                break
-        yield hop
+@lru_cache(maxsize=None)
+def _hop_list(mesh_shape):
+    total = n_ranks(mesh_shape)
+    hops = []
+    idx = [0] * len(mesh_shape)
+    for _ in range(total):
+        hops.append(next((d for d in range(len(mesh_shape)) if idx[d] + 1 != mesh_shape[d]), None))
         # advance the odometer (dimension 0 fastest)
-        for d in range(len(shape)):
+        for d in range(len(mesh_shape)):
             idx[d] += 1
-            if idx[d] < shape[d]:
+            if idx[d] < mesh_shape[d]:
                 break
             idx[d] = 0
+    return tuple(hops)
 
 
-def _neighbours(ring: LocalRing, dim: int):
-    me = one_dim_to_n_dim(ring.rank, ring.mesh_shape)
-    size = ring.mesh_shape[dim]
-    send_to = n_dim_to_one_dim(shift_tuple_element(me, dim, 1, size), ring.mesh_shape)
-    recv_from = n_dim_to_one_dim(shift_tuple_element(me, dim, -1, size), ring.mesh_shape)
+def _hops(ring: LocalRing):
+    """The mesh dimension of the hop at every step in generated-loop order: innermost mesh dimension first, a hop on
+    the next dimension when the inner loop wraps, None after the very last step."""
+    return _hop_list(ring.mesh_shape)
+
+
+@lru_cache(maxsize=None)
+def _neighbour_ranks(mesh_shape, rank, dim):
+    me = one_dim_to_n_dim(rank, mesh_shape)
+    size = mesh_shape[dim]
+    send_to = n_dim_to_one_dim(shift_tuple_element(me, dim, 1, size), mesh_shape)
+    recv_from = n_dim_to_one_dim(shift_tuple_element(me, dim, -1, size), mesh_shape)
     return send_to, recv_from
 
 
-def _fwd_params(q, k, v, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra):
-    params = get_default_args(_flash_attn_forward).copy()
-    params.update({
-        "q": q, "k": k, "v": v,
-        "dropout_p": dropout_p,
-        "softmax_scale": softmax_scale,
-        "causal": causal,
-        "alibi_slopes": alibi_slopes,
-        "return_softmax": True and dropout_p > 0,
-        "window_size_left": window_size[0],
-        "window_size_right": window_size[1],
-    })
-    params.update(extra)
-    return params
+def _neighbours(ring: LocalRing, dim: int):
+    return _neighbour_ranks(ring.mesh_shape, ring.rank, dim)
+
+
+def _block_forward(q, k, v, softmax_scale, dropout_p, causal, window_size, alibi_slopes, q_descale=None, k_descale=None,
+                   v_descale=None):
+    """The block operator on the values a generated step passes it by keyword."""
+    return _flash_attn_forward(q, k, v, dropout_p, softmax_scale, causal, window_size[0], window_size[1], 0.0, alibi_slopes,
+                               dropout_p > 0, q_descale, k_descale, v_descale)
+
+
+def _as_rows(t):
+    """``t`` if the kernels take its rows as they are (contiguous last dimension, 16-byte aligned), else a copy."""
+    unit = 16 // t.element_size()
+    fine = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(st % unit == 0 for st in t.stride()[:-1])
+    return t if fine else t.contiguous()
 
 
 _SIDE_STREAMS = {}
@@ -112,7 +117,7 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
     _lse = None
     _kv = None
     _next_kv = None
-    steps = list(_hops(ring))
+    steps = _hops(ring)
     ring_divide = int(ring_divide)
     Sc = kv.shape[2]
     if ring_divide < 1 or Sc % ring_divide:
@@ -140,9 +145,9 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
             LocalRing(ring.mesh_shape, ring.rank, [c[:, :, rows] for c in ring.chunks], copy=ring.copy)
         for step, hop in enumerate(steps):
             if step == 0:
-                _kv = kv[:, :, rows].contiguous()
+                _kv = _as_rows(kv if ring_divide == 1 else kv[:, :, rows])
                 kv_ready = None
-                if side is not None and part > 0:      # the sub-chunk copy above sits behind earlier launches
+                if side is not None and part > 0:      # a copy above sits behind earlier launches
                     kv_ready = torch.cuda.Event()
                     kv_ready.record(main)
             else:
@@ -157,19 +162,17 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
                 if side is not None:                   # what the hop enqueued on the current stream ends here
                     next_ready = torch.cuda.Event()
                     next_ready.record(main)
-            _k = _kv[0]
-            _v = _kv[1]
-            params = _fwd_params(q, _k, _v, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra)
+            _k, _v = _kv.unbind(0)
             if side is not None and done % 2 == 1:
                 if kv_ready is not None:
                     side.wait_event(kv_ready)
                 _kv.record_stream(side)              # may have been allocated by the hop on the current stream
                 with torch.cuda.stream(side):
-                    outputs = _flash_attn_forward(**params)
+                    outputs = _block_forward(q, _k, _v, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra)
                 for t in outputs[:2]:
                     t.record_stream(main)            # allocated under the side stream, read by the fold on the main one
             else:
-                outputs = _flash_attn_forward(**params)
+                outputs = _block_forward(q, _k, _v, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra)
             assert len(outputs) == 4
             block_out, block_lse, _, _ = outputs
             done += 1
@@ -251,8 +254,8 @@ def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=F
             send_to, recv_from = _neighbours(ring, hop)
             _next_kv = ring.send_recv(send_to, recv_from, _kv)
             ring.commit()
-        outputs = _flash_attn_forward(**_fwd_params(q, _kv[0], _kv[1], softmax_scale, dropout_p, causal,
-                                                    window_size, alibi_slopes))
+        _k, _v = _kv.unbind(0)
+        outputs = _block_forward(q, _k, _v, softmax_scale, dropout_p, causal, window_size, alibi_slopes)
         assert len(outputs) == 4
         block_out, block_lse, _, _ = outputs
         buf = pack_block(block_out, block_lse, reduce_into=buf)
@@ -284,8 +287,7 @@ def flash_attn_expose_reduce_q_ring(qs, kvs, os_, lses, softmax_scale, dropout_p
         buf = []
         for r in range(world):
             kv = kvs[r]
-            outputs = _flash_attn_forward(**_fwd_params(q_cur[r], kv[0], kv[1], softmax_scale, dropout_p, causal,
-                                                        window_size, alibi_slopes))
+            outputs = _block_forward(q_cur[r], kv[0], kv[1], softmax_scale, dropout_p, causal, window_size, alibi_slopes)
             assert len(outputs) == 4
             block_out, block_lse, _, _ = outputs
             buf.append(pack_block(block_out, block_lse, reduce_into=arrived[r]))
@@ -335,8 +337,7 @@ def zigzag_causal_pack_kv(q, kv, o, lse, softmax_scale, dropout_p=0, causal=True
             bq, bk, bv, bc, sl = q, _kv[0][:, :half], _kv[1][:, :half], False, None
         else:
             bq, bk, bv, bc, sl = q[:, half:], _kv[0], _kv[1], False, (slice(None), slice(half, None))
-        outputs = _flash_attn_forward(**_fwd_params(bq, bk, bv, softmax_scale, dropout_p, bc,
-                                                    window_size, alibi_slopes))
+        outputs = _block_forward(bq, bk, bv, softmax_scale, dropout_p, bc, window_size, alibi_slopes)
         block_out, block_lse, _, _ = outputs
         if defer:
             blocks.append((block_out, block_lse, 0 if sl is None else half))
@@ -354,6 +355,9 @@ def quantize_e4m3(x: torch.Tensor):
     tensor), x_q = round-to-nearest-even(clamp(x / s, -448, 448)) as ``torch.float8_e4m3fn``.  Returns
     ``(x_q, s)`` with ``s`` a 0-dim fp32 tensor on the device (the block kernel's descale).  fp32 or bf16
     input on the GPU."""
+    done = N.host.quantize_e4m3(x)
+    if done is not None:
+        return done
     N.require_cuda(x)
     if x.dtype not in (torch.float32, torch.bfloat16):
         raise RuntimeError("quantize_e4m3 takes float32 or bfloat16")
@@ -425,8 +429,8 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
                 block_dkv = torch.empty(_kv.shape, dtype=_kv.dtype, device=_kv.device)
             if dkv_chunks is not None:
                 chunk_grad = dkv_chunks[chunk_id] = torch.empty(_kv.shape, dtype=torch.float32, device=_kv.device)
-            kv_rows = _kv if aligned_rows(_kv[0], _kv[1]) else _kv.contiguous()
-            attn_bwd_chunk(dout, q, kv_rows[0], kv_rows[1], o, lse, dq if write_dq else None, reduce_dq, step == 0,
+            _k, _v = _as_rows(_kv).unbind(0)
+            attn_bwd_chunk(dout, q, _k, _v, o, lse, dq if write_dq else None, reduce_dq, step == 0,
                            write_dq and hop is None, block_dkv, chunk_grad, softmax_scale)
             if mine and not direct:
                 dkv[...] = block_dkv

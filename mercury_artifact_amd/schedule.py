@@ -230,6 +230,38 @@ def zigzag_step(rank: int, step: int, world: int) -> Tuple[str, int]:
     return ("kv_first_half", src) if src < rank else ("q_second_half", src)
 
 
+@lru_cache(maxsize=None)
+def _hop_sources(mesh_shape: Tuple[int, ...], dim: int) -> Tuple[int, ...]:
+    """For every rank of the mesh the rank it receives from when all make a hop along ``dim``."""
+    return tuple(n_dim_to_one_dim(shift_tuple_element(one_dim_to_n_dim(r, mesh_shape), dim, -1, mesh_shape[dim]), mesh_shape)
+                 for r in range(n_ranks(mesh_shape)))
+
+
+@lru_cache(maxsize=None)
+def _hop_dim(mesh_shape: Tuple[int, ...], rank: int, to_rank: int, from_rank: int) -> Optional[int]:
+    """Mesh dimension of the hop in which ``rank`` sends to ``to_rank`` and receives from ``from_rank``; None if it
+    sends to itself."""
+    mine = one_dim_to_n_dim(rank, mesh_shape)
+    to = one_dim_to_n_dim(to_rank, mesh_shape)
+    moved = [d for d in range(len(mine)) if mine[d] != to[d]]
+    if len(moved) > 1:
+        raise RuntimeError("a ring hop moves along exactly one mesh dimension")
+    if not moved:
+        return None
+    dim = moved[0]
+    if shift_tuple_element(mine, dim, 1, mesh_shape[dim]) != to or \
+       shift_tuple_element(mine, dim, -1, mesh_shape[dim]) != one_dim_to_n_dim(from_rank, mesh_shape):
+        raise RuntimeError("LocalRing only replays hops that send to +1 and receive from -1")
+    return dim
+
+
+def n_ranks(mesh_shape: Tuple[int, ...]) -> int:
+    world = 1
+    for size in mesh_shape:
+        world *= size
+    return world
+
+
 class LocalRing:
     """Single-process replay of the neighbour exchange (stand-in for ``SendRecv``,
     mercury/backend/pytorch/utils.py:9-39).
@@ -266,28 +298,14 @@ class LocalRing:
         return self.chunks[self.current]
 
     def hop(self, dim: int) -> int:
-        size = self.mesh_shape[dim]
-        nxt = list(self.held)
-        for r in range(self.world):
-            to = n_dim_to_one_dim(shift_tuple_element(one_dim_to_n_dim(r, self.mesh_shape), dim, 1, size),
-                                  self.mesh_shape)
-            nxt[to] = self.held[r]
-        self.held = nxt
+        self.held = [self.held[r] for r in _hop_sources(self.mesh_shape, dim)]
         return self.current
 
     # -- SendRecv protocol -------------------------------------------------------------------------
     def send_recv(self, to_rank: int, from_rank: int, send_tensor: torch.Tensor,
                   recv_tensor: Optional[torch.Tensor] = None) -> torch.Tensor:
-        mine = one_dim_to_n_dim(self.rank, self.mesh_shape)
-        to = one_dim_to_n_dim(to_rank, self.mesh_shape)
-        moved = [d for d in range(len(mine)) if mine[d] != to[d]]
-        if len(moved) > 1:
-            raise RuntimeError("a ring hop moves along exactly one mesh dimension")
-        if moved:
-            dim = moved[0]
-            if shift_tuple_element(mine, dim, 1, self.mesh_shape[dim]) != to or \
-               shift_tuple_element(mine, dim, -1, self.mesh_shape[dim]) != one_dim_to_n_dim(from_rank, self.mesh_shape):
-                raise RuntimeError("LocalRing only replays hops that send to +1 and receive from -1")
+        dim = _hop_dim(self.mesh_shape, self.rank, to_rank, from_rank)
+        if dim is not None:
             self.hop(dim)
         self._pending = True
         got = self.chunks[self.current] if self.chunks is not None else send_tensor

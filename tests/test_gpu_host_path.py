@@ -1,0 +1,141 @@
+"""The compiled host module against the Python functions it stands in for: same results bit for bit where it takes a
+call, the Python function's own handling or error where it does not, the registered operator wherever a mode, a
+transform or autograd is at work."""
+import pytest
+import torch
+
+import oracle as O
+from mercury_artifact_amd import _native as N
+
+pytestmark = pytest.mark.gpu
+
+
+class _Absent:
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def _bits(x):
+    if isinstance(x, (tuple, list)):
+        return [_bits(y) for y in x]
+    return x.contiguous().reshape(-1).view(torch.uint8).cpu()
+
+
+def _same(a, b):
+    if isinstance(a, list):
+        return len(a) == len(b) and all(_same(x, y) for x, y in zip(a, b))
+    return torch.equal(a, b)
+
+
+def _data(B=2, Sq=70, Sc=90, Hq=4, Hkv=2, D=64):
+    g = torch.Generator(device="cuda").manual_seed(3)
+    mk = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    return mk(B, Sq, Hq, D), mk(2, B, Sc, Hkv, D), mk(B, Sq, Hq, D)
+
+
+def _calls():
+    import mercury_artifact_amd as M
+
+    q, kv, dout = _data()
+    out, lse = M.attn_fwd_block(q, kv[0], kv[1], 0.1)
+    wide = torch.zeros(2, 70, 4, 128, device="cuda", dtype=torch.bfloat16)
+    wide[..., :64] = q
+    B, S, H, D = q.shape
+    acc, accl = torch.randn(B, S, H, D, device="cuda"), torch.randn(B, S, H, 1, device="cuda")
+    q8, sc = M.quantize_e4m3(torch.randn(B, S, H, D, device="cuda"))
+
+    def given():
+        o, l = torch.empty_like(q), torch.empty(B, H, S, device="cuda")
+        assert M.attn_fwd_block(q, kv[0], kv[1], 0.1, True, out=o, lse=l)[0] is o
+        return o, l
+
+    def backward(acc_too):
+        dq, dkv = torch.empty_like(q), torch.empty_like(kv)
+        dq_acc = torch.full(q.shape, 0.5, device="cuda") if acc_too else None
+        d = M.attn_bwd_block(dout, q, kv[0], kv[1], out, lse, dq, dkv[0], dkv[1], 0.1, dq_acc=dq_acc)
+        return [d, dq, dkv] + ([dq_acc] if acc_too else [])
+
+    def fold(begins):
+        o, l = torch.empty_like(q), torch.empty(B, H, S, device="cuda")
+        sl = [0, 0] if begins is None else begins
+        M.merge_many([out[:, b:].contiguous() for b in sl], [lse[:, :, b:].contiguous() for b in sl], o, l, begins)
+        return o, l
+
+    def merged(first, final):
+        d = (None, None) if final else (torch.empty_like(acc), torch.empty_like(accl))
+        f = (torch.empty_like(q), torch.empty(B, H, S, device="cuda")) if final else (None, None)
+        M.merge_into(*((None, None) if first else (acc, accl)), out, lse, *d, *f)
+        return [t for t in (*d, *f) if t is not None]
+
+    return {
+        "forward": lambda: M.attn_fwd_block(q, kv[0], kv[1], 0.1),
+        "forward of a view, descale a Python number": lambda: M.attn_fwd_block(wide[..., :64], kv[0], kv[1], 0.1, q_descale=1.0),
+        "forward into given tensors": given,
+        "forward e4m3": lambda: M.attn_fwd_block(q8, q8, q8, 0.1, q_descale=sc, k_descale=sc, v_descale=sc),
+        "operator": lambda: M._flash_attn_forward(q, kv[0], kv[1], 0.0, 0.1, True, -1, -1, 0.0, None, False)[:2],
+        "backward": lambda: backward(False),
+        "backward with accumulator": lambda: backward(True),
+        "fold": lambda: fold(None),
+        "fold of tails": lambda: fold([0, 33]),
+        "first merge": lambda: merged(True, False),
+        "merge": lambda: merged(False, False),
+        "last merge": lambda: merged(False, True),
+        "pack": lambda: M.pack_block(out, lse),
+        "pack and reduce": lambda: M.pack_block(out, lse, torch.cat([acc, accl], -1)),
+        "quantise": lambda: M.quantize_e4m3(acc),
+        "quantise a view": lambda: M.quantize_e4m3(acc[:, :, 1:3]),
+    }
+
+
+def test_host_module_gives_the_python_functions_results(monkeypatch):
+    calls = _calls()
+    for name, call in calls.items():
+        print(name, flush=True)
+        fast = _bits(call())
+        with monkeypatch.context() as m:
+            m.setattr(N, "host", _Absent())
+            slow = _bits(call())
+        assert _same(fast, slow), name
+
+
+def test_what_the_host_module_declines_is_reported_as_before():
+    import mercury_artifact_amd as M
+
+    q, kv, _ = _data()
+    with pytest.raises(RuntimeError, match="GPU only"):
+        M.attn_fwd_block(q.cpu(), kv[0], kv[1], 0.1)
+    with pytest.raises(RuntimeError, match="dtype"):
+        M.attn_fwd_block(q.half(), kv[0].half(), kv[1].half(), 0.1)
+    with pytest.raises(RuntimeError, match="shape mismatch"):
+        M.attn_fwd_block(q, kv[0][:, :3], kv[1], 0.1)
+    with pytest.raises(RuntimeError, match="softmax scale"):
+        M.attn_fwd_block(q, kv[0], kv[1], -1.0)
+    with pytest.raises(RuntimeError, match="dropout"):
+        M._flash_attn_forward(q, kv[0], kv[1], 0.5, 0.1, False, -1, -1, 0.0, None, False)
+    with pytest.raises(RuntimeError):
+        M._flash_attn_forward(q, kv[0])
+    with pytest.raises(RuntimeError, match="final_out"):
+        M.merge_many([q], [torch.zeros(2, 4, 70, device="cuda")], q.float(), torch.zeros(2, 4, 70, device="cuda"))
+
+
+def test_the_operator_goes_through_the_dispatcher_where_something_watches():
+    import mercury_artifact_amd as M
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    q, kv, _ = _data()
+    args = (q, kv[0], kv[1], 0.0, 0.1, False, -1, -1, 0.0, None, False)
+    seen = []
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, a=(), kw=None):
+            seen.append(str(func))
+            return func(*a, **(kw or {}))
+
+    with Watch():
+        M._flash_attn_forward(*args)
+    assert any("mercury_amd._flash_attn_forward" in s for s in seen)
+    out = M._flash_attn_forward(q.detach().requires_grad_(), *args[1:])[0]
+    with torch.no_grad():
+        plain = M._flash_attn_forward(q.detach().requires_grad_(), *args[1:])[0]
+    assert torch.equal(out, plain) and not plain.requires_grad
+    assert torch.ops.mercury_amd._flash_attn_forward(*args)[0].equal(plain)
