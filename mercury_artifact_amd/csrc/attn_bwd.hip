@@ -64,8 +64,12 @@ struct BwdParams {
   int heads_per_xcd;   // (batch, stationary head) pairs per XCD when they divide evenly, else 0
 };
 
-template <bool DQ, bool CAUSAL>
+// KK = k-steps of 16 head-dim values in T1 / T2: 8 computes on all 128 on-chip columns; 4 is the instantiation for head
+// dimensions up to 64, which leaves out the MFMAs, accumulators and fragments of the zero columns.  The vector work of a
+// tile is the same, so a T1 / T2 slot carries twice of it: 4096 x 4096, H32, D 64 takes 473 us instead of 654.
+template <bool DQ, bool CAUSAL, int KK>
 __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p) {
+  constexpr int DB = KK / 2;                    // blocks of 32 head-dim values in the accumulators
   // The dQ pass needs half the accumulators of the dK / dV pass and fits two wavefronts per SIMD: its workgroup
   // is eight wavefronts sharing the streamed K / V tiles.
   constexpr int kWavesWg = DQ ? 8 : 4;
@@ -121,7 +125,7 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
   // ---- stationary operands: B operands of T1 / T2, lane (ln, hf) holds row[16 ks + 8 hf .. +7]; for dQ the
   // query is the stationary row and its lse2 / delta are per-lane scalars.  All loaded further down, behind
   // the first tile copies, so that one wait covers both latencies. ---------------------------------------
-  bf16x8 xf[8], yf[8];
+  bf16x8 xf[KK], yf[KK];
   float lse2_lane = 0.f, delta_lane = 0.f;
 
   // ---- streamed tiles ---------------------------------------------------------------------------------
@@ -222,19 +226,19 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
   };
 
   // row-major operand reads (A of T1 / T2): lane (ln, hf) reads chunk 2 kk + hf of row 32 mb + ln
-  int rm_rd[8];                                       // + mb * 8192
+  int rm_rd[KK];                                      // + mb * 8192
 #pragma unroll
-  for (int kk = 0; kk < 8; ++kk) rm_rd[kk] = ln * 256 + (((2 * kk + hf) ^ lds_row_swizzle(ln)) << 4);
+  for (int kk = 0; kk < KK; ++kk) rm_rd[kk] = ln * 256 + (((2 * kk + hf) ^ lds_row_swizzle(ln)) << 4);
   // transposed operand reads (A of the second MFMAs) for head-dim block db and k-step (mb, j2): the lane's
   // 8 streamed rows are R + {0..3} and R + 8 + {0..3}, R = 32 mb + 16 j2 + 4 hf -- the rows its P / dS
   // registers hold.  One ds_read_b64_tr_b16 per group of 4 rows: within 16 lanes, lane s supplies the
   // address of row R + s/4, head-dim values 4 (s%4) .. +3 of the 16-column strip, and receives column s.
-  int tr_rd[4][2];                                    // [db][second four rows]  + mb * 8192 + j2 * 4096
+  int tr_rd[DB][2];                                   // [db][second four rows]  + mb * 8192 + j2 * 4096
   {
     const int s16 = lane & 15, strip = (lane >> 4) & 1;
     const int cl = 2 * strip + ((s16 & 3) >> 1);
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+    for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int row = 8 * h + 4 * hf + (s16 >> 2);
@@ -243,15 +247,15 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
   }
   typedef __attribute__((address_space(3))) bf16x4* lds_bf16x4;
   typedef __attribute__((address_space(3))) const bf16x8* lds_bf16x8;
-  f32x16 acc1[4], acc2[4];      // DQ: acc1 = dQ^T.  Otherwise acc1 = dK^T, acc2 = dV^T
+  f32x16 acc1[DB], acc2[DB];    // DQ: acc1 = dQ^T.  Otherwise acc1 = dK^T, acc2 = dV^T
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < DB; ++i)
 #pragma unroll
     for (int j = 0; j < 16; ++j) { acc1[i][j] = 0.f; acc2[i][j] = 0.f; }
   const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
   // Tile t lives in stage t % 4 and is processed as two halves of 32 streamed rows.  Per tile the matrix
-  // pipe sees one unbroken sequence of MFMA slots in four phases:
+  // pipe sees one unbroken sequence of MFMA slots in four phases (half as many slots in each on 64 columns):
   //   P0  T1 / T2 of (t, second half)      16 slots, each carrying P / dS of one register of (t, first half)
   //   P1  accumulate (t, first half)       16 slots (8 for dQ)
   //   P2  T1 / T2 of (t+1, first half)     16 slots, each carrying P / dS of one register of (t, second half)
@@ -264,8 +268,10 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
   // stays the same.
   // operand reads in flight ahead of the MFMAs (2, 4 and 8 measure the same; 2 keeps the dQ pass inside 256 registers)
   constexpr int kDepth = DQ ? 2 : 4;
-  constexpr int kAcc = DQ ? 8 : 16;                        // slots of an accumulate phase
-  constexpr int kP1 = 16, kP2 = 16 + kAcc, kP3 = 32 + kAcc, kSlots = 32 + 2 * kAcc;
+  constexpr int kT = 2 * KK;                               // slots of a T1 / T2 phase
+  constexpr int kAcc = DQ ? 2 * DB : 4 * DB;               // slots of an accumulate phase
+  constexpr int kP1 = kT, kP2 = kT + kAcc, kP3 = 2 * kT + kAcc, kSlots = 2 * (kT + kAcc);
+  constexpr int kVec = 16 / kT;                            // steps of the vector pipeline per slot
   typedef __attribute__((address_space(3))) const f32x4* lds_f32x4;
   // LDS addresses of the operand reads.  rm_a / tr_a hold, per lane, the addresses inside ONE tile's stage and are
   // moved on to the next stage in place, each at a point of the slot sequence where no read of its kind is due
@@ -273,13 +279,13 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
   // those of the next tile start at slot kP2 - kDepth; tr_a in the last kDepth slots, after the last transposed read).
   // ld_cur / ld_next address lse2 / -delta of the current and the next tile.  Everything else about an address
   // is an immediate offset of the LDS instruction.
-  int rm_a[8], tr_a[4][2];
+  int rm_a[KK], tr_a[DB][2];
 #pragma unroll
-  for (int kk = 0; kk < 8; ++kk) rm_a[kk] = rm_rd[kk] + (int)lds_base;
+  for (int kk = 0; kk < KK; ++kk) rm_a[kk] = rm_rd[kk] + (int)lds_base;
 #pragma unroll
-  for (int db = 0; db < 4; ++db) { tr_a[db][0] = tr_rd[db][0] + (int)lds_base; tr_a[db][1] = tr_rd[db][1] + (int)lds_base; }
+  for (int db = 0; db < DB; ++db) { tr_a[db][0] = tr_rd[db][0] + (int)lds_base; tr_a[db][1] = tr_rd[db][1] + (int)lds_base; }
   int ld_cur = (int)lds_base + hf * 16, ld_next = ld_cur + kStageBytes;
-  // slot i (0..15) of the T1 / T2 sequence of one half: k-step i / 2, X (T1) on even and Y (T2) on odd slots
+  // slot i of the T1 / T2 sequence of one half: k-step i / 2, X (T1) on even and Y (T2) on odd slots
   auto read_rm = [&](int mb, int i) -> bf16x8 {
     return *(lds_bf16x8)(uintptr_t)(uint32_t)(rm_a[i >> 1] + mb * 8192 + ((i & 1) ? kOffY : 0));
   };
@@ -294,9 +300,9 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
   // slot i of an accumulate phase of half mb: head-dim block and k-step, X^T (dS) / Y^T (P) alternating for dK, dV
   auto read_acc = [&](int mb, int i) -> bf16x8 {
     const int m = DQ ? i : (i >> 1);
-    const int off = mb * 8192 + (m >> 2) * 4096 + ((!DQ && (i & 1)) ? kOffY : 0);
-    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(tr_a[m & 3][0] + off));
-    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(tr_a[m & 3][1] + off));
+    const int off = mb * 8192 + (m / DB) * 4096 + ((!DQ && (i & 1)) ? kOffY : 0);
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(tr_a[m % DB][0] + off));
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(tr_a[m % DB][1] + off));
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
 
@@ -372,10 +378,15 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
         dsfrag[j2] = __builtin_bit_cast(bf16x8, wd);
       }
   };
-  constexpr int kVecTail = DQ ? 4 : 8;      // accumulate-phase slots that still carry vector work
+  // steps 16 .. of the vector pipeline, behind the T1 / T2 phase, run in the first slots of the accumulate phase
+  auto vector_tail = [&](int i, f32x16& c1, f32x16& c2, int mb) {
+#pragma unroll
+    for (int v = 0; v < kVec; ++v)
+      if (i * kVec + v < (DQ ? 4 : 8)) vector_slot(16 + i * kVec + v, c1, c2, mb);
+  };
   auto acc_mfma = [&](int i, const bf16x8& a) {
     const int m = DQ ? i : (i >> 1);
-    const int db = m & 3, j2 = m >> 2;
+    const int db = m % DB, j2 = m / DB;
     if (DQ || !(i & 1)) acc1[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, dsfrag[j2], acc1[db], 0, 0, 0);
     else acc2[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pfrag[j2], acc2[db], 0, 0, 0);
   };
@@ -388,7 +399,7 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
     if (s < kP3) return read_rm(0, s - kP2);
     return read_acc(1, s - kP3);
   };
-  static_assert(kP2 - kDepth >= 16 && 4 % kDepth == 0, "rm_a moves in the last kDepth slots of P0, tr_a in the last kDepth slots of P3");
+  static_assert(kP2 - kDepth >= kT && KK % kDepth == 0 && 2 * DB % kDepth == 0, "rm_a moves in the last kDepth slots of P0, tr_a in the last kDepth slots of P3");
 
   // Stationary rows: read straight into the fragment layout every load instruction would touch 32 rows (24 such loads
   // per wavefront in the dQ pass, one wait for all of them and the tiles).  They are copied to LDS instead, four whole
@@ -412,9 +423,9 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
         copy16_to_lds(src + (int64_t)row_of(u) * st_ss + (col < p.D ? col : 0), dst + u * 1024);
       }
     };
-    auto read_rows = [&](uint32_t src, bf16x8 (&f)[8]) {
+    auto read_rows = [&](uint32_t src, bf16x8 (&f)[KK]) {
 #pragma unroll
-      for (int ks = 0; ks < 8; ++ks) {
+      for (int ks = 0; ks < KK; ++ks) {
         f[ks] = *(lds_bf16x8)(uintptr_t)(src + rm_rd[ks]);
         if (ks * 16 + hf * 8 >= p.D) f[ks] = bf16x8{};
       }
@@ -425,7 +436,7 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
     // kernel that does gets its 256 registers split 128 / 128).
     auto pin = [&]() {
 #pragma unroll
-      for (int ks = 0; ks < 8; ++ks) {
+      for (int ks = 0; ks < KK; ++ks) {
         if (DQ) { asm volatile("" : "+v"(xf[ks])); asm volatile("" : "+v"(yf[ks])); }
         else { asm volatile("" : "+a"(xf[ks])); asm volatile("" : "+a"(yf[ks])); }
       }
@@ -500,9 +511,9 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
 #pragma unroll
     for (int i = 0; i < kDepth; ++i) ring[i] = read_rm(0, i);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
+    for (int i = 0; i < kT; ++i) {
       t_mfma(i, ring[i % kDepth], ta1, ta2);
-      if (i + kDepth < 16) ring[i % kDepth] = read_rm(0, i + kDepth);
+      if (i + kDepth < kT) ring[i % kDepth] = read_rm(0, i + kDepth);
     }
 #pragma unroll
     for (int i = 0; i < kDepth; ++i) ring[i] = read_rm(1, i);            // slots 0 .. 3 of tile 0
@@ -522,51 +533,54 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
     // byte distance from this tile's stage to the next tile's, and from that one to the one after
     const int step1 = ((t + 1) & 3) == 0 ? -3 * kStageBytes : kStageBytes;
     const int step2 = ((t + 2) & 3) == 0 ? -3 * kStageBytes : kStageBytes;
-    static_assert(kSlots % kDepth == 0 && 16 % kDepth == 0, "the ring position is the slot number modulo its depth");
+    static_assert(kSlots % kDepth == 0 && kT % kDepth == 0 && kAcc % kDepth == 0, "the ring position is the slot number modulo its depth");
     mask_half(ta1, c0);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {                       // P0, carrying the copies of tile t+3
+    for (int i = 0; i < kT; ++i) {                       // P0, carrying the copies of tile t+3
       t_mfma(i, ring[i % kDepth], tb1, tb2);
-      vector_slot(i, ta1, ta2, 0);
-      if (i < kCopiesPerTile) copy_piece(i, (t + 3) & 3);
-      ring[i % kDepth] = read_slot(i + kDepth);
-      if (i >= 16 - kDepth) {                            // the last read of this tile's T1 / T2 operands is out: on to the next
 #pragma unroll
-        for (int j = 0; j < 8 / kDepth; ++j) rm_a[(i - (16 - kDepth)) * (8 / kDepth) + j] += step1;
+      for (int v = 0; v < kVec; ++v) vector_slot(i * kVec + v, ta1, ta2, 0);
+#pragma unroll
+      for (int piece = i; piece < kCopiesPerTile; piece += kT) copy_piece(piece, (t + 3) & 3);
+      ring[i % kDepth] = read_slot(i + kDepth);
+      if (i >= kT - kDepth) {                            // the last read of this tile's T1 / T2 operands is out: on to the next
+#pragma unroll
+        for (int j = 0; j < KK / kDepth; ++j) rm_a[(i - (kT - kDepth)) * (KK / kDepth) + j] += step1;
       }
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int i = 0; i < kAcc; ++i) {                     // P1
-      if (i < kVecTail) vector_slot(16 + i, ta1, ta2, 0);
+      vector_tail(i, ta1, ta2, 0);
       acc_mfma(i, ring[(kP1 + i) % kDepth]);
       if (!DQ && i == kAcc - 2) read_ld(false, 1, 0, lv[0]);
       // -delta for T2 of (t+1, first half), which starts in P2: read once the vector work on this half's dP is
-      // through (slot 7), so that the values can land in the registers T2 accumulates in
-      if (!DQ && i >= 8 && i < 12) read_nd(true, 0, i - 8);
+      // through (half of the slots), so that the values can land in the registers T2 accumulates in
+      if (!DQ && i >= kAcc / 2 && i < kAcc / 2 + 4) read_nd(true, 0, i - kAcc / 2);
       ring[(kP1 + i) % kDepth] = read_slot(kP1 + i + kDepth);
       __builtin_amdgcn_sched_barrier(0);
     }
     mask_half(tb1, c0 + 32);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {                       // P2
+    for (int i = 0; i < kT; ++i) {                       // P2
       t_mfma(i, ring[(kP2 + i) % kDepth], ta1, ta2);
-      vector_slot(i, tb1, tb2, 1);
+#pragma unroll
+      for (int v = 0; v < kVec; ++v) vector_slot(i * kVec + v, tb1, tb2, 1);
       ring[(kP2 + i) % kDepth] = read_slot(kP2 + i + kDepth);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int i = 0; i < kAcc; ++i) {                     // P3
-      if (i < kVecTail) vector_slot(16 + i, tb1, tb2, 1);
+      vector_tail(i, tb1, tb2, 1);
       acc_mfma(i, ring[(kP3 + i) % kDepth]);
       if (!DQ && i == kAcc - 2) read_ld(true, 0, 0, lv[0]);
-      if (!DQ && i >= 8 && i < 12) read_nd(true, 1, i - 8);            // T2 of (t+1, second half): P0 of the next tile
+      if (!DQ && i >= kAcc / 2 && i < kAcc / 2 + 4) read_nd(true, 1, i - kAcc / 2);   // T2 of (t+1, second half): P0 of the next tile
       ring[(kP3 + i) % kDepth] = read_slot(kP3 + i + kDepth);
       if (i >= kAcc - kDepth) {                          // the last transposed read of this tile has been issued
 #pragma unroll
-        for (int j = 0; j < 4 / kDepth; ++j) {
-          const int db = (i - (kAcc - kDepth)) * (4 / kDepth) + j;
-          tr_a[db][0] += step1; tr_a[db][1] += step1;
+        for (int j = 0; j < 2 * DB / kDepth; ++j) {
+          const int a = (i - (kAcc - kDepth)) * (2 * DB / kDepth) + j;
+          tr_a[a >> 1][a & 1] += step1;
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -577,12 +591,12 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the zero-filled copies of tiles past the end
 
   // ---- epilogue: acc^T[d][r] -> rows of the output through LDS --------------------------------------------
-  auto write_out = [&](const f32x16 (&acc)[4], float mul, uint16_t* dst, int64_t d_sb, int64_t d_ss,
+  auto write_out = [&](const f32x16 (&acc)[DB], float mul, uint16_t* dst, int64_t d_sb, int64_t d_ss,
                        int64_t d_sh, int head) {
     __syncthreads();
     unsigned char* os = smem + wave * (32 * kOStride * 2);
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+    for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         u32x2 w;
@@ -606,11 +620,11 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
   // The same with fp32 rows on the way (512 bytes, the 32 chunks of 4 columns swizzled by the row): `finish` gets the
   // lane's 8 columns of a row, whole rows per instruction.  A lane's own accumulator columns are 16 bytes of 32
   // different rows, which is what reading and writing dq_acc from the accumulators cost.
-  auto write_out32 = [&](const f32x16 (&acc)[4], float mul, auto&& finish) {
+  auto write_out32 = [&](const f32x16 (&acc)[DB], float mul, auto&& finish) {
     __syncthreads();
     unsigned char* os = smem + wave * (32 * kD * 4);
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+    for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         f32x4 v;
@@ -707,6 +721,18 @@ int scratch_address(void** ptr) {
   return MHIP_OK;
 }
 
+template <bool DQ, int KK>
+void launch_pass_kk(const BwdParams& p, bool causal, hipStream_t st) {
+  const dim3 grid(p.per_xcd * 8), block(DQ ? 512 : 256);
+  if (causal) hipLaunchKernelGGL((bwd_main<DQ, true, KK>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((bwd_main<DQ, false, KK>), grid, block, 0, st, p);
+}
+template <bool DQ>
+void launch_pass(const BwdParams& p, bool causal, hipStream_t st) {
+  if (p.D <= 64) launch_pass_kk<DQ, 4>(p, causal, st);
+  else launch_pass_kk<DQ, 8>(p, causal, st);
+}
+
 // own_scratch: take the workspace from `scratch` (resolved after the arguments have been checked)
 int bwd_block(const void* dout, const void* q, const void* k, const void* v,
               const void* out, const float* lse,
@@ -775,8 +801,7 @@ int bwd_block(const void* dout, const void* q, const void* k, const void* v,
     p.total = B * Hq * p.n_tiles;
     p.per_xcd = (p.total + 7) / 8;
     p.heads_per_xcd = (B * Hq) % 8 == 0 ? (B * Hq) / 8 : 0;
-    if (causal) hipLaunchKernelGGL((bwd_main<true, true>), dim3(p.per_xcd * 8), dim3(512), 0, st, p);
-    else hipLaunchKernelGGL((bwd_main<true, false>), dim3(p.per_xcd * 8), dim3(512), 0, st, p);
+    launch_pass<true>(p, causal, st);
   }
   if (Sc > 0) {
     // dK, dV: one workgroup per 128 keys of one kv head
@@ -784,8 +809,7 @@ int bwd_block(const void* dout, const void* q, const void* k, const void* v,
     p.total = B * Hkv * p.n_tiles;
     p.per_xcd = (p.total + 7) / 8;
     p.heads_per_xcd = (B * Hkv) % 8 == 0 ? (B * Hkv) / 8 : 0;
-    if (causal) hipLaunchKernelGGL((bwd_main<false, true>), dim3(p.per_xcd * 8), dim3(256), 0, st, p);
-    else hipLaunchKernelGGL((bwd_main<false, false>), dim3(p.per_xcd * 8), dim3(256), 0, st, p);
+    launch_pass<false>(p, causal, st);
   }
   return launch_status();
 }

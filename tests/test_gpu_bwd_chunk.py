@@ -3,7 +3,8 @@ ones for the rank's own chunk, at ragged rows and head dimensions.
 
 The kernels round P and dS to bf16 (relative 2^-9 each, random): rel-L2 of a gradient within 2^-8; the largest element
 within 2^-8 of the sum of the magnitudes that enter it, for which 12 root mean squares are allowed here; bf16 results
-add 2^-9."""
+add 2^-9.  Where the gradient is exactly zero (one key: dP = delta) the fp32 sums of D products of N(0,1) values, |dP| up
+to 40, leave up to D 2^-24 40 in dS; 1e-4 is allowed absolutely."""
 import pytest
 import torch
 
@@ -15,8 +16,8 @@ pytestmark = pytest.mark.gpu
 def _close(name, got, ref):
     got, ref = got.float().cpu(), ref.float()
     rms = ref.square().mean().sqrt()
-    assert (got - ref).norm() <= 2 ** -8 * 1.5 * ref.norm() + 1e-6, (name, ((got - ref).norm() / ref.norm()).item())
-    assert (got - ref).abs().max() <= 12 * 2 ** -8 * rms + 2 ** -8 * ref.abs().max(), name
+    assert (got - ref).norm() <= 2 ** -8 * 1.5 * ref.norm() + 1e-4, (name, ((got - ref).norm() / ref.norm()).item())
+    assert (got - ref).abs().max() <= 12 * 2 ** -8 * rms + 2 ** -8 * ref.abs().max() + 1e-4, name
 
 
 @pytest.mark.parametrize("W,S,Hq,Hkv,D", [(1, 300, 2, 2, 128), (2, 129, 4, 2, 64), (3, 257, 3, 1, 40), (4, 64, 2, 2, 128)])
@@ -46,3 +47,29 @@ def test_backward_step_carries_the_sums(W, S, Hq, Hkv, D, dq_dtype, keep):
     for c in range(W) if keep else ():
         assert got[c].dtype == torch.float32
         _close(f"dkv {c}", got[c], torch.stack(tuple(rdkv[c])))
+
+
+@pytest.mark.parametrize("D", [8, 56, 64, 72])
+@pytest.mark.parametrize("Sq,Sc,Hq,Hkv,causal", [(1, 1, 2, 1, False), (65, 129, 4, 2, False), (257, 63, 2, 2, True),
+                                                 (320, 400, 3, 3, True), (130, 700, 2, 1, False)])
+def test_backward_block_on_narrow_heads(D, Sq, Sc, Hq, Hkv, causal):
+    """Both sides of the line between the 64-column and the 128-column kernels, ragged rows and keys, several turns of
+    the tile ring."""
+    import mercury_artifact_amd as M
+
+    print(f"D{D} Sq{Sq} Sc{Sc} Hq{Hq} Hkv{Hkv} causal={causal}", flush=True)
+    g = torch.Generator().manual_seed(D * 1000 + Sq)
+    q, dout = (torch.randn(2, Sq, Hq, D, generator=g).bfloat16() for _ in range(2))
+    kv = torch.randn(2, 2, Sc, Hkv, D, generator=g).bfloat16()
+    scale = D ** -0.5
+    o, lse = O.block_attention(q.float(), kv[0].float(), kv[1].float(), scale, causal=causal)
+    refs = O.block_backward(dout.float(), q.float(), kv[0].float(), kv[1].float(), o.bfloat16().float(), lse, scale, causal=causal)
+    dev = [x.cuda() for x in (dout, q, kv[0], kv[1], o.bfloat16(), lse)]
+    dq = torch.full_like(dev[1], float("nan"))
+    dkv = torch.full((2, *dev[2].shape), float("nan"), dtype=torch.bfloat16, device="cuda")
+    delta = M.attn_bwd_block(*dev, dq, dkv[0], dkv[1], scale, causal=causal)
+    torch.cuda.synchronize()
+    for name, got, ref in zip(("dq", "dk", "dv"), (dq, dkv[0], dkv[1]), refs):
+        _close(name, got, ref)
+    want = (dout.float() * o.bfloat16().float()).sum(-1).transpose(1, 2)
+    assert (delta.cpu() - want).abs().max() <= 1e-4
