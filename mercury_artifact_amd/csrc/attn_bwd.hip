@@ -4,16 +4,18 @@
 //     P = exp(scale * q k^T - lse),  delta = rowsum(dout * out)
 //     dV = P^T dout,  dP = dout v^T,  dS = P * (dP - delta),  dQ = scale * dS k,  dK = scale * dS^T q
 //
-// Two kernels, launched in this order, no atomics (so every run is deterministic):
-//   bwd_main<DQ=true>   one workgroup per 256 query rows of one head (eight wavefronts, two per SIMD: this pass
-//                has half the accumulators of the other and fits 256 registers): Q and dout rows stay in
-//                registers, K / V tiles stream through LDS; accumulates dQ.  Its prologue also works out, per
-//                query row, delta = sum_d dout * out and lse2 = lse * log2(e) (with -inf, a row that saw no key,
-//                turned into +inf so that P = exp2(s - lse2) = 0 there) and leaves them in the workspace
-//   bwd_main<DQ=false>  one workgroup per 128 keys of one KV head: K and V rows stay in registers,
-//                Q / dout tiles of the (grouped) query heads stream through LDS together with their lse2 /
-//                delta from the workspace; accumulates dK, dV
-// Both instances share one body.  "Stationary" rows (32 per wavefront) sit in the lane index of every
+// Two passes, no atomics (so every run is deterministic):
+//   dQ       one workgroup per 256 (128) query rows of one head: Q and dout rows stay in registers, K / V tiles stream
+//            through LDS; accumulates dQ
+//   dK / dV  one workgroup per 128 keys of one KV head: K and V rows stay in registers, Q / dout tiles of the (grouped)
+//            query heads stream through LDS together with their lse2 / delta from the workspace; accumulates dK, dV
+// Per query row, delta = sum_d dout * out and lse2 = lse * log2(e) (with -inf, a row that saw no key, turned into +inf so
+// that P = exp2(s - lse2) = 0 there) are worked out once and left in the workspace.
+// Launches that fill the chip run the passes one after the other (bwd_main): dQ first, with eight wavefronts per
+// workgroup, two per SIMD (it has half the accumulators of the other and fits 256 registers), and its prologue does
+// delta and lse2.  Smaller ones run both passes side by side in one launch (bwd_joint) behind a small one for delta and
+// lse2 (bwd_prepare).
+// All of them share one body (bwd_pass).  "Stationary" rows (32 per wavefront) sit in the lane index of every
 // MFMA accumulator, "streamed" rows in its registers, exactly as in the forward kernel:
 //     T1[c][r] = X_str[c] . X_st[r]      (scores)          T2[c][r] = Y_str[c] . Y_st[r]      (dP)
 //     acc^T[d][r] += X_str^T[d][c] dS[c][r]                (dQ or dK)
@@ -24,6 +26,8 @@
 // of the second MFMAs are gathered from the same tiles with ds_read_b64_tr_b16, in the key order the
 // accumulator registers hold.
 #include "mhip_common.hpp"
+
+#include <math.h>
 
 #include <atomic>
 
@@ -58,55 +62,65 @@ struct BwdParams {
   int D;            // head dimension of the tensors, a multiple of 8 up to kD; columns D .. kD-1 are zeros on chip
   int64_t q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, dk_sb, dk_ss, dk_sh, dq_sb, dq_ss, dq_sh, o_sb, o_ss, o_sh;
   float scale, scale_log2;
-  int n_tiles;      // stationary tiles per (batch, head)
+};
+
+// The workgroups of a pass: one per stationary tile of a (batch, head).
+struct TileMap {
+  int n_tiles;         // stationary tiles per (batch, head)
   int total;
-  int per_xcd;
+  int per_xcd;         // ceil(total / 8); the pass takes 8 * per_xcd workgroups
   int heads_per_xcd;   // (batch, stationary head) pairs per XCD when they divide evenly, else 0
 };
 
 // KK = k-steps of 16 head-dim values in T1 / T2: 8 computes on all 128 on-chip columns; 4 is the instantiation for head
 // dimensions up to 64, which leaves out the MFMAs, accumulators and fragments of the zero columns.  The vector work of a
 // tile is the same, so a T1 / T2 slot carries twice of it: 4096 x 4096, H32, D 64 takes 473 us instead of 654.
-template <bool DQ, bool CAUSAL, int KK>
-__global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p) {
+//
+// WAVES = 8 wavefronts of 32 stationary rows (dQ: two per SIMD) or 4 (one per SIMD).  PREPARED: lse2 and delta of the
+// query rows are in the workspace already; otherwise the dQ pass works them out.
+template <bool DQ, int WAVES>
+constexpr int kStageBytesOf = DQ ? 2 * kTileBytes : kOffDelta + kTile * 4;
+template <bool DQ, int WAVES>
+constexpr int kSmemBytesOf = WAVES == 8 ? 3 * kStageBytesOf<DQ, WAVES> + WAVES * 32 * kD * 2 : kStages * kStageBytesOf<DQ, WAVES>;
+
+template <bool DQ, bool CAUSAL, int KK, int WAVES, bool PREPARED>
+__device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, const int block, unsigned char* smem) {
+  static_assert(DQ || WAVES == 4, "the dK / dV pass has no room for two wavefronts per SIMD");
+  static_assert(PREPARED || WAVES == 8, "the pass that prepares is the one with a launch of its own");
   constexpr int DB = KK / 2;                    // blocks of 32 head-dim values in the accumulators
-  // The dQ pass needs half the accumulators of the dK / dV pass and fits two wavefronts per SIMD: its workgroup
-  // is eight wavefronts sharing the streamed K / V tiles.
-  constexpr int kWavesWg = DQ ? 8 : 4;
+  constexpr int kWavesWg = WAVES;
   constexpr int kRowsPerWg = kWavesWg * 32;
   constexpr int kCpy = 16 / kWavesWg;           // copy instructions per wavefront for one 16 KB tile
   constexpr int kRowsBytes = kRowsPerWg * kD * 2;       // one tensor's stationary rows
   // X tile, Y tile, and in the dK / dV pass lse2 and delta of the streamed rows
-  constexpr int kStageBytes = DQ ? 2 * kTileBytes : kOffDelta + kTile * 4;
-  // The stationary rows pass through LDS on their way into registers: the dQ pass has room for its Q rows in the last
-  // stage and 32 KB behind it and for dout in the two stages before that, the dK / dV pass for K and V in one each.
-  constexpr int kXRows = 3 * kStageBytes, kYRows = DQ ? kStageBytes : 2 * kStageBytes;
-  constexpr int kSmemBytes = DQ ? kXRows + kRowsBytes : kStages * kStageBytes;      // 163840 / 133120
-  static_assert(kYRows + kRowsBytes <= kXRows, "the rows' places do not overlap");
-  __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytes];
+  constexpr int kStageBytes = kStageBytesOf<DQ, WAVES>;
+  // The stationary rows pass through LDS on their way into registers, in one stage each; with eight wavefronts X takes
+  // the last stage and 32 KB behind it and Y the two stages before.
+  constexpr int kXRows = 3 * kStageBytes, kYRows = WAVES == 8 ? kStageBytes : 2 * kStageBytes;
+  static_assert(kYRows + kRowsBytes <= kXRows && kXRows + kRowsBytes <= kSmemBytesOf<DQ, WAVES>, "the rows' places");
 
   // Workgroup i runs on XCD i % 8: every XCD gets a contiguous range of (batch, head) pairs.  Under the
   // causal mask the work of a stationary tile grows (query tiles) or shrinks (key tiles) with its index:
   // such launches run the longest tiles first, across all heads.
   int st_tile, bh;
   if (!CAUSAL) {
-    const int logical = (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);
-    if (logical >= p.total) return;
-    st_tile = logical % p.n_tiles;
-    bh = logical / p.n_tiles;
+    const int logical = (block & 7) * w.per_xcd + (block >> 3);
+    if (logical >= w.total) return;
+    st_tile = logical % w.n_tiles;
+    bh = logical / w.n_tiles;
   } else {
     int rank;                                       // position in longest-first order
-    if (p.heads_per_xcd > 0) {
-      const int local = blockIdx.x >> 3;
-      rank = local / p.heads_per_xcd;
-      bh = (blockIdx.x & 7) * p.heads_per_xcd + local % p.heads_per_xcd;
+    if (w.heads_per_xcd > 0) {
+      const int local = block >> 3;
+      rank = local / w.heads_per_xcd;
+      bh = (block & 7) * w.heads_per_xcd + local % w.heads_per_xcd;
     } else {
-      if ((int)blockIdx.x >= p.total) return;
-      const int nbh = p.total / p.n_tiles;
-      rank = (int)blockIdx.x / nbh;
-      bh = (int)blockIdx.x % nbh;
+      if (block >= w.total) return;
+      const int nbh = w.total / w.n_tiles;
+      rank = block / nbh;
+      bh = block % nbh;
     }
-    st_tile = DQ ? p.n_tiles - 1 - rank : rank;
+    st_tile = DQ ? w.n_tiles - 1 - rank : rank;
   }
   const int hs = DQ ? bh % p.Hq : bh % p.Hkv;       // stationary head: a q head (DQ) or a kv head
   const int b = DQ ? bh / p.Hq : bh / p.Hkv;
@@ -266,8 +280,8 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
   // wavefront and nobody reads tile t-1 any more, whose stage then receives tile t+3.  Tiles past the end
   // are copied as zeros (and their T1 / T2 computed, unused) so that the number of copies in flight
   // stays the same.
-  // operand reads in flight ahead of the MFMAs (2, 4 and 8 measure the same; 2 keeps the dQ pass inside 256 registers)
-  constexpr int kDepth = DQ ? 2 : 4;
+  // operand reads in flight ahead of the MFMAs (2, 4 and 8 measure the same; 2 keeps eight wavefronts inside 256 registers)
+  constexpr int kDepth = WAVES == 8 ? 2 : 4;
   constexpr int kT = 2 * KK;                               // slots of a T1 / T2 phase
   constexpr int kAcc = DQ ? 2 * DB : 4 * DB;               // slots of an accumulate phase
   constexpr int kP1 = kT, kP2 = kT + kAcc, kP3 = 2 * kT + kAcc, kSlots = 2 * (kT + kAcc);
@@ -441,7 +455,7 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
         else { asm volatile("" : "+a"(xf[ks])); asm volatile("" : "+a"(yf[ks])); }
       }
     };
-    if (DQ) {
+    if (!PREPARED) {
       // This pass runs first and prepares what both passes need per query row: delta = rowsum(dout * out), kept
       // negated (the dP products start from it), and lse2 = lse * log2(e) with -inf (a row that saw no key) turned
       // into +inf so that P = exp2(s - lse2) = 0 there.
@@ -487,6 +501,12 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
       __builtin_amdgcn_s_barrier();                  // the rows' places are stages 1 .. 3 from here on
       if (ntiles > 0) { copy_tile(1, 1); copy_tile(2, 2); }
     } else if (ntiles > 0) {
+      if (DQ) {
+        const int64_t r = ((int64_t)b * p.Hq + hs) * p.Sq + (my_r < n_st ? my_r : n_st - 1);
+        lse2_lane = p.lse2[r];
+        delta_lane = p.delta[r];
+        asm volatile("" : "+v"(lse2_lane), "+v"(delta_lane));
+      }
       copy_tile(0, 0);
       copy_rows(xsrc, x_lds);
       copy_rows(ysrc, y_lds);
@@ -681,6 +701,45 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p)
   }
 }
 
+template <bool DQ, bool CAUSAL, int KK>
+__global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p, const TileMap w) {
+  constexpr int kWaves = DQ ? 8 : 4;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<DQ, kWaves>];
+  bwd_pass<DQ, CAUSAL, KK, kWaves, !DQ>(p, w, (int)blockIdx.x, smem);
+}
+
+// Both passes side by side, for launches that leave CUs idle one after the other.
+template <bool CAUSAL, int KK>
+__global__ __launch_bounds__(256, 1) void bwd_joint(const BwdParams p, const TileMap wq, const TileMap wk) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<false, 4>];
+  static_assert(kSmemBytesOf<true, 4> <= kSmemBytesOf<false, 4>, "one array for both");
+  const int first_q = wk.per_xcd * 8;         // a multiple of 8: both halves keep their XCDs
+  if ((int)blockIdx.x < first_q) bwd_pass<false, CAUSAL, KK, 4, true>(p, wk, (int)blockIdx.x, smem);
+  else bwd_pass<true, CAUSAL, KK, 4, true>(p, wq, (int)blockIdx.x - first_q, smem);
+}
+
+// lse2 and delta for bwd_joint: 16 lanes per query row.
+__global__ __launch_bounds__(256) void bwd_prepare(const BwdParams p, int rows) {
+  const int i = blockIdx.x * 16 + (threadIdx.x >> 4), col = (threadIdx.x & 15) * 8;
+  const int at = i < rows ? i : rows - 1;
+  const int h = at % p.Hq, bs = at / p.Hq, srow = bs % p.Sq, b = bs / p.Sq;
+  float part = 0.f;
+  if (col < p.D) {
+    const bf16x8 d8 = *reinterpret_cast<const bf16x8*>(p.dout + b * p.q_sb + (int64_t)srow * p.q_ss + h * p.q_sh + col);
+    const bf16x8 o8 = *reinterpret_cast<const bf16x8*>(p.out + b * p.o_sb + (int64_t)srow * p.o_ss + h * p.o_sh + col);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) part = __builtin_fmaf((float)d8[j], (float)o8[j], part);
+  }
+  const float delta = row16_sum(part);
+  if (i < rows && col == 0) {
+    const int64_t r = ((int64_t)b * p.Hq + h) * p.Sq + srow;
+    const float l = p.lse[r];
+    p.lse2[r] = (l == -INFINITY) ? INFINITY : l * kLog2e;
+    p.delta[r] = -delta;
+    if (p.softmax_d) p.softmax_d[r] = delta;
+  }
+}
+
 }  // namespace
 }  // namespace mhip
 
@@ -721,16 +780,65 @@ int scratch_address(void** ptr) {
   return MHIP_OK;
 }
 
-template <bool DQ, int KK>
-void launch_pass_kk(const BwdParams& p, bool causal, hipStream_t st) {
-  const dim3 grid(p.per_xcd * 8), block(DQ ? 512 : 256);
-  if (causal) hipLaunchKernelGGL((bwd_main<DQ, true, KK>), grid, block, 0, st, p);
-  else hipLaunchKernelGGL((bwd_main<DQ, false, KK>), grid, block, 0, st, p);
+TileMap tile_map(int heads, int seq, int rows) {
+  TileMap w;
+  w.n_tiles = (seq + rows - 1) / rows;
+  w.total = heads * w.n_tiles;
+  w.per_xcd = (w.total + 7) / 8;
+  w.heads_per_xcd = heads % 8 == 0 ? heads / 8 : 0;
+  return w;
 }
-template <bool DQ>
-void launch_pass(const BwdParams& p, bool causal, hipStream_t st) {
-  if (p.D <= 64) launch_pass_kk<DQ, 4>(p, causal, st);
-  else launch_pass_kk<DQ, 8>(p, causal, st);
+
+template <bool CAUSAL, int KK>
+void launch_bwd(const BwdParams& p, bool joint, hipStream_t st) {
+  const TileMap wk = tile_map(p.B * p.Hkv, p.Sc, kRowsKv);
+  if (joint) {
+    const int rows = p.B * p.Hq * p.Sq;
+    hipLaunchKernelGGL(bwd_prepare, dim3((rows + 15) / 16), dim3(256), 0, st, p, rows);
+    const TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ / 2);
+    hipLaunchKernelGGL((bwd_joint<CAUSAL, KK>), dim3((wk.per_xcd + wq.per_xcd) * 8), dim3(256), 0, st, p, wq, wk);
+    return;
+  }
+  if (p.Sq > 0) {
+    // dQ (and delta / lse2 for both passes): one workgroup per 256 query rows; has to run before the dK / dV pass
+    const TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ);
+    hipLaunchKernelGGL((bwd_main<true, CAUSAL, KK>), dim3(wq.per_xcd * 8), dim3(512), 0, st, p, wq);
+  }
+  // dK, dV: one workgroup per 128 keys of one kv head
+  if (p.Sc > 0) hipLaunchKernelGGL((bwd_main<false, CAUSAL, KK>), dim3(wk.per_xcd * 8), dim3(256), 0, st, p, wk);
+}
+
+// Estimated time (us) of n workgroups that visit `most` tiles at most and `mean` on average, one workgroup per CU at a
+// time: `fixed` per workgroup and `step` per tile, plus `busy` times the share of the CUs at work (clock and L2).
+struct Cost { float fixed, step, busy; };
+float launch_time(float n, float mean, float most, const Cost& c) {
+  const float full = floorf(n / 256.f), part = n / 256.f - full;
+  const float share = n < 256.f ? part : 1.f;
+  const float longest = c.fixed + most * (c.step + share * c.busy);
+  float spread = full * (c.fixed + mean * (c.step + c.busy));
+  if (part > 0.f) spread += c.fixed + mean * (c.step + part * c.busy);
+  return longest > spread ? longest : spread;
+}
+
+// Whether both passes go into one launch, behind a small one that prepares delta and lse2: faster while one pass alone
+// leaves CUs idle (its dQ wavefronts run one per SIMD instead of two, which costs 4 % once the chip is full).  Costs fitted
+// to the measured block times, us (two launches / one):
+//     B1 H4   256 x 256     23.0 / 12.3      B4 H5    512 x 512    35.1 / 19.7      B1 H2 4096 x 4096   183 / 89.8
+//     B1 H32 1024 x 1024    70.6 / 64.1      B1 H16 2048 x 2048     122 /  109      B1 H32 2048 x 2048  205 / 214
+//     B1 H32 4096 x 4096     756 /  786      causal: B1 H8 2048 x 2048  103 / 52.3, B1 H32 4096 x 4096  424 / 439
+bool side_by_side(const BwdParams& p, bool causal) {
+  const bool narrow = p.D <= 64;
+  const Cost dq8 = narrow ? Cost{6.f, 0.95f, 0.45f} : Cost{7.f, 1.45f, 0.75f};
+  const Cost dkv = narrow ? Cost{6.f, 0.75f, 0.25f} : Cost{7.f, 1.15f, 0.55f};
+  const Cost both = narrow ? Cost{6.f, 0.75f, 0.12f} : Cost{7.f, 1.15f, 0.29f};
+  constexpr float kPrepare = 5.f;
+  const float tq = (float)((p.Sc + kTile - 1) / kTile), tk = (float)((p.Sq + kTile - 1) / kTile) * p.group;
+  const float half = causal ? 0.53f : 1.f;          // mean share of the tiles under the diagonal
+  const float nq8 = (float)tile_map(p.B * p.Hq, p.Sq, kRowsQ).total, nq4 = (float)tile_map(p.B * p.Hq, p.Sq, kRowsQ / 2).total;
+  const float nk = (float)tile_map(p.B * p.Hkv, p.Sc, kRowsKv).total;
+  const float two = launch_time(nq8, half * tq, tq, dq8) + launch_time(nk, half * tk, tk, dkv);
+  const float n = nq4 + nk, mean = half * (nq4 * tq + nk * tk) / n;
+  return kPrepare + launch_time(n, mean, tq > tk ? tq : tk, both) < two;
 }
 
 // own_scratch: take the workspace from `scratch` (resolved after the arguments have been checked)
@@ -795,22 +903,9 @@ int bwd_block(const void* dout, const void* q, const void* k, const void* v,
   p.scale = softmax_scale; p.scale_log2 = softmax_scale * kLog2e;
   const bool causal = mask == MHIP_MASK_CAUSAL;
 
-  if (Sq > 0) {
-    // dQ (and delta / lse2 for both passes): one workgroup per 256 query rows; has to run before the dK / dV pass
-    p.n_tiles = (Sq + kRowsQ - 1) / kRowsQ;
-    p.total = B * Hq * p.n_tiles;
-    p.per_xcd = (p.total + 7) / 8;
-    p.heads_per_xcd = (B * Hq) % 8 == 0 ? (B * Hq) / 8 : 0;
-    launch_pass<true>(p, causal, st);
-  }
-  if (Sc > 0) {
-    // dK, dV: one workgroup per 128 keys of one kv head
-    p.n_tiles = (Sc + kRowsKv - 1) / kRowsKv;
-    p.total = B * Hkv * p.n_tiles;
-    p.per_xcd = (p.total + 7) / 8;
-    p.heads_per_xcd = (B * Hkv) % 8 == 0 ? (B * Hkv) / 8 : 0;
-    launch_pass<false>(p, causal, st);
-  }
+  const bool joint = Sq > 0 && Sc > 0 && side_by_side(p, causal);
+  if (D <= 64) causal ? launch_bwd<true, 4>(p, joint, st) : launch_bwd<false, 4>(p, joint, st);
+  else causal ? launch_bwd<true, 8>(p, joint, st) : launch_bwd<false, 8>(p, joint, st);
   return launch_status();
 }
 }  // namespace

@@ -49,18 +49,13 @@ def test_backward_step_carries_the_sums(W, S, Hq, Hkv, D, dq_dtype, keep):
         _close(f"dkv {c}", got[c], torch.stack(tuple(rdkv[c])))
 
 
-@pytest.mark.parametrize("D", [8, 56, 64, 72])
-@pytest.mark.parametrize("Sq,Sc,Hq,Hkv,causal", [(1, 1, 2, 1, False), (65, 129, 4, 2, False), (257, 63, 2, 2, True),
-                                                 (320, 400, 3, 3, True), (130, 700, 2, 1, False)])
-def test_backward_block_on_narrow_heads(D, Sq, Sc, Hq, Hkv, causal):
-    """Both sides of the line between the 64-column and the 128-column kernels, ragged rows and keys, several turns of
-    the tile ring."""
+def _block(B, Sq, Sc, Hq, Hkv, D, causal):
     import mercury_artifact_amd as M
 
-    print(f"D{D} Sq{Sq} Sc{Sc} Hq{Hq} Hkv{Hkv} causal={causal}", flush=True)
+    print(f"B{B} D{D} Sq{Sq} Sc{Sc} Hq{Hq} Hkv{Hkv} causal={causal}", flush=True)
     g = torch.Generator().manual_seed(D * 1000 + Sq)
-    q, dout = (torch.randn(2, Sq, Hq, D, generator=g).bfloat16() for _ in range(2))
-    kv = torch.randn(2, 2, Sc, Hkv, D, generator=g).bfloat16()
+    q, dout = (torch.randn(B, Sq, Hq, D, generator=g).bfloat16() for _ in range(2))
+    kv = torch.randn(2, B, Sc, Hkv, D, generator=g).bfloat16()
     scale = D ** -0.5
     o, lse = O.block_attention(q.float(), kv[0].float(), kv[1].float(), scale, causal=causal)
     refs = O.block_backward(dout.float(), q.float(), kv[0].float(), kv[1].float(), o.bfloat16().float(), lse, scale, causal=causal)
@@ -73,3 +68,19 @@ def test_backward_block_on_narrow_heads(D, Sq, Sc, Hq, Hkv, causal):
         _close(name, got, ref)
     want = (dout.float() * o.bfloat16().float()).sum(-1).transpose(1, 2)
     assert (delta.cpu() - want).abs().max() <= 1e-4
+
+
+@pytest.mark.parametrize("D", [8, 56, 64, 72])
+@pytest.mark.parametrize("Sq,Sc,Hq,Hkv,causal", [(1, 1, 2, 1, False), (65, 129, 4, 2, False), (257, 63, 2, 2, True),
+                                                 (320, 400, 3, 3, True), (130, 700, 2, 1, False)])
+def test_backward_block_on_narrow_heads(D, Sq, Sc, Hq, Hkv, causal):
+    """Both sides of the line between the 64-column and the 128-column kernels, ragged rows and keys, several turns of
+    the tile ring; launches this small run both passes side by side."""
+    _block(2, Sq, Sc, Hq, Hkv, D, causal)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Sq,Sc,causal", [(130, 129, False), (257, 64, True), (300, 385, True)])
+def test_backward_block_in_two_launches(D, Sq, Sc, causal):
+    """Enough heads to fill the chip with either pass: one launch each, dQ with eight wavefronts."""
+    _block(2, Sq, Sc, 128, 128, D, causal)
