@@ -237,14 +237,20 @@ def _store_packed(buf, o, lse, fused: bool):
 
 def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=False,
                              window_size=(-1, -1), alibi_slopes=None, deterministic=False, *,
-                             ring: LocalRing, fused_epilogue: bool = True):
-    """Managed-reduction form (template utils/flash_attn_dsl.py:345-408) with the KV ring: block
-    results are packed ``(out | lse)`` and folded by ``flash_reduce``; pack and reduce run as one
-    kernel."""
+                             ring: LocalRing, fused_epilogue: bool = True, deferred_merge: bool = True):
+    """Managed-reduction form (template utils/flash_attn_dsl.py:345-408) with the KV ring: the reduction buffer
+    ``(out | lse)`` stays on the rank, so with ``deferred_merge`` the bf16 block results are kept and folded by ONE
+    ``merge_many`` call after the last chunk, straight into ``o`` and ``lse`` (results agree with the packed chain to fp32
+    rounding).  Otherwise -- and with ``fused_epilogue=False``, the literal stores -- block results are packed and folded
+    by ``flash_reduce`` chunk by chunk; pack and reduce run as one kernel."""
     buf = None
     _kv = None
     _next_kv = None
-    for step, hop in enumerate(_hops(ring)):
+    hops = _hops(ring)
+    blocks = []
+    defer = (fused_epilogue and deferred_merge and len(hops) <= MAX_MERGE_MANY and o.dtype == torch.bfloat16
+             and o.is_contiguous() and lse.is_contiguous())
+    for step, hop in enumerate(hops):
         if step == 0:
             _kv = kv.contiguous()
         else:
@@ -258,7 +264,13 @@ def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=F
         outputs = _block_forward(q, _k, _v, softmax_scale, dropout_p, causal, window_size, alibi_slopes)
         assert len(outputs) == 4
         block_out, block_lse, _, _ = outputs
-        buf = pack_block(block_out, block_lse, reduce_into=buf)
+        if defer:
+            blocks.append((block_out, block_lse))
+        else:
+            buf = pack_block(block_out, block_lse, reduce_into=buf)
+    if defer:
+        merge_many([b[0] for b in blocks], [b[1] for b in blocks], o, lse)
+        return
     _store_packed(buf, o, lse, fused_epilogue)
 
 
