@@ -113,7 +113,7 @@ int mhip_attn_bwd_block(const void* dout, const void* q, const void* k, const vo
  * mhip_attn_bwd_block without the workspace argument.  No counterpart in the reference: it is for callers
  * that cannot hand over (or allocate) scratch memory -- code under HIP graph capture, serving loops and
  * harnesses that forbid hipMalloc.  delta and lse2 go to an array built into the library (a file-scope
- * __device__ array of 8 MiB + 32 bytes, held by every GPU the library runs on until the process ends), so
+ * __device__ array of 40 MiB + 32 bytes, held by every GPU the library runs on until the process ends), so
  * the block is limited to B * Hq * Sq <= 1048576 (MHIP_ETOOLARGE beyond).  The first call on a device asks
  * the runtime for that device's address of the array (hipGetSymbolAddress, MHIP_ERUNTIME if that fails), which
  * is a runtime query and must not happen while the stream is being captured: call mhip_init() on the device

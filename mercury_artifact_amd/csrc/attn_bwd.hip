@@ -66,7 +66,9 @@ struct BwdParams {
 
 // The workgroups of a pass: one per stationary tile of a (batch, head).
 struct TileMap {
-  int n_tiles;         // stationary tiles per (batch, head)
+  int splits;          // workgroups that share a stationary tile, each with its part of the streamed tiles
+  float* partial;      // with splits > 1: their sums, [split] x the layout of dQ, or of dK and behind all of it dV, fp32
+  int n_tiles;         // stationary tiles per (batch, head), times splits
   int total;
   int per_xcd;         // ceil(total / 8); the pass takes 8 * per_xcd workgroups
   int heads_per_xcd;   // (batch, stationary head) pairs per XCD when they divide evenly, else 0
@@ -83,7 +85,8 @@ constexpr int kStageBytesOf = DQ ? 2 * kTileBytes : kOffDelta + kTile * 4;
 template <bool DQ, int WAVES>
 constexpr int kSmemBytesOf = WAVES == 8 ? 3 * kStageBytesOf<DQ, WAVES> + WAVES * 32 * kD * 2 : kStages * kStageBytesOf<DQ, WAVES>;
 
-template <bool DQ, bool CAUSAL, int KK, int WAVES, bool PREPARED>
+// SPLIT: the workgroups of the pass may share their stationary tile (w.splits).
+template <bool DQ, bool CAUSAL, int KK, int WAVES, bool PREPARED, bool SPLIT>
 __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, const int block, unsigned char* smem) {
   static_assert(DQ || WAVES == 4, "the dK / dV pass has no room for two wavefronts per SIMD");
   static_assert(PREPARED || WAVES == 8, "the pass that prepares is the one with a launch of its own");
@@ -102,11 +105,12 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   // Workgroup i runs on XCD i % 8: every XCD gets a contiguous range of (batch, head) pairs.  Under the
   // causal mask the work of a stationary tile grows (query tiles) or shrinks (key tiles) with its index:
   // such launches run the longest tiles first, across all heads.
-  int st_tile, bh;
+  int st_tile, bh, split;
   if (!CAUSAL) {
     const int logical = (block & 7) * w.per_xcd + (block >> 3);
     if (logical >= w.total) return;
-    st_tile = logical % w.n_tiles;
+    st_tile = SPLIT ? logical % w.n_tiles / w.splits : logical % w.n_tiles;
+    split = SPLIT ? logical % w.n_tiles % w.splits : 0;
     bh = logical / w.n_tiles;
   } else {
     int rank;                                       // position in longest-first order
@@ -120,7 +124,9 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
       rank = block / nbh;
       bh = block % nbh;
     }
-    st_tile = DQ ? w.n_tiles - 1 - rank : rank;
+    split = SPLIT ? rank % w.splits : 0;
+    if (SPLIT) rank /= w.splits;
+    st_tile = DQ ? (SPLIT ? w.n_tiles / w.splits : w.n_tiles) - 1 - rank : rank;
   }
   const int hs = DQ ? bh % p.Hq : bh % p.Hkv;       // stationary head: a q head (DQ) or a kv head
   const int b = DQ ? bh / p.Hq : bh / p.Hkv;
@@ -159,7 +165,13 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     }
   }
   const int span = tiles_per_head - first_tile;
-  const int ntiles = span * heads_str;
+  // this workgroup's part of the stream: tiles t0 .. t0 + ntiles - 1 of the pass's sequence
+  int t0 = 0, ntiles = span * heads_str;
+  if (SPLIT && w.splits > 1) {
+    const int all = ntiles, part = (all + w.splits - 1) / w.splits;
+    t0 = split * part < all ? split * part : all;
+    ntiles = all - t0 < part ? all - t0 : part;
+  }
 
   const uint16_t* xbase; const uint16_t* ybase; int64_t s_ss, s_sh; uint32_t s_bytes;
   if (DQ) {
@@ -176,8 +188,8 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   const u32x4 yrs = rsrc_words(ybase, s_bytes);
 
   // tile index -> (head of the group, first streamed row)
-  auto tile_head = [&](int t) { return DQ ? 0 : t / span; };
-  auto tile_row0 = [&](int t) { return (first_tile + (DQ ? t : t % span)) * kTile; };
+  auto tile_head = [&](int t) { return DQ ? 0 : (t0 + t) / span; };
+  auto tile_row0 = [&](int t) { return (first_tile + (DQ ? t0 + t : (t0 + t) % span)) * kTile; };
 
   // Wavefront w copies rows 16w .. 16w+15 of the X and the Y tile: four instructions of 1 KB each; lane l
   // of instruction u lands at row 16w + 4u + l/16, chunk position l%16, and fetches the chunk that lives
@@ -218,17 +230,18 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   // head of the group) instead of a division per tile: every scalar instruction of the loop takes an issue slot of
   // the one wavefront a SIMD runs in the dK / dV pass.
   int cp_soff = 0, cp_ld_soff = 0;
-  int nx_r = DQ ? 3 : (span > 0 ? 3 % span : 0), nx_h = DQ ? 0 : (span > 0 ? 3 / span : 0);
+  int nx_r = DQ ? t0 + 3 : (span > 0 ? (t0 + 3) % span : 0), nx_h = DQ ? 0 : (span > 0 ? (t0 + 3) / span : 0), nx_t = 3;
   const uint32_t ld_rows = (uint32_t)p.B * (uint32_t)p.Hq * (uint32_t)p.Sq;     // the host keeps this below 2^30
   const u32x4 ldrs = rsrc_words((wave & 1) ? p.delta : p.lse2, ld_rows * 4u);
   auto copy_setup = [&]() {
-    const bool live = DQ ? nx_r < span : nx_h < heads_str;
+    const bool live = SPLIT ? nx_t < ntiles : DQ ? nx_r < span : nx_h < heads_str;
     const uint32_t hq = DQ ? 0u : (uint32_t)(hs * p.group + (live ? nx_h : 0));
     const uint32_t c0 = (uint32_t)((first_tile + (live ? nx_r : 0)) * kTile);
     // element offsets stay below 2^31 (checked by the host), so 32-bit arithmetic is exact
     cp_soff = live ? (int)((c0 * (uint32_t)s_ss + hq * (uint32_t)s_sh) * 2u) : kNoTile;
     if (!DQ) cp_ld_soff = live ? (int)((((uint32_t)b * (uint32_t)p.Hq + hq) * (uint32_t)p.Sq + c0) * 4u) : kNoTile;
     ++nx_r;
+    if (SPLIT) ++nx_t;
     if (!DQ && nx_r == span) { nx_r = 0; ++nx_h; }
   };
   auto copy_piece = [&](int piece, int stage) {
@@ -543,10 +556,10 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
       for (int g = 0; g < 4; ++g) read_nd(false, 1, g);        // for T2 of the second half, first thing in the loop
     }
   }
-  int cur_r = 0;                                         // t % span
+  int cur_r = !DQ && span > 0 ? t0 % span : t0;          // (t0 + t) % span
   for (int t = 0; t < ntiles; ++t) {
     const int c0 = (first_tile + cur_r) * kTile;
-    if (++cur_r == span) cur_r = 0;                      // (t + 1) % span
+    if (++cur_r == span) cur_r = 0;
     asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kCopiesPerTile) : "memory");          // one tile of copies stays in flight
     __builtin_amdgcn_s_barrier();
     copy_setup();
@@ -669,7 +682,19 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   auto pack8 = [](const f32x4 (&v)[2]) {
     return u32x4{pack_bf16(v[0][0], v[0][1]), pack_bf16(v[0][2], v[0][3]), pack_bf16(v[1][0], v[1][1]), pack_bf16(v[1][2], v[1][3])};
   };
-  if (DQ) {
+  if (SPLIT && w.splits > 1) {
+    // fp32 sums for bwd_reduce, (b, row, head, column) like the gradient itself
+    const int64_t size = (int64_t)p.B * n_st * (DQ ? p.Hq : p.Hkv) * p.D;
+    auto part = [&](float* base) {
+      return [=](f32x4 (&v)[2], int row, int col) {
+        f32x4* op = reinterpret_cast<f32x4*>(base + split * size + (((int64_t)b * n_st + row) * (DQ ? p.Hq : p.Hkv) + hs) * p.D + col);
+        op[0] = v[0];
+        op[1] = v[1];
+      };
+    };
+    write_out32(acc1, p.scale, part(w.partial));
+    if (!DQ) write_out32(acc2, 1.f, part(w.partial + w.splits * size));
+  } else if (DQ) {
     if (p.dq_acc == nullptr) {
       write_out(acc1, p.scale, p.dq, p.dq_sb, p.dq_ss, p.dq_sh, hs);
     } else {
@@ -705,17 +730,17 @@ template <bool DQ, bool CAUSAL, int KK>
 __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p, const TileMap w) {
   constexpr int kWaves = DQ ? 8 : 4;
   __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<DQ, kWaves>];
-  bwd_pass<DQ, CAUSAL, KK, kWaves, !DQ>(p, w, (int)blockIdx.x, smem);
+  bwd_pass<DQ, CAUSAL, KK, kWaves, !DQ, false>(p, w, (int)blockIdx.x, smem);
 }
 
 // Both passes side by side, for launches that leave CUs idle one after the other.
-template <bool CAUSAL, int KK>
+template <bool CAUSAL, int KK, bool SPLIT>
 __global__ __launch_bounds__(256, 1) void bwd_joint(const BwdParams p, const TileMap wq, const TileMap wk) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<false, 4>];
   static_assert(kSmemBytesOf<true, 4> <= kSmemBytesOf<false, 4>, "one array for both");
   const int first_q = wk.per_xcd * 8;         // a multiple of 8: both halves keep their XCDs
-  if ((int)blockIdx.x < first_q) bwd_pass<false, CAUSAL, KK, 4, true>(p, wk, (int)blockIdx.x, smem);
-  else bwd_pass<true, CAUSAL, KK, 4, true>(p, wq, (int)blockIdx.x - first_q, smem);
+  if ((int)blockIdx.x < first_q) bwd_pass<false, CAUSAL, KK, 4, true, SPLIT>(p, wk, (int)blockIdx.x, smem);
+  else bwd_pass<true, CAUSAL, KK, 4, true, SPLIT>(p, wq, (int)blockIdx.x - first_q, smem);
 }
 
 // lse2 and delta for bwd_joint: 16 lanes per query row.
@@ -740,22 +765,57 @@ __global__ __launch_bounds__(256) void bwd_prepare(const BwdParams p, int rows) 
   }
 }
 
+// The sums of the workgroups that shared a stationary tile, added in the order of their parts, and stored the way the
+// pass itself would have: 16 lanes per row, 8 columns each.  Rows of dQ first (if that pass was split), then of dK and dV.
+__global__ __launch_bounds__(256) void bwd_reduce(const BwdParams p, const TileMap wq, const TileMap wk, int q_rows, int kv_rows) {
+  int row = blockIdx.x * 16 + (threadIdx.x >> 4);
+  const int col = (threadIdx.x & 15) * 8;
+  if (row >= q_rows + 2 * kv_rows || col >= p.D) return;
+  const bool is_q = row < q_rows;
+  const bool is_v = row >= q_rows + kv_rows;
+  row -= is_q ? 0 : is_v ? q_rows + kv_rows : q_rows;
+  const int heads = is_q ? p.Hq : p.Hkv, seq = is_q ? p.Sq : p.Sc, splits = is_q ? wq.splits : wk.splits;
+  const int64_t size = (int64_t)p.B * seq * heads * p.D, at = (int64_t)row * p.D + col;
+  const float* src = (is_q ? wq.partial : wk.partial) + (is_v ? splits * size : 0) + at;
+  f32x4 v[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  for (int i = 0; i < splits; ++i) {
+    const f32x4* part = reinterpret_cast<const f32x4*>(src + i * size);
+    v[0] += part[0];
+    v[1] += part[1];
+  }
+  auto pack8 = [](const f32x4 (&x)[2]) {
+    return u32x4{pack_bf16(x[0][0], x[0][1]), pack_bf16(x[0][2], x[0][3]), pack_bf16(x[1][0], x[1][1]), pack_bf16(x[1][2], x[1][3])};
+  };
+  const int h = row % heads, srow = row / heads % seq, b = row / heads / seq;
+  if (is_q) {
+    u32x4* qp = reinterpret_cast<u32x4*>(p.dq + b * p.dq_sb + (int64_t)srow * p.dq_ss + h * p.dq_sh + col);
+    if (p.dq_acc == nullptr || (p.dq_mode == kDqAdd && p.dq)) *qp = pack8(v);
+    if (p.dq_acc == nullptr) return;
+    f32x4* ap = reinterpret_cast<f32x4*>(p.dq_acc + at);
+    if (p.dq_mode != kDqFirst) { v[0] += ap[0]; v[1] += ap[1]; }
+    if (p.dq_mode != kDqLast) { ap[0] = v[0]; ap[1] = v[1]; }
+    else *qp = pack8(v);
+  } else {
+    const u32x4 x = pack8(v);
+    if (p.dk32) {
+      f32x4* op = reinterpret_cast<f32x4*>((is_v ? p.dv32 : p.dk32) + at);
+      op[0] = f32x4{bf16_lo(x[0]), bf16_hi(x[0]), bf16_lo(x[1]), bf16_hi(x[1])};
+      op[1] = f32x4{bf16_lo(x[2]), bf16_hi(x[2]), bf16_lo(x[3]), bf16_hi(x[3])};
+    }
+    uint16_t* out16 = is_v ? p.dv : p.dk;
+    if (out16) *reinterpret_cast<u32x4*>(out16 + b * p.dk_sb + (int64_t)srow * p.dk_ss + h * p.dk_sh + col) = x;
+  }
+}
+
 }  // namespace
 }  // namespace mhip
 
 using namespace mhip;
 
-extern "C" int64_t mhip_attn_bwd_workspace_bytes(int B, int Sq, int Sc, int Hq, int Hkv, int D) {
-  (void)Sc; (void)Hkv; (void)D;
-  if (B < 0 || Sq < 0 || Hq < 0) return 0;
-  // -delta, lse2 and delta, (B, Hq, Sq) fp32 each, every one starting on a 16-byte boundary
-  return ((((int64_t)B * Hq * Sq + 3) & ~int64_t(3)) * 3) * 4;
-}
-
 // Scratch of the entry point that allocates nothing: delta and lse2 of up to kScratchRows (batch, head, row)
-// triples.  Every GPU the library runs on holds its own copy until the process ends.
+// triples, and the sums of split passes.  Every GPU the library runs on holds its own copy until the process ends.
 constexpr int64_t kScratchRows = int64_t(1) << 20;
-static __device__ __align__(256) unsigned char scratch[kScratchRows * 8 + 32];
+static __device__ __align__(256) unsigned char scratch[kScratchRows * 8 + 32 + (int64_t(32) << 20)];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -780,32 +840,15 @@ int scratch_address(void** ptr) {
   return MHIP_OK;
 }
 
-TileMap tile_map(int heads, int seq, int rows) {
+TileMap tile_map(int heads, int seq, int rows, int splits = 1, float* partial = nullptr) {
   TileMap w;
-  w.n_tiles = (seq + rows - 1) / rows;
+  w.splits = splits;
+  w.partial = partial;
+  w.n_tiles = (seq + rows - 1) / rows * splits;
   w.total = heads * w.n_tiles;
   w.per_xcd = (w.total + 7) / 8;
   w.heads_per_xcd = heads % 8 == 0 ? heads / 8 : 0;
   return w;
-}
-
-template <bool CAUSAL, int KK>
-void launch_bwd(const BwdParams& p, bool joint, hipStream_t st) {
-  const TileMap wk = tile_map(p.B * p.Hkv, p.Sc, kRowsKv);
-  if (joint) {
-    const int rows = p.B * p.Hq * p.Sq;
-    hipLaunchKernelGGL(bwd_prepare, dim3((rows + 15) / 16), dim3(256), 0, st, p, rows);
-    const TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ / 2);
-    hipLaunchKernelGGL((bwd_joint<CAUSAL, KK>), dim3((wk.per_xcd + wq.per_xcd) * 8), dim3(256), 0, st, p, wq, wk);
-    return;
-  }
-  if (p.Sq > 0) {
-    // dQ (and delta / lse2 for both passes): one workgroup per 256 query rows; has to run before the dK / dV pass
-    const TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ);
-    hipLaunchKernelGGL((bwd_main<true, CAUSAL, KK>), dim3(wq.per_xcd * 8), dim3(512), 0, st, p, wq);
-  }
-  // dK, dV: one workgroup per 128 keys of one kv head
-  if (p.Sc > 0) hipLaunchKernelGGL((bwd_main<false, CAUSAL, KK>), dim3(wk.per_xcd * 8), dim3(256), 0, st, p, wk);
 }
 
 // Estimated time (us) of n workgroups that visit `most` tiles at most and `mean` on average, one workgroup per CU at a
@@ -820,27 +863,90 @@ float launch_time(float n, float mean, float most, const Cost& c) {
   return longest > spread ? longest : spread;
 }
 
-// Whether both passes go into one launch, behind a small one that prepares delta and lse2: faster while one pass alone
-// leaves CUs idle (its dQ wavefronts run one per SIMD instead of two, which costs 4 % once the chip is full).  Costs fitted
-// to the measured block times, us (two launches / one):
+// How a block runs.  Both passes go into one launch (joint), behind a small one that prepares delta and lse2, while one
+// pass alone leaves CUs idle (its dQ wavefronts run one per SIMD instead of two, which costs 4 % once the chip is full).
+// Costs fitted to the measured block times, us (two launches / one):
 //     B1 H4   256 x 256     23.0 / 12.3      B4 H5    512 x 512    35.1 / 19.7      B1 H2 4096 x 4096   183 / 89.8
 //     B1 H32 1024 x 1024    70.6 / 64.1      B1 H16 2048 x 2048     122 /  109      B1 H32 2048 x 2048  205 / 214
 //     B1 H32 4096 x 4096     756 /  786      causal: B1 H8 2048 x 2048  103 / 52.3, B1 H32 4096 x 4096  424 / 439
-bool side_by_side(const BwdParams& p, bool causal) {
-  const bool narrow = p.D <= 64;
+// In one launch a stationary tile may further be shared by several workgroups (sq of the dQ pass, sk of the dK / dV pass),
+// where one workgroup's chain of tiles -- with grouped heads, all query heads of the group -- is what the launch waits for;
+// their sums meet in a third launch (one / with it):
+//     B1 H8/1 512 x 512      82.6 / 27.6     B1 H8/1 2048 x 2048    310 / 73.6     B1 H8/1 4096 x 4096   636 /  221
+//     B1 H2/2 4096 x 4096    85.2 / 69.8     B1 H32/4 2048 x 2048   338 /  220     causal, D 64: H8/1 2048 x 2048  249 / 49.5
+struct Plan { bool joint; int sq, sk; };
+constexpr int64_t kPartialMost = int64_t(32) << 20;     // bytes of sums a block may leave for bwd_reduce
+int64_t partial_bytes(int B, int S, int H, int D, int tensors, int splits) {
+  return splits > 1 ? (int64_t)B * S * H * D * 4 * tensors * splits : 0;
+}
+Plan plan_block(int B, int Sq, int Sc, int Hq, int Hkv, int D, bool causal) {
+  Plan best = {false, 1, 1};
+  if (Sq == 0 || Sc == 0 || B == 0) return best;
+  const bool narrow = D <= 64;
   const Cost dq8 = narrow ? Cost{6.f, 0.95f, 0.45f} : Cost{7.f, 1.45f, 0.75f};
   const Cost dkv = narrow ? Cost{6.f, 0.75f, 0.25f} : Cost{7.f, 1.15f, 0.55f};
   const Cost both = narrow ? Cost{6.f, 0.75f, 0.12f} : Cost{7.f, 1.15f, 0.29f};
-  constexpr float kPrepare = 5.f;
-  const float tq = (float)((p.Sc + kTile - 1) / kTile), tk = (float)((p.Sq + kTile - 1) / kTile) * p.group;
+  constexpr float kPrepare = 5.f, kReduce = 4.f, kBytesPerUs = 4e6f;
+  const float tq = (float)((Sc + kTile - 1) / kTile), tk = (float)((Sq + kTile - 1) / kTile) * (Hq / Hkv);
   const float half = causal ? 0.53f : 1.f;          // mean share of the tiles under the diagonal
-  const float nq8 = (float)tile_map(p.B * p.Hq, p.Sq, kRowsQ).total, nq4 = (float)tile_map(p.B * p.Hq, p.Sq, kRowsQ / 2).total;
-  const float nk = (float)tile_map(p.B * p.Hkv, p.Sc, kRowsKv).total;
-  const float two = launch_time(nq8, half * tq, tq, dq8) + launch_time(nk, half * tk, tk, dkv);
-  const float n = nq4 + nk, mean = half * (nq4 * tq + nk * tk) / n;
-  return kPrepare + launch_time(n, mean, tq > tk ? tq : tk, both) < two;
+  const float nq8 = (float)tile_map(B * Hq, Sq, kRowsQ).total, nq4 = (float)tile_map(B * Hq, Sq, kRowsQ / 2).total;
+  const float nk = (float)tile_map(B * Hkv, Sc, kRowsKv).total;
+  float best_time = launch_time(nq8, half * tq, tq, dq8) + launch_time(nk, half * tk, tk, dkv);
+  for (int sq = 1; sq <= 16; sq *= 2)
+    for (int sk = 1; sk <= 16; sk *= 2) {
+      if ((sq > 1 && tq < 2.f * sq) || (sk > 1 && tk < 2.f * sk)) continue;
+      const int64_t bytes = partial_bytes(B, Sq, Hq, D, 1, sq) + partial_bytes(B, Sc, Hkv, D, 2, sk);
+      if (bytes > kPartialMost) continue;
+      const float n = nq4 * sq + nk * sk, mean = half * (nq4 * tq + nk * tk) / n;
+      const float most = tq / sq > tk / sk ? tq / sq : tk / sk;
+      const float time = kPrepare + launch_time(n, mean, most, both) + (bytes > 0 ? kReduce + 2.f * (float)bytes / kBytesPerUs : 0.f);
+      if (time < best_time) { best_time = time; best = {true, sq, sk}; }
+    }
+  return best;
 }
 
+template <bool CAUSAL, int KK>
+void launch_bwd(const BwdParams& p, const Plan& plan, float* partial, hipStream_t st) {
+  if (plan.joint) {
+    const int rows = p.B * p.Hq * p.Sq;
+    hipLaunchKernelGGL(bwd_prepare, dim3((rows + 15) / 16), dim3(256), 0, st, p, rows);
+    const TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ / 2, plan.sq, partial);
+    const TileMap wk = tile_map(p.B * p.Hkv, p.Sc, kRowsKv, plan.sk, partial + partial_bytes(p.B, p.Sq, p.Hq, p.D, 1, plan.sq) / 4);
+    const dim3 grid((wk.per_xcd + wq.per_xcd) * 8), block(256);
+    // (a kernel of its own: the bookkeeping of shared tiles costs 0.6 us where there are none)
+    if (plan.sq > 1 || plan.sk > 1) hipLaunchKernelGGL((bwd_joint<CAUSAL, KK, true>), grid, block, 0, st, p, wq, wk);
+    else hipLaunchKernelGGL((bwd_joint<CAUSAL, KK, false>), grid, block, 0, st, p, wq, wk);
+    const int q_rows = plan.sq > 1 ? p.B * p.Sq * p.Hq : 0, kv_rows = plan.sk > 1 ? p.B * p.Sc * p.Hkv : 0;
+    if (q_rows + kv_rows > 0)
+      hipLaunchKernelGGL(bwd_reduce, dim3((q_rows + 2 * kv_rows + 15) / 16), dim3(256), 0, st, p, wq, wk, q_rows, kv_rows);
+    return;
+  }
+  const TileMap wk = tile_map(p.B * p.Hkv, p.Sc, kRowsKv);
+  if (p.Sq > 0) {
+    // dQ (and delta / lse2 for both passes): one workgroup per 256 query rows; has to run before the dK / dV pass
+    const TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ);
+    hipLaunchKernelGGL((bwd_main<true, CAUSAL, KK>), dim3(wq.per_xcd * 8), dim3(512), 0, st, p, wq);
+  }
+  // dK, dV: one workgroup per 128 keys of one kv head
+  if (p.Sc > 0) hipLaunchKernelGGL((bwd_main<false, CAUSAL, KK>), dim3(wk.per_xcd * 8), dim3(256), 0, st, p, wk);
+}
+
+// -delta, lse2 and delta, (B, Hq, Sq) fp32 each, every one starting on a 16-byte boundary
+int64_t row_bytes(int B, int Sq, int Hq) { return ((((int64_t)B * Hq * Sq + 3) & ~int64_t(3)) * 3) * 4; }
+}  // namespace
+
+extern "C" int64_t mhip_attn_bwd_workspace_bytes(int B, int Sq, int Sc, int Hq, int Hkv, int D) {
+  if (B < 0 || Sq < 0 || Sc < 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0) return 0;
+  int64_t partial = 0;
+  for (int causal = 0; causal < 2; ++causal) {
+    const Plan plan = plan_block(B, Sq, Sc, Hq, Hkv, D, causal != 0);
+    const int64_t bytes = partial_bytes(B, Sq, Hq, D, 1, plan.sq) + partial_bytes(B, Sc, Hkv, D, 2, plan.sk);
+    partial = bytes > partial ? bytes : partial;
+  }
+  return row_bytes(B, Sq, Hq) + partial;
+}
+
+namespace {
 // own_scratch: take the workspace from `scratch` (resolved after the arguments have been checked)
 int bwd_block(const void* dout, const void* q, const void* k, const void* v,
               const void* out, const float* lse,
@@ -889,6 +995,8 @@ int bwd_block(const void* dout, const void* q, const void* k, const void* v,
   float* lse2_buf = delta_buf + slot;
   float* softmax_d = own_scratch ? nullptr : lse2_buf + slot;      // the built-in scratch has no room for it
   p.lse2 = lse2_buf; p.delta = delta_buf; p.softmax_d = softmax_d;
+  // sums of split passes: behind the three row vectors (in the built-in scratch, which has its own place for them)
+  float* partial = own_scratch ? delta_buf + (2 * kScratchRows + 8) : lse2_buf + 2 * slot;
   p.out = static_cast<const uint16_t*>(out); p.lse = lse;
   p.dq = static_cast<uint16_t*>(dq); p.dk = static_cast<uint16_t*>(dk); p.dv = static_cast<uint16_t*>(dv);
   p.dq_acc = dq_acc; p.dq_mode = dq_mode;
@@ -903,9 +1011,9 @@ int bwd_block(const void* dout, const void* q, const void* k, const void* v,
   p.scale = softmax_scale; p.scale_log2 = softmax_scale * kLog2e;
   const bool causal = mask == MHIP_MASK_CAUSAL;
 
-  const bool joint = Sq > 0 && Sc > 0 && side_by_side(p, causal);
-  if (D <= 64) causal ? launch_bwd<true, 4>(p, joint, st) : launch_bwd<false, 4>(p, joint, st);
-  else causal ? launch_bwd<true, 8>(p, joint, st) : launch_bwd<false, 8>(p, joint, st);
+  const Plan plan = plan_block(B, Sq, Sc, Hq, Hkv, D, causal);
+  if (D <= 64) causal ? launch_bwd<true, 4>(p, plan, partial, st) : launch_bwd<false, 4>(p, plan, partial, st);
+  else causal ? launch_bwd<true, 8>(p, plan, partial, st) : launch_bwd<false, 8>(p, plan, partial, st);
   return launch_status();
 }
 }  // namespace

@@ -20,7 +20,8 @@ def _close(name, got, ref):
     assert (got - ref).abs().max() <= 12 * 2 ** -8 * rms + 2 ** -8 * ref.abs().max() + 1e-4, name
 
 
-@pytest.mark.parametrize("W,S,Hq,Hkv,D", [(1, 300, 2, 2, 128), (2, 129, 4, 2, 64), (3, 257, 3, 1, 40), (4, 64, 2, 2, 128)])
+@pytest.mark.parametrize("W,S,Hq,Hkv,D", [(1, 300, 2, 2, 128), (2, 129, 4, 2, 64), (3, 257, 3, 1, 40), (4, 64, 2, 2, 128),
+                                           (2, 400, 8, 1, 128)])
 @pytest.mark.parametrize("dq_dtype,keep", [(torch.bfloat16, True), (torch.float32, True), (torch.bfloat16, False)])
 def test_backward_step_carries_the_sums(W, S, Hq, Hkv, D, dq_dtype, keep):
     import mercury_artifact_amd as M
@@ -84,3 +85,12 @@ def test_backward_block_on_narrow_heads(D, Sq, Sc, Hq, Hkv, causal):
 def test_backward_block_in_two_launches(D, Sq, Sc, causal):
     """Enough heads to fill the chip with either pass: one launch each, dQ with eight wavefronts."""
     _block(2, Sq, Sc, 128, 128, D, causal)
+
+
+@pytest.mark.parametrize("D", [40, 128])
+@pytest.mark.parametrize("B,Sq,Sc,Hq,Hkv,causal", [(1, 321, 130, 8, 1, False), (1, 700, 777, 8, 1, True), (2, 513, 400, 12, 2, True),
+                                                   (1, 130, 3000, 1, 1, False), (1, 3000, 130, 1, 1, True)])
+def test_backward_block_with_shared_tiles(B, Sq, Sc, Hq, Hkv, causal, D):
+    """Long chains of tiles on few workgroups (grouped heads, one head): their stationary tiles are shared and the sums
+    added by the third launch."""
+    _block(B, Sq, Sc, Hq, Hkv, D, causal)
