@@ -26,6 +26,7 @@ from typing import Optional
 import torch
 
 from . import _native as N
+from . import flash_attn_interface as _ops
 from .flash_attn_interface import (_flash_attn_backward, _flash_attn_forward, aligned_rows, attn_bwd_block,
                                    attn_bwd_chunk)
 from .merge import (MAX_MERGE_MANY, get_default_args, grad_accumulate, merge_into, merge_many, pack_block,
@@ -74,10 +75,27 @@ def _neighbours(ring: LocalRing, dim: int):
 
 
 def _block_forward(q, k, v, softmax_scale, dropout_p, causal, window_size, alibi_slopes, q_descale=None, k_descale=None,
-                   v_descale=None):
-    """The block operator on the values a generated step passes it by keyword."""
-    return _flash_attn_forward(q, k, v, dropout_p, softmax_scale, causal, window_size[0], window_size[1], 0.0, alibi_slopes,
-                               dropout_p > 0, q_descale, k_descale, v_descale)
+                   v_descale=None, into=None):
+    """(out, lse) of the block operator on the values a generated step passes it by keyword; ``into`` gives the two
+    tensors to write (see :func:`_block_results`)."""
+    if into is not None:
+        return _ops.attn_fwd_block(q, k, v, softmax_scale, causal, q_descale, k_descale, v_descale, *into)
+    outputs = _flash_attn_forward(q, k, v, dropout_p, softmax_scale, causal, window_size[0], window_size[1], 0.0, alibi_slopes,
+                                  dropout_p > 0, q_descale, k_descale, v_descale)
+    assert len(outputs) == 4
+    return outputs[:2]
+
+
+def _block_results(n, q, kv, dropout_p, window_size, alibi_slopes, **descales):
+    """Places for the results of a step's ``n`` blocks over all rows of ``q``, from one allocation each for the outputs and
+    the LSEs; None for every block where the operator has something to report or to record."""
+    if (dropout_p or alibi_slopes is not None or window_size[0] not in (-1, None) or window_size[1] not in (-1, None)
+            or q.dim() != 4 or not N.host.undispatched(q, kv, *descales.values())):
+        return [None] * n
+    B, Sq, Hq, D = q.shape
+    outs = torch.empty((n, B, Sq, Hq, D), dtype=torch.bfloat16, device=q.device)
+    lses = torch.empty((n, B, Hq, Sq), dtype=torch.float32, device=q.device)
+    return list(zip(outs.unbind(0), lses.unbind(0)))
 
 
 def _as_rows(t):
@@ -133,6 +151,7 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
                       f"{MAX_MERGE_MANY} blocks and writes contiguous bfloat16, so this step merges block by block "
                       "(same result, one pass over the fp32 accumulator per block)", RuntimeWarning, stacklevel=3)
     done = 0
+    places = _block_results(n_blocks, q, kv, dropout_p, window_size, alibi_slopes, **extra) if defer else [None] * n_blocks
     main = side = None
     kv_ready = next_ready = None
     if two_streams and defer:
@@ -168,13 +187,13 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
                     side.wait_event(kv_ready)
                 _kv.record_stream(side)              # may have been allocated by the hop on the current stream
                 with torch.cuda.stream(side):
-                    outputs = _block_forward(q, _k, _v, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra)
-                for t in outputs[:2]:
-                    t.record_stream(main)            # allocated under the side stream, read by the fold on the main one
+                    block_out, block_lse = _block_forward(q, _k, _v, softmax_scale, dropout_p, causal, window_size,
+                                                          alibi_slopes, into=places[done], **extra)
+                for t in (block_out, block_lse):
+                    t.record_stream(side if places[done] is not None else main)      # the stream it was not allocated under
             else:
-                outputs = _block_forward(q, _k, _v, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra)
-            assert len(outputs) == 4
-            block_out, block_lse, _, _ = outputs
+                block_out, block_lse = _block_forward(q, _k, _v, softmax_scale, dropout_p, causal, window_size, alibi_slopes,
+                                                      into=places[done], **extra)
             done += 1
             if defer:
                 blocks.append((block_out, block_lse))
@@ -250,6 +269,7 @@ def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=F
     blocks = []
     defer = (fused_epilogue and deferred_merge and len(hops) <= MAX_MERGE_MANY and o.dtype == torch.bfloat16
              and o.is_contiguous() and lse.is_contiguous())
+    places = _block_results(len(hops), q, kv, dropout_p, window_size, alibi_slopes) if defer else [None] * len(hops)
     for step, hop in enumerate(hops):
         if step == 0:
             _kv = kv.contiguous()
@@ -261,9 +281,8 @@ def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=F
             _next_kv = ring.send_recv(send_to, recv_from, _kv)
             ring.commit()
         _k, _v = _kv.unbind(0)
-        outputs = _block_forward(q, _k, _v, softmax_scale, dropout_p, causal, window_size, alibi_slopes)
-        assert len(outputs) == 4
-        block_out, block_lse, _, _ = outputs
+        block_out, block_lse = _block_forward(q, _k, _v, softmax_scale, dropout_p, causal, window_size, alibi_slopes,
+                                              into=places[step])
         if defer:
             blocks.append((block_out, block_lse))
         else:
@@ -299,9 +318,8 @@ def flash_attn_expose_reduce_q_ring(qs, kvs, os_, lses, softmax_scale, dropout_p
         buf = []
         for r in range(world):
             kv = kvs[r]
-            outputs = _block_forward(q_cur[r], kv[0], kv[1], softmax_scale, dropout_p, causal, window_size, alibi_slopes)
-            assert len(outputs) == 4
-            block_out, block_lse, _, _ = outputs
+            block_out, block_lse = _block_forward(q_cur[r], kv[0], kv[1], softmax_scale, dropout_p, causal, window_size,
+                                                  alibi_slopes)
             buf.append(pack_block(block_out, block_lse, reduce_into=arrived[r]))
         if step + 1 != world:
             q_next, arrived = [None] * world, [None] * world
@@ -349,8 +367,7 @@ def zigzag_causal_pack_kv(q, kv, o, lse, softmax_scale, dropout_p=0, causal=True
             bq, bk, bv, bc, sl = q, _kv[0][:, :half], _kv[1][:, :half], False, None
         else:
             bq, bk, bv, bc, sl = q[:, half:], _kv[0], _kv[1], False, (slice(None), slice(half, None))
-        outputs = _block_forward(bq, bk, bv, softmax_scale, dropout_p, bc, window_size, alibi_slopes)
-        block_out, block_lse, _, _ = outputs
+        block_out, block_lse = _block_forward(bq, bk, bv, softmax_scale, dropout_p, bc, window_size, alibi_slopes)
         if defer:
             blocks.append((block_out, block_lse, 0 if sl is None else half))
             continue
