@@ -140,11 +140,13 @@ int mhip_attn_bwd_block_noalloc(const void* dout, const void* q, const void* k, 
  *   not last:  dq_acc = T                 (dq is not used)
  *   last:      dq = bf16(T)               (dq_acc is read unless first, not written)
  * dk / dv receive the chunk's gradients in bf16 and dk32 / dv32 (fp32, (B, Sc, Hkv, D) contiguous) the same values in
- * fp32; either pair may be NULL, not both.  Everything else as in mhip_attn_bwd_block (the same workspace).
+ * fp32; either pair may be NULL, not both.  rowsum(dout * out) and the scaled LSE are the same for every chunk:
+ * `prepared` says that the workspace holds them, left at its start by a call with the same dout, out, lse, B, Sq and Hq.
+ * Everything else as in mhip_attn_bwd_block (the same workspace).
  */
 int mhip_attn_bwd_chunk(const void* dout, const void* q, const void* k, const void* v,
                         const void* out, const float* lse,
-                        void* dq, float* dq_acc, int first, int last,
+                        void* dq, float* dq_acc, int first, int last, int prepared,
                         void* dk, void* dv, float* dk32, float* dv32,
                         int B, int Sq, int Sc, int Hq, int Hkv, int D,
                         int64_t q_sb, int64_t q_ss, int64_t q_sh,     /* q, dout  */

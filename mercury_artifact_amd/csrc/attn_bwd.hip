@@ -58,6 +58,7 @@ struct BwdParams {
   float* dk32; float* dv32;                // the same bf16 values in fp32, (B, Sc, Hkv, D) contiguous, or null; dk / dv
                                            // may be null then
   int dq_mode;                             // what dq_acc is for: kDq*
+  bool prepared;                           // delta and lse2 are in the workspace already
   int B, Sq, Sc, Hq, Hkv, group;
   int D;            // head dimension of the tensors, a multiple of 8 up to kD; columns D .. kD-1 are zeros on chip
   int64_t q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, dk_sb, dk_ss, dk_sh, dq_sb, dq_ss, dq_sh, o_sb, o_ss, o_sh;
@@ -520,15 +521,17 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
         delta_lane = p.delta[r];
         asm volatile("" : "+v"(lse2_lane), "+v"(delta_lane));
       }
+      constexpr bool kEarly = WAVES == 4;            // stage 1 is not part of the rows' places
       copy_tile(0, 0);
       copy_rows(xsrc, x_lds);
       copy_rows(ysrc, y_lds);
-      copy_tile(1, 1);
-      asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kCopiesPerTile) : "memory");
+      if (kEarly) copy_tile(1, 1);
+      asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kEarly ? kCopiesPerTile : 0) : "memory");
       read_rows(x_lds, xf);
       read_rows(y_lds, yf);
       pin();
-      __builtin_amdgcn_s_barrier();                  // tile 0 is there for everybody, stages 2 and 3 are free
+      __builtin_amdgcn_s_barrier();                  // tile 0 is there for everybody, the rows' places are free
+      if (!kEarly) copy_tile(1, 1);
       copy_tile(2, 2);
     }
   }
@@ -726,11 +729,11 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   }
 }
 
-template <bool DQ, bool CAUSAL, int KK>
+template <bool DQ, bool CAUSAL, int KK, bool PREPARED>
 __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p, const TileMap w) {
   constexpr int kWaves = DQ ? 8 : 4;
   __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<DQ, kWaves>];
-  bwd_pass<DQ, CAUSAL, KK, kWaves, !DQ, false>(p, w, (int)blockIdx.x, smem);
+  bwd_pass<DQ, CAUSAL, KK, kWaves, PREPARED, false>(p, w, (int)blockIdx.x, smem);
 }
 
 // Both passes side by side, for launches that leave CUs idle one after the other.
@@ -909,7 +912,7 @@ template <bool CAUSAL, int KK>
 void launch_bwd(const BwdParams& p, const Plan& plan, float* partial, hipStream_t st) {
   if (plan.joint) {
     const int rows = p.B * p.Hq * p.Sq;
-    hipLaunchKernelGGL(bwd_prepare, dim3((rows + 15) / 16), dim3(256), 0, st, p, rows);
+    if (!p.prepared) hipLaunchKernelGGL(bwd_prepare, dim3((rows + 15) / 16), dim3(256), 0, st, p, rows);
     const TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ / 2, plan.sq, partial);
     const TileMap wk = tile_map(p.B * p.Hkv, p.Sc, kRowsKv, plan.sk, partial + partial_bytes(p.B, p.Sq, p.Hq, p.D, 1, plan.sq) / 4);
     const dim3 grid((wk.per_xcd + wq.per_xcd) * 8), block(256);
@@ -925,10 +928,11 @@ void launch_bwd(const BwdParams& p, const Plan& plan, float* partial, hipStream_
   if (p.Sq > 0) {
     // dQ (and delta / lse2 for both passes): one workgroup per 256 query rows; has to run before the dK / dV pass
     const TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ);
-    hipLaunchKernelGGL((bwd_main<true, CAUSAL, KK>), dim3(wq.per_xcd * 8), dim3(512), 0, st, p, wq);
+    if (p.prepared) hipLaunchKernelGGL((bwd_main<true, CAUSAL, KK, true>), dim3(wq.per_xcd * 8), dim3(512), 0, st, p, wq);
+    else hipLaunchKernelGGL((bwd_main<true, CAUSAL, KK, false>), dim3(wq.per_xcd * 8), dim3(512), 0, st, p, wq);
   }
   // dK, dV: one workgroup per 128 keys of one kv head
-  if (p.Sc > 0) hipLaunchKernelGGL((bwd_main<false, CAUSAL, KK>), dim3(wk.per_xcd * 8), dim3(256), 0, st, p, wk);
+  if (p.Sc > 0) hipLaunchKernelGGL((bwd_main<false, CAUSAL, KK, true>), dim3(wk.per_xcd * 8), dim3(256), 0, st, p, wk);
 }
 
 // -delta, lse2 and delta, (B, Hq, Sq) fp32 each, every one starting on a 16-byte boundary
@@ -950,7 +954,7 @@ namespace {
 // own_scratch: take the workspace from `scratch` (resolved after the arguments have been checked)
 int bwd_block(const void* dout, const void* q, const void* k, const void* v,
               const void* out, const float* lse,
-              void* dq, void* dk, void* dv, float* dq_acc, int dq_mode, float* dk32, float* dv32,
+              void* dq, void* dk, void* dv, float* dq_acc, int dq_mode, float* dk32, float* dv32, bool prepared,
               int B, int Sq, int Sc, int Hq, int Hkv, int D,
               int64_t q_sb, int64_t q_ss, int64_t q_sh,
               int64_t k_sb, int64_t k_ss, int64_t k_sh,
@@ -999,7 +1003,7 @@ int bwd_block(const void* dout, const void* q, const void* k, const void* v,
   float* partial = own_scratch ? delta_buf + (2 * kScratchRows + 8) : lse2_buf + 2 * slot;
   p.out = static_cast<const uint16_t*>(out); p.lse = lse;
   p.dq = static_cast<uint16_t*>(dq); p.dk = static_cast<uint16_t*>(dk); p.dv = static_cast<uint16_t*>(dv);
-  p.dq_acc = dq_acc; p.dq_mode = dq_mode;
+  p.dq_acc = dq_acc; p.dq_mode = dq_mode; p.prepared = prepared;
   p.dk32 = dk32; p.dv32 = dv32;
   p.B = B; p.Sq = Sq; p.Sc = Sc; p.Hq = Hq; p.Hkv = Hkv; p.group = Hq / Hkv;
   p.D = D;
@@ -1038,7 +1042,7 @@ extern "C" int mhip_attn_bwd_block(const void* dout, const void* q, const void* 
                                    float softmax_scale, int mask, int deterministic,
                                    void* workspace, void* stream) {
   (void)deterministic;   // there are no atomics: every run is deterministic
-  return bwd_block(dout, q, k, v, out, lse, dq, dk, dv, dq_acc, kDqAdd, nullptr, nullptr, B, Sq, Sc, Hq, Hkv, D, q_sb, q_ss, q_sh,
+  return bwd_block(dout, q, k, v, out, lse, dq, dk, dv, dq_acc, kDqAdd, nullptr, nullptr, false, B, Sq, Sc, Hq, Hkv, D, q_sb, q_ss, q_sh,
                    k_sb, k_ss, k_sh, dk_sb, dk_ss, dk_sh, dq_sb, dq_ss, dq_sh, o_sb, o_ss, o_sh, softmax_scale, mask,
                    workspace, false,
                    static_cast<hipStream_t>(stream));
@@ -1056,7 +1060,7 @@ extern "C" int mhip_attn_bwd_block_noalloc(const void* dout, const void* q, cons
                                            float softmax_scale, int mask, int deterministic, void* stream) {
   (void)deterministic;
   // the dQ pass overwrites the part of the scratch the dK / dV pass reads, so nothing has to be cleared
-  return bwd_block(dout, q, k, v, out, lse, dq, dk, dv, dq_acc, kDqAdd, nullptr, nullptr, B, Sq, Sc, Hq, Hkv, D, q_sb, q_ss, q_sh,
+  return bwd_block(dout, q, k, v, out, lse, dq, dk, dv, dq_acc, kDqAdd, nullptr, nullptr, false, B, Sq, Sc, Hq, Hkv, D, q_sb, q_ss, q_sh,
                    k_sb, k_ss, k_sh, dk_sb, dk_ss, dk_sh, dq_sb, dq_ss, dq_sh, o_sb, o_ss, o_sh, softmax_scale, mask,
                    nullptr, true,
                    static_cast<hipStream_t>(stream));
@@ -1064,7 +1068,7 @@ extern "C" int mhip_attn_bwd_block_noalloc(const void* dout, const void* q, cons
 
 extern "C" int mhip_attn_bwd_chunk(const void* dout, const void* q, const void* k, const void* v,
                                    const void* out, const float* lse,
-                                   void* dq, float* dq_acc, int first, int last,
+                                   void* dq, float* dq_acc, int first, int last, int prepared,
                                    void* dk, void* dv, float* dk32, float* dv32,
                                    int B, int Sq, int Sc, int Hq, int Hkv, int D,
                                    int64_t q_sb, int64_t q_ss, int64_t q_sh,
@@ -1076,7 +1080,7 @@ extern "C" int mhip_attn_bwd_chunk(const void* dout, const void* q, const void* 
   const bool only = first && last;      // the only chunk: nothing to carry
   if (!first && !dq_acc) return MHIP_EINVAL;
   return bwd_block(dout, q, k, v, out, lse, dq, dk, dv, only ? nullptr : dq_acc,
-                   only ? kDqAdd : first ? kDqFirst : last ? kDqLast : kDqMiddle, dk32, dv32,
+                   only ? kDqAdd : first ? kDqFirst : last ? kDqLast : kDqMiddle, dk32, dv32, prepared != 0,
                    B, Sq, Sc, Hq, Hkv, D, q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, dk_sb, dk_ss, dk_sh, dq_sb, dq_ss, dq_sh,
                    o_sb, o_ss, o_sh, softmax_scale, mask, workspace, false, static_cast<hipStream_t>(stream));
 }

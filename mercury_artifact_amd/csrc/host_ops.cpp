@@ -225,10 +225,10 @@ PyObject* bwd_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// (dout, q, k, v, out, softmax_lse, dq, dq_acc, first, last, dkv, dkv32, softmax_scale) -> True
+// (dout, q, k, v, out, softmax_lse, dq, dq_acc, first, last, dkv, dkv32, softmax_scale, workspace) -> workspace
 PyObject* bwd_chunk(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  ENTER(13);
+  ENTER(14);
   Args in{a};
   const Tensor &dout = in.tensor(0), &q = in.tensor(1), &k = in.tensor(2), &v = in.tensor(3), &out = in.tensor(4),
                &lse = in.tensor(5);
@@ -256,11 +256,16 @@ PyObject* bwd_chunk(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   const int first = PyObject_IsTrue(a[8]), last = PyObject_IsTrue(a[9]);
   const double scale = PyFloat_AsDouble(a[12]);
   if (first < 0 || last < 0 || (scale == -1.0 && PyErr_Occurred())) { PyErr_Clear(); SLOW; }
+  const Tensor* kept;
+  if (!optional(a[13], q, kept)) SLOW;
+  if (kept && (kept->scalar_type() != at::kByte || !kept->is_contiguous() ||
+               kept->numel() != entry.bwd_bytes(B, Sq, Sc, Hq, Hkv, D)))
+    SLOW;
   OnDevice on(q);
-  const Tensor ws = bwd_workspace(q, Sc, Hkv);
+  const Tensor ws = kept ? *kept : bwd_workspace(q, Sc, Hkv);
   auto second16 = [](const Tensor* t) { return t ? static_cast<void*>(static_cast<char*>(t->data_ptr()) + 2 * t->stride(0)) : nullptr; };
   const int code = entry.chunk(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), floats(&lse),
-                               data(dq), floats(acc), first, last, data(dkv), second16(dkv),
+                               data(dq), floats(acc), first, last, kept != nullptr, data(dkv), second16(dkv),
                                floats(dkv32), dkv32 ? floats(dkv32) + dkv32->stride(0) : nullptr, B, Sq, Sc, Hq, Hkv, D,
                                q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
                                dkv ? dkv->stride(1) : 0, dkv ? dkv->stride(2) : 0, dkv ? dkv->stride(3) : 0,
@@ -268,7 +273,7 @@ PyObject* bwd_chunk(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
                                out.stride(0), out.stride(1), out.stride(2), (float)scale, MHIP_MASK_NONE, ws.data_ptr(),
                                on.stream);
   if (code != MHIP_OK) SLOW;
-  Py_RETURN_TRUE;
+  return give(ws);
   END_HANDLE_TH_ERRORS
 }
 

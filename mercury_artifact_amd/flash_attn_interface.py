@@ -240,13 +240,15 @@ def attn_bwd_block(dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_scale, c
 
 def attn_bwd_chunk(dout, q, k, v, out, softmax_lse, dq: Optional[torch.Tensor], dq_acc: Optional[torch.Tensor],
                    first: bool, last: bool, dkv: Optional[torch.Tensor], dkv32: Optional[torch.Tensor],
-                   softmax_scale) -> None:
+                   softmax_scale, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """One chunk of a ring step's backward through mhip_attn_bwd_chunk: ``dq_acc`` (fp32, contiguous, q's shape) carries
     the sum of the chunks' dq from the ``first`` to the ``last`` one, which writes it to ``dq`` (bf16) instead;
     ``dkv`` (2, B, Sc, Hkv, D) receives the chunk's dk and dv in bf16 and ``dkv32`` (contiguous) the same values in fp32;
-    either may be None.  All operands are taken as they are: 16-byte aligned rows, q and dout of one layout."""
-    if N.host.bwd_chunk(dout, q, k, v, out, softmax_lse, dq, dq_acc, first, last, dkv, dkv32, softmax_scale):
-        return
+    either may be None.  All operands are taken as they are: 16-byte aligned rows, q and dout of one layout.  Returns the
+    workspace, which a later chunk of the same shape, dout, out and LSE may be given: rowsum(dout * out) is in it then."""
+    done = N.host.bwd_chunk(dout, q, k, v, out, softmax_lse, dq, dq_acc, first, last, dkv, dkv32, softmax_scale, workspace)
+    if done is not None:
+        return done
     _check_block_inputs(q, k, v, 0, -1, -1, 0.0, None)
     N.require_cuda(dout, out, softmax_lse, dq, dq_acc, dkv, dkv32)
     B, Sq, Hq, D = q.shape
@@ -262,18 +264,23 @@ def attn_bwd_chunk(dout, q, k, v, out, softmax_lse, dq: Optional[torch.Tensor], 
     if dkv is not None and (dkv.shape != (2, *k.shape) or dkv.dtype != torch.bfloat16):
         raise RuntimeError(f"dkv must be bfloat16 of shape {(2, *k.shape)}")
     lib = N.lib()
-    ws = torch.empty((int(lib.mhip_attn_bwd_workspace_bytes(B, Sq, Sc, Hq, Hkv, D)),), dtype=torch.uint8,
-                     device=q.device)
+    size = int(lib.mhip_attn_bwd_workspace_bytes(B, Sq, Sc, Hq, Hkv, D))
+    if workspace is not None and (workspace.dtype != torch.uint8 or workspace.numel() != size
+                                  or not workspace.is_contiguous()):
+        raise RuntimeError("workspace must be what a call of the same shape returned")
+    N.require_cuda(workspace)
+    ws = torch.empty((size,), dtype=torch.uint8, device=q.device) if workspace is None else workspace
     z3 = (0, 0, 0)
     with torch.cuda.device(q.device):
         code = lib.mhip_attn_bwd_chunk(
             N.ptr(dout), N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(out), N.ptr(softmax_lse), N.ptr(dq), N.ptr(dq_acc),
-            int(first), int(last), *((None, None) if dkv is None else (N.ptr(dkv[0]), N.ptr(dkv[1]))),
+            int(first), int(last), int(workspace is not None), *((None, None) if dkv is None else (N.ptr(dkv[0]), N.ptr(dkv[1]))),
             *((None, None) if dkv32 is None else (N.ptr(dkv32[0]), N.ptr(dkv32[1]))),
             B, Sq, Sc, Hq, Hkv, D, *_strides3(q), *_strides3(k), *(z3 if dkv is None else _strides3(dkv[0])),
             *(z3 if dq is None else _strides3(dq)), *_strides3(out),
             float(softmax_scale), N.MASK_NONE, N.ptr(ws), N.stream_of(q))
     N.check(code, "mhip_attn_bwd_chunk")
+    return ws
 
 
 def aligned_rows(*ts: torch.Tensor) -> bool:

@@ -435,7 +435,7 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
         reduce_dq = torch.zeros(q.shape, dtype=torch.float32, device=q.device)
     elif carried and not (write_dq and ring.world == 1):
         reduce_dq = torch.empty(q.shape, dtype=torch.float32, device=q.device)
-    _kv = _next_kv = None
+    _kv = _next_kv = prepared = None
     own = ring.current
     for step, hop in enumerate(_hops(ring)):
         if step == 0:
@@ -459,8 +459,12 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
             if dkv_chunks is not None:
                 chunk_grad = dkv_chunks[chunk_id] = torch.empty(_kv.shape, dtype=torch.float32, device=_kv.device)
             _k, _v = _as_rows(_kv).unbind(0)
-            attn_bwd_chunk(dout, q, _k, _v, o, lse, dq if write_dq else None, reduce_dq, step == 0,
-                           write_dq and hop is None, block_dkv, chunk_grad, softmax_scale)
+            # rowsum(dout * o) and the scaled lse are the same for every chunk: worked out with the first one
+            usual = _kv.shape == kv.shape
+            ws = attn_bwd_chunk(dout, q, _k, _v, o, lse, dq if write_dq else None, reduce_dq, step == 0,
+                                write_dq and hop is None, block_dkv, chunk_grad, softmax_scale,
+                                prepared if usual else None)
+            prepared = ws if usual else prepared
             if mine and not direct:
                 dkv[...] = block_dkv
             continue
