@@ -9,28 +9,46 @@ missing library or host module is an error, not a reason to take another path.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 from ctypes import c_float, c_int, c_int64, c_void_p
 from typing import Optional
 
 import torch
 
-try:
-    from .csrc import _mercury_host as host
-except ImportError as _e:               # reported by lib(), the first thing every operator asks for
-
-    class _NoHost:
-        reason = str(_e)
-
-        def __getattr__(self, name):
-            return lambda *args: None
-
-    host = _NoHost()
-
 # MERCURY_HIP_LIB is a deployment option: the path of the built library when it is not kept next to the package.
-LIB_PATH = os.environ.get("MERCURY_HIP_LIB") or os.path.join(
-    os.path.dirname(os.path.abspath(__file__)), "csrc", "libmercury_hip.so")
+_BUILT = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
+LIB_PATH = os.environ.get("MERCURY_HIP_LIB") or os.path.join(_BUILT, "libmercury_hip.so")
 ABI_VERSION = 4      # MHIP_ABI_VERSION of include/mercury_hip.h the signatures below were written against
+
+
+class _NoHost:
+    """Stands in for a host module that is not there: no call is taken; lib() says why."""
+
+    def __init__(self, reason):
+        self.reason = reason
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def _load_host():
+    """The host module from beside the library, or from where the package is built."""
+    reason = "not built"
+    for folder in (os.path.dirname(LIB_PATH), _BUILT):
+        path = os.path.join(folder, "_mercury_host.so")
+        if os.path.exists(path):
+            try:
+                spec = importlib.util.spec_from_file_location(f"{__package__}.csrc._mercury_host", path)
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+                return module
+            except ImportError as e:
+                reason = str(e)
+    return _NoHost(reason)
+
+
+host = _load_host()
 
 MHIP_BF16, MHIP_E4M3, MHIP_F32 = 0, 1, 2
 MASK_NONE, MASK_CAUSAL = 0, 1
@@ -61,7 +79,7 @@ EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 
 
 def lib() -> ctypes.CDLL:
-    global _lib
+    global _lib, host
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise RuntimeError(
@@ -80,6 +98,8 @@ def lib() -> ctypes.CDLL:
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
+        if isinstance(host, _NoHost):          # built since the package was imported
+            host = _load_host()
         if host.bind({name: ctypes.cast(getattr(handle, name), c_void_p).value for name in _SIGNATURES}) is not True:
             raise RuntimeError("the host module _mercury_host is missing or stale: build it with "
                                f"`python -m mercury_artifact_amd.csrc.build` ({getattr(host, 'reason', 'entry points')})")

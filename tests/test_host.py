@@ -296,3 +296,19 @@ def test_local_mesh_reports_the_first_failure_and_releases_the_waiting_ranks():
         return int(got.item())
 
     assert mesh.run(again) == [13, 10, 11, 12]
+
+
+def test_host_module_built_after_the_import_is_found(monkeypatch):
+    """A build from the package itself imports it first, without a host module: lib() looks again."""
+    from mercury_artifact_amd import _native as N
+
+    monkeypatch.setattr(N, "host", N._NoHost("not built"))
+    monkeypatch.setattr(N, "_lib", None)
+    N.lib()
+    assert not isinstance(N.host, N._NoHost)
+    # a module that is not there is reported, not passed over
+    monkeypatch.setattr(N, "host", N._NoHost("not built"))
+    monkeypatch.setattr(N, "_lib", None)
+    monkeypatch.setattr(N, "_load_host", lambda: N._NoHost("not built"))
+    with pytest.raises(RuntimeError, match="_mercury_host"):
+        N.lib()
