@@ -550,8 +550,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
     }
     float l_tot = 0.f;
 #pragma unroll
-    for (int g = 0; g < KS; ++g)
-      if (st[g][1] > 0.f) l_tot += st[g][1] * fast_exp2((st[g][0] - m_all) * p.scale_log2);
+    for (int g = 0; g < KS; ++g)       // (a sum of NaN is no smaller than 0 and goes into the row's)
+      l_tot += st[g][1] > 0.f ? st[g][1] * fast_exp2((st[g][0] - m_all) * p.scale_log2) : st[g][1];
     const float weight = l_own > 0.f ? fast_exp2((m_ref - m_all) * p.scale_log2) / l_tot : 0.f;
     if (kg == 0 && hf == 0 && my_q < p.Sq)
       p.lse[((int64_t)b * p.Hq + hq) * p.Sq + my_q] =

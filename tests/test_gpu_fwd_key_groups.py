@@ -61,3 +61,19 @@ def test_key_groups_with_one_dominant_group(slope, causal):
     kv = torch.randn(2, B, Sc, H, D, generator=g)
     kv[0, ..., 0] = slope / 8.0 * torch.arange(Sc)[None, :, None]
     _compare(q.bfloat16(), kv.bfloat16(), 1.0, causal, f"slope {slope} causal={causal}")
+
+
+@pytest.mark.parametrize("launch", [4, 2, 1])
+def test_a_key_of_nan_reaches_the_row_whatever_group_holds_it(launch):
+    """A row that meets NaN gets an output of NaN and, as with one key group, an LSE of -inf; other rows see nothing."""
+    import mercury_artifact_amd as M
+
+    B, Hq, Hkv = LAUNCHES[launch]
+    g = torch.Generator().manual_seed(11)
+    q = torch.randn(B, 256, Hq, 128, generator=g).bfloat16()
+    kv = torch.randn(2, B, 320, Hkv, 128, generator=g).bfloat16()
+    clean, clean_lse = M.attn_fwd_block(q.cuda(), kv[0].cuda(), kv[1].cuda(), 0.1, causal=True)
+    kv[0, :, 240] = float("nan")                  # hidden from the rows below 176
+    out, lse = M.attn_fwd_block(q.cuda(), kv[0].cuda(), kv[1].cuda(), 0.1, causal=True)
+    assert torch.equal(out[:, :176], clean[:, :176]) and torch.equal(lse[..., :176], clean_lse[..., :176])
+    assert bool(out[:, 176:].isnan().all()) and bool((lse[..., 176:] == -torch.inf).all())
