@@ -164,7 +164,9 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
             LocalRing(ring.mesh_shape, ring.rank, [c[:, :, rows] for c in ring.chunks], copy=ring.copy)
         for step, hop in enumerate(steps):
             if step == 0:
-                _kv = _as_rows(kv if ring_divide == 1 else kv[:, :, rows])
+                _kv = kv if ring_divide == 1 else kv[:, :, rows]
+                # (a subclass may send it, and transports want it in one piece)
+                _kv = _as_rows(_kv) if type(ring) is LocalRing else _kv.contiguous()
                 kv_ready = None
                 if side is not None and part > 0:      # a copy above sits behind earlier launches
                     kv_ready = torch.cuda.Event()

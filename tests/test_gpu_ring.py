@@ -273,3 +273,23 @@ def test_two_stream_step_is_bit_identical(copy, ring_divide):
         assert torch.equal(o, ref_o) and torch.equal(lse, ref_l)
     ro, rl = O.ring_forward(q.float().cpu(), [c.float().cpu() for c in kvs], O.single_ring_order(rank, W), scale)
     assert (ref_o.float().cpu() - ro).abs().max().item() <= 2e-2
+
+
+def test_a_ring_of_another_class_sends_contiguous_chunks():
+    import mercury_artifact_amd as M
+
+    class Sender(M.LocalRing):
+        def send_recv(self, to_rank, from_rank, send_tensor, recv_tensor=None):
+            assert send_tensor.is_contiguous()
+            return super().send_recv(to_rank, from_rank, send_tensor, recv_tensor)
+
+    g = torch.Generator(device="cuda").manual_seed(2)
+    wide = [torch.randn(2, 1, 64, 4, 128, generator=g, device="cuda").bfloat16() for _ in range(2)]
+    q = torch.randn(1, 64, 2, 128, generator=g, device="cuda").bfloat16()
+    out, lse = {}, {}
+    for chunks in ([w[:, :, :, :2] for w in wide], [w[:, :, :, :2].contiguous() for w in wide]):
+        key = chunks[0].is_contiguous()
+        out[key], lse[key] = torch.empty_like(q), torch.empty(1, 2, 64, device="cuda")
+        ring = (M.LocalRing if key else Sender)((2,), 0, chunks)
+        M.flash_attn_pack_kv(q, chunks[0], out[key], lse[key], 0.1, ring=ring)
+    assert torch.equal(out[True], out[False]) and torch.equal(lse[True], lse[False])
