@@ -46,7 +46,8 @@ const Tensor* plain(PyObject* o) {
   const auto keys = t.key_set();
   if (!t.is_cuda() || t.layout() != at::kStrided || keys.has(c10::DispatchKey::Python) ||
       keys.has(c10::DispatchKey::Functionalize) || keys.has(c10::DispatchKey::FuncTorchBatched) ||
-      keys.has(c10::DispatchKey::FuncTorchGradWrapper))
+      keys.has(c10::DispatchKey::FuncTorchGradWrapper) || keys.has(c10::DispatchKey::Negative) ||
+      keys.has(c10::DispatchKey::Conjugate) || keys.has(c10::DispatchKey::ZeroTensor))
     return nullptr;
   return &t;
 }
@@ -129,6 +130,19 @@ PyObject* undispatched(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     yes = t && !(grad && t->requires_grad());
   }
   return PyBool_FromLong(yes);
+}
+
+// Says that the tensors have been written to, as an operator does for the arguments it mutates: autograd compares the
+// count with what it saved.
+PyObject* written(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  for (Py_ssize_t i = 0; i < nargs; ++i) {
+    if (!THPVariable_Check(a[i])) continue;
+    const Tensor& t = THPVariable_Unpack(a[i]);
+    if (t.defined() && !t.is_inference()) t.unsafeGetTensorImpl()->bump_version();
+  }
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
 }
 
 // (q, k, v, softmax_scale, causal, q_descale, k_descale, v_descale, out, lse)
@@ -429,7 +443,7 @@ PyObject* bind(PyObject*, PyObject* table) {
 
 #define FAST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    FAST(undispatched), FAST(fwd_block), FAST(no_dropout), FAST(bwd_block), FAST(bwd_chunk), FAST(merge_into),
+    FAST(undispatched), FAST(written), FAST(fwd_block), FAST(no_dropout), FAST(bwd_block), FAST(bwd_chunk), FAST(merge_into),
     FAST(merge_many), FAST(pack_block), FAST(unpack_into), FAST(quantize_e4m3),
     {"bind", bind, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};

@@ -325,7 +325,9 @@ def _backward_now(dout, q, k, v, out, softmax_lse, dq, dk, dv, dropout_p, softma
             or window_size_right not in (-1, None)
             or not N.host.undispatched(dout, q, k, v, out, softmax_lse, dq, dk, dv)):
         return None
-    return attn_bwd_block(dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_scale, bool(causal), bool(deterministic))
+    delta = attn_bwd_block(dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_scale, bool(causal), bool(deterministic))
+    N.host.written(dq, dk, dv)
+    return delta
 
 
 class _BackwardOp(type(_flash_attn_backward)):

@@ -500,3 +500,5 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
             dkv[...] = red.to(dkv.dtype)
     if not write_dq:
         dq[...] = reduce_dq.to(dq.dtype)
+    if carried:
+        N.host.written(dq, dkv)

@@ -139,3 +139,24 @@ def test_the_operator_goes_through_the_dispatcher_where_something_watches():
         plain = M._flash_attn_forward(q.detach().requires_grad_(), *args[1:])[0]
     assert torch.equal(out, plain) and not plain.requires_grad
     assert torch.ops.mercury_amd._flash_attn_forward(*args)[0].equal(plain)
+
+
+def test_gradients_count_as_written():
+    """The operator says that it writes dq, dk and dv; so does a call that goes past the dispatcher, and the driver."""
+    import mercury_artifact_amd as M
+
+    q, kv, dout = _data()
+    out, lse = M.attn_fwd_block(q, kv[0], kv[1], 0.1)
+    for mode in (torch.no_grad, torch.inference_mode):
+        dq, dkv = torch.empty_like(q), torch.empty_like(kv)
+        before = dq._version, dkv._version
+        with mode():
+            M._flash_attn_backward(dout, q, kv[0], kv[1], out, lse, dq, dkv[0], dkv[1], 0.0, 0.1, False, -1, -1, 0.0, None, False)
+        assert dq._version > before[0] and dkv._version > before[1]
+        before = dq._version, dkv._version
+        with mode():
+            M.flash_attn_backward(q, kv, out, lse, dout, dq, dkv, 0.1, ring=M.LocalRing((1,), 0, [kv]))
+            inside = torch.empty_like(q)                 # an inference tensor keeps no count
+            M._flash_attn_backward(dout, q, kv[0], kv[1], out, lse, inside, dkv[0], dkv[1], 0.0, 0.1, False, -1, -1, 0.0,
+                                   None, False)
+        assert dq._version > before[0] and dkv._version > before[1]
