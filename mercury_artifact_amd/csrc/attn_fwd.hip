@@ -60,8 +60,9 @@ struct FwdParams {
   int heads_per_xcd; // (batch, head) pairs per XCD when they divide evenly, else 0
 };
 
-// KK = k-steps of 16 head-dim values in S^T: 8 computes on all 128 on-chip columns; 4 is the instantiation for head
-// dimensions up to 64, which leaves out the MFMAs that would only see the zero columns (half of both products).
+// KK = k-steps of 16 head-dim values in S^T: 8 computes on all 128 on-chip columns; 4 and 6 are the instantiations for
+// head dimensions up to 64 and up to 96, which leave out the MFMAs that would only see the zero columns (half and a
+// quarter of both products).
 //
 // KS = key groups of a workgroup.  With one group the eight wavefronts hold 8 x 32 Q rows and all visit every key
 // tile.  A launch of few (batch, head, 256-row) items leaves most CUs without a workgroup then, and its time is the
@@ -72,7 +73,7 @@ struct FwdParams {
 // of four, of 64-key tiles (KS = 2) or 32-key tiles (KS = 4): 128 KB of LDS in all three cases.
 template <bool CAUSAL, int KK = 8, int KS = 1>
 __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdParams p) {
-  static_assert(KK == 8 || KK == 4, "128 or 64 on-chip head-dim columns");
+  static_assert(KK == 8 || KK == 6 || KK == 4, "128, 96 or 64 on-chip head-dim columns");
   static_assert(KS == 1 || KS == 2 || KS == 4, "key groups");
   constexpr int DB = KK / 2;        // blocks of 32 head-dim values in O^T
   constexpr int RG = kWaves / KS;   // row groups of 32
@@ -642,8 +643,9 @@ int key_groups(const FwdParams& p, bool causal) {
   if ((int64_t)p.Sc * p.k_ss >= (1 << 29) || (int64_t)p.Sc * p.v_ss >= (1 << 29)) return 1;
   struct Cost { float fixed, step, busy; };
   static constexpr Cost kCost128[3] = {{7.0f, 1.10f, 0.80f}, {6.5f, 1.19f, 0.90f}, {5.2f, 0.81f, 0.49f}};
+  static constexpr Cost kCost96[3] = {{6.5f, 1.07f, 0.49f}, {6.2f, 1.08f, 0.58f}, {4.9f, 0.76f, 0.30f}};
   static constexpr Cost kCost64[3] = {{6.0f, 1.05f, 0.17f}, {6.0f, 0.98f, 0.27f}, {4.7f, 0.72f, 0.12f}};
-  const Cost* cost = p.D <= 64 ? kCost64 : kCost128;
+  const Cost* cost = p.D <= 64 ? kCost64 : p.D <= 96 ? kCost96 : kCost128;
   int best = 1;
   float best_time = 0.f;
   for (int i = 0; i < 3; ++i) {
@@ -697,6 +699,7 @@ int attn_fwd_bf16(const void* q, const void* k, const void* v, void* out, float*
   const bool causal = mask == MHIP_MASK_CAUSAL;
   const int groups = key_groups(p, causal);
   if (D <= 64) launch_fwd<4>(p, causal, groups, stream);        // half the on-chip columns, half the MFMAs
+  else if (D <= 96) launch_fwd<6>(p, causal, groups, stream);   // three quarters of both
   else launch_fwd<8>(p, causal, groups, stream);
   return launch_status();
 }

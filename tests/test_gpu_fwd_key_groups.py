@@ -16,7 +16,7 @@ LAUNCHES = {4: (1, 3, 1), 2: (2, 64, 8), 1: (4, 64, 8)}
 EDGES = [
     # Sq, Sc, D: rows around 32, 64, 128, 256, keys around 32, 64, 128, 256 and the rings' wrap
     (1, 1, 128), (31, 32, 128), (64, 33, 128), (65, 127, 64), (129, 128, 128), (130, 129, 40), (255, 257, 128),
-    (257, 520, 64), (192, 700, 96),
+    (257, 520, 64), (192, 700, 96), (33, 65, 72), (129, 257, 96),
 ]
 
 
