@@ -44,8 +44,6 @@ constexpr int kOStride = kD + 8;   // epilogue staging of O, bf16 elements per r
 constexpr int kNoColumn = 0x7fff0000;  // vector offset that is out of every descriptor's range (spans stay below 2^31,
                                        // and so does the scalar tile offset added to it: no 32-bit wrap)
 constexpr int kFragDepth = 4;      // LDS operand reads in flight ahead of the MFMAs (6 and 8 measure the same)
-constexpr int kEarlyPairs = 2;     // exponential pairs of a tile computed inside the matrix phase (4 .. 8: 1-3 % slower)
-constexpr int kEarlyStep = 2;      // matrix-phase slots between them
 
 struct FwdParams {
   const uint16_t* q; const uint16_t* k; const uint16_t* v;
@@ -280,7 +278,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
   // The first kEarlyPairs pairs are computed inside the matrix phase, between the O^T MFMAs: measured with
   // cycle counters the vector phase is the longer of the two (1314 against 1265 ticks per 64-key tile), and
   // two pairs moved over make the step 3 % faster (four and more slow the matrix phase down by as much as
-  // they shorten the other).  A pair may overwrite the P^T operand of k-step ks only after the last MFMA of
+  // they shorten the other; on 64 columns, where it has half the MFMAs, six do).  A pair may overwrite the P^T operand of k-step ks only after the last MFMA of
   // that k-step has been issued.
   float rs = 0.f;
   auto sm_pair = [&](int idx) {
@@ -320,10 +318,12 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
   };
   // slot of the matrix phase after which early pair idx runs: k-step idx / 4 of the tile before is read by the
   // O^T slots kSlotsS + DB (idx / 4) .. + DB - 1, and the pairs are spread two slots apart behind that
-  constexpr int kEarlyGap = MB * DB >= 4 ? kEarlyStep : 1;
+  constexpr bool kShortMatrix = KS == 1 && KK < 8;
+  constexpr int kEarlyPairs = KS == 1 && KK == 4 ? 6 : 2;
+  constexpr int kEarlyGap = kEarlyPairs > 2 || MB * DB < 4 ? 1 : 2;
   auto early_slot = [](int idx) { return kSlotsS + DB + kEarlyGap * idx; };
-  static_assert(kEarlyPairs <= 4 && DB + kEarlyGap * (kEarlyPairs - 1) < kSlotsO,
-                "the early pairs have to fit behind the O^T slots of k-step 0");
+  static_assert(DB + kEarlyGap * (kEarlyPairs - 1) < kSlotsO && (kEarlyPairs <= 4 || (DB + kEarlyGap * 4 >= 2 * DB && kEarlyPairs <= 8)),
+                "the early pairs have to fit behind the O^T slots of their k-steps");
   auto sm_tile = [&]() {
 #pragma unroll
     for (int idx = kEarlyPairs; idx < 8 * MB; ++idx) sm_pair(idx);
@@ -369,6 +369,15 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
         const int db = i - (kSlotsS + kSlotsO - DB);
         v_a[db][0] += v_step;
         v_a[db][1] += v_step;
+      }
+      // On fewer than 128 columns the vector phase, which is the same length, would hold up a matrix phase that is half or
+      // three quarters as long: there the tile copies go out between the S^T MFMAs (K(t) and V(t-1) are read by then,
+      // see the main loop).  With that and the early pairs 2048 x 2048 H24 takes 33.3 instead of 39.6 us at D 64 and 41.9
+      // instead of 43.9 at D 96, 4096 x 4096 H32 131.6 / 145.4 and 174.7 / 182.8; on 128 columns it is 1 % slower.
+      if (kShortMatrix && i < kSlotsS && i % (kSlotsS / 4) == 1) {
+        const int u = i / (kSlotsS / 4);
+        if (u < 2) copy16_to_lds(krs, lds_base + (t & 3) * kTile + u * 1024, kvoff[u % kCpy], tile_offset(t + 4, k_tile_bytes));
+        else copy16_to_lds(vrs, lds_base + kVBase + ((t + 3) & 3) * kTile + (u - 2) * 1024, vvoff[u % kCpy], tile_offset(t + 3, v_tile_bytes));
       }
       // S^T(t+1) is complete after its last slot; its softmax starts here, in the shadow of the O^T MFMAs
       if (i == kSlotsS) sm_mask(t + 1);
@@ -431,9 +440,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
     }
     // Phase p of the main loop: group A (waves 0-3) runs the matrix phase of tile p/2 on even p and its
     // vector phase on odd p; group B does the same one phase later.  K(t) and V(t) live in stage t % 4 of
-    // their rings.  In the vector phase of tile t every wavefront starts its share of the copies of K(t+4)
+    // their rings.  In the vector phase of tile t (on fewer than 128 columns in the matrix phase before it, when the
+    // other group is past its matrix phase of tile t-1 too) every wavefront starts its share of the copies of K(t+4)
     // (over K(t), last read in the matrix phase of tile t-1) and V(t+3) (over V(t-1)), and before the
-    // barrier that ends the phase waits for the copies it started one tile earlier: those are then visible
+    // barrier that ends the vector phase waits for the copies it started one tile earlier: those are then visible
     // to every wavefront two barriers later, in time for first_frags of K(t+3) and the matrix phase of V(t+2).
     if (group_b) __builtin_amdgcn_s_barrier();
     for (int t = 0; t + 1 < ntiles; ++t) {
@@ -445,8 +455,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
       // ---- vector phase: softmax(t+1), copies of the tiles ahead ---------------------------------------------
       asm volatile("" : "+v"(s[0]), "+v"(s[MB - 1]));   // keeps the exponentials behind the barrier
       sm_tile();
-      copy_k(t + 4, t & 3);
-      copy_v(t + 3, (t + 3) & 3);
+      if (!kShortMatrix) {
+        copy_k(t + 4, t & 3);
+        copy_v(t + 3, (t + 3) & 3);
+      }
       if (t + 2 < ntiles) first_frags();                        // K(t+2), for the next matrix phase
       asm volatile("s_waitcnt vmcnt(4)" ::: "memory");          // the four copies of one tile ago are done
       __builtin_amdgcn_s_barrier();
@@ -635,16 +647,16 @@ void launch_fwd(FwdParams& p, bool causal, int groups, hipStream_t stream) {
 // `step` us, plus `busy` us times the share of the CUs at work (clock and L2).  Fitted to launches of 4 .. 2048
 // workgroups over 64 .. 4096 keys, which it gives to within 15 %; measured (us, groups 1 / 2 / 4):
 //     B1 H4  256 x 256      11.2 /  9.2 /  7.8      B4 H5   512 x 512     16.1 / 12.5 / 10.7
-//     B1 H32 1024 x 1024    28.8 / 22.6 / 29.6      B2 H16 1237 x 1237    33.2 / 41.8 / 46.6  (D 80)
+//     B1 H32 1024 x 1024    28.8 / 22.6 / 29.6      B2 H16 1237 x 1237    25.2 / 35.4 / 38.7  (D 80)
 //     B1 H1  4096 x 4096    70.3 / 45.6 / 33.8      B1 H20 4096 x 4096     187 /  176 /  200
-//     B1 H32 4096 x 4096     228 /  255 /  357      B2 H12 1500 x 1500    36.8 / 21.8 / 29.0  (D 64, causal)
+//     B1 H32 4096 x 4096     228 /  255 /  357      B2 H12 1500 x 1500    24.2 / 18.5 / 24.6  (D 64, causal)
 // The split kernel puts whole tiles out of range through 32-bit offsets, which asks for spans below 2^30 bytes.
 int key_groups(const FwdParams& p, bool causal) {
   if ((int64_t)p.Sc * p.k_ss >= (1 << 29) || (int64_t)p.Sc * p.v_ss >= (1 << 29)) return 1;
   struct Cost { float fixed, step, busy; };
   static constexpr Cost kCost128[3] = {{7.0f, 1.10f, 0.80f}, {6.5f, 1.19f, 0.90f}, {5.2f, 0.81f, 0.49f}};
-  static constexpr Cost kCost96[3] = {{6.5f, 1.07f, 0.49f}, {6.2f, 1.08f, 0.58f}, {4.9f, 0.76f, 0.30f}};
-  static constexpr Cost kCost64[3] = {{6.0f, 1.05f, 0.17f}, {6.0f, 0.98f, 0.27f}, {4.7f, 0.72f, 0.12f}};
+  static constexpr Cost kCost96[3] = {{6.5f, 0.62f, 0.66f}, {6.2f, 1.08f, 0.58f}, {4.9f, 0.76f, 0.30f}};
+  static constexpr Cost kCost64[3] = {{6.0f, 0.65f, 0.30f}, {6.0f, 0.98f, 0.27f}, {4.7f, 0.72f, 0.12f}};
   const Cost* cost = p.D <= 64 ? kCost64 : p.D <= 96 ? kCost96 : kCost128;
   int best = 1;
   float best_time = 0.f;
