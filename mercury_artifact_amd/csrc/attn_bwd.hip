@@ -75,9 +75,11 @@ struct TileMap {
   int heads_per_xcd;   // (batch, stationary head) pairs per XCD when they divide evenly, else 0
 };
 
-// KK = k-steps of 16 head-dim values in T1 / T2: 8 computes on all 128 on-chip columns; 4 is the instantiation for head
-// dimensions up to 64, which leaves out the MFMAs, accumulators and fragments of the zero columns.  The vector work of a
-// tile is the same, so a T1 / T2 slot carries twice of it: 4096 x 4096, H32, D 64 takes 473 us instead of 654.
+// KK = k-steps of 16 head-dim values in T1 / T2: 8 computes on all 128 on-chip columns; 4 and 6 are the instantiations for
+// head dimensions up to 64 and up to 96, which leave out the MFMAs, accumulators and fragments of the zero columns.  The
+// vector work of a tile is the same, so a T1 / T2 slot carries more of it: 4096 x 4096, H32 takes 473 us instead of 654 at
+// D 64 and 616 instead of 709 at D 96, 1237 x 1237, B2 H16/8, D 80 78.1 instead of 88.6, 512 x 512, B4 H5, D 96 16.9
+// instead of 18.5; results bit-identical.
 //
 // WAVES = 8 wavefronts of 32 stationary rows (dQ: two per SIMD) or 4 (one per SIMD).  PREPARED: lse2 and delta of the
 // query rows are in the workspace already; otherwise the dQ pass works them out.
@@ -283,7 +285,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
   // Tile t lives in stage t % 4 and is processed as two halves of 32 streamed rows.  Per tile the matrix
-  // pipe sees one unbroken sequence of MFMA slots in four phases (half as many slots in each on 64 columns):
+  // pipe sees one unbroken sequence of MFMA slots in four phases (half as many slots in each on 64 columns, three quarters on 96):
   //   P0  T1 / T2 of (t, second half)      16 slots, each carrying P / dS of one register of (t, first half)
   //   P1  accumulate (t, first half)       16 slots (8 for dQ)
   //   P2  T1 / T2 of (t+1, first half)     16 slots, each carrying P / dS of one register of (t, second half)
@@ -299,7 +301,8 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   constexpr int kT = 2 * KK;                               // slots of a T1 / T2 phase
   constexpr int kAcc = DQ ? 2 * DB : 4 * DB;               // slots of an accumulate phase
   constexpr int kP1 = kT, kP2 = kT + kAcc, kP3 = 2 * kT + kAcc, kSlots = 2 * (kT + kAcc);
-  constexpr int kVec = 16 / kT;                            // steps of the vector pipeline per slot
+  // The 16 steps of the vector pipeline are spread over the slots of a T1 / T2 phase: slot i runs steps vec0(i) .. vec0(i + 1) - 1.
+  auto vec0 = [](int i) -> int { return i * 16 / kT; };
   typedef __attribute__((address_space(3))) const f32x4* lds_f32x4;
   // LDS addresses of the operand reads.  rm_a / tr_a hold, per lane, the addresses inside ONE tile's stage and are
   // moved on to the next stage in place, each at a point of the slot sequence where no read of its kind is due
@@ -409,8 +412,8 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   // steps 16 .. of the vector pipeline, behind the T1 / T2 phase, run in the first slots of the accumulate phase
   auto vector_tail = [&](int i, f32x16& c1, f32x16& c2, int mb) {
 #pragma unroll
-    for (int v = 0; v < kVec; ++v)
-      if (i * kVec + v < (DQ ? 4 : 8)) vector_slot(16 + i * kVec + v, c1, c2, mb);
+    for (int v = vec0(i); v < vec0(i + 1); ++v)
+      if (v < (DQ ? 4 : 8)) vector_slot(16 + v, c1, c2, mb);
   };
   auto acc_mfma = [&](int i, const bf16x8& a) {
     const int m = DQ ? i : (i >> 1);
@@ -427,7 +430,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     if (s < kP3) return read_rm(0, s - kP2);
     return read_acc(1, s - kP3);
   };
-  static_assert(kP2 - kDepth >= kT && KK % kDepth == 0 && 2 * DB % kDepth == 0, "rm_a moves in the last kDepth slots of P0, tr_a in the last kDepth slots of P3");
+  static_assert(kP2 - kDepth >= kT && kAcc >= kDepth, "rm_a moves in the last kDepth slots of P0, tr_a in the last kDepth slots of P3");
 
   // Stationary rows: read straight into the fragment layout every load instruction would touch 32 rows (24 such loads
   // per wavefront in the dQ pass, one wait for all of them and the tiles).  They are copied to LDS instead, four whole
@@ -569,19 +572,19 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     // byte distance from this tile's stage to the next tile's, and from that one to the one after
     const int step1 = ((t + 1) & 3) == 0 ? -3 * kStageBytes : kStageBytes;
     const int step2 = ((t + 2) & 3) == 0 ? -3 * kStageBytes : kStageBytes;
-    static_assert(kSlots % kDepth == 0 && kT % kDepth == 0 && kAcc % kDepth == 0, "the ring position is the slot number modulo its depth");
+    static_assert(kSlots % kDepth == 0, "the ring position is the slot number modulo its depth");
     mask_half(ta1, c0);
 #pragma unroll
     for (int i = 0; i < kT; ++i) {                       // P0, carrying the copies of tile t+3
       t_mfma(i, ring[i % kDepth], tb1, tb2);
 #pragma unroll
-      for (int v = 0; v < kVec; ++v) vector_slot(i * kVec + v, ta1, ta2, 0);
+      for (int v = vec0(i); v < vec0(i + 1); ++v) vector_slot(v, ta1, ta2, 0);
 #pragma unroll
       for (int piece = i; piece < kCopiesPerTile; piece += kT) copy_piece(piece, (t + 3) & 3);
       ring[i % kDepth] = read_slot(i + kDepth);
       if (i >= kT - kDepth) {                            // the last read of this tile's T1 / T2 operands is out: on to the next
 #pragma unroll
-        for (int j = 0; j < KK / kDepth; ++j) rm_a[(i - (kT - kDepth)) * (KK / kDepth) + j] += step1;
+        for (int a = (i - (kT - kDepth)) * KK / kDepth; a < (i + 1 - (kT - kDepth)) * KK / kDepth; ++a) rm_a[a] += step1;
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -601,7 +604,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     for (int i = 0; i < kT; ++i) {                       // P2
       t_mfma(i, ring[(kP2 + i) % kDepth], ta1, ta2);
 #pragma unroll
-      for (int v = 0; v < kVec; ++v) vector_slot(i * kVec + v, tb1, tb2, 1);
+      for (int v = vec0(i); v < vec0(i + 1); ++v) vector_slot(v, tb1, tb2, 1);
       ring[(kP2 + i) % kDepth] = read_slot(kP2 + i + kDepth);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -614,10 +617,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
       ring[(kP3 + i) % kDepth] = read_slot(kP3 + i + kDepth);
       if (i >= kAcc - kDepth) {                          // the last transposed read of this tile has been issued
 #pragma unroll
-        for (int j = 0; j < 2 * DB / kDepth; ++j) {
-          const int a = (i - (kAcc - kDepth)) * (2 * DB / kDepth) + j;
-          tr_a[a >> 1][a & 1] += step1;
-        }
+        for (int a = (i - (kAcc - kDepth)) * 2 * DB / kDepth; a < (i + 1 - (kAcc - kDepth)) * 2 * DB / kDepth; ++a) tr_a[a >> 1][a & 1] += step1;
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -885,7 +885,7 @@ int64_t partial_bytes(int B, int S, int H, int D, int tensors, int splits) {
 Plan plan_block(int B, int Sq, int Sc, int Hq, int Hkv, int D, bool causal) {
   Plan best = {false, 1, 1};
   if (Sq == 0 || Sc == 0 || B == 0) return best;
-  const bool narrow = D <= 64;
+  const bool narrow = D <= 64;      // 96 columns: the costs of 128, of which both forms save the same 12 %
   const Cost dq8 = narrow ? Cost{6.f, 0.95f, 0.45f} : Cost{7.f, 1.45f, 0.75f};
   const Cost dkv = narrow ? Cost{6.f, 0.75f, 0.25f} : Cost{7.f, 1.15f, 0.55f};
   const Cost both = narrow ? Cost{6.f, 0.75f, 0.12f} : Cost{7.f, 1.15f, 0.29f};
@@ -1017,6 +1017,7 @@ int bwd_block(const void* dout, const void* q, const void* k, const void* v,
 
   const Plan plan = plan_block(B, Sq, Sc, Hq, Hkv, D, causal);
   if (D <= 64) causal ? launch_bwd<true, 4>(p, plan, partial, st) : launch_bwd<false, 4>(p, plan, partial, st);
+  else if (D <= 96) causal ? launch_bwd<true, 6>(p, plan, partial, st) : launch_bwd<false, 6>(p, plan, partial, st);
   else causal ? launch_bwd<true, 8>(p, plan, partial, st) : launch_bwd<false, 8>(p, plan, partial, st);
   return launch_status();
 }

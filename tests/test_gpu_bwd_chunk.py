@@ -21,7 +21,7 @@ def _close(name, got, ref):
 
 
 @pytest.mark.parametrize("W,S,Hq,Hkv,D", [(1, 300, 2, 2, 128), (2, 129, 4, 2, 64), (3, 257, 3, 1, 40), (4, 64, 2, 2, 128),
-                                           (2, 400, 8, 1, 128)])
+                                           (2, 400, 8, 1, 128), (2, 193, 4, 2, 96)])
 @pytest.mark.parametrize("dq_dtype,keep", [(torch.bfloat16, True), (torch.float32, True), (torch.bfloat16, False)])
 def test_backward_step_carries_the_sums(W, S, Hq, Hkv, D, dq_dtype, keep):
     import mercury_artifact_amd as M
@@ -71,23 +71,23 @@ def _block(B, Sq, Sc, Hq, Hkv, D, causal):
     assert (delta.cpu() - want).abs().max() <= 1e-4
 
 
-@pytest.mark.parametrize("D", [8, 56, 64, 72])
+@pytest.mark.parametrize("D", [8, 56, 64, 72, 96, 104])
 @pytest.mark.parametrize("Sq,Sc,Hq,Hkv,causal", [(1, 1, 2, 1, False), (65, 129, 4, 2, False), (257, 63, 2, 2, True),
                                                  (320, 400, 3, 3, True), (130, 700, 2, 1, False)])
 def test_backward_block_on_narrow_heads(D, Sq, Sc, Hq, Hkv, causal):
-    """Both sides of the line between the 64-column and the 128-column kernels, ragged rows and keys, several turns of
+    """Both sides of the lines between the 64-, 96- and 128-column kernels, ragged rows and keys, several turns of
     the tile ring; launches this small run both passes side by side."""
     _block(2, Sq, Sc, Hq, Hkv, D, causal)
 
 
-@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("D", [64, 80, 128])
 @pytest.mark.parametrize("Sq,Sc,causal", [(130, 129, False), (257, 64, True), (300, 385, True)])
 def test_backward_block_in_two_launches(D, Sq, Sc, causal):
     """Enough heads to fill the chip with either pass: one launch each, dQ with eight wavefronts."""
     _block(2, Sq, Sc, 128, 128, D, causal)
 
 
-@pytest.mark.parametrize("D", [40, 128])
+@pytest.mark.parametrize("D", [40, 88, 128])
 @pytest.mark.parametrize("B,Sq,Sc,Hq,Hkv,causal", [(1, 321, 130, 8, 1, False), (1, 700, 777, 8, 1, True), (2, 513, 400, 12, 2, True),
                                                    (1, 130, 3000, 1, 1, False), (1, 3000, 130, 1, 1, True)])
 def test_backward_block_with_shared_tiles(B, Sq, Sc, Hq, Hkv, causal, D):
