@@ -132,7 +132,7 @@ def test_fp8_block_with_a_dominant_first_key(gap_nats):
     _check(out, lse, ref_a, ref_a, f"fp8 sink {gap_nats}", p_bound, check_b=False)
 
 
-@pytest.mark.parametrize("D,causal", [(64, False), (48, True), (16, False), (112, True)])
+@pytest.mark.parametrize("D,causal", [(64, False), (48, True), (16, False), (112, True), (80, False), (96, True)])
 def test_fp8_block_smaller_head_dims(D, causal):
     """Head dimensions below 128 (multiples of 16) through the e4m3 kernel: q, k, v and out are COLUMN slices of
     128-wide tensors whose other columns hold the e4m3 NaN code (inputs) or a sentinel (output), so a kernel that
