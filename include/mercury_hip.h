@@ -66,7 +66,7 @@ const char* mhip_error_string(int code);
  * they may be written by earlier work on the stream, and a captured graph uses the values present
  * at replay); NULL means 1.  They must be positive and finite (not checked: the values never
  * reach the host).  Ignored for MHIP_BF16.
- * Head dimension: MHIP_BF16 any multiple of 8 up to 128 (the kernel computes on 128 columns, on 64 for D <= 64;
+ * Head dimension: MHIP_BF16 any multiple of 8 up to 128 (the kernels compute on 64, 96 or 128 columns;
  * the missing ones are zeros that exist only on chip -- no padded copy, no extra memory traffic -- and the K / V
  * span Sc * stride of one (batch, head) must stay below 2^30 bytes, MHIP_EUNSUPPORTED beyond); MHIP_E4M3 any
  * multiple of 16 up to 128, in the same way.  MHIP_EHEADDIM otherwise.

@@ -27,8 +27,6 @@ typedef __attribute__((__vector_size__(8 * sizeof(int)))) int i32x8;
 typedef __attribute__((__vector_size__(2 * sizeof(int)))) int i32x2;
 
 constexpr int kD = 128;
-constexpr int kWaves = 8;
-constexpr int kBM = kWaves * 32;
 constexpr int kBN = 128;              // keys per tile
 constexpr int kTileBytes = kBN * kD;  // 16384: one K or V tile in LDS, 128 rows of 128 bytes
 constexpr int kStages = 4;
@@ -60,8 +58,16 @@ __device__ __forceinline__ constexpr int swz8(int row) { return (((row >> 1) & 3
 // and 2 k-steps of 64 in S^T).  The vector work of a tile stays, which bounds the kernel: 4096 x 4096 H32 takes 112 us
 // instead of 134 at D 64 and 136 instead of 142 at D 96, causal 8192 x 8192 H16/4 D 64 118 instead of 142, 512 x 512 H4
 // D 64 11.0 instead of 12.6; results the same.
-template <bool CAUSAL, int DB>
-__global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_fp8_d128(const Fp8Params p) {
+//
+// WAVES = wavefronts of 32 Q rows in a workgroup: eight, two per SIMD, or four where a launch of eight leaves half of the
+// CUs without a workgroup.  The vector unit bounds a tile step, so one wavefront per SIMD takes less time
+// for it: 256 x 256 H4 7.6 us instead of 9.1, 2048 x 2048 H16 28.2 / 37.0, 4096 x 4096 H2 47.6 / 66.3, causal 1024 x 1024
+// H32/8 17.2 / 22.5; results the same.
+template <bool CAUSAL, int DB, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const Fp8Params p) {
+  static_assert(WAVES == 8 || WAVES == 4, "two wavefronts per SIMD or one");
+  constexpr int kBM = WAVES * 32;
+  constexpr int kCpy = 16 / WAVES;              // copy instructions per wavefront for one 16 KB tile
   static_assert(DB >= 2 && DB <= 4, "64, 96 or 128 on-chip head-dim columns");
   constexpr int KK = (DB + 1) / 2;              // k-steps of 64 head-dim values in S^T
   __shared__ __attribute__((aligned(16))) unsigned char smem[2 * kStages * kTileBytes];
@@ -116,17 +122,17 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_fp8_d128(const Fp8Par
   const int my_q = q0 + wave * 32 + ln;
   i32x8 qf[KK];    // loaded after the first tile copies are under way, so that one wait covers both latencies
 
-  // ---- global -> LDS copies: wavefront w copies rows 16w .. 16w+15 of every K and V tile with two
-  // instructions of 1 KB; lane l of instruction u lands at row 16w + 8u + l/8, chunk position l%8, and
+  // ---- global -> LDS copies: wavefront w copies 8 kCpy rows of every K and V tile, 1 KB per
+  // instruction; lane l of instruction u lands at row 8 (kCpy w + u) + l/8, chunk position l%8, and
   // fetches the chunk that lives there.  Rows past the end of the chunk arrive as zeros. ---------------------
   // Chunks past the head dimension (D < 128) carry an offset that is out of range for every tile and arrive as
   // zeros too: a tile in LDS always has 128 columns, at no cost in memory traffic.
   const u32x4 krs = rsrc_words(p.k + b * p.k_sb + hk * p.k_sh, (uint32_t)((int64_t)(p.Sc - 1) * p.k_ss + p.D));
   const u32x4 vrs = rsrc_words(p.v + b * p.v_sb + hk * p.v_sh, (uint32_t)((int64_t)(p.Sc - 1) * p.v_ss + p.D));
-  int kvoff[2], vvoff[2];
+  int kvoff[kCpy], vvoff[kCpy];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int row = 16 * wave + 8 * u + (lane >> 3);
+  for (int u = 0; u < kCpy; ++u) {
+    const int row = 8 * (kCpy * wave + u) + (lane >> 3);
     const int chunk = (lane & 7) ^ swz8(row);
     const bool real = chunk * 16 < p.D;
     kvoff[u] = real ? (int)(row * p.k_ss) + chunk * 16 : kNoColumn;
@@ -134,12 +140,12 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_fp8_d128(const Fp8Par
   }
   const int k_tile_bytes = (int)(kBN * p.k_ss);
   const int v_tile_bytes = (int)(kBN * p.v_ss);
-  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem + wave * 2048;
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem + wave * (kCpy * 1024);
   auto copy_tile = [&](int t, int stage) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u) copy16_to_lds(krs, lds_base + stage * kTileBytes + u * 1024, kvoff[u], t * k_tile_bytes);
+    for (int u = 0; u < kCpy; ++u) copy16_to_lds(krs, lds_base + stage * kTileBytes + u * 1024, kvoff[u], t * k_tile_bytes);
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < kCpy; ++u)
       copy16_to_lds(vrs, lds_base + kVBase + stage * kTileBytes + u * 1024, vvoff[u], t * v_tile_bytes);
   };
 
@@ -279,7 +285,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_fp8_d128(const Fp8Par
     for (int ks = 0; ks < KK; ++ks) asm volatile("" : "+v"(qf[ks]));
   }
   for (int t = 0; t < ntiles; ++t) {
-    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");      // two tiles of four copies each
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(4 * kCpy) : "memory");      // two tiles of 2 kCpy copies each
     __builtin_amdgcn_s_barrier();
     copy_tile(t + 3, (t + 3) & 3);
     const unsigned char* ks_ = smem + (t & 3) * kTileBytes;
@@ -364,6 +370,13 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_fp8_d128(const Fp8Par
   }
 }
 
+template <int DB, int WAVES>
+void launch_fp8(const Fp8Params& p, bool causal, hipStream_t stream) {
+  const dim3 grid(p.per_xcd * 8), block(WAVES * 64);
+  if (causal) hipLaunchKernelGGL((attn_fwd_fp8_d128<true, DB, WAVES>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((attn_fwd_fp8_d128<false, DB, WAVES>), grid, block, 0, stream, p);
+}
+
 }  // namespace
 
 int attn_fwd_fp8(const void* q, const void* k, const void* v, void* out, float* lse,
@@ -380,16 +393,18 @@ int attn_fwd_fp8(const void* q, const void* k, const void* v, void* out, float* 
   p.o_sb = st[9]; p.o_ss = st[10]; p.o_sh = st[11];
   p.scale = scale;
   p.q_descale = q_descale; p.k_descale = k_descale; p.v_descale = v_descale;
-  p.nq_tiles = (Sq + kBM - 1) / kBM;
+  // Four wavefronts while the launch has at most 256 workgroups of 128 rows: twice the CUs at work.  With more, they
+  // would take turns on the CUs.
+  const bool wide = (int64_t)B * Hq * ((Sq + 127) / 128) > 256;
+  const int rows = wide ? 256 : 128;
+  p.nq_tiles = (Sq + rows - 1) / rows;
   p.total = B * Hq * p.nq_tiles;
   p.per_xcd = (p.total + 7) / 8;
   p.heads_per_xcd = (B * Hq) % 8 == 0 ? (B * Hq) / 8 : 0;
-  const dim3 grid(p.per_xcd * 8), block(kWaves * 64);
   const bool causal = mask == MHIP_MASK_CAUSAL;
-  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, stream, p); };
-  if (D <= 64) launch(causal ? attn_fwd_fp8_d128<true, 2> : attn_fwd_fp8_d128<false, 2>);
-  else if (D <= 96) launch(causal ? attn_fwd_fp8_d128<true, 3> : attn_fwd_fp8_d128<false, 3>);
-  else launch(causal ? attn_fwd_fp8_d128<true, 4> : attn_fwd_fp8_d128<false, 4>);
+  if (D <= 64) wide ? launch_fp8<2, 8>(p, causal, stream) : launch_fp8<2, 4>(p, causal, stream);
+  else if (D <= 96) wide ? launch_fp8<3, 8>(p, causal, stream) : launch_fp8<3, 4>(p, causal, stream);
+  else wide ? launch_fp8<4, 8>(p, causal, stream) : launch_fp8<4, 4>(p, causal, stream);
   return launch_status();
 }
 

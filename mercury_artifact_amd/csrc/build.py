@@ -23,7 +23,9 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall",
 # attn_bwd.hip keeps 128 accumulator registers per lane for dK^T / dV^T and works on T1 / T2 with the vector
 # unit: with MFMA results in arithmetic registers (and only the stationary operands in accumulation
 # registers) there are no copies between the two register files in its main loop.
-EXTRA_FLAGS = {"attn_bwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# attn_fwd_fp8.hip: the form with one wavefront per SIMD would get accumulation registers and copy every score out of them.
+VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
+EXTRA_FLAGS = {"attn_bwd.hip": VGPR_FORM, "attn_fwd_fp8.hip": VGPR_FORM}
 
 
 def _run(cmd):

@@ -165,6 +165,24 @@ def test_fp8_block_smaller_head_dims(D, causal):
     assert (ow[..., :off] == 7.0).all()
 
 
+@pytest.mark.parametrize("D", [64, 96, 128])
+@pytest.mark.parametrize("Sq,Sc,H,causal", [(129, 260, 128, False), (129, 260, 129, False), (257, 130, 88, True), (257, 700, 80, True)])
+def test_fp8_block_on_both_workgroup_sizes(Sq, Sc, H, causal, D):
+    """Both sides of the line between workgroups of four and of eight wavefronts (256 workgroups of 128 rows), rows just
+    past a multiple of either's."""
+    import mercury_artifact_amd as M
+
+    print(f"fp8 Sq{Sq} Sc{Sc} H{H} D{D} causal={causal}", flush=True)
+    (q, k, v), (qq, kq, vq), (sq, sk, sv) = _quantised(1, Sq, Sc, H, H, seed=D + H, D=D)
+    scale = D ** -0.5
+    deq = (O.dequantize(qq, sq), O.dequantize(kq, sk), O.dequantize(vq, sv))
+    out, lse = M.attn_fwd_block(qq.cuda(), kq.cuda(), vq.cuda(), scale, causal=causal, q_descale=sq.cuda(),
+                                k_descale=sk.cuda(), v_descale=sv.cuda())
+    torch.cuda.synchronize()
+    ref_a = O.block_attention(*deq, scale, causal=causal)
+    _check(out, lse, ref_a, ref_a, f"fp8 H{H}", O.e4m3_p_rounding_bound(*deq, scale, causal=causal), check_b=False)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("shape", [(4, 300, 3, 128), (1003,), (7,), (2, 4099)])
 def test_fp8_product_quantiser_bits(dtype, shape):
