@@ -394,14 +394,17 @@ int attn_fwd_fp8(const void* q, const void* k, const void* v, void* out, float* 
   p.scale = scale;
   p.q_descale = q_descale; p.k_descale = k_descale; p.v_descale = v_descale;
   // Four wavefronts while the launch has at most 256 workgroups of 128 rows: twice the CUs at work.  With more, they
-  // would take turns on the CUs.
-  const bool wide = (int64_t)B * Hq * ((Sq + 127) / 128) > 256;
+  // take turns on the CUs (us, eight / four: 2048 x 2048 H16, 256 of them, 37.0 / 28.2; 2176 x 2176 H16 39.2 / 54.3;
+  // 2048 x 2048 H32 42.8 / 53.2).  Under the causal mask of a square or tall block the longest workgroups hold up the
+  // launch until there is twice as much work (2048 x 2048 H20 38.4 / 28.0, H32, 512 workgroups, 39.0 / 33.1, H40
+  // 40.1 / 46.1; 4096 x 2048 H16 37.8 / 28.1).
+  const bool causal = mask == MHIP_MASK_CAUSAL;
+  const bool wide = (int64_t)B * Hq * ((Sq + 127) / 128) > (causal && Sc <= Sq ? 512 : 256);
   const int rows = wide ? 256 : 128;
   p.nq_tiles = (Sq + rows - 1) / rows;
   p.total = B * Hq * p.nq_tiles;
   p.per_xcd = (p.total + 7) / 8;
   p.heads_per_xcd = (B * Hq) % 8 == 0 ? (B * Hq) / 8 : 0;
-  const bool causal = mask == MHIP_MASK_CAUSAL;
   if (D <= 64) wide ? launch_fp8<2, 8>(p, causal, stream) : launch_fp8<2, 4>(p, causal, stream);
   else if (D <= 96) wide ? launch_fp8<3, 8>(p, causal, stream) : launch_fp8<3, 4>(p, causal, stream);
   else wide ? launch_fp8<4, 8>(p, causal, stream) : launch_fp8<4, 4>(p, causal, stream);

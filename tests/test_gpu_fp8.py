@@ -166,10 +166,11 @@ def test_fp8_block_smaller_head_dims(D, causal):
 
 
 @pytest.mark.parametrize("D", [64, 96, 128])
-@pytest.mark.parametrize("Sq,Sc,H,causal", [(129, 260, 128, False), (129, 260, 129, False), (257, 130, 88, True), (257, 700, 80, True)])
+@pytest.mark.parametrize("Sq,Sc,H,causal", [(129, 260, 128, False), (129, 260, 129, False), (257, 130, 88, True), (257, 700, 80, True),
+                                            (257, 257, 170, True), (257, 257, 171, True), (129, 130, 129, True)])
 def test_fp8_block_on_both_workgroup_sizes(Sq, Sc, H, causal, D):
-    """Both sides of the line between workgroups of four and of eight wavefronts (256 workgroups of 128 rows), rows just
-    past a multiple of either's."""
+    """Both sides of the line between workgroups of four and of eight wavefronts (256 workgroups of 128 rows, 512 under the
+    causal mask), rows just past a multiple of either's."""
     import mercury_artifact_amd as M
 
     print(f"fp8 Sq{Sq} Sc{Sc} H{H} D{D} causal={causal}", flush=True)
