@@ -4,10 +4,10 @@
 // small block take 10).
 //
 // Every function takes the same arguments as the Python function of its name and does the whole call when the arguments
-// are what the kernels take as they are; for anything else -- another type, layout or device, a wrong shape, a tensor
-// subclass -- it returns None without having done anything, and the Python function goes on to convert or to report.
-// The entry points of the library are handed over by address (bind), so that there is one place that decides which
-// library is loaded.
+// are what the kernels take as they are; for anything else -- another type or layout, a device that is not the current one,
+// a wrong shape, a tensor subclass -- it returns None without having done anything, and the Python function goes on to
+// convert or to report.  The entry points of the library are handed over by address (bind), so that there is one place
+// that decides which library is loaded.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -15,7 +15,6 @@
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
-#include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/PythonTorchFunctionTLS.h>
@@ -73,13 +72,13 @@ struct Args {                 // tensors of one call, all on one device
   }
 };
 
-// Makes the tensor's device current for the scope; the common case is that it is.
+// The tensor's current stream if its device is the current one.  A call for another device is left to the Python function,
+// which changes the device for its duration (c10::hip's guards do not take the device of a tensor, whose type is "cuda").
 struct OnDevice {
-  c10::hip::OptionalHIPGuard guard;
-  hipStream_t stream;
-  explicit OnDevice(const Tensor& t) {
-    if (c10::hip::current_device() != t.device().index()) guard.set_device(t.device());
-    stream = c10::hip::getCurrentHIPStream(t.device().index()).stream();
+  bool current;
+  hipStream_t stream = nullptr;
+  explicit OnDevice(const Tensor& t) : current(c10::hip::current_device() == t.device().index()) {
+    if (current) stream = c10::hip::getCurrentHIPStream(t.device().index()).stream();
   }
 };
 
@@ -172,6 +171,7 @@ PyObject* fwd_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   if (out_given && (!shape4(*out_given, B, Sq, Hq, D) || out_given->scalar_type() != at::kBFloat16 || out_given->stride(3) != 1)) SLOW;
   if (lse_given && (!shape3(*lse_given, B, Hq, Sq) || lse_given->scalar_type() != at::kFloat || !lse_given->is_contiguous())) SLOW;
   OnDevice on(q);
+  if (!on.current) SLOW;
   const Tensor out = out_given ? *out_given : at::empty({B, Sq, Hq, D}, q.options().dtype(at::kBFloat16).requires_grad(false));
   const Tensor lse = lse_given ? *lse_given : at::empty({B, Hq, Sq}, q.options().dtype(at::kFloat).requires_grad(false));
   const int code = entry.fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), floats(&lse),
@@ -225,6 +225,7 @@ PyObject* bwd_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   if (!optional(a[12], q, acc)) SLOW;
   if (acc && (acc->sizes() != q.sizes() || acc->scalar_type() != at::kFloat || !acc->is_contiguous())) SLOW;
   OnDevice on(q);
+  if (!on.current) SLOW;
   const Tensor ws = bwd_workspace(q, Sc, Hkv);
   const int code = entry.bwd(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), floats(&lse),
                              dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), floats(acc), B, Sq, Sc, Hq, Hkv, D,
@@ -276,6 +277,7 @@ PyObject* bwd_chunk(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
                kept->numel() != entry.bwd_bytes(B, Sq, Sc, Hq, Hkv, D)))
     SLOW;
   OnDevice on(q);
+  if (!on.current) SLOW;
   const Tensor ws = kept ? *kept : bwd_workspace(q, Sc, Hkv);
   auto second16 = [](const Tensor* t) { return t ? static_cast<void*>(static_cast<char*>(t->data_ptr()) + 2 * t->stride(0)) : nullptr; };
   const int code = entry.chunk(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), floats(&lse),
@@ -314,6 +316,7 @@ PyObject* merge_into(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
                !t[7]->is_contiguous() || t[6]->scalar_type() != at::kBFloat16 || t[7]->scalar_type() != at::kFloat))
     SLOW;
   OnDevice on(*bo);
+  if (!on.current) SLOW;
   auto st = [](const Tensor* x, int i) { return x ? x->stride(i) : int64_t(0); };
   const int code = entry.merge(floats(t[0]), floats(t[1]), bo->data_ptr(), floats(bl), floats(t[4]), floats(t[5]),
                                data(t[6]), floats(t[7]), B, Sq, Hq, D, st(t[0], 0), st(t[0], 1), st(t[0], 2),
@@ -365,6 +368,7 @@ PyObject* merge_many(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     begins[i] = (int)begin;
   }
   OnDevice on(*out);
+  if (!on.current) SLOW;
   if (entry.many(outs, lses, batch, begins, (int)n, out->data_ptr(), floats(lse), B, Sq, Hq, D, ss, sh, on.stream) != MHIP_OK) SLOW;
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -382,6 +386,7 @@ PyObject* pack_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     SLOW;
   if (lhs && (!shape4(*lhs, B, Sq, Hq, D + 1) || lhs->scalar_type() != at::kFloat || !lhs->is_contiguous())) SLOW;
   OnDevice on(*bo);
+  if (!on.current) SLOW;
   const Tensor dst = at::empty({B, Sq, Hq, D + 1}, bo->options().dtype(at::kFloat).requires_grad(false));
   if (entry.pack(floats(lhs), bo->data_ptr(), floats(bl), floats(&dst), B, Sq, Hq, D, on.stream) != MHIP_OK) SLOW;
   return give(dst);
@@ -401,6 +406,7 @@ PyObject* unpack_into(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
       lse.scalar_type() != at::kFloat || !lse.is_contiguous() || !fits({B, Sq, Hq, D}))
     SLOW;
   OnDevice on(buf);
+  if (!on.current) SLOW;
   if (entry.unpack(floats(&buf), out.data_ptr(), floats(&lse), B, Sq, Hq, D, on.stream) != MHIP_OK) SLOW;
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -413,6 +419,7 @@ PyObject* quantize_e4m3(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   const Tensor* x = plain(a[0]);
   if (!x || (x->scalar_type() != at::kFloat && x->scalar_type() != at::kBFloat16) || !x->is_contiguous()) SLOW;
   OnDevice on(*x);
+  if (!on.current) SLOW;
   const Tensor xq = at::empty(x->sizes(), x->options().dtype(at::kFloat8_e4m3fn).requires_grad(false));
   const Tensor ws = at::empty({2}, x->options().dtype(at::kFloat).requires_grad(false));      // scale, scratch
   float* w = floats(&ws);

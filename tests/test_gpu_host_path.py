@@ -1,6 +1,8 @@
 """The compiled host module against the Python functions it stands in for: same results bit for bit where it takes a
 call, the Python function's own handling or error where it does not, the registered operator wherever a mode, a
 transform or autograd is at work."""
+import ctypes
+
 import pytest
 import torch
 
@@ -160,3 +162,34 @@ def test_gradients_count_as_written():
             M._flash_attn_backward(dout, q, kv[0], kv[1], out, lse, inside, dkv[0], dkv[1], 0.0, 0.1, False, -1, -1, 0.0,
                                    None, False)
         assert dq._version > before[0] and dkv._version > before[1]
+
+
+def _on_device(t, index):
+    """``t``'s memory as a tensor that says it is on another GPU: nothing may touch it, so there need not be one."""
+    class Head(ctypes.Structure):
+        _fields_ = [("data", ctypes.c_void_p), ("device_type", ctypes.c_int), ("device_id", ctypes.c_int)]
+
+    pointer = ctypes.pythonapi.PyCapsule_GetPointer
+    pointer.restype, pointer.argtypes = ctypes.c_void_p, [ctypes.py_object, ctypes.c_char_p]
+    capsule = torch.utils.dlpack.to_dlpack(t)
+    Head.from_address(pointer(capsule, b"dltensor")).device_id = index
+    return torch.utils.dlpack.from_dlpack(capsule)
+
+
+def test_tensors_of_another_device_are_left_to_the_python_function():
+    """The Python functions make the tensors' device current for the call; the host module declines."""
+    q, kv, dout = (_on_device(t, 1) for t in _data(Sq=64, Sc=64, Hq=2))
+    N.lib()
+    assert q.device.index == 1 and torch.cuda.current_device() == 0
+    k, v = kv.unbind(0)
+    B, S, H, D = q.shape
+    f32 = lambda *shape: _on_device(torch.zeros(shape, device="cuda"), 1)
+    lse, acc, accl, packed = f32(B, H, S), f32(B, S, H, D), f32(B, S, H, 1), f32(B, S, H, D + 1)
+    assert N.host.fwd_block(q, k, v, 0.1, False, None, None, None, None, None) is None
+    assert N.host.bwd_block(dout, q, k, v, q, lse, dout, k, v, 0.1, False, False, None) is None
+    assert N.host.bwd_chunk(dout, q, k, v, q, lse, dout, None, True, True, kv, None, 0.1, None) is None
+    assert N.host.merge_into(None, None, q, lse, acc, accl, None, None) is None
+    assert N.host.merge_many([q], [lse], dout, lse, None) is None
+    assert N.host.pack_block(q, lse, None) is None
+    assert N.host.unpack_into(packed, q, lse) is None
+    assert N.host.quantize_e4m3(acc) is None
