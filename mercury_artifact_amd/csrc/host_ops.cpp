@@ -33,6 +33,7 @@ struct Entry {
   decltype(&mhip_pack_reduce) pack = nullptr;
   decltype(&mhip_unpack) unpack = nullptr;
   decltype(&mhip_quantize_e4m3) quantize = nullptr;
+  decltype(&mhip_error_string) error_string = nullptr;
 } entry;
 bool bound = false;
 
@@ -110,6 +111,18 @@ PyObject* give2(const Tensor& a, const Tensor& b) {
   return r;
 }
 #define SLOW do { Py_RETURN_NONE; } while (0)
+
+// What a code other than MHIP_OK means for the call: None for arguments the library refused before it launched anything
+// (the Python function converts them or reports them); an error for anything else -- a kernel may have run, and a second
+// call would add to its sums.
+PyObject* refused(int code, const char* what) {
+  switch (code) {
+    case MHIP_EINVAL: case MHIP_EDTYPE: case MHIP_EHEADDIM: case MHIP_EALIGN: case MHIP_EUNSUPPORTED: case MHIP_ETOOLARGE:
+      Py_RETURN_NONE;
+    default:
+      return PyErr_Format(PyExc_RuntimeError, "%s: %s (code %d)", what, entry.error_string(code), code);
+  }
+}
 #define ENTER(n) if (nargs != (n) || !bound) SLOW
 
 // Whether the torch operator of the name would do nothing but call its kernel: no mode, transform or trace is active and
@@ -180,7 +193,7 @@ PyObject* fwd_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
                              (float)scale, causal ? MHIP_MASK_CAUSAL : MHIP_MASK_NONE,
                              type == at::kBFloat16 ? MHIP_BF16 : MHIP_E4M3, floats(descale[0]), floats(descale[1]),
                              floats(descale[2]), on.stream);
-  if (code != MHIP_OK) SLOW;
+  if (code != MHIP_OK) return refused(code, "mhip_attn_fwd_block");
   return give2(out, lse);
   END_HANDLE_TH_ERRORS
 }
@@ -233,7 +246,7 @@ PyObject* bwd_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
                              dk.stride(0), dk.stride(1), dk.stride(2), dq.stride(0), dq.stride(1), dq.stride(2),
                              out.stride(0), out.stride(1), out.stride(2), (float)scale,
                              causal ? MHIP_MASK_CAUSAL : MHIP_MASK_NONE, deterministic, ws.data_ptr(), on.stream);
-  if (code != MHIP_OK) SLOW;
+  if (code != MHIP_OK) return refused(code, "mhip_attn_bwd_block");
   // the workspace is (-delta | lse in base 2 | delta), each in a slot rounded up to 4 elements
   const int64_t rows = B * Hq * Sq, slot = (rows + 3) & ~int64_t(3);
   return give(ws.view(at::kFloat).narrow(0, 2 * slot, rows).view({B, Hq, Sq}));
@@ -288,7 +301,7 @@ PyObject* bwd_chunk(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
                                dq ? dq->stride(0) : 0, dq ? dq->stride(1) : 0, dq ? dq->stride(2) : 0,
                                out.stride(0), out.stride(1), out.stride(2), (float)scale, MHIP_MASK_NONE, ws.data_ptr(),
                                on.stream);
-  if (code != MHIP_OK) SLOW;
+  if (code != MHIP_OK) return refused(code, "mhip_attn_bwd_chunk");
   return give(ws);
   END_HANDLE_TH_ERRORS
 }
@@ -323,7 +336,7 @@ PyObject* merge_into(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
                                st(t[1], 0), st(t[1], 1), st(t[1], 2), bo->stride(0), bo->stride(1), bo->stride(2),
                                bl->stride(0), bl->stride(1), st(t[4], 0), st(t[4], 1), st(t[4], 2), st(t[5], 0),
                                st(t[5], 1), st(t[5], 2), on.stream);
-  if (code != MHIP_OK) SLOW;
+  if (code != MHIP_OK) return refused(code, "mhip_lse_merge");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
@@ -369,7 +382,8 @@ PyObject* merge_many(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   }
   OnDevice on(*out);
   if (!on.current) SLOW;
-  if (entry.many(outs, lses, batch, begins, (int)n, out->data_ptr(), floats(lse), B, Sq, Hq, D, ss, sh, on.stream) != MHIP_OK) SLOW;
+  const int code = entry.many(outs, lses, batch, begins, (int)n, out->data_ptr(), floats(lse), B, Sq, Hq, D, ss, sh, on.stream);
+  if (code != MHIP_OK) return refused(code, "mhip_lse_merge_many");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
@@ -388,7 +402,8 @@ PyObject* pack_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   OnDevice on(*bo);
   if (!on.current) SLOW;
   const Tensor dst = at::empty({B, Sq, Hq, D + 1}, bo->options().dtype(at::kFloat).requires_grad(false));
-  if (entry.pack(floats(lhs), bo->data_ptr(), floats(bl), floats(&dst), B, Sq, Hq, D, on.stream) != MHIP_OK) SLOW;
+  const int code = entry.pack(floats(lhs), bo->data_ptr(), floats(bl), floats(&dst), B, Sq, Hq, D, on.stream);
+  if (code != MHIP_OK) return refused(code, "mhip_pack_reduce");
   return give(dst);
   END_HANDLE_TH_ERRORS
 }
@@ -407,7 +422,8 @@ PyObject* unpack_into(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     SLOW;
   OnDevice on(buf);
   if (!on.current) SLOW;
-  if (entry.unpack(floats(&buf), out.data_ptr(), floats(&lse), B, Sq, Hq, D, on.stream) != MHIP_OK) SLOW;
+  const int code = entry.unpack(floats(&buf), out.data_ptr(), floats(&lse), B, Sq, Hq, D, on.stream);
+  if (code != MHIP_OK) return refused(code, "mhip_unpack");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
@@ -423,9 +439,9 @@ PyObject* quantize_e4m3(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   const Tensor xq = at::empty(x->sizes(), x->options().dtype(at::kFloat8_e4m3fn).requires_grad(false));
   const Tensor ws = at::empty({2}, x->options().dtype(at::kFloat).requires_grad(false));      // scale, scratch
   float* w = floats(&ws);
-  if (entry.quantize(x->data_ptr(), x->scalar_type() == at::kFloat ? MHIP_F32 : MHIP_BF16, x->numel(), xq.data_ptr(), w, w + 1,
-                     on.stream) != MHIP_OK)
-    SLOW;
+  const int code = entry.quantize(x->data_ptr(), x->scalar_type() == at::kFloat ? MHIP_F32 : MHIP_BF16, x->numel(), xq.data_ptr(),
+                                  w, w + 1, on.stream);
+  if (code != MHIP_OK) return refused(code, "mhip_quantize_e4m3");
   return give2(xq, ws.select(0, 0));
   END_HANDLE_TH_ERRORS
 }
@@ -442,7 +458,7 @@ PyObject* bind(PyObject*, PyObject* table) {
                   take(entry.bwd, "mhip_attn_bwd_block") && take(entry.chunk, "mhip_attn_bwd_chunk") &&
                   take(entry.merge, "mhip_lse_merge") && take(entry.many, "mhip_lse_merge_many") &&
                   take(entry.pack, "mhip_pack_reduce") && take(entry.unpack, "mhip_unpack") &&
-                  take(entry.quantize, "mhip_quantize_e4m3");
+                  take(entry.quantize, "mhip_quantize_e4m3") && take(entry.error_string, "mhip_error_string");
   if (PyErr_Occurred()) return nullptr;
   bound = ok;
   return PyBool_FromLong(ok);

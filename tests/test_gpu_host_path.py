@@ -193,3 +193,31 @@ def test_tensors_of_another_device_are_left_to_the_python_function():
     assert N.host.pack_block(q, lse, None) is None
     assert N.host.unpack_into(packed, q, lse) is None
     assert N.host.quantize_e4m3(acc) is None
+
+
+@pytest.mark.parametrize("code,error", [(-5, "kernel launch failed"), (-8, "runtime query failed"), (1, "unknown")])
+def test_a_failed_launch_is_reported_once_and_not_repeated(code, error):
+    """A launch that reports an error may have run all the same: a second one would add its dq to dq_acc again."""
+    import mercury_artifact_amd as M
+
+    q, kv, dout = _data()
+    out, lse = M.attn_fwd_block(q, kv[0], kv[1], 0.1)
+    table = {name: ctypes.cast(getattr(N.lib(), name), ctypes.c_void_p).value for name in N.EXPORTED_SYMBOLS}
+    calls, stubs = [], {}
+    for name in ("mhip_attn_fwd_block", "mhip_attn_bwd_block", "mhip_lse_merge_many"):
+        stub = ctypes.CFUNCTYPE(*([N._SIGNATURES[name][0]] + N._SIGNATURES[name][1]))(lambda *a: calls.append(len(a)) or code)
+        stubs[name] = (stub, ctypes.cast(stub, ctypes.c_void_p).value)
+    dq, dkv, acc = torch.empty_like(q), torch.empty_like(kv), torch.zeros(q.shape, device="cuda")
+    try:
+        assert N.host.bind({**table, **{name: address for name, (_, address) in stubs.items()}})
+        for name, call in (
+                ("mhip_attn_fwd_block", lambda: M.attn_fwd_block(q, kv[0], kv[1], 0.1)),
+                ("mhip_attn_fwd_block", lambda: M._flash_attn_forward(q, kv[0], kv[1], 0.0, 0.1, False, -1, -1, 0.0, None, False)),
+                ("mhip_attn_bwd_block", lambda: M.attn_bwd_block(dout, q, kv[0], kv[1], out, lse, dq, dkv[0], dkv[1], 0.1, dq_acc=acc)),
+                ("mhip_lse_merge_many", lambda: M.merge_many([out], [lse], torch.empty_like(q), torch.empty_like(lse)))):
+            with pytest.raises(RuntimeError, match=f"{name}: .*{error}"):
+                call()
+    finally:
+        assert N.host.bind(table)
+    assert len(calls) == 4
+    assert not acc.any()
