@@ -46,7 +46,8 @@ extern "C" {
 #define MHIP_MASK_CAUSAL  1   /* query i sees key j iff j <= i + (Sc - Sq) (bottom-right) */
 
 /* Bumped whenever an entry point's argument list changes (a caller built against another value must not call).
- * 3: the three descales of mhip_attn_fwd_block are device pointers; mhip_attn_bwd_block takes five stride triples. */
+ * 3: the three descales of mhip_attn_fwd_block are device pointers; mhip_attn_bwd_block takes five stride triples.
+ * 4: the backward's workspace also holds partial sums (it is larger than its three row arrays); mhip_attn_bwd_chunk. */
 #define MHIP_ABI_VERSION 4
 int         mhip_abi_version(void);   /* the MHIP_ABI_VERSION the library was built with */
 int         mhip_version(void);
@@ -90,7 +91,9 @@ int mhip_attn_fwd_block(const void* q, const void* k, const void* v, void* out, 
  * of utils/attn_bwd_dsl.py:117-122 folded into the kernel.  `workspace` must hold
  * mhip_attn_bwd_workspace_bytes(...) bytes of device memory: three (B, Hq, Sq) fp32 arrays, each rounded up to a
  * multiple of 4 elements -- -delta (= -rowsum(dout * out), stored negated because the kernels start dP from it),
- * the LSE in base 2, and delta itself, which is what flash-attn returns as softmax_d.  dq and out have element strides of their own:
+ * the LSE in base 2, and delta itself, which is what flash-attn returns as softmax_d -- and behind them 32 MiB for
+ * the partial sums of launches whose workgroups share a tile.  The size depends on B, Sq and Hq alone: one workspace
+ * serves chunks of any length (calls that overlap in time need one each).  dq and out have element strides of their own:
  * the call site allocates block_dq with torch.empty (contiguous, utils/attn_bwd_dsl.py:83) while q, out and
  * dout are views of the step's buffers; q and dout, k and v, dk and dv share a stride triple each.
  * Head dimension: any multiple of 8 up to 128, as for the bf16 forward (for D < 128 the q / dout span of one

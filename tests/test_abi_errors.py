@@ -77,6 +77,16 @@ def test_backward_rejects(lib):
     assert lib.mhip_attn_bwd_workspace_bytes(2, 100, 64, 4, 2, 128) >= 2 * 2 * 4 * 100 * 4
 
 
+@pytest.mark.parametrize("B,Sq,Hq", [(1, 64, 1), (1, 512, 8), (2, 1500, 12), (1, 4096, 32), (4, 512, 5)])
+def test_one_backward_workspace_serves_every_chunk(lib, B, Sq, Hq):
+    """A call does not say how large its workspace is, so a workspace kept over chunks of different lengths, for either
+    mask, has to be large enough for all of them: the three row arrays and the largest partial sums."""
+    sizes = {lib.mhip_attn_bwd_workspace_bytes(B, Sq, Sc, Hq, Hkv, D)
+             for Sc in (0, 1, 64, 333, 1024, 4096, 65536) for Hkv in (1, Hq) for D in (8, 64, 96, 128)}
+    assert sizes == {(B * Sq * Hq + 3) // 4 * 4 * 12 + (32 << 20)}
+    assert lib.mhip_attn_bwd_workspace_bytes(B, 0, 64, Hq, 1, 64) == 0
+
+
 def test_elementwise_rejects(lib):
     assert lib.mhip_flash_reduce(P, P, None, 8, 128, None) == EINVAL
     assert lib.mhip_flash_reduce(P, P + 4, P, 8, 128, None) == EALIGN

@@ -94,3 +94,29 @@ def test_backward_block_with_shared_tiles(B, Sq, Sc, Hq, Hkv, causal, D):
     """Long chains of tiles on few workgroups (grouped heads, one head): their stationary tiles are shared and the sums
     added by the third launch."""
     _block(B, Sq, Sc, Hq, Hkv, D, causal)
+
+
+def test_partial_sums_stay_inside_the_workspace():
+    """One workspace, sized with the first chunk, for chunks of other lengths and for both masks, among them launches that
+    leave the most partial sums: nothing behind its end is written, and the results are those of a fresh one."""
+    import mercury_artifact_amd as M
+    from mercury_artifact_amd import _native as N
+
+    B, Sq, Hq, Hkv, D = 1, 1000, 8, 1, 128
+    g = torch.Generator(device="cuda").manual_seed(9)
+    mk = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    q, dout, kv = mk(B, Sq, Hq, D), mk(B, Sq, Hq, D), mk(2, B, 3000, Hkv, D)
+    size = N.lib().mhip_attn_bwd_workspace_bytes(B, Sq, 64, Hq, Hkv, D)
+    memory = torch.full((size + (32 << 20),), 0xA5, dtype=torch.uint8, device="cuda")
+    for Sc, causal in ((64, False), (3000, False), (1000, True), (130, False), (2048, True)):
+        print(f"Sc{Sc} causal={causal}", flush=True)
+        k, v = kv[0, :, :Sc], kv[1, :, :Sc]
+        out, lse = M.attn_fwd_block(q, k, v, 0.1, causal=causal)
+        want, got = (tuple(torch.empty_like(t) for t in (q, k, v)) for _ in range(2))
+        M.attn_bwd_block(dout, q, k, v, out, lse, *want, 0.1, causal=causal)
+        strides = [st for t in (q, k, got[1], got[0], out) for st in t.stride()[:3]]
+        N.check(N.lib().mhip_attn_bwd_block(*map(N.ptr, (dout, q, k, v, out, lse, *got)), None, B, Sq, Sc, Hq, Hkv, D, *strides,
+                                            0.1, int(causal), 0, N.ptr(memory), N.stream_of(q)), "mhip_attn_bwd_block")
+        torch.cuda.synchronize()
+        assert bool((memory[size:] == 0xA5).all())
+        assert all(torch.equal(a, b) for a, b in zip(want, got))
