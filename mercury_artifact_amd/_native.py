@@ -100,9 +100,17 @@ def lib() -> ctypes.CDLL:
             fn.argtypes = args
         if isinstance(host, _NoHost):          # built since the package was imported
             host = _load_host()
-        if host.bind({name: ctypes.cast(getattr(handle, name), c_void_p).value for name in _SIGNATURES}) is not True:
+        if isinstance(host, _NoHost):
+            reason = host.reason
+        elif getattr(host, "abi_version", None) != ABI_VERSION:     # it would call with another argument list
+            reason = f"compiled for ABI version {getattr(host, 'abi_version', None)}, not {ABI_VERSION}"
+        elif host.bind({name: ctypes.cast(getattr(handle, name), c_void_p).value for name in _SIGNATURES}) is not True:
+            reason = "entry points"
+        else:
+            reason = None
+        if reason is not None:
             raise RuntimeError("the host module _mercury_host is missing or stale: build it with "
-                               f"`python -m mercury_artifact_amd.csrc.build` ({getattr(host, 'reason', 'entry points')})")
+                               f"`python -m mercury_artifact_amd.csrc.build` ({reason})")
         _lib = handle
     return _lib
 

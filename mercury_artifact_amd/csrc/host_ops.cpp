@@ -474,4 +474,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_mercury_host", nullptr, -1, metho
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__mercury_host() { return PyModule_Create(&module); }
+// abi_version: of the header this module was compiled with; whoever binds a library compares it with the library's
+PyMODINIT_FUNC PyInit__mercury_host() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddIntConstant(m, "abi_version", MHIP_ABI_VERSION) < 0) Py_CLEAR(m);
+  return m;
+}

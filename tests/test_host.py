@@ -312,3 +312,27 @@ def test_host_module_built_after_the_import_is_found(monkeypatch):
     monkeypatch.setattr(N, "_load_host", lambda: N._NoHost("not built"))
     with pytest.raises(RuntimeError, match="_mercury_host"):
         N.lib()
+
+
+def test_host_module_of_another_abi_is_refused(monkeypatch):
+    """Every entry point is there by name, but the module was compiled against another argument list."""
+    from mercury_artifact_amd import _native as N
+
+    bound = []
+
+    class Stale:
+        def bind(self, table):
+            bound.append(table)
+            return True
+
+    for version in (N.ABI_VERSION - 1, N.ABI_VERSION + 1, None):
+        stale = Stale()
+        if version is not None:                    # a module from before there was a version has none
+            stale.abi_version = version
+        monkeypatch.setattr(N, "host", stale)
+        monkeypatch.setattr(N, "_lib", None)
+        with pytest.raises(RuntimeError, match=f"stale.*{version}"):
+            N.lib()
+    assert not bound
+    monkeypatch.undo()
+    assert N.host.abi_version == N.ABI_VERSION == N.lib().mhip_abi_version()
