@@ -11,6 +11,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/record_function.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -125,10 +126,11 @@ PyObject* refused(int code, const char* what) {
 }
 #define ENTER(n) if (nargs != (n) || !bound) SLOW
 
-// Whether the torch operator of the name would do nothing but call its kernel: no mode, transform or trace is active and
-// none of the tensors asks for a gradient.
+// Whether the torch operator of the name would do nothing but call its kernel: no mode, transform, trace or profiler is
+// active and none of the tensors asks for a gradient.
 PyObject* undispatched(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
-  bool yes = bound && !c10::impl::TorchDispatchModeTLS::any_modes_set() && !at::impl::torch_function_mode_enabled();
+  bool yes = bound && !c10::impl::TorchDispatchModeTLS::any_modes_set() && !at::impl::torch_function_mode_enabled() &&
+             !(at::isRecordFunctionEnabled() && at::hasCallbacks());
   if (yes) {
     using K = c10::DispatchKey;
     const auto in = c10::impl::tls_local_dispatch_key_set().included_;

@@ -221,3 +221,22 @@ def test_a_failed_launch_is_reported_once_and_not_repeated(code, error):
         assert N.host.bind(table)
     assert len(calls) == 4
     assert not acc.any()
+
+
+def test_a_profiler_sees_the_operators():
+    """The dispatcher is where a profiler hears of an operator: under one, plain calls and the drivers' blocks go there."""
+    import mercury_artifact_amd as M
+    from torch.profiler import ProfilerActivity, profile
+
+    q, kv, dout = _data()
+    fwd = lambda: M._flash_attn_forward(q, kv[0], kv[1], 0.0, 0.1, False, -1, -1, 0.0, None, False)
+    out, lse = fwd()[:2]
+    dq, dkv = torch.empty_like(q), torch.empty_like(kv)
+    o, l = torch.empty_like(out), torch.empty_like(lse)
+    with profile(activities=[ProfilerActivity.CPU]) as seen:
+        again = fwd()
+        M._flash_attn_backward(dout, q, kv[0], kv[1], out, lse, dq, dkv[0], dkv[1], 0.0, 0.1, False, -1, -1, 0.0, None, False)
+        M.gqa_pack_kv(q, kv, o, l, 0.1, ring=M.LocalRing((3,), 0, [kv] * 3))
+    counts = {e.key: e.count for e in seen.key_averages()}
+    assert counts.get("mercury_amd::_flash_attn_forward") == 4 and counts.get("mercury_amd::_flash_attn_backward") == 1
+    assert torch.equal(again[0], out) and torch.equal(again[1], lse)
