@@ -139,15 +139,26 @@ def _flash_attn_forward(
     return out, lse, empty, rng
 
 
+_NUMBER, _INTEGER, _FLAG = {float, int}, {int}, {bool}
+
+
+def as_declared(numbers, integers, flags) -> bool:
+    """Whether plain arguments have the very types the operators' schemas declare.  Of any other type the schema converts
+    some and refuses the rest: such a call goes to the dispatcher."""
+    return (_NUMBER.issuperset(map(type, numbers)) and _INTEGER.issuperset(map(type, integers))
+            and _FLAG.issuperset(map(type, flags)))
+
+
 def _forward_now(q, k, v, dropout_p, softmax_scale, causal, window_size_left, window_size_right, softcap, alibi_slopes,
                  return_softmax, q_descale=None, k_descale=None, v_descale=None):
     """What the operator returns, without the dispatcher, where that would do nothing but call the kernel; else None."""
-    if (dropout_p or softcap or alibi_slopes is not None or window_size_left not in (-1, None)
-            or window_size_right not in (-1, None) or not N.host.undispatched(q, k, v, q_descale, k_descale, v_descale)):
+    if (not as_declared((dropout_p, softmax_scale, softcap), (window_size_left, window_size_right), (causal, return_softmax))
+            or dropout_p or softcap or alibi_slopes is not None or window_size_left != -1 or window_size_right != -1
+            or not N.host.undispatched(q, k, v, q_descale, k_descale, v_descale)):
         return None
     if k.dtype != q.dtype or k.dim() != 4 or q.dim() != 4:      # for the operator to report
         return None
-    out, lse = attn_fwd_block(q, k, v, softmax_scale, bool(causal), q_descale, k_descale, v_descale)
+    out, lse = attn_fwd_block(q, k, v, softmax_scale, causal, q_descale, k_descale, v_descale)
     return (out, lse, *N.host.no_dropout(q))
 
 
@@ -321,11 +332,12 @@ def _flash_attn_backward(
 
 def _backward_now(dout, q, k, v, out, softmax_lse, dq, dk, dv, dropout_p, softmax_scale, causal, window_size_left,
                   window_size_right, softcap, alibi_slopes, deterministic, rng_state=None):
-    if (dropout_p or softcap or alibi_slopes is not None or window_size_left not in (-1, None)
-            or window_size_right not in (-1, None)
+    if (not as_declared((dropout_p, softmax_scale, softcap), (window_size_left, window_size_right), (causal, deterministic))
+            or dropout_p or softcap or alibi_slopes is not None or window_size_left != -1 or window_size_right != -1
+            or rng_state is not None
             or not N.host.undispatched(dout, q, k, v, out, softmax_lse, dq, dk, dv)):
         return None
-    delta = attn_bwd_block(dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_scale, bool(causal), bool(deterministic))
+    delta = attn_bwd_block(dout, q, k, v, out, softmax_lse, dq, dk, dv, softmax_scale, causal, deterministic)
     N.host.written(dq, dk, dv)
     return delta
 

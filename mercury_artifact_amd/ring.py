@@ -86,10 +86,11 @@ def _block_forward(q, k, v, softmax_scale, dropout_p, causal, window_size, alibi
     return outputs[:2]
 
 
-def _block_results(n, q, kv, dropout_p, window_size, alibi_slopes, **descales):
+def _block_results(n, q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **descales):
     """Places for the results of a step's ``n`` blocks over all rows of ``q``, from one allocation each for the outputs and
     the LSEs; None for every block where the operator has something to report or to record."""
-    if (dropout_p or alibi_slopes is not None or window_size[0] not in (-1, None) or window_size[1] not in (-1, None)
+    if (not _ops.as_declared((softmax_scale, dropout_p), window_size, (causal,))
+            or dropout_p or alibi_slopes is not None or window_size[0] != -1 or window_size[1] != -1
             or q.dim() != 4 or not N.host.undispatched(q, kv, *descales.values())):
         return [None] * n
     B, Sq, Hq, D = q.shape
@@ -151,7 +152,9 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
                       f"{MAX_MERGE_MANY} blocks and writes contiguous bfloat16, so this step merges block by block "
                       "(same result, one pass over the fp32 accumulator per block)", RuntimeWarning, stacklevel=3)
     done = 0
-    places = _block_results(n_blocks, q, kv, dropout_p, window_size, alibi_slopes, **extra) if defer else [None] * n_blocks
+    places = [None] * n_blocks
+    if defer:
+        places = _block_results(n_blocks, q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra)
     main = side = None
     kv_ready = next_ready = None
     if two_streams and defer:
@@ -271,7 +274,9 @@ def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=F
     blocks = []
     defer = (fused_epilogue and deferred_merge and len(hops) <= MAX_MERGE_MANY and o.dtype == torch.bfloat16
              and o.is_contiguous() and lse.is_contiguous())
-    places = _block_results(len(hops), q, kv, dropout_p, window_size, alibi_slopes) if defer else [None] * len(hops)
+    places = [None] * len(hops)
+    if defer:
+        places = _block_results(len(hops), q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes)
     for step, hop in enumerate(hops):
         if step == 0:
             _kv = kv.contiguous()

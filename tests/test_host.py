@@ -336,3 +336,58 @@ def test_host_module_of_another_abi_is_refused(monkeypatch):
     assert not bound
     monkeypatch.undo()
     assert N.host.abi_version == N.ABI_VERSION == N.lib().mhip_abi_version()
+
+
+_NOT_THE_SCHEMAS = [("dropout_p", None), ("dropout_p", 0j), ("softmax_scale", "0.1"), ("softmax_scale", None), ("causal", "x"),
+                    ("causal", []), ("window_size_left", None), ("window_size_right", -1.0), ("softcap", None)]
+
+
+@pytest.mark.parametrize("name,value", _NOT_THE_SCHEMAS + [("return_softmax", "a"), ("q_descale", 1.0), ("alibi_slopes", 1)])
+def test_forward_operator_refuses_what_its_schema_refuses(monkeypatch, name, value):
+    _refuses(monkeypatch, "_flash_attn_forward", {"return_softmax": False, "alibi_slopes": None}, name, value)
+
+
+@pytest.mark.parametrize("name,value", _NOT_THE_SCHEMAS + [("deterministic", "a"), ("rng_state", 1), ("alibi_slopes", 1)])
+def test_backward_operator_refuses_what_its_schema_refuses(monkeypatch, name, value):
+    t = torch.zeros(1, 2, 1, 8, dtype=torch.bfloat16)
+    more = {k: t for k in ("dout", "out", "softmax_lse", "dq", "dk", "dv")}
+    _refuses(monkeypatch, "_flash_attn_backward", {**more, "deterministic": False, "alibi_slopes": None}, name, value)
+
+
+def _refuses(monkeypatch, op, more, name, value):
+    """Also where the call would go past the dispatcher, which is where the schema is checked."""
+    import mercury_artifact_amd.flash_attn_interface as I
+
+    taken = []
+
+    class Eager:
+        undispatched = staticmethod(lambda *ts: all(t is None or isinstance(t, torch.Tensor) for t in ts))
+        no_dropout = staticmethod(lambda q: (q, q))
+        written = staticmethod(lambda *ts: None)
+
+    monkeypatch.setattr(I.N, "host", Eager())
+    monkeypatch.setattr(I, "attn_fwd_block", lambda *a: taken.append("f") or a[:2])
+    monkeypatch.setattr(I, "attn_bwd_block", lambda *a: taken.append("b") or a[0])
+    t = torch.zeros(1, 2, 1, 8, dtype=torch.bfloat16)
+    args = {"q": t, "k": t, "v": t, "dropout_p": 0, "softmax_scale": 0.1, "causal": False, "window_size_left": -1,
+            "window_size_right": -1, "softcap": 0.0, **more}
+    getattr(I, op)(**args)
+    assert len(taken) == 1                                   # as it should be, it needs no dispatcher
+    with pytest.raises(RuntimeError, match="Expected a value of type"):
+        getattr(I, op)(**{**args, name: value})
+    assert len(taken) == 1
+
+
+@pytest.mark.parametrize("values", [{"dropout_p": None}, {"softmax_scale": "0.1"}, {"causal": "x"}, {"window_size": (None, -1)},
+                                    {"window_size": (-1, -1.0)}])
+def test_drivers_leave_odd_arguments_to_the_operator(monkeypatch, values):
+    import mercury_artifact_amd.ring as R
+
+    class Eager:
+        undispatched = staticmethod(lambda *ts: True)
+
+    monkeypatch.setattr(R.N, "host", Eager())
+    q = torch.zeros(1, 2, 1, 8, dtype=torch.bfloat16)
+    args = {"softmax_scale": 0.1, "dropout_p": 0, "causal": False, "window_size": (-1, -1), "alibi_slopes": None}
+    assert R._block_results(2, q, q, **args)[1] is not None
+    assert R._block_results(2, q, q, **{**args, **values}) == [None, None]
