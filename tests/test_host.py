@@ -391,3 +391,19 @@ def test_drivers_leave_odd_arguments_to_the_operator(monkeypatch, values):
     args = {"softmax_scale": 0.1, "dropout_p": 0, "causal": False, "window_size": (-1, -1), "alibi_slopes": None}
     assert R._block_results(2, q, q, **args)[1] is not None
     assert R._block_results(2, q, q, **{**args, **values}) == [None, None]
+
+
+@pytest.mark.parametrize("dtype,D,row_bytes,taken", [
+    (torch.bfloat16, 128, 1 << 20, True), (torch.bfloat16, 128, 1 << 21, False), (torch.bfloat16, 64, (1 << 20) - 16, True),
+    (torch.bfloat16, 64, 1 << 20, False), (torch.float8_e4m3fn, 128, 1 << 21, False), (torch.float8_e4m3fn, 96, 1 << 20, False),
+    (torch.float8_e4m3fn, 96, 1 << 19, True), (torch.bfloat16, 128, 1032, False)])
+def test_own_chunk_out_of_the_kernels_reach_is_copied(dtype, D, row_bytes, taken):
+    """1024 rows of one layer of a packed cache: a view whose rows lie further apart than a 32-bit offset reaches (or do
+    not start on 16 bytes) becomes a copy, as the driver's own chunk always did once."""
+    from mercury_artifact_amd.ring import _as_rows
+
+    row = row_bytes // dtype.itemsize
+    chunk = torch.empty_strided((2, 1, 1024, 2, D), (1024 * row, 1024 * row, row, D, 1), dtype=dtype, device="meta")
+    got = _as_rows(chunk)
+    assert (got is chunk) == taken and (taken or got.is_contiguous())
+    assert _as_rows(got) is got
