@@ -109,6 +109,18 @@ def _as_rows(t):
     return t if fine else t.contiguous()
 
 
+def _extent(t):
+    """First and last address of a tensor's elements."""
+    start = t.data_ptr()
+    return start, start + (sum((n - 1) * st for n, st in zip(t.shape, t.stride())) + 1) * t.element_size()
+
+
+def _apart(t, *others):
+    """Whether no other tensor has elements between the first and the last of ``t``'s."""
+    first, last = _extent(t)
+    return all(a >= last or b <= first for a, b in map(_extent, others))
+
+
 _SIDE_STREAMS = {}
 
 
@@ -432,14 +444,17 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
 
     ``fused_accumulate=True`` (default) lets the block kernels do the sums: dq's carries over from chunk to chunk in
     fp32 (the sum sees the unrounded block gradients) and is written in q's type by the last one, and a chunk's dK/dV
-    are written in fp32 where ``dkv_chunks`` asks for them: no pass over the gradients besides.  ``False`` is the literal sequence: block backward
-    through ``_flash_attn_backward(**params)``, then ``torch.add`` on the bf16 block gradients."""
+    are written in fp32 where ``dkv_chunks`` asks for them: no pass over the gradients besides.  ``False`` is the literal
+    sequence: block backward through ``_flash_attn_backward(**params)``, then ``torch.add`` on the bf16 block gradients.
+
+    ``dq`` may lie over ``q``, ``dout`` or ``o`` and ``dkv`` over the own chunk: where a gradient's place overlaps what the
+    launch that would write it reads, it is stored behind that launch."""
     if dropout_p != 0 or alibi_slopes is not None or tuple(window_size) != (-1, -1):
         fused_accumulate = False                # let the operator report what it does not support
     # operands of other layouts go through the block operator, which copies them where it has to
     carried = (fused_accumulate and aligned_rows(q, dout) and aligned_rows(o) and lse.is_contiguous()
                and q.shape == o.shape == dout.shape)
-    write_dq = carried and aligned_rows(dq) and dq.shape == q.shape
+    write_dq = carried and aligned_rows(dq) and dq.shape == q.shape and _apart(dq, q, dout, o, lse, kv)
     reduce_dq = None
     if not carried and fused_accumulate:
         reduce_dq = torch.zeros(q.shape, dtype=torch.float32, device=q.device)
@@ -460,7 +475,10 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
             ring.commit()
         if carried:
             mine = chunk_id == own
-            direct = mine and dkv.shape == _kv.shape and aligned_rows(dkv[0], dkv[1])
+            direct = (mine and dkv.shape == _kv.shape and aligned_rows(dkv[0], dkv[1])
+                      and _apart(dkv, q, dout, o, lse, _kv))
+            if hop is None and write_dq and step > 0:
+                write_dq = _apart(dq, _kv)
             block_dkv = chunk_grad = None
             if direct:
                 block_dkv = dkv

@@ -120,3 +120,23 @@ def test_partial_sums_stay_inside_the_workspace():
         torch.cuda.synchronize()
         assert bool((memory[size:] == 0xA5).all())
         assert all(torch.equal(a, b) for a, b in zip(want, got))
+
+
+@pytest.mark.parametrize("W", [1, 2])
+@pytest.mark.parametrize("dq_over", ["q", "dout", "o"])
+def test_backward_step_in_place(W, dq_over):
+    """dq over q, dout or o and dkv over the own chunk: bit for bit the gradients that separate places receive."""
+    import mercury_artifact_amd as M
+
+    B, S, H, D = 1, 700, 4, 64
+    g = torch.Generator(device="cuda").manual_seed(4)
+    mk = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    t = {"q": mk(B, S, H, D), "dout": mk(B, S, H, D), "o": mk(B, S, H, D)}
+    chunks = [mk(2, B, S, H, D) for _ in range(W)]
+    lse = M.attn_fwd_block(t["q"], chunks[0][0], chunks[0][1], 0.1)[1]
+    want = torch.empty_like(t["q"]), torch.empty_like(chunks[0])
+    M.flash_attn_backward(t["q"], chunks[0], t["o"], lse, t["dout"], *want, 0.1, ring=M.LocalRing((W,), 0, chunks))
+    got = t[dq_over], chunks[0]
+    M.flash_attn_backward(t["q"], chunks[0], t["o"], lse, t["dout"], *got, 0.1, ring=M.LocalRing((W,), 0, chunks))
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])

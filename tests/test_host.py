@@ -407,3 +407,45 @@ def test_own_chunk_out_of_the_kernels_reach_is_copied(dtype, D, row_bytes, taken
     got = _as_rows(chunk)
     assert (got is chunk) == taken and (taken or got.is_contiguous())
     assert _as_rows(got) is got
+
+
+@pytest.mark.parametrize("W", [1, 3])
+@pytest.mark.parametrize("dq_over", ["", "q", "dout", "o", "half of q", "last chunk"])
+@pytest.mark.parametrize("dkv_over", ["", "kv"])
+def test_backward_step_in_place_writes_nothing_a_launch_still_reads(monkeypatch, W, dq_over, dkv_over):
+    """Gradients that lie over operands: no launch writes what it (or another workgroup of it) reads, and they are stored
+    all the same.  Without an overlap the launches store them directly."""
+    import mercury_artifact_amd.ring as R
+    from mercury_artifact_amd.schedule import LocalRing
+
+    B, S, H, D = 1, 16, 2, 8
+    memory = torch.zeros(2, B, 2 * S, H, D, dtype=torch.bfloat16)
+    t = {"q": memory[0, :, :S], "dout": memory[1, :, S:], "o": torch.zeros(B, S, H, D, dtype=torch.bfloat16)}
+    chunks = [torch.zeros(2, B, S, H, D, dtype=torch.bfloat16) for _ in range(W)]
+    lse = torch.zeros(B, H, S)
+    last_chunk = chunks[1 % W]                          # of rank 0's order 0, W - 1, ..., 1
+    dq = {"": torch.zeros_like(t["o"]), "half of q": memory[0, :, S // 2: S // 2 + S], "last chunk": last_chunk[0]}.get(dq_over)
+    dq = t[dq_over] if dq is None else dq
+    dkv = chunks[0] if dkv_over else torch.zeros_like(chunks[0])
+    direct = []
+
+    def span(x):
+        return x.data_ptr(), x.data_ptr() + x.numel() * x.element_size()          # (contiguous, all of them)
+
+    def launch(dout, q, k, v, out, l, dq, acc, first, last, dkv, dkv32, scale, workspace=None):
+        total = 1.0 if first else acc.max().item() + 1.0
+        for written in [x for x in (dkv, dkv32, dq if last else None, None if last else acc) if x is not None]:
+            for read in (dout, q, k, v, out, l):
+                (a, b), (c, d) = span(written), span(read)
+                assert b <= c or d <= a
+        (dq if last else acc).fill_(total)
+        dkv.fill_(7.0)
+        direct.append((last, dkv.data_ptr()))
+        return torch.empty(1, dtype=torch.uint8)
+
+    monkeypatch.setattr(R, "attn_bwd_chunk", launch)
+    R.flash_attn_backward(t["q"], chunks[0], t["o"], lse, t["dout"], dq, dkv, 0.1, ring=LocalRing((W,), 0, chunks))
+    assert bool((dq == W).all())
+    if not (dq_over == "last chunk" and dkv_over and W == 1):       # (dq over the place dkv is in)
+        assert bool((dkv == 7).all())
+    assert direct[-1][0] == (dq_over == "") and (direct[0][1] == dkv.data_ptr()) == (dkv_over == "")
