@@ -84,6 +84,17 @@ struct OnDevice {
   }
 };
 
+// Runs f while other Python threads may run, as every torch operator and every call through ctypes does: an allocation may
+// wait for the device, and a launch waits while the queue is full.
+template <class F>
+int without_gil(F&& f) {
+  struct Released {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Released() { PyEval_RestoreThread(state); }
+  } released;
+  return f();
+}
+
 bool shape4(const Tensor& t, int64_t a, int64_t b, int64_t c, int64_t d) {
   return t.dim() == 4 && t.size(0) == a && t.size(1) == b && t.size(2) == c && t.size(3) == d;
 }
@@ -187,14 +198,17 @@ PyObject* fwd_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   if (lse_given && (!shape3(*lse_given, B, Hq, Sq) || lse_given->scalar_type() != at::kFloat || !lse_given->is_contiguous())) SLOW;
   OnDevice on(q);
   if (!on.current) SLOW;
-  const Tensor out = out_given ? *out_given : at::empty({B, Sq, Hq, D}, q.options().dtype(at::kBFloat16).requires_grad(false));
-  const Tensor lse = lse_given ? *lse_given : at::empty({B, Hq, Sq}, q.options().dtype(at::kFloat).requires_grad(false));
-  const int code = entry.fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), floats(&lse),
-                             B, Sq, Sc, Hq, Hkv, D, q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1),
-                             k.stride(2), v.stride(0), v.stride(1), v.stride(2), out.stride(0), out.stride(1), out.stride(2),
-                             (float)scale, causal ? MHIP_MASK_CAUSAL : MHIP_MASK_NONE,
-                             type == at::kBFloat16 ? MHIP_BF16 : MHIP_E4M3, floats(descale[0]), floats(descale[1]),
-                             floats(descale[2]), on.stream);
+  Tensor out, lse;
+  const int code = without_gil([&] {
+    out = out_given ? *out_given : at::empty({B, Sq, Hq, D}, q.options().dtype(at::kBFloat16).requires_grad(false));
+    lse = lse_given ? *lse_given : at::empty({B, Hq, Sq}, q.options().dtype(at::kFloat).requires_grad(false));
+    return entry.fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), floats(&lse),
+                     B, Sq, Sc, Hq, Hkv, D, q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1),
+                     k.stride(2), v.stride(0), v.stride(1), v.stride(2), out.stride(0), out.stride(1), out.stride(2),
+                     (float)scale, causal ? MHIP_MASK_CAUSAL : MHIP_MASK_NONE,
+                     type == at::kBFloat16 ? MHIP_BF16 : MHIP_E4M3, floats(descale[0]), floats(descale[1]),
+                     floats(descale[2]), on.stream);
+  });
   if (code != MHIP_OK) return refused(code, "mhip_attn_fwd_block");
   return give2(out, lse);
   END_HANDLE_TH_ERRORS
@@ -241,13 +255,16 @@ PyObject* bwd_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   if (acc && (acc->sizes() != q.sizes() || acc->scalar_type() != at::kFloat || !acc->is_contiguous())) SLOW;
   OnDevice on(q);
   if (!on.current) SLOW;
-  const Tensor ws = bwd_workspace(q, Sc, Hkv);
-  const int code = entry.bwd(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), floats(&lse),
-                             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), floats(acc), B, Sq, Sc, Hq, Hkv, D,
-                             q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
-                             dk.stride(0), dk.stride(1), dk.stride(2), dq.stride(0), dq.stride(1), dq.stride(2),
-                             out.stride(0), out.stride(1), out.stride(2), (float)scale,
-                             causal ? MHIP_MASK_CAUSAL : MHIP_MASK_NONE, deterministic, ws.data_ptr(), on.stream);
+  Tensor ws;
+  const int code = without_gil([&] {
+    ws = bwd_workspace(q, Sc, Hkv);
+    return entry.bwd(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), floats(&lse),
+                     dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), floats(acc), B, Sq, Sc, Hq, Hkv, D,
+                     q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
+                     dk.stride(0), dk.stride(1), dk.stride(2), dq.stride(0), dq.stride(1), dq.stride(2),
+                     out.stride(0), out.stride(1), out.stride(2), (float)scale,
+                     causal ? MHIP_MASK_CAUSAL : MHIP_MASK_NONE, deterministic, ws.data_ptr(), on.stream);
+  });
   if (code != MHIP_OK) return refused(code, "mhip_attn_bwd_block");
   // the workspace is (-delta | lse in base 2 | delta), each in a slot rounded up to 4 elements
   const int64_t rows = B * Hq * Sq, slot = (rows + 3) & ~int64_t(3);
@@ -293,16 +310,19 @@ PyObject* bwd_chunk(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     SLOW;
   OnDevice on(q);
   if (!on.current) SLOW;
-  const Tensor ws = kept ? *kept : bwd_workspace(q, Sc, Hkv);
+  Tensor ws;
   auto second16 = [](const Tensor* t) { return t ? static_cast<void*>(static_cast<char*>(t->data_ptr()) + 2 * t->stride(0)) : nullptr; };
-  const int code = entry.chunk(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), floats(&lse),
-                               data(dq), floats(acc), first, last, kept != nullptr, data(dkv), second16(dkv),
-                               floats(dkv32), dkv32 ? floats(dkv32) + dkv32->stride(0) : nullptr, B, Sq, Sc, Hq, Hkv, D,
-                               q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
-                               dkv ? dkv->stride(1) : 0, dkv ? dkv->stride(2) : 0, dkv ? dkv->stride(3) : 0,
-                               dq ? dq->stride(0) : 0, dq ? dq->stride(1) : 0, dq ? dq->stride(2) : 0,
-                               out.stride(0), out.stride(1), out.stride(2), (float)scale, MHIP_MASK_NONE, ws.data_ptr(),
-                               on.stream);
+  const int code = without_gil([&] {
+    ws = kept ? *kept : bwd_workspace(q, Sc, Hkv);
+    return entry.chunk(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), floats(&lse),
+                       data(dq), floats(acc), first, last, kept != nullptr, data(dkv), second16(dkv),
+                       floats(dkv32), dkv32 ? floats(dkv32) + dkv32->stride(0) : nullptr, B, Sq, Sc, Hq, Hkv, D,
+                       q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
+                       dkv ? dkv->stride(1) : 0, dkv ? dkv->stride(2) : 0, dkv ? dkv->stride(3) : 0,
+                       dq ? dq->stride(0) : 0, dq ? dq->stride(1) : 0, dq ? dq->stride(2) : 0,
+                       out.stride(0), out.stride(1), out.stride(2), (float)scale, MHIP_MASK_NONE, ws.data_ptr(),
+                       on.stream);
+  });
   if (code != MHIP_OK) return refused(code, "mhip_attn_bwd_chunk");
   return give(ws);
   END_HANDLE_TH_ERRORS
@@ -333,11 +353,13 @@ PyObject* merge_into(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   OnDevice on(*bo);
   if (!on.current) SLOW;
   auto st = [](const Tensor* x, int i) { return x ? x->stride(i) : int64_t(0); };
-  const int code = entry.merge(floats(t[0]), floats(t[1]), bo->data_ptr(), floats(bl), floats(t[4]), floats(t[5]),
-                               data(t[6]), floats(t[7]), B, Sq, Hq, D, st(t[0], 0), st(t[0], 1), st(t[0], 2),
-                               st(t[1], 0), st(t[1], 1), st(t[1], 2), bo->stride(0), bo->stride(1), bo->stride(2),
-                               bl->stride(0), bl->stride(1), st(t[4], 0), st(t[4], 1), st(t[4], 2), st(t[5], 0),
-                               st(t[5], 1), st(t[5], 2), on.stream);
+  const int code = without_gil([&] {
+    return entry.merge(floats(t[0]), floats(t[1]), bo->data_ptr(), floats(bl), floats(t[4]), floats(t[5]),
+                       data(t[6]), floats(t[7]), B, Sq, Hq, D, st(t[0], 0), st(t[0], 1), st(t[0], 2),
+                       st(t[1], 0), st(t[1], 1), st(t[1], 2), bo->stride(0), bo->stride(1), bo->stride(2),
+                       bl->stride(0), bl->stride(1), st(t[4], 0), st(t[4], 1), st(t[4], 2), st(t[5], 0),
+                       st(t[5], 1), st(t[5], 2), on.stream);
+  });
   if (code != MHIP_OK) return refused(code, "mhip_lse_merge");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -384,7 +406,9 @@ PyObject* merge_many(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   }
   OnDevice on(*out);
   if (!on.current) SLOW;
-  const int code = entry.many(outs, lses, batch, begins, (int)n, out->data_ptr(), floats(lse), B, Sq, Hq, D, ss, sh, on.stream);
+  const int code = without_gil([&] {
+    return entry.many(outs, lses, batch, begins, (int)n, out->data_ptr(), floats(lse), B, Sq, Hq, D, ss, sh, on.stream);
+  });
   if (code != MHIP_OK) return refused(code, "mhip_lse_merge_many");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -403,8 +427,11 @@ PyObject* pack_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   if (lhs && (!shape4(*lhs, B, Sq, Hq, D + 1) || lhs->scalar_type() != at::kFloat || !lhs->is_contiguous())) SLOW;
   OnDevice on(*bo);
   if (!on.current) SLOW;
-  const Tensor dst = at::empty({B, Sq, Hq, D + 1}, bo->options().dtype(at::kFloat).requires_grad(false));
-  const int code = entry.pack(floats(lhs), bo->data_ptr(), floats(bl), floats(&dst), B, Sq, Hq, D, on.stream);
+  Tensor dst;
+  const int code = without_gil([&] {
+    dst = at::empty({B, Sq, Hq, D + 1}, bo->options().dtype(at::kFloat).requires_grad(false));
+    return entry.pack(floats(lhs), bo->data_ptr(), floats(bl), floats(&dst), B, Sq, Hq, D, on.stream);
+  });
   if (code != MHIP_OK) return refused(code, "mhip_pack_reduce");
   return give(dst);
   END_HANDLE_TH_ERRORS
@@ -424,7 +451,7 @@ PyObject* unpack_into(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     SLOW;
   OnDevice on(buf);
   if (!on.current) SLOW;
-  const int code = entry.unpack(floats(&buf), out.data_ptr(), floats(&lse), B, Sq, Hq, D, on.stream);
+  const int code = without_gil([&] { return entry.unpack(floats(&buf), out.data_ptr(), floats(&lse), B, Sq, Hq, D, on.stream); });
   if (code != MHIP_OK) return refused(code, "mhip_unpack");
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -438,11 +465,14 @@ PyObject* quantize_e4m3(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   if (!x || (x->scalar_type() != at::kFloat && x->scalar_type() != at::kBFloat16) || !x->is_contiguous()) SLOW;
   OnDevice on(*x);
   if (!on.current) SLOW;
-  const Tensor xq = at::empty(x->sizes(), x->options().dtype(at::kFloat8_e4m3fn).requires_grad(false));
-  const Tensor ws = at::empty({2}, x->options().dtype(at::kFloat).requires_grad(false));      // scale, scratch
-  float* w = floats(&ws);
-  const int code = entry.quantize(x->data_ptr(), x->scalar_type() == at::kFloat ? MHIP_F32 : MHIP_BF16, x->numel(), xq.data_ptr(),
-                                  w, w + 1, on.stream);
+  Tensor xq, ws;                                   // ws: scale, scratch
+  const int code = without_gil([&] {
+    xq = at::empty(x->sizes(), x->options().dtype(at::kFloat8_e4m3fn).requires_grad(false));
+    ws = at::empty({2}, x->options().dtype(at::kFloat).requires_grad(false));
+    float* w = floats(&ws);
+    return entry.quantize(x->data_ptr(), x->scalar_type() == at::kFloat ? MHIP_F32 : MHIP_BF16, x->numel(), xq.data_ptr(), w, w + 1,
+                          on.stream);
+  });
   if (code != MHIP_OK) return refused(code, "mhip_quantize_e4m3");
   return give2(xq, ws.select(0, 0));
   END_HANDLE_TH_ERRORS

@@ -240,3 +240,33 @@ def test_a_profiler_sees_the_operators():
     counts = {e.key: e.count for e in seen.key_averages()}
     assert counts.get("mercury_amd::_flash_attn_forward") == 4 and counts.get("mercury_amd::_flash_attn_backward") == 1
     assert torch.equal(again[0], out) and torch.equal(again[1], lse)
+
+
+def test_other_threads_run_while_a_launch_blocks():
+    """A launch blocks while the queue is full.  poll(2) stands in for one here: called with the quantiser's arguments --
+    (x, MHIP_BF16 = 0 descriptors, the number of elements as milliseconds, ...) -- it waits and touches nothing."""
+    import threading
+    import time
+
+    x = torch.zeros(400, device="cuda", dtype=torch.bfloat16)
+    table = {name: ctypes.cast(getattr(N.lib(), name), ctypes.c_void_p).value for name in N.EXPORTED_SYMBOLS}
+    poll = ctypes.cast(ctypes.CDLL(None).poll, ctypes.c_void_p).value
+    ticks, stop = [], threading.Event()
+
+    def tick():
+        while not stop.wait(0.005):
+            ticks.append(time.monotonic())
+
+    thread = threading.Thread(target=tick)
+    try:
+        assert N.host.bind({**table, "mhip_quantize_e4m3": poll})
+        thread.start()
+        begin = time.monotonic()
+        assert N.host.quantize_e4m3(x) is not None
+        end = time.monotonic()
+    finally:
+        stop.set()
+        assert N.host.bind(table)
+    thread.join()
+    assert end - begin >= 0.39
+    assert sum(begin + 0.05 < t < end - 0.05 for t in ticks) >= 5
