@@ -170,6 +170,27 @@ PyObject* written(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// (t, *others): whether no other tensor has elements between the first and the last of t's.
+PyObject* apart(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  auto extent = [](const Tensor& t) {
+    const char* first = static_cast<const char*>(t.const_data_ptr());
+    int64_t last = 0;
+    for (int64_t i = 0; i < t.dim(); ++i) last += (t.size(i) - 1) * t.stride(i);
+    return std::make_pair(first, t.numel() ? first + (last + 1) * t.element_size() : first);
+  };
+  for (Py_ssize_t i = 0; i < nargs; ++i)
+    if (!THPVariable_Check(a[i])) SLOW;
+  if (nargs < 1) SLOW;
+  const auto mine = extent(THPVariable_Unpack(a[0]));
+  for (Py_ssize_t i = 1; i < nargs; ++i) {
+    const auto other = extent(THPVariable_Unpack(a[i]));
+    if (other.first < mine.second && mine.first < other.second) Py_RETURN_FALSE;
+  }
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+
 // (q, k, v, softmax_scale, causal, q_descale, k_descale, v_descale, out, lse)
 PyObject* fwd_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
@@ -498,7 +519,7 @@ PyObject* bind(PyObject*, PyObject* table) {
 
 #define FAST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    FAST(undispatched), FAST(written), FAST(fwd_block), FAST(no_dropout), FAST(bwd_block), FAST(bwd_chunk), FAST(merge_into),
+    FAST(undispatched), FAST(written), FAST(apart), FAST(fwd_block), FAST(no_dropout), FAST(bwd_block), FAST(bwd_chunk), FAST(merge_into),
     FAST(merge_many), FAST(pack_block), FAST(unpack_into), FAST(quantize_e4m3),
     {"bind", bind, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};

@@ -109,18 +109,6 @@ def _as_rows(t):
     return t if fine else t.contiguous()
 
 
-def _extent(t):
-    """First and last address of a tensor's elements."""
-    start = t.data_ptr()
-    return start, start + (sum((n - 1) * st for n, st in zip(t.shape, t.stride())) + 1) * t.element_size()
-
-
-def _apart(t, *others):
-    """Whether no other tensor has elements between the first and the last of ``t``'s."""
-    first, last = _extent(t)
-    return all(a >= last or b <= first for a, b in map(_extent, others))
-
-
 _SIDE_STREAMS = {}
 
 
@@ -454,7 +442,7 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
     # operands of other layouts go through the block operator, which copies them where it has to
     carried = (fused_accumulate and aligned_rows(q, dout) and aligned_rows(o) and lse.is_contiguous()
                and q.shape == o.shape == dout.shape)
-    write_dq = carried and aligned_rows(dq) and dq.shape == q.shape and _apart(dq, q, dout, o, lse, kv)
+    write_dq = carried and aligned_rows(dq) and dq.shape == q.shape and N.host.apart(dq, q, dout, o, lse, kv)
     reduce_dq = None
     if not carried and fused_accumulate:
         reduce_dq = torch.zeros(q.shape, dtype=torch.float32, device=q.device)
@@ -476,9 +464,9 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
         if carried:
             mine = chunk_id == own
             direct = (mine and dkv.shape == _kv.shape and aligned_rows(dkv[0], dkv[1])
-                      and _apart(dkv, q, dout, o, lse, _kv))
+                      and N.host.apart(dkv, q, dout, o, lse, _kv))
             if hop is None and write_dq and step > 0:
-                write_dq = _apart(dq, _kv)
+                write_dq = N.host.apart(dq, _kv)
             block_dkv = chunk_grad = None
             if direct:
                 block_dkv = dkv
