@@ -40,7 +40,8 @@ bool bound = false;
 
 using at::Tensor;
 
-// A device tensor that needs nothing of the dispatcher: exactly torch.Tensor, strided, no wrapper of a transform.
+// A device tensor that needs nothing of the dispatcher: exactly torch.Tensor, strided, no wrapper of a transform, no
+// names (which the operators' schemas refuse).
 const Tensor* plain(PyObject* o) {
   if (!THPVariable_CheckExact(o)) return nullptr;
   const Tensor& t = THPVariable_Unpack(o);
@@ -48,7 +49,7 @@ const Tensor* plain(PyObject* o) {
   if (!t.is_cuda() || t.layout() != at::kStrided || keys.has(c10::DispatchKey::Python) ||
       keys.has(c10::DispatchKey::Functionalize) || keys.has(c10::DispatchKey::FuncTorchBatched) ||
       keys.has(c10::DispatchKey::FuncTorchGradWrapper) || keys.has(c10::DispatchKey::Negative) ||
-      keys.has(c10::DispatchKey::Conjugate) || keys.has(c10::DispatchKey::ZeroTensor))
+      keys.has(c10::DispatchKey::Conjugate) || keys.has(c10::DispatchKey::ZeroTensor) || keys.has(c10::DispatchKey::Named))
     return nullptr;
   return &t;
 }

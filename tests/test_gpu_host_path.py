@@ -270,3 +270,17 @@ def test_other_threads_run_while_a_launch_blocks():
     thread.join()
     assert end - begin >= 0.39
     assert sum(begin + 0.05 < t < end - 0.05 for t in ticks) >= 5
+
+
+def test_named_tensors_are_refused_by_the_operator():
+    import warnings
+
+    import mercury_artifact_amd as M
+
+    q, kv, _ = _data()
+    M.attn_fwd_block(q, kv[0], kv[1], 0.1)
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")
+        named = q.refine_names("b", "s", "h", "d")
+    with pytest.raises(RuntimeError, match="[Nn]amed"):
+        M._flash_attn_forward(named, kv[0], kv[1], 0.0, 0.1, False, -1, -1, 0.0, None, False)
