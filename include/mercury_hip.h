@@ -47,8 +47,9 @@ extern "C" {
 
 /* Bumped whenever an entry point's argument list changes (a caller built against another value must not call).
  * 3: the three descales of mhip_attn_fwd_block are device pointers; mhip_attn_bwd_block takes five stride triples.
- * 4: the backward's workspace also holds partial sums (it is larger than its three row arrays); mhip_attn_bwd_chunk. */
-#define MHIP_ABI_VERSION 4
+ * 4: the backward's workspace also holds partial sums (it is larger than its three row arrays); mhip_attn_bwd_chunk.
+ * 5: the workspace's size depends on B, Sq and Hq alone; mhip_attn_fwd_plan, mhip_attn_bwd_plan. */
+#define MHIP_ABI_VERSION 5
 int         mhip_abi_version(void);   /* the MHIP_ABI_VERSION the library was built with */
 int         mhip_version(void);
 /* Optional: per-device set-up the entry points otherwise do on their first call on a device (today: the address
@@ -158,6 +159,18 @@ int mhip_attn_bwd_chunk(const void* dout, const void* q, const void* k, const vo
                         int64_t dq_sb, int64_t dq_ss, int64_t dq_sh,  /* dq       */
                         int64_t o_sb, int64_t o_ss, int64_t o_sh,     /* out      */
                         float softmax_scale, int mask, void* workspace, void* stream);
+
+/*
+ * Which form of the kernels a call of the given sizes takes (host functions, nothing is launched; for tests and profiles,
+ * which would otherwise not know what they ran).  No counterpart in the reference.
+ * mhip_attn_fwd_plan: key groups per workgroup (1, 2 or 4) for MHIP_BF16, wavefronts per workgroup (4 or 8) for MHIP_E4M3;
+ * k_ss and v_ss are the row strides of k and v in elements.
+ * mhip_attn_bwd_plan: 1 if both passes run side by side in one launch, 2 if one after the other; splits[0] and splits[1]
+ * receive the number of workgroups that share a stationary tile of the dQ and of the dK / dV pass.
+ * Negative: an MHIP_E* code.
+ */
+int mhip_attn_fwd_plan(int B, int Sq, int Sc, int Hq, int D, int64_t k_ss, int64_t v_ss, int mask, int dtype);
+int mhip_attn_bwd_plan(int B, int Sq, int Sc, int Hq, int Hkv, int D, int mask, int* splits);
 
 /*
  * LSE-rescale merge.  Replaces the TorchScript `_update_out_and_lse`

@@ -9,6 +9,8 @@ int attn_fwd_bf16(const void* q, const void* k, const void* v, void* out, float*
 int attn_fwd_fp8(const void* q, const void* k, const void* v, void* out, float* lse,
                  int B, int Sq, int Sc, int Hq, int Hkv, int D, const int64_t* strides, float scale, int mask,
                  const float* q_descale, const float* k_descale, const float* v_descale, hipStream_t stream);
+int attn_fwd_bf16_plan(int B, int Sq, int Sc, int Hq, int D, int64_t k_ss, int64_t v_ss, int mask);
+int attn_fwd_fp8_plan(int B, int Sq, int Sc, int Hq, int mask);
 }  // namespace mhip
 
 using namespace mhip;
@@ -76,4 +78,11 @@ extern "C" int mhip_attn_fwd_block(const void* q, const void* k, const void* v, 
                         q_descale, k_descale, v_descale, st);
   }
   return attn_fwd_bf16(q, k, v, out, lse, B, Sq, Sc, Hq, Hkv, D, strides, softmax_scale, mask, st);
+}
+
+extern "C" int mhip_attn_fwd_plan(int B, int Sq, int Sc, int Hq, int D, int64_t k_ss, int64_t v_ss, int mask, int dtype) {
+  if (B < 0 || Sq < 0 || Sc < 0 || Hq <= 0 || D <= 0 || D > 128 || k_ss < 0 || v_ss < 0) return MHIP_EINVAL;
+  if (mask != MHIP_MASK_NONE && mask != MHIP_MASK_CAUSAL) return MHIP_EINVAL;
+  if (dtype == MHIP_E4M3) return attn_fwd_fp8_plan(B, Sq, Sc, Hq, mask);
+  return dtype == MHIP_BF16 ? attn_fwd_bf16_plan(B, Sq, Sc, Hq, D, k_ss, v_ss, mask) : MHIP_EDTYPE;
 }

@@ -949,6 +949,15 @@ extern "C" int64_t mhip_attn_bwd_workspace_bytes(int B, int Sq, int Sc, int Hq, 
   return rows > 0 ? rows + kPartialMost : 0;
 }
 
+extern "C" int mhip_attn_bwd_plan(int B, int Sq, int Sc, int Hq, int Hkv, int D, int mask, int* splits) {
+  if (B < 0 || Sq < 0 || Sc < 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || D <= 0 || D > kD || !splits) return MHIP_EINVAL;
+  if (mask != MHIP_MASK_NONE && mask != MHIP_MASK_CAUSAL) return MHIP_EINVAL;
+  const Plan plan = plan_block(B, Sq, Sc, Hq, Hkv, D, mask == MHIP_MASK_CAUSAL);
+  splits[0] = plan.sq;
+  splits[1] = plan.sk;
+  return plan.joint ? 1 : 2;
+}
+
 namespace {
 // own_scratch: take the workspace from `scratch` (resolved after the arguments have been checked)
 int bwd_block(const void* dout, const void* q, const void* k, const void* v,

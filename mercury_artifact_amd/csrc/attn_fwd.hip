@@ -691,6 +691,13 @@ int key_groups(const FwdParams& p, bool causal) {
 
 }  // namespace
 
+int attn_fwd_bf16_plan(int B, int Sq, int Sc, int Hq, int D, int64_t k_ss, int64_t v_ss, int mask) {
+  FwdParams p{};
+  p.B = B; p.Sq = Sq; p.Sc = Sc; p.Hq = Hq; p.D = D;
+  p.k_ss = k_ss; p.v_ss = v_ss;
+  return key_groups(p, mask == MHIP_MASK_CAUSAL);
+}
+
 int attn_fwd_bf16(const void* q, const void* k, const void* v, void* out, float* lse,
                   int B, int Sq, int Sc, int Hq, int Hkv, int D,
                   const int64_t* st, float scale, int mask, hipStream_t stream) {

@@ -379,6 +379,15 @@ void launch_fp8(const Fp8Params& p, bool causal, hipStream_t stream) {
 
 }  // namespace
 
+// Wavefronts per workgroup.  Four while the launch has at most 256 workgroups of 128 rows: twice the CUs at work.  With
+// more, they take turns on the CUs (us, eight / four: 2048 x 2048 H16, 256 of them, 37.0 / 28.2; 2176 x 2176 H16
+// 39.2 / 54.3; 2048 x 2048 H32 42.8 / 53.2).  Under the causal mask of a square or tall block the longest workgroups hold
+// up the launch until there is twice as much work (2048 x 2048 H20 38.4 / 28.0, H32, 512 workgroups, 39.0 / 33.1, H40
+// 40.1 / 46.1; 4096 x 2048 H16 37.8 / 28.1).
+int attn_fwd_fp8_plan(int B, int Sq, int Sc, int Hq, int mask) {
+  return (int64_t)B * Hq * ((Sq + 127) / 128) > (mask == MHIP_MASK_CAUSAL && Sc <= Sq ? 512 : 256) ? 8 : 4;
+}
+
 int attn_fwd_fp8(const void* q, const void* k, const void* v, void* out, float* lse,
                  int B, int Sq, int Sc, int Hq, int Hkv, int D, const int64_t* st, float scale, int mask,
                  const float* q_descale, const float* k_descale, const float* v_descale, hipStream_t stream) {
@@ -393,13 +402,8 @@ int attn_fwd_fp8(const void* q, const void* k, const void* v, void* out, float* 
   p.o_sb = st[9]; p.o_ss = st[10]; p.o_sh = st[11];
   p.scale = scale;
   p.q_descale = q_descale; p.k_descale = k_descale; p.v_descale = v_descale;
-  // Four wavefronts while the launch has at most 256 workgroups of 128 rows: twice the CUs at work.  With more, they
-  // take turns on the CUs (us, eight / four: 2048 x 2048 H16, 256 of them, 37.0 / 28.2; 2176 x 2176 H16 39.2 / 54.3;
-  // 2048 x 2048 H32 42.8 / 53.2).  Under the causal mask of a square or tall block the longest workgroups hold up the
-  // launch until there is twice as much work (2048 x 2048 H20 38.4 / 28.0, H32, 512 workgroups, 39.0 / 33.1, H40
-  // 40.1 / 46.1; 4096 x 2048 H16 37.8 / 28.1).
   const bool causal = mask == MHIP_MASK_CAUSAL;
-  const bool wide = (int64_t)B * Hq * ((Sq + 127) / 128) > (causal && Sc <= Sq ? 512 : 256);
+  const bool wide = attn_fwd_fp8_plan(B, Sq, Sc, Hq, mask) == 8;
   const int rows = wide ? 256 : 128;
   p.nq_tiles = (Sq + rows - 1) / rows;
   p.total = B * Hq * p.nq_tiles;

@@ -136,11 +136,10 @@ def test_fwd_block_monotone_scores(direction, fp8):
 @pytest.mark.parametrize("D", [128, 64, 40])
 @pytest.mark.parametrize("causal", [False, True])
 def test_fwd_block_monotone_scores_by_head_dim(direction, D, causal):
-    """The same ramp of about 20 binades per key tile on the 64-column instantiation (D = 64: other slot
-    arithmetic for the exponential pairs that ride in the matrix phase, the packed P overwritten right behind two
-    O^T MFMAs) and on a head dimension below 128 of the 128-column one (D = 40), with and without the causal
-    mask, so that the path that moves the reference runs together with masking.  The first 16 head-dim values
-    carry the ramp."""
+    """The same ramp of about 20 binades per key tile on 128 and 64 columns (also with a head dimension below the
+    columns, D = 40), with and without the causal mask, so that the path that moves the reference runs together with
+    masking.  A launch this small runs four key groups; tests/test_gpu_fwd_key_groups.py has the ramp for the other
+    splits.  The first 16 head-dim values carry the ramp."""
     import mercury_artifact_amd as M
 
     B, Sq, Sc, H = 1, 320, 640, 2

@@ -1,0 +1,50 @@
+"""What the sizes of the GPU tests make the launch rules choose (host functions: no GPU needed).  A test names the kernels
+it is for; when a rule moves, these assertions say which kernels have been left without one."""
+import ctypes
+
+import pytest
+
+from mercury_artifact_amd import _native as N
+from tests import test_gpu_fwd_key_groups as G
+
+
+def _columns(D):
+    return 64 if D <= 64 else 96 if D <= 96 else 128
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("columns", [64, 96, 128])
+@pytest.mark.parametrize("groups", [1, 2, 4])
+def test_every_forward_split_has_its_cases(groups, columns, causal):
+    """Edge cases with at least five tiles for every key group, whole and ragged, for each instantiation; and a ramp."""
+    step = 64 if groups == 1 else 128                 # keys that all groups together take per tile (32 each with four)
+    deep = [c for c in G.CASES if c[0] == groups and _columns(c[3]) == columns and c[4] == causal and c[2] > 4 * step]
+    assert deep and any(c[1] % 32 and c[2] % step for c in deep)
+    ramps = [r for r in G.RAMPS if r[0] == groups and _columns(r[3]) == columns]
+    assert ramps and all(r[2] > 4 * step and G.launch(*r, causal) for r in ramps)
+
+
+def test_forward_rule():
+    plan = N.lib().mhip_attn_fwd_plan
+    # rows too far apart for a tile put out of range by its 32-bit offset: one group
+    assert plan(1, 256, 256, 4, 128, 512, 512, 0, N.MHIP_BF16) == 4
+    assert plan(1, 256, 256, 4, 128, 1 << 21, 512, 0, N.MHIP_BF16) == plan(1, 256, 256, 4, 128, 512, 1 << 21, 0, N.MHIP_BF16) == 1
+    assert plan(1, 4096, 4096, 32, 128, 4096, 4096, 0, N.MHIP_BF16) == 1
+    assert plan(1, 256, 256, 4, 144, 512, 512, 0, N.MHIP_BF16) < 0 and plan(1, 256, 256, 4, 64, 512, 512, 0, N.MHIP_F32) < 0
+    # nothing to do, nothing to see: any split does
+    for Sq, Sc in ((0, 64), (64, 0)):
+        assert plan(1, Sq, Sc, 4, 128, 512, 512, 1, N.MHIP_BF16) in (1, 2, 4)
+
+
+def bwd_plan(B, Sq, Sc, Hq, Hkv, D, causal):
+    splits = (ctypes.c_int * 2)()
+    launches = N.lib().mhip_attn_bwd_plan(B, Sq, Sc, Hq, Hkv, D, int(causal), splits)
+    return launches, splits[0], splits[1]
+
+
+def test_backward_rule():
+    assert bwd_plan(1, 4096, 4096, 32, 32, 128, False) == (2, 1, 1)
+    assert bwd_plan(1, 256, 256, 4, 4, 128, False) == (1, 1, 1)
+    assert bwd_plan(1, 2048, 2048, 8, 1, 128, False)[2] > 1
+    assert bwd_plan(1, 0, 64, 4, 4, 128, False) == bwd_plan(1, 64, 0, 4, 4, 128, False) == (2, 1, 1)
+    assert bwd_plan(1, 64, 64, 4, 3, 128, False)[0] < 0
