@@ -5,12 +5,21 @@ The kernels round P and dS to bf16 (relative 2^-9 each, random): rel-L2 of a gra
 within 2^-8 of the sum of the magnitudes that enter it, for which 12 root mean squares are allowed here; bf16 results
 add 2^-9.  Where the gradient is exactly zero (one key: dP = delta) the fp32 sums of D products of N(0,1) values, |dP| up
 to 40, leave up to D 2^-24 40 in dS; 1e-4 is allowed absolutely."""
+import ctypes
+
 import pytest
 import torch
 
 import oracle as O
+from mercury_artifact_amd import _native as N
 
 pytestmark = pytest.mark.gpu
+
+
+def taken(B, Sq, Sc, Hq, Hkv, D, causal):
+    """(launches of the two passes, workgroups per stationary tile of the dQ pass, of the dK / dV pass) of a block."""
+    splits = (ctypes.c_int * 2)()
+    return N.lib().mhip_attn_bwd_plan(B, Sq, Sc, Hq, Hkv, D, int(causal), splits), splits[0], splits[1]
 
 
 def _close(name, got, ref):
@@ -20,14 +29,20 @@ def _close(name, got, ref):
     assert (got - ref).abs().max() <= 12 * 2 ** -8 * rms + 2 ** -8 * ref.abs().max() + 1e-4, name
 
 
-@pytest.mark.parametrize("W,S,Hq,Hkv,D", [(1, 300, 2, 2, 128), (2, 129, 4, 2, 64), (3, 257, 3, 1, 40), (4, 64, 2, 2, 128),
-                                           (2, 400, 8, 1, 128), (2, 193, 4, 2, 96)])
+JOINT = [(1, 300, 2, 2, 128), (2, 129, 4, 2, 64), (3, 257, 3, 1, 40), (4, 64, 2, 2, 128), (2, 400, 8, 1, 128), (2, 193, 4, 2, 96)]
+# one launch per pass: from the second chunk on the dQ pass with eight wavefronts finds lse2 and delta prepared
+IN_TURN = [(3, 130, 128, 128, 64), (3, 130, 128, 64, 88), (3, 130, 128, 128, 128), (2, 257, 128, 128, 40), (3, 257, 128, 128, 96),
+           (2, 257, 128, 64, 128), (4, 65, 256, 256, 128)]
+
+
+@pytest.mark.parametrize("W,S,Hq,Hkv,D", JOINT + IN_TURN)
 @pytest.mark.parametrize("dq_dtype,keep", [(torch.bfloat16, True), (torch.float32, True), (torch.bfloat16, False)])
 def test_backward_step_carries_the_sums(W, S, Hq, Hkv, D, dq_dtype, keep):
     import mercury_artifact_amd as M
 
     print(f"W{W} S{S} Hq{Hq} Hkv{Hkv} D{D} {dq_dtype} keep={keep}", flush=True)
     B, rank, scale = 2, W - 1, D ** -0.5
+    assert taken(B, S, S, Hq, Hkv, D, False)[0] == (2 if (W, S, Hq, Hkv, D) in IN_TURN else 1)
     g = torch.Generator().manual_seed(W * 1000 + S)
     q, dout = (torch.randn(B, S, Hq, D, generator=g).bfloat16() for _ in range(2))
     kvs = [torch.randn(2, B, S, Hkv, D, generator=g).bfloat16() for _ in range(W)]
@@ -50,8 +65,11 @@ def test_backward_step_carries_the_sums(W, S, Hq, Hkv, D, dq_dtype, keep):
         _close(f"dkv {c}", got[c], torch.stack(tuple(rdkv[c])))
 
 
-def _block(B, Sq, Sc, Hq, Hkv, D, causal):
+def _block(B, Sq, Sc, Hq, Hkv, D, causal, launches=1, shared=None):
     import mercury_artifact_amd as M
+
+    plan = taken(B, Sq, Sc, Hq, Hkv, D, causal)
+    assert plan[0] == launches and (shared is None or (max(plan[1:]) > 1) == shared)
 
     print(f"B{B} D{D} Sq{Sq} Sc{Sc} Hq{Hq} Hkv{Hkv} causal={causal}", flush=True)
     g = torch.Generator().manual_seed(D * 1000 + Sq)
@@ -84,7 +102,7 @@ def test_backward_block_on_narrow_heads(D, Sq, Sc, Hq, Hkv, causal):
 @pytest.mark.parametrize("Sq,Sc,causal", [(130, 129, False), (257, 64, True), (300, 385, True)])
 def test_backward_block_in_two_launches(D, Sq, Sc, causal):
     """Enough heads to fill the chip with either pass: one launch each, dQ with eight wavefronts."""
-    _block(2, Sq, Sc, 128, 128, D, causal)
+    _block(2, Sq, Sc, 128, 128, D, causal, launches=2)
 
 
 @pytest.mark.parametrize("D", [40, 88, 128])
@@ -93,15 +111,13 @@ def test_backward_block_in_two_launches(D, Sq, Sc, causal):
 def test_backward_block_with_shared_tiles(B, Sq, Sc, Hq, Hkv, causal, D):
     """Long chains of tiles on few workgroups (grouped heads, one head): their stationary tiles are shared and the sums
     added by the third launch."""
-    _block(B, Sq, Sc, Hq, Hkv, D, causal)
+    _block(B, Sq, Sc, Hq, Hkv, D, causal, shared=True)
 
 
 def test_partial_sums_stay_inside_the_workspace():
     """One workspace, sized with the first chunk, for chunks of other lengths and for both masks, among them launches that
     leave the most partial sums: nothing behind its end is written, and the results are those of a fresh one."""
     import mercury_artifact_amd as M
-    from mercury_artifact_amd import _native as N
-
     B, Sq, Hq, Hkv, D = 1, 1000, 8, 1, 128
     g = torch.Generator(device="cuda").manual_seed(9)
     mk = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
@@ -109,7 +125,7 @@ def test_partial_sums_stay_inside_the_workspace():
     size = N.lib().mhip_attn_bwd_workspace_bytes(B, Sq, 64, Hq, Hkv, D)
     memory = torch.full((size + (32 << 20),), 0xA5, dtype=torch.uint8, device="cuda")
     for Sc, causal in ((64, False), (3000, False), (1000, True), (130, False), (2048, True)):
-        print(f"Sc{Sc} causal={causal}", flush=True)
+        print(f"Sc{Sc} causal={causal} {taken(B, Sq, Sc, Hq, Hkv, D, causal)}", flush=True)
         k, v = kv[0, :, :Sc], kv[1, :, :Sc]
         out, lse = M.attn_fwd_block(q, k, v, 0.1, causal=causal)
         want, got = (tuple(torch.empty_like(t) for t in (q, k, v)) for _ in range(2))

@@ -12,6 +12,7 @@ import pytest
 import torch
 
 import oracle as O
+from mercury_artifact_amd import _native as N
 
 pytestmark = pytest.mark.gpu
 
@@ -166,14 +167,16 @@ def test_fp8_block_smaller_head_dims(D, causal):
 
 
 @pytest.mark.parametrize("D", [64, 96, 128])
-@pytest.mark.parametrize("Sq,Sc,H,causal", [(129, 260, 128, False), (129, 260, 129, False), (257, 130, 88, True), (257, 700, 80, True),
-                                            (257, 257, 170, True), (257, 257, 171, True), (129, 130, 129, True)])
-def test_fp8_block_on_both_workgroup_sizes(Sq, Sc, H, causal, D):
+@pytest.mark.parametrize("waves,Sq,Sc,H,causal", [
+    (4, 129, 260, 128, False), (8, 129, 260, 129, False), (4, 257, 130, 88, True), (4, 257, 700, 80, True),
+    (4, 257, 257, 170, True), (8, 257, 257, 171, True), (8, 129, 130, 129, True)])
+def test_fp8_block_on_both_workgroup_sizes(waves, Sq, Sc, H, causal, D):
     """Both sides of the line between workgroups of four and of eight wavefronts (256 workgroups of 128 rows, 512 under the
     causal mask), rows just past a multiple of either's."""
     import mercury_artifact_amd as M
 
     print(f"fp8 Sq{Sq} Sc{Sc} H{H} D{D} causal={causal}", flush=True)
+    assert N.lib().mhip_attn_fwd_plan(1, Sq, Sc, H, D, H * D, H * D, int(causal), N.MHIP_E4M3) == waves
     (q, k, v), (qq, kq, vq), (sq, sk, sv) = _quantised(1, Sq, Sc, H, H, seed=D + H, D=D)
     scale = D ** -0.5
     deq = (O.dequantize(qq, sq), O.dequantize(kq, sk), O.dequantize(vq, sv))

@@ -1,11 +1,10 @@
 """What the sizes of the GPU tests make the launch rules choose (host functions: no GPU needed).  A test names the kernels
 it is for; when a rule moves, these assertions say which kernels have been left without one."""
-import ctypes
-
 import pytest
 
 from mercury_artifact_amd import _native as N
 from tests import test_gpu_fwd_key_groups as G
+from tests.test_gpu_bwd_chunk import IN_TURN, JOINT, taken as bwd_plan
 
 
 def _columns(D):
@@ -36,15 +35,17 @@ def test_forward_rule():
         assert plan(1, Sq, Sc, 4, 128, 512, 512, 1, N.MHIP_BF16) in (1, 2, 4)
 
 
-def bwd_plan(B, Sq, Sc, Hq, Hkv, D, causal):
-    splits = (ctypes.c_int * 2)()
-    launches = N.lib().mhip_attn_bwd_plan(B, Sq, Sc, Hq, Hkv, D, int(causal), splits)
-    return launches, splits[0], splits[1]
-
-
 def test_backward_rule():
     assert bwd_plan(1, 4096, 4096, 32, 32, 128, False) == (2, 1, 1)
     assert bwd_plan(1, 256, 256, 4, 4, 128, False) == (1, 1, 1)
     assert bwd_plan(1, 2048, 2048, 8, 1, 128, False)[2] > 1
     assert bwd_plan(1, 0, 64, 4, 4, 128, False) == bwd_plan(1, 64, 0, 4, 4, 128, False) == (2, 1, 1)
     assert bwd_plan(1, 64, 64, 4, 3, 128, False)[0] < 0
+
+
+@pytest.mark.parametrize("columns", [64, 96, 128])
+def test_carried_sums_are_tested_in_both_forms(columns):
+    """First, middle and last chunk (three chunks or more) with one launch per pass on every column count."""
+    steps = [c for c in IN_TURN if _columns(c[4]) == columns]
+    assert any(c[0] >= 3 for c in steps) and all(bwd_plan(2, c[1], c[1], *c[2:], False)[0] == 2 for c in steps)
+    assert any(_columns(c[4]) == columns and bwd_plan(2, c[1], c[1], *c[2:], False)[0] == 1 for c in JOINT)
