@@ -74,7 +74,9 @@ def test_fp8_block_matches_oracle(B, Sq, Sc, Hq, Hkv, causal):
 @pytest.mark.parametrize("direction", ["rising", "falling"])
 @pytest.mark.parametrize("binades_per_tile", [0.75, 6.0])
 @pytest.mark.parametrize("causal", [False, True])
-def test_fp8_block_monotone_scores(direction, binades_per_tile, causal):
+@pytest.mark.parametrize("waves,Sq,H,D", [(4, 320, 2, 128), (4, 100, 2, 64), (4, 100, 2, 96), (8, 130, 130, 128), (8, 130, 130, 64),
+                                          (8, 130, 130, 96)])
+def test_fp8_block_monotone_scores(direction, binades_per_tile, causal, waves, Sq, H, D):
     """Scores that climb (or fall) steadily from one 128-key tile to the next.  The kernel keeps the first tile's row
     maximum as the reference of its exponentials and watches the sums of groups of 16 values of 2^4 P instead of the
     maxima: a slow climb (0.75 binades per tile) makes a group sum reach the e4m3 maximum while every single value
@@ -82,8 +84,9 @@ def test_fp8_block_monotone_scores(direction, binades_per_tile, causal):
     is and send the later tiles towards the small end of e4m3."""
     import mercury_artifact_amd as M
 
-    B, Sq, Sc, H, D = 1, 320, 1024, 2, 128
-    print(f"fp8 monotone {direction} {binades_per_tile} causal={causal}", flush=True)
+    B, Sc = 1, 1024
+    print(f"fp8 monotone {direction} {binades_per_tile} causal={causal} Sq{Sq} H{H} D{D}", flush=True)
+    assert N.lib().mhip_attn_fwd_plan(B, Sq, Sc, H, D, H * D, H * D, int(causal), N.MHIP_E4M3) == waves
     g = torch.Generator().manual_seed(91)
     q = torch.randn(B, Sq, H, D, generator=g) * 0.25
     k = torch.randn(B, Sc, H, D, generator=g) * 0.25
@@ -107,14 +110,16 @@ def test_fp8_block_monotone_scores(direction, binades_per_tile, causal):
 
 
 @pytest.mark.parametrize("gap_nats", [4.0, 8.0])
-def test_fp8_block_with_a_dominant_first_key(gap_nats):
+@pytest.mark.parametrize("waves,Sq,H", [(4, 256, 2), (8, 130, 130)])
+def test_fp8_block_with_a_dominant_first_key(gap_nats, waves, Sq, H):
     """One key of the first tile scores ``gap_nats`` above thousands of others (an attention sink).  The kernel's
     reference stays at that key's score, so every other probability sits far down in e4m3 (at 8 nats: in its subnormal
     range, as 2^4 P); their sum still carries a large part of the row's weight and has to come out right."""
     import mercury_artifact_amd as M
 
-    B, Sq, Sc, H, D = 1, 256, 4096, 2, 128
-    print(f"fp8 dominant first key, gap {gap_nats}", flush=True)
+    B, Sc, D = 1, 4096, 128
+    print(f"fp8 dominant first key, gap {gap_nats} Sq{Sq} H{H}", flush=True)
+    assert N.lib().mhip_attn_fwd_plan(B, Sq, Sc, H, D, H * D, H * D, 0, N.MHIP_E4M3) == waves
     g = torch.Generator().manual_seed(int(gap_nats))
     q = torch.randn(B, Sq, H, D, generator=g) * 0.1
     k = torch.randn(B, Sc, H, D, generator=g) * 0.1
