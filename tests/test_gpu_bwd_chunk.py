@@ -87,6 +87,11 @@ def _block(B, Sq, Sc, Hq, Hkv, D, causal, launches=1, shared=None):
         _close(name, got, ref)
     want = (dout.float() * o.bfloat16().float()).sum(-1).transpose(1, 2)
     assert (delta.cpu() - want).abs().max() <= 1e-4
+    # with an accumulator: the same dq, and the sum before its rounding (fp32 addition to 0.25: 2^-24 relative)
+    acc, again = torch.full(dq.shape, 0.25, device="cuda"), torch.full_like(dq, float("nan"))
+    M.attn_bwd_block(*dev, again, torch.empty_like(dkv[0]), torch.empty_like(dkv[1]), scale, causal=causal, dq_acc=acc)
+    assert torch.equal(again, dq)
+    assert bool(((acc - 0.25 - dq.float()).abs() <= 2 ** -8 * dq.float().abs() + 2 ** -22).all())
 
 
 @pytest.mark.parametrize("D", [8, 56, 64, 72, 96, 104])
