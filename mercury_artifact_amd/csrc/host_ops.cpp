@@ -171,6 +171,20 @@ PyObject* written(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// (chunk): whether the kernels take the rows of a chunk (2, B, Sc, Hkv, D) as they are -- contiguous last dimension, 16-byte
+// aligned, the rows of one head within the reach of their 32-bit offsets (2 GiB; 1 GiB below 128 columns).
+PyObject* rows_fit(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 1 || !THPVariable_Check(a[0])) SLOW;
+  const Tensor& t = THPVariable_Unpack(a[0]);
+  const int64_t size = t.element_size(), unit = 16 / size, last = t.dim() - 1;
+  bool fit = last >= 3 && t.stride(last) == 1 && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0;
+  for (int64_t i = 0; fit && i < last; ++i) fit = t.stride(i) % unit == 0;
+  fit = fit && t.size(2) * t.stride(2) * size < int64_t(1) << (t.size(last) == 128 ? 31 : 30);
+  return PyBool_FromLong(fit);
+  END_HANDLE_TH_ERRORS
+}
+
 // (t, *others): whether no other tensor has elements between the first and the last of t's.
 PyObject* apart(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
@@ -520,8 +534,8 @@ PyObject* bind(PyObject*, PyObject* table) {
 
 #define FAST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    FAST(undispatched), FAST(written), FAST(apart), FAST(fwd_block), FAST(no_dropout), FAST(bwd_block), FAST(bwd_chunk), FAST(merge_into),
-    FAST(merge_many), FAST(pack_block), FAST(unpack_into), FAST(quantize_e4m3),
+    FAST(undispatched), FAST(written), FAST(apart), FAST(rows_fit), FAST(fwd_block), FAST(no_dropout), FAST(bwd_block),
+    FAST(bwd_chunk), FAST(merge_into), FAST(merge_many), FAST(pack_block), FAST(unpack_into), FAST(quantize_e4m3),
     {"bind", bind, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_mercury_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -100,13 +100,8 @@ def _block_results(n, q, kv, softmax_scale, dropout_p, causal, window_size, alib
 
 
 def _as_rows(t):
-    """A chunk (2, B, Sc, Hkv, D) if the kernels take its rows as they are -- contiguous last dimension, 16-byte aligned, the
-    rows of one head within the reach of their 32-bit offsets (2 GiB; 1 GiB below 128 columns) -- else a copy."""
-    unit = 16 // t.element_size()
-    reach = 1 << (31 if t.shape[-1] == 128 else 30)
-    fine = (t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(st % unit == 0 for st in t.stride()[:-1])
-            and t.shape[2] * t.stride(2) * t.element_size() < reach)
-    return t if fine else t.contiguous()
+    """A chunk if the kernels take its rows as they are (alignment, 32-bit reach), else a copy."""
+    return t if N.host.rows_fit(t) else t.contiguous()
 
 
 _SIDE_STREAMS = {}
