@@ -473,7 +473,7 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
             # rowsum(dout * o) and the scaled lse are the same for every chunk: worked out with the first one
             usual = _kv.shape == kv.shape
             ws = attn_bwd_chunk(dout, q, _k, _v, o, lse, dq if write_dq else None, reduce_dq, step == 0,
-                                write_dq and hop is None, block_dkv, chunk_grad, softmax_scale,
+                                bool(write_dq and hop is None), block_dkv, chunk_grad, softmax_scale,
                                 prepared if usual else None)
             prepared = ws if usual else prepared
             if mine and not direct:

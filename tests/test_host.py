@@ -449,3 +449,26 @@ def test_backward_step_in_place_writes_nothing_a_launch_still_reads(monkeypatch,
     if not (dq_over == "last chunk" and dkv_over and W == 1):       # (dq over the place dkv is in)
         assert bool((dkv == 7).all())
     assert direct[-1][0] == (dq_over == "") and (direct[0][1] == dkv.data_ptr()) == (dkv_over == "")
+
+
+def test_backward_step_without_the_host_modules_answers(monkeypatch):
+    """A host module that declines every question: copies and staged stores, not a wrong call."""
+    import mercury_artifact_amd.ring as R
+    from mercury_artifact_amd.schedule import LocalRing
+
+    class Declines:
+        def __getattr__(self, name):
+            return lambda *args: None
+
+    def launch(dout, q, k, v, out, lse, dq, acc, first, last, dkv, dkv32, scale, workspace=None):
+        assert type(first) is bool and last is False and acc is not None
+        acc.fill_(3.0)
+        dkv.fill_(7.0)
+        return torch.empty(1, dtype=torch.uint8)
+
+    monkeypatch.setattr(R.N, "host", Declines())
+    monkeypatch.setattr(R, "attn_bwd_chunk", launch)
+    q, kv = torch.zeros(1, 4, 1, 8, dtype=torch.bfloat16), torch.zeros(2, 1, 4, 1, 8, dtype=torch.bfloat16)
+    dq, dkv = torch.zeros_like(q), torch.zeros_like(kv)
+    R.flash_attn_backward(q, kv, q, torch.zeros(1, 1, 4), q, dq, dkv, 0.1, ring=LocalRing((1,), 0, [kv]))
+    assert bool((dq == 3).all()) and bool((dkv == 7).all())
