@@ -3,8 +3,8 @@
 // (v_mfma_f32_32x32x64_f8f6f4, twice the rate of the bf16 one), fp32 softmax.  Not in the reference; same
 // call boundary as the bf16 kernel (utils/flash_attn_dsl.py:159-176) with three extra descale arguments.
 //
-// Same decomposition as the bf16 kernel: 8 wavefronts x 32 Q rows per workgroup, S^T = K Q^T keeps one Q
-// row per lane, P^T feeds the second MFMA from the accumulator registers, K and V tiles are copied
+// Same decomposition as the bf16 kernel: wavefronts of 32 Q rows, eight per workgroup or, in small launches,
+// four; S^T = K Q^T keeps one Q row per lane, P^T feeds the second MFMA from the accumulator registers, K and V tiles are copied
 // global -> LDS without registers in between, four stages deep.  Differences:
 //   * a main-loop tile is 128 keys (as many bytes as the 64-key bf16 tile), rows of 128 bytes whose eight
 //     16-byte chunks are XOR-swizzled;
@@ -55,13 +55,13 @@ __device__ __forceinline__ constexpr int swz8(int row) { return (((row >> 1) & 3
 
 // DB = blocks of 32 head-dim values in O^T: 4 computes on all 128 on-chip columns; 2 and 3 are the instantiations for head
 // dimensions up to 64 and up to 96, which leave out the MFMAs, operand reads and accumulators of the zero columns (1
-// and 2 k-steps of 64 in S^T).  The vector work of a tile stays, which bounds the kernel: 4096 x 4096 H32 takes 112 us
-// instead of 134 at D 64 and 136 instead of 142 at D 96, causal 8192 x 8192 H16/4 D 64 118 instead of 142, 512 x 512 H4
+// and 2 k-steps of 64 in S^T).  The vector work of a tile stays, and it is the larger part (cycles busy at 4096 x 4096
+// H32 D 64: vector 67 %, MFMA 24 %): 4096 x 4096 H32 takes 112 us instead of 134 at D 64 and 136 instead of 142 at D 96, causal 8192 x 8192 H16/4 D 64 118 instead of 142, 512 x 512 H4
 // D 64 11.0 instead of 12.6; results the same.
 //
 // WAVES = wavefronts of 32 Q rows in a workgroup: eight, two per SIMD, or four where a launch of eight leaves half of the
-// CUs without a workgroup.  The vector unit bounds a tile step, so one wavefront per SIMD takes less time
-// for it: 256 x 256 H4 7.6 us instead of 9.1, 2048 x 2048 H16 28.2 / 37.0, 4096 x 4096 H2 47.6 / 66.3, causal 1024 x 1024
+// CUs without a workgroup.  A tile step is vector and matrix work that hardly overlap (62 % and 43 % of the cycles busy
+// with two wavefronts per SIMD at 16384 x 16384), so a wavefront with a SIMD to itself takes less time for it: 256 x 256 H4 7.6 us instead of 9.1, 2048 x 2048 H16 28.2 / 37.0, 4096 x 4096 H2 47.6 / 66.3, causal 1024 x 1024
 // H32/8 17.2 / 22.5; results the same.
 template <bool CAUSAL, int DB, int WAVES>
 __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const Fp8Params p) {

@@ -5,8 +5,9 @@ name (utils/flash_attn_dsl.py:127-180, 182-235, 237-291, 345-408; utils/attn_bwd
 ``ring`` keyword: the :class:`~mercury_artifact_amd.schedule.LocalRing` that stands in for the
 neighbour exchange.  The body is the loop the code generator emits for that template
 (mercury/backend/pytorch/codegen.py:264-355, 443-523): take the current KV chunk, start the hop for
-the next one, run the block kernel through ``_flash_attn_forward(**params)``, fold with
-``update_out_and_lse``, and store after the last step.
+the next one, run the block kernel, fold with ``update_out_and_lse``, and store after the last step.  A
+forward driver's blocks go through ``_flash_attn_forward`` unless it would do nothing but call the kernel;
+then they are written straight into places allocated once per step.
 
 Two defaults of the forward drivers depart from the literal sequence without changing what is computed:
 ``deferred_merge=True`` keeps the bf16 block results of all chunks and folds them with ONE

@@ -472,3 +472,19 @@ def test_backward_step_without_the_host_modules_answers(monkeypatch):
     dq, dkv = torch.zeros_like(q), torch.zeros_like(kv)
     R.flash_attn_backward(q, kv, q, torch.zeros(1, 1, 4), q, dq, dkv, 0.1, ring=LocalRing((1,), 0, [kv]))
     assert bool((dq == 3).all()) and bool((dkv == 7).all())
+
+
+def test_documents_state_the_abi_version_and_every_entry_point():
+    """The stub of INTEGRATION.md asserts the header's version, and its table names all the library exports."""
+    import os
+    import re
+
+    from mercury_artifact_amd import _native as N
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    text = open(os.path.join(root, "INTEGRATION.md")).read()
+    header = open(os.path.join(root, "include", "mercury_hip.h")).read()
+    assert set(re.findall(r"mhip_abi_version\(\) == (\d+)", text) + re.findall(r"`MHIP_ABI_VERSION` \((\d+)\)", text)) == {str(N.ABI_VERSION)}
+    assert re.findall(r"#define MHIP_ABI_VERSION (\d+)", header) == [str(N.ABI_VERSION)]
+    assert f"\n * {N.ABI_VERSION}: " in header                      # what the value changed
+    assert [name for name in N.EXPORTED_SYMBOLS if f"`{name}`" not in text] == []
