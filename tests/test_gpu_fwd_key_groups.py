@@ -12,10 +12,14 @@ from mercury_artifact_amd import _native as N
 
 pytestmark = pytest.mark.gpu
 
+# B, Hq, Hkv of a small, a larger and a large launch
+LAUNCHES = {4: (1, 3, 1), 2: (2, 64, 8), 1: (4, 64, 8)}
 EDGES = [
     # Sq, Sc, D: rows around 32, 64, 128, 256, keys around 32, 64, 128, 256 and the rings' wrap
     (1, 1, 128), (31, 32, 128), (64, 33, 128), (65, 127, 64), (129, 128, 128), (130, 129, 40), (255, 257, 128),
     (257, 520, 64), (192, 700, 96), (33, 65, 72), (129, 257, 96),
+]
+DEEP = [
     # five and more tiles for every key group, the last one whole, of one key, or short of one
     (65, 640, 64), (100, 641, 96), (129, 703, 128), (257, 385, 64), (161, 321, 40), (130, 447, 72), (33, 769, 104),
     (65, 673, 128),
@@ -35,7 +39,7 @@ def launch(groups, Sq, Sc, D, causal):
     return next((h for h in HEADS if taken(h[0], Sq, Sc, h[1], h[2], D, causal) == groups), None)
 
 
-CASES = [(groups, Sq, Sc, D, causal) for groups in (4, 2, 1) for Sq, Sc, D in EDGES for causal in (False, True)
+CASES = [(groups, Sq, Sc, D, causal) for groups in (4, 2, 1) for Sq, Sc, D in EDGES + DEEP for causal in (False, True)
          if launch(groups, Sq, Sc, D, causal)]
 
 
@@ -53,8 +57,24 @@ def _compare(q, kv, scale, causal, tag):
     assert bool(((lse[seen] - rl[seen]).abs() <= 1e-5 * rl[seen].abs().clamp_min(1.0)).all()), tag
 
 
+@pytest.mark.parametrize("groups", [4, 2, 1])
+@pytest.mark.parametrize("Sq,Sc,D", EDGES)
+def test_key_groups_at_tile_edges(groups, Sq, Sc, D):
+    """Three launch sizes with whatever split the rule gives them (the largest has one key group at most of the edges)."""
+    B, Hq, Hkv = LAUNCHES[groups]
+    if groups == 1 and Sq * Sc > 140000:
+        B = 2
+    for causal in (False, True):
+        tag = f"{taken(B, Sq, Sc, Hq, Hkv, D, causal)} groups B{B} Hq{Hq} Sq{Sq} Sc{Sc} D{D} causal={causal}"
+        print(tag, flush=True)
+        g = torch.Generator().manual_seed(Sq * 1009 + Sc)
+        q = torch.randn(B, Sq, Hq, D, generator=g).bfloat16()
+        kv = torch.randn(2, B, Sc, Hkv, D, generator=g).bfloat16()
+        _compare(q, kv, D ** -0.5, causal, tag)
+
+
 @pytest.mark.parametrize("groups,Sq,Sc,D,causal", CASES)
-def test_key_groups_at_tile_edges(groups, Sq, Sc, D, causal):
+def test_every_split_at_its_edges(groups, Sq, Sc, D, causal):
     B, Hq, Hkv = launch(groups, Sq, Sc, D, causal)
     tag = f"groups {groups} B{B} Hq{Hq} Hkv{Hkv} Sq{Sq} Sc{Sc} D{D} causal={causal}"
     print(tag, flush=True)

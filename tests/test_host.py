@@ -475,7 +475,7 @@ def test_backward_step_without_the_host_modules_answers(monkeypatch):
 
 
 def test_documents_state_the_abi_version_and_every_entry_point():
-    """The stub of INTEGRATION.md asserts the header's version, and its table names all the library exports."""
+    """The integration notes: their stub asserts the header's version, and their table names all the library exports."""
     import os
     import re
 

@@ -1,10 +1,10 @@
 """What the sizes of the GPU tests make the launch rules choose (host functions: no GPU needed).  A test names the kernels
 it is for; when a rule moves, these assertions say which kernels have been left without one."""
 import pytest
+import test_gpu_fwd_key_groups as G
+from test_gpu_bwd_chunk import IN_TURN, JOINT, taken as bwd_plan
 
 from mercury_artifact_amd import _native as N
-from tests import test_gpu_fwd_key_groups as G
-from tests.test_gpu_bwd_chunk import IN_TURN, JOINT, taken as bwd_plan
 
 
 def _columns(D):
