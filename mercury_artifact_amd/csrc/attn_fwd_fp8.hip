@@ -18,6 +18,12 @@
 //     probabilities keep their relative precision; the reference score of a row is its first tile's maximum
 //     and moves only when the sum of a group of 16 values of 2^4 P reaches the e4m3 maximum of 448 (the sums
 //     are watched, not the maxima: the common path has no maximum, no cross-lane exchange, no rescale of O).
+//
+// What bounds it: the vector work of the softmax (64 fma, exponentials and adds and 32 conversions per 128 keys and lane,
+// about 1470 cycles beside 1024 of MFMA) and, with both units at work, the board's power.  A tile is therefore handled
+// as two halves, the MFMAs of the halves before and after threaded through the exponentials of the current one: at 16384 x
+// 16384 H32 4.07 M cycles instead of 4.86 M (vector unit 72 % busy instead of 62 %, matrix pipe 52 % instead of 43 %), of
+// which the clock gives a part back (1.88 GHz instead of 2.0): 2078 us instead of 2212.
 #include "mhip_common.hpp"
 
 namespace mhip {
@@ -55,14 +61,13 @@ __device__ __forceinline__ constexpr int swz8(int row) { return (((row >> 1) & 3
 
 // DB = blocks of 32 head-dim values in O^T: 4 computes on all 128 on-chip columns; 2 and 3 are the instantiations for head
 // dimensions up to 64 and up to 96, which leave out the MFMAs, operand reads and accumulators of the zero columns (1
-// and 2 k-steps of 64 in S^T).  The vector work of a tile stays, and it is the larger part (cycles busy at 4096 x 4096
-// H32 D 64: vector 67 %, MFMA 24 %): 4096 x 4096 H32 takes 112 us instead of 134 at D 64 and 136 instead of 142 at D 96, causal 8192 x 8192 H16/4 D 64 118 instead of 142, 512 x 512 H4
-// D 64 11.0 instead of 12.6; results the same.
+// and 2 k-steps of 64 in S^T).  The vector work of a tile stays, and it is the larger part: 4096 x 4096 H32 takes 104.6 us
+// at D 64 and 129.8 at D 96 where 128 columns take 139.2; results the same.
 //
 // WAVES = wavefronts of 32 Q rows in a workgroup: eight, two per SIMD, or four where a launch of eight leaves half of the
-// CUs without a workgroup.  A tile step is vector and matrix work that hardly overlap (62 % and 43 % of the cycles busy
-// with two wavefronts per SIMD at 16384 x 16384), so a wavefront with a SIMD to itself takes less time for it: 256 x 256 H4 7.6 us instead of 9.1, 2048 x 2048 H16 28.2 / 37.0, 4096 x 4096 H2 47.6 / 66.3, causal 1024 x 1024
-// H32/8 17.2 / 22.5; results the same.
+// CUs without a workgroup.  A wavefront with a SIMD to itself takes less time for a tile than two that share one
+// (four / eight): 2048 x 2048 H16 24.2 / 32.4 us, 4096 x 4096 H2 39.8 / 56.9, causal 1024 x 1024 H32/8 15.5 / 21.3; results
+// the same.
 template <bool CAUSAL, int DB, int WAVES>
 __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const Fp8Params p) {
   static_assert(WAVES == 8 || WAVES == 4, "two wavefronts per SIMD or one");
@@ -141,28 +146,26 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
   const int k_tile_bytes = (int)(kBN * p.k_ss);
   const int v_tile_bytes = (int)(kBN * p.v_ss);
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem + wave * (kCpy * 1024);
-  auto copy_tile = [&](int t, int stage) {
-#pragma unroll
-    for (int u = 0; u < kCpy; ++u) copy16_to_lds(krs, lds_base + stage * kTileBytes + u * 1024, kvoff[u], t * k_tile_bytes);
-#pragma unroll
-    for (int u = 0; u < kCpy; ++u)
-      copy16_to_lds(vrs, lds_base + kVBase + stage * kTileBytes + u * 1024, vvoff[u], t * v_tile_bytes);
-  };
+  auto copy_k = [&](int u, int t) { copy16_to_lds(krs, lds_base + (t & 3) * kTileBytes + u * 1024, kvoff[u], t * k_tile_bytes); };
+  auto copy_v = [&](int u, int t) { copy16_to_lds(vrs, lds_base + kVBase + (t & 3) * kTileBytes + u * 1024, vvoff[u], t * v_tile_bytes); };
 
   // K operand of S^T: MFMA row m of block mb is key 32 mb + pi(m), pi(8 g + 4 h + e) = 16 h + 4 g + e, so
   // that accumulator register i of lane half hf is key 32 mb + 16 hf + i.  The lane reads chunks
   // 4 ks + 2 hf and 4 ks + 2 hf + 1 of that row.
   const int pi = 16 * ((ln >> 2) & 1) + 4 * (ln >> 3) + (ln & 3);
-  int k_rd[KK][2];                                    // [ks][second 16 bytes]  + mb * 4096
+  // k_a and v_a hold the LDS addresses inside the stage that is read next and move on in place; everything else about an
+  // address is an immediate offset.
+  const int lds_smem = (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+  int k_a[KK][2];                                     // [ks][second 16 bytes]  + mb * 4096
 #pragma unroll
   for (int ks = 0; ks < KK; ++ks)
 #pragma unroll
-    for (int u = 0; u < 2; ++u) k_rd[ks][u] = pi * 128 + (((4 * ks + 2 * hf + u) ^ swz8(pi)) << 4);
+    for (int u = 0; u < 2; ++u) k_a[ks][u] = lds_smem + pi * 128 + (((4 * ks + 2 * hf + u) ^ swz8(pi)) << 4);
   // V^T operand of O^T for head-dim block db and k-step ks2 (keys 64 ks2 .. +63): bytes 8 n .. 8 n + 7 of
   // the lane's 32 are keys 64 ks2 + 32 (n / 2) + 16 hf + 8 (n % 2) + 0..7, the keys of its P registers.
   // One ds_read_b64_tr_b8 per n: within 16 lanes, lane s supplies the address of row (first key) + s/2,
   // head-dim bytes 8 (s%2) .. +7 of the 16-column strip, and receives column s.
-  int v_rd[DB][2];                                    // [db][n % 2]  + ks2 * 8192 + (n / 2) * 4096
+  int v_a[DB][2];                                     // [db][n % 2]  + ks2 * 8192 + (n / 2) * 4096
   {
     const int s16 = lane & 15, strip = (lane >> 4) & 1;
 #pragma unroll
@@ -170,24 +173,25 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
 #pragma unroll
       for (int o = 0; o < 2; ++o) {
         const int row = 16 * hf + 8 * o + (s16 >> 1);
-        v_rd[db][o] = row * 128 + (((2 * db + strip) ^ swz8(row)) << 4) + (s16 & 1) * 8;
+        v_a[db][o] = lds_smem + kVBase + row * 128 + (((2 * db + strip) ^ swz8(row)) << 4) + (s16 & 1) * 8;
       }
   }
   typedef __attribute__((address_space(3))) i32x2* lds_i32x2;
-  auto read_k = [&](const unsigned char* ks_, int mb, int ks) -> i32x8 {
-    const u32x4 lo = *reinterpret_cast<const u32x4*>(ks_ + k_rd[ks][0] + mb * 4096);
-    const u32x4 hi = *reinterpret_cast<const u32x4*>(ks_ + k_rd[ks][1] + mb * 4096);
+  typedef __attribute__((address_space(3))) const u32x4* lds_u32x4;
+  auto read_k = [&](int mb, int ks) -> i32x8 {
+    const u32x4 lo = *(lds_u32x4)(uintptr_t)(uint32_t)(k_a[ks][0] + mb * 4096);
+    const u32x4 hi = *(lds_u32x4)(uintptr_t)(uint32_t)(k_a[ks][1] + mb * 4096);
     i32x8 r;
 #pragma unroll
     for (int e = 0; e < 4; ++e) { r[e] = (int)lo[e]; r[4 + e] = (int)hi[e]; }
     return r;
   };
-  auto read_v = [&](const unsigned char* vs_, int db, int ks2) -> i32x8 {
+  auto read_v = [&](int db, int ks2) -> i32x8 {
     i32x8 r;
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
       const i32x2 t = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-          (lds_i32x2)(vs_ + v_rd[db][n & 1] + ks2 * 8192 + (n >> 1) * 4096));
+          (lds_i32x2)(uintptr_t)(uint32_t)(v_a[db][n & 1] + ks2 * 8192 + (n >> 1) * 4096));
       r[2 * n] = t[0]; r[2 * n + 1] = t[1];
     }
     return r;
@@ -206,16 +210,18 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
   // the row maximum seen so far (O and the running sum are rescaled) and the tile's exponentials are redone, after
   // which every 2^4 P is at most 16.
   float m_ref = 0.f, msc = -kPShift, l_run = 0.f;      // l_run sums 2^4 P (this lane's half of the keys)
-  float rs_sum = 0.f;
-  i32x8 pf[2] = {};          // P^T operands; pf[ks2]: dwords 0-3 = keys of block 2 ks2, dwords 4-7 = block 2 ks2 + 1
   const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  f32x16 s[4];               // S^T tile: 128 keys x 32 q rows per wave
-  auto set_reference = [&](bool first) {
+  f32x16 sa[2], sb[2];       // S^T of a tile's first and second half: 64 keys x 32 q rows per wavefront each
+  i32x8 pa = {}, pb = {};    // their P^T operands: dwords 0-3 = keys of the half's first 32-key block, dwords 4-7 = second
+  auto largest = [&](const f32x16 (&s)[2]) -> float {
     float mx = s[0][0];
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
+    for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
       for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[mb][j]);
+    return mx;
+  };
+  auto set_reference = [&](bool first, float mx) {     // mx: the largest of this lane's scores
     mx = pair_max(mx);
     const bool move = first ? (mx != -INFINITY) : (mx > m_ref);      // false for NaN
     if (!first) {
@@ -229,46 +235,126 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
     m_ref = move ? mx : m_ref;
     msc = m_ref * scale_log2 - kPShift;            // exponent of 2^4 P
   };
-  // 2^4 P of the tile into the P^T operands; returns whether one of the four group sums reached the trigger (or is
-  // inf / NaN) and leaves their total in rs_sum.  s stays intact, so that the pass can be repeated against a new
-  // reference.
-  auto exponentials = [&]() -> bool {
-    bool big = false;
-    rs_sum = 0.f;
+  // 2^4 P of a half into its P^T operand, in eight groups of four scores: step g works out the arguments of group g, adds
+  // up and converts group g - 1 and takes the exponentials of group g, so that nothing waits for the instruction
+  // before it.  r[] are the sums of the two 32-key blocks (this lane's 16 keys of each).  The scores stay intact, so that
+  // the pass can be repeated against a new reference.
+  float r[2], x[2][4];
+  auto vector_step = [&](int g, const f32x16 (&s)[2], i32x8& pw) {
+    if (g < 8) {
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
-      float e[16];
-      float r = 0.f;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        e[j] = fast_exp2(__builtin_fmaf(s[mb][j], scale_log2, -msc));
-        r += e[j];
-      }
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        // the first conversion writes the low half and the second the high half of the operand register, so
-        // what it held before (the P of the previous tile) needs no clearing
-        int packed = pf[mb >> 1][(mb & 1) * 4 + w];
-        packed = __builtin_amdgcn_cvt_pk_fp8_f32(e[4 * w], e[4 * w + 1], packed, false);
-        packed = __builtin_amdgcn_cvt_pk_fp8_f32(e[4 * w + 2], e[4 * w + 3], packed, true);
-        pf[mb >> 1][(mb & 1) * 4 + w] = packed;
-      }
-      big = big || !(r < kTrigger);
-      rs_sum += r;
+      for (int j = 0; j < 4; ++j) x[g & 1][j] = __builtin_fmaf(s[g >> 2][(g & 3) * 4 + j], scale_log2, -msc);
     }
-    return big;
+    if (g > 0) {
+      const int o = g - 1;
+      const float (&e)[4] = x[o & 1];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) r[o >> 2] = (o & 3) == 0 && j == 0 ? e[0] : r[o >> 2] + e[j];
+      // the first conversion writes the low half and the second the high half of the operand register, so
+      // what it held before needs no clearing
+      int packed = pw[o];
+      packed = __builtin_amdgcn_cvt_pk_fp8_f32(e[0], e[1], packed, false);
+      packed = __builtin_amdgcn_cvt_pk_fp8_f32(e[2], e[3], packed, true);
+      pw[o] = packed;
+    }
+    if (g < 8) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[g & 1][j] = fast_exp2(x[g & 1][j]);
+    }
+  };
+  auto mask_half = [&](f32x16 (&s)[2], int kv0) {
+    bool need_mask = kv0 + kBN / 2 > p.Sc;
+    if (CAUSAL) need_mask = need_mask || (kv0 + kBN / 2 - 1 > q0 + causal_shift);
+    if (need_mask) {
+      int lim = p.Sc - 1;
+      if (CAUSAL) { const int c = my_q + causal_shift; lim = c < lim ? c : lim; }
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const int key = kv0 + mb * 32 + hf * 16 + j;
+          if (key > lim) s[mb][j] = -INFINITY;
+        }
+    }
+  };
+  // after a half's last vector step: move the reference and repeat if a sum reached the trigger (or is inf / NaN)
+  auto finish_half = [&](const f32x16 (&s)[2], i32x8& pw) {
+    if (__builtin_amdgcn_ballot_w64(!(r[0] < kTrigger) || !(r[1] < kTrigger)) != 0) {
+      set_reference(false, largest(s));
+#pragma unroll
+      for (int g = 0; g <= 8; ++g) vector_step(g, s, pw);
+    }
+    l_run += r[0] + r[1];
   };
 
-  // Tile t lives in stage t % 4 of the K and the V ring.  An iteration starts by waiting for this
-  // wavefront's copies of tile t (those of tiles t+1 and t+2 stay in flight) and a barrier: after it tile t
-  // is complete for every wavefront and nobody reads tile t-1 any more, whose stages then receive tile t+3.
-  // Tiles past the end are copied as zeros so that the number of copies in flight stays the same.
+  // Tile t lives in stage t % 4 of the K and the V ring and is processed as two halves of 64 keys.  Every phase of the
+  // main loop is one sequence of kSlots MFMAs, S^T of the half after the current one and O^T of the half before it, with
+  // the exponentials of the current half between them: the matrix pipe and the vector unit are at work at the same time
+  // in every wavefront, whichever way the two wavefronts of a SIMD happen to be aligned.
+  //   phase 0 of tile t   S^T(t, second half)    O^T(t-1, second half)   exponentials (t, first half)
+  //   phase 1             S^T(t+1, first half)   O^T(t, first half)      exponentials (t, second half)
+  // The LDS operand of slot i+2 is read in slot i, across phase and tile boundaries.  An iteration starts by waiting for
+  // this wavefront's copies of K(t+1) and V(t) (those of K(t+2) and V(t+1) stay in flight) and a barrier: after it
+  // they are complete for every wavefront and nobody reads K(t-1) and V(t-2) any more, whose stages then receive K(t+3)
+  // and V(t+2).  Tiles past the end are copied as zeros so that the number of copies in flight stays the same.
+  constexpr int kSlotsS = 2 * KK, kSlots = kSlotsS + DB;
+  i32x8 ring[2];
+  auto read_slot = [&](int half, int i) -> i32x8 {         // half: which phase the slot belongs to
+    if (i >= kSlots) { i -= kSlots; half ^= 1; }
+    if (i < kSlotsS) return read_k((half ? 0 : 2) + (i & 1), i >> 1);
+    return read_v(i - kSlotsS, half ? 0 : 1);
+  };
+  auto s_mfma = [&](int i, const i32x8& a, f32x16 (&s)[2]) {
+    s[i & 1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, qf[i >> 1], i < 2 ? zero : s[i & 1], 0, 0, 0, 0, 0, 0);
+  };
+  auto o_mfma = [&](int db, const i32x8& a, const i32x8& pw) {
+    o_acc[db] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, pw, o_acc[db], 0, 0, 0, 0, 0, 0);
+  };
+  auto phase = [&](int half, int t, f32x16 (&cur)[2], f32x16 (&next)[2], const i32x8& p_before, i32x8& p_cur) {
+    mask_half(cur, t * kBN + half * (kBN / 2));
+#pragma unroll
+    for (int i = 0; i < kSlots; ++i) {
+      i32x8& operand = ring[(half * kSlots + i) & 1];
+      if (i < kSlotsS) s_mfma(i, operand, next);
+      else o_mfma(i - kSlotsS, operand, p_before);
+      operand = read_slot(half, i + 2);
+      if (half == 0) {
+#pragma unroll
+        for (int c = i; c < 2 * kCpy; c += kSlots) {
+          if (c < kCpy) copy_k(c, t + 3);
+          else copy_v(c - kCpy, t + 2);
+        }
+        // the last K read of this phase was slot kSlotsS - 1's, the last V read slot kSlots - 1's
+        if (i == kSlotsS - 2) {
+          const int step = ((t + 1) & 3) == 0 ? -3 * kTileBytes : kTileBytes;
+#pragma unroll
+          for (int ks = 0; ks < KK; ++ks) { k_a[ks][0] += step; k_a[ks][1] += step; }
+        }
+        if (i == kSlots - 2) {                       // (V(0) stands in for V(-1), whose P is zero)
+          const int step = t == 0 ? 0 : (t & 3) == 0 ? -3 * kTileBytes : kTileBytes;
+#pragma unroll
+          for (int db = 0; db < DB; ++db) { v_a[db][0] += step; v_a[db][1] += step; }
+        }
+      }
+#pragma unroll
+      for (int g = i * 8 / kSlots; g < (i + 1) * 8 / kSlots; ++g) vector_step(g, cur, p_cur);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    vector_step(8, cur, p_cur);
+    finish_half(cur, p_cur);
+  };
+
   if (ntiles > 0) {
-    copy_tile(0, 0);
-    copy_tile(1, 1);
-    copy_tile(2, 2);
-  }
-  {
+#pragma unroll
+    for (int u = 0; u < kCpy; ++u) copy_k(u, 0);
+#pragma unroll
+    for (int u = 0; u < kCpy; ++u) copy_v(u, 0);
+#pragma unroll
+    for (int u = 0; u < kCpy; ++u) copy_k(u, 1);
+#pragma unroll
+    for (int u = 0; u < kCpy; ++u) copy_k(u, 2);
+#pragma unroll
+    for (int u = 0; u < kCpy; ++u) copy_v(u, 1);
     const int row = my_q < p.Sq ? my_q : p.Sq - 1;
     const uint8_t* qp = p.q + b * p.q_sb + (int64_t)row * p.q_ss + hq * p.q_sh + hf * 32;
 #pragma unroll
@@ -283,56 +369,28 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
     // pin the loads here: the copies are invisible to the compiler's wait counting
 #pragma unroll
     for (int ks = 0; ks < KK; ++ks) asm volatile("" : "+v"(qf[ks]));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int i = 0; i < kSlotsS; ++i) {
+      s_mfma(i, read_k(i & 1, i >> 1), sa);
+      s_mfma(i, read_k(2 + (i & 1), i >> 1), sb);     // here for the maximum; phase 0 computes it again
+    }
+    mask_half(sa, 0);
+    mask_half(sb, kBN / 2);
+    set_reference(true, fmaxf(largest(sa), largest(sb)));
+    ring[0] = read_slot(0, 0);
+    ring[1] = read_slot(0, 1);
   }
   for (int t = 0; t < ntiles; ++t) {
-    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(4 * kCpy) : "memory");      // two tiles of 2 kCpy copies each
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * kCpy) : "memory");
     __builtin_amdgcn_s_barrier();
-    copy_tile(t + 3, (t + 3) & 3);
-    const unsigned char* ks_ = smem + (t & 3) * kTileBytes;
-    const unsigned char* vs_ = smem + kVBase + (t & 3) * kTileBytes;
-
-    // ---- S^T tile ---------------------------------------------------------------------------------------
+    phase(0, t, sa, sb, pb, pa);
+    phase(1, t, sb, sa, pa, pb);
+  }
+  if (ntiles > 0) {
 #pragma unroll
-    for (int ks = 0; ks < KK; ++ks) {
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
-        const i32x8 kf = read_k(ks_, mb, ks);
-        s[mb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(kf, qf[ks], ks == 0 ? zero : s[mb], 0, 0, 0, 0, 0, 0);
-      }
-    }
-
-    const int kv0 = t * kBN;
-    bool need_mask = kv0 + kBN > p.Sc;
-    if (CAUSAL) need_mask = need_mask || (kv0 + kBN - 1 > q0 + causal_shift);
-    if (need_mask) {
-      int lim = p.Sc - 1;
-      if (CAUSAL) { const int c = my_q + causal_shift; lim = c < lim ? c : lim; }
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const int key = kv0 + mb * 32 + hf * 16 + j;
-          if (key > lim) s[mb][j] = -INFINITY;
-        }
-    }
-
-    // ---- softmax against a reference that moves only when it has to -----------------------------------------
-    if (t == 0) set_reference(true);
-    if (__builtin_amdgcn_ballot_w64(exponentials()) != 0) {
-      set_reference(false);
-      exponentials();
-    }
-    l_run += rs_sum;
-
-    // ---- O^T += V^T P^T -----------------------------------------------------------------------------------
-#pragma unroll
-    for (int ks2 = 0; ks2 < 2; ++ks2) {
-#pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        const i32x8 vf = read_v(vs_, db, ks2);
-        o_acc[db] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf, pf[ks2], o_acc[db], 0, 0, 0, 0, 0, 0);
-      }
-    }
+    for (int db = 0; db < DB; ++db) o_mfma(db, read_v(db, 1), pb);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the zero-filled copies of tiles past the end
 
@@ -380,10 +438,10 @@ void launch_fp8(const Fp8Params& p, bool causal, hipStream_t stream) {
 }  // namespace
 
 // Wavefronts per workgroup.  Four while the launch has at most 256 workgroups of 128 rows: twice the CUs at work.  With
-// more, they take turns on the CUs (us, eight / four: 2048 x 2048 H16, 256 of them, 37.0 / 28.2; 2176 x 2176 H16
-// 39.2 / 54.3; 2048 x 2048 H32 42.8 / 53.2).  Under the causal mask of a square or tall block the longest workgroups hold
-// up the launch until there is twice as much work (2048 x 2048 H20 38.4 / 28.0, H32, 512 workgroups, 39.0 / 33.1, H40
-// 40.1 / 46.1; 4096 x 2048 H16 37.8 / 28.1).
+// more, they take turns on the CUs (us, eight / four: 2048 x 2048 H16, 256 of them, 32.4 / 24.2; 2176 x 2176 H16
+// 34.2 / 46.5; 2048 x 2048 H32 39.7 / 46.3).  Under the causal mask of a square or tall block the longest workgroups hold
+// up the launch until there is twice as much work (2048 x 2048 H20 35.2 / 24.4, H32, 512 workgroups, 36.6 / 30.3, H40
+// 38.0 / 42.0; 4096 x 2048 H16 34.6 / 24.6).
 int attn_fwd_fp8_plan(int B, int Sq, int Sc, int Hq, int mask) {
   return (int64_t)B * Hq * ((Sq + 127) / 128) > (mask == MHIP_MASK_CAUSAL && Sc <= Sq ? 512 : 256) ? 8 : 4;
 }

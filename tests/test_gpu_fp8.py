@@ -71,6 +71,28 @@ def test_fp8_block_matches_oracle(B, Sq, Sc, Hq, Hkv, causal):
     _check(out, lse, ref_a, ref_b, "fp8 block", p_bound, check_b=Sc >= 1000)
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("waves,Sq,H,D", [(4, 70, 2, 128), (4, 70, 2, 96), (4, 70, 2, 64), (8, 130, 260, 128), (8, 130, 260, 96),
+                                          (8, 130, 260, 64)])
+def test_fp8_block_ends_in_either_half_of_a_tile(causal, waves, Sq, H, D):
+    """A 128-key tile is worked on as two halves of 64 keys, one ahead of and one behind the exponentials: chunks that end
+    in, or at the edge of, either half of the first, second and fifth tile (five tiles wrap the four stages of LDS)."""
+    import mercury_artifact_amd as M
+
+    scale = D ** -0.5
+    for Sc in (1, 63, 64, 65, 127, 128, 129, 192, 193, 576, 577, 640):
+        print(f"fp8 half tiles Sq{Sq} Sc{Sc} H{H} D{D} causal={causal}", flush=True)
+        assert N.lib().mhip_attn_fwd_plan(1, Sq, Sc, H, D, D, D, int(causal), N.MHIP_E4M3) == waves
+        (q, k, v), (qq, kq, vq), (sq, sk, sv) = _quantised(1, Sq, Sc, H, 1, seed=Sc, D=D)
+        deq = (O.dequantize(qq, sq), O.dequantize(kq, sk), O.dequantize(vq, sv))
+        ref_a = O.block_attention(*deq, scale, causal=causal)
+        out, lse = M.attn_fwd_block(qq.cuda(), kq.cuda(), vq.cuda(), scale, causal=causal, q_descale=sq.cuda(),
+                                    k_descale=sk.cuda(), v_descale=sv.cuda())
+        torch.cuda.synchronize()
+        p_bound = O.e4m3_p_rounding_bound(*deq, scale, causal=causal)
+        _check(out, lse, ref_a, ref_a, f"fp8 half tiles Sc{Sc}", p_bound, check_b=False)
+
+
 @pytest.mark.parametrize("direction", ["rising", "falling"])
 @pytest.mark.parametrize("binades_per_tile", [0.75, 6.0])
 @pytest.mark.parametrize("causal", [False, True])
