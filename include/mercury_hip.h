@@ -48,8 +48,9 @@ extern "C" {
 /* Bumped whenever an entry point's argument list changes (a caller built against another value must not call).
  * 3: the three descales of mhip_attn_fwd_block are device pointers; mhip_attn_bwd_block takes five stride triples.
  * 4: the backward's workspace also holds partial sums (it is larger than its three row arrays); mhip_attn_bwd_chunk.
- * 5: the workspace's size depends on B, Sq and Hq alone; mhip_attn_fwd_plan, mhip_attn_bwd_plan. */
-#define MHIP_ABI_VERSION 5
+ * 5: the workspace's size depends on B, Sq and Hq alone; mhip_attn_fwd_plan, mhip_attn_bwd_plan.
+ * 6: mhip_attn_fwd_blocks, mhip_attn_fwd_group. */
+#define MHIP_ABI_VERSION 6
 int         mhip_abi_version(void);   /* the MHIP_ABI_VERSION the library was built with */
 int         mhip_version(void);
 /* Optional: per-device set-up the entry points otherwise do on their first call on a device (today: the address
@@ -82,6 +83,26 @@ int mhip_attn_fwd_block(const void* q, const void* k, const void* v, void* out, 
                         float softmax_scale, int mask, int dtype,
                         const float* q_descale, const float* k_descale, const float* v_descale,
                         void* stream);
+
+/*
+ * n blocks of one ring step in one launch: the same q against the n chunks ks[i], vs[i] (host arrays of device pointers,
+ * one set of strides and one Sc for all), block i's results at out + i * o_sn (elements) and at lse + i * B * Hq * Sq.
+ * Each block's results are those of mhip_attn_fwd_block, up to how a launch of this size splits its keys.
+ * 1 <= n <= MHIP_MAX_GROUP.
+ * mhip_attn_fwd_group: how many blocks of a step of `blocks` blocks to put into one launch -- 1 when a block fills the
+ * chip by itself (host function, launches nothing).
+ */
+#define MHIP_MAX_GROUP 16
+int mhip_attn_fwd_blocks(const void* q, const void* const* ks, const void* const* vs, int n, void* out, int64_t o_sn, float* lse,
+                         int B, int Sq, int Sc, int Hq, int Hkv, int D,
+                         int64_t q_sb, int64_t q_ss, int64_t q_sh,
+                         int64_t k_sb, int64_t k_ss, int64_t k_sh,
+                         int64_t v_sb, int64_t v_ss, int64_t v_sh,
+                         int64_t o_sb, int64_t o_ss, int64_t o_sh,
+                         float softmax_scale, int mask, int dtype,
+                         const float* q_descale, const float* k_descale, const float* v_descale,
+                         void* stream);
+int mhip_attn_fwd_group(int B, int Sq, int Hq, int blocks);
 
 /*
  * Block backward from the saved (final, merged) out and lse.

@@ -46,16 +46,27 @@ constexpr int kNoColumn = 0x7fff0000;  // vector offset that is out of every des
 constexpr int kFragDepth = 4;      // LDS operand reads in flight ahead of the MFMAs (6 and 8 measure the same)
 
 struct FwdParams {
-  const uint16_t* q; const uint16_t* k; const uint16_t* v;
-  uint16_t* out; float* lse;
-  int B, Sq, Sc, Hq, Hkv, group;
-  int D;             // head dimension of the tensors, a multiple of 8 up to kD; columns D .. kD-1 are zeros on chip
-  int64_t q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, v_sb, v_ss, v_sh, o_sb, o_ss, o_sh;
-  float scale, scale_log2;
-  int nq_tiles;      // ceil(Sq / rows per workgroup)
-  int total;         // B * Hq * nq_tiles
+  // what a workgroup needs before its first copy: read by one group of loads (see load_now)
   int per_xcd;       // ceil(total / 8)
-  int heads_per_xcd; // (batch, head) pairs per XCD when they divide evenly, else 0
+  int total;         // blocks * B * Hq * nq_tiles
+  int blocks;        // blocks of the launch: the same q against as many chunks
+  int nq_tiles;      // ceil(Sq / rows per workgroup)
+  int heads_per_xcd; // (block, batch, head) triples per XCD when they divide evenly, else 0
+  int Sq, Sc;
+  int D;             // head dimension of the tensors, a multiple of 8 up to kD; columns D .. kD-1 are zeros on chip
+  Divisor by_q_tiles, by_hq, by_group;
+  Divisor by_order;  // causal: by the (block, batch, head) triples, or by those of an XCD
+  const uint16_t* q; const uint16_t* k0; const uint16_t* v0;         // k0, v0: the first block's chunk
+  int64_t q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, v_sb, v_ss, v_sh;
+  float scale, scale_log2;
+  // the rest
+  Divisor by_heads;  // by B * Hq
+  int heads;         // B * Hq
+  int B, Hq;
+  uint16_t* out; float* lse;
+  int64_t o_sb, o_ss, o_sh;
+  int64_t o_sn, l_sn;    // from one block's results to the next one's, elements
+  const uint16_t* k[kMaxGroup]; const uint16_t* v[kMaxGroup];        // the chunk of every block
 };
 
 // KK = k-steps of 16 head-dim values in S^T: 8 computes on all 128 on-chip columns; 4 and 6 are the instantiations for
@@ -91,26 +102,36 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
   // Under the causal mask a Q tile's work grows with its index, so there the order is longest tiles
   // first across all heads (of the XCD when the heads divide evenly over the XCDs, of the launch
   // otherwise): the short tiles fill the tail.
+  load_now<CAUSAL>(p, p.scale_log2);
   int qt, bh;
   if (!CAUSAL) {
     const int logical = (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);
     if (logical >= p.total) return;
-    qt = logical % p.nq_tiles;
-    bh = logical / p.nq_tiles;
+    bh = p.by_q_tiles.quotient(logical, qt);
   } else if (p.heads_per_xcd > 0) {
-    const int local = blockIdx.x >> 3;
-    qt = p.nq_tiles - 1 - local / p.heads_per_xcd;
-    bh = (blockIdx.x & 7) * p.heads_per_xcd + local % p.heads_per_xcd;
+    qt = p.nq_tiles - 1 - p.by_order.quotient(blockIdx.x >> 3, bh);
+    bh += (blockIdx.x & 7) * p.heads_per_xcd;
   } else {
     if ((int)blockIdx.x >= p.total) return;
-    const int nbh = p.B * p.Hq;
-    qt = p.nq_tiles - 1 - (int)blockIdx.x / nbh;
-    bh = (int)blockIdx.x % nbh;
+    qt = p.nq_tiles - 1 - p.by_order.quotient(blockIdx.x, bh);
   }
-  const int hq = bh % p.Hq;
-  const int b = bh / p.Hq;
-  const int hk = hq / p.group;
+  // Several blocks of a step in one launch are so many times the (batch, head) pairs.  (The
+  // first one's addresses come with the arguments above: a lone block does not wait for a second round of loads.)
+  const uint16_t* kp = p.k0; const uint16_t* vp = p.v0;
+  int blk = 0;
+  if (p.blocks > 1) {
+    blk = p.by_heads.quotient(bh, bh);
+    kp = p.k[blk];
+    vp = p.v[blk];
+  }
+  int hq;
+  const int b = p.by_hq.quotient(bh, hq);
+  const int hk = p.by_group.quotient(hq);
   const int q0 = qt * kRows;
+  // Kept in a register: a scalar load that may be under way where the main loop begins turns its waits for one LDS operand
+  // into waits for all of them (2048 x 2048 H24, D 64: 32.5 us instead of 30.9).
+  float scale_log2 = p.scale_log2;
+  asm volatile("" : "+s"(scale_log2));
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // scalar: role branches stay uniform
@@ -144,8 +165,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
   // when it is below 128: their lanes carry an offset that is out of range for every tile, so a tile in
   // LDS always has 128 columns, the upper ones zero, at no cost in memory traffic.
   auto swz = [](int row) { return lds_row_swizzle(row); };
-  const u32x4 krs = rsrc_words(p.k + b * p.k_sb + hk * p.k_sh, (uint32_t)(((int64_t)(p.Sc - 1) * p.k_ss + p.D) * 2));
-  const u32x4 vrs = rsrc_words(p.v + b * p.v_sb + hk * p.v_sh, (uint32_t)(((int64_t)(p.Sc - 1) * p.v_ss + p.D) * 2));
+  const u32x4 krs = rsrc_words(kp + b * p.k_sb + hk * p.k_sh, (uint32_t)(((int64_t)(p.Sc - 1) * p.k_ss + p.D) * 2));
+  const u32x4 vrs = rsrc_words(vp + b * p.v_sb + hk * p.v_sh, (uint32_t)(((int64_t)(p.Sc - 1) * p.v_ss + p.D) * 2));
   constexpr int kCpy = BN / RG / 4;                  // copy instructions per wavefront, tile and tensor (4 rows each)
   int kvoff[kCpy], vvoff[kCpy];
 #pragma unroll
@@ -283,8 +304,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
   float rs = 0.f;
   auto sm_pair = [&](int idx) {
     const int mb = idx >> 3, r = (idx & 7) * 2;
-    float x0 = fast_exp2(__builtin_fmaf(s[mb][r], p.scale_log2, nmsc));
-    float x1 = fast_exp2(__builtin_fmaf(s[mb][r + 1], p.scale_log2, nmsc));
+    float x0 = fast_exp2(__builtin_fmaf(s[mb][r], scale_log2, nmsc));
+    float x1 = fast_exp2(__builtin_fmaf(s[mb][r + 1], scale_log2, nmsc));
     if (idx == 0) rs = x0 + x1; else rs += x0 + x1;
     uint32_t w = pack_bf16(x0, x1);
     asm volatile("" : "+v"(w), "+v"(rs));          // keeps the pair where it is written
@@ -303,7 +324,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
 #pragma unroll
       for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[mb][j]);
     mx = pair_max(mx);
-    const float grown = (mx - m_ref) * p.scale_log2;               // NaN when mx = -inf on the first tile
+    const float grown = (mx - m_ref) * scale_log2;               // NaN when mx = -inf on the first tile
     const bool move = first ? (mx != -INFINITY) : (grown > kSlack);   // false for NaN
     if (!first) {
       const float alpha = move ? fast_exp2(-grown) : 1.f;
@@ -314,7 +335,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
       l_run *= alpha;
     }
     m_ref = move ? mx : m_ref;
-    nmsc = -m_ref * p.scale_log2;
+    nmsc = -m_ref * scale_log2;
   };
   // slot of the matrix phase after which early pair idx runs: k-step idx / 4 of the tile before is read by the
   // O^T slots kSlotsS + DB (idx / 4) .. + DB - 1, and the pairs are spread two slots apart behind that
@@ -471,7 +492,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     if (hf == 0 && my_q < p.Sq) {
       const float lse = l_tot > 0.f ? m_ref * p.scale + fast_log2(l_tot) * kLn2 : -INFINITY;
-      p.lse[((int64_t)b * p.Hq + hq) * p.Sq + my_q] = lse;
+      p.lse[blk * p.l_sn + ((int64_t)b * p.Hq + hq) * p.Sq + my_q] = lse;
     }
 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // zero-filled copies of tiles past the end included
@@ -489,7 +510,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
     __syncthreads();
     {
       const int chunk = lane & 15;
-      uint16_t* op = p.out + b * p.o_sb + hq * p.o_sh + chunk * 8;
+      uint16_t* op = p.out + blk * p.o_sn + b * p.o_sb + hq * p.o_sh + chunk * 8;
 #pragma unroll
       for (int it = 0; it < 8; ++it) {
         const int r = (lane >> 4) + 4 * it;
@@ -564,10 +585,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
     float l_tot = 0.f;
 #pragma unroll
     for (int g = 0; g < KS; ++g)       // (a sum of NaN is no smaller than 0 and goes into the row's)
-      l_tot += st[g][1] > 0.f ? st[g][1] * fast_exp2((st[g][0] - m_all) * p.scale_log2) : st[g][1];
-    const float weight = l_own > 0.f ? fast_exp2((m_ref - m_all) * p.scale_log2) / l_tot : 0.f;
+      l_tot += st[g][1] > 0.f ? st[g][1] * fast_exp2((st[g][0] - m_all) * scale_log2) : st[g][1];
+    const float weight = l_own > 0.f ? fast_exp2((m_ref - m_all) * scale_log2) / l_tot : 0.f;
     if (kg == 0 && hf == 0 && my_q < p.Sq)
-      p.lse[((int64_t)b * p.Hq + hq) * p.Sq + my_q] =
+      p.lse[blk * p.l_sn + ((int64_t)b * p.Hq + hq) * p.Sq + my_q] =
           l_tot > 0.f ? m_all * p.scale + fast_log2(l_tot) * kLn2 : -INFINITY;
     // slot (row group, finishing group, giving group): kShare vectors of 64 lanes x 16 bytes
     auto slot = [&](int to, int from) {
@@ -607,7 +628,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
     {
       constexpr int kRowsPerWave = kRows / kWaves;
       const int chunk = lane & 15;
-      uint16_t* op = p.out + b * p.o_sb + hq * p.o_sh + chunk * 8;
+      uint16_t* op = p.out + blk * p.o_sn + b * p.o_sb + hq * p.o_sh + chunk * 8;
 #pragma unroll
       for (int it = 0; it < kRowsPerWave / 4; ++it) {
         const int r = wave * kRowsPerWave + (lane >> 4) + 4 * it;
@@ -624,9 +645,11 @@ template <bool CAUSAL, int KK, int KS>
 void launch_one(FwdParams& p, hipStream_t stream) {
   const int rows = kBM / KS;
   p.nq_tiles = (p.Sq + rows - 1) / rows;
-  p.total = p.B * p.Hq * p.nq_tiles;
+  p.total = p.blocks * p.heads * p.nq_tiles;
   p.per_xcd = (p.total + 7) / 8;
-  p.heads_per_xcd = (p.B * p.Hq) % 8 == 0 ? (p.B * p.Hq) / 8 : 0;
+  p.heads_per_xcd = (p.blocks * p.heads) % 8 == 0 ? p.blocks * p.heads / 8 : 0;
+  p.by_q_tiles = Divisor(p.nq_tiles);
+  p.by_order = Divisor(p.heads_per_xcd > 0 ? p.heads_per_xcd : p.blocks * p.heads);
   hipLaunchKernelGGL((attn_fwd_bf16_d128<CAUSAL, KK, KS>), dim3(p.per_xcd * 8), dim3(kWaves * 64), 0, stream, p);
 }
 template <int KK>
@@ -664,7 +687,7 @@ int key_groups(const FwdParams& p, bool causal) {
     const int groups = 1 << i;
     const int rows = kBM / groups, tile = groups == 4 ? 32 : kBN;
     const int64_t q_tiles = (p.Sq + rows - 1) / rows;
-    const float n = (float)((int64_t)p.B * p.Hq * q_tiles);
+    const float n = (float)((int64_t)p.blocks * p.B * p.Hq * q_tiles);
     auto steps = [&](int64_t keys) { return (float)((keys + tile * groups - 1) / (tile * groups)); };
     float time;
     if (!causal) {
@@ -691,23 +714,30 @@ int key_groups(const FwdParams& p, bool causal) {
 
 }  // namespace
 
-int attn_fwd_bf16_plan(int B, int Sq, int Sc, int Hq, int D, int64_t k_ss, int64_t v_ss, int mask) {
+int attn_fwd_bf16_plan(int blocks, int B, int Sq, int Sc, int Hq, int D, int64_t k_ss, int64_t v_ss, int mask) {
   FwdParams p{};
+  p.blocks = blocks;
   p.B = B; p.Sq = Sq; p.Sc = Sc; p.Hq = Hq; p.D = D;
   p.k_ss = k_ss; p.v_ss = v_ss;
   return key_groups(p, mask == MHIP_MASK_CAUSAL);
 }
 
-int attn_fwd_bf16(const void* q, const void* k, const void* v, void* out, float* lse,
+int attn_fwd_bf16(const void* q, const void* const* ks, const void* const* vs, int blocks, void* out, int64_t o_sn, float* lse,
                   int B, int Sq, int Sc, int Hq, int Hkv, int D,
                   const int64_t* st, float scale, int mask, hipStream_t stream) {
   FwdParams p;
   p.q = static_cast<const uint16_t*>(q);
-  p.k = static_cast<const uint16_t*>(k);
-  p.v = static_cast<const uint16_t*>(v);
+  for (int i = 0; i < kMaxGroup; ++i) {
+    p.k[i] = i < blocks ? static_cast<const uint16_t*>(ks[i]) : nullptr;
+    p.v[i] = i < blocks ? static_cast<const uint16_t*>(vs[i]) : nullptr;
+  }
+  p.k0 = p.k[0]; p.v0 = p.v[0];
+  p.blocks = blocks; p.heads = B * Hq;
+  p.o_sn = o_sn; p.l_sn = (int64_t)B * Hq * Sq;
   p.out = static_cast<uint16_t*>(out);
   p.lse = lse;
-  p.B = B; p.Sq = Sq; p.Sc = Sc; p.Hq = Hq; p.Hkv = Hkv; p.group = Hq / Hkv;
+  p.B = B; p.Sq = Sq; p.Sc = Sc; p.Hq = Hq;
+  p.by_heads = Divisor(B * Hq); p.by_hq = Divisor(Hq); p.by_group = Divisor(Hq / Hkv);
   p.D = D;
   p.q_sb = st[0]; p.q_ss = st[1]; p.q_sh = st[2];
   p.k_sb = st[3]; p.k_ss = st[4]; p.k_sh = st[5];

@@ -44,14 +44,24 @@ constexpr int kNoColumn = 0x7fff0000;  // vector offset that is out of every des
                                        // when it is used, and so does the scalar tile offset added to it)
 
 struct Fp8Params {
-  const uint8_t* q; const uint8_t* k; const uint8_t* v;
-  uint16_t* out; float* lse;
-  int B, Sq, Sc, Hq, Hkv, group;
+  // what a workgroup needs before its first copy: read by one group of loads (see load_now)
+  int per_xcd, total, blocks, nq_tiles, heads_per_xcd;       // as in the bf16 kernel
+  int Sq, Sc;
   int D;             // head dimension of the tensors, a multiple of 16 up to kD; columns D .. kD-1 are zeros on chip
-  int64_t q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, v_sb, v_ss, v_sh, o_sb, o_ss, o_sh;
-  float scale;           // softmax scale
+  Divisor by_q_tiles, by_hq, by_group;
+  Divisor by_order;  // causal: by the (block, batch, head) triples, or by those of an XCD
+  const uint8_t* q; const uint8_t* k0; const uint8_t* v0;            // k0, v0: the first block's chunk
+  int64_t q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, v_sb, v_ss, v_sh;
   const float* q_descale; const float* k_descale; const float* v_descale;   // device scalars, NULL = 1
-  int nq_tiles, total, per_xcd, heads_per_xcd;
+  float scale;       // softmax scale
+  // the rest
+  Divisor by_heads;  // by B * Hq
+  int heads;         // B * Hq
+  int B, Hq;
+  uint16_t* out; float* lse;
+  int64_t o_sb, o_ss, o_sh;
+  int64_t o_sn, l_sn;    // from one block's results to the next one's, elements
+  const uint8_t* k[kMaxGroup]; const uint8_t* v[kMaxGroup];          // the chunk of every block
 };
 
 // Chunk c (16 bytes) of row r of a tile lives at chunk position c ^ swz8(r).  Row pairs share a 256-byte
@@ -88,25 +98,31 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
   // Workgroup i runs on XCD i % 8: every XCD gets a contiguous range of (batch, head) pairs, so the
   // workgroups that share a K/V head share an L2.  Causal launches run the longest Q tiles first,
   // across all heads.
+  load_now<CAUSAL>(p, p.scale);
   int qt, bh;
   if (!CAUSAL) {
     const int logical = (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);
     if (logical >= p.total) return;
-    qt = logical % p.nq_tiles;
-    bh = logical / p.nq_tiles;
+    bh = p.by_q_tiles.quotient(logical, qt);
   } else if (p.heads_per_xcd > 0) {
-    const int local = blockIdx.x >> 3;
-    qt = p.nq_tiles - 1 - local / p.heads_per_xcd;
-    bh = (blockIdx.x & 7) * p.heads_per_xcd + local % p.heads_per_xcd;
+    qt = p.nq_tiles - 1 - p.by_order.quotient(blockIdx.x >> 3, bh);
+    bh += (blockIdx.x & 7) * p.heads_per_xcd;
   } else {
     if ((int)blockIdx.x >= p.total) return;
-    const int nbh = p.B * p.Hq;
-    qt = p.nq_tiles - 1 - (int)blockIdx.x / nbh;
-    bh = (int)blockIdx.x % nbh;
+    qt = p.nq_tiles - 1 - p.by_order.quotient(blockIdx.x, bh);
   }
-  const int hq = bh % p.Hq;
-  const int b = bh / p.Hq;
-  const int hk = hq / p.group;
+  // Several blocks of a step in one launch are so many times the (batch, head) pairs.  (The
+  // first one's addresses come with the arguments above: a lone block does not wait for a second round of loads.)
+  const uint8_t* kp = p.k0; const uint8_t* vp = p.v0;
+  int blk = 0;
+  if (p.blocks > 1) {
+    blk = p.by_heads.quotient(bh, bh);
+    kp = p.k[blk];
+    vp = p.v[blk];
+  }
+  int hq;
+  const int b = p.by_hq.quotient(bh, hq);
+  const int hk = p.by_group.quotient(hq);
   const int q0 = qt * kBM;
 
   const int tid = threadIdx.x;
@@ -132,8 +148,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
   // fetches the chunk that lives there.  Rows past the end of the chunk arrive as zeros. ---------------------
   // Chunks past the head dimension (D < 128) carry an offset that is out of range for every tile and arrive as
   // zeros too: a tile in LDS always has 128 columns, at no cost in memory traffic.
-  const u32x4 krs = rsrc_words(p.k + b * p.k_sb + hk * p.k_sh, (uint32_t)((int64_t)(p.Sc - 1) * p.k_ss + p.D));
-  const u32x4 vrs = rsrc_words(p.v + b * p.v_sb + hk * p.v_sh, (uint32_t)((int64_t)(p.Sc - 1) * p.v_ss + p.D));
+  const u32x4 krs = rsrc_words(kp + b * p.k_sb + hk * p.k_sh, (uint32_t)((int64_t)(p.Sc - 1) * p.k_ss + p.D));
+  const u32x4 vrs = rsrc_words(vp + b * p.v_sb + hk * p.v_sh, (uint32_t)((int64_t)(p.Sc - 1) * p.v_ss + p.D));
   int kvoff[kCpy], vvoff[kCpy];
 #pragma unroll
   for (int u = 0; u < kCpy; ++u) {
@@ -399,7 +415,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
   const float inv = l_tot > 0.f ? out_mul / l_tot : 0.f;           // the two factors 2^4 cancel
   if (hf == 0 && my_q < p.Sq) {
     const float lse = l_tot > 0.f ? m_ref * scale_eff + (fast_log2(l_tot) - kPShift) * kLn2 : -INFINITY;
-    p.lse[((int64_t)b * p.Hq + hq) * p.Sq + my_q] = lse;
+    p.lse[blk * p.l_sn + ((int64_t)b * p.Hq + hq) * p.Sq + my_q] = lse;
   }
   __syncthreads();
   unsigned char* os = smem + wave * (32 * kOStride * 2);
@@ -415,7 +431,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
   __syncthreads();
   {
     const int chunk = lane & 15;
-    uint16_t* op = p.out + b * p.o_sb + hq * p.o_sh + chunk * 8;
+    uint16_t* op = p.out + blk * p.o_sn + b * p.o_sb + hq * p.o_sh + chunk * 8;
 #pragma unroll
     for (int it = 0; it < 8; ++it) {
       const int r = (lane >> 4) + 4 * it;
@@ -442,17 +458,25 @@ void launch_fp8(const Fp8Params& p, bool causal, hipStream_t stream) {
 // 34.2 / 46.5; 2048 x 2048 H32 39.7 / 46.3).  Under the causal mask of a square or tall block the longest workgroups hold
 // up the launch until there is twice as much work (2048 x 2048 H20 35.2 / 24.4, H32, 512 workgroups, 36.6 / 30.3, H40
 // 38.0 / 42.0; 4096 x 2048 H16 34.6 / 24.6).
-int attn_fwd_fp8_plan(int B, int Sq, int Sc, int Hq, int mask) {
-  return (int64_t)B * Hq * ((Sq + 127) / 128) > (mask == MHIP_MASK_CAUSAL && Sc <= Sq ? 512 : 256) ? 8 : 4;
+int attn_fwd_fp8_plan(int blocks, int B, int Sq, int Sc, int Hq, int mask) {
+  return (int64_t)blocks * B * Hq * ((Sq + 127) / 128) > (mask == MHIP_MASK_CAUSAL && Sc <= Sq ? 512 : 256) ? 8 : 4;
 }
 
-int attn_fwd_fp8(const void* q, const void* k, const void* v, void* out, float* lse,
+int attn_fwd_fp8(const void* q, const void* const* ks, const void* const* vs, int blocks, void* out, int64_t o_sn, float* lse,
                  int B, int Sq, int Sc, int Hq, int Hkv, int D, const int64_t* st, float scale, int mask,
                  const float* q_descale, const float* k_descale, const float* v_descale, hipStream_t stream) {
   Fp8Params p;
-  p.q = static_cast<const uint8_t*>(q); p.k = static_cast<const uint8_t*>(k); p.v = static_cast<const uint8_t*>(v);
+  p.q = static_cast<const uint8_t*>(q);
+  for (int i = 0; i < kMaxGroup; ++i) {
+    p.k[i] = i < blocks ? static_cast<const uint8_t*>(ks[i]) : nullptr;
+    p.v[i] = i < blocks ? static_cast<const uint8_t*>(vs[i]) : nullptr;
+  }
+  p.k0 = p.k[0]; p.v0 = p.v[0];
+  p.blocks = blocks; p.heads = B * Hq;
+  p.o_sn = o_sn; p.l_sn = (int64_t)B * Hq * Sq;
   p.out = static_cast<uint16_t*>(out); p.lse = lse;
-  p.B = B; p.Sq = Sq; p.Sc = Sc; p.Hq = Hq; p.Hkv = Hkv; p.group = Hq / Hkv;
+  p.B = B; p.Sq = Sq; p.Sc = Sc; p.Hq = Hq;
+  p.by_heads = Divisor(B * Hq); p.by_hq = Divisor(Hq); p.by_group = Divisor(Hq / Hkv);
   p.D = D;
   p.q_sb = st[0]; p.q_ss = st[1]; p.q_sh = st[2];
   p.k_sb = st[3]; p.k_ss = st[4]; p.k_sh = st[5];
@@ -461,12 +485,14 @@ int attn_fwd_fp8(const void* q, const void* k, const void* v, void* out, float* 
   p.scale = scale;
   p.q_descale = q_descale; p.k_descale = k_descale; p.v_descale = v_descale;
   const bool causal = mask == MHIP_MASK_CAUSAL;
-  const bool wide = attn_fwd_fp8_plan(B, Sq, Sc, Hq, mask) == 8;
+  const bool wide = attn_fwd_fp8_plan(blocks, B, Sq, Sc, Hq, mask) == 8;
   const int rows = wide ? 256 : 128;
   p.nq_tiles = (Sq + rows - 1) / rows;
-  p.total = B * Hq * p.nq_tiles;
+  p.total = blocks * p.heads * p.nq_tiles;
   p.per_xcd = (p.total + 7) / 8;
-  p.heads_per_xcd = (B * Hq) % 8 == 0 ? (B * Hq) / 8 : 0;
+  p.heads_per_xcd = (blocks * p.heads) % 8 == 0 ? blocks * p.heads / 8 : 0;
+  p.by_q_tiles = Divisor(p.nq_tiles);
+  p.by_order = Divisor(p.heads_per_xcd > 0 ? p.heads_per_xcd : blocks * p.heads);
   if (D <= 64) wide ? launch_fp8<2, 8>(p, causal, stream) : launch_fp8<2, 4>(p, causal, stream);
   else if (D <= 96) wide ? launch_fp8<3, 8>(p, causal, stream) : launch_fp8<3, 4>(p, causal, stream);
   else wide ? launch_fp8<4, 8>(p, causal, stream) : launch_fp8<4, 4>(p, causal, stream);

@@ -7,7 +7,8 @@ neighbour exchange.  The body is the loop the code generator emits for that temp
 (mercury/backend/pytorch/codegen.py:264-355, 443-523): take the current KV chunk, start the hop for
 the next one, run the block kernel, fold with ``update_out_and_lse``, and store after the last step.  A
 forward driver's blocks go through ``_flash_attn_forward`` unless it would do nothing but call the kernel;
-then they are written straight into places allocated once per step.
+then they are written straight into places allocated once per step, and where one block would leave most of the chip
+idle, the driver waits for further chunks and launches their blocks together.
 
 Two defaults of the forward drivers depart from the literal sequence without changing what is computed:
 ``deferred_merge=True`` keeps the bf16 block results of all chunks and folds them with ONE
@@ -87,17 +88,50 @@ def _block_forward(q, k, v, softmax_scale, dropout_p, causal, window_size, alibi
     return outputs[:2]
 
 
+class _Places(list):
+    """(out, lse) per block, or None per block; ``stacked`` are the two tensors the places are slices of."""
+    stacked = None
+
+
 def _block_results(n, q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **descales):
     """Places for the results of a step's ``n`` blocks over all rows of ``q``, from one allocation each for the outputs and
     the LSEs; None for every block where the operator has something to report or to record."""
     if (not _ops.as_declared((softmax_scale, dropout_p), window_size, (causal,))
             or dropout_p or alibi_slopes is not None or window_size[0] != -1 or window_size[1] != -1
             or q.dim() != 4 or not N.host.undispatched(q, kv, *descales.values())):
-        return [None] * n
+        return _Places([None] * n)
     B, Sq, Hq, D = q.shape
     outs = torch.empty((n, B, Sq, Hq, D), dtype=torch.bfloat16, device=q.device)
     lses = torch.empty((n, B, Hq, Sq), dtype=torch.float32, device=q.device)
-    return list(zip(outs.unbind(0), lses.unbind(0)))
+    places = _Places(zip(outs.unbind(0), lses.unbind(0)))
+    places.stacked = outs, lses
+    return places
+
+
+class _Groups:
+    """Block forwards of one query tensor over a step's chunks, several to a launch where one block leaves most of the chip
+    idle and the ring lets its chunks lie (mhip_attn_fwd_group has the rule); ``size`` is 1 where every block goes its own
+    way."""
+
+    def __init__(self, q, places, ring, softmax_scale, causal, q_descale=None, k_descale=None, v_descale=None):
+        self.size = 1
+        if places.stacked is not None and type(ring).__dict__.get("keeps_chunks"):
+            self.size = N.host.fwd_group(q, len(places)) or 1
+        if self.size > 1:
+            self.q, self.places, self.done, self.chunks = q, places, 0, []
+            self.args = (softmax_scale, causal, q_descale, k_descale, v_descale)
+
+    def add(self, chunk) -> int:
+        """Takes the next chunk, launches if that makes a group or completes the step, and returns how many blocks are done
+        or waiting."""
+        self.chunks.append(chunk)
+        seen = self.done + len(self.chunks)
+        if len(self.chunks) == self.size or seen == len(self.places):
+            if N.host.fwd_blocks(self.q, self.chunks, *self.args, *self.places.stacked, self.done) is None:
+                for chunk, place in zip(self.chunks, self.places[self.done:]):
+                    _ops.attn_fwd_block(self.q, chunk[0], chunk[1], *self.args, *place)
+            self.done, self.chunks = seen, []
+        return seen
 
 
 def _as_rows(t):
@@ -151,9 +185,11 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
                       f"{MAX_MERGE_MANY} blocks and writes contiguous bfloat16, so this step merges block by block "
                       "(same result, one pass over the fp32 accumulator per block)", RuntimeWarning, stacklevel=3)
     done = 0
-    places = [None] * n_blocks
+    places = _Places([None] * n_blocks)
     if defer:
         places = _block_results(n_blocks, q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra)
+    # (a divided ring is one that wants to hold little of other ranks' keys at a time)
+    groups = _Groups(q, _Places() if two_streams or ring_divide > 1 else places, ring, softmax_scale, causal, **extra)
     main = side = None
     kv_ready = next_ready = None
     if two_streams and defer:
@@ -185,6 +221,12 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
                 if side is not None:                   # what the hop enqueued on the current stream ends here
                     next_ready = torch.cuda.Event()
                     next_ready.record(main)
+            if groups.size > 1:
+                done = groups.add(_kv)
+                if done == n_blocks:
+                    merge_many([p[0] for p in places], [p[1] for p in places], o, lse)
+                    return
+                continue
             _k, _v = _kv.unbind(0)
             if side is not None and done % 2 == 1:
                 if kv_ready is not None:
@@ -273,9 +315,10 @@ def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=F
     blocks = []
     defer = (fused_epilogue and deferred_merge and len(hops) <= MAX_MERGE_MANY and o.dtype == torch.bfloat16
              and o.is_contiguous() and lse.is_contiguous())
-    places = [None] * len(hops)
+    places = _Places([None] * len(hops))
     if defer:
         places = _block_results(len(hops), q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes)
+    groups = _Groups(q, places, ring, softmax_scale, causal)
     for step, hop in enumerate(hops):
         if step == 0:
             _kv = kv.contiguous()
@@ -286,6 +329,9 @@ def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=F
             send_to, recv_from = _neighbours(ring, hop)
             _next_kv = ring.send_recv(send_to, recv_from, _kv)
             ring.commit()
+        if groups.size > 1:
+            groups.add(_kv)
+            continue
         _k, _v = _kv.unbind(0)
         block_out, block_lse = _block_forward(q, _k, _v, softmax_scale, dropout_p, causal, window_size, alibi_slopes,
                                               into=places[step])
@@ -294,6 +340,7 @@ def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=F
         else:
             buf = pack_block(block_out, block_lse, reduce_into=buf)
     if defer:
+        blocks = places if groups.size > 1 else blocks
         merge_many([b[0] for b in blocks], [b[1] for b in blocks], o, lse)
         return
     _store_packed(buf, o, lse, fused_epilogue)
@@ -356,7 +403,15 @@ def zigzag_causal_pack_kv(q, kv, o, lse, softmax_scale, dropout_p=0, causal=True
     defer = (deferred_merge and world <= MAX_MERGE_MANY and o.dtype == torch.bfloat16
              and o.is_contiguous() and lse.is_contiguous())
     blocks = []
-    for step in range(world):
+    kinds = [zigzag_step(ring.rank, step, world)[0] for step in range(world)]
+    place_of, groups = {}, {}
+    for kind, rows in (("diag", q), ("kv_first_half", q), ("q_second_half", q[:, half:])):
+        n = kinds.count(kind)
+        places = _Places([None] * n)
+        if defer and n:
+            places = _block_results(n, rows, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes)
+        place_of[kind], groups[kind] = iter(places), _Groups(rows, places, ring, softmax_scale, kind == "diag")
+    for step, kind in enumerate(kinds):
         if step == 0:
             _kv = kv.contiguous()
         else:
@@ -366,14 +421,18 @@ def zigzag_causal_pack_kv(q, kv, o, lse, softmax_scale, dropout_p=0, causal=True
             send_to, recv_from = _neighbours(ring, 0)
             _next_kv = ring.send_recv(send_to, recv_from, _kv)
             ring.commit()
-        kind, _ = zigzag_step(ring.rank, step, world)
-        if kind == "diag":
-            bq, bk, bv, bc, sl = q, _kv[0], _kv[1], True, None
-        elif kind == "kv_first_half":
-            bq, bk, bv, bc, sl = q, _kv[0][:, :half], _kv[1][:, :half], False, None
+        bq, bkv, sl = q, _kv, None
+        if kind == "kv_first_half":
+            bkv = _kv[:, :, :half]
+        elif kind == "q_second_half":
+            bq, sl = q[:, half:], (slice(None), slice(half, None))
+        place = next(place_of[kind])
+        if groups[kind].size > 1:
+            groups[kind].add(bkv)
+            block_out, block_lse = place
         else:
-            bq, bk, bv, bc, sl = q[:, half:], _kv[0], _kv[1], False, (slice(None), slice(half, None))
-        block_out, block_lse = _block_forward(bq, bk, bv, softmax_scale, dropout_p, bc, window_size, alibi_slopes)
+            block_out, block_lse = _block_forward(bq, bkv[0], bkv[1], softmax_scale, dropout_p, kind == "diag", window_size,
+                                                  alibi_slopes, into=place)
         if defer:
             blocks.append((block_out, block_lse, 0 if sl is None else half))
             continue

@@ -273,6 +273,11 @@ class LocalRing:
     have received.
     """
 
+    # What a wait has delivered stays as it is for the rest of the step.  A ring class says so for itself (a class
+    # derived from this one may receive into buffers it uses again); drivers may then wait for several chunks first and
+    # launch their blocks together.
+    keeps_chunks = True
+
     def __init__(self, mesh_shape: Sequence[int], rank: int,
                  chunks: Optional[Sequence[torch.Tensor]] = None, copy: bool = False):
         self.mesh_shape = tuple(int(x) for x in mesh_shape)

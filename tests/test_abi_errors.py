@@ -132,3 +132,14 @@ def test_elementwise_rejects(lib):
     assert lib.mhip_quantize_e4m3(P, 2, 64, P, None, P, None) == EINVAL
     assert lib.mhip_quantize_e4m3(None, 2, 64, P, P, P, None) == EINVAL
     assert lib.mhip_quantize_e4m3(P + 4, 2, 64, P, P, P, None) == EALIGN
+
+
+def test_forward_blocks_reject(lib):
+    def blocks(ks=(P, P), vs=(P, P), n=2, o_sn=8192, out=P):
+        array = ctypes.c_void_p * 17
+        return lib.mhip_attn_fwd_blocks(P, array(*ks) if ks else None, array(*vs) if vs else None, n, out, o_sn, P, 1, 64, 64, 1, 1, 128,
+                                        *[8192, 128, 128] * 4, 0.1, 0, 0, None, None, None, None)
+
+    assert blocks(n=0) == blocks(n=17, ks=[P] * 17, vs=[P] * 17) == blocks(n=-1) == EINVAL
+    assert blocks(ks=None) == blocks(vs=None) == blocks(ks=(P, 0)) == blocks(vs=(P, 0)) == blocks(out=None) == EINVAL
+    assert blocks(ks=(P, P + 8)) == blocks(vs=(P, P + 8)) == blocks(o_sn=8196) == EALIGN

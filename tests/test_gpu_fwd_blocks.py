@@ -1,0 +1,105 @@
+"""Several block forwards of a step in one launch (mhip_attn_fwd_blocks) against the oracle, and which rings get them."""
+import pytest
+import torch
+
+import oracle as O
+from mercury_artifact_amd import _native as N
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(n, B, Sq, Sc, Hq, Hkv, D, fp8):
+    g = torch.Generator().manual_seed(n * 1000 + Sq + Sc)
+    q = torch.randn(B, Sq, Hq, D, generator=g)
+    chunks = [torch.randn(2, B, Sc, Hkv, D, generator=g) for _ in range(n)]
+    if fp8:
+        (qq, sq), made = O.quantize_e4m3(q), [O.quantize_e4m3(c) for c in chunks]
+        scale = max(s for _, s in made)
+        chunks = [(c / scale).clamp(-448, 448).to(torch.float8_e4m3fn) for c in chunks]
+        return qq, chunks, sq, scale
+    return q.bfloat16(), [c.bfloat16() for c in chunks], None, None
+
+
+@pytest.mark.parametrize("n,B,Sq,Sc,Hq,Hkv,D,causal,fp8", [
+    (1, 1, 64, 64, 1, 1, 128, False, False), (16, 1, 33, 70, 2, 1, 128, False, False), (4, 1, 256, 256, 4, 4, 64, False, False),
+    (5, 2, 257, 130, 3, 3, 96, False, False), (3, 1, 100, 0, 2, 2, 64, False, False), (7, 2, 300, 200, 4, 2, 80, True, False),
+    (4, 1, 512, 512, 8, 8, 128, True, False), (2, 1, 1024, 384, 32, 8, 128, False, False), (3, 1, 200, 300, 5, 5, 64, True, False),
+    (4, 1, 256, 256, 4, 4, 128, False, True), (9, 1, 129, 200, 2, 1, 64, False, True), (4, 1, 512, 300, 8, 8, 96, True, True)])
+def test_blocks_of_a_launch_match_the_oracle(n, B, Sq, Sc, Hq, Hkv, D, causal, fp8):
+    """Every block of a launch, with ragged tiles, grouped heads and (batch, head) counts that do and do not divide over
+    the XCDs, into places behind a first one that stays as it was.  bf16: one rounding of the result and of P, 2^-8 each
+    of |out| <= max |v| < 5.5; e4m3: the bound of rounding P to e4m3 besides."""
+    q, chunks, sq, sc = _inputs(n, B, Sq, Sc, Hq, Hkv, D, fp8)
+    scale = D ** -0.5
+    print(f"n{n} B{B} Sq{Sq} Sc{Sc} H{Hq}/{Hkv} D{D} causal={causal} fp8={fp8}", flush=True)
+    outs = torch.full((n + 1, B, Sq, Hq, D), 7.0, dtype=torch.bfloat16, device="cuda")
+    lses = torch.full((n + 1, B, Hq, Sq), 7.0, device="cuda")
+    ds = [None] * 3 if not fp8 else [t.cuda().reshape(()) for t in (sq, sc, sc)]
+    assert N.host.fwd_blocks(q.cuda(), [c.cuda() for c in chunks], scale, causal, *ds, outs, lses, 1) is True
+    torch.cuda.synchronize()
+    assert (outs[0] == 7).all() and (lses[0] == 7).all()
+    for i, c in enumerate(chunks):
+        if fp8:
+            ops = (O.dequantize(q, sq), O.dequantize(c[0], sc), O.dequantize(c[1], sc))
+            bound = O.e4m3_p_rounding_bound(*ops, scale, causal=causal)
+        else:
+            ops, bound = (q.float(), c[0].float(), c[1].float()), 0.0
+        ro, rl = O.block_attention(*ops, scale, causal=causal)
+        got, lse = outs[i + 1].float().cpu(), lses[i + 1].cpu()
+        assert ((got - ro).abs() - (bound + 2 ** -8 * ro.abs())).max().item() <= 2e-2, i
+        assert torch.equal(torch.isinf(lse), torch.isinf(rl)), i
+        seen = ~torch.isinf(rl)
+        assert not seen.any() or ((lse[seen] - rl[seen]).abs() / rl[seen].abs().clamp_min(1.0)).max().item() <= 1e-3, i
+
+
+def test_blocks_refuse_what_a_launch_cannot_take():
+    """Chunks of another shape or layout, too many of them, places too few: left to the caller, nothing written."""
+    q, chunks, _, _ = _inputs(3, 1, 64, 64, 2, 2, 64, False)
+    q, chunks = q.cuda(), [c.cuda() for c in chunks]
+    outs, lses = torch.full((3, 1, 64, 2, 64), 7.0, dtype=torch.bfloat16, device="cuda"), torch.full((3, 1, 2, 64), 7.0, device="cuda")
+
+    def call(cs, first=0, q=q):
+        return N.host.fwd_blocks(q, cs, 0.1, False, None, None, None, outs, lses, first)
+
+    strided = torch.empty(2, 1, 64, 2, 128, dtype=torch.bfloat16, device="cuda")[..., :64]
+    assert call([]) is call(chunks, 1) is call(chunks, -1) is call(chunks * 6) is None
+    assert call([chunks[0], chunks[1][:, :, :32]]) is call([chunks[0], strided]) is call([chunks[0], chunks[1].float()]) is None
+    assert call([chunks[0], chunks[1].cpu()]) is call(chunks, q=q.float()) is None
+    torch.cuda.synchronize()
+    assert (outs == 7).all() and (lses == 7).all()
+    assert call([strided] * 3) is True                                  # one layout for all, rows 256 bytes apart
+
+
+@pytest.mark.parametrize("path", ["ring", "packed", "zigzag"])
+@pytest.mark.parametrize("own_class", [False, True])
+def test_only_rings_that_keep_their_chunks_get_grouped_launches(path, own_class):
+    """A class derived from LocalRing may receive into a buffer it uses again, as this one does: its blocks are launched one
+    by one, before the next hop overwrites their chunk.  Same results either way."""
+    import mercury_artifact_amd as M
+    from mercury_artifact_amd import flash_attn_interface as FI
+
+    class OneBuffer(M.LocalRing):
+        def send_recv(self, to, source, x, recv_tensor=None):
+            got = super().send_recv(to, source, x)
+            self.spare = getattr(self, "spare", None)
+            if self.spare is None:
+                self.spare = [torch.empty_like(got), torch.empty_like(got)]
+            self.spare.reverse()
+            return self.spare[0].copy_(got)
+
+    q, chunks, _, _ = _inputs(4, 1, 130, 130, 2, 2, 64, False)
+    q, chunks = q.cuda(), [c.cuda() for c in chunks]
+    o, lse = torch.empty_like(q), torch.empty(1, 2, 130, device="cuda")
+    step = {"ring": M.flash_attn_pack_kv, "packed": M.flash_attn_expose_reduce, "zigzag": M.zigzag_causal_pack_kv}[path]
+    blocks, real = [], FI.attn_fwd_block
+    FI.attn_fwd_block = lambda *a: blocks.append(1) or real(*a)
+    try:
+        step(q, chunks[2], o, lse, 0.125, ring=(OneBuffer if own_class else M.LocalRing)((4,), 2, chunks))
+    finally:
+        FI.attn_fwd_block = real
+    torch.cuda.synchronize()
+    # (zigzag at rank 2: the diagonal and, alone of its kind, the one chunk of a later rank have launches of their own)
+    assert len(blocks) == (4 if own_class else {"ring": 0, "packed": 0, "zigzag": 2}[path])
+    want, wl = torch.empty_like(o), torch.empty_like(lse)
+    step(q, chunks[2], want, wl, 0.125, ring=M.LocalRing((4,), 2, chunks), deferred_merge=False)
+    assert (o.float() - want.float()).abs().max().item() <= 2e-2 and (lse - wl).abs().max().item() <= 1e-3

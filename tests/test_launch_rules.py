@@ -49,3 +49,13 @@ def test_carried_sums_are_tested_in_both_forms(columns):
     steps = [c for c in IN_TURN if _columns(c[4]) == columns]
     assert any(c[0] >= 3 for c in steps) and all(bwd_plan(2, c[1], c[1], *c[2:], False)[0] == 2 for c in steps)
     assert any(_columns(c[4]) == columns and bwd_plan(2, c[1], c[1], *c[2:], False)[0] == 1 for c in JOINT)
+
+
+def test_blocks_of_a_step_share_a_launch_until_it_fills_the_chip():
+    group = N.lib().mhip_attn_fwd_group
+    assert group(1, 4096, 32, 8) == group(1, 1025, 32, 8) == 1                # half of the CUs or more by itself
+    assert group(1, 1024, 32, 8) == 2 and group(1, 512, 32, 7) == 4           # 4 + 3
+    assert group(4, 512, 5, 8) == 4                                           # six would fit; two launches of four
+    assert group(1, 256, 4, 4) == 4 and group(1, 16, 1, 64) == 16             # never more than an argument list holds
+    assert group(1, 256, 4, 1) == 1 and group(1, 0, 4, 8) == group(0, 64, 4, 8) == 1
+    assert group(1, 64, 0, 8) < 0 and group(1, 64, 4, 0) < 0 and group(-1, 64, 4, 1) < 0
