@@ -49,8 +49,9 @@ extern "C" {
  * 3: the three descales of mhip_attn_fwd_block are device pointers; mhip_attn_bwd_block takes five stride triples.
  * 4: the backward's workspace also holds partial sums (it is larger than its three row arrays); mhip_attn_bwd_chunk.
  * 5: the workspace's size depends on B, Sq and Hq alone; mhip_attn_fwd_plan, mhip_attn_bwd_plan.
- * 6: mhip_attn_fwd_blocks, mhip_attn_fwd_group. */
-#define MHIP_ABI_VERSION 6
+ * 6: mhip_attn_fwd_blocks, mhip_attn_fwd_group.
+ * 7: mhip_attn_bwd_chunks, mhip_attn_bwd_group. */
+#define MHIP_ABI_VERSION 7
 int         mhip_abi_version(void);   /* the MHIP_ABI_VERSION the library was built with */
 int         mhip_version(void);
 /* Optional: per-device set-up the entry points otherwise do on their first call on a device (today: the address
@@ -89,8 +90,8 @@ int mhip_attn_fwd_block(const void* q, const void* k, const void* v, void* out, 
  * one set of strides and one Sc for all), block i's results at out + i * o_sn (elements) and at lse + i * B * Hq * Sq.
  * Each block's results are those of mhip_attn_fwd_block, up to how a launch of this size splits its keys.
  * 1 <= n <= MHIP_MAX_GROUP.
- * mhip_attn_fwd_group: how many blocks of a step of `blocks` blocks to put into one launch -- 1 when a block fills the
- * chip by itself (host function, launches nothing).
+ * mhip_attn_fwd_group: how many blocks of a step of `blocks` blocks to put into one launch when all of its chunks are there
+ * (host function, launches nothing).
  */
 #define MHIP_MAX_GROUP 16
 int mhip_attn_fwd_blocks(const void* q, const void* const* ks, const void* const* vs, int n, void* out, int64_t o_sn, float* lse,
@@ -180,6 +181,26 @@ int mhip_attn_bwd_chunk(const void* dout, const void* q, const void* k, const vo
                         int64_t dq_sb, int64_t dq_ss, int64_t dq_sh,  /* dq       */
                         int64_t o_sb, int64_t o_ss, int64_t o_sh,     /* out      */
                         float softmax_scale, int mask, void* workspace, void* stream);
+
+/*
+ * n chunks of a ring step in one launch, 1 <= n <= MHIP_MAX_GROUP: what n calls of mhip_attn_bwd_chunk without a mask do, with
+ * T the sum over all of them.  ks, vs, dks, dvs, dk32s and dv32s are host arrays of n device pointers (entries of the
+ * last four may be NULL, as there); all chunks have one Sc and one set of strides.
+ * mhip_attn_bwd_group: how many chunks of a step of `chunks` chunks to put into one launch when all of them are there (host
+ * function, launches nothing).
+ */
+int mhip_attn_bwd_chunks(const void* dout, const void* q, const void* const* ks, const void* const* vs, int n,
+                         const void* out, const float* lse,
+                         void* dq, float* dq_acc, int first, int last, int prepared,
+                         void* const* dks, void* const* dvs, float* const* dk32s, float* const* dv32s,
+                         int B, int Sq, int Sc, int Hq, int Hkv, int D,
+                         int64_t q_sb, int64_t q_ss, int64_t q_sh,     /* q, dout  */
+                         int64_t k_sb, int64_t k_ss, int64_t k_sh,     /* k, v     */
+                         int64_t dk_sb, int64_t dk_ss, int64_t dk_sh,  /* dk, dv   */
+                         int64_t dq_sb, int64_t dq_ss, int64_t dq_sh,  /* dq       */
+                         int64_t o_sb, int64_t o_ss, int64_t o_sh,     /* out      */
+                         float softmax_scale, void* workspace, void* stream);
+int mhip_attn_bwd_group(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks);
 
 /*
  * Which form of the kernels a call of the given sizes takes (host functions, nothing is launched; for tests and profiles,

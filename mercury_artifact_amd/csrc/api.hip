@@ -98,16 +98,18 @@ extern "C" int mhip_attn_fwd_block(const void* q, const void* k, const void* v, 
                               o_sb, o_ss, o_sh, softmax_scale, mask, dtype, q_descale, k_descale, v_descale, stream);
 }
 
-// As many blocks as find room on the 256 CUs side by side, in workgroups of 256 query rows, over launches of even size.  A
-// block that leaves half of the chip or more idle pays for the launch, for a workgroup's prologue and epilogue and,
-// where its keys are split so that more CUs get a part, for bringing the parts together; waiting for further chunks of
-// a step costs no more than one launch of this size.  Whole ring steps, us, block by block / in groups: 4 blocks 256 x 256
-// H4 D64 35.3 / 20.9, 8 blocks 512 x 512 B4 H5 86.3 / 42.3, 8 blocks 1024 x 1024 H32 195 / 158.
+// Blocks per launch, over launches of even size: as many as make up to kGroupWorkgroups workgroups of 256 query rows, eight rounds
+// of one per CU.  A block that leaves CUs idle shares them with the next ones, without splitting its keys over more
+// workgroups, and the last, partly empty round of a launch comes once instead of once per block; from eight rounds on
+// there is little left of that (8 blocks 4096 x 4096 H32, 512 workgroups each: 1742 us one by one, 1713 / 1700 / 1692
+// in groups of 2 / 4 / 8).  Whole ring steps, one by one / grouped, us: 4 blocks 256 x 256 H4 D64 35.3 / 20.9, 8 blocks 512 x 512
+// B4 H5 86.3 / 41.3, 1024 x 1024 H32 168 / 137, 1237 x 1237 B2 H16/8 D80 202 / 171, 2048 x 2048 H32 501 / 470; e4m3 1024 x 1024
+// H32 150 / 100.
 extern "C" int mhip_attn_fwd_group(int B, int Sq, int Hq, int blocks) {
   if (B < 0 || Sq < 0 || Hq <= 0 || blocks < 1) return MHIP_EINVAL;
   const int64_t wgs = (int64_t)B * Hq * (((int64_t)Sq + 255) / 256);
-  if (wgs == 0 || 2 * wgs > 256) return 1;
-  int most = (int)(256 / wgs);
+  if (wgs == 0 || 2 * wgs > kGroupWorkgroups) return 1;
+  int most = (int)(kGroupWorkgroups / wgs);
   if (most > kMaxGroup) most = kMaxGroup;
   const int launches = (blocks + most - 1) / most;
   return (blocks + launches - 1) / launches;

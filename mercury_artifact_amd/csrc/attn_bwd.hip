@@ -60,6 +60,7 @@ struct BwdParams {
   int dq_mode;                             // what dq_acc is for: kDq*
   bool prepared;                           // delta and lse2 are in the workspace already
   int B, Sq, Sc, Hq, Hkv, group;
+  Divisor by_hq, by_hkv, by_group;
   int D;            // head dimension of the tensors, a multiple of 8 up to kD; columns D .. kD-1 are zeros on chip
   int64_t q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, dk_sb, dk_ss, dk_sh, dq_sb, dq_ss, dq_sh, o_sb, o_ss, o_sh;
   float scale, scale_log2;
@@ -67,12 +68,24 @@ struct BwdParams {
 
 // The workgroups of a pass: one per stationary tile of a (batch, head).
 struct TileMap {
-  int splits;          // workgroups that share a stationary tile, each with its part of the streamed tiles
+  int splits;          // workgroups that share a stationary tile, each with its part of the streamed tiles: a power of two
+  int log_splits;
   float* partial;      // with splits > 1: their sums, [split] x the layout of dQ, or of dK and behind all of it dV, fp32
   int n_tiles;         // stationary tiles per (batch, head), times splits
   int total;
   int per_xcd;         // ceil(total / 8); the pass takes 8 * per_xcd workgroups
   int heads_per_xcd;   // (batch, stationary head) pairs per XCD when they divide evenly, else 0
+  Divisor by_tiles;
+  Divisor by_order;    // causal: by all (batch, stationary head) pairs, or by those of an XCD
+};
+
+// Several chunks of a step in one launch: the places of BwdParams that differ from chunk to chunk.
+struct Chunks {
+  int n;
+  Divisor by_heads;    // by B * Hkv
+  const uint16_t* k[kMaxGroup]; const uint16_t* v[kMaxGroup];
+  uint16_t* dk[kMaxGroup]; uint16_t* dv[kMaxGroup];
+  float* dk32[kMaxGroup]; float* dv32[kMaxGroup];
 };
 
 // KK = k-steps of 16 head-dim values in T1 / T2: 8 computes on all 128 on-chip columns; 4 and 6 are the instantiations for
@@ -89,9 +102,15 @@ template <bool DQ, int WAVES>
 constexpr int kSmemBytesOf = WAVES == 8 ? 3 * kStageBytesOf<DQ, WAVES> + WAVES * 32 * kD * 2 : kStages * kStageBytesOf<DQ, WAVES>;
 
 // SPLIT: the workgroups of the pass may share their stationary tile (w.splits).
-template <bool DQ, bool CAUSAL, int KK, int WAVES, bool PREPARED, bool SPLIT>
-__device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, const int block, unsigned char* smem) {
+//
+// CHUNKS: several chunks of a step at once.  The dK / dV pass has a workgroup per key tile of every chunk; a workgroup of
+// the dQ pass visits the chunks one after the other, as the dK / dV pass visits the query heads of a group, so dQ meets the
+// sum carried from launch to launch once per launch instead of once per chunk.
+template <bool DQ, bool CAUSAL, int KK, int WAVES, bool PREPARED, bool SPLIT, bool CHUNKS = false>
+__device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, const int block, unsigned char* smem,
+                                         const Chunks* chunks = nullptr) {
   static_assert(DQ || WAVES == 4, "the dK / dV pass has no room for two wavefronts per SIMD");
+  static_assert(!CHUNKS || (!SPLIT && !CAUSAL), "launches of several chunks are not split further");
   static_assert(PREPARED || WAVES == 8, "the pass that prepares is the one with a launch of its own");
   constexpr int DB = KK / 2;                    // blocks of 32 head-dim values in the accumulators
   constexpr int kWavesWg = WAVES;
@@ -105,6 +124,15 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   constexpr int kXRows = 3 * kStageBytes, kYRows = WAVES == 8 ? kStageBytes : 2 * kStageBytes;
   static_assert(kYRows + kRowsBytes <= kXRows && kXRows + kRowsBytes <= kSmemBytesOf<DQ, WAVES>, "the rows' places");
 
+  // One round of argument loads instead of one before each first use (load_now in the common header says why).
+  {
+    const Divisor& by = CAUSAL ? w.by_order : w.by_tiles;
+    const Divisor& heads = DQ ? p.by_hq : p.by_hkv;
+    asm volatile("" ::"s"(w.per_xcd), "s"(w.total), "s"(by.mul), "s"(by.shift), "s"(by.d), "s"(heads.mul), "s"(heads.shift),
+                 "s"(heads.d), "s"(p.by_group.mul), "s"(p.by_group.shift), "s"(p.q), "s"(p.k), "s"(p.v), "s"(p.dout), "s"(p.lse2),
+                 "s"(p.delta), "s"(p.B), "s"(p.Sq), "s"(p.Sc), "s"(p.Hq), "s"(p.group), "s"(p.D), "s"(p.q_sb), "s"(p.q_ss),
+                 "s"(p.q_sh), "s"(p.k_sb), "s"(p.k_ss), "s"(p.k_sh), "s"(p.scale_log2));
+  }
   // Workgroup i runs on XCD i % 8: every XCD gets a contiguous range of (batch, head) pairs.  Under the
   // causal mask the work of a stationary tile grows (query tiles) or shrinks (key tiles) with its index:
   // such launches run the longest tiles first, across all heads.
@@ -112,27 +140,37 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   if (!CAUSAL) {
     const int logical = (block & 7) * w.per_xcd + (block >> 3);
     if (logical >= w.total) return;
-    st_tile = SPLIT ? logical % w.n_tiles / w.splits : logical % w.n_tiles;
-    split = SPLIT ? logical % w.n_tiles % w.splits : 0;
-    bh = logical / w.n_tiles;
+    bh = w.by_tiles.quotient(logical, st_tile);
+    split = 0;
+    if (SPLIT) {
+      split = st_tile & (w.splits - 1);
+      st_tile >>= w.log_splits;
+    }
   } else {
     int rank;                                       // position in longest-first order
     if (w.heads_per_xcd > 0) {
-      const int local = block >> 3;
-      rank = local / w.heads_per_xcd;
-      bh = (block & 7) * w.heads_per_xcd + local % w.heads_per_xcd;
+      rank = w.by_order.quotient(block >> 3, bh);
+      bh += (block & 7) * w.heads_per_xcd;
     } else {
       if (block >= w.total) return;
-      const int nbh = w.total / w.n_tiles;
-      rank = block / nbh;
-      bh = block % nbh;
+      rank = w.by_order.quotient(block, bh);
     }
-    split = SPLIT ? rank % w.splits : 0;
-    if (SPLIT) rank /= w.splits;
-    st_tile = DQ ? (SPLIT ? w.n_tiles / w.splits : w.n_tiles) - 1 - rank : rank;
+    split = 0;
+    if (SPLIT) {
+      split = rank & (w.splits - 1);
+      rank >>= w.log_splits;
+    }
+    st_tile = DQ ? (SPLIT ? w.n_tiles >> w.log_splits : w.n_tiles) - 1 - rank : rank;
   }
-  const int hs = DQ ? bh % p.Hq : bh % p.Hkv;       // stationary head: a q head (DQ) or a kv head
-  const int b = DQ ? bh / p.Hq : bh / p.Hkv;
+  const uint16_t* kp = p.k; const uint16_t* vp = p.v;       // the chunk a dK / dV workgroup belongs to; dQ: the first one
+  int chunk = 0;
+  if (CHUNKS) {
+    if (!DQ) chunk = chunks->by_heads.quotient(bh, bh);
+    kp = chunks->k[chunk];
+    vp = chunks->v[chunk];
+  }
+  int hs;                                           // stationary head: a q head (DQ) or a kv head
+  const int b = (DQ ? p.by_hq : p.by_hkv).quotient(bh, hs);
   const int r0 = st_tile * kRowsPerWg;
   const int n_st = DQ ? p.Sq : p.Sc;                // stationary / streamed sequence lengths
   const int n_str = DQ ? p.Sc : p.Sq;
@@ -154,7 +192,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   // ---- streamed tiles ---------------------------------------------------------------------------------
   // DQ: K / V rows of kv head hs / group.  Otherwise: Q / dout rows of the `group` query heads that share
   // kv head hs, one head after the other.
-  const int heads_str = DQ ? 1 : p.group;
+  const int heads_str = DQ ? (CHUNKS ? chunks->n : 1) : p.group;      // (DQ: chunks)
   int first_tile = 0, tiles_per_head = (n_str + kTile - 1) / kTile;
   if (CAUSAL) {
     if (DQ) {   // keys beyond the last row's diagonal are hidden
@@ -171,15 +209,15 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   // this workgroup's part of the stream: tiles t0 .. t0 + ntiles - 1 of the pass's sequence
   int t0 = 0, ntiles = span * heads_str;
   if (SPLIT && w.splits > 1) {
-    const int all = ntiles, part = (all + w.splits - 1) / w.splits;
+    const int all = ntiles, part = (all + w.splits - 1) >> w.log_splits;
     t0 = split * part < all ? split * part : all;
     ntiles = all - t0 < part ? all - t0 : part;
   }
 
   const uint16_t* xbase; const uint16_t* ybase; int64_t s_ss, s_sh; uint32_t s_bytes;
+  const int64_t kv_at = DQ ? b * p.k_sb + p.by_group.quotient(hs) * p.k_sh : 0;
   if (DQ) {
-    const int hk = hs / p.group;
-    xbase = p.k + b * p.k_sb + hk * p.k_sh; ybase = p.v + b * p.k_sb + hk * p.k_sh;
+    xbase = kp + kv_at; ybase = vp + kv_at;
     s_ss = p.k_ss; s_sh = 0;
     s_bytes = (uint32_t)(((int64_t)(p.Sc - 1) * p.k_ss + p.D) * 2);
   } else {
@@ -187,12 +225,17 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     s_ss = p.q_ss; s_sh = p.q_sh;
     s_bytes = (uint32_t)(((int64_t)(p.Sq - 1) * p.q_ss + (int64_t)(p.Hq - 1) * p.q_sh + p.D) * 2);
   }
-  const u32x4 xrs = rsrc_words(xbase, s_bytes);
-  const u32x4 yrs = rsrc_words(ybase, s_bytes);
-
-  // tile index -> (head of the group, first streamed row)
-  auto tile_head = [&](int t) { return DQ ? 0 : (t0 + t) / span; };
-  auto tile_row0 = [&](int t) { return (first_tile + (DQ ? t0 + t : (t0 + t) % span)) * kTile; };
+  u32x4 xrs = rsrc_words(xbase, s_bytes);
+  u32x4 yrs = rsrc_words(ybase, s_bytes);
+  // The address words of chunk i's descriptors in lane i: a scalar load of them inside the main loop would make its waits for
+  // one LDS operand waits for all.
+  uint32_t k_words[2] = {}, v_words[2] = {};
+  if (CHUNKS && DQ) {
+    const uint64_t ka = (uint64_t)(chunks->k[lane & (kMaxGroup - 1)] + kv_at), va = (uint64_t)(chunks->v[lane & (kMaxGroup - 1)] + kv_at);
+    k_words[0] = (uint32_t)ka; k_words[1] = (uint32_t)(ka >> 32) & 0xffffu;
+    v_words[0] = (uint32_t)va; v_words[1] = (uint32_t)(va >> 32) & 0xffffu;
+    asm volatile("" : "+v"(k_words[0]), "+v"(k_words[1]), "+v"(v_words[0]), "+v"(v_words[1]));
+  }
 
   // Wavefront w copies rows 16w .. 16w+15 of the X and the Y tile: four instructions of 1 KB each; lane l
   // of instruction u lands at row 16w + 4u + l/16, chunk position l%16, and fetches the chunk that lives
@@ -210,49 +253,50 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     cvoff[u] = chunk * 8 < p.D ? (int)(row * s_ss * 2) + (chunk << 4) : kNoColumn;
   }
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
-  auto copy_tile = [&](int t, int stage) {
-    const bool live = t < ntiles;
-    const int hq = DQ ? 0 : hs * p.group + tile_head(live ? t : 0);
-    const int c0 = tile_row0(live ? t : 0);
-    const int soff = live ? (int)(((int64_t)c0 * s_ss + (int64_t)hq * s_sh) * 2) : kNoTile;
-    const uint32_t dst = lds_base + stage * kStageBytes + wave * (kCpy * 1024);
-#pragma unroll
-    for (int u = 0; u < kCpy; ++u) copy16_to_lds(xrs, dst + u * 1024, cvoff[u], soff);
-#pragma unroll
-    for (int u = 0; u < kCpy; ++u) copy16_to_lds(yrs, dst + kOffY + u * 1024, cvoff[u], soff);
-    if (!DQ) {
-      const float* src = ((wave & 1) ? p.delta : p.lse2) + ((int64_t)b * p.Hq + hq) * p.Sq;
-      copy4_to_lds(rsrc_words(src, (uint32_t)p.Sq * 4u), lds_base + stage * kStageBytes + ((wave & 1) ? kOffDelta : kOffLse),
-                   lane * 4, live ? c0 * 4 : kNoTile);
-    }
-  };
   constexpr int kCopiesPerTile = DQ ? 2 * kCpy : 2 * kCpy + 1;
-  // The same copies one instruction at a time (piece 0 .. kCopiesPerTile - 1), so that the main loop can
-  // issue them between MFMAs; the scalar offsets are worked out once per tile by copy_setup.
-  // Which tile comes three tiles ahead is kept as a pair of running counters (position inside the head's span,
-  // head of the group) instead of a division per tile: every scalar instruction of the loop takes an issue slot of
+  // The copies of a tile go out one instruction at a time (piece 0 .. kCopiesPerTile - 1), in the main loop between
+  // MFMAs; copy_setup works out the scalar offsets of the next tile that has not been requested yet.  Which one that is is
+  // kept as a pair of running counters (position inside the head's span, head of the group; dQ: position in the chunk,
+  // chunk) instead of a division per tile: every scalar instruction of the loop takes an issue slot of
   // the one wavefront a SIMD runs in the dK / dV pass.
-  int cp_soff = 0, cp_ld_soff = 0;
-  int nx_r = DQ ? t0 + 3 : (span > 0 ? (t0 + 3) % span : 0), nx_h = DQ ? 0 : (span > 0 ? (t0 + 3) / span : 0), nx_t = 3;
+  int cp_soff = 0, cp_ld_soff = 0, cp_ld_voff = 0;
+  int nx_h = SPLIT && !DQ && span > 0 ? t0 / span : 0, nx_t = 0;
+  int nx_r = t0 - nx_h * span;
+  int cur_r = nx_r;                                   // position of the tile being worked on
   const uint32_t ld_rows = (uint32_t)p.B * (uint32_t)p.Hq * (uint32_t)p.Sq;     // the host keeps this below 2^30
   const u32x4 ldrs = rsrc_words((wave & 1) ? p.delta : p.lse2, ld_rows * 4u);
   auto copy_setup = [&]() {
-    const bool live = SPLIT ? nx_t < ntiles : DQ ? nx_r < span : nx_h < heads_str;
+    const bool live = SPLIT ? nx_t < ntiles : DQ && !CHUNKS ? nx_r < span : nx_h < heads_str;
     const uint32_t hq = DQ ? 0u : (uint32_t)(hs * p.group + (live ? nx_h : 0));
     const uint32_t c0 = (uint32_t)((first_tile + (live ? nx_r : 0)) * kTile);
     // element offsets stay below 2^31 (checked by the host), so 32-bit arithmetic is exact
     cp_soff = live ? (int)((c0 * (uint32_t)s_ss + hq * (uint32_t)s_sh) * 2u) : kNoTile;
-    if (!DQ) cp_ld_soff = live ? (int)((((uint32_t)b * (uint32_t)p.Hq + hq) * (uint32_t)p.Sq + c0) * 4u) : kNoTile;
+    if (!DQ) {
+      cp_ld_soff = live ? (int)((((uint32_t)b * (uint32_t)p.Hq + hq) * (uint32_t)p.Sq + c0) * 4u) : kNoTile;
+      // rows past the end are another head's: out of range (their scores are hidden, but 0 * infinity is not 0)
+      cp_ld_voff = (int)c0 + lane < p.Sq ? lane * 4 : kNoColumn;
+    }
+    if (CHUNKS && DQ && nx_r == 0 && live) {          // the copies of this chunk start here
+      xrs[0] = __builtin_amdgcn_readlane(k_words[0], nx_h);
+      xrs[1] = __builtin_amdgcn_readlane(k_words[1], nx_h);
+      yrs[0] = __builtin_amdgcn_readlane(v_words[0], nx_h);
+      yrs[1] = __builtin_amdgcn_readlane(v_words[1], nx_h);
+    }
     ++nx_r;
     if (SPLIT) ++nx_t;
-    if (!DQ && nx_r == span) { nx_r = 0; ++nx_h; }
+    if ((!DQ || CHUNKS) && nx_r == span) { nx_r = 0; ++nx_h; }
   };
   auto copy_piece = [&](int piece, int stage) {
     const uint32_t dst = lds_base + stage * kStageBytes + wave * (kCpy * 1024);
     if (piece < kCpy) copy16_to_lds(xrs, dst + piece * 1024, cvoff[piece < kCpy ? piece : 0], cp_soff);
     else if (piece < 2 * kCpy) copy16_to_lds(yrs, dst + kOffY + (piece - kCpy) * 1024, cvoff[piece < 2 * kCpy ? piece - kCpy : 0], cp_soff);
     else if (!DQ)
-      copy4_to_lds(ldrs, lds_base + stage * kStageBytes + ((wave & 1) ? kOffDelta : kOffLse), lane * 4, cp_ld_soff);
+      copy4_to_lds(ldrs, lds_base + stage * kStageBytes + ((wave & 1) ? kOffDelta : kOffLse), cp_ld_voff, cp_ld_soff);
+  };
+  auto copy_tile = [&](int stage) {                   // the next tile, all at once (prologue)
+    copy_setup();
+#pragma unroll
+    for (int piece = 0; piece < kCopiesPerTile; ++piece) copy_piece(piece, stage);
   };
 
   // row-major operand reads (A of T1 / T2): lane (ln, hf) reads chunk 2 kk + hf of row 32 mb + ln
@@ -304,6 +348,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   // The 16 steps of the vector pipeline are spread over the slots of a T1 / T2 phase: slot i runs steps vec0(i) .. vec0(i + 1) - 1.
   auto vec0 = [](int i) -> int { return i * 16 / kT; };
   typedef __attribute__((address_space(3))) const f32x4* lds_f32x4;
+  typedef __attribute__((address_space(3))) const float* lds_f32;
   // LDS addresses of the operand reads.  rm_a / tr_a hold, per lane, the addresses inside ONE tile's stage and are
   // moved on to the next stage in place, each at a point of the slot sequence where no read of its kind is due
   // (rm_a in the last kDepth slots of P0: the reads of the current tile's T1 / T2 operands are all issued by then and
@@ -439,8 +484,8 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   // repeat the last one, columns past the head dimension are cleared in the fragment.
   {
     const uint32_t x_lds = lds_base + kXRows + wave * 8192, y_lds = lds_base + kYRows + wave * 8192;
-    const uint16_t* xsrc = DQ ? p.q + b * p.q_sb + hs * p.q_sh : p.k + b * p.k_sb + hs * p.k_sh;
-    const uint16_t* ysrc = DQ ? p.dout + b * p.q_sb + hs * p.q_sh : p.v + b * p.k_sb + hs * p.k_sh;
+    const uint16_t* xsrc = DQ ? p.q + b * p.q_sb + hs * p.q_sh : kp + b * p.k_sb + hs * p.k_sh;
+    const uint16_t* ysrc = DQ ? p.dout + b * p.q_sb + hs * p.q_sh : vp + b * p.k_sb + hs * p.k_sh;
     const int64_t st_ss = DQ ? p.q_ss : p.k_ss;
     auto row_of = [&](int u) {                        // row and column of the lane's 16 bytes in copy u
       const int row = r0 + wave * 32 + 4 * u + (lane >> 4);
@@ -476,7 +521,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
       // This pass runs first and prepares what both passes need per query row: delta = rowsum(dout * out), kept
       // negated (the dP products start from it), and lse2 = lse * log2(e) with -inf (a row that saw no key) turned
       // into +inf so that P = exp2(s - lse2) = 0 there.
-      if (ntiles > 0) copy_tile(0, 0);
+      if (ntiles > 0) copy_tile(0);
       copy_rows(ysrc, y_lds);
       copy_rows(xsrc, x_lds);
       const uint16_t* osrc = p.out + b * p.o_sb + hs * p.o_sh;
@@ -516,26 +561,34 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
       }
       asm volatile("" : "+v"(lse2_lane), "+v"(delta_lane));
       __builtin_amdgcn_s_barrier();                  // the rows' places are stages 1 .. 3 from here on
-      if (ntiles > 0) { copy_tile(1, 1); copy_tile(2, 2); }
+      if (ntiles > 0) { copy_tile(1); copy_tile(2); }
     } else if (ntiles > 0) {
-      if (DQ) {
-        const int64_t r = ((int64_t)b * p.Hq + hs) * p.Sq + (my_r < n_st ? my_r : n_st - 1);
+      constexpr bool kEarly = WAVES == 4;            // stage 1 is not part of the rows' places
+      const int64_t r = DQ ? ((int64_t)b * p.Hq + hs) * p.Sq + (my_r < n_st ? my_r : n_st - 1) : 0;
+      const uint32_t ld_lds = lds_base + kSmemBytesOf<true, 4> + wave * 256;     // 32 rows' lse2, then their delta
+      if (DQ && !kEarly) {
         lse2_lane = p.lse2[r];
         delta_lane = p.delta[r];
         asm volatile("" : "+v"(lse2_lane), "+v"(delta_lane));
       }
-      constexpr bool kEarly = WAVES == 4;            // stage 1 is not part of the rows' places
-      copy_tile(0, 0);
+      copy_tile(0);
+      // (through LDS like the rows: loads into registers would be waited for before the first copy or with the last)
+      if (DQ && kEarly) copy4_to_lds((hf ? p.delta : p.lse2) + r, ld_lds);
       copy_rows(xsrc, x_lds);
       copy_rows(ysrc, y_lds);
-      if (kEarly) copy_tile(1, 1);
+      if (kEarly) copy_tile(1);
       asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kEarly ? kCopiesPerTile : 0) : "memory");
+      if (DQ && kEarly) {
+        lse2_lane = *(lds_f32)(uintptr_t)(ld_lds + ln * 4);
+        delta_lane = *(lds_f32)(uintptr_t)(ld_lds + 128 + ln * 4);
+      }
       read_rows(x_lds, xf);
       read_rows(y_lds, yf);
       pin();
+      if (DQ && kEarly) asm volatile("" : "+v"(lse2_lane), "+v"(delta_lane));
       __builtin_amdgcn_s_barrier();                  // tile 0 is there for everybody, the rows' places are free
-      if (!kEarly) copy_tile(1, 1);
-      copy_tile(2, 2);
+      if (!kEarly) copy_tile(1);
+      copy_tile(2);
     }
   }
   if (ntiles > 0) {
@@ -562,7 +615,6 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
       for (int g = 0; g < 4; ++g) read_nd(false, 1, g);        // for T2 of the second half, first thing in the loop
     }
   }
-  int cur_r = !DQ && span > 0 ? t0 % span : t0;          // (t0 + t) % span
   for (int t = 0; t < ntiles; ++t) {
     const int c0 = (first_tile + cur_r) * kTile;
     if (++cur_r == span) cur_r = 0;
@@ -711,9 +763,9 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
         else *qp = pack8(v);
       });
     }
-  } else if (p.dk32 == nullptr) {
-    write_out(acc1, p.scale, p.dk, p.dk_sb, p.dk_ss, p.dk_sh, hs);
-    write_out(acc2, 1.f, p.dv, p.dk_sb, p.dk_ss, p.dk_sh, hs);
+  } else if ((CHUNKS ? chunks->dk32[chunk] : p.dk32) == nullptr) {
+    write_out(acc1, p.scale, CHUNKS ? chunks->dk[chunk] : p.dk, p.dk_sb, p.dk_ss, p.dk_sh, hs);
+    write_out(acc2, 1.f, CHUNKS ? chunks->dv[chunk] : p.dv, p.dk_sb, p.dk_ss, p.dk_sh, hs);
   } else {
     auto store = [&](float* out32, uint16_t* out16) {
       return [=](f32x4 (&v)[2], int row, int col) {
@@ -724,8 +776,8 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
         if (out16) *reinterpret_cast<u32x4*>(out16 + b * p.dk_sb + (int64_t)row * p.dk_ss + hs * p.dk_sh + col) = w;
       };
     };
-    write_out32(acc1, p.scale, store(p.dk32, p.dk));
-    write_out32(acc2, 1.f, store(p.dv32, p.dv));
+    write_out32(acc1, p.scale, store(CHUNKS ? chunks->dk32[chunk] : p.dk32, CHUNKS ? chunks->dk[chunk] : p.dk));
+    write_out32(acc2, 1.f, store(CHUNKS ? chunks->dv32[chunk] : p.dv32, CHUNKS ? chunks->dv[chunk] : p.dv));
   }
 }
 
@@ -740,10 +792,19 @@ __global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p,
 template <bool CAUSAL, int KK, bool SPLIT>
 __global__ __launch_bounds__(256, 1) void bwd_joint(const BwdParams p, const TileMap wq, const TileMap wk) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<false, 4>];
-  static_assert(kSmemBytesOf<true, 4> <= kSmemBytesOf<false, 4>, "one array for both");
+  static_assert(kSmemBytesOf<true, 4> + 1024 <= kSmemBytesOf<false, 4>, "one array for both, and lse2 and delta of the dQ rows");
   const int first_q = wk.per_xcd * 8;         // a multiple of 8: both halves keep their XCDs
   if ((int)blockIdx.x < first_q) bwd_pass<false, CAUSAL, KK, 4, true, SPLIT>(p, wk, (int)blockIdx.x, smem);
   else bwd_pass<true, CAUSAL, KK, 4, true, SPLIT>(p, wq, (int)blockIdx.x - first_q, smem);
+}
+
+// The same for several chunks of a step.  The dQ workgroups, whose chains are the longest, come first.
+template <int KK>
+__global__ __launch_bounds__(256, 1) void bwd_joint_chunks(const BwdParams p, const TileMap wq, const TileMap wk, const Chunks chunks) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<false, 4>];
+  const int first_k = wq.per_xcd * 8;
+  if ((int)blockIdx.x < first_k) bwd_pass<true, false, KK, 4, true, false, true>(p, wq, (int)blockIdx.x, smem, &chunks);
+  else bwd_pass<false, false, KK, 4, true, false, true>(p, wk, (int)blockIdx.x - first_k, smem, &chunks);
 }
 
 // lse2 and delta for bwd_joint: 16 lanes per query row.
@@ -846,11 +907,14 @@ int scratch_address(void** ptr) {
 TileMap tile_map(int heads, int seq, int rows, int splits = 1, float* partial = nullptr) {
   TileMap w;
   w.splits = splits;
+  for (w.log_splits = 0; (1 << w.log_splits) < splits; ++w.log_splits) {}
   w.partial = partial;
   w.n_tiles = (seq + rows - 1) / rows * splits;
   w.total = heads * w.n_tiles;
   w.per_xcd = (w.total + 7) / 8;
   w.heads_per_xcd = heads % 8 == 0 ? heads / 8 : 0;
+  w.by_tiles = Divisor(w.n_tiles);
+  w.by_order = Divisor(w.heads_per_xcd > 0 ? w.heads_per_xcd : heads);
   return w;
 }
 
@@ -877,18 +941,19 @@ float launch_time(float n, float mean, float most, const Cost& c) {
 // their sums meet in a third launch (one / with it):
 //     B1 H8/1 512 x 512      82.6 / 27.6     B1 H8/1 2048 x 2048    310 / 73.6     B1 H8/1 4096 x 4096   636 /  221
 //     B1 H2/2 4096 x 4096    85.2 / 69.8     B1 H32/4 2048 x 2048   338 /  220     causal, D 64: H8/1 2048 x 2048  249 / 49.5
-struct Plan { bool joint; int sq, sk; };
+Cost joint_cost(int D) { return D <= 64 ? Cost{6.f, 0.75f, 0.12f} : Cost{7.f, 1.15f, 0.29f}; }
+struct Plan { bool joint; int sq, sk; float time; };       // time: estimated, without preparing delta and lse2
 constexpr int64_t kPartialMost = int64_t(32) << 20;     // bytes of sums a block may leave for bwd_reduce
 int64_t partial_bytes(int B, int S, int H, int D, int tensors, int splits) {
   return splits > 1 ? (int64_t)B * S * H * D * 4 * tensors * splits : 0;
 }
 Plan plan_block(int B, int Sq, int Sc, int Hq, int Hkv, int D, bool causal) {
-  Plan best = {false, 1, 1};
+  Plan best = {false, 1, 1, 0.f};
   if (Sq == 0 || Sc == 0 || B == 0) return best;
   const bool narrow = D <= 64;      // 96 columns: the costs of 128, of which both forms save the same 12 %
   const Cost dq8 = narrow ? Cost{6.f, 0.95f, 0.45f} : Cost{7.f, 1.45f, 0.75f};
   const Cost dkv = narrow ? Cost{6.f, 0.75f, 0.25f} : Cost{7.f, 1.15f, 0.55f};
-  const Cost both = narrow ? Cost{6.f, 0.75f, 0.12f} : Cost{7.f, 1.15f, 0.29f};
+  const Cost both = joint_cost(D);
   constexpr float kPrepare = 5.f, kReduce = 4.f, kBytesPerUs = 4e6f;
   const float tq = (float)((Sc + kTile - 1) / kTile), tk = (float)((Sq + kTile - 1) / kTile) * (Hq / Hkv);
   const float half = causal ? 0.53f : 1.f;          // mean share of the tiles under the diagonal
@@ -903,8 +968,36 @@ Plan plan_block(int B, int Sq, int Sc, int Hq, int Hkv, int D, bool causal) {
       const float n = nq4 * sq + nk * sk, mean = half * (nq4 * tq + nk * tk) / n;
       const float most = tq / sq > tk / sk ? tq / sq : tk / sk;
       const float time = kPrepare + launch_time(n, mean, most, both) + (bytes > 0 ? kReduce + 2.f * (float)bytes / kBytesPerUs : 0.f);
-      if (time < best_time) { best_time = time; best = {true, sq, sk}; }
+      if (time < best_time) { best_time = time; best = {true, sq, sk, 0.f}; }
     }
+  best.time = best_time - (best.joint ? kPrepare : 0.f);
+  return best;
+}
+
+// Chunks of a step that share a launch: the number of which the estimate expects the least time for the step, up to
+// kGroupWorkgroups workgroups.  Together the chunks fill the chip, and dQ's workgroups load their rows and meet the carried
+// sum once per launch instead of once per chunk; against it stands that a dQ workgroup's chain of tiles is as many times as
+// long.  Us a step, chunk by chunk / in launches of 2 / 4 / 8:
+//     8 chunks 512 x 512 B4 H5      162 /  117 / 95.8 / 89.5      1024 x 1024 H32                557 /  497 /  465 /  448
+//     256 x 256 H16                 104 / 67.2 / 56.8 / 52.3      512 x 512 H8/1                 201 /  337 /  174 / 90.2
+//     1237 x 1237 B2 H16/8 D80      632 /  605 /  510 /  499      700 x 700 H12 D64              141 /  100 / 82.8 / 72.9
+int group_chunks(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks) {
+  if (B == 0 || Sq == 0 || Sc == 0) return 1;
+  const int64_t nq = tile_map(B * Hq, Sq, kRowsQ / 2).total, nk = tile_map(B * Hkv, Sc, kRowsKv).total;
+  const float tq = (float)((Sc + kTile - 1) / kTile), tk = (float)((Sq + kTile - 1) / kTile) * (Hq / Hkv);
+  const Cost c = joint_cost(D);
+  int best = 1;
+  float best_time = plan_block(B, Sq, Sc, Hq, Hkv, D, false).time * chunks;
+  for (int launches = chunks; launches >= 1; --launches) {
+    const int n = (chunks + launches - 1) / launches;
+    const int64_t workgroups = nq + n * nk;
+    if (n > kMaxGroup || workgroups > kGroupWorkgroups) break;
+    const float share = workgroups < 256 ? (float)workgroups / 256.f : 1.f, step = c.step + share * c.busy;
+    const float longest = c.fixed + (n * tq > tk ? n * tq : tk) * step;
+    const float spread = (nq * (c.fixed + n * tq * step) + n * nk * (c.fixed + tk * step)) / 256.f;
+    const float time = ((chunks + n - 1) / n) * (longest > spread ? longest : spread);
+    if (n > 1 && time < best_time) { best_time = time; best = n; }
+  }
   return best;
 }
 
@@ -935,6 +1028,15 @@ void launch_bwd(const BwdParams& p, const Plan& plan, float* partial, hipStream_
   if (p.Sc > 0) hipLaunchKernelGGL((bwd_main<false, CAUSAL, KK, true>), dim3(wk.per_xcd * 8), dim3(256), 0, st, p, wk);
 }
 
+template <int KK>
+void launch_chunks(const BwdParams& p, const Chunks& chunks, hipStream_t st) {
+  const int rows = p.B * p.Hq * p.Sq;
+  if (!p.prepared) hipLaunchKernelGGL(bwd_prepare, dim3((rows + 15) / 16), dim3(256), 0, st, p, rows);
+  const TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ / 2);
+  const TileMap wk = tile_map(chunks.n * p.B * p.Hkv, p.Sc, kRowsKv);
+  hipLaunchKernelGGL((bwd_joint_chunks<KK>), dim3((wk.per_xcd + wq.per_xcd) * 8), dim3(256), 0, st, p, wq, wk, chunks);
+}
+
 // -delta, lse2 and delta, (B, Hq, Sq) fp32 each, every one starting on a 16-byte boundary
 int64_t row_bytes(int B, int Sq, int Hq) { return ((((int64_t)B * Hq * Sq + 3) & ~int64_t(3)) * 3) * 4; }
 }  // namespace
@@ -959,7 +1061,8 @@ extern "C" int mhip_attn_bwd_plan(int B, int Sq, int Sc, int Hq, int Hkv, int D,
 }
 
 namespace {
-// own_scratch: take the workspace from `scratch` (resolved after the arguments have been checked)
+// own_scratch: take the workspace from `scratch` (resolved after the arguments have been checked).  chunks: several of them,
+// the first one's places given as k .. dv32 too; they have been checked.
 int bwd_block(const void* dout, const void* q, const void* k, const void* v,
               const void* out, const float* lse,
               void* dq, void* dk, void* dv, float* dq_acc, int dq_mode, float* dk32, float* dv32, bool prepared,
@@ -969,7 +1072,7 @@ int bwd_block(const void* dout, const void* q, const void* k, const void* v,
               int64_t dk_sb, int64_t dk_ss, int64_t dk_sh,
               int64_t dq_sb, int64_t dq_ss, int64_t dq_sh,
               int64_t o_sb, int64_t o_ss, int64_t o_sh,
-              float softmax_scale, int mask, void* workspace, bool own_scratch, hipStream_t st) {
+              float softmax_scale, int mask, void* workspace, bool own_scratch, hipStream_t st, const Chunks* chunks = nullptr) {
   if (B < 0 || Sq < 0 || Sc < 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0) return MHIP_EINVAL;
   if (!(softmax_scale > 0.f) || !(softmax_scale < INFINITY)) return MHIP_EINVAL;
   if (mask != MHIP_MASK_NONE && mask != MHIP_MASK_CAUSAL) return MHIP_EINVAL;
@@ -1014,6 +1117,7 @@ int bwd_block(const void* dout, const void* q, const void* k, const void* v,
   p.dq_acc = dq_acc; p.dq_mode = dq_mode; p.prepared = prepared;
   p.dk32 = dk32; p.dv32 = dv32;
   p.B = B; p.Sq = Sq; p.Sc = Sc; p.Hq = Hq; p.Hkv = Hkv; p.group = Hq / Hkv;
+  p.by_hq = Divisor(Hq); p.by_hkv = Divisor(Hkv); p.by_group = Divisor(Hq / Hkv);
   p.D = D;
   p.q_sb = q_sb; p.q_ss = q_ss; p.q_sh = q_sh;
   p.k_sb = k_sb; p.k_ss = k_ss; p.k_sh = k_sh;
@@ -1023,6 +1127,12 @@ int bwd_block(const void* dout, const void* q, const void* k, const void* v,
   p.scale = softmax_scale; p.scale_log2 = softmax_scale * kLog2e;
   const bool causal = mask == MHIP_MASK_CAUSAL;
 
+  if (chunks) {
+    if (D <= 64) launch_chunks<4>(p, *chunks, st);
+    else if (D <= 96) launch_chunks<6>(p, *chunks, st);
+    else launch_chunks<8>(p, *chunks, st);
+    return launch_status();
+  }
   const Plan plan = plan_block(B, Sq, Sc, Hq, Hkv, D, causal);
   if (D <= 64) causal ? launch_bwd<true, 4>(p, plan, partial, st) : launch_bwd<false, 4>(p, plan, partial, st);
   else if (D <= 96) causal ? launch_bwd<true, 6>(p, plan, partial, st) : launch_bwd<false, 6>(p, plan, partial, st);
@@ -1092,4 +1202,53 @@ extern "C" int mhip_attn_bwd_chunk(const void* dout, const void* q, const void* 
                    only ? kDqAdd : first ? kDqFirst : last ? kDqLast : kDqMiddle, dk32, dv32, prepared != 0,
                    B, Sq, Sc, Hq, Hkv, D, q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, dk_sb, dk_ss, dk_sh, dq_sb, dq_ss, dq_sh,
                    o_sb, o_ss, o_sh, softmax_scale, mask, workspace, false, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int mhip_attn_bwd_group(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks) {
+  if (B < 0 || Sq < 0 || Sc < 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || D <= 0 || D > kD || chunks < 1) return MHIP_EINVAL;
+  return group_chunks(B, Sq, Sc, Hq, Hkv, D, chunks);
+}
+
+extern "C" int mhip_attn_bwd_chunks(const void* dout, const void* q, const void* const* ks, const void* const* vs, int n,
+                                    const void* out, const float* lse,
+                                    void* dq, float* dq_acc, int first, int last, int prepared,
+                                    void* const* dks, void* const* dvs, float* const* dk32s, float* const* dv32s,
+                                    int B, int Sq, int Sc, int Hq, int Hkv, int D,
+                                    int64_t q_sb, int64_t q_ss, int64_t q_sh,
+                                    int64_t k_sb, int64_t k_ss, int64_t k_sh,
+                                    int64_t dk_sb, int64_t dk_ss, int64_t dk_sh,
+                                    int64_t dq_sb, int64_t dq_ss, int64_t dq_sh,
+                                    int64_t o_sb, int64_t o_ss, int64_t o_sh,
+                                    float softmax_scale, void* workspace, void* stream) {
+  if (n < 1 || n > kMaxGroup || !ks || !vs || !dks || !dvs || !dk32s || !dv32s) return MHIP_EINVAL;
+  if (n == 1 || B == 0 || Sq == 0 || Sc == 0) {
+    for (int i = 0; i < n; ++i) {
+      const int rc = mhip_attn_bwd_chunk(dout, q, ks[i], vs[i], out, lse, dq, dq_acc, first && i == 0, last && i + 1 == n,
+                                         prepared || i > 0, dks[i], dvs[i], dk32s[i], dv32s[i], B, Sq, Sc, Hq, Hkv, D, q_sb, q_ss, q_sh,
+                                         k_sb, k_ss, k_sh, dk_sb, dk_ss, dk_sh, dq_sb, dq_ss, dq_sh, o_sb, o_ss, o_sh, softmax_scale,
+                                         MHIP_MASK_NONE, workspace, stream);
+      if (rc != MHIP_OK) return rc;
+    }
+    return MHIP_OK;
+  }
+  if ((int64_t)n * B * Hkv * (((int64_t)Sc + 127) / 128) >= (int64_t(1) << 30)) return MHIP_EUNSUPPORTED;    // workgroups in 32 bits
+  Chunks c;
+  c.n = n;
+  c.by_heads = Divisor(B * (int64_t)Hkv > 0 ? B * Hkv : 1);
+  for (int i = 0; i < kMaxGroup; ++i) {
+    const int j = i < n ? i : 0;
+    c.k[i] = static_cast<const uint16_t*>(ks[j]); c.v[i] = static_cast<const uint16_t*>(vs[j]);
+    c.dk[i] = static_cast<uint16_t*>(dks[j]); c.dv[i] = static_cast<uint16_t*>(dvs[j]);
+    c.dk32[i] = dk32s[j]; c.dv32[i] = dv32s[j];
+    if (!c.k[i] || !c.v[i] || !c.dk32[i] != !c.dv32[i] || !c.dk[i] != !c.dv[i] || (!c.dk32[i] && !c.dk[i])) return MHIP_EINVAL;
+    const void* ptrs[] = {c.k[i], c.v[i], c.dk[i], c.dv[i], c.dk32[i], c.dv32[i]};
+    for (const void* ptr : ptrs)
+      if (ptr && !aligned16(ptr)) return MHIP_EALIGN;
+  }
+  const bool only = first && last;
+  if (!first && !dq_acc) return MHIP_EINVAL;
+  return bwd_block(dout, q, ks[0], vs[0], out, lse, dq, dks[0], dvs[0], only ? nullptr : dq_acc,
+                   only ? kDqAdd : first ? kDqFirst : last ? kDqLast : kDqMiddle, dk32s[0], dv32s[0], prepared != 0,
+                   B, Sq, Sc, Hq, Hkv, D, q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, dk_sb, dk_ss, dk_sh, dq_sb, dq_ss, dq_sh,
+                   o_sb, o_ss, o_sh, softmax_scale, MHIP_MASK_NONE, workspace, false, static_cast<hipStream_t>(stream), &c);
 }

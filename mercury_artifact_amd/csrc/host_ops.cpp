@@ -31,6 +31,8 @@ struct Entry {
   decltype(&mhip_attn_bwd_workspace_bytes) bwd_bytes = nullptr;
   decltype(&mhip_attn_bwd_block) bwd = nullptr;
   decltype(&mhip_attn_bwd_chunk) chunk = nullptr;
+  decltype(&mhip_attn_bwd_chunks) bwd_many = nullptr;
+  decltype(&mhip_attn_bwd_group) bwd_group = nullptr;
   decltype(&mhip_lse_merge) merge = nullptr;
   decltype(&mhip_lse_merge_many) many = nullptr;
   decltype(&mhip_pack_reduce) pack = nullptr;
@@ -434,6 +436,89 @@ PyObject* bwd_chunk(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// (q, chunk, chunks): how many of a step's chunks to launch together
+PyObject* bwd_group(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ENTER(3);
+  const Tensor *q = plain(a[0]), *c = plain(a[1]);
+  const long n = PyLong_AsLong(a[2]);
+  if (n == -1 && PyErr_Occurred()) { PyErr_Clear(); SLOW; }
+  if (!q || !c || q->dim() != 4 || c->dim() != 5 || c->size(3) == 0 || q->size(2) % c->size(3) ||
+      !fits({q->size(0), q->size(1), q->size(2), q->size(3), c->size(2), n}))
+    SLOW;
+  const int most = entry.bwd_group(q->size(0), q->size(1), c->size(2), q->size(2), c->size(3), q->size(3), n);
+  if (most < 1) SLOW;
+  return PyLong_FromLong(most);
+  END_HANDLE_TH_ERRORS
+}
+
+// (dout, q, chunks, out, softmax_lse, dq, dq_acc, first, last, dkvs, dkv32s, softmax_scale, workspace) -> workspace: bwd_chunk
+// over the (2, B, Sc, Hkv, D) tensors of a list in one launch; dkvs and dkv32s are lists of as many tensors or Nones
+PyObject* bwd_chunks(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ENTER(13);
+  for (int i : {2, 9, 10})
+    if (!PyList_CheckExact(a[i]) || PyList_GET_SIZE(a[i]) != PyList_GET_SIZE(a[2])) SLOW;
+  const Py_ssize_t n = PyList_GET_SIZE(a[2]);
+  if (n < 1 || n > MHIP_MAX_GROUP) SLOW;
+  const Tensor *dout = plain(a[0]), *q = plain(a[1]), *c0 = plain(PyList_GET_ITEM(a[2], 0)), *out = plain(a[3]), *lse = plain(a[4]);
+  if (!dout || !q || !c0 || !out || !lse || q->dim() != 4 || c0->dim() != 5) SLOW;
+  const int64_t B = q->size(0), Sq = q->size(1), Hq = q->size(2), D = q->size(3), Sc = c0->size(2), Hkv = c0->size(3);
+  const Tensor *dq, *acc, *kept;
+  if (!optional(a[5], *q, dq) || !optional(a[6], *q, acc) || !optional(a[12], *q, kept)) SLOW;
+  for (const Tensor* t : {dout, q, out, dq})
+    if (t && (!shape4(*t, B, Sq, Hq, D) || !rows16(*t) || t->device() != q->device())) SLOW;
+  if (Hkv == 0 || Hq % Hkv || !same_layout(*q, *dout) || lse->device() != q->device() || !shape3(*lse, B, Hq, Sq) ||
+      lse->scalar_type() != at::kFloat || !lse->is_contiguous() || !fits({B, Sq, Sc, Hq}))
+    SLOW;
+  if (acc && (acc->sizes() != q->sizes() || acc->scalar_type() != at::kFloat || !acc->is_contiguous())) SLOW;
+  auto rows = [](const Tensor& t) {
+    return t.scalar_type() == at::kBFloat16 && t.stride(4) == 1 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && t.stride(2) % 8 == 0 &&
+           t.stride(3) % 8 == 0;
+  };
+  const void *ks[MHIP_MAX_GROUP], *vs[MHIP_MAX_GROUP];
+  void *dks[MHIP_MAX_GROUP], *dvs[MHIP_MAX_GROUP];
+  float *dk32s[MHIP_MAX_GROUP], *dv32s[MHIP_MAX_GROUP];
+  const Tensor* g0 = nullptr;                     // the bf16 gradients have one layout
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    const Tensor *c = plain(PyList_GET_ITEM(a[2], i)), *g, *g32;
+    if (!c || c->device() != q->device() || c->dim() != 5 || c->size(0) != 2 || c->size(1) != B || c->size(2) != Sc ||
+        c->size(3) != Hkv || c->size(4) != D || !rows(*c) || c->strides() != c0->strides() ||
+        !optional(PyList_GET_ITEM(a[9], i), *q, g) || !optional(PyList_GET_ITEM(a[10], i), *q, g32))
+      SLOW;
+    if (g && (g->sizes() != c0->sizes() || !rows(*g) || (g0 && g->strides() != g0->strides()))) SLOW;
+    if (g32 && (g32->sizes() != c0->sizes() || g32->scalar_type() != at::kFloat || !g32->is_contiguous())) SLOW;
+    if (g && !g0) g0 = g;
+    ks[i] = c->data_ptr();
+    vs[i] = static_cast<const char*>(ks[i]) + 2 * c->stride(0);
+    dks[i] = data(g);
+    dvs[i] = g ? static_cast<char*>(dks[i]) + 2 * g->stride(0) : nullptr;
+    dk32s[i] = floats(g32);
+    dv32s[i] = g32 ? dk32s[i] + g32->stride(0) : nullptr;
+  }
+  const int first = PyObject_IsTrue(a[7]), last = PyObject_IsTrue(a[8]);
+  const double scale = PyFloat_AsDouble(a[11]);
+  if (first < 0 || last < 0 || (scale == -1.0 && PyErr_Occurred())) { PyErr_Clear(); SLOW; }
+  if (kept && (kept->scalar_type() != at::kByte || !kept->is_contiguous() ||
+               kept->numel() != entry.bwd_bytes(B, Sq, Sc, Hq, Hkv, D)))
+    SLOW;
+  OnDevice on(*q);
+  if (!on.current) SLOW;
+  Tensor ws;
+  const int code = without_gil([&] {
+    ws = kept ? *kept : bwd_workspace(*q, Sc, Hkv);
+    return entry.bwd_many(dout->data_ptr(), q->data_ptr(), ks, vs, (int)n, out->data_ptr(), floats(lse), data(dq), floats(acc), first,
+                          last, kept != nullptr, dks, dvs, dk32s, dv32s, B, Sq, Sc, Hq, Hkv, D,
+                          q->stride(0), q->stride(1), q->stride(2), c0->stride(1), c0->stride(2), c0->stride(3),
+                          g0 ? g0->stride(1) : 0, g0 ? g0->stride(2) : 0, g0 ? g0->stride(3) : 0,
+                          dq ? dq->stride(0) : 0, dq ? dq->stride(1) : 0, dq ? dq->stride(2) : 0,
+                          out->stride(0), out->stride(1), out->stride(2), (float)scale, ws.data_ptr(), on.stream);
+  });
+  if (code != MHIP_OK) return refused(code, "mhip_attn_bwd_chunks");
+  return give(ws);
+  END_HANDLE_TH_ERRORS
+}
+
 // (acc_out, acc_lse, block_out, block_lse, dst_out, dst_lse, final_out, final_lse) -> True
 PyObject* merge_into(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
@@ -595,6 +680,7 @@ PyObject* bind(PyObject*, PyObject* table) {
   const bool ok = take(entry.fwd, "mhip_attn_fwd_block") && take(entry.fwd_many, "mhip_attn_fwd_blocks") &&
                   take(entry.fwd_group, "mhip_attn_fwd_group") && take(entry.bwd_bytes, "mhip_attn_bwd_workspace_bytes") &&
                   take(entry.bwd, "mhip_attn_bwd_block") && take(entry.chunk, "mhip_attn_bwd_chunk") &&
+                  take(entry.bwd_many, "mhip_attn_bwd_chunks") && take(entry.bwd_group, "mhip_attn_bwd_group") &&
                   take(entry.merge, "mhip_lse_merge") && take(entry.many, "mhip_lse_merge_many") &&
                   take(entry.pack, "mhip_pack_reduce") && take(entry.unpack, "mhip_unpack") &&
                   take(entry.quantize, "mhip_quantize_e4m3") && take(entry.error_string, "mhip_error_string");
@@ -606,7 +692,7 @@ PyObject* bind(PyObject*, PyObject* table) {
 #define FAST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     FAST(undispatched), FAST(written), FAST(apart), FAST(rows_fit), FAST(fwd_block), FAST(fwd_group), FAST(fwd_blocks), FAST(no_dropout), FAST(bwd_block),
-    FAST(bwd_chunk), FAST(merge_into), FAST(merge_many), FAST(pack_block), FAST(unpack_into), FAST(quantize_e4m3),
+    FAST(bwd_chunk), FAST(bwd_group), FAST(bwd_chunks), FAST(merge_into), FAST(merge_many), FAST(pack_block), FAST(unpack_into), FAST(quantize_e4m3),
     {"bind", bind, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_mercury_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

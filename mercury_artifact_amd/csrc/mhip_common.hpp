@@ -19,7 +19,8 @@ typedef __attribute__((__vector_size__(2 * sizeof(float)))) float f32x2;
 typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
 typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2;
 
-constexpr int kMaxGroup = MHIP_MAX_GROUP;     // blocks of a step in one launch
+constexpr int kMaxGroup = MHIP_MAX_GROUP;     // blocks of a step in one launch,
+constexpr int kGroupWorkgroups = 2048;        // and their workgroups: eight rounds on 256 CUs
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
@@ -111,6 +112,12 @@ __device__ __forceinline__ void copy16_to_lds(const void* src, uint32_t lds_addr
                :: "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(src) : "memory");
 }
 
+// The same for 4 bytes per lane.
+__device__ __forceinline__ void copy4_to_lds(const void* src, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
+               :: "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(src) : "memory");
+}
+
 // Tiles copied that way are rows of 256 bytes (128 bf16) without padding; chunk c (16 bytes) of row r is
 // kept at chunk position c ^ lds_row_swizzle(r).  With this map both access patterns of the MFMA operand
 // reads are free of bank conflicts: 32 consecutive rows x one chunk (ds_read_b128 of a row-major operand)
@@ -124,7 +131,7 @@ struct Divisor {
   uint32_t mul, shift, d;
   Divisor() = default;
   explicit Divisor(int divisor) : d((uint32_t)(divisor > 0 ? divisor : 1)) {
-    for (shift = 0; (uint64_t(1) << shift) < d; ++shift) {}
+    shift = d > 1 ? 32 - __builtin_clz(d - 1) : 0;
     mul = (uint32_t)(((uint64_t(1) << 32) * ((uint64_t(1) << shift) - d)) / d + 1);
   }
   __device__ __forceinline__ int quotient(int n, int& rest) const {

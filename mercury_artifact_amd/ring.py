@@ -7,8 +7,8 @@ neighbour exchange.  The body is the loop the code generator emits for that temp
 (mercury/backend/pytorch/codegen.py:264-355, 443-523): take the current KV chunk, start the hop for
 the next one, run the block kernel, fold with ``update_out_and_lse``, and store after the last step.  A
 forward driver's blocks go through ``_flash_attn_forward`` unless it would do nothing but call the kernel;
-then they are written straight into places allocated once per step, and where one block would leave most of the chip
-idle, the driver waits for further chunks and launches their blocks together.
+then they are written straight into places allocated once per step, and where a ring's chunks all lie in this GPU's
+memory (``LocalRing.resident``), the blocks of several are launched together if one launch each is too small for the chip.
 
 Two defaults of the forward drivers depart from the literal sequence without changing what is computed:
 ``deferred_merge=True`` keeps the bf16 block results of all chunks and folds them with ONE
@@ -109,13 +109,12 @@ def _block_results(n, q, kv, softmax_scale, dropout_p, causal, window_size, alib
 
 
 class _Groups:
-    """Block forwards of one query tensor over a step's chunks, several to a launch where one block leaves most of the chip
-    idle and the ring lets its chunks lie (mhip_attn_fwd_group has the rule); ``size`` is 1 where every block goes its own
-    way."""
+    """Block forwards of one query tensor over a step's chunks, several to a launch where the ring's chunks are all there
+    (mhip_attn_fwd_group has the rule); ``size`` is 1 where every block goes its own way."""
 
     def __init__(self, q, places, ring, softmax_scale, causal, q_descale=None, k_descale=None, v_descale=None):
         self.size = 1
-        if places.stacked is not None and type(ring).__dict__.get("keeps_chunks"):
+        if places.stacked is not None and type(ring).__dict__.get("resident"):
             self.size = N.host.fwd_group(q, len(places)) or 1
         if self.size > 1:
             self.q, self.places, self.done, self.chunks = q, places, 0, []
@@ -505,6 +504,9 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
         reduce_dq = torch.empty(q.shape, dtype=torch.float32, device=q.device)
     _kv = _next_kv = prepared = None
     own = ring.current
+    group, waiting = 1, []
+    if carried and type(ring).__dict__.get("resident"):
+        group = N.host.bwd_group(q, kv, ring.world) or 1
     for step, hop in enumerate(_hops(ring)):
         if step == 0:
             _kv = kv.contiguous()
@@ -517,27 +519,44 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
             _next_kv = ring.send_recv(send_to, recv_from, _kv)
             ring.commit()
         if carried:
-            mine = chunk_id == own
-            direct = (mine and dkv.shape == _kv.shape and aligned_rows(dkv[0], dkv[1])
-                      and N.host.apart(dkv, q, dout, o, lse, _kv))
+            waiting.append((chunk_id, _kv))
+            if len(waiting) < group and hop is not None:
+                continue
+            chunks = [c for _, c in waiting]
             if hop is None and write_dq and step > 0:
-                write_dq = N.host.apart(dq, _kv)
-            block_dkv = chunk_grad = None
-            if direct:
-                block_dkv = dkv
-            elif mine or dkv_chunks is None:
-                block_dkv = torch.empty(_kv.shape, dtype=_kv.dtype, device=_kv.device)
-            if dkv_chunks is not None:
-                chunk_grad = dkv_chunks[chunk_id] = torch.empty(_kv.shape, dtype=torch.float32, device=_kv.device)
-            _k, _v = _as_rows(_kv).unbind(0)
+                write_dq = N.host.apart(dq, *chunks)
+            block_dkvs, chunk_grads, staged = [], [], None
+            for i, c in waiting:
+                direct = (i == own and dkv.shape == c.shape and aligned_rows(dkv[0], dkv[1])
+                          and N.host.apart(dkv, q, dout, o, lse, *chunks))
+                block_dkv = chunk_grad = None
+                if direct:
+                    block_dkv = dkv
+                elif i == own or dkv_chunks is None:
+                    block_dkv = torch.empty(c.shape, dtype=c.dtype, device=c.device)
+                    staged = block_dkv if i == own else staged
+                if dkv_chunks is not None:
+                    chunk_grad = dkv_chunks[i] = torch.empty(c.shape, dtype=torch.float32, device=c.device)
+                block_dkvs.append(block_dkv)
+                chunk_grads.append(chunk_grad)
             # rowsum(dout * o) and the scaled lse are the same for every chunk: worked out with the first one
-            usual = _kv.shape == kv.shape
-            ws = attn_bwd_chunk(dout, q, _k, _v, o, lse, dq if write_dq else None, reduce_dq, step == 0,
-                                bool(write_dq and hop is None), block_dkv, chunk_grad, softmax_scale,
-                                prepared if usual else None)
-            prepared = ws if usual else prepared
-            if mine and not direct:
-                dkv[...] = block_dkv
+            rows = [_as_rows(c) for c in chunks]
+            first, last = step + 1 == len(chunks), bool(write_dq and hop is None)
+            done = None
+            if len(chunks) > 1:
+                done = N.host.bwd_chunks(dout, q, rows, o, lse, dq if last else None, reduce_dq, first, last, block_dkvs,
+                                         chunk_grads, softmax_scale, prepared)
+                prepared = done if prepared is None else prepared
+            for n, c in enumerate(rows if done is None else ()):
+                _k, _v = c.unbind(0)
+                usual = c.shape == kv.shape
+                ws = attn_bwd_chunk(dout, q, _k, _v, o, lse, dq if write_dq else None, reduce_dq, first and n == 0,
+                                    last and n + 1 == len(rows), block_dkvs[n], chunk_grads[n], softmax_scale,
+                                    prepared if usual else None)
+                prepared = ws if usual else prepared
+            if staged is not None:
+                dkv[...] = staged
+            waiting = []
             continue
         block_dq = torch.empty(q.shape, dtype=q.dtype, device=q.device)
         block_dkv = torch.empty(_kv.shape, dtype=kv.dtype, device=kv.device)

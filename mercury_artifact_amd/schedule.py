@@ -273,10 +273,11 @@ class LocalRing:
     have received.
     """
 
-    # What a wait has delivered stays as it is for the rest of the step.  A ring class says so for itself (a class
-    # derived from this one may receive into buffers it uses again); drivers may then wait for several chunks first and
-    # launch their blocks together.
-    keeps_chunks = True
+    # Every chunk lies in this GPU's memory for the whole step -- the emulated exchange, or chunks gathered beforehand -- and
+    # a hop only says whose turn it is.  Drivers may then take several chunks before they launch, and launch their
+    # blocks together.  A ring class says so for itself: with one that receives its chunks, derived from this one or not, a
+    # block is launched when its chunk is there, so that the next hop runs beside it.
+    resident = True
 
     def __init__(self, mesh_shape: Sequence[int], rank: int,
                  chunks: Optional[Sequence[torch.Tensor]] = None, copy: bool = False):

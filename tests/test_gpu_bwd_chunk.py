@@ -161,3 +161,96 @@ def test_backward_step_in_place(W, dq_over):
     M.flash_attn_backward(t["q"], chunks[0], t["o"], lse, t["dout"], *got, 0.1, ring=M.LocalRing((W,), 0, chunks))
     torch.cuda.synchronize()
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+GROUPED = [(8, 1, 64, 2, 2, 128, 8), (5, 2, 129, 4, 2, 64, 5), (3, 1, 300, 5, 1, 96, 3), (5, 1, 1024, 32, 32, 128, 5), (8, 2, 512, 5, 5, 128, 8), (7, 1, 257, 8, 8, 80, 7),
+           (6, 2, 65, 3, 3, 40, 6), (16, 1, 200, 2, 1, 128, 16), (17, 1, 100, 2, 2, 64, 9)]
+
+
+@pytest.mark.parametrize("W,B,S,Hq,Hkv,D,group", GROUPED)
+@pytest.mark.parametrize("dq_dtype,keep", [(torch.bfloat16, True), (torch.float32, True), (torch.bfloat16, False)])
+def test_backward_step_in_grouped_launches(W, B, S, Hq, Hkv, D, group, dq_dtype, keep):
+    """Steps whose chunks share launches: one to three launches, chunks of one to eight tiles (the dQ pass changes chunks
+    before, at and behind the tiles its prologue requests), ragged rows, grouped heads."""
+    import mercury_artifact_amd as M
+
+    print(f"grouped W{W} B{B} S{S} Hq{Hq} Hkv{Hkv} D{D} {dq_dtype} keep={keep}", flush=True)
+    assert N.lib().mhip_attn_bwd_group(B, S, S, Hq, Hkv, D, W) == group
+    rank, scale = W // 2, D ** -0.5
+    g = torch.Generator().manual_seed(W * 1000 + S)
+    q, dout = (torch.randn(B, S, Hq, D, generator=g).bfloat16() for _ in range(2))
+    kvs = [torch.randn(2, B, S, Hkv, D, generator=g).bfloat16() for _ in range(W)]
+    order = O.single_ring_order(rank, W)
+    o, lse = O.ring_forward(q.float(), [c.float() for c in kvs], order, scale)
+    rdq, rdkv = O.ring_backward(q.float(), [c.float() for c in kvs], order, o.bfloat16().float(), lse, dout.float(), scale)
+    dev = [c.cuda() for c in kvs]
+    dq = torch.full(q.shape, float("nan"), dtype=dq_dtype, device="cuda")
+    dkv = torch.full_like(dev[rank], float("nan"))
+    got = {} if keep else None
+    M.flash_attn_backward(q.cuda(), dev[rank], o.bfloat16().cuda(), lse.cuda(), dout.cuda(), dq, dkv, scale,
+                          ring=M.LocalRing((W,), rank, dev), dkv_chunks=got)
+    torch.cuda.synchronize()
+    _close("dq", dq, rdq)
+    _close("own dkv", dkv, torch.stack(tuple(rdkv[rank])))
+    for c in range(W) if keep else ():
+        assert got[c].dtype == torch.float32
+        _close(f"dkv {c}", got[c], torch.stack(tuple(rdkv[c])))
+
+    class Other(M.LocalRing):            # makes no promise about its chunks: one launch each, the same gradients
+        pass
+
+    dq1, dkv1, got1 = torch.empty_like(dq), torch.empty_like(dkv), {} if keep else None
+    M.flash_attn_backward(q.cuda(), dev[rank], o.bfloat16().cuda(), lse.cuda(), dout.cuda(), dq1, dkv1, scale,
+                          ring=Other((W,), rank, dev), dkv_chunks=got1)
+    _close("dq, chunk by chunk", dq1, rdq)
+    _close("dkv, chunk by chunk", dkv1, torch.stack(tuple(rdkv[rank])))
+
+
+@pytest.mark.parametrize("over", ["own chunk", "other chunk", "q"])
+def test_grouped_gradients_over_operands(over):
+    """dq or dkv over something a grouped launch reads: stored behind the launch, same values."""
+    import mercury_artifact_amd as M
+
+    W, B, S, H, D = 4, 1, 200, 4, 64
+    assert N.lib().mhip_attn_bwd_group(B, S, S, H, H, D, W) == 4
+    g = torch.Generator().manual_seed(3)
+
+    def fresh():
+        g.manual_seed(3)
+        q, dout, o = (torch.randn(B, S, H, D, generator=g).bfloat16().cuda() for _ in range(3))
+        chunks = [torch.randn(2, B, S, H, D, generator=g).bfloat16().cuda() for _ in range(W)]
+        return q, dout, o, chunks, torch.full((B, H, S), 6.0, device="cuda")
+
+    def step(q, dout, o, chunks, lse, dq, dkv):
+        got = {}
+        M.flash_attn_backward(q, chunks[1], o, lse, dout, dq, dkv, 0.125, ring=M.LocalRing((W,), 1, chunks), dkv_chunks=got)
+        return dq.clone(), dkv.clone(), got
+
+    t = fresh()
+    want = step(*t, torch.empty_like(t[0]), torch.empty_like(t[3][1]))
+    t = fresh()
+    dq = t[0] if over == "q" else torch.empty_like(t[0])
+    dkv = t[3][1] if over == "own chunk" else t[3][2] if over == "other chunk" else torch.empty_like(t[3][1])
+    have = step(*t, dq, dkv)
+    assert torch.equal(have[1], want[1]) and (have[0].float() - want[0].float()).abs().max() <= 2 ** -7 * want[0].float().abs().max()
+    assert all(torch.equal(have[2][i], want[2][i]) for i in range(W))
+
+
+def test_rows_past_the_end_are_no_other_heads():
+    """A head whose dout is not finite leaves the next head's gradients alone, also in the ragged last tile of a long stream."""
+    import mercury_artifact_amd as M
+
+    B, S, H, D = 1, 330, 3, 64
+    g = torch.Generator().manual_seed(8)
+    q, dout, o = (torch.randn(B, S, H, D, generator=g).bfloat16().cuda() for _ in range(3))
+    kv = torch.randn(2, B, S, H, D, generator=g).bfloat16().cuda()
+    lse = torch.full((B, H, S), 6.0, device="cuda")
+    grads = []
+    for bad in (0.0, float("inf"), float("nan")):
+        d = dout.clone()
+        d[:, :, 1] = d[:, :, 1] + bad
+        dq, dkv = torch.empty_like(q), torch.empty_like(kv)
+        M.attn_bwd_block(d, q, kv[0], kv[1], o, lse, dq, dkv[0], dkv[1], 0.125)
+        grads.append(torch.stack((dq, dkv[0], dkv[1]))[:, :, :, ::2])
+    assert torch.isfinite(grads[0].float()).all()
+    assert torch.equal(grads[1], grads[0]) and torch.equal(grads[2], grads[0])

@@ -72,7 +72,7 @@ def test_blocks_refuse_what_a_launch_cannot_take():
 
 @pytest.mark.parametrize("path", ["ring", "packed", "zigzag"])
 @pytest.mark.parametrize("own_class", [False, True])
-def test_only_rings_that_keep_their_chunks_get_grouped_launches(path, own_class):
+def test_only_rings_with_resident_chunks_get_grouped_launches(path, own_class):
     """A class derived from LocalRing may receive into a buffer it uses again, as this one does: its blocks are launched one
     by one, before the next hop overwrites their chunk.  Same results either way."""
     import mercury_artifact_amd as M

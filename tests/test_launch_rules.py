@@ -51,11 +51,22 @@ def test_carried_sums_are_tested_in_both_forms(columns):
     assert any(_columns(c[4]) == columns and bwd_plan(2, c[1], c[1], *c[2:], False)[0] == 1 for c in JOINT)
 
 
-def test_blocks_of_a_step_share_a_launch_until_it_fills_the_chip():
+def test_blocks_of_a_step_share_a_launch_of_up_to_eight_rounds():
     group = N.lib().mhip_attn_fwd_group
-    assert group(1, 4096, 32, 8) == group(1, 1025, 32, 8) == 1                # half of the CUs or more by itself
-    assert group(1, 1024, 32, 8) == 2 and group(1, 512, 32, 7) == 4           # 4 + 3
-    assert group(4, 512, 5, 8) == 4                                           # six would fit; two launches of four
-    assert group(1, 256, 4, 4) == 4 and group(1, 16, 1, 64) == 16             # never more than an argument list holds
+    assert group(1, 16384, 32, 8) == group(1, 8193, 32, 8) == 1               # more than four rounds by itself
+    assert group(1, 8192, 32, 8) == 2 and group(1, 4096, 32, 8) == 4 and group(1, 2048, 32, 8) == 8
+    assert group(1, 4096, 32, 7) == 4 and group(1, 4096, 32, 5) == 3          # 4 + 3, 3 + 2
+    assert group(4, 512, 5, 8) == 8 and group(1, 256, 4, 4) == 4
+    assert group(1, 16, 1, 64) == 16                                          # what an argument list holds
     assert group(1, 256, 4, 1) == 1 and group(1, 0, 4, 8) == group(0, 64, 4, 8) == 1
     assert group(1, 64, 0, 8) < 0 and group(1, 64, 4, 0) < 0 and group(-1, 64, 4, 1) < 0
+
+
+def test_chunks_of_a_backward_step_share_a_launch():
+    group = N.lib().mhip_attn_bwd_group
+    assert group(1, 4096, 4096, 32, 32, 128, 8) == 1                          # 2048 workgroups by itself
+    assert group(4, 512, 512, 5, 5, 128, 8) == group(1, 512, 512, 8, 1, 128, 8) == 8
+    assert group(1, 1024, 1024, 32, 32, 128, 8) == 4                          # at most 2048 workgroups
+    assert group(1, 64, 64, 1, 1, 64, 40) == 14                               # of at most 16: three launches
+    assert group(1, 256, 256, 4, 4, 64, 1) == group(0, 64, 64, 4, 4, 64, 8) == group(1, 0, 64, 4, 4, 64, 8) == 1
+    assert group(1, 64, 64, 4, 3, 64, 8) < 0 and group(1, 64, 64, 4, 4, 136, 8) < 0 and group(1, 64, 64, 4, 4, 64, 0) < 0
