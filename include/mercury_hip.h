@@ -50,8 +50,9 @@ extern "C" {
  * 4: the backward's workspace also holds partial sums (it is larger than its three row arrays); mhip_attn_bwd_chunk.
  * 5: the workspace's size depends on B, Sq and Hq alone; mhip_attn_fwd_plan, mhip_attn_bwd_plan.
  * 6: mhip_attn_fwd_blocks, mhip_attn_fwd_group.
- * 7: mhip_attn_bwd_chunks, mhip_attn_bwd_group. */
-#define MHIP_ABI_VERSION 7
+ * 7: mhip_attn_bwd_chunks, mhip_attn_bwd_group.
+ * 8: mhip_attn_fwd_blocks takes the number of chunks of a result; mhip_attn_fwd_chain. */
+#define MHIP_ABI_VERSION 8
 int         mhip_abi_version(void);   /* the MHIP_ABI_VERSION the library was built with */
 int         mhip_version(void);
 /* Optional: per-device set-up the entry points otherwise do on their first call on a device (today: the address
@@ -89,12 +90,15 @@ int mhip_attn_fwd_block(const void* q, const void* k, const void* v, void* out, 
  * n blocks of one ring step in one launch: the same q against the n chunks ks[i], vs[i] (host arrays of device pointers,
  * one set of strides and one Sc for all), block i's results at out + i * o_sn (elements) and at lse + i * B * Hq * Sq.
  * Each block's results are those of mhip_attn_fwd_block, up to how a launch of this size splits its keys.
- * 1 <= n <= MHIP_MAX_GROUP.
+ * 1 <= n <= MHIP_MAX_GROUP.  With per > 1 a result stands for `per` consecutive chunks (the last one for what is left): attention
+ * over all of their keys, so there are ceil(n / per) of them; without a mask and with the same row stride in k and v
+ * (MHIP_EUNSUPPORTED otherwise).
  * mhip_attn_fwd_group: how many blocks of a step of `blocks` blocks to put into one launch when all of its chunks are there
  * (host function, launches nothing).
  */
 #define MHIP_MAX_GROUP 16
-int mhip_attn_fwd_blocks(const void* q, const void* const* ks, const void* const* vs, int n, void* out, int64_t o_sn, float* lse,
+int mhip_attn_fwd_blocks(const void* q, const void* const* ks, const void* const* vs, int n, int per, void* out, int64_t o_sn,
+                         float* lse,
                          int B, int Sq, int Sc, int Hq, int Hkv, int D,
                          int64_t q_sb, int64_t q_ss, int64_t q_sh,
                          int64_t k_sb, int64_t k_ss, int64_t k_sh,
@@ -104,6 +108,8 @@ int mhip_attn_fwd_blocks(const void* q, const void* const* ks, const void* const
                          const float* q_descale, const float* k_descale, const float* v_descale,
                          void* stream);
 int mhip_attn_fwd_group(int B, int Sq, int Hq, int blocks);
+/* How many chunks of a launch of n to put into one result (1 where separate results and their fold are expected to be faster). */
+int mhip_attn_fwd_chain(int B, int Sq, int Sc, int Hq, int D, int n, int dtype);
 
 /*
  * Block backward from the saved (final, merged) out and lse.

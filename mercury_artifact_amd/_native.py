@@ -19,7 +19,7 @@ import torch
 # MERCURY_HIP_LIB is a deployment option: the path of the built library when it is not kept next to the package.
 _BUILT = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB_PATH = os.environ.get("MERCURY_HIP_LIB") or os.path.join(_BUILT, "libmercury_hip.so")
-ABI_VERSION = 7      # MHIP_ABI_VERSION of include/mercury_hip.h the signatures below were written against
+ABI_VERSION = 8      # MHIP_ABI_VERSION of include/mercury_hip.h the signatures below were written against
 
 
 class _NoHost:
@@ -62,8 +62,9 @@ _SIGNATURES = {
     "mhip_init": (c_int, []),
     "mhip_error_string": (ctypes.c_char_p, [_I]),
     "mhip_attn_fwd_block": (c_int, [_P] * 5 + [_I] * 6 + [_L] * 12 + [_F, _I, _I, _P, _P, _P, _P]),
-    "mhip_attn_fwd_blocks": (c_int, [_P] * 3 + [_I, _P, _L, _P] + [_I] * 6 + [_L] * 12 + [_F, _I, _I, _P, _P, _P, _P]),
+    "mhip_attn_fwd_blocks": (c_int, [_P] * 3 + [_I, _I, _P, _L, _P] + [_I] * 6 + [_L] * 12 + [_F, _I, _I, _P, _P, _P, _P]),
     "mhip_attn_fwd_group": (c_int, [_I] * 4),
+    "mhip_attn_fwd_chain": (c_int, [_I] * 7),
     "mhip_attn_bwd_workspace_bytes": (c_int64, [_I] * 6),
     "mhip_attn_bwd_block": (c_int, [_P] * 10 + [_I] * 6 + [_L] * 15 + [_F, _I, _I, _P, _P]),
     "mhip_attn_bwd_block_noalloc": (c_int, [_P] * 10 + [_I] * 6 + [_L] * 15 + [_F, _I, _I, _P]),

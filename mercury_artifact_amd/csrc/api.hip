@@ -3,13 +3,15 @@
 #include "mhip_common.hpp"
 
 namespace mhip {
-int attn_fwd_bf16(const void* q, const void* const* ks, const void* const* vs, int blocks, void* out, int64_t o_sn, float* lse,
+int attn_fwd_bf16(const void* q, const void* const* ks, const void* const* vs, int n, int per, void* out, int64_t o_sn, float* lse,
                   int B, int Sq, int Sc, int Hq, int Hkv, int D,
                   const int64_t* strides, float scale, int mask, hipStream_t stream);
-int attn_fwd_fp8(const void* q, const void* const* ks, const void* const* vs, int blocks, void* out, int64_t o_sn, float* lse,
+int attn_fwd_fp8(const void* q, const void* const* ks, const void* const* vs, int n, int per, void* out, int64_t o_sn, float* lse,
                  int B, int Sq, int Sc, int Hq, int Hkv, int D, const int64_t* strides, float scale, int mask,
                  const float* q_descale, const float* k_descale, const float* v_descale, hipStream_t stream);
+int attn_fwd_bf16_chain(int n, int B, int Sq, int Sc, int Hq, int D);
 int attn_fwd_bf16_plan(int blocks, int B, int Sq, int Sc, int Hq, int D, int64_t k_ss, int64_t v_ss, int mask);
+int attn_fwd_fp8_chain(int n, int B, int Sq, int Sc, int Hq, int D);
 int attn_fwd_fp8_plan(int blocks, int B, int Sq, int Sc, int Hq, int mask);
 }  // namespace mhip
 
@@ -37,7 +39,7 @@ namespace {
 bool mult8(int64_t x) { return (x & 7) == 0; }
 }  // namespace
 
-extern "C" int mhip_attn_fwd_blocks(const void* q, const void* const* ks, const void* const* vs, int n, void* out, int64_t o_sn,
+extern "C" int mhip_attn_fwd_blocks(const void* q, const void* const* ks, const void* const* vs, int n, int per, void* out, int64_t o_sn,
                                     float* lse, int B, int Sq, int Sc, int Hq, int Hkv, int D,
                                     int64_t q_sb, int64_t q_ss, int64_t q_sh,
                                     int64_t k_sb, int64_t k_ss, int64_t k_sh,
@@ -46,7 +48,7 @@ extern "C" int mhip_attn_fwd_blocks(const void* q, const void* const* ks, const 
                                     float softmax_scale, int mask, int dtype,
                                     const float* q_descale, const float* k_descale, const float* v_descale,
                                     void* stream) {
-  if (n < 1 || n > kMaxGroup || !ks || !vs) return MHIP_EINVAL;
+  if (n < 1 || n > kMaxGroup || per < 1 || !ks || !vs) return MHIP_EINVAL;
   if (B < 0 || Sq < 0 || Sc < 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0) return MHIP_EINVAL;
   if (!(softmax_scale > 0.f) || !(softmax_scale < INFINITY)) return MHIP_EINVAL;
   if (mask != MHIP_MASK_NONE && mask != MHIP_MASK_CAUSAL) return MHIP_EINVAL;
@@ -79,10 +81,10 @@ extern "C" int mhip_attn_fwd_blocks(const void* q, const void* const* ks, const 
     if ((reinterpret_cast<uintptr_t>(q_descale) | reinterpret_cast<uintptr_t>(k_descale) |
          reinterpret_cast<uintptr_t>(v_descale)) & 3u)
       return MHIP_EALIGN;
-    return attn_fwd_fp8(q, ks, vs, n, out, o_sn, lse, B, Sq, Sc, Hq, Hkv, D, strides, softmax_scale, mask,
+    return attn_fwd_fp8(q, ks, vs, n, per, out, o_sn, lse, B, Sq, Sc, Hq, Hkv, D, strides, softmax_scale, mask,
                         q_descale, k_descale, v_descale, st);
   }
-  return attn_fwd_bf16(q, ks, vs, n, out, o_sn, lse, B, Sq, Sc, Hq, Hkv, D, strides, softmax_scale, mask, st);
+  return attn_fwd_bf16(q, ks, vs, n, per, out, o_sn, lse, B, Sq, Sc, Hq, Hkv, D, strides, softmax_scale, mask, st);
 }
 
 extern "C" int mhip_attn_fwd_block(const void* q, const void* k, const void* v, void* out, float* lse,
@@ -94,7 +96,7 @@ extern "C" int mhip_attn_fwd_block(const void* q, const void* k, const void* v, 
                                    float softmax_scale, int mask, int dtype,
                                    const float* q_descale, const float* k_descale, const float* v_descale,
                                    void* stream) {
-  return mhip_attn_fwd_blocks(q, &k, &v, 1, out, 0, lse, B, Sq, Sc, Hq, Hkv, D, q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, v_sb, v_ss, v_sh,
+  return mhip_attn_fwd_blocks(q, &k, &v, 1, 1, out, 0, lse, B, Sq, Sc, Hq, Hkv, D, q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, v_sb, v_ss, v_sh,
                               o_sb, o_ss, o_sh, softmax_scale, mask, dtype, q_descale, k_descale, v_descale, stream);
 }
 
@@ -113,6 +115,13 @@ extern "C" int mhip_attn_fwd_group(int B, int Sq, int Hq, int blocks) {
   if (most > kMaxGroup) most = kMaxGroup;
   const int launches = (blocks + most - 1) / most;
   return (blocks + launches - 1) / launches;
+}
+
+extern "C" int mhip_attn_fwd_chain(int B, int Sq, int Sc, int Hq, int D, int n, int dtype) {
+  if (B < 0 || Sq < 0 || Sc < 0 || Hq <= 0 || D <= 0 || D > 128 || n < 1) return MHIP_EINVAL;
+  if (dtype != MHIP_BF16 && dtype != MHIP_E4M3) return MHIP_EDTYPE;
+  if (n == 1 || n > kMaxGroup || B == 0 || Sq == 0) return 1;
+  return dtype == MHIP_E4M3 ? attn_fwd_fp8_chain(n, B, Sq, Sc, Hq, D) : attn_fwd_bf16_chain(n, B, Sq, Sc, Hq, D);
 }
 
 extern "C" int mhip_attn_fwd_plan(int B, int Sq, int Sc, int Hq, int D, int64_t k_ss, int64_t v_ss, int mask, int dtype) {

@@ -49,7 +49,7 @@ struct FwdParams {
   // what a workgroup needs before its first copy: read by one group of loads (see load_now)
   int per_xcd;       // ceil(total / 8)
   int total;         // blocks * B * Hq * nq_tiles
-  int blocks;        // blocks of the launch: the same q against as many chunks
+  int blocks;        // results of the launch: the same q against as many chunks, or runs of them
   int nq_tiles;      // ceil(Sq / rows per workgroup)
   int heads_per_xcd; // (block, batch, head) triples per XCD when they divide evenly, else 0
   int Sq, Sc;
@@ -60,6 +60,7 @@ struct FwdParams {
   int64_t q_sb, q_ss, q_sh, k_sb, k_ss, k_sh, v_sb, v_ss, v_sh;
   float scale, scale_log2;
   // the rest
+  int per, chunks;   // consecutive chunks of a result, chunks of the launch
   Divisor by_heads;  // by B * Hq
   int heads;         // B * Hq
   int B, Hq;
@@ -80,10 +81,15 @@ struct FwdParams {
 // (O, sum) of a row meet in LDS at the end.  Twice (four times) as many workgroups, each with half (a quarter) of the
 // serial chain; the price is as many times the L2 -> LDS traffic per row.  A key group has rings of two stages instead
 // of four, of 64-key tiles (KS = 2) or 32-key tiles (KS = 4): 128 KB of LDS in all three cases.
-template <bool CAUSAL, int KK = 8, int KS = 1>
+//
+// CHAIN: a workgroup visits p.per chunks one after the other, their tiles as one sequence: the ends of a workgroup's life
+// (arguments, Q, first tiles, O out) come once instead of once per chunk, and one result stands for all of them, which the
+// fold would otherwise write and read back as many times.
+template <bool CAUSAL, int KK = 8, int KS = 1, bool CHAIN = false>
 __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdParams p) {
   static_assert(KK == 8 || KK == 6 || KK == 4, "128, 96 or 64 on-chip head-dim columns");
   static_assert(KS == 1 || KS == 2 || KS == 4, "key groups");
+  static_assert(!CHAIN || (KS == 1 && !CAUSAL), "chunks are visited one after the other by workgroups of one key group");
   constexpr int DB = KK / 2;        // blocks of 32 head-dim values in O^T
   constexpr int RG = kWaves / KS;   // row groups of 32
   constexpr int kRows = 32 * RG;    // Q rows of the workgroup
@@ -118,11 +124,12 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
   // Several blocks of a step in one launch are so many times the (batch, head) pairs.  (The
   // first one's addresses come with the arguments above: a lone block does not wait for a second round of loads.)
   const uint16_t* kp = p.k0; const uint16_t* vp = p.v0;
-  int blk = 0;
+  int blk = 0, chunk = 0;
   if (p.blocks > 1) {
     blk = p.by_heads.quotient(bh, bh);
-    kp = p.k[blk];
-    vp = p.v[blk];
+    chunk = CHAIN ? blk * p.per : blk;
+    kp = p.k[chunk];
+    vp = p.v[chunk];
   }
   int hq;
   const int b = p.by_hq.quotient(bh, hq);
@@ -149,7 +156,12 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
     kv_end = lim < kv_end ? lim : kv_end;
     if (kv_end < 0) kv_end = 0;
   }
-  const int ntiles = (kv_end + BN * KS - 1) / (BN * KS);   // of each key group; tiles past the end are hidden whole
+  int ntiles = (kv_end + BN * KS - 1) / (BN * KS);   // of each key group; tiles past the end are hidden whole
+  int chunks_left = 0;                               // CHAIN: behind the first one
+  if (CHAIN) {
+    chunks_left = (p.chunks - chunk < p.per ? p.chunks - chunk : p.per) - 1;
+    ntiles *= chunks_left + 1;
+  }
 
   // ---- Q fragment: B operand of S^T = K Q^T, lane (ln, hf) holds Q[row][16 ks + 8 hf .. +7] -----
   const int my_q = q0 + rg * 32 + ln;
@@ -165,8 +177,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
   // when it is below 128: their lanes carry an offset that is out of range for every tile, so a tile in
   // LDS always has 128 columns, the upper ones zero, at no cost in memory traffic.
   auto swz = [](int row) { return lds_row_swizzle(row); };
-  const u32x4 krs = rsrc_words(kp + b * p.k_sb + hk * p.k_sh, (uint32_t)(((int64_t)(p.Sc - 1) * p.k_ss + p.D) * 2));
-  const u32x4 vrs = rsrc_words(vp + b * p.v_sb + hk * p.v_sh, (uint32_t)(((int64_t)(p.Sc - 1) * p.v_ss + p.D) * 2));
+  u32x4 krs = rsrc_words(kp + b * p.k_sb + hk * p.k_sh, (uint32_t)(((int64_t)(p.Sc - 1) * p.k_ss + p.D) * 2));
+  u32x4 vrs = rsrc_words(vp + b * p.v_sb + hk * p.v_sh, (uint32_t)(((int64_t)(p.Sc - 1) * p.v_ss + p.D) * 2));
   constexpr int kCpy = BN / RG / 4;                  // copy instructions per wavefront, tile and tensor (4 rows each)
   int kvoff[kCpy], vvoff[kCpy];
 #pragma unroll
@@ -188,16 +200,44 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
     const int tile = t * KS + kg;
     return tile * BN < p.Sc ? tile * tile_bytes : kNoTile;
   };
+  // CHAIN: K and V tiles are requested in order; k_off and v_off are the offsets of the next ones inside their chunks.  (The
+  // address of a chunk is loaded inside its branch and waited for there.)
+  const int chunk_bytes = CHAIN ? (int)((uint32_t)((p.Sc + BN - 1) / BN) * (uint32_t)k_tile_bytes) : 0;
+  int k_off = 0, v_off = 0, k_chunk = chunk, v_chunk = chunk;
+  const int last_chunk = chunk + chunks_left;
+  auto enter = [&](u32x4& rs, const uint16_t* base) {
+    asm volatile("" : "+s"(base));
+    rs[0] = (uint32_t)(uint64_t)base;
+    rs[1] = (uint32_t)((uint64_t)base >> 32) & 0xffffu;
+  };
+  auto chain_k = [&]() {                             // behind the copy of a K tile
+    k_off += k_tile_bytes;
+    if (k_off == chunk_bytes && k_chunk != last_chunk) {
+      k_off = 0;
+      ++k_chunk;
+      enter(krs, p.k[k_chunk] + b * p.k_sb + hk * p.k_sh);
+    }
+  };
+  auto chain_v = [&]() {
+    v_off += k_tile_bytes;
+    if (v_off == chunk_bytes && v_chunk != last_chunk) {
+      v_off = 0;
+      ++v_chunk;
+      enter(vrs, p.v[v_chunk] + b * p.v_sb + hk * p.v_sh);
+    }
+  };
   auto copy_k = [&](int t, int stage) {
-    const int soff = tile_offset(t, k_tile_bytes);
+    const int soff = CHAIN ? k_off : tile_offset(t, k_tile_bytes);
 #pragma unroll
     for (int u = 0; u < kCpy; ++u) copy16_to_lds(krs, lds_base + stage * kTile + u * 1024, kvoff[u], soff);
+    if (CHAIN) chain_k();
   };
   auto copy_v = [&](int t, int stage) {
-    const int soff = tile_offset(t, v_tile_bytes);
+    const int soff = CHAIN ? v_off : tile_offset(t, v_tile_bytes);
 #pragma unroll
     for (int u = 0; u < kCpy; ++u)
       copy16_to_lds(vrs, lds_base + kVBase + stage * kTile + u * 1024, vvoff[u], soff);
+    if (CHAIN) chain_v();
   };
 
   // K operand of S^T (A, 32 keys x 16 head-dim values): lane (ln, hf) reads chunk 2 kk + hf of row
@@ -278,8 +318,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
   };
 
   // keys past the chunk end and the causal diagonal -> -inf
+  int chain_kv0 = 0;                                        // first key of the next tile inside its chunk
   auto sm_mask = [&](int t) {
-    const int kv0 = (t * KS + kg) * BN;
+    const int kv0 = CHAIN ? chain_kv0 : (t * KS + kg) * BN;
+    if (CHAIN) chain_kv0 = kv0 + BN < p.Sc ? kv0 + BN : 0;
     bool need_mask = kv0 + BN > p.Sc;
     if (CAUSAL) need_mask = need_mask || (kv0 + BN - 1 > q0 + causal_shift);
     if (need_mask) {
@@ -289,8 +331,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
       for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-          const int key = kv0 + mb * 32 + (j >> 2) * 8 + hf * 4 + (j & 3);
-          if (key > lim) s[mb][j] = -INFINITY;
+          const int at = mb * 32 + (j >> 2) * 8 + (j & 3);
+          if (CHAIN ? at + hf * 4 > lim - kv0 : kv0 + at + hf * 4 > lim) s[mb][j] = -INFINITY;
         }
     }
   };
@@ -397,8 +439,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
       // instead of 43.9 at D 96, 4096 x 4096 H32 131.6 / 145.4 and 174.7 / 182.8; on 128 columns it is 1 % slower.
       if (kShortMatrix && i < kSlotsS && i % (kSlotsS / 4) == 1) {
         const int u = i / (kSlotsS / 4);
-        if (u < 2) copy16_to_lds(krs, lds_base + (t & 3) * kTile + u * 1024, kvoff[u % kCpy], tile_offset(t + 4, k_tile_bytes));
-        else copy16_to_lds(vrs, lds_base + kVBase + ((t + 3) & 3) * kTile + (u - 2) * 1024, vvoff[u % kCpy], tile_offset(t + 3, v_tile_bytes));
+        if (u < 2) copy16_to_lds(krs, lds_base + (t & 3) * kTile + u * 1024, kvoff[u % kCpy], CHAIN ? k_off : tile_offset(t + 4, k_tile_bytes));
+        else copy16_to_lds(vrs, lds_base + kVBase + ((t + 3) & 3) * kTile + (u - 2) * 1024, vvoff[u % kCpy], CHAIN ? v_off : tile_offset(t + 3, v_tile_bytes));
       }
       // S^T(t+1) is complete after its last slot; its softmax starts here, in the shadow of the O^T MFMAs
       if (i == kSlotsS) sm_mask(t + 1);
@@ -479,6 +521,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
       if (!kShortMatrix) {
         copy_k(t + 4, t & 3);
         copy_v(t + 3, (t + 3) & 3);
+      } else if (CHAIN) {
+        chain_k();
+        chain_v();
       }
       if (t + 2 < ntiles) first_frags();                        // K(t+2), for the next matrix phase
       asm volatile("s_waitcnt vmcnt(4)" ::: "memory");          // the four copies of one tile ago are done
@@ -653,6 +698,16 @@ void launch_one(FwdParams& p, hipStream_t stream) {
   hipLaunchKernelGGL((attn_fwd_bf16_d128<CAUSAL, KK, KS>), dim3(p.per_xcd * 8), dim3(kWaves * 64), 0, stream, p);
 }
 template <int KK>
+void launch_chain(FwdParams& p, hipStream_t stream) {
+  p.nq_tiles = (p.Sq + kBM - 1) / kBM;
+  p.total = p.blocks * p.heads * p.nq_tiles;
+  p.per_xcd = (p.total + 7) / 8;
+  p.heads_per_xcd = 0;
+  p.by_q_tiles = Divisor(p.nq_tiles);
+  p.by_order = Divisor(1);
+  hipLaunchKernelGGL((attn_fwd_bf16_d128<false, KK, 1, true>), dim3(p.per_xcd * 8), dim3(kWaves * 64), 0, stream, p);
+}
+template <int KK>
 void launch_fwd(FwdParams& p, bool causal, int groups, hipStream_t stream) {
   if (causal) {
     if (groups == 4) launch_one<true, KK, 4>(p, stream);
@@ -674,13 +729,15 @@ void launch_fwd(FwdParams& p, bool causal, int groups, hipStream_t stream) {
 //     B1 H1  4096 x 4096    70.3 / 45.6 / 33.8      B1 H20 4096 x 4096     187 /  176 /  200
 //     B1 H32 4096 x 4096     228 /  255 /  357      B2 H12 1500 x 1500    24.2 / 18.5 / 24.6  (D 64, causal)
 // The split kernel puts whole tiles out of range through 32-bit offsets, which asks for spans below 2^30 bytes.
-int key_groups(const FwdParams& p, bool causal) {
+const LaunchCost* costs(int D) {
+  static constexpr LaunchCost kCost128[3] = {{7.0f, 1.10f, 0.80f}, {6.5f, 1.19f, 0.90f}, {5.2f, 0.81f, 0.49f}};
+  static constexpr LaunchCost kCost96[3] = {{6.5f, 0.62f, 0.66f}, {6.2f, 1.08f, 0.58f}, {4.9f, 0.76f, 0.30f}};
+  static constexpr LaunchCost kCost64[3] = {{6.0f, 0.65f, 0.30f}, {6.0f, 0.98f, 0.27f}, {4.7f, 0.72f, 0.12f}};
+  return D <= 64 ? kCost64 : D <= 96 ? kCost96 : kCost128;
+}
+int key_groups(const FwdParams& p, bool causal, float* time_of_best = nullptr) {
   if ((int64_t)p.Sc * p.k_ss >= (1 << 29) || (int64_t)p.Sc * p.v_ss >= (1 << 29)) return 1;
-  struct Cost { float fixed, step, busy; };
-  static constexpr Cost kCost128[3] = {{7.0f, 1.10f, 0.80f}, {6.5f, 1.19f, 0.90f}, {5.2f, 0.81f, 0.49f}};
-  static constexpr Cost kCost96[3] = {{6.5f, 0.62f, 0.66f}, {6.2f, 1.08f, 0.58f}, {4.9f, 0.76f, 0.30f}};
-  static constexpr Cost kCost64[3] = {{6.0f, 0.65f, 0.30f}, {6.0f, 0.98f, 0.27f}, {4.7f, 0.72f, 0.12f}};
-  const Cost* cost = p.D <= 64 ? kCost64 : p.D <= 96 ? kCost96 : kCost128;
+  const LaunchCost* cost = costs(p.D);
   int best = 1;
   float best_time = 0.f;
   for (int i = 0; i < 3; ++i) {
@@ -691,9 +748,7 @@ int key_groups(const FwdParams& p, bool causal) {
     auto steps = [&](int64_t keys) { return (float)((keys + tile * groups - 1) / (tile * groups)); };
     float time;
     if (!causal) {
-      const float full = floorf(n / 256.f), part = n / 256.f - full, t = steps(p.Sc);
-      time = full * (cost[i].fixed + t * (cost[i].step + cost[i].busy));
-      if (part > 0.f) time += cost[i].fixed + t * (cost[i].step + part * cost[i].busy);
+      time = rounds_time(n, steps(p.Sc), cost[i]);
     } else {
       // longest tiles first: the longest workgroup, or all of the work spread over the CUs
       const int64_t shift = (int64_t)p.Sc - p.Sq;
@@ -709,6 +764,7 @@ int key_groups(const FwdParams& p, bool causal) {
     }
     if (i == 0 || time < best_time) { best = groups; best_time = time; }
   }
+  if (time_of_best) *time_of_best = best_time;
   return best;
 }
 
@@ -722,17 +778,47 @@ int attn_fwd_bf16_plan(int blocks, int B, int Sq, int Sc, int Hq, int D, int64_t
   return key_groups(p, mask == MHIP_MASK_CAUSAL);
 }
 
-int attn_fwd_bf16(const void* q, const void* const* ks, const void* const* vs, int blocks, void* out, int64_t o_sn, float* lse,
+// Chunks of a result (1, or how many a workgroup visits one after the other) of a launch of n chunks: the count with the least
+// estimated time, the fold of the results included (which is nothing where there is only one).  Where the blocks would all
+// run side by side a run of chunks would only make the longest chain longer.  Whole steps of 8 chunks, us, one / two / four /
+// eight chunks to a result: 512 x 512 B4 H5 43.9 / 36.0 / 49.7 / 76.1, 1024 x 1024 H32 148 / 133 / 128 / 154, 2048 x 2048 H32
+// 488 / 471 / 464 / 441, 4096 x 4096 H32 1790 / 1772 / 1761 / 1720, 1237 x 1237 B2 H16/8 D80 161 / 173 / 210 / 172, 700 x 700 H12
+// D64 40.0 / 32.7 / 51.8 / 87.4, 3000 x 3000 H16 D96 414 / 423 / 475 / 440.
+int attn_fwd_bf16_chain(int n, int B, int Sq, int Sc, int Hq, int D) {
+  if (n < 2 || Sc == 0) return 1;
+  FwdParams p{};
+  p.blocks = n; p.B = B; p.Sq = Sq; p.Sc = Sc; p.Hq = Hq; p.D = D;
+  const float wgs = (float)B * Hq * ((Sq + kBM - 1) / kBM);
+  if (wgs * n <= 256.f) return 1;
+  int best = 1;
+  float best_time;
+  key_groups(p, false, &best_time);
+  best_time += fold_time(n, B, Sq, Hq, D);
+  for (int results = n; results >= 1; --results) {
+    const int per = (n + results - 1) / results;
+    if (per == 1 || (n + per - 1) / per != results) continue;
+    // (a chain's tiles take a little longer: its launch has no pauses in which the clock recovers)
+    LaunchCost c = costs(D)[0];
+    c.step *= D > 96 ? 1.05f : 1.08f;
+    c.busy *= D > 96 ? 1.05f : 1.08f;
+    const float time = rounds_time(wgs * results, (float)per * ((Sc + kBN - 1) / kBN), c) + fold_time(results, B, Sq, Hq, D);
+    if (time < best_time) { best_time = time; best = per; }
+  }
+  return best;
+}
+
+int attn_fwd_bf16(const void* q, const void* const* ks, const void* const* vs, int n, int per, void* out, int64_t o_sn, float* lse,
                   int B, int Sq, int Sc, int Hq, int Hkv, int D,
                   const int64_t* st, float scale, int mask, hipStream_t stream) {
   FwdParams p;
   p.q = static_cast<const uint16_t*>(q);
   for (int i = 0; i < kMaxGroup; ++i) {
-    p.k[i] = i < blocks ? static_cast<const uint16_t*>(ks[i]) : nullptr;
-    p.v[i] = i < blocks ? static_cast<const uint16_t*>(vs[i]) : nullptr;
+    p.k[i] = i < n ? static_cast<const uint16_t*>(ks[i]) : nullptr;
+    p.v[i] = i < n ? static_cast<const uint16_t*>(vs[i]) : nullptr;
   }
   p.k0 = p.k[0]; p.v0 = p.v[0];
-  p.blocks = blocks; p.heads = B * Hq;
+  p.per = per; p.chunks = n;
+  p.blocks = (n + per - 1) / per; p.heads = B * Hq;
   p.o_sn = o_sn; p.l_sn = (int64_t)B * Hq * Sq;
   p.out = static_cast<uint16_t*>(out);
   p.lse = lse;
@@ -746,6 +832,13 @@ int attn_fwd_bf16(const void* q, const void* const* ks, const void* const* vs, i
   p.scale = scale;
   p.scale_log2 = scale * kLog2e;
   const bool causal = mask == MHIP_MASK_CAUSAL;
+  if (per > 1) {
+    if (causal || Sc == 0 || p.k_ss != p.v_ss) return MHIP_EUNSUPPORTED;
+    if (D <= 64) launch_chain<4>(p, stream);
+    else if (D <= 96) launch_chain<6>(p, stream);
+    else launch_chain<8>(p, stream);
+    return launch_status();
+  }
   const int groups = key_groups(p, causal);
   if (D <= 64) launch_fwd<4>(p, causal, groups, stream);        // half the on-chip columns, half the MFMAs
   else if (D <= 96) launch_fwd<6>(p, causal, groups, stream);   // three quarters of both

@@ -55,6 +55,7 @@ struct Fp8Params {
   const float* q_descale; const float* k_descale; const float* v_descale;   // device scalars, NULL = 1
   float scale;       // softmax scale
   // the rest
+  int per, chunks;   // as in the bf16 kernel: consecutive chunks of a result, chunks of the launch
   Divisor by_heads;  // by B * Hq
   int heads;         // B * Hq
   int B, Hq;
@@ -78,7 +79,9 @@ __device__ __forceinline__ constexpr int swz8(int row) { return (((row >> 1) & 3
 // CUs without a workgroup.  A wavefront with a SIMD to itself takes less time for a tile than two that share one
 // (four / eight): 2048 x 2048 H16 24.2 / 32.4 us, 4096 x 4096 H2 39.8 / 56.9, causal 1024 x 1024 H32/8 15.5 / 21.3; results
 // the same.
-template <bool CAUSAL, int DB, int WAVES>
+//
+// CHAIN: a workgroup visits p.per chunks one after the other, as in the bf16 kernel.
+template <bool CAUSAL, int DB, int WAVES, bool CHAIN = false>
 __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const Fp8Params p) {
   static_assert(WAVES == 8 || WAVES == 4, "two wavefronts per SIMD or one");
   constexpr int kBM = WAVES * 32;
@@ -114,11 +117,12 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
   // Several blocks of a step in one launch are so many times the (batch, head) pairs.  (The
   // first one's addresses come with the arguments above: a lone block does not wait for a second round of loads.)
   const uint8_t* kp = p.k0; const uint8_t* vp = p.v0;
-  int blk = 0;
+  int blk = 0, chunk = 0;
   if (p.blocks > 1) {
     blk = p.by_heads.quotient(bh, bh);
-    kp = p.k[blk];
-    vp = p.v[blk];
+    chunk = CHAIN ? blk * p.per : blk;
+    kp = p.k[chunk];
+    vp = p.v[chunk];
   }
   int hq;
   const int b = p.by_hq.quotient(bh, hq);
@@ -137,7 +141,12 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
     kv_end = lim < kv_end ? lim : kv_end;
     if (kv_end < 0) kv_end = 0;
   }
-  const int ntiles = (kv_end + kBN - 1) / kBN;
+  int ntiles = (kv_end + kBN - 1) / kBN;
+  int chunks_left = 0;                          // CHAIN: behind the first one
+  if (CHAIN) {
+    chunks_left = (p.chunks - chunk < p.per ? p.chunks - chunk : p.per) - 1;
+    ntiles *= chunks_left + 1;
+  }
 
   // ---- Q fragment: B operand of S^T, lane (ln, hf) holds bytes [64 ks + 32 hf, +32) of its row ------------
   const int my_q = q0 + wave * 32 + ln;
@@ -148,8 +157,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
   // fetches the chunk that lives there.  Rows past the end of the chunk arrive as zeros. ---------------------
   // Chunks past the head dimension (D < 128) carry an offset that is out of range for every tile and arrive as
   // zeros too: a tile in LDS always has 128 columns, at no cost in memory traffic.
-  const u32x4 krs = rsrc_words(kp + b * p.k_sb + hk * p.k_sh, (uint32_t)((int64_t)(p.Sc - 1) * p.k_ss + p.D));
-  const u32x4 vrs = rsrc_words(vp + b * p.v_sb + hk * p.v_sh, (uint32_t)((int64_t)(p.Sc - 1) * p.v_ss + p.D));
+  u32x4 krs = rsrc_words(kp + b * p.k_sb + hk * p.k_sh, (uint32_t)((int64_t)(p.Sc - 1) * p.k_ss + p.D));
+  u32x4 vrs = rsrc_words(vp + b * p.v_sb + hk * p.v_sh, (uint32_t)((int64_t)(p.Sc - 1) * p.v_ss + p.D));
   int kvoff[kCpy], vvoff[kCpy];
 #pragma unroll
   for (int u = 0; u < kCpy; ++u) {
@@ -162,8 +171,40 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
   const int k_tile_bytes = (int)(kBN * p.k_ss);
   const int v_tile_bytes = (int)(kBN * p.v_ss);
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem + wave * (kCpy * 1024);
-  auto copy_k = [&](int u, int t) { copy16_to_lds(krs, lds_base + (t & 3) * kTileBytes + u * 1024, kvoff[u], t * k_tile_bytes); };
-  auto copy_v = [&](int u, int t) { copy16_to_lds(vrs, lds_base + kVBase + (t & 3) * kTileBytes + u * 1024, vvoff[u], t * v_tile_bytes); };
+  // CHAIN: K and V tiles are requested in order; k_off and v_off are the offsets of the next ones inside their chunks.  (The
+  // address of a chunk is loaded inside its branch and waited for there.)
+  const int chunk_bytes = CHAIN ? (int)((uint32_t)((p.Sc + kBN - 1) / kBN) * (uint32_t)k_tile_bytes) : 0;
+  int k_off = 0, v_off = 0, k_chunk = chunk, v_chunk = chunk;
+  const int last_chunk = chunk + chunks_left;
+  auto enter = [&](u32x4& rs, const uint8_t* base) {
+    asm volatile("" : "+s"(base));
+    rs[0] = (uint32_t)(uint64_t)base;
+    rs[1] = (uint32_t)((uint64_t)base >> 32) & 0xffffu;
+  };
+  auto copy_k = [&](int u, int t) {
+    copy16_to_lds(krs, lds_base + (t & 3) * kTileBytes + u * 1024, kvoff[u], CHAIN ? k_off : t * k_tile_bytes);
+  };
+  auto copy_v = [&](int u, int t) {
+    copy16_to_lds(vrs, lds_base + kVBase + (t & 3) * kTileBytes + u * 1024, vvoff[u], CHAIN ? v_off : t * v_tile_bytes);
+  };
+  auto chain_k = [&]() {                        // behind the copies of a K tile
+    if (!CHAIN) return;
+    k_off += k_tile_bytes;
+    if (k_off == chunk_bytes && k_chunk != last_chunk) {
+      k_off = 0;
+      ++k_chunk;
+      enter(krs, p.k[k_chunk] + b * p.k_sb + hk * p.k_sh);
+    }
+  };
+  auto chain_v = [&]() {
+    if (!CHAIN) return;
+    v_off += k_tile_bytes;
+    if (v_off == chunk_bytes && v_chunk != last_chunk) {
+      v_off = 0;
+      ++v_chunk;
+      enter(vrs, p.v[v_chunk] + b * p.v_sb + hk * p.v_sh);
+    }
+  };
 
   // K operand of S^T: MFMA row m of block mb is key 32 mb + pi(m), pi(8 g + 4 h + e) = 16 h + 4 g + e, so
   // that accumulator register i of lane half hf is key 32 mb + 16 hf + i.  The lane reads chunks
@@ -284,13 +325,13 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
     if (need_mask) {
       int lim = p.Sc - 1;
       if (CAUSAL) { const int c = my_q + causal_shift; lim = c < lim ? c : lim; }
+      int rest = lim - kv0 - hf * 16;              // CHAIN: one register to compare constants with (32 would count along
+      if (CHAIN) asm volatile("" : "+v"(rest));    // with the position in a chunk)
 #pragma unroll
       for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const int key = kv0 + mb * 32 + hf * 16 + j;
-          if (key > lim) s[mb][j] = -INFINITY;
-        }
+        for (int j = 0; j < 16; ++j)
+          if (CHAIN ? mb * 32 + j > rest : kv0 + mb * 32 + hf * 16 + j > lim) s[mb][j] = -INFINITY;
     }
   };
   // after a half's last vector step: move the reference and repeat if a sum reached the trigger (or is inf / NaN)
@@ -326,8 +367,10 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
   auto o_mfma = [&](int db, const i32x8& a, const i32x8& pw) {
     o_acc[db] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, pw, o_acc[db], 0, 0, 0, 0, 0, 0);
   };
+  int chain_kv0 = 0;                              // CHAIN: first key of the tile inside its chunk
   auto phase = [&](int half, int t, f32x16 (&cur)[2], f32x16 (&next)[2], const i32x8& p_before, i32x8& p_cur) {
-    mask_half(cur, t * kBN + half * (kBN / 2));
+    mask_half(cur, (CHAIN ? chain_kv0 : t * kBN) + half * (kBN / 2));
+    if (CHAIN && half == 1) chain_kv0 = chain_kv0 + kBN < p.Sc ? chain_kv0 + kBN : 0;
 #pragma unroll
     for (int i = 0; i < kSlots; ++i) {
       i32x8& operand = ring[(half * kSlots + i) & 1];
@@ -358,19 +401,28 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
     }
     vector_step(8, cur, p_cur);
     finish_half(cur, p_cur);
+    if (half == 0) {                              // (a branch between the MFMAs would cost 60 registers)
+      chain_k();
+      chain_v();
+    }
   };
 
   if (ntiles > 0) {
 #pragma unroll
     for (int u = 0; u < kCpy; ++u) copy_k(u, 0);
+    chain_k();
 #pragma unroll
     for (int u = 0; u < kCpy; ++u) copy_v(u, 0);
+    chain_v();
 #pragma unroll
     for (int u = 0; u < kCpy; ++u) copy_k(u, 1);
+    chain_k();
 #pragma unroll
     for (int u = 0; u < kCpy; ++u) copy_k(u, 2);
+    chain_k();
 #pragma unroll
     for (int u = 0; u < kCpy; ++u) copy_v(u, 1);
+    chain_v();
     const int row = my_q < p.Sq ? my_q : p.Sq - 1;
     const uint8_t* qp = p.q + b * p.q_sb + (int64_t)row * p.q_ss + hq * p.q_sh + hf * 32;
 #pragma unroll
@@ -398,9 +450,33 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
     ring[0] = read_slot(0, 0);
     ring[1] = read_slot(0, 1);
   }
+  // CHAIN: where a chunk begins the reference becomes the maximum of its first tile, up or down, as if the chunk had a
+  // workgroup of its own: P is rounded relative to it.  The half whose P is still due goes into O first.
+  auto enter_chunk = [&]() {
+#pragma unroll
+    for (int db = 0; db < DB; ++db) o_mfma(db, read_v(db, 1), pb);
+    pb = i32x8{};
+#pragma unroll
+    for (int i = 0; i < kSlotsS; ++i) s_mfma(i, read_k(2 + (i & 1), i >> 1), sb);    // phase 0 computes it again
+    mask_half(sa, chain_kv0);
+    mask_half(sb, chain_kv0 + kBN / 2);
+    const float mx = pair_max(fmaxf(largest(sa), largest(sb)));
+    // (down by 2^60 at most: beyond that the chunk adds nothing, and O has to stay finite)
+    const float grown = (mx - m_ref) * scale_log2;
+    const bool move = mx != -INFINITY && grown > -60.f;               // false for NaN
+    const float alpha = move ? fast_exp2(-grown) : 1.f;
+    l_run *= alpha;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) o_acc[db][j] *= alpha;
+    m_ref = move ? mx : m_ref;
+    msc = m_ref * scale_log2 - kPShift;
+  };
   for (int t = 0; t < ntiles; ++t) {
     asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * kCpy) : "memory");
     __builtin_amdgcn_s_barrier();
+    if (CHAIN && chain_kv0 == 0 && t > 0) enter_chunk();
     phase(0, t, sa, sb, pb, pa);
     phase(1, t, sb, sa, pa, pb);
   }
@@ -447,7 +523,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
 template <int DB, int WAVES>
 void launch_fp8(const Fp8Params& p, bool causal, hipStream_t stream) {
   const dim3 grid(p.per_xcd * 8), block(WAVES * 64);
-  if (causal) hipLaunchKernelGGL((attn_fwd_fp8_d128<true, DB, WAVES>), grid, block, 0, stream, p);
+  if (p.per > 1) hipLaunchKernelGGL((attn_fwd_fp8_d128<false, DB, WAVES, true>), grid, block, 0, stream, p);
+  else if (causal) hipLaunchKernelGGL((attn_fwd_fp8_d128<true, DB, WAVES>), grid, block, 0, stream, p);
   else hipLaunchKernelGGL((attn_fwd_fp8_d128<false, DB, WAVES>), grid, block, 0, stream, p);
 }
 
@@ -462,16 +539,41 @@ int attn_fwd_fp8_plan(int blocks, int B, int Sq, int Sc, int Hq, int mask) {
   return (int64_t)blocks * B * Hq * ((Sq + 127) / 128) > (mask == MHIP_MASK_CAUSAL && Sc <= Sq ? 512 : 256) ? 8 : 4;
 }
 
-int attn_fwd_fp8(const void* q, const void* const* ks, const void* const* vs, int blocks, void* out, int64_t o_sn, float* lse,
+// Chunks of a result of a launch of n chunks, as for the bf16 kernels.  Costs of workgroups of eight and of four
+// wavefronts, fitted to the launches above and 4096 x 4096 H32 at 64, 96 and 128 columns.  Whole steps of 8 chunks, us, one / two /
+// four / eight chunks to a result: 1024 x 1024 H32 114 / 94.3 / 89.8 / 92.4, 4096 x 4096 H32 1146 / 1102 / 1094 / 1060.
+int attn_fwd_fp8_chain(int n, int B, int Sq, int Sc, int Hq, int D) {
+  if (n < 2 || Sc == 0 || (float)n * B * Hq * ((Sq + 255) / 256) <= 256.f) return 1;
+  const LaunchCost eight = {6.5f, D <= 64 ? 1.1f : D <= 96 ? 1.45f : 1.55f, D <= 64 ? 0.3f : 0.4f};
+  const LaunchCost four = {6.f, D <= 64 ? 0.8f : 1.f, 0.07f};
+  auto time = [&](int results, int per) {
+    const bool wide = attn_fwd_fp8_plan(results, B, Sq, Sc, Hq, MHIP_MASK_NONE) == 8;
+    const float wgs = (float)results * B * Hq * (wide ? (Sq + 255) / 256 : (Sq + 127) / 128);
+    return rounds_time(wgs, (float)per * ((Sc + kBN - 1) / kBN), wide ? eight : four) + fold_time(results, B, Sq, Hq, D);
+  };
+  int best = 1;
+  float best_time = time(n, 1);
+  for (int results = n; results >= 1; --results) {
+    const int per = (n + results - 1) / results;
+    if (per == 1 || (n + per - 1) / per != results) continue;
+    const float t = time(results, per);
+    if (t < best_time) { best_time = t; best = per; }
+  }
+  return best;
+}
+
+int attn_fwd_fp8(const void* q, const void* const* ks, const void* const* vs, int n, int per, void* out, int64_t o_sn, float* lse,
                  int B, int Sq, int Sc, int Hq, int Hkv, int D, const int64_t* st, float scale, int mask,
                  const float* q_descale, const float* k_descale, const float* v_descale, hipStream_t stream) {
   Fp8Params p;
   p.q = static_cast<const uint8_t*>(q);
   for (int i = 0; i < kMaxGroup; ++i) {
-    p.k[i] = i < blocks ? static_cast<const uint8_t*>(ks[i]) : nullptr;
-    p.v[i] = i < blocks ? static_cast<const uint8_t*>(vs[i]) : nullptr;
+    p.k[i] = i < n ? static_cast<const uint8_t*>(ks[i]) : nullptr;
+    p.v[i] = i < n ? static_cast<const uint8_t*>(vs[i]) : nullptr;
   }
   p.k0 = p.k[0]; p.v0 = p.v[0];
+  const int blocks = (n + per - 1) / per;
+  p.per = per; p.chunks = n;
   p.blocks = blocks; p.heads = B * Hq;
   p.o_sn = o_sn; p.l_sn = (int64_t)B * Hq * Sq;
   p.out = static_cast<uint16_t*>(out); p.lse = lse;
@@ -485,6 +587,7 @@ int attn_fwd_fp8(const void* q, const void* const* ks, const void* const* vs, in
   p.scale = scale;
   p.q_descale = q_descale; p.k_descale = k_descale; p.v_descale = v_descale;
   const bool causal = mask == MHIP_MASK_CAUSAL;
+  if (per > 1 && (causal || Sc == 0 || p.k_ss != p.v_ss)) return MHIP_EUNSUPPORTED;
   const bool wide = attn_fwd_fp8_plan(blocks, B, Sq, Sc, Hq, mask) == 8;
   const int rows = wide ? 256 : 128;
   p.nq_tiles = (Sq + rows - 1) / rows;

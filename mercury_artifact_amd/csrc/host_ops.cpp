@@ -28,6 +28,7 @@ struct Entry {
   decltype(&mhip_attn_fwd_block) fwd = nullptr;
   decltype(&mhip_attn_fwd_blocks) fwd_many = nullptr;
   decltype(&mhip_attn_fwd_group) fwd_group = nullptr;
+  decltype(&mhip_attn_fwd_chain) fwd_chain = nullptr;
   decltype(&mhip_attn_bwd_workspace_bytes) bwd_bytes = nullptr;
   decltype(&mhip_attn_bwd_block) bwd = nullptr;
   decltype(&mhip_attn_bwd_chunk) chunk = nullptr;
@@ -268,15 +269,34 @@ PyObject* fwd_group(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// (q, chunks, softmax_scale, causal, q_descale, k_descale, v_descale, outs, lses, first): the blocks of q against every
-// (2, B, Sc, Hkv, D) tensor of the list in one launch, their results into outs[first:] and lses[first:] -> True
+// (q, chunk, n): how many of n chunks to put into one result
+PyObject* fwd_chain(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ENTER(3);
+  const Tensor *q = plain(a[0]), *c = plain(a[1]);
+  const long n = PyLong_AsLong(a[2]);
+  if (n == -1 && PyErr_Occurred()) { PyErr_Clear(); SLOW; }
+  if (!q || !c || q->dim() != 4 || c->dim() != 5 || q->size(2) == 0 ||
+      !fits({q->size(0), q->size(1), q->size(2), q->size(3), c->size(2), n}))
+    SLOW;
+  const auto type = q->scalar_type();
+  if (type != at::kBFloat16 && type != at::kFloat8_e4m3fn) SLOW;
+  const int per = entry.fwd_chain(q->size(0), q->size(1), c->size(2), q->size(2), q->size(3), n > MHIP_MAX_GROUP ? MHIP_MAX_GROUP : n,
+                                  type == at::kBFloat16 ? MHIP_BF16 : MHIP_E4M3);
+  if (per < 1) SLOW;
+  return PyLong_FromLong(per);
+  END_HANDLE_TH_ERRORS
+}
+
+// (q, chunks, per, softmax_scale, causal, q_descale, k_descale, v_descale, outs, lses, first): the blocks of q against every
+// (2, B, Sc, Hkv, D) tensor of the list in one launch, a result per `per` of them, into outs[first:] and lses[first:] -> True
 PyObject* fwd_blocks(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  ENTER(10);
+  ENTER(11);
   if (!PyList_CheckExact(a[1])) SLOW;
   const Py_ssize_t n = PyList_GET_SIZE(a[1]);
   if (n < 1 || n > MHIP_MAX_GROUP) SLOW;
-  const Tensor *q = plain(a[0]), *c0 = plain(PyList_GET_ITEM(a[1], 0)), *outs = plain(a[7]), *lses = plain(a[8]);
+  const Tensor *q = plain(a[0]), *c0 = plain(PyList_GET_ITEM(a[1], 0)), *outs = plain(a[8]), *lses = plain(a[9]);
   if (!q || !c0 || !outs || !lses || q->dim() != 4 || c0->dim() != 5) SLOW;
   const int64_t B = q->size(0), Sq = q->size(1), Hq = q->size(2), D = q->size(3), Sc = c0->size(2), Hkv = c0->size(3);
   const auto type = q->scalar_type();
@@ -292,24 +312,26 @@ PyObject* fwd_blocks(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     ks[i] = c->data_ptr();
     vs[i] = static_cast<const char*>(ks[i]) + c->stride(0) * c->element_size();
   }
-  const double scale = PyFloat_AsDouble(a[2]);
+  const double scale = PyFloat_AsDouble(a[3]);
   if (scale == -1.0 && PyErr_Occurred()) { PyErr_Clear(); SLOW; }
-  const int causal = PyObject_IsTrue(a[3]);
-  const long first = PyLong_AsLong(a[9]);
-  if (causal < 0 || (first == -1 && PyErr_Occurred())) { PyErr_Clear(); SLOW; }
+  const int causal = PyObject_IsTrue(a[4]);
+  const long first = PyLong_AsLong(a[10]), per = PyLong_AsLong(a[2]);
+  if (causal < 0 || ((first == -1 || per == -1) && PyErr_Occurred())) { PyErr_Clear(); SLOW; }
+  if (per < 1 || per > MHIP_MAX_GROUP) SLOW;
+  const Py_ssize_t results = (n + per - 1) / per;
   const Tensor* descale[3];
   for (int i = 0; i < 3; ++i) {
-    if (!optional(a[4 + i], *q, descale[i])) SLOW;
+    if (!optional(a[5 + i], *q, descale[i])) SLOW;
     if (descale[i] && (descale[i]->numel() != 1 || descale[i]->scalar_type() != at::kFloat)) SLOW;
   }
-  if (outs->dim() != 5 || lses->dim() != 4 || first < 0 || first + n > outs->size(0) || first + n > lses->size(0) ||
+  if (outs->dim() != 5 || lses->dim() != 4 || first < 0 || first + results > outs->size(0) || first + results > lses->size(0) ||
       outs->sizes().slice(1) != q->sizes() || lses->size(1) != B || lses->size(2) != Hq || lses->size(3) != Sq ||
       outs->scalar_type() != at::kBFloat16 || lses->scalar_type() != at::kFloat || outs->stride(4) != 1 || !lses->is_contiguous())
     SLOW;
   OnDevice on(*q);
   if (!on.current) SLOW;
   const int code = without_gil([&] {
-    return entry.fwd_many(q->data_ptr(), ks, vs, (int)n, static_cast<char*>(outs->data_ptr()) + 2 * first * outs->stride(0),
+    return entry.fwd_many(q->data_ptr(), ks, vs, (int)n, (int)per, static_cast<char*>(outs->data_ptr()) + 2 * first * outs->stride(0),
                           outs->stride(0), floats(lses) + first * lses->stride(0), B, Sq, Sc, Hq, Hkv, D,
                           q->stride(0), q->stride(1), q->stride(2), c0->stride(1), c0->stride(2), c0->stride(3),
                           c0->stride(1), c0->stride(2), c0->stride(3), outs->stride(1), outs->stride(2), outs->stride(3),
@@ -678,7 +700,8 @@ PyObject* bind(PyObject*, PyObject* table) {
   bound = false;
   auto take = [&](auto& f, const char* name) { f = reinterpret_cast<std::decay_t<decltype(f)>>(get(name)); return f != nullptr; };
   const bool ok = take(entry.fwd, "mhip_attn_fwd_block") && take(entry.fwd_many, "mhip_attn_fwd_blocks") &&
-                  take(entry.fwd_group, "mhip_attn_fwd_group") && take(entry.bwd_bytes, "mhip_attn_bwd_workspace_bytes") &&
+                  take(entry.fwd_group, "mhip_attn_fwd_group") && take(entry.fwd_chain, "mhip_attn_fwd_chain") &&
+                  take(entry.bwd_bytes, "mhip_attn_bwd_workspace_bytes") &&
                   take(entry.bwd, "mhip_attn_bwd_block") && take(entry.chunk, "mhip_attn_bwd_chunk") &&
                   take(entry.bwd_many, "mhip_attn_bwd_chunks") && take(entry.bwd_group, "mhip_attn_bwd_group") &&
                   take(entry.merge, "mhip_lse_merge") && take(entry.many, "mhip_lse_merge_many") &&
@@ -691,7 +714,7 @@ PyObject* bind(PyObject*, PyObject* table) {
 
 #define FAST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    FAST(undispatched), FAST(written), FAST(apart), FAST(rows_fit), FAST(fwd_block), FAST(fwd_group), FAST(fwd_blocks), FAST(no_dropout), FAST(bwd_block),
+    FAST(undispatched), FAST(written), FAST(apart), FAST(rows_fit), FAST(fwd_block), FAST(fwd_group), FAST(fwd_chain), FAST(fwd_blocks), FAST(no_dropout), FAST(bwd_block),
     FAST(bwd_chunk), FAST(bwd_group), FAST(bwd_chunks), FAST(merge_into), FAST(merge_many), FAST(pack_block), FAST(unpack_into), FAST(quantize_e4m3),
     {"bind", bind, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};

@@ -156,6 +156,18 @@ __device__ __forceinline__ void load_now(const P& p, const float& scale) {
                "s"(p.q_sh), "s"(p.k_sb), "s"(p.k_ss), "s"(p.k_sh), "s"(p.v_sb), "s"(p.v_ss), "s"(p.v_sh), "s"(scale));
 }
 
+// Estimated time (us) of a launch of n workgroups of t tile steps each, one workgroup per CU at a time: `fixed` per workgroup
+// and `step` per tile, plus `busy` times the share of the CUs at work (clock and L2).
+struct LaunchCost { float fixed, step, busy; };
+inline float rounds_time(float n, float t, const LaunchCost& c) {
+  const float full = (float)(int64_t)(n / 256.f), part = n / 256.f - full;
+  return full * (c.fixed + t * (c.step + c.busy)) + (part > 0.f ? c.fixed + t * (c.step + part * c.busy) : 0.f);
+}
+// and of the fold of a step's results, which is not needed for one
+inline float fold_time(int results, int B, int Sq, int Hq, int D) {
+  return results > 1 ? 4.f + (results + 1) * (2.f * B * Sq * Hq * D) / 5.3e6f : 0.f;
+}
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 inline int launch_status() {

@@ -36,6 +36,8 @@ from .merge import (MAX_MERGE_MANY, get_default_args, grad_accumulate, merge_int
 from .schedule import (LocalRing, n_dim_to_one_dim, n_ranks, one_dim_to_n_dim, reduce_buffer_route,
                        shift_tuple_element, zigzag_step)
 
+MAX_GROUP = 16           # MHIP_MAX_GROUP: chunks of a launch
+
 __all__ = ["flash_attn_pack_kv", "gqa_pack_kv", "flash_attn_pack_split_kv", "flash_attn_expose_reduce",
            "flash_attn_expose_reduce_q_ring",
            "flash_attn_backward", "zigzag_causal_pack_kv", "fp8_pack_split_kv", "quantize_e4m3"]
@@ -88,49 +90,73 @@ def _block_forward(q, k, v, softmax_scale, dropout_p, causal, window_size, alibi
     return outputs[:2]
 
 
-class _Places(list):
-    """(out, lse) per block, or None per block; ``stacked`` are the two tensors the places are slices of."""
-    stacked = None
+def _straight(q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **descales) -> bool:
+    """Whether the block operator would do nothing but call the kernel: nothing to report, nothing to record."""
+    return bool(_ops.as_declared((softmax_scale, dropout_p), window_size, (causal,))
+                and not (dropout_p or alibi_slopes is not None or window_size[0] != -1 or window_size[1] != -1)
+                and q.dim() == 4 and N.host.undispatched(q, kv, *descales.values()))
 
 
-def _block_results(n, q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **descales):
-    """Places for the results of a step's ``n`` blocks over all rows of ``q``, from one allocation each for the outputs and
-    the LSEs; None for every block where the operator has something to report or to record."""
-    if (not _ops.as_declared((softmax_scale, dropout_p), window_size, (causal,))
-            or dropout_p or alibi_slopes is not None or window_size[0] != -1 or window_size[1] != -1
-            or q.dim() != 4 or not N.host.undispatched(q, kv, *descales.values())):
-        return _Places([None] * n)
+def _result_places(n, q):
+    """(outs, lses) for ``n`` block results over all rows of ``q``, from one allocation each."""
     B, Sq, Hq, D = q.shape
-    outs = torch.empty((n, B, Sq, Hq, D), dtype=torch.bfloat16, device=q.device)
-    lses = torch.empty((n, B, Hq, Sq), dtype=torch.float32, device=q.device)
-    places = _Places(zip(outs.unbind(0), lses.unbind(0)))
-    places.stacked = outs, lses
-    return places
+    return (torch.empty((n, B, Sq, Hq, D), dtype=torch.bfloat16, device=q.device),
+            torch.empty((n, B, Hq, Sq), dtype=torch.float32, device=q.device))
 
 
-class _Groups:
-    """Block forwards of one query tensor over a step's chunks, several to a launch where the ring's chunks are all there
-    (mhip_attn_fwd_group has the rule); ``size`` is 1 where every block goes its own way."""
+def _block_results(n, q, kv, *args, **kwargs):
+    """Places for the results of a step's ``n`` blocks over all rows of ``q``; None for every block where the operator has
+    something to report or to record."""
+    if not _straight(q, kv, *args, **kwargs):
+        return [None] * n
+    outs, lses = _result_places(n, q)
+    return list(zip(outs.unbind(0), lses.unbind(0)))
 
-    def __init__(self, q, places, ring, softmax_scale, causal, q_descale=None, k_descale=None, v_descale=None):
-        self.size = 1
-        if places.stacked is not None and type(ring).__dict__.get("resident"):
-            self.size = N.host.fwd_group(q, len(places)) or 1
-        if self.size > 1:
-            self.q, self.places, self.done, self.chunks = q, places, 0, []
-            self.args = (softmax_scale, causal, q_descale, k_descale, v_descale)
 
-    def add(self, chunk) -> int:
-        """Takes the next chunk, launches if that makes a group or completes the step, and returns how many blocks are done
-        or waiting."""
+class _Together:
+    """Block forwards of one query tensor over ``n`` chunks of a ring whose chunks are all there, several to a launch
+    (mhip_attn_fwd_group) and, where that is faster, a run of chunks to a result (mhip_attn_fwd_chain).  ``size``, the
+    chunks of a launch, is 1 where every block goes its own way.  With ``into`` = (o, lse) a single result is written
+    there if neither overlaps anything the launch reads."""
+
+    def __init__(self, n, q, kv, ring, softmax_scale, dropout_p, causal, window_size, alibi_slopes, q_descale=None, k_descale=None,
+                 v_descale=None, into=None):
+        self.size = self.per = 1
+        if (n < 2 or not type(ring).__dict__.get("resident")
+                or not _straight(q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes, q_descale=q_descale,
+                                 k_descale=k_descale, v_descale=v_descale)):
+            return
+        self.per = 1 if causal else N.host.fwd_chain(q, kv, n) or 1
+        launches = -(-n // MAX_GROUP) if self.per > 1 else 0
+        self.size = -(-n // launches) if launches else N.host.fwd_group(q, n) or 1
+        if self.size < 2:
+            return
+        self.q, self.n, self.args = q, n, (softmax_scale, causal, q_descale, k_descale, v_descale)
+        self.seen, self.chunks, self.results = 0, [], []
+        total = sum(-(-min(self.size, n - at) // self.per) for at in range(0, n, self.size))
+        read = [t for t in (q, kv, *(ring.chunks or ()), q_descale, k_descale, v_descale) if t is not None]
+        self.direct = (total == 1 and into is not None and N.host.apart(into[0], into[1], *read) is True
+                       and N.host.apart(into[1], *read) is True)
+        self.outs, self.lses = (into[0][None], into[1][None]) if self.direct else _result_places(total, q)
+
+    def add(self, chunk) -> bool:
+        """Takes the next chunk, launches if that makes a group or completes the step; whether it did complete it."""
         self.chunks.append(chunk)
-        seen = self.done + len(self.chunks)
-        if len(self.chunks) == self.size or seen == len(self.places):
-            if N.host.fwd_blocks(self.q, self.chunks, *self.args, *self.places.stacked, self.done) is None:
-                for chunk, place in zip(self.chunks, self.places[self.done:]):
-                    _ops.attn_fwd_block(self.q, chunk[0], chunk[1], *self.args, *place)
-            self.done, self.chunks = seen, []
-        return seen
+        self.seen += 1
+        last = self.seen == self.n
+        if len(self.chunks) == self.size or last:
+            at = len(self.results)
+            if N.host.fwd_blocks(self.q, self.chunks, self.per, *self.args, self.outs, self.lses, at) is True:
+                self.results += [(self.outs[i], self.lses[i]) for i in range(at, at - (-len(self.chunks) // self.per))]
+            else:                               # layouts a launch cannot take together
+                self.direct = False
+                self.results += [_ops.attn_fwd_block(self.q, c[0], c[1], *self.args) for c in self.chunks]
+            self.chunks = []
+        return last
+
+    def fold(self, o, lse):
+        if not self.direct:
+            merge_many([r[0] for r in self.results], [r[1] for r in self.results], o, lse)
 
 
 def _as_rows(t):
@@ -184,11 +210,14 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
                       f"{MAX_MERGE_MANY} blocks and writes contiguous bfloat16, so this step merges block by block "
                       "(same result, one pass over the fp32 accumulator per block)", RuntimeWarning, stacklevel=3)
     done = 0
-    places = _Places([None] * n_blocks)
-    if defer:
-        places = _block_results(n_blocks, q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra)
+    places = [None] * n_blocks
+    together = None
     # (a divided ring is one that wants to hold little of other ranks' keys at a time)
-    groups = _Groups(q, _Places() if two_streams or ring_divide > 1 else places, ring, softmax_scale, causal, **extra)
+    if defer and not two_streams and ring_divide == 1:
+        together = _Together(n_blocks, q, kv, ring, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra, into=(o, lse))
+        together = together if together.size > 1 else None
+    if defer and together is None:
+        places = _block_results(n_blocks, q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra)
     main = side = None
     kv_ready = next_ready = None
     if two_streams and defer:
@@ -220,11 +249,9 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
                 if side is not None:                   # what the hop enqueued on the current stream ends here
                     next_ready = torch.cuda.Event()
                     next_ready.record(main)
-            if groups.size > 1:
-                done = groups.add(_kv)
-                if done == n_blocks:
-                    merge_many([p[0] for p in places], [p[1] for p in places], o, lse)
-                    return
+            if together is not None:
+                if together.add(_kv):
+                    together.fold(o, lse)
                 continue
             _k, _v = _kv.unbind(0)
             if side is not None and done % 2 == 1:
@@ -253,6 +280,8 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
                 merge_into(_out, _lse, block_out, block_lse, None, None, o, lse)
                 return
             _out, _lse = update_out_and_lse(_out, _lse, block_out, block_lse)
+    if together is not None:
+        return
     o[:, :, :, :] = _out.to(o.dtype)
     lse[:, :, :] = _lse.squeeze(dim=-1).transpose(1, 2)
 
@@ -314,10 +343,13 @@ def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=F
     blocks = []
     defer = (fused_epilogue and deferred_merge and len(hops) <= MAX_MERGE_MANY and o.dtype == torch.bfloat16
              and o.is_contiguous() and lse.is_contiguous())
-    places = _Places([None] * len(hops))
+    places = [None] * len(hops)
+    together = None
     if defer:
+        together = _Together(len(hops), q, kv, ring, softmax_scale, dropout_p, causal, window_size, alibi_slopes, into=(o, lse))
+        together = together if together.size > 1 else None
+    if defer and together is None:
         places = _block_results(len(hops), q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes)
-    groups = _Groups(q, places, ring, softmax_scale, causal)
     for step, hop in enumerate(hops):
         if step == 0:
             _kv = kv.contiguous()
@@ -328,8 +360,9 @@ def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=F
             send_to, recv_from = _neighbours(ring, hop)
             _next_kv = ring.send_recv(send_to, recv_from, _kv)
             ring.commit()
-        if groups.size > 1:
-            groups.add(_kv)
+        if together is not None:
+            if together.add(_kv):
+                together.fold(o, lse)
             continue
         _k, _v = _kv.unbind(0)
         block_out, block_lse = _block_forward(q, _k, _v, softmax_scale, dropout_p, causal, window_size, alibi_slopes,
@@ -338,8 +371,9 @@ def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=F
             blocks.append((block_out, block_lse))
         else:
             buf = pack_block(block_out, block_lse, reduce_into=buf)
+    if together is not None:
+        return
     if defer:
-        blocks = places if groups.size > 1 else blocks
         merge_many([b[0] for b in blocks], [b[1] for b in blocks], o, lse)
         return
     _store_packed(buf, o, lse, fused_epilogue)
@@ -403,13 +437,13 @@ def zigzag_causal_pack_kv(q, kv, o, lse, softmax_scale, dropout_p=0, causal=True
              and o.is_contiguous() and lse.is_contiguous())
     blocks = []
     kinds = [zigzag_step(ring.rank, step, world)[0] for step in range(world)]
-    place_of, groups = {}, {}
-    for kind, rows in (("diag", q), ("kv_first_half", q), ("q_second_half", q[:, half:])):
+    places, together = {}, {}
+    how = (softmax_scale, dropout_p, causal, window_size, alibi_slopes)
+    for kind, rows, keys in (("diag", q, kv), ("kv_first_half", q, kv[:, :, :half]), ("q_second_half", q[:, half:], kv)):
         n = kinds.count(kind)
-        places = _Places([None] * n)
-        if defer and n:
-            places = _block_results(n, rows, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes)
-        place_of[kind], groups[kind] = iter(places), _Groups(rows, places, ring, softmax_scale, kind == "diag")
+        together[kind] = _Together(n if defer else 0, rows, keys, ring, softmax_scale, dropout_p, kind == "diag", window_size, alibi_slopes)
+        grouped = together[kind].size > 1
+        places[kind] = iter([None] * n if grouped or not defer or not n else _block_results(n, rows, keys, *how))
     for step, kind in enumerate(kinds):
         if step == 0:
             _kv = kv.contiguous()
@@ -425,13 +459,12 @@ def zigzag_causal_pack_kv(q, kv, o, lse, softmax_scale, dropout_p=0, causal=True
             bkv = _kv[:, :, :half]
         elif kind == "q_second_half":
             bq, sl = q[:, half:], (slice(None), slice(half, None))
-        place = next(place_of[kind])
-        if groups[kind].size > 1:
-            groups[kind].add(bkv)
-            block_out, block_lse = place
-        else:
-            block_out, block_lse = _block_forward(bq, bkv[0], bkv[1], softmax_scale, dropout_p, kind == "diag", window_size,
-                                                  alibi_slopes, into=place)
+        if together[kind].size > 1:
+            if together[kind].add(bkv):
+                blocks += [(*r, 0 if sl is None else half) for r in together[kind].results]
+            continue
+        block_out, block_lse = _block_forward(bq, bkv[0], bkv[1], softmax_scale, dropout_p, kind == "diag", window_size,
+                                              alibi_slopes, into=next(places[kind]))
         if defer:
             blocks.append((block_out, block_lse, 0 if sl is None else half))
             continue

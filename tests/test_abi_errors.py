@@ -135,11 +135,12 @@ def test_elementwise_rejects(lib):
 
 
 def test_forward_blocks_reject(lib):
-    def blocks(ks=(P, P), vs=(P, P), n=2, o_sn=8192, out=P):
+    def blocks(ks=(P, P), vs=(P, P), n=2, o_sn=8192, out=P, per=1, mask=0):
         array = ctypes.c_void_p * 17
-        return lib.mhip_attn_fwd_blocks(P, array(*ks) if ks else None, array(*vs) if vs else None, n, out, o_sn, P, 1, 64, 64, 1, 1, 128,
-                                        *[8192, 128, 128] * 4, 0.1, 0, 0, None, None, None, None)
+        return lib.mhip_attn_fwd_blocks(P, array(*ks) if ks else None, array(*vs) if vs else None, n, per, out, o_sn, P, 1, 64, 64, 1, 1, 128,
+                                        *[8192, 128, 128] * 4, 0.1, mask, 0, None, None, None, None)
 
+    assert blocks(per=0) == blocks(per=-1) == EINVAL and blocks(per=2, mask=1) == EUNSUPPORTED
     assert blocks(n=0) == blocks(n=17, ks=[P] * 17, vs=[P] * 17) == blocks(n=-1) == EINVAL
     assert blocks(ks=None) == blocks(vs=None) == blocks(ks=(P, 0)) == blocks(vs=(P, 0)) == blocks(out=None) == EINVAL
     assert blocks(ks=(P, P + 8)) == blocks(vs=(P, P + 8)) == blocks(o_sn=8196) == EALIGN

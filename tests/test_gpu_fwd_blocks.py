@@ -8,6 +8,11 @@ from mercury_artifact_amd import _native as N
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def _loaded():
+    N.lib()                    # the host module answers once it knows the library's entry points
+
+
 def _inputs(n, B, Sq, Sc, Hq, Hkv, D, fp8):
     g = torch.Generator().manual_seed(n * 1000 + Sq + Sc)
     q = torch.randn(B, Sq, Hq, D, generator=g)
@@ -35,7 +40,7 @@ def test_blocks_of_a_launch_match_the_oracle(n, B, Sq, Sc, Hq, Hkv, D, causal, f
     outs = torch.full((n + 1, B, Sq, Hq, D), 7.0, dtype=torch.bfloat16, device="cuda")
     lses = torch.full((n + 1, B, Hq, Sq), 7.0, device="cuda")
     ds = [None] * 3 if not fp8 else [t.cuda().reshape(()) for t in (sq, sc, sc)]
-    assert N.host.fwd_blocks(q.cuda(), [c.cuda() for c in chunks], scale, causal, *ds, outs, lses, 1) is True
+    assert N.host.fwd_blocks(q.cuda(), [c.cuda() for c in chunks], 1, scale, causal, *ds, outs, lses, 1) is True
     torch.cuda.synchronize()
     assert (outs[0] == 7).all() and (lses[0] == 7).all()
     for i, c in enumerate(chunks):
@@ -59,7 +64,7 @@ def test_blocks_refuse_what_a_launch_cannot_take():
     outs, lses = torch.full((3, 1, 64, 2, 64), 7.0, dtype=torch.bfloat16, device="cuda"), torch.full((3, 1, 2, 64), 7.0, device="cuda")
 
     def call(cs, first=0, q=q):
-        return N.host.fwd_blocks(q, cs, 0.1, False, None, None, None, outs, lses, first)
+        return N.host.fwd_blocks(q, cs, 1, 0.1, False, None, None, None, outs, lses, first)
 
     strided = torch.empty(2, 1, 64, 2, 128, dtype=torch.bfloat16, device="cuda")[..., :64]
     assert call([]) is call(chunks, 1) is call(chunks, -1) is call(chunks * 6) is None
@@ -103,3 +108,95 @@ def test_only_rings_with_resident_chunks_get_grouped_launches(path, own_class):
     want, wl = torch.empty_like(o), torch.empty_like(lse)
     step(q, chunks[2], want, wl, 0.125, ring=M.LocalRing((4,), 2, chunks), deferred_merge=False)
     assert (o.float() - want.float()).abs().max().item() <= 2e-2 and (lse - wl).abs().max().item() <= 1e-3
+
+
+@pytest.mark.parametrize("n,per,B,Sq,Sc,Hq,Hkv,D", [
+    (2, 2, 1, 64, 64, 1, 1, 128), (16, 16, 1, 33, 1, 2, 1, 128), (5, 2, 2, 257, 65, 3, 3, 96), (5, 5, 1, 300, 257, 4, 2, 64),
+    (3, 2, 1, 200, 320, 8, 8, 128), (7, 3, 1, 130, 200, 2, 2, 80), (4, 4, 1, 512, 512, 4, 4, 128), (9, 8, 2, 100, 130, 5, 5, 40),
+    (6, 6, 1, 70, 448, 2, 1, 64), (8, 4, 1, 256, 383, 2, 2, 96)])
+@pytest.mark.parametrize("ramp", [0.0, 30.0])
+def test_chunks_of_one_result_match_the_oracle(n, per, B, Sq, Sc, Hq, Hkv, D, ramp):
+    """Runs of chunks as one sequence of tiles: chunks of one tile to eight (fewer than, as many as and more than are requested
+    ahead), ragged ends inside the sequence, a last run that is shorter; with a ramp the scores climb by 30 nats from the
+    first chunk to the last, so that the reference of a row moves in later chunks.  Against attention over all keys of a
+    run in fp32: one rounding of P and of the result."""
+    q, chunks, _, _ = _inputs(n, B, Sq, Sc, Hq, Hkv, D, False)
+    scale = D ** -0.5
+    if ramp:
+        q[..., :8] = 2.0
+        for i, c in enumerate(chunks):
+            c[0][..., :8] = ramp * i / max(n - 1, 1) / 16.0 / scale
+    print(f"n{n} per{per} B{B} Sq{Sq} Sc{Sc} H{Hq}/{Hkv} D{D} ramp={ramp}", flush=True)
+    runs = [chunks[i:i + per] for i in range(0, n, per)]
+    outs = torch.full((len(runs) + 1, B, Sq, Hq, D), 7.0, dtype=torch.bfloat16, device="cuda")
+    lses = torch.full((len(runs) + 1, B, Hq, Sq), 7.0, device="cuda")
+    assert N.host.fwd_blocks(q.cuda(), [c.cuda() for c in chunks], per, scale, False, None, None, None, outs, lses, 0) is True
+    torch.cuda.synchronize()
+    assert (outs[-1] == 7).all() and (lses[-1] == 7).all()
+    for i, run in enumerate(runs):
+        k, v = torch.cat([c[0] for c in run], 1).float(), torch.cat([c[1] for c in run], 1).float()
+        ro, rl = O.block_attention(q.float(), k, v, scale)
+        got = outs[i].float().cpu()
+        assert ((got - ro).abs() - 2 ** -8 * ro.abs()).max().item() <= 2e-2, i
+        assert (got - ro).norm() <= 1e-2 * ro.norm(), i
+        assert ((lses[i].cpu() - rl).abs() / rl.abs().clamp_min(1.0)).max().item() <= 1e-3, i
+
+
+def test_a_run_of_chunks_needs_one_row_stride_and_no_mask():
+    q, chunks, _, _ = _inputs(4, 1, 64, 64, 2, 2, 64, False)
+    q, chunks = q.cuda(), [c.cuda() for c in chunks]
+    outs, lses = torch.full((2, 1, 64, 2, 64), 7.0, dtype=torch.bfloat16, device="cuda"), torch.full((2, 1, 2, 64), 7.0, device="cuda")
+    call = lambda per, causal, first=0: N.host.fwd_blocks(q, chunks, per, 0.1, causal, None, None, None, outs, lses, first)
+    assert call(2, True) is call(0, False) is call(17, False) is call(2, False, 1) is call(1, False) is None
+    torch.cuda.synchronize()
+    assert (outs == 7).all() and (lses == 7).all()
+    assert call(2, False) is True
+
+
+def test_the_only_result_of_a_step_goes_straight_out_unless_the_output_is_read():
+    """Steps whose chunks all go into one result write the caller's tensors; an output that lies over the queries or over a
+    chunk is written by a fold behind the launch instead."""
+    import mercury_artifact_amd as M
+
+    W, S, H, D = 2, 1024, 64, 128
+    assert N.lib().mhip_attn_fwd_chain(1, S, S, H, D, W, N.MHIP_BF16) == W
+    q, chunks, _, _ = _inputs(W, 1, S, S, H, H, D, False)
+    want = None
+    for over in ("nothing", "q", "chunk"):
+        qd, dev = q.cuda(), [c.cuda() for c in chunks]
+        o = {"nothing": torch.empty_like(qd), "q": qd, "chunk": dev[1][0]}[over]
+        lse = torch.empty(1, H, S, device="cuda")
+        M.flash_attn_pack_kv(qd, dev[0], o, lse, D ** -0.5, ring=M.LocalRing((W,), 0, dev))
+        torch.cuda.synchronize()
+        if want is None:
+            want = o.clone(), lse.clone()
+            ro, rl = O.block_attention(q.float(), *(torch.cat([c[i] for c in chunks], 1).float() for i in (0, 1)), D ** -0.5)
+            assert (o.float().cpu() - ro).norm() <= 1e-2 * ro.norm()
+        assert torch.equal(o, want[0]) and (lse - want[1]).abs().max().item() <= 1e-5, over
+
+
+@pytest.mark.parametrize("n,per,B,Sq,Sc,Hq,Hkv,D", [
+    (2, 2, 1, 64, 64, 1, 1, 128), (16, 16, 1, 33, 1, 2, 1, 128), (5, 2, 2, 257, 129, 3, 3, 96), (5, 5, 1, 300, 257, 4, 2, 64),
+    (3, 3, 1, 200, 640, 4, 4, 128), (7, 3, 1, 130, 200, 2, 2, 80), (4, 2, 1, 130, 320, 130, 130, 128), (9, 8, 1, 130, 70, 130, 1, 64),
+    (4, 4, 1, 130, 191, 130, 130, 96)])
+def test_e4m3_chunks_of_one_result_match_the_oracle(n, per, B, Sq, Sc, Hq, Hkv, D):
+    """The same for e4m3, with workgroups of four and (130 heads) of eight wavefronts."""
+    q, chunks, sq, sc = _inputs(n, B, Sq, Sc, Hq, Hkv, D, True)
+    scale = D ** -0.5
+    runs = [chunks[i:i + per] for i in range(0, n, per)]
+    print(f"e4m3 n{n} per{per} B{B} Sq{Sq} Sc{Sc} H{Hq}/{Hkv} D{D}", flush=True)
+    assert N.lib().mhip_attn_fwd_plan(B * len(runs), Sq, Sc, Hq, D, D, D, 0, N.MHIP_E4M3) == (8 if Hq == 130 else 4)
+    outs = torch.full((len(runs) + 1, B, Sq, Hq, D), 7.0, dtype=torch.bfloat16, device="cuda")
+    lses = torch.full((len(runs) + 1, B, Hq, Sq), 7.0, device="cuda")
+    ds = [t.cuda().reshape(()) for t in (sq, sc, sc)]
+    assert N.host.fwd_blocks(q.cuda(), [c.cuda() for c in chunks], per, scale, False, *ds, outs, lses, 0) is True
+    torch.cuda.synchronize()
+    assert (outs[-1] == 7).all() and (lses[-1] == 7).all()
+    for i, run in enumerate(runs):
+        ops = [O.dequantize(q, sq)] + [torch.cat([O.dequantize(c[j], sc) for c in run], 1) for j in (0, 1)]
+        ro, rl = O.block_attention(*ops, scale)
+        bound = O.e4m3_p_rounding_bound(*ops, scale)
+        got = outs[i].float().cpu()
+        assert ((got - ro).abs() - (bound + 2 ** -8 * ro.abs())).max().item() <= 2e-3, i
+        assert (got - ro).norm() <= 6e-2 * ro.norm(), i
+        assert ((lses[i].cpu() - rl).abs() / rl.abs().clamp_min(1.0)).max().item() <= 1e-3, i

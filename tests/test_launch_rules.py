@@ -70,3 +70,16 @@ def test_chunks_of_a_backward_step_share_a_launch():
     assert group(1, 64, 64, 1, 1, 64, 40) == 14                               # of at most 16: three launches
     assert group(1, 256, 256, 4, 4, 64, 1) == group(0, 64, 64, 4, 4, 64, 8) == group(1, 0, 64, 4, 4, 64, 8) == 1
     assert group(1, 64, 64, 4, 3, 64, 8) < 0 and group(1, 64, 64, 4, 4, 136, 8) < 0 and group(1, 64, 64, 4, 4, 64, 0) < 0
+
+
+def test_runs_of_chunks_where_blocks_would_take_turns_on_the_cus():
+    chain = N.lib().mhip_attn_fwd_chain
+    for dtype in (N.MHIP_BF16, N.MHIP_E4M3):
+        assert chain(1, 4096, 4096, 32, 128, 8, dtype) == chain(1, 2048, 2048, 32, 128, 8, dtype) == 8
+        assert chain(1, 256, 256, 4, 64, 4, dtype) == chain(1, 512, 512, 8, 128, 16, dtype) == 1      # all side by side
+        assert chain(1, 4096, 4096, 32, 128, 1, dtype) == chain(1, 4096, 0, 32, 128, 8, dtype) == chain(0, 64, 64, 4, 128, 8, dtype) == 1
+        assert chain(1, 4096, 4096, 32, 128, 17, dtype) == 1                                          # more than a launch takes
+        assert chain(1, 64, 64, 0, 128, 8, dtype) < 0 and chain(1, 64, 64, 4, 136, 8, dtype) < 0 and chain(1, 64, 64, 4, 64, 0, dtype) < 0
+    assert chain(1, 1024, 1024, 32, 128, 8, N.MHIP_BF16) == 4             # 256 workgroups, and two results to fold
+    assert chain(2, 1237, 1237, 16, 80, 8, N.MHIP_BF16) == 1              # 160 workgroups: any run leaves a ragged round
+    assert chain(1, 64, 64, 4, 64, 8, N.MHIP_F32) < 0
