@@ -578,11 +578,39 @@ PyObject* merge_into(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// (block_outs, block_lses, final_out, final_lse, row_begin or None): lists or tuples -> True
+// (block_outs, block_lses, final_out, final_lse, row_begin or None): lists or tuples, or the blocks' results over all rows
+// stacked in one tensor each, (n, B, Sq, Hq, D) and (n, B, Hq, Sq) -> True
 PyObject* merge_many(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   ENTER(5);
   constexpr Py_ssize_t kMost = 64;
+  if (const Tensor *outs = plain(a[0]), *lses = plain(a[1]); outs && lses) {
+    const Tensor *out = plain(a[2]), *lse = plain(a[3]);
+    if (a[4] != Py_None || !out || !lse || outs->dim() != 5 || lses->dim() != 4 || out->dim() != 4) SLOW;
+    const int64_t n = outs->size(0), B = out->size(0), Sq = out->size(1), Hq = out->size(2), D = out->size(3);
+    if (n < 1 || n > kMost || outs->sizes().slice(1) != out->sizes() || lses->size(0) != n || lses->size(1) != B || lses->size(2) != Hq ||
+        lses->size(3) != Sq || outs->device() != out->device() || lses->device() != out->device() || lse->device() != out->device() ||
+        outs->scalar_type() != at::kBFloat16 || !outs->is_contiguous() || lses->scalar_type() != at::kFloat || !lses->is_contiguous() ||
+        out->scalar_type() != at::kBFloat16 || !out->is_contiguous() || !shape3(*lse, B, Hq, Sq) ||
+        lse->scalar_type() != at::kFloat || !lse->is_contiguous() || B * Sq * Hq == 0 || !fits({B, Sq, Hq}))
+      SLOW;
+    const void* block_outs[kMost];
+    const float* block_lses[kMost];
+    int64_t strides[kMost];
+    for (int64_t i = 0; i < n; ++i) {
+      block_outs[i] = static_cast<const char*>(outs->data_ptr()) + 2 * i * outs->stride(0);
+      block_lses[i] = floats(lses) + i * lses->stride(0);
+      strides[i] = outs->stride(1);
+    }
+    OnDevice on(*out);
+    if (!on.current) SLOW;
+    const int code = without_gil([&] {
+      return entry.many(block_outs, block_lses, strides, nullptr, (int)n, out->data_ptr(), floats(lse), B, Sq, Hq, D, outs->stride(2),
+                        outs->stride(3), on.stream);
+    });
+    if (code != MHIP_OK) return refused(code, "mhip_lse_merge_many");
+    Py_RETURN_TRUE;
+  }
   auto list = [](PyObject* o) { return PyList_CheckExact(o) || PyTuple_CheckExact(o); };
   if (!list(a[0]) || !list(a[1]) || !(a[4] == Py_None || list(a[4]))) SLOW;
   const Py_ssize_t n = PySequence_Fast_GET_SIZE(a[0]);

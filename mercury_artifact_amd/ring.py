@@ -131,32 +131,63 @@ class _Together:
         self.size = -(-n // launches) if launches else N.host.fwd_group(q, n) or 1
         if self.size < 2:
             return
-        self.q, self.n, self.args = q, n, (softmax_scale, causal, q_descale, k_descale, v_descale)
-        self.seen, self.chunks, self.results = 0, [], []
-        total = sum(-(-min(self.size, n - at) // self.per) for at in range(0, n, self.size))
-        read = [t for t in (q, kv, *(ring.chunks or ()), q_descale, k_descale, v_descale) if t is not None]
-        self.direct = (total == 1 and into is not None and N.host.apart(into[0], into[1], *read) is True
-                       and N.host.apart(into[1], *read) is True)
+        self.q, self.args = q, (softmax_scale, causal, q_descale, k_descale, v_descale)
+        total = n if self.per == 1 else sum(-(-min(self.size, n - at) // self.per) for at in range(0, n, self.size))
+        self.direct = False
+        if total == 1 and into is not None:
+            read = [t for t in (q, kv, *(ring.chunks or ()), q_descale, k_descale, v_descale) if t is not None]
+            self.direct = N.host.apart(into[0], into[1], *read) is True and N.host.apart(into[1], *read) is True
         self.outs, self.lses = (into[0][None], into[1][None]) if self.direct else _result_places(total, q)
 
-    def add(self, chunk) -> bool:
-        """Takes the next chunk, launches if that makes a group or completes the step; whether it did complete it."""
-        self.chunks.append(chunk)
-        self.seen += 1
-        last = self.seen == self.n
-        if len(self.chunks) == self.size or last:
-            at = len(self.results)
-            if N.host.fwd_blocks(self.q, self.chunks, self.per, *self.args, self.outs, self.lses, at) is True:
-                self.results += [(self.outs[i], self.lses[i]) for i in range(at, at - (-len(self.chunks) // self.per))]
-            else:                               # layouts a launch cannot take together
+    def run(self, chunks):
+        """The (out, lse) results over the step's chunks, in two lists (or tensors stacked alike)."""
+        done, apart = 0, None                   # apart: results of launches whose chunks were not of one layout
+        for at in range(0, len(chunks), self.size):
+            part = chunks[at:at + self.size]
+            if apart is None and N.host.fwd_blocks(self.q, part, self.per, *self.args, self.outs, self.lses, done) is True:
+                done -= -len(part) // self.per
+                continue
+            if apart is None:
+                apart = list(zip(self.outs[:done].unbind(0), self.lses[:done].unbind(0)))
                 self.direct = False
-                self.results += [_ops.attn_fwd_block(self.q, c[0], c[1], *self.args) for c in self.chunks]
-            self.chunks = []
-        return last
+            apart += [_ops.attn_fwd_block(self.q, c[0], c[1], *self.args) for c in part]
+        return (self.outs, self.lses) if apart is None else ([r[0] for r in apart], [r[1] for r in apart])
 
-    def fold(self, o, lse):
-        if not self.direct:
-            merge_many([r[0] for r in self.results], [r[1] for r in self.results], o, lse)
+    def step(self, chunks, o, lse):
+        """The whole step: results and, unless the only one was written straight out, their fold."""
+        outs, lses = self.run(chunks)
+        if self.direct or N.host.merge_many(outs, lses, o, lse, None) is not None:
+            return
+        merge_many(list(outs), list(lses), o, lse)
+
+
+@lru_cache(maxsize=256)
+def _visits(mesh_shape, rank, held):
+    """The chunks ``rank`` holds at the steps of a ring that starts with ``held``, and what everyone holds in the end."""
+    ring = LocalRing(mesh_shape, rank)
+    ring.held = list(held)
+    seen = [ring.current]
+    for hop in _hop_list(mesh_shape)[:-1]:
+        seen.append(ring.hop(hop))
+    return tuple(seen), ring.held
+
+
+def _resident_chunks(ring, kv):
+    """A step's chunks in visiting order, for a ring whose chunks are all there; leaves the ring where the hops would."""
+    chunks = [_as_rows(kv)]
+    if (type(ring) is LocalRing and ring.chunks is not None and not ring.copy and not ring._committed
+            and ring.__dict__.keys().isdisjoint(("send_recv", "commit", "wait", "hop"))):       # nobody looks on
+        seen, held = _visits(ring.mesh_shape, ring.rank, tuple(ring.held))
+        chunks += [ring.chunks[i] for i in seen[1:]]
+        ring.held = list(held)
+        return chunks
+    for step, hop in enumerate(_hops(ring)):
+        if step > 0:
+            ring.wait()
+        if hop is not None:
+            chunks.append(ring.send_recv(*_neighbours(ring, hop), chunks[-1]))
+            ring.commit()
+    return chunks
 
 
 def _as_rows(t):
@@ -211,12 +242,13 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
                       "(same result, one pass over the fp32 accumulator per block)", RuntimeWarning, stacklevel=3)
     done = 0
     places = [None] * n_blocks
-    together = None
     # (a divided ring is one that wants to hold little of other ranks' keys at a time)
     if defer and not two_streams and ring_divide == 1:
         together = _Together(n_blocks, q, kv, ring, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra, into=(o, lse))
-        together = together if together.size > 1 else None
-    if defer and together is None:
+        if together.size > 1:
+            together.step(_resident_chunks(ring, kv), o, lse)
+            return
+    if defer:
         places = _block_results(n_blocks, q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra)
     main = side = None
     kv_ready = next_ready = None
@@ -249,10 +281,6 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
                 if side is not None:                   # what the hop enqueued on the current stream ends here
                     next_ready = torch.cuda.Event()
                     next_ready.record(main)
-            if together is not None:
-                if together.add(_kv):
-                    together.fold(o, lse)
-                continue
             _k, _v = _kv.unbind(0)
             if side is not None and done % 2 == 1:
                 if kv_ready is not None:
@@ -280,8 +308,6 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
                 merge_into(_out, _lse, block_out, block_lse, None, None, o, lse)
                 return
             _out, _lse = update_out_and_lse(_out, _lse, block_out, block_lse)
-    if together is not None:
-        return
     o[:, :, :, :] = _out.to(o.dtype)
     lse[:, :, :] = _lse.squeeze(dim=-1).transpose(1, 2)
 
@@ -344,11 +370,11 @@ def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=F
     defer = (fused_epilogue and deferred_merge and len(hops) <= MAX_MERGE_MANY and o.dtype == torch.bfloat16
              and o.is_contiguous() and lse.is_contiguous())
     places = [None] * len(hops)
-    together = None
     if defer:
         together = _Together(len(hops), q, kv, ring, softmax_scale, dropout_p, causal, window_size, alibi_slopes, into=(o, lse))
-        together = together if together.size > 1 else None
-    if defer and together is None:
+        if together.size > 1:
+            together.step(_resident_chunks(ring, kv), o, lse)
+            return
         places = _block_results(len(hops), q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes)
     for step, hop in enumerate(hops):
         if step == 0:
@@ -360,10 +386,6 @@ def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=F
             send_to, recv_from = _neighbours(ring, hop)
             _next_kv = ring.send_recv(send_to, recv_from, _kv)
             ring.commit()
-        if together is not None:
-            if together.add(_kv):
-                together.fold(o, lse)
-            continue
         _k, _v = _kv.unbind(0)
         block_out, block_lse = _block_forward(q, _k, _v, softmax_scale, dropout_p, causal, window_size, alibi_slopes,
                                               into=places[step])
@@ -371,8 +393,6 @@ def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=F
             blocks.append((block_out, block_lse))
         else:
             buf = pack_block(block_out, block_lse, reduce_into=buf)
-    if together is not None:
-        return
     if defer:
         merge_many([b[0] for b in blocks], [b[1] for b in blocks], o, lse)
         return
@@ -437,7 +457,7 @@ def zigzag_causal_pack_kv(q, kv, o, lse, softmax_scale, dropout_p=0, causal=True
              and o.is_contiguous() and lse.is_contiguous())
     blocks = []
     kinds = [zigzag_step(ring.rank, step, world)[0] for step in range(world)]
-    places, together = {}, {}
+    places, together, waiting = {}, {}, []
     how = (softmax_scale, dropout_p, causal, window_size, alibi_slopes)
     for kind, rows, keys in (("diag", q, kv), ("kv_first_half", q, kv[:, :, :half]), ("q_second_half", q[:, half:], kv)):
         n = kinds.count(kind)
@@ -460,8 +480,10 @@ def zigzag_causal_pack_kv(q, kv, o, lse, softmax_scale, dropout_p=0, causal=True
         elif kind == "q_second_half":
             bq, sl = q[:, half:], (slice(None), slice(half, None))
         if together[kind].size > 1:
-            if together[kind].add(bkv):
-                blocks += [(*r, 0 if sl is None else half) for r in together[kind].results]
+            waiting.append(bkv)
+            if step + 1 == world or kinds[step + 1] != kind:
+                blocks += [(*r, 0 if sl is None else half) for r in zip(*(list(t) for t in together[kind].run(waiting)))]
+                waiting = []
             continue
         block_out, block_lse = _block_forward(bq, bkv[0], bkv[1], softmax_scale, dropout_p, kind == "diag", window_size,
                                               alibi_slopes, into=next(places[kind]))
