@@ -38,10 +38,7 @@ constexpr int kD = 128;
 constexpr int kTile = 64;             // streamed rows per main-loop tile
 constexpr int kRowsKv = 128;          // stationary key rows per workgroup of the dK / dV pass (4 wavefronts x 32)
 constexpr int kRowsQ = 256;           // stationary query rows per workgroup of the dQ pass (8 wavefronts x 32)
-constexpr int kTileBytes = kTile * kD * 2;             // 16384: 64 rows of 256 bytes
-constexpr int kOffY = kTileBytes, kOffLse = 2 * kTileBytes, kOffDelta = kOffLse + kTile * 4;
 constexpr int kStages = 4;
-constexpr int kOStride = kD + 8;
 constexpr int kNoTile = 0x7fff0000;   // scalar offset that puts every lane of a copy out of range
 constexpr int kNoColumn = 0x7fff0000; // vector offset with the same effect for one lane (the sum of the two is
                                       // below 2^32: no wrap)
@@ -90,16 +87,24 @@ struct Chunks {
 
 // KK = k-steps of 16 head-dim values in T1 / T2: 8 computes on all 128 on-chip columns; 4 and 6 are the instantiations for
 // head dimensions up to 64 and up to 96, which leave out the MFMAs, accumulators and fragments of the zero columns.  The
-// vector work of a tile is the same, so a T1 / T2 slot carries more of it: 4096 x 4096, H32 takes 473 us instead of 654 at
+// vector work of a tile is the same, so a T1 / T2 slot carries more of it: 4096 x 4096, H32 takes 426 us instead of 654 at
 // D 64 and 616 instead of 709 at D 96, 1237 x 1237, B2 H16/8, D 80 78.1 instead of 88.6, 512 x 512, B4 H5, D 96 16.9
 // instead of 18.5; results bit-identical.
 //
 // WAVES = 8 wavefronts of 32 stationary rows (dQ: two per SIMD) or 4 (one per SIMD).  PREPARED: lse2 and delta of the
 // query rows are in the workspace already; otherwise the dQ pass works them out.
-template <bool DQ, int WAVES>
-constexpr int kStageBytesOf = DQ ? 2 * kTileBytes : kOffDelta + kTile * 4;
-template <bool DQ, int WAVES>
-constexpr int kSmemBytesOf = WAVES == 8 ? 3 * kStageBytesOf<DQ, WAVES> + WAVES * 32 * kD * 2 : kStages * kStageBytesOf<DQ, WAVES>;
+//
+// A row is 256 bytes on chip, on 64 columns 128: with half the LDS and at most 256 registers two workgroups of four
+// wavefronts share a CU there, two wavefronts per SIMD, so that the vector work of one runs beside the MFMAs of the other:
+// 4096 x 4096 H32 D 64 475 us to 426, 2048 x 2048 H16 70.3 to 59.9, causal 1500 x 1500 B2 H12 47.1 to 40.4, 8192 x 8192 H4
+// 245 to 209.
+template <int KK>
+constexpr int kRowBytesOf = KK == 4 ? 128 : 256;
+template <bool DQ, int KK>
+constexpr int kStageBytesOf = 2 * kTile * kRowBytesOf<KK> + (DQ ? 0 : 2 * kTile * 4);
+template <bool DQ, int WAVES, int KK>
+constexpr int kSmemBytesOf =
+    WAVES == 8 ? 3 * kStageBytesOf<DQ, KK> + WAVES * 32 * kRowBytesOf<KK> : kStages * kStageBytesOf<DQ, KK>;
 
 // SPLIT: the workgroups of the pass may share their stationary tile (w.splits).
 //
@@ -109,20 +114,26 @@ constexpr int kSmemBytesOf = WAVES == 8 ? 3 * kStageBytesOf<DQ, WAVES> + WAVES *
 template <bool DQ, bool CAUSAL, int KK, int WAVES, bool PREPARED, bool SPLIT, bool CHUNKS = false>
 __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, const int block, unsigned char* smem,
                                          const Chunks* chunks = nullptr) {
-  static_assert(DQ || WAVES == 4, "the dK / dV pass has no room for two wavefronts per SIMD");
+  static_assert(DQ || WAVES == 4, "the dK / dV pass has no room for eight wavefronts in a workgroup");
   static_assert(!CHUNKS || (!SPLIT && !CAUSAL), "launches of several chunks are not split further");
   static_assert(PREPARED || WAVES == 8, "the pass that prepares is the one with a launch of its own");
   constexpr int DB = KK / 2;                    // blocks of 32 head-dim values in the accumulators
   constexpr int kWavesWg = WAVES;
   constexpr int kRowsPerWg = kWavesWg * 32;
-  constexpr int kCpy = 16 / kWavesWg;           // copy instructions per wavefront for one 16 KB tile
-  constexpr int kRowsBytes = kRowsPerWg * kD * 2;       // one tensor's stationary rows
+  constexpr int kRow = kRowBytesOf<KK>;
+  constexpr int kLanes = kRow / 16, kRowsPerCopy = 64 / kLanes;      // a copy instruction: whole rows, 16 bytes per lane
+  constexpr int kTileBytes = kTile * kRow;
+  constexpr int kCpy = kTileBytes / 1024 / kWavesWg;    // copy instructions per wavefront for one tile
+  constexpr int kRowsBytes = kRowsPerWg * kRow;         // one tensor's stationary rows
   // X tile, Y tile, and in the dK / dV pass lse2 and delta of the streamed rows
-  constexpr int kStageBytes = kStageBytesOf<DQ, WAVES>;
+  constexpr int kStageBytes = kStageBytesOf<DQ, KK>;
+  constexpr int kOffY = kTileBytes, kOffLse = 2 * kTileBytes, kOffDelta = kOffLse + kTile * 4;
+  // chunk c (16 bytes) of row r of a tile is kept at chunk position c ^ swz(r)
+  auto swz = [](int row) { return kRow == 256 ? lds_row_swizzle(row) : lds_half_row_swizzle(row); };
   // The stationary rows pass through LDS on their way into registers, in one stage each; with eight wavefronts X takes
   // the last stage and 32 KB behind it and Y the two stages before.
   constexpr int kXRows = 3 * kStageBytes, kYRows = WAVES == 8 ? kStageBytes : 2 * kStageBytes;
-  static_assert(kYRows + kRowsBytes <= kXRows && kXRows + kRowsBytes <= kSmemBytesOf<DQ, WAVES>, "the rows' places");
+  static_assert(kYRows + kRowsBytes <= kXRows && kXRows + kRowsBytes <= kSmemBytesOf<DQ, WAVES, KK>, "the rows' places");
 
   // One round of argument loads instead of one before each first use (load_now in the common header says why).
   {
@@ -246,8 +257,8 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   int cvoff[kCpy];
 #pragma unroll
   for (int u = 0; u < kCpy; ++u) {
-    const int row = 4 * kCpy * wave + 4 * u + (lane >> 4);
-    const int chunk = (lane & 15) ^ lds_row_swizzle(row);
+    const int row = kRowsPerCopy * (kCpy * wave + u) + lane / kLanes;
+    const int chunk = (lane % kLanes) ^ swz(row);
     // chunks past the head dimension: an offset that is out of the descriptor's range for every tile, so they
     // arrive as zeros and a tile in LDS always has 128 columns
     cvoff[u] = chunk * 8 < p.D ? (int)(row * s_ss * 2) + (chunk << 4) : kNoColumn;
@@ -300,14 +311,14 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   };
 
   // row-major operand reads (A of T1 / T2): lane (ln, hf) reads chunk 2 kk + hf of row 32 mb + ln
-  int rm_rd[KK];                                      // + mb * 8192
+  int rm_rd[KK];                                      // + mb * 32 rows
 #pragma unroll
-  for (int kk = 0; kk < KK; ++kk) rm_rd[kk] = ln * 256 + (((2 * kk + hf) ^ lds_row_swizzle(ln)) << 4);
+  for (int kk = 0; kk < KK; ++kk) rm_rd[kk] = ln * kRow + (((2 * kk + hf) ^ swz(ln)) << 4);
   // transposed operand reads (A of the second MFMAs) for head-dim block db and k-step (mb, j2): the lane's
   // 8 streamed rows are R + {0..3} and R + 8 + {0..3}, R = 32 mb + 16 j2 + 4 hf -- the rows its P / dS
   // registers hold.  One ds_read_b64_tr_b16 per group of 4 rows: within 16 lanes, lane s supplies the
   // address of row R + s/4, head-dim values 4 (s%4) .. +3 of the 16-column strip, and receives column s.
-  int tr_rd[DB][2];                                   // [db][second four rows]  + mb * 8192 + j2 * 4096
+  int tr_rd[DB][2];                                   // [db][second four rows]  + mb * 32 rows + j2 * 16 rows
   {
     const int s16 = lane & 15, strip = (lane >> 4) & 1;
     const int cl = 2 * strip + ((s16 & 3) >> 1);
@@ -316,7 +327,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int row = 8 * h + 4 * hf + (s16 >> 2);
-        tr_rd[db][h] = row * 256 + (((4 * db + cl) ^ lds_row_swizzle(row)) << 4) + (s16 & 1) * 8;
+        tr_rd[db][h] = row * kRow + (((4 * db + cl) ^ swz(row)) << 4) + (s16 & 1) * 8;
       }
   }
   typedef __attribute__((address_space(3))) bf16x4* lds_bf16x4;
@@ -363,7 +374,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   int ld_cur = (int)lds_base + hf * 16, ld_next = ld_cur + kStageBytes;
   // slot i of the T1 / T2 sequence of one half: k-step i / 2, X (T1) on even and Y (T2) on odd slots
   auto read_rm = [&](int mb, int i) -> bf16x8 {
-    return *(lds_bf16x8)(uintptr_t)(uint32_t)(rm_a[i >> 1] + mb * 8192 + ((i & 1) ? kOffY : 0));
+    return *(lds_bf16x8)(uintptr_t)(uint32_t)(rm_a[i >> 1] + mb * (32 * kRow) + ((i & 1) ? kOffY : 0));
   };
   // T2 starts from -delta of the half's streamed rows (dQ pass: of this lane's stationary row), so that what
   // the vector unit receives is dP - delta already
@@ -376,7 +387,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   // slot i of an accumulate phase of half mb: head-dim block and k-step, X^T (dS) / Y^T (P) alternating for dK, dV
   auto read_acc = [&](int mb, int i) -> bf16x8 {
     const int m = DQ ? i : (i >> 1);
-    const int off = mb * 8192 + (m / DB) * 4096 + ((!DQ && (i & 1)) ? kOffY : 0);
+    const int off = mb * (32 * kRow) + (m / DB) * (16 * kRow) + ((!DQ && (i & 1)) ? kOffY : 0);
     const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(tr_a[m % DB][0] + off));
     const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(tr_a[m % DB][1] + off));
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -483,18 +494,19 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   // passes, 256 x 256 H4 27.3 -> 23.3 us, 1024 x 1024 H32 71.0 -> 65.4, 4096 x 4096 H32 768 -> 760).  Rows past the end
   // repeat the last one, columns past the head dimension are cleared in the fragment.
   {
-    const uint32_t x_lds = lds_base + kXRows + wave * 8192, y_lds = lds_base + kYRows + wave * 8192;
+    const uint32_t x_lds = lds_base + kXRows + wave * (32 * kRow), y_lds = lds_base + kYRows + wave * (32 * kRow);
     const uint16_t* xsrc = DQ ? p.q + b * p.q_sb + hs * p.q_sh : kp + b * p.k_sb + hs * p.k_sh;
     const uint16_t* ysrc = DQ ? p.dout + b * p.q_sb + hs * p.q_sh : vp + b * p.k_sb + hs * p.k_sh;
     const int64_t st_ss = DQ ? p.q_ss : p.k_ss;
     auto row_of = [&](int u) {                        // row and column of the lane's 16 bytes in copy u
-      const int row = r0 + wave * 32 + 4 * u + (lane >> 4);
+      const int row = r0 + wave * 32 + kRowsPerCopy * u + lane / kLanes;
       return row < n_st ? row : n_st - 1;
     };
-    auto col_of = [&](int u) { return ((lane & 15) ^ lds_row_swizzle(4 * u + (lane >> 4))) * 8; };
+    auto col_of = [&](int u) { return ((lane % kLanes) ^ swz(kRowsPerCopy * u + lane / kLanes)) * 8; };
+    constexpr int kCopies = 32 / kRowsPerCopy;
     auto copy_rows = [&](const uint16_t* src, uint32_t dst) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
+      for (int u = 0; u < kCopies; ++u) {
         const int col = col_of(u);
         copy16_to_lds(src + (int64_t)row_of(u) * st_ss + (col < p.D ? col : 0), dst + u * 1024);
       }
@@ -508,12 +520,12 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     };
     // Pin the fragments (the copies are invisible to the compiler's wait counting).  The dK / dV pass keeps these
     // MFMA operands in accumulation registers: its arithmetic registers are needed for the tiles of T1 / T2 that
-    // the vector unit works on.  The dQ pass at two wavefronts per SIMD uses no accumulation registers at all (a
-    // kernel that does gets its 256 registers split 128 / 128).
+    // the vector unit works on.  At two wavefronts per SIMD -- the dQ pass, 64 columns -- no accumulation registers are used
+    // at all (a kernel that does gets its 256 registers split 128 / 128).
     auto pin = [&]() {
 #pragma unroll
       for (int ks = 0; ks < KK; ++ks) {
-        if (DQ) { asm volatile("" : "+v"(xf[ks])); asm volatile("" : "+v"(yf[ks])); }
+        if (DQ || KK == 4) { asm volatile("" : "+v"(xf[ks])); asm volatile("" : "+v"(yf[ks])); }
         else { asm volatile("" : "+a"(xf[ks])); asm volatile("" : "+a"(yf[ks])); }
       }
     };
@@ -525,9 +537,9 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
       copy_rows(ysrc, y_lds);
       copy_rows(xsrc, x_lds);
       const uint16_t* osrc = p.out + b * p.o_sb + hs * p.o_sh;
-      bf16x8 o8[8];
+      bf16x8 o8[kCopies];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
+      for (int u = 0; u < kCopies; ++u) {
         const int col = col_of(u);
         o8[u] = bf16x8{};
         if (col < p.D) o8[u] = *reinterpret_cast<const bf16x8*>(osrc + (int64_t)row_of(u) * p.o_ss + col);
@@ -536,19 +548,21 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
       const int64_t r = ((int64_t)b * p.Hq + hs) * p.Sq + row;
       const float l = p.lse[r];
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      // Lane (g, i) of four groups of 16 has columns of row 4 u + g of out and dout in copy u: the sum over the group is
-      // the row's delta, left in all of its lanes; lane i keeps the one of copy i % 8, and lane ln fetches row ln's.
+      // Lane (g, i) of four groups of 16 (64 columns: eight of 8) has columns of row 4 u + g (8 u + g) of out and dout in copy
+      // u: the sum over the group is the row's delta, left in all of its lanes; lane i keeps the one of copy i % 8
+      // (i % 4), and lane ln fetches row ln's.
       float mine = 0.f;
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
+      for (int u = 0; u < kCopies; ++u) {
         const bf16x8 d8 = *(lds_bf16x8)(uintptr_t)(y_lds + u * 1024 + lane * 16);
         float part = 0.f;
 #pragma unroll
         for (int j = 0; j < 8; ++j) part = __builtin_fmaf((float)d8[j], (float)o8[u][j], part);
-        part = row16_sum(part);
-        mine = (lane & 7) == u ? part : mine;
+        part = kLanes == 16 ? row16_sum(part) : row8_sum(part);
+        mine = lane % kCopies == u ? part : mine;
       }
-      const float delta = __int_as_float(__builtin_amdgcn_ds_bpermute((((ln & 3) << 4) | (ln >> 2)) << 2, __float_as_int(mine)));
+      const int holder = ln % kRowsPerCopy * kLanes + ln / kRowsPerCopy;
+      const float delta = __int_as_float(__builtin_amdgcn_ds_bpermute(holder << 2, __float_as_int(mine)));
       read_rows(y_lds, yf);
       read_rows(x_lds, xf);
       pin();
@@ -565,7 +579,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     } else if (ntiles > 0) {
       constexpr bool kEarly = WAVES == 4;            // stage 1 is not part of the rows' places
       const int64_t r = DQ ? ((int64_t)b * p.Hq + hs) * p.Sq + (my_r < n_st ? my_r : n_st - 1) : 0;
-      const uint32_t ld_lds = lds_base + kSmemBytesOf<true, 4> + wave * 256;     // 32 rows' lse2, then their delta
+      const uint32_t ld_lds = lds_base + kSmemBytesOf<true, 4, KK> + wave * 256;     // 32 rows' lse2, then their delta
       if (DQ && !kEarly) {
         lse2_lane = p.lse2[r];
         delta_lane = p.delta[r];
@@ -682,6 +696,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   auto write_out = [&](const f32x16 (&acc)[DB], float mul, uint16_t* dst, int64_t d_sb, int64_t d_ss,
                        int64_t d_sh, int head) {
     __syncthreads();
+    constexpr int kOStride = kRow / 2 + 8;
     unsigned char* os = smem + wave * (32 * kOStride * 2);
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -705,12 +720,13 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
       }
     }
   };
-  // The same with fp32 rows on the way (512 bytes, the 32 chunks of 4 columns swizzled by the row): `finish` gets the
+  // The same with fp32 rows on the way (512 or 256 bytes, their chunks of 4 columns swizzled by the row): `finish` gets the
   // lane's 8 columns of a row, whole rows per instruction.  A lane's own accumulator columns are 16 bytes of 32
   // different rows, which is what reading and writing dq_acc from the accumulators cost.
   auto write_out32 = [&](const f32x16 (&acc)[DB], float mul, auto&& finish) {
     __syncthreads();
-    unsigned char* os = smem + wave * (32 * kD * 4);
+    constexpr int kRow32 = 2 * kRow, kPlaces = kRow32 / 16;
+    unsigned char* os = smem + wave * (32 * kRow32);
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -718,7 +734,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
         f32x4 v;
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = acc[db][4 * g + e] * mul;
-        *reinterpret_cast<f32x4*>(os + ln * 512 + (((db * 8 + g * 2 + hf) ^ ln) << 4)) = v;
+        *reinterpret_cast<f32x4*>(os + ln * kRow32 + (((db * 8 + g * 2 + hf) ^ (ln % kPlaces)) << 4)) = v;
       }
     __syncthreads();
     const int chunk = lane & 15;
@@ -729,7 +745,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
       if (row < n_st && chunk * 8 < p.D) {
         f32x4 v[2];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) v[h] = *reinterpret_cast<const f32x4*>(os + r * 512 + (((2 * chunk + h) ^ r) << 4));
+        for (int h = 0; h < 2; ++h) v[h] = *reinterpret_cast<const f32x4*>(os + r * kRow32 + (((2 * chunk + h) ^ (r % kPlaces)) << 4));
         finish(v, row, chunk * 8);
       }
     }
@@ -782,17 +798,17 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
 }
 
 template <bool DQ, bool CAUSAL, int KK, bool PREPARED>
-__global__ __launch_bounds__(DQ ? 512 : 256, 1) void bwd_main(const BwdParams p, const TileMap w) {
+__global__ __launch_bounds__(DQ ? 512 : 256, !DQ && KK == 4 ? 2 : 1) void bwd_main(const BwdParams p, const TileMap w) {
   constexpr int kWaves = DQ ? 8 : 4;
-  __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<DQ, kWaves>];
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<DQ, kWaves, KK>];
   bwd_pass<DQ, CAUSAL, KK, kWaves, PREPARED, false>(p, w, (int)blockIdx.x, smem);
 }
 
 // Both passes side by side, for launches that leave CUs idle one after the other.
 template <bool CAUSAL, int KK, bool SPLIT>
-__global__ __launch_bounds__(256, 1) void bwd_joint(const BwdParams p, const TileMap wq, const TileMap wk) {
-  __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<false, 4>];
-  static_assert(kSmemBytesOf<true, 4> + 1024 <= kSmemBytesOf<false, 4>, "one array for both, and lse2 and delta of the dQ rows");
+__global__ __launch_bounds__(256, KK == 4 ? 2 : 1) void bwd_joint(const BwdParams p, const TileMap wq, const TileMap wk) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<false, 4, KK>];
+  static_assert(kSmemBytesOf<true, 4, KK> + 1024 <= kSmemBytesOf<false, 4, KK>, "one array for both, and lse2 and delta of the dQ rows");
   const int first_q = wk.per_xcd * 8;         // a multiple of 8: both halves keep their XCDs
   if ((int)blockIdx.x < first_q) bwd_pass<false, CAUSAL, KK, 4, true, SPLIT>(p, wk, (int)blockIdx.x, smem);
   else bwd_pass<true, CAUSAL, KK, 4, true, SPLIT>(p, wq, (int)blockIdx.x - first_q, smem);
@@ -800,8 +816,8 @@ __global__ __launch_bounds__(256, 1) void bwd_joint(const BwdParams p, const Til
 
 // The same for several chunks of a step.  The dQ workgroups, whose chains are the longest, come first.
 template <int KK>
-__global__ __launch_bounds__(256, 1) void bwd_joint_chunks(const BwdParams p, const TileMap wq, const TileMap wk, const Chunks chunks) {
-  __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<false, 4>];
+__global__ __launch_bounds__(256, KK == 4 ? 2 : 1) void bwd_joint_chunks(const BwdParams p, const TileMap wq, const TileMap wk, const Chunks chunks) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<false, 4, KK>];
   const int first_k = wq.per_xcd * 8;
   if ((int)blockIdx.x < first_k) bwd_pass<true, false, KK, 4, true, false, true>(p, wq, (int)blockIdx.x, smem, &chunks);
   else bwd_pass<false, false, KK, 4, true, false, true>(p, wk, (int)blockIdx.x - first_k, smem, &chunks);
@@ -940,7 +956,7 @@ float launch_time(float n, float mean, float most, const Cost& c) {
 // where one workgroup's chain of tiles -- with grouped heads, all query heads of the group -- is what the launch waits for;
 // their sums meet in a third launch (one / with it):
 //     B1 H8/1 512 x 512      82.6 / 27.6     B1 H8/1 2048 x 2048    310 / 73.6     B1 H8/1 4096 x 4096   636 /  221
-//     B1 H2/2 4096 x 4096    85.2 / 69.8     B1 H32/4 2048 x 2048   338 /  220     causal, D 64: H8/1 2048 x 2048  249 / 49.5
+//     B1 H2/2 4096 x 4096    85.2 / 69.8     B1 H32/4 2048 x 2048   338 /  220     causal, D 64: H8/1 2048 x 2048  249 / 45.3
 Cost joint_cost(int D) { return D <= 64 ? Cost{6.f, 0.75f, 0.12f} : Cost{7.f, 1.15f, 0.29f}; }
 struct Plan { bool joint; int sq, sk; float time; };       // time: estimated, without preparing delta and lse2
 constexpr int64_t kPartialMost = int64_t(32) << 20;     // bytes of sums a block may leave for bwd_reduce
@@ -980,7 +996,7 @@ Plan plan_block(int B, int Sq, int Sc, int Hq, int Hkv, int D, bool causal) {
 // long.  Us a step, chunk by chunk / in launches of 2 / 4 / 8:
 //     8 chunks 512 x 512 B4 H5      162 /  117 / 95.8 / 89.5      1024 x 1024 H32                557 /  497 /  465 /  448
 //     256 x 256 H16                 104 / 67.2 / 56.8 / 52.3      512 x 512 H8/1                 201 /  337 /  174 / 90.2
-//     1237 x 1237 B2 H16/8 D80      632 /  605 /  510 /  499      700 x 700 H12 D64              141 /  100 / 82.8 / 72.9
+//     1237 x 1237 B2 H16/8 D80      632 /  605 /  510 /  499      700 x 700 H12 D64              135 / 99.0 / 90.5 / 80.6
 int group_chunks(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks) {
   if (B == 0 || Sq == 0 || Sc == 0) return 1;
   const int64_t nq = tile_map(B * Hq, Sq, kRowsQ / 2).total, nk = tile_map(B * Hkv, Sc, kRowsKv).total;

@@ -70,6 +70,17 @@ __device__ __forceinline__ float row16_sum(float x) {
   return x;
 }
 
+// and over its group of 8
+__device__ __forceinline__ float row8_sum(float x) {
+  auto permuted = [](float v, auto ctrl) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xf, 0xf, false));
+  };
+  x += permuted(x, std::integral_constant<int, 0xb1>{});     // the other of a pair
+  x += permuted(x, std::integral_constant<int, 0x4e>{});     // the other pair of four
+  x += permuted(x, std::integral_constant<int, 0x141>{});    // the other four of eight, mirrored
+  return x;
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 
@@ -167,6 +178,10 @@ inline float rounds_time(float n, float t, const LaunchCost& c) {
 inline float fold_time(int results, int B, int Sq, int Hq, int D) {
   return results > 1 ? 4.f + (results + 1) * (2.f * B * Sq * Hq * D) / 5.3e6f : 0.f;
 }
+
+// The same for rows of 128 bytes (64 bf16), of which two share the 256 bytes that cover all banks: 16 consecutive rows x one
+// chunk take each of the 16 places once, and so do 4 rows x 4 consecutive chunks.
+__device__ __forceinline__ constexpr int lds_half_row_swizzle(int row) { return (((row >> 1) & 1) << 2) | ((row >> 2) & 3); }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 

@@ -110,6 +110,14 @@ def test_backward_block_in_two_launches(D, Sq, Sc, causal):
     _block(2, Sq, Sc, 128, 128, D, causal, launches=2)
 
 
+@pytest.mark.parametrize("D", [8, 24, 64])
+@pytest.mark.parametrize("Sq,Sc,Hq,Hkv,causal", [(449, 385, 24, 24, False), (383, 577, 32, 8, False), (513, 512, 40, 20, True)])
+def test_two_workgroups_on_a_cu(D, Sq, Sc, Hq, Hkv, causal):
+    """64 columns: more workgroups than CUs, so that two of them share a CU's LDS; streams of more tiles than the tile ring
+    has stages, with a last tile of 1, 63 or 64 rows."""
+    _block(2, Sq, Sc, Hq, Hkv, D, causal, launches=taken(2, Sq, Sc, Hq, Hkv, D, causal)[0])
+
+
 @pytest.mark.parametrize("D", [40, 88, 128])
 @pytest.mark.parametrize("B,Sq,Sc,Hq,Hkv,causal", [(1, 321, 130, 8, 1, False), (1, 700, 777, 8, 1, True), (2, 513, 400, 12, 2, True),
                                                    (1, 130, 3000, 1, 1, False), (1, 3000, 130, 1, 1, True)])
