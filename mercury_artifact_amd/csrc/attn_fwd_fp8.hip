@@ -171,10 +171,11 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
   const int k_tile_bytes = (int)(kBN * p.k_ss);
   const int v_tile_bytes = (int)(kBN * p.v_ss);
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem + wave * (kCpy * 1024);
-  // CHAIN: K and V tiles are requested in order; k_off and v_off are the offsets of the next ones inside their chunks.  (The
-  // address of a chunk is loaded inside its branch and waited for there.)
-  const int chunk_bytes = CHAIN ? (int)((uint32_t)((p.Sc + kBN - 1) / kBN) * (uint32_t)k_tile_bytes) : 0;
-  int k_off = 0, v_off = 0, k_chunk = chunk, v_chunk = chunk;
+  // CHAIN: K and V tiles are requested in order; k_off and v_off are the offsets of the next ones inside their chunks, k_pos
+  // and v_pos their numbers (rows may all lie at one place).  (The address of a chunk is loaded inside its branch and waited
+  // for there.)
+  const int chunk_tiles = (p.Sc + kBN - 1) / kBN;
+  int k_off = 0, v_off = 0, k_pos = 0, v_pos = 0, k_chunk = chunk, v_chunk = chunk;
   const int last_chunk = chunk + chunks_left;
   auto enter = [&](u32x4& rs, const uint8_t* base) {
     asm volatile("" : "+s"(base));
@@ -190,17 +191,17 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
   auto chain_k = [&]() {                        // behind the copies of a K tile
     if (!CHAIN) return;
     k_off += k_tile_bytes;
-    if (k_off == chunk_bytes && k_chunk != last_chunk) {
-      k_off = 0;
+    if (++k_pos == chunk_tiles && k_chunk != last_chunk) {
+      k_off = k_pos = 0;
       ++k_chunk;
       enter(krs, p.k[k_chunk] + b * p.k_sb + hk * p.k_sh);
     }
   };
   auto chain_v = [&]() {
     if (!CHAIN) return;
-    v_off += k_tile_bytes;
-    if (v_off == chunk_bytes && v_chunk != last_chunk) {
-      v_off = 0;
+    v_off += v_tile_bytes;
+    if (++v_pos == chunk_tiles && v_chunk != last_chunk) {
+      v_off = v_pos = 0;
       ++v_chunk;
       enter(vrs, p.v[v_chunk] + b * p.v_sb + hk * p.v_sh);
     }

@@ -153,6 +153,23 @@ def test_a_run_of_chunks_needs_one_row_stride_and_no_mask():
     assert call(2, False) is True
 
 
+@pytest.mark.parametrize("fp8,D", [(False, 64), (False, 128), (True, 128)])
+def test_a_run_of_chunks_whose_rows_lie_at_one_place(fp8, D):
+    """Row stride 0 (an expanded chunk): every chunk of the run is visited for all of its keys, bit for bit as where the same
+    keys lie in memory."""
+    g = torch.Generator(device="cuda").manual_seed(21)
+    q = torch.randn(1, 300, 4, D, generator=g, device="cuda")
+    one = [torch.randn(2, 1, 1, 4, D, generator=g, device="cuda") * (i + 1) for i in range(3)]
+    kind = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    q, one, got = q.to(kind), [c.to(kind) for c in one], []
+    descale = torch.ones((), device="cuda") if fp8 else None
+    for chunks in ([c.expand(-1, -1, 200, -1, -1) for c in one], [c.expand(-1, -1, 200, -1, -1).contiguous() for c in one]):
+        out, lse = torch.empty(1, 1, 300, 4, D, dtype=torch.bfloat16, device="cuda"), torch.empty(1, 1, 4, 300, device="cuda")
+        assert N.host.fwd_blocks(q, chunks, 3, 0.125, False, descale, descale, descale, out, lse, 0) is True
+        got.append((out, lse))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 def test_the_only_result_of_a_step_goes_straight_out_unless_the_output_is_read():
     """Steps whose chunks all go into one result write the caller's tensors; an output that lies over the queries or over a
     chunk is written by a fold behind the launch instead."""
