@@ -211,34 +211,54 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
     rs[0] = (uint32_t)(uint64_t)base;
     rs[1] = (uint32_t)((uint64_t)base >> 32) & 0xffffu;
   };
-  auto chain_k = [&]() {                             // behind the copy of a K tile
+  auto cross_k = [&]() {                             // behind the last K tile of a chunk that is not the last one
+    k_off = k_pos = 0;
+    ++k_chunk;
+    enter(krs, p.k[k_chunk] + b * p.k_sb + hk * p.k_sh);
+  };
+  auto cross_v = [&]() {
+    v_off = v_pos = 0;
+    ++v_chunk;
+    enter(vrs, p.v[v_chunk] + b * p.v_sb + hk * p.v_sh);
+  };
+  auto chain_k = [&]() {                             // behind the copy of a K tile of the prologue
     k_off += k_tile_bytes;
-    if (++k_pos == chunk_tiles && k_chunk != last_chunk) {
-      k_off = k_pos = 0;
-      ++k_chunk;
-      enter(krs, p.k[k_chunk] + b * p.k_sb + hk * p.k_sh);
-    }
+    if (++k_pos == chunk_tiles && k_chunk != last_chunk) cross_k();
   };
   auto chain_v = [&]() {
     v_off += v_tile_bytes;
-    if (++v_pos == chunk_tiles && v_chunk != last_chunk) {
-      v_off = v_pos = 0;
-      ++v_chunk;
-      enter(vrs, p.v[v_chunk] + b * p.v_sb + hk * p.v_sh);
+    if (++v_pos == chunk_tiles && v_chunk != last_chunk) cross_v();
+  };
+  // The main loop counts down to the next end of a chunk in either sequence: one test per tile instead of two with their
+  // detours (8 chunks, us: 1237 x 1237 B2 H16/8 D80 in pairs 161 to 152, 2048 x 2048 H16 D64 in fours 147 to 143, 700 x 700 H12
+  // D64 in pairs 27.0 to 26.1; on 128 columns, where the clock decides, no change).
+  int span = 0, till = 0;
+  auto next_end = [&]() {
+    const int k_left = k_chunk != last_chunk ? chunk_tiles - k_pos : 0x7fffffff;
+    const int v_left = v_chunk != last_chunk ? chunk_tiles - v_pos : 0x7fffffff;
+    till = span = k_left < v_left ? k_left : v_left;
+  };
+  auto chain = [&]() {                               // behind the copies of a K and a V tile
+    k_off += k_tile_bytes;
+    v_off += v_tile_bytes;
+    if (__builtin_expect(--till == 0, 0)) {
+      k_pos += span;
+      v_pos += span;
+      if (k_pos == chunk_tiles && k_chunk != last_chunk) cross_k();
+      if (v_pos == chunk_tiles && v_chunk != last_chunk) cross_v();
+      next_end();
     }
   };
   auto copy_k = [&](int t, int stage) {
     const int soff = CHAIN ? k_off : tile_offset(t, k_tile_bytes);
 #pragma unroll
     for (int u = 0; u < kCpy; ++u) copy16_to_lds(krs, lds_base + stage * kTile + u * 1024, kvoff[u], soff);
-    if (CHAIN) chain_k();
   };
   auto copy_v = [&](int t, int stage) {
     const int soff = CHAIN ? v_off : tile_offset(t, v_tile_bytes);
 #pragma unroll
     for (int u = 0; u < kCpy; ++u)
       copy16_to_lds(vrs, lds_base + kVBase + stage * kTile + u * 1024, vvoff[u], soff);
-    if (CHAIN) chain_v();
   };
 
   // K operand of S^T (A, 32 keys x 16 head-dim values): lane (ln, hf) reads chunk 2 kk + hf of row
@@ -479,11 +499,15 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
       // wavefront has its fragments.  Tiles past the chunk arrive as zeros.
       const uint32_t q_lds = lds_smem + (wave < 4 ? 0 : kVBase) + 2 * kTile + (wave & 3) * 8192;
       copy_k(0, 0);
+      if (CHAIN) chain_k();
 #pragma unroll
       for (int u = 0; u < 8; ++u) copy_q(32 * wave + 4 * u, q_lds + u * 1024);
       copy_v(0, 0);
+      if (CHAIN) chain_v();
       copy_k(1, 1);
+      if (CHAIN) chain_k();
       copy_v(1, 1);
+      if (CHAIN) chain_v();
       asm volatile("s_waitcnt vmcnt(%0)" :: "n"(3 * kCpy) : "memory");     // K(0) and Q
       read_q(q_lds);
       // pinned here: otherwise the first use sits inside the main loop and so does the wait for the reads
@@ -491,8 +515,12 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
       for (int kk = 0; kk < KK; ++kk) asm volatile("" : "+v"(qf[kk]));
       __builtin_amdgcn_s_barrier();
       copy_k(2, 2);
+      if (CHAIN) chain_k();
       copy_k(3, 3);
+      if (CHAIN) chain_k();
       copy_v(2, 2);
+      if (CHAIN) chain_v();
+      if (CHAIN) next_end();
       qk();
       sm_mask(0);
       sm_fix(true);
@@ -522,10 +550,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
       if (!kShortMatrix) {
         copy_k(t + 4, t & 3);
         copy_v(t + 3, (t + 3) & 3);
-      } else if (CHAIN) {
-        chain_k();
-        chain_v();
       }
+      if (CHAIN) chain();
       if (t + 2 < ntiles) first_frags();                        // K(t+2), for the next matrix phase
       asm volatile("s_waitcnt vmcnt(4)" ::: "memory");          // the four copies of one tile ago are done
       __builtin_amdgcn_s_barrier();
@@ -783,8 +809,8 @@ int attn_fwd_bf16_plan(int blocks, int B, int Sq, int Sc, int Hq, int D, int64_t
 // estimated time, the fold of the results included (which is nothing where there is only one).  Where the blocks would all
 // run side by side a run of chunks would only make the longest chain longer.  Whole steps of 8 chunks, us, one / two / four /
 // eight chunks to a result: 512 x 512 B4 H5 43.9 / 36.0 / 49.7 / 76.1, 1024 x 1024 H32 148 / 133 / 128 / 154, 2048 x 2048 H32
-// 488 / 471 / 464 / 441, 4096 x 4096 H32 1790 / 1772 / 1761 / 1720, 1237 x 1237 B2 H16/8 D80 161 / 173 / 210 / 172, 700 x 700 H12
-// D64 40.0 / 32.7 / 51.8 / 87.4, 3000 x 3000 H16 D96 414 / 423 / 475 / 440.
+// 488 / 471 / 464 / 441, 4096 x 4096 H32 1790 / 1772 / 1761 / 1720, 1237 x 1237 B2 H16/8 D80 160 / 162 / 195 / 160, 700 x 700 H12
+// D64 35.2 / 31.2 / 50.3 / 85.1, 3000 x 3000 H16 D96 411 / 402 / 438 / 411.
 int attn_fwd_bf16_chain(int n, int B, int Sq, int Sc, int Hq, int D) {
   if (n < 2 || Sc == 0) return 1;
   FwdParams p{};
