@@ -552,7 +552,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
         copy_v(t + 3, (t + 3) & 3);
       }
       if (CHAIN) chain();
-      if (t + 2 < ntiles) first_frags();                        // K(t+2), for the next matrix phase
+      // K(t+2), for the next matrix phase; a chain also reads them where there is none: without the branch its D 64 loop takes
+      // 6 % less (2 chunks of 4096 keys, 8192 rows H32: 579 us to 547) and the others 0.4 %, a lone block's 6 % more
+      if (CHAIN || t + 2 < ntiles) first_frags();
       asm volatile("s_waitcnt vmcnt(4)" ::: "memory");          // the four copies of one tile ago are done
       __builtin_amdgcn_s_barrier();
     }
@@ -809,8 +811,8 @@ int attn_fwd_bf16_plan(int blocks, int B, int Sq, int Sc, int Hq, int D, int64_t
 // estimated time, the fold of the results included (which is nothing where there is only one).  Where the blocks would all
 // run side by side a run of chunks would only make the longest chain longer.  Whole steps of 8 chunks, us, one / two / four /
 // eight chunks to a result: 512 x 512 B4 H5 43.9 / 36.0 / 49.7 / 76.1, 1024 x 1024 H32 148 / 133 / 128 / 154, 2048 x 2048 H32
-// 488 / 471 / 464 / 441, 4096 x 4096 H32 1790 / 1772 / 1761 / 1720, 1237 x 1237 B2 H16/8 D80 160 / 162 / 195 / 160, 700 x 700 H12
-// D64 35.2 / 31.2 / 50.3 / 85.1, 3000 x 3000 H16 D96 411 / 402 / 438 / 411.
+// 488 / 471 / 464 / 441, 4096 x 4096 H32 1790 / 1772 / 1761 / 1720, 1237 x 1237 B2 H16/8 D80 168 / 167 / 199 / 163, 700 x 700 H12
+// D64 36.2 / 29.2 / 45.4 / 75.2, 3000 x 3000 H16 D96 433 / 424 / 455 / 432.
 int attn_fwd_bf16_chain(int n, int B, int Sq, int Sc, int Hq, int D) {
   if (n < 2 || Sc == 0) return 1;
   FwdParams p{};
@@ -824,10 +826,11 @@ int attn_fwd_bf16_chain(int n, int B, int Sq, int Sc, int Hq, int D) {
   for (int results = n; results >= 1; --results) {
     const int per = (n + results - 1) / results;
     if (per == 1 || (n + per - 1) / per != results) continue;
-    // (a chain's tiles take a little longer: its launch has no pauses in which the clock recovers)
+    // (a chain's tiles take a little longer: as one chunk of twice the keys, 2 x 4096 keys take 1.2 % more on 128 columns, up
+    // to 4 % on 64, and its launch has no pauses in which the clock recovers)
     LaunchCost c = costs(D)[0];
-    c.step *= D > 96 ? 1.05f : 1.08f;
-    c.busy *= D > 96 ? 1.05f : 1.08f;
+    c.step *= D > 96 ? 1.03f : 1.05f;
+    c.busy *= D > 96 ? 1.03f : 1.05f;
     const float time = rounds_time(wgs * results, (float)per * ((Sc + kBN - 1) / kBN), c) + fold_time(results, B, Sq, Hq, D);
     if (time < best_time) { best_time = time; best = per; }
   }
