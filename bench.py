@@ -3,11 +3,11 @@
 
 Workload = the headline bf16 configuration: batch 1, 32 heads, head dim 128, local Q of 4096 rows, 8 KV chunks
 of 4096 rows (32768 keys), non-causal, N(0,1) inputs cast to bf16, softmax scale 128^-0.5.
-A step = 8 block-forward kernels + ONE fold of the 8 block results into the bf16 output and the (B,H,S) LSE
-(the ring drivers' default: the fold is associative, so the chain of 7 LSE merges and the epilogue copies of
-the generated code collapse into one pass over the block outputs; that literal chain is timed beside it),
-driven through the same block operator Mercury's generated code calls.  Inputs are resident in HBM before
-the timed region.  Prints ONE JSON line.
+A step = the ring driver's default on a ring whose chunks are all in memory: ONE launch of the forward kernel whose
+workgroups visit the 8 chunks one after the other and write the bf16 output and the (B,H,S) LSE (drivers on other
+rings launch a block per chunk and fold the results in one pass; the generated code's literal chain of block
+operators and LSE merges, and its fold, are timed beside it).  Inputs are resident in HBM before the timed region.
+Prints ONE JSON line.
 """
 from __future__ import annotations
 
@@ -24,7 +24,7 @@ PEAK_BF16_TFLOPS = 2500.0      # MI355X dense bf16 MFMA
 PEAK_HBM_GBS = 8000.0          # MI355X HBM3E
 # HBM bytes per launch from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of this script, each counter scaled
 # by its reading for the calibration launch at the end of main() (profiles/ring_step_config1_hbm_traffic.md)
-TRAFFIC_FWD_BYTES = 134.9e6
+TRAFFIC_FWD_BYTES = 604.7e6
 TRAFFIC_MERGE_BYTES = 171.5e6
 TRAFFIC_MANY_BYTES = 321.0e6
 
@@ -217,7 +217,6 @@ def main() -> int:
     import torch
 
     import mercury_artifact_amd as M
-    from mercury_artifact_amd import flash_attn_interface as FI
     from mercury_artifact_amd import merge as MG
 
     if not torch.cuda.is_available():
@@ -233,12 +232,12 @@ def main() -> int:
     scale = D ** -0.5
 
     # per-kernel durations: HIP events on the stream the kernels are launched on (torch's current one), inside
-    # the timed region.  An event pair costs a few microseconds of stream time, so each step brackets ONE of its
-    # forward launches (rotating through the chunks) and the fold; the literal chain further down brackets ONE
-    # of its plain merges per step.
-    fwd_events, merge_events = [], []
-    real_fwd, real_merge = FI.attn_fwd_block, MG.merge_into
-    recording = {"on": False, "step": 0, "fwd": 0, "merge": 0}
+    # the timed region.  An event pair costs a few microseconds of stream time: each step brackets its forward
+    # launch (over all chunks); the fold is timed on its own further down, and the literal chain brackets ONE of
+    # its plain merges per step.
+    fwd_events, chunks_timed, merge_events = [], [], []
+    real_merge = MG.merge_into
+    recording = {"on": False, "step": 0, "merge": 0}
 
     def timed(real, bucket, kind, per_step, eligible):
         def wrapper(*a, **kw):
@@ -256,25 +255,30 @@ def main() -> int:
             return r
         return wrapper
 
-    FI.attn_fwd_block = timed(real_fwd, fwd_events, "fwd", W, lambda a: True)
+    class Host:                                # the driver's compiled calls, with its forward launches bracketed
+        def __init__(self, real):
+            self.real = real
+
+        def __getattr__(self, name):
+            return getattr(self.real, name)
+
+        def fwd_blocks(self, *a):
+            if not recording["on"]:
+                return self.real.fwd_blocks(*a)
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            r = self.real.fwd_blocks(*a)
+            e1.record()
+            fwd_events.append((e0, e1))
+            chunks_timed.append(len(a[1]))
+            return r
+
+    from mercury_artifact_amd import _native as N
+
+    N.lib()                                    # loads and binds the compiled calls
+    real_host, N.host = N.host, Host(N.host)
     # plain merges only (they run in the literal chain timed further down): the first call is a cast
     MG.merge_into = timed(real_merge, merge_events, "merge", W - 1, lambda a: a[0] is not None and a[4] is not None)
-
-    many_events = []
-    real_many = MG.merge_many
-
-    def timed_many(*a, **kw):
-        if not recording["on"]:
-            return real_many(*a, **kw)
-        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        e0.record()
-        r = real_many(*a, **kw)
-        e1.record()
-        many_events.append((e0, e1))
-        return r
-
-    from mercury_artifact_amd import ring as RG
-    RG.merge_many = timed_many
 
     def step(literal=False):
         ring = M.LocalRing((W,), rank, kvs)
@@ -287,7 +291,7 @@ def main() -> int:
     recording["on"] = True
     t0 = time.perf_counter()
     for i in range(args.steps):
-        recording.update(step=i, fwd=0, merge=0)
+        recording.update(step=i)
         step()
     torch.cuda.synchronize()
     dt = time.perf_counter() - t0
@@ -316,9 +320,25 @@ def main() -> int:
     value = flops_per_step / (ms_per_step * 1e-3) / 1e12
 
     fwd_ms = sum(e0.elapsed_time(e1) for e0, e1 in fwd_events) / max(len(fwd_events), 1)
-    fwd_tflops = flops_per_block / (fwd_ms * 1e-3) / 1e12
+    fwd_tflops = flops_per_block * sum(chunks_timed) / len(chunks_timed) / (fwd_ms * 1e-3) / 1e12
+    N.host = real_host
     rows = B * Sq * H
     many_bytes = rows * (W * (D * 2 + 4) + D * 2 + 4)
+    # the fold of 8 block results, each behind the block forward that made the last of them
+    results = [M.attn_fwd_block(q, c[0], c[1], scale) for c in kvs]
+    many_events = []
+    for _ in range(2):
+        M.merge_many([x[0] for x in results], [x[1] for x in results], o, lse)
+    torch.cuda.synchronize()
+    for _ in range(args.steps):
+        M.attn_fwd_block(q, kvs[-1][0], kvs[-1][1], scale, out=results[-1][0], lse=results[-1][1])
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        e0.record()
+        M.merge_many([x[0] for x in results], [x[1] for x in results], o, lse)
+        e1.record()
+        many_events.append((e0, e1))
+    torch.cuda.synchronize()
+    del results
     many_ms = sum(e0.elapsed_time(e1) for e0, e1 in many_events) / max(len(many_events), 1)
     many_gbs = many_bytes / (many_ms * 1e-3) / 1e9
 
@@ -331,7 +351,7 @@ def main() -> int:
     recording["on"] = True
     t0 = time.perf_counter()
     for i in range(args.steps):
-        recording.update(step=i, fwd=W + 1, merge=0)      # forward launches are not sampled again
+        recording.update(step=i, merge=0)
         step(True)
     torch.cuda.synchronize()
     unfused_ms = (time.perf_counter() - t0) / args.steps * 1e3
@@ -359,7 +379,7 @@ def main() -> int:
     # the drop-in boundary itself: a step function spelled the way the generator spells it (bare names resolved in
     # the exec namespace, update_out_and_lse per chunk, the two epilogue stores), run unchanged in
     # namespace(lazy_merge=True), where the merges of the step are recorded and folded once by the epilogue
-    FI.attn_fwd_block, MG.merge_into, RG.merge_many = real_fwd, real_merge, real_many
+    MG.merge_into = real_merge
     drop_in_ms = {}
     for lazy in (False, True):
         ring_box = {}
@@ -380,7 +400,7 @@ def main() -> int:
         torch.cuda.synchronize()
         drop_in_ms[lazy] = (time.perf_counter() - t0) / args.steps * 1e3
 
-    # the same step replayed as one HIP graph (one launch instead of ~25; identical kernels and results)
+    # the same step replayed as one HIP graph (identical kernels and results)
     graph_ms, graph_same = None, None
     try:
         graphed = M.GraphedStep(step)
@@ -397,7 +417,7 @@ def main() -> int:
     except RuntimeError as exc:      # reported, never fatal for the headline number
         print(f"bench.py: graph replay skipped: {exc}", file=sys.stderr)
 
-    # the same step with every other block launch on a second stream (the driver's two_streams option): the tail
+    # the step with a launch per block, every other one on a second stream (the driver's two_streams option): the tail
     # of one launch overlaps the head of the next.  Reported next to the headline, not part of it: per-launch
     # durations cannot be bracketed in this mode.
     def step_two_streams():
@@ -405,10 +425,15 @@ def main() -> int:
 
     two_streams_ms, two_same = None, None
     if not args.no_variants:                 # overlapping launches would spoil a profiler's per-kernel averages
+        class Hops(M.LocalRing):               # chunks hop by hop: a block launch each on one stream
+            pass
+
+        M.flash_attn_pack_kv(q, kvs[rank], o, lse, scale, ring=Hops((W,), rank, kvs))
+        one_o, one_lse = o.clone(), lse.clone()
         for _ in range(3):
             step_two_streams()
         torch.cuda.synchronize()
-        two_same = bool(torch.equal(o, eager_o) and torch.equal(lse, eager_lse)) if graph_same is not None else None
+        two_same = bool(torch.equal(o, one_o) and torch.equal(lse, one_lse))
         t0 = time.perf_counter()
         for _ in range(args.steps):
             step_two_streams()
@@ -454,7 +479,7 @@ def main() -> int:
         "dtype": "bf16",
         "data": "synthetic",
         "config": {"workload": "headline bf16 configuration: non-causal MHA, B1 H32 D128, local Q 4096 x 8 KV chunks "
-                               "of 4096 (single ring, rank 0), 8 block forwards + one fold of the 8 block results",
+                               "of 4096 (single ring, rank 0), one forward launch over the 8 chunks",
                    "flops_per_step": flops_per_step, "pct_of_bf16_mfma_peak": round(100 * value / PEAK_BF16_TFLOPS, 2),
                    "literal_merge_chain_ms_per_step": round(unfused_ms, 4),
                    "generated_text_ms_per_step": round(drop_in_ms[False], 4),
