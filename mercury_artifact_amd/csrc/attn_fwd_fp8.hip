@@ -261,12 +261,12 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
   for (int i = 0; i < DB; ++i)
 #pragma unroll
     for (int j = 0; j < 16; ++j) o_acc[i][j] = 0.f;
-  // m_ref: the raw score the exponentials of this lane's Q row are taken relative to.  It is set to the first
-  // tile's row maximum and moves only when a later tile would overflow e4m3: what is watched is the sum of each
-  // group of 16 exponentials (one compare per tile), not the maxima.  A group sum below 448 means every 2^4 P in
-  // it is below the e4m3 maximum; P = 1 for all 16 gives 256.  When a sum reaches 448 the reference moves up to
-  // the row maximum seen so far (O and the running sum are rescaled) and the tile's exponentials are redone, after
-  // which every 2^4 P is at most 16.
+  // m_ref: the raw score the exponentials of this lane's Q row are taken relative to.  It is set to the first tile's row
+  // maximum and moves up only when a later half tile would overflow e4m3: what is watched are the sums of its two groups of
+  // 16 exponentials (one compare each), not the maxima.  A group sum below 448 means every 2^4 P in it is below the e4m3
+  // maximum; P = 1 for all 16 gives 256.  When a sum reaches 448 the reference moves up to the largest score of the half
+  // (O and the running sum are rescaled) and the half's exponentials are redone, after which every 2^4 P is at most 16.  In a
+  // run of chunks it also moves, in either direction, where a chunk begins (enter_chunk).
   float m_ref = 0.f, msc = -kPShift, l_run = 0.f;      // l_run sums 2^4 P (this lane's half of the keys)
   const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   f32x16 sa[2], sb[2];       // S^T of a tile's first and second half: 64 keys x 32 q rows per wavefront each
@@ -462,10 +462,11 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
     mask_half(sa, chain_kv0);
     mask_half(sb, chain_kv0 + kBN / 2);
     const float mx = pair_max(fmaxf(largest(sa), largest(sb)));
-    // (down by 2^60 at most: beyond that the chunk adds nothing, and O has to stay finite)
-    const float grown = (mx - m_ref) * scale_log2;
-    const bool move = mx != -INFINITY && grown > -60.f;               // false for NaN
-    const float alpha = move ? fast_exp2(-grown) : 1.f;
+    // Down only as far as the row's sum stays below 2^64, over however many chunks, and with it O, of which no element is
+    // larger than 448 times the sum.  A chunk that is not followed is 2^40 below what the row has: it adds nothing.
+    const float down = fast_exp2((m_ref - mx) * scale_log2);
+    const bool move = mx != -INFINITY && pair_sum(l_run) * down < 0x1p64f;      // false for NaN
+    const float alpha = move ? down : 1.f;
     l_run *= alpha;
 #pragma unroll
     for (int db = 0; db < DB; ++db)

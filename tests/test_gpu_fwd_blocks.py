@@ -1,4 +1,6 @@
 """Several block forwards of a step in one launch (mhip_attn_fwd_blocks) against the oracle, and which rings get them."""
+import math
+
 import pytest
 import torch
 
@@ -217,3 +219,68 @@ def test_e4m3_chunks_of_one_result_match_the_oracle(n, per, B, Sq, Sc, Hq, Hkv, 
         assert ((got - ro).abs() - (bound + 2 ** -8 * ro.abs())).max().item() <= 2e-3, i
         assert (got - ro).norm() <= 6e-2 * ro.norm(), i
         assert ((lses[i].cpu() - rl).abs() / rl.abs().clamp_min(1.0)).max().item() <= 1e-3, i
+
+
+# row maxima of a run's chunks against those of the first one, in factors of 2
+LEVELS = {"2 x -58": [0, -58, -116], "3 x -40": [0, -40, -80, -120], "4 x -45": [0, -45, -90, -135, -180],
+          "7 x -17": [-17 * i for i in range(8)], "15 x -8": [-8 * i for i in range(16)], "2 x -70": [0, -70, -140],
+          "7 x +17": [17 * i for i in range(8)], "fall, climb": [0, -58, -116, -30, 0, 3], "climb, fall": [-60, 0, 60, 2, -58, -118],
+          "zigzag": [0, -50, 0, -50, 2, -59, 2, -59]}
+
+
+def _levelled(name, B, Sq, Sc, Hq, D, fp8, scale):
+    """Inputs whose scores lie around LEVELS[name] (natural units: times log 2), chunk by chunk: 16 columns of q are 4, and
+    those of a chunk's keys alike."""
+    levels = LEVELS[name]
+    g = torch.Generator().manual_seed(len(levels) * 100 + Sq)
+    q = torch.randn(B, Sq, Hq, D, generator=g)
+    chunks = [torch.randn(2, B, Sc, Hq, D, generator=g) for _ in levels]
+    q[..., :16] = 4.0
+    for c, level in zip(chunks, levels):
+        c[0][..., :16] = level * math.log(2) / scale / 64.0
+    if not fp8:
+        return q.bfloat16(), [c.bfloat16() for c in chunks], None, None, None
+    top = [max(c[j].abs().max() for c in chunks) / 448.0 for j in (0, 1)]
+    (qq, sq) = O.quantize_e4m3(q)
+    return qq, [torch.stack([c[j] / top[j] for j in (0, 1)]).clamp(-448, 448).to(torch.float8_e4m3fn) for c in chunks], sq, *top
+
+
+@pytest.mark.parametrize("name", LEVELS)
+@pytest.mark.parametrize("B,Sq,Sc,Hq,D", [(1, 70, 200, 2, 128), (1, 130, 130, 130, 128), (1, 100, 300, 3, 64), (1, 33, 64, 2, 96)])
+def test_e4m3_runs_of_chunks_whose_scores_fall_and_climb(name, B, Sq, Sc, Hq, D):
+    """The reference of a row moves in both directions where a chunk begins, over a run by far more than fp32 has room for: the
+    sum and O stay finite and what is left out is nothing.  With workgroups of four and (130 heads) of eight wavefronts.
+    Bounds as above."""
+    scale = D ** -0.5
+    q, chunks, sq, sk, sv = _levelled(name, B, Sq, Sc, Hq, D, True, scale)
+    n = len(chunks)
+    print(f"e4m3 levels {name} B{B} Sq{Sq} Sc{Sc} H{Hq} D{D}", flush=True)
+    assert N.lib().mhip_attn_fwd_plan(B, Sq, Sc, Hq, D, D, D, 0, N.MHIP_E4M3) == (8 if Hq == 130 else 4)
+    out, lse = torch.empty(1, B, Sq, Hq, D, dtype=torch.bfloat16, device="cuda"), torch.empty(1, B, Hq, Sq, device="cuda")
+    ds = [t.cuda().reshape(()) for t in (sq, sk, sv)]
+    assert N.host.fwd_blocks(q.cuda(), [c.cuda() for c in chunks], n, scale, False, *ds, out, lse, 0) is True
+    torch.cuda.synchronize()
+    assert torch.isfinite(out.float()).all() and torch.isfinite(lse).all()
+    ops = [O.dequantize(q, sq)] + [torch.cat([O.dequantize(c[j], s) for c in chunks], 1) for j, s in ((0, sk), (1, sv))]
+    ro, rl = O.block_attention(*ops, scale)
+    bound = O.e4m3_p_rounding_bound(*ops, scale)
+    got = out[0].float().cpu()
+    assert ((got - ro).abs() - (bound + 2 ** -8 * ro.abs())).max().item() <= 2e-3
+    assert (got - ro).norm() <= 6e-2 * ro.norm()
+    assert ((lse[0].cpu() - rl).abs() / rl.abs().clamp_min(1.0)).max().item() <= 1e-3
+
+
+@pytest.mark.parametrize("name", LEVELS)
+@pytest.mark.parametrize("B,Sq,Sc,Hq,D", [(1, 70, 200, 2, 128), (1, 300, 65, 3, 64)])
+def test_runs_of_chunks_whose_scores_fall_and_climb(name, B, Sq, Sc, Hq, D):
+    """The same in bf16, where the reference only moves up: chunks far below it add nothing.  Bounds as above."""
+    scale = D ** -0.5
+    q, chunks, *_ = _levelled(name, B, Sq, Sc, Hq, D, False, scale)
+    out, lse = torch.empty(1, B, Sq, Hq, D, dtype=torch.bfloat16, device="cuda"), torch.empty(1, B, Hq, Sq, device="cuda")
+    assert N.host.fwd_blocks(q.cuda(), [c.cuda() for c in chunks], len(chunks), scale, False, None, None, None, out, lse, 0) is True
+    torch.cuda.synchronize()
+    ro, rl = O.block_attention(q.float(), *(torch.cat([c[j] for c in chunks], 1).float() for j in (0, 1)), scale)
+    got = out[0].float().cpu()
+    assert ((got - ro).abs() - 2 ** -8 * ro.abs()).max().item() <= 2e-2
+    assert (got - ro).norm() <= 1e-2 * ro.norm()
+    assert ((lse[0].cpu() - rl).abs() / rl.abs().clamp_min(1.0)).max().item() <= 1e-3
