@@ -311,6 +311,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
   float l_run = 0.f;         // this lane's share of the running sum (the other 32 keys: lane ^ 32)
   constexpr float kTrigger = 1048576.f;   // a lane's 32 exponentials of one tile sum to less than this, or
   constexpr float kSlack = 14.f;          // rows whose maximum exceeds the reference by 2^kSlack move it
+  constexpr float kNoScore = -0x1p64f;    // the reference of a row whose first tile holds scores of -inf only
   const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   f32x16 s[MB];              // S^T tile: BN keys x 32 q rows per wave
   u32x4 pw[2 * MB];          // P^T of the current tile as packed bf16 B operands, one per k-step
@@ -387,8 +388,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
 #pragma unroll
       for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[mb][j]);
     mx = pair_max(mx);
-    const float grown = (mx - m_ref) * scale_log2;               // NaN when mx = -inf on the first tile
-    const bool move = first ? (mx != -INFINITY) : (grown > kSlack);   // false for NaN
+    const float grown = (mx - m_ref) * scale_log2;
+    const bool move = first || grown > kSlack;                   // false for NaN
     if (!first) {
       const float alpha = move ? fast_exp2(-grown) : 1.f;
 #pragma unroll
@@ -397,7 +398,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const FwdPa
         for (int j = 0; j < 16; ++j) o_acc[db][j] *= alpha;
       l_run *= alpha;
     }
-    m_ref = move ? mx : m_ref;
+    // (with scores of -inf alone it stays below any other score, so that the first key that counts moves it)
+    if (move) m_ref = first ? fmaxf(mx, kNoScore) : mx;
     nmsc = -m_ref * scale_log2;
   };
   // slot of the matrix phase after which early pair idx runs: k-step idx / 4 of the tile before is read by the

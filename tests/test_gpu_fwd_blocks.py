@@ -284,3 +284,28 @@ def test_runs_of_chunks_whose_scores_fall_and_climb(name, B, Sq, Sc, Hq, D):
     assert ((got - ro).abs() - 2 ** -8 * ro.abs()).max().item() <= 2e-2
     assert (got - ro).norm() <= 1e-2 * ro.norm()
     assert ((lse[0].cpu() - rl).abs() / rl.abs().clamp_min(1.0)).max().item() <= 1e-3
+
+
+@pytest.mark.parametrize("fill", [float("-inf"), torch.finfo(torch.bfloat16).min])
+@pytest.mark.parametrize("n,Sc,D", [(2, 200, 128), (3, 64, 64), (4, 100, 96)])
+def test_a_run_that_begins_with_hidden_chunks(fill, n, Sc, D):
+    """Keys of -inf or of the type's lowest value in every chunk but the last, whose scores are all far below zero: the
+    attention over the last chunk.  (The scores are -inf: no product of q is negative, and lowest values add up to it.)  One
+    rounding of P and of the result."""
+    g = torch.Generator().manual_seed(n * 10 + D)
+    q = (torch.rand(1, 130, 2, D, generator=g) + 0.5).bfloat16()
+    chunks = [torch.randn(2, 1, Sc, 2, D, generator=g) for _ in range(n)]
+    for c in chunks[:-1]:
+        c[0] = fill
+    scale = D ** -0.5
+    chunks[-1][0] -= 200.0 / scale / D
+    chunks = [c.bfloat16() for c in chunks]
+    ro, rl = O.block_attention(q.float(), chunks[-1][0].float(), chunks[-1][1].float(), scale)
+    assert rl.max() < -100
+    out, lse = torch.empty(2, *q.shape, dtype=torch.bfloat16, device="cuda"), torch.empty(2, 1, 2, 130, device="cuda")
+    assert N.host.fwd_blocks(q.cuda(), [c.cuda() for c in chunks], n, scale, False, None, None, None, out, lse, 0) is True
+    assert N.host.fwd_blocks(q.cuda(), [torch.cat(chunks, 2).cuda()], 1, scale, False, None, None, None, out, lse, 1) is True
+    torch.cuda.synchronize()
+    for i in range(2):                   # the run, and its keys as one block (whose workgroups split them)
+        assert ((lse[i].cpu() - rl).abs() / rl.abs()).max().item() <= 1e-3, i
+        assert ((out[i].float().cpu() - ro).abs() - 2 ** -8 * ro.abs()).max().item() <= 2e-2, i
