@@ -116,11 +116,10 @@ def _block_results(n, q, kv, *args, **kwargs):
 class _Together:
     """Block forwards of one query tensor over ``n`` chunks of a ring whose chunks are all there, several to a launch
     (mhip_attn_fwd_group) and, where that is faster, a run of chunks to a result (mhip_attn_fwd_chain).  ``size``, the
-    chunks of a launch, is 1 where every block goes its own way.  With ``into`` = (o, lse) a single result is written
-    there if neither overlaps anything the launch reads."""
+    chunks of a launch, is 1 where every block goes its own way."""
 
     def __init__(self, n, q, kv, ring, softmax_scale, dropout_p, causal, window_size, alibi_slopes, q_descale=None, k_descale=None,
-                 v_descale=None, into=None):
+                 v_descale=None):
         self.size = self.per = 1
         if (n < 2 or not type(ring).__dict__.get("resident")
                 or not _straight(q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes, q_descale=q_descale,
@@ -129,34 +128,33 @@ class _Together:
         self.per = 1 if causal else N.host.fwd_chain(q, kv, n) or 1
         launches = -(-n // MAX_GROUP) if self.per > 1 else 0
         self.size = -(-n // launches) if launches else N.host.fwd_group(q, n) or 1
-        if self.size < 2:
-            return
         self.q, self.args = q, (softmax_scale, causal, q_descale, k_descale, v_descale)
-        total = n if self.per == 1 else sum(-(-min(self.size, n - at) // self.per) for at in range(0, n, self.size))
-        self.direct = False
-        if total == 1 and into is not None:
-            read = [t for t in (q, kv, *(ring.chunks or ()), q_descale, k_descale, v_descale) if t is not None]
-            self.direct = N.host.apart(into[0], into[1], *read) is True and N.host.apart(into[1], *read) is True
-        self.outs, self.lses = (into[0][None], into[1][None]) if self.direct else _result_places(total, q)
+        self.results = n if self.per == 1 else sum(-(-min(self.size, n - at) // self.per) for at in range(0, n, self.size))
 
-    def run(self, chunks):
-        """The (out, lse) results over the step's chunks, in two lists (or tensors stacked alike)."""
+    def run(self, chunks, places=None):
+        """The (out, lse) results over the step's chunks, in two lists or, all of them, as the tensors of ``places``."""
+        outs, lses = places or _result_places(self.results, self.q)
         done, apart = 0, None                   # apart: results of launches whose chunks were not of one layout
         for at in range(0, len(chunks), self.size):
             part = chunks[at:at + self.size]
-            if apart is None and N.host.fwd_blocks(self.q, part, self.per, *self.args, self.outs, self.lses, done) is True:
+            if apart is None and N.host.fwd_blocks(self.q, part, self.per, *self.args, outs, lses, done) is True:
                 done -= -len(part) // self.per
                 continue
             if apart is None:
-                apart = list(zip(self.outs[:done].unbind(0), self.lses[:done].unbind(0)))
-                self.direct = False
+                apart = list(zip(outs[:done].unbind(0), lses[:done].unbind(0)))
             apart += [_ops.attn_fwd_block(self.q, c[0], c[1], *self.args) for c in part]
-        return (self.outs, self.lses) if apart is None else ([r[0] for r in apart], [r[1] for r in apart])
+        return (outs, lses) if apart is None else ([r[0] for r in apart], [r[1] for r in apart])
 
     def step(self, chunks, o, lse):
-        """The whole step: results and, unless the only one was written straight out, their fold."""
-        outs, lses = self.run(chunks)
-        if self.direct or N.host.merge_many(outs, lses, o, lse, None) is not None:
+        """The whole step: results and their fold.  A single result is written straight to ``o`` and ``lse`` if neither overlaps
+        anything the launch reads."""
+        places = None
+        if self.results == 1:
+            read = [t for t in (self.q, *chunks, *self.args[2:]) if t is not None]
+            if N.host.apart(o, lse, *read) is True and N.host.apart(lse, *read) is True:
+                places = o[None], lse[None]
+        outs, lses = self.run(chunks, places)
+        if (places and outs is places[0]) or N.host.merge_many(outs, lses, o, lse, None) is not None:
             return
         merge_many(list(outs), list(lses), o, lse)
 
@@ -244,7 +242,7 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
     places = [None] * n_blocks
     # (a divided ring is one that wants to hold little of other ranks' keys at a time)
     if defer and not two_streams and ring_divide == 1:
-        together = _Together(n_blocks, q, kv, ring, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra, into=(o, lse))
+        together = _Together(n_blocks, q, kv, ring, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra)
         if together.size > 1:
             together.step(_resident_chunks(ring, kv), o, lse)
             return
@@ -371,7 +369,7 @@ def flash_attn_expose_reduce(q, kv, o, lse, softmax_scale, dropout_p=0, causal=F
              and o.is_contiguous() and lse.is_contiguous())
     places = [None] * len(hops)
     if defer:
-        together = _Together(len(hops), q, kv, ring, softmax_scale, dropout_p, causal, window_size, alibi_slopes, into=(o, lse))
+        together = _Together(len(hops), q, kv, ring, softmax_scale, dropout_p, causal, window_size, alibi_slopes)
         if together.size > 1:
             together.step(_resident_chunks(ring, kv), o, lse)
             return

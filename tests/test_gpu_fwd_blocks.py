@@ -309,3 +309,43 @@ def test_a_run_that_begins_with_hidden_chunks(fill, n, Sc, D):
     for i in range(2):                   # the run, and its keys as one block (whose workgroups split them)
         assert ((lse[i].cpu() - rl).abs() / rl.abs()).max().item() <= 1e-3, i
         assert ((out[i].float().cpu() - ro).abs() - 2 ** -8 * ro.abs()).max().item() <= 2e-2, i
+
+
+def test_a_ring_whose_chunks_are_one_stacked_tensor():
+    """The chunks of all ranks as the first dimension of one tensor, in a step with one result and in one with several."""
+    import mercury_artifact_amd as M
+
+    for W, S, H, D in [(2, 1024, 64, 128), (4, 256, 4, 64)]:
+        q, chunks, _, _ = _inputs(W, 1, S, S, H, H, D, False)
+        q, stacked, got = q.cuda(), torch.stack(chunks).cuda(), []
+        for held in (stacked, list(stacked.unbind(0))):
+            o, lse = torch.empty_like(q), torch.empty(1, H, S, device="cuda")
+            M.flash_attn_pack_kv(q, held[0], o, lse, D ** -0.5, ring=M.LocalRing((W,), 0, held))
+            got.append((o, lse))
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+def test_the_only_result_over_a_chunk_that_only_the_hop_knows():
+    """A resident ring of one's own need not list its chunks: an output over one of them is written behind the launch."""
+    import mercury_artifact_amd as M
+
+    class Own(M.LocalRing):
+        resident = True
+
+        def __init__(self, mesh, rank, mine):
+            super().__init__(mesh, rank)
+            self.mine = mine
+
+        def send_recv(self, to, source, x, recv_tensor=None):
+            super().send_recv(to, source, x)
+            return self.mine[self.current]
+
+    W, S, H, D = 2, 1024, 64, 128
+    q, chunks, _, _ = _inputs(W, 1, S, S, H, H, D, False)
+    q, got = q.cuda(), []
+    for over in (False, True):
+        dev = [c.cuda() for c in chunks]
+        o, lse = dev[1][1] if over else torch.empty_like(q), torch.empty(1, H, S, device="cuda")
+        M.flash_attn_pack_kv(q, dev[0], o, lse, D ** -0.5, ring=Own((W,), 0, dev))
+        got.append((o, lse))
+    assert torch.equal(got[0][0], got[1][0]) and (got[0][1] - got[1][1]).abs().max().item() <= 1e-5
