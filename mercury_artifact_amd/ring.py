@@ -113,6 +113,12 @@ def _block_results(n, q, kv, *args, **kwargs):
     return list(zip(outs.unbind(0), lses.unbind(0)))
 
 
+def _resident(ring) -> bool:
+    """Whether a step may take several chunks of the ring before it launches.  Not where every hop makes a copy: a step
+    would hold as many of them as there are chunks, instead of the ones in use and the next."""
+    return bool(type(ring).__dict__.get("resident")) and not getattr(ring, "copy", False)
+
+
 class _Together:
     """Block forwards of one query tensor over ``n`` chunks of a ring whose chunks are all there, several to a launch
     (mhip_attn_fwd_group) and, where that is faster, a run of chunks to a result (mhip_attn_fwd_chain).  ``size``, the
@@ -121,7 +127,7 @@ class _Together:
     def __init__(self, n, q, kv, ring, softmax_scale, dropout_p, causal, window_size, alibi_slopes, q_descale=None, k_descale=None,
                  v_descale=None):
         self.size = self.per = 1
-        if (n < 2 or not type(ring).__dict__.get("resident")
+        if (n < 2 or not _resident(ring)
                 or not _straight(q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes, q_descale=q_descale,
                                  k_descale=k_descale, v_descale=v_descale)):
             return
@@ -173,7 +179,7 @@ def _visits(mesh_shape, rank, held):
 def _resident_chunks(ring, kv):
     """A step's chunks in visiting order, for a ring whose chunks are all there; leaves the ring where the hops would."""
     chunks = [_as_rows(kv)]
-    if (type(ring) is LocalRing and ring.chunks is not None and not ring.copy and not ring._committed
+    if (type(ring) is LocalRing and ring.chunks is not None and not ring._committed
             and ring.__dict__.keys().isdisjoint(("send_recv", "commit", "wait", "hop"))):       # nobody looks on
         seen, held = _visits(ring.mesh_shape, ring.rank, tuple(ring.held))
         chunks += [ring.chunks[i] for i in seen[1:]]
@@ -558,7 +564,7 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
     _kv = _next_kv = prepared = None
     own = ring.current
     group, waiting = 1, []
-    if carried and type(ring).__dict__.get("resident"):
+    if carried and _resident(ring):
         group = N.host.bwd_group(q, kv, ring.world) or 1
     for step, hop in enumerate(_hops(ring)):
         if step == 0:

@@ -276,7 +276,7 @@ class LocalRing:
     # Every chunk lies in this GPU's memory for the whole step -- the emulated exchange, or chunks gathered beforehand -- and
     # a hop only says whose turn it is.  Drivers may then take several chunks before they launch, and launch their
     # blocks together.  A ring class says so for itself: with one that receives its chunks, derived from this one or not, a
-    # block is launched when its chunk is there, so that the next hop runs beside it.
+    # block is launched when its chunk is there, so that the next hop runs beside it.  (So is one of a ring with copy=True.)
     resident = True
 
     def __init__(self, mesh_shape: Sequence[int], rank: int,

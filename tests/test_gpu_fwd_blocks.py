@@ -349,3 +349,30 @@ def test_the_only_result_over_a_chunk_that_only_the_hop_knows():
         M.flash_attn_pack_kv(q, dev[0], o, lse, D ** -0.5, ring=Own((W,), 0, dev))
         got.append((o, lse))
     assert torch.equal(got[0][0], got[1][0]) and (got[0][1] - got[1][1]).abs().max().item() <= 1e-5
+
+
+@pytest.mark.parametrize("path", ["ring", "packed", "zigzag", "backward"])
+def test_a_ring_that_copies_holds_few_copies_at_a_time(path):
+    """LocalRing(copy=True) hands out a copy per hop: a step holds the last block's, the next block's and the one that hop makes,
+    however many chunks there are."""
+    import mercury_artifact_amd as M
+
+    W, S, H, D = 8, 256, 4, 128
+    q, chunks, _, _ = _inputs(W, 1, S, S, H, H, D, False)
+    q, chunks = q.cuda(), [c.cuda() for c in chunks]
+    o, lse, dq, dkv = torch.empty_like(q), torch.zeros(1, H, S, device="cuda"), torch.empty_like(q), torch.empty_like(chunks[0])
+    step = {"ring": M.flash_attn_pack_kv, "packed": M.flash_attn_expose_reduce, "zigzag": M.zigzag_causal_pack_kv,
+            "backward": lambda q, kv, o, lse, scale, ring: M.flash_attn_backward(q, kv, o, lse, q, dq, dkv, scale, ring=ring)}[path]
+
+    class Hops(M.LocalRing):             # hands over the chunks themselves, one by one
+        pass
+
+    def peak(ring):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        step(q, chunks[1], o, lse, 0.1, ring=ring)
+        return torch.cuda.max_memory_allocated() - before
+
+    one_by_one = peak(Hops((W,), 1, chunks))
+    assert peak(M.LocalRing((W,), 1, chunks, copy=True)) <= one_by_one + 3 * chunks[0].numel() * 2
