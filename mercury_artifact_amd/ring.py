@@ -37,6 +37,7 @@ from .schedule import (LocalRing, n_dim_to_one_dim, n_ranks, one_dim_to_n_dim, r
                        shift_tuple_element, zigzag_step)
 
 MAX_GROUP = 16           # MHIP_MAX_GROUP: chunks of a launch
+UNKEPT_BYTES = 32 << 20  # gradients that a launch over several chunks may make for nobody (or one chunk's, if that is more)
 
 __all__ = ["flash_attn_pack_kv", "gqa_pack_kv", "flash_attn_pack_split_kv", "flash_attn_expose_reduce",
            "flash_attn_expose_reduce_q_ring",
@@ -566,6 +567,8 @@ def flash_attn_backward(q, kv, o, lse, dout, dq, dkv, softmax_scale, dropout_p=0
     group, waiting = 1, []
     if carried and _resident(ring):
         group = N.host.bwd_group(q, kv, ring.world) or 1
+        if dkv_chunks is None:                  # the other ranks' chunks' gradients need places all the same
+            group = min(group, max(1, UNKEPT_BYTES // max(1, kv.numel() * kv.element_size())))
     for step, hop in enumerate(_hops(ring)):
         if step == 0:
             _kv = kv.contiguous()

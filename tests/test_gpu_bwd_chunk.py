@@ -262,3 +262,30 @@ def test_rows_past_the_end_are_no_other_heads():
         grads.append(torch.stack((dq, dkv[0], dkv[1]))[:, :, :, ::2])
     assert torch.isfinite(grads[0].float()).all()
     assert torch.equal(grads[1], grads[0]) and torch.equal(grads[2], grads[0])
+
+
+def test_gradients_nobody_keeps_take_bounded_memory():
+    """Without dkv_chunks the gradients of the other ranks' chunks are made and dropped: launches over several chunks hold
+    32 MiB of them, whatever the step would have grouped."""
+    import mercury_artifact_amd as M
+
+    W, S, H, D = 8, 2048, 8, 128
+    assert N.lib().mhip_attn_bwd_group(1, S, S, H, H, D, W) * 2 * S * H * D * 2 > 60 << 20
+    g = torch.Generator(device="cuda").manual_seed(2)
+    q, dout, o = (torch.randn(1, S, H, D, generator=g, device="cuda").bfloat16() for _ in range(3))
+    chunks = [torch.randn(2, 1, S, H, D, generator=g, device="cuda").bfloat16() for _ in range(W)]
+    lse = torch.full((1, H, S), 9.0, device="cuda")
+    dq, dkv = torch.empty_like(q), torch.empty_like(chunks[0])
+
+    class Hops(M.LocalRing):             # a launch per chunk: one such gradient at a time
+        pass
+
+    def peak(ring):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        M.flash_attn_backward(q, chunks[1], o, lse, dout, dq, dkv, D ** -0.5, ring=ring)
+        return torch.cuda.max_memory_allocated() - before
+
+    one_by_one = peak(Hops((W,), 1, chunks))
+    assert peak(M.LocalRing((W,), 1, chunks)) <= one_by_one + (32 << 20)
