@@ -177,11 +177,18 @@ def _visits(mesh_shape, rank, held):
     return tuple(seen), ring.held
 
 
+def _hop_methods():
+    return LocalRing.send_recv, LocalRing.commit, LocalRing.wait, LocalRing.hop
+
+
+_HOP = _hop_methods()       # as this package defines them: a wrapper put over one, on a ring or on the class, sees every hop
+
+
 def _resident_chunks(ring, kv):
     """A step's chunks in visiting order, for a ring whose chunks are all there; leaves the ring where the hops would."""
     chunks = [_as_rows(kv)]
     if (type(ring) is LocalRing and ring.chunks is not None and not ring._committed
-            and ring.__dict__.keys().isdisjoint(("send_recv", "commit", "wait", "hop"))):       # nobody looks on
+            and ring.__dict__.keys().isdisjoint(("send_recv", "commit", "wait", "hop")) and _hop_methods() == _HOP):  # nobody looks on
         seen, held = _visits(ring.mesh_shape, ring.rank, tuple(ring.held))
         chunks += [ring.chunks[i] for i in seen[1:]]
         ring.held = list(held)

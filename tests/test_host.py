@@ -451,6 +451,25 @@ def test_backward_step_in_place_writes_nothing_a_launch_still_reads(monkeypatch,
     assert direct[-1][0] == (dq_over == "") and (direct[0][1] == dkv.data_ptr()) == (dkv_over == "")
 
 
+@pytest.mark.parametrize("name", ["send_recv", "commit", "wait", "hop"])
+@pytest.mark.parametrize("on", ["ring", "class"])
+def test_a_wrapper_over_a_hop_sees_every_hop(monkeypatch, name, on):
+    """A step that collects its chunks at once calls what is put over a ring's methods, on the ring or on its class, as a
+    step that goes hop by hop does; the same chunks and the same places afterwards as with nothing put over them."""
+    import mercury_artifact_amd.ring as R
+    from mercury_artifact_amd.schedule import LocalRing
+
+    chunks = [torch.full((2, 1, 8, 1, 8), float(i), dtype=torch.bfloat16) for i in range(8)]
+    plain = LocalRing((4, 2), 5, chunks)
+    want = R._resident_chunks(plain, chunks[5])
+    ring, calls = LocalRing((4, 2), 5, chunks), []
+    over, real = (ring, getattr(ring, name)) if on == "ring" else (LocalRing, getattr(LocalRing, name))
+    monkeypatch.setattr(over, name, lambda *a, **kw: calls.append(1) or real(*a, **kw))
+    got = R._resident_chunks(ring, chunks[5])
+    assert len(calls) == 7 and ring.held == plain.held
+    assert len(got) == 8 and all(a is b for a, b in zip(got[1:], want[1:])) and torch.equal(got[0], want[0])
+
+
 def test_backward_step_without_the_host_modules_answers(monkeypatch):
     """A host module that declines every question: copies and staged stores, not a wrong call."""
     import mercury_artifact_amd.ring as R
