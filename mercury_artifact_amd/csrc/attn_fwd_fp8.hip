@@ -62,6 +62,8 @@ struct Fp8Params {
   uint16_t* out; float* lse;
   int64_t o_sb, o_ss, o_sh;
   int64_t o_sn, l_sn;    // from one block's results to the next one's, elements
+};
+struct Fp8Chunks : Fp8Params {       // of a launch over several chunks, as in the bf16 kernel
   const uint8_t* k[kMaxGroup]; const uint8_t* v[kMaxGroup];          // the chunk of every block
 };
 
@@ -81,8 +83,10 @@ __device__ __forceinline__ constexpr int swz8(int row) { return (((row >> 1) & 3
 // the same.
 //
 // CHAIN: a workgroup visits p.per chunks one after the other, as in the bf16 kernel.
-template <bool CAUSAL, int DB, int WAVES, bool CHAIN = false>
-__global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const Fp8Params p) {
+template <bool CAUSAL, int DB, int WAVES, class P, bool CHAIN = false>
+__global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const P p) {
+  constexpr bool kLone = std::is_same<P, Fp8Params>::value;
+  static_assert(!CHAIN || !kLone, "a run of chunks needs their addresses");
   static_assert(WAVES == 8 || WAVES == 4, "two wavefronts per SIMD or one");
   constexpr int kBM = WAVES * 32;
   constexpr int kCpy = 16 / WAVES;              // copy instructions per wavefront for one 16 KB tile
@@ -118,12 +122,13 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
   // first one's addresses come with the arguments above: a lone block does not wait for a second round of loads.)
   const uint8_t* kp = p.k0; const uint8_t* vp = p.v0;
   int blk = 0, chunk = 0;
-  if (p.blocks > 1) {
-    blk = p.by_heads.quotient(bh, bh);
-    chunk = CHAIN ? blk * p.per : blk;
-    kp = p.k[chunk];
-    vp = p.v[chunk];
-  }
+  if constexpr (!kLone)
+    if (p.blocks > 1) {
+      blk = p.by_heads.quotient(bh, bh);
+      chunk = CHAIN ? blk * p.per : blk;
+      kp = p.k[chunk];
+      vp = p.v[chunk];
+    }
   int hq;
   const int b = p.by_hq.quotient(bh, hq);
   const int hk = p.by_group.quotient(hq);
@@ -194,7 +199,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
     if (++k_pos == chunk_tiles && k_chunk != last_chunk) {
       k_off = k_pos = 0;
       ++k_chunk;
-      enter(krs, p.k[k_chunk] + b * p.k_sb + hk * p.k_sh);
+      if constexpr (CHAIN) enter(krs, p.k[k_chunk] + b * p.k_sb + hk * p.k_sh);
     }
   };
   auto chain_v = [&]() {
@@ -203,7 +208,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
     if (++v_pos == chunk_tiles && v_chunk != last_chunk) {
       v_off = v_pos = 0;
       ++v_chunk;
-      enter(vrs, p.v[v_chunk] + b * p.v_sb + hk * p.v_sh);
+      if constexpr (CHAIN) enter(vrs, p.v[v_chunk] + b * p.v_sb + hk * p.v_sh);
     }
   };
 
@@ -522,12 +527,23 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void attn_fwd_fp8_d128(const
   }
 }
 
+// A launch of one block takes the short arguments (see FwdChunks of the bf16 kernels; graphs of such launches, us, with the
+// chunks' addresses / without: 64 x 64 H1 6.32 / 6.03, 256 x 256 H4 7.15 / 6.93, causal 1024 x 1024 H8 14.5 / 14.0).  Not so
+// four wavefronts on 64 columns, whose main loop, the same instructions on other registers, takes longer then (1024 x 1024 H8
+// 12.2 / 12.5, 4096 x 4096 H2 34.9 / 36.7).
 template <int DB, int WAVES>
-void launch_fp8(const Fp8Params& p, bool causal, hipStream_t stream) {
+void launch_fp8(const Fp8Chunks& p, bool causal, hipStream_t stream) {
   const dim3 grid(p.per_xcd * 8), block(WAVES * 64);
-  if (p.per > 1) hipLaunchKernelGGL((attn_fwd_fp8_d128<false, DB, WAVES, true>), grid, block, 0, stream, p);
-  else if (causal) hipLaunchKernelGGL((attn_fwd_fp8_d128<true, DB, WAVES>), grid, block, 0, stream, p);
-  else hipLaunchKernelGGL((attn_fwd_fp8_d128<false, DB, WAVES>), grid, block, 0, stream, p);
+  if constexpr (DB > 2 || WAVES > 4)
+    if (p.blocks == 1 && p.per == 1) {
+      const Fp8Params& lone = p;
+      if (causal) hipLaunchKernelGGL((attn_fwd_fp8_d128<true, DB, WAVES, Fp8Params>), grid, block, 0, stream, lone);
+      else hipLaunchKernelGGL((attn_fwd_fp8_d128<false, DB, WAVES, Fp8Params>), grid, block, 0, stream, lone);
+      return;
+    }
+  if (p.per > 1) hipLaunchKernelGGL((attn_fwd_fp8_d128<false, DB, WAVES, Fp8Chunks, true>), grid, block, 0, stream, p);
+  else if (causal) hipLaunchKernelGGL((attn_fwd_fp8_d128<true, DB, WAVES, Fp8Chunks>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((attn_fwd_fp8_d128<false, DB, WAVES, Fp8Chunks>), grid, block, 0, stream, p);
 }
 
 }  // namespace
@@ -567,7 +583,7 @@ int attn_fwd_fp8_chain(int n, int B, int Sq, int Sc, int Hq, int D) {
 int attn_fwd_fp8(const void* q, const void* const* ks, const void* const* vs, int n, int per, void* out, int64_t o_sn, float* lse,
                  int B, int Sq, int Sc, int Hq, int Hkv, int D, const int64_t* st, float scale, int mask,
                  const float* q_descale, const float* k_descale, const float* v_descale, hipStream_t stream) {
-  Fp8Params p;
+  Fp8Chunks p;
   p.q = static_cast<const uint8_t*>(q);
   for (int i = 0; i < kMaxGroup; ++i) {
     p.k[i] = i < n ? static_cast<const uint8_t*>(ks[i]) : nullptr;

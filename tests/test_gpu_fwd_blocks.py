@@ -376,3 +376,33 @@ def test_a_ring_that_copies_holds_few_copies_at_a_time(path):
 
     one_by_one = peak(Hops((W,), 1, chunks))
     assert peak(M.LocalRing((W,), 1, chunks, copy=True)) <= one_by_one + 3 * chunks[0].numel() * 2
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("B,Sq,Sc,Hq,Hkv,D", [
+    (1, 1, 1, 1, 1, 64), (1, 256, 256, 4, 4, 64), (1, 130, 300, 2, 1, 128), (2, 257, 130, 3, 3, 96), (1, 1000, 200, 72, 8, 128),
+    (1, 1024, 257, 72, 72, 64), (1, 1024, 70, 72, 24, 96)])
+def test_a_block_alone_and_beside_another_one(B, Sq, Sc, Hq, Hkv, D, fp8, causal):
+    """A launch of one block has arguments and kernels of its own: bit for bit the block's result in a launch of two, for
+    operands and places with gaps between their rows too."""
+    q, chunks, sq, sc = _inputs(2, B, Sq, Sc, Hq, Hkv, D, fp8)
+    print(f"alone B{B} Sq{Sq} Sc{Sc} H{Hq}/{Hkv} D{D} fp8={fp8} causal={causal}", flush=True)
+    plans = [N.lib().mhip_attn_fwd_plan(k * B, Sq, Sc, Hq, D, Hkv * D, Hkv * D, int(causal), N.MHIP_E4M3 if fp8 else N.MHIP_BF16) for k in (1, 2)]
+    assert plans[0] == plans[1]
+
+    def gaps(t):
+        wide = torch.zeros(*t.shape[:-1], D + 16, dtype=t.dtype, device="cuda")
+        wide[..., :D] = t.cuda()
+        return wide[..., :D]
+
+    ds = [None] * 3 if not fp8 else [t.cuda().reshape(()) for t in (sq, sc, sc)]
+    for form in (lambda t: t.cuda(), gaps):
+        qd, dev = form(q), [form(c) for c in chunks]
+        outs = form(torch.full((4, B, Sq, Hq, D), 7.0, dtype=torch.bfloat16))
+        lses = torch.full((4, B, Hq, Sq), 7.0, device="cuda")
+        assert N.host.fwd_blocks(qd, dev, 1, D ** -0.5, causal, *ds, outs, lses, 0) is True
+        for i in (0, 1):
+            assert N.host.fwd_blocks(qd, dev[i:i + 1], 1, D ** -0.5, causal, *ds, outs, lses, 2 + i) is True
+        torch.cuda.synchronize()
+        assert torch.equal(outs[:2], outs[2:]) and torch.equal(lses[:2], lses[2:]) and not (lses == 7).any()
