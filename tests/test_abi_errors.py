@@ -144,3 +144,33 @@ def test_forward_blocks_reject(lib):
     assert blocks(n=0) == blocks(n=17, ks=[P] * 17, vs=[P] * 17) == blocks(n=-1) == EINVAL
     assert blocks(ks=None) == blocks(vs=None) == blocks(ks=(P, 0)) == blocks(vs=(P, 0)) == blocks(out=None) == EINVAL
     assert blocks(ks=(P, P + 8)) == blocks(vs=(P, P + 8)) == blocks(o_sn=8196) == EALIGN
+
+
+def test_backward_chunks_reject(lib):
+    def chunks(n=3, ks=(P,) * 17, vs=(P,) * 17, dks=(P,) * 17, dvs=(P,) * 17, dk32s=(0,) * 17, dv32s=(0,) * 17, dout=P, q=P, out=P, lse=P,
+               dq=P, acc=P, first=1, last=1, B=1, Sq=64, Sc=64, Hq=2, Hkv=2, D=128, k_ss=256, scale=0.1, workspace=P):
+        lists = [None if x is None else (ctypes.c_void_p * 17)(*x) for x in (ks, vs, dks, dvs, dk32s, dv32s)]
+        return lib.mhip_attn_bwd_chunks(dout, q, *lists[:2], n, out, lse, dq, acc, first, last, 0, *lists[2:], B, Sq, Sc, Hq, Hkv, D,
+                                        Sq * 256, 256, 128, Sc * k_ss, k_ss, 128, *[Sc * 256, 256, 128] * 3, scale, workspace, None)
+
+    def at(i, value, fill=P):
+        return tuple(value if j == i else fill for j in range(17))
+
+    assert chunks(n=0) == chunks(n=17) == chunks(n=-1) == EINVAL
+    for name in ("ks", "vs", "dks", "dvs", "dk32s", "dv32s"):
+        assert chunks(**{name: None}) == EINVAL
+    for i in (0, 2):                     # the first element, which other checks see too, and one that only the list holds
+        assert chunks(ks=at(i, 0)) == chunks(vs=at(i, 0)) == EINVAL
+        assert chunks(dks=at(i, 0)) == chunks(dvs=at(i, 0)) == EINVAL                               # dk without dv, dv without dk
+        assert chunks(dk32s=at(i, P, 0)) == chunks(dv32s=at(i, P, 0)) == EINVAL
+        assert chunks(dks=at(i, 0), dvs=at(i, 0)) == EINVAL                                         # no place in either type
+        for name in ("ks", "vs", "dks", "dvs"):
+            assert chunks(**{name: at(i, P + 8)}) == EALIGN
+        assert chunks(dk32s=at(i, P + 4, 0), dv32s=at(i, P, 0)) == chunks(dk32s=at(i, P, 0), dv32s=at(i, P + 4, 0)) == EALIGN
+    assert chunks(first=0, acc=None) == chunks(first=0, last=0, acc=None) == chunks(last=0, acc=None) == EINVAL
+    assert chunks(dq=None) == chunks(q=None) == chunks(dout=None) == chunks(out=None) == chunks(lse=None) == chunks(workspace=None) == EINVAL
+    assert chunks(Hkv=0) == chunks(Hkv=3) == chunks(Sq=-1) == chunks(scale=0.0) == EINVAL
+    assert chunks(D=132) == chunks(D=0) == EHEADDIM and chunks(k_ss=260) == EALIGN
+    assert chunks(Sc=1 << 20, k_ss=1024) == EUNSUPPORTED                                            # a span of 2 GiB
+    assert chunks(Sc=1 << 30, k_ss=0, Hq=16, Hkv=16, n=16) == EUNSUPPORTED                          # 2^31 workgroups
+    assert chunks(B=0) == OK
