@@ -4,10 +4,10 @@
 Workload = the headline bf16 configuration: batch 1, 32 heads, head dim 128, local Q of 4096 rows, 8 KV chunks
 of 4096 rows (32768 keys), non-causal, N(0,1) inputs cast to bf16, softmax scale 128^-0.5.
 A step = the ring driver's default on a ring whose chunks are all in memory: ONE launch of the forward kernel whose
-workgroups visit the 8 chunks one after the other and write the bf16 output and the (B,H,S) LSE (drivers on other
-rings launch a block per chunk and fold the results in one pass; the generated code's literal chain of block
-operators and LSE merges, and its fold, are timed beside it).  Inputs are resident in HBM before the timed region.
-Prints ONE JSON line.
+workgroups visit the 8 chunks one after the other and write the bf16 output and the (B,H,S) LSE.  Timed beside it: the
+same driver on a ring that receives its chunks, which launches a block forward per chunk and folds the 8 results in one
+pass (`launch_per_chunk_*`, `roofline_block`), the generated code's literal chain of block operators and LSE merges, and
+the fold.  Inputs are resident in HBM before the timed region.  Prints ONE JSON line.
 """
 from __future__ import annotations
 
@@ -24,7 +24,8 @@ PEAK_BF16_TFLOPS = 2500.0      # MI355X dense bf16 MFMA
 PEAK_HBM_GBS = 8000.0          # MI355X HBM3E
 # HBM bytes per launch from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of this script, each counter scaled
 # by its reading for the calibration launch at the end of main() (profiles/ring_step_config1_hbm_traffic.md)
-TRAFFIC_FWD_BYTES = 604.7e6
+TRAFFIC_FWD_BYTES = 604.7e6    # the launch over 8 chunks
+TRAFFIC_BLOCK_BYTES = 134.9e6  # and over one
 TRAFFIC_MERGE_BYTES = 171.5e6
 TRAFFIC_MANY_BYTES = 321.0e6
 
@@ -217,6 +218,7 @@ def main() -> int:
     import torch
 
     import mercury_artifact_amd as M
+    from mercury_artifact_amd import flash_attn_interface as FI
     from mercury_artifact_amd import merge as MG
 
     if not torch.cuda.is_available():
@@ -237,7 +239,7 @@ def main() -> int:
     # its plain merges per step.
     fwd_events, chunks_timed, merge_events = [], [], []
     real_merge = MG.merge_into
-    recording = {"on": False, "step": 0, "merge": 0}
+    recording = {"on": False, "step": 0, "merge": 0, "block": 0}
 
     def timed(real, bucket, kind, per_step, eligible):
         def wrapper(*a, **kw):
@@ -342,6 +344,33 @@ def main() -> int:
     many_ms = sum(e0.elapsed_time(e1) for e0, e1 in many_events) / max(len(many_events), 1)
     many_gbs = many_bytes / (many_ms * 1e-3) / 1e9
 
+    # the same step on a ring that receives its chunks: a block forward per chunk on the kernels' per-rank shape, launched
+    # when the chunk is there, and one fold of the 8 results.  One of its block launches per step, another one every
+    # time, is bracketed by events.
+    class Hops(M.LocalRing):
+        pass
+
+    def step_hops():
+        M.flash_attn_pack_kv(q, kvs[rank], o, lse, scale, ring=Hops((W,), rank, kvs))
+
+    block_events = []
+    real_block = FI.attn_fwd_block
+    FI.attn_fwd_block = timed(real_block, block_events, "block", W, lambda a: True)
+    for _ in range(args.steps):                # the clock has to settle again behind the fold's launches above
+        step_hops()
+    torch.cuda.synchronize()
+    recording["on"] = True
+    t0 = time.perf_counter()
+    for i in range(args.steps):
+        recording.update(step=i, block=0)
+        step_hops()
+    torch.cuda.synchronize()
+    hops_ms = (time.perf_counter() - t0) / args.steps * 1e3
+    recording["on"] = False
+    FI.attn_fwd_block = real_block
+    block_ms = sum(e0.elapsed_time(e1) for e0, e1 in block_events) / max(len(block_events), 1)
+    block_tflops = flops_per_block / (block_ms * 1e-3) / 1e12
+
     # the same step as the generated code spells it: update_out_and_lse after every chunk (the fp32
     # accumulator read and written once per chunk), then the cast and the transposed copy of the epilogue.
     # Also timed, with one plain merge per step bracketed by events.
@@ -425,10 +454,7 @@ def main() -> int:
 
     two_streams_ms, two_same = None, None
     if not args.no_variants:                 # overlapping launches would spoil a profiler's per-kernel averages
-        class Hops(M.LocalRing):               # chunks hop by hop: a block launch each on one stream
-            pass
-
-        M.flash_attn_pack_kv(q, kvs[rank], o, lse, scale, ring=Hops((W,), rank, kvs))
+        step_hops()                            # the same launches on one stream
         one_o, one_lse = o.clone(), lse.clone()
         for _ in range(3):
             step_two_streams()
@@ -481,6 +507,8 @@ def main() -> int:
         "config": {"workload": "headline bf16 configuration: non-causal MHA, B1 H32 D128, local Q 4096 x 8 KV chunks "
                                "of 4096 (single ring, rank 0), one forward launch over the 8 chunks",
                    "flops_per_step": flops_per_step, "pct_of_bf16_mfma_peak": round(100 * value / PEAK_BF16_TFLOPS, 2),
+                   "launch_per_chunk_ms_per_step": round(hops_ms, 4),
+                   "launch_per_chunk_tflops": round(flops_per_step / hops_ms / 1e9, 1),
                    "literal_merge_chain_ms_per_step": round(unfused_ms, 4),
                    "generated_text_ms_per_step": round(drop_in_ms[False], 4),
                    "generated_text_lazy_namespace_ms_per_step": round(drop_in_ms[True], 4),
@@ -492,6 +520,9 @@ def main() -> int:
         "roofline": {"bound": "mfma", "kernel": "attn_fwd_bf16_d128", "achieved": round(fwd_tflops, 2),
                      "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": round(fwd_tflops / PEAK_BF16_TFLOPS, 4),
                      "traffic": TRAFFIC_FWD_BYTES, "avg_launch_ms": round(fwd_ms, 4), "launches": len(fwd_events)},
+        "roofline_block": {"bound": "mfma", "kernel": "attn_fwd_bf16_d128", "achieved": round(block_tflops, 2),
+                           "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": round(block_tflops / PEAK_BF16_TFLOPS, 4),
+                           "traffic": TRAFFIC_BLOCK_BYTES, "avg_launch_ms": round(block_ms, 4), "launches": len(block_events)},
         "roofline_merge_many": {"bound": "hbm", "kernel": "lse_merge_many_kernel", "achieved": round(many_gbs, 1),
                                 "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": round(many_gbs / PEAK_HBM_GBS, 4),
                                 "traffic": TRAFFIC_MANY_BYTES, "avg_launch_ms": round(many_ms, 5), "launches": len(many_events),
