@@ -319,7 +319,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
   float l_run = 0.f;         // this lane's share of the running sum (the other 32 keys: lane ^ 32)
   constexpr float kTrigger = 1048576.f;   // a lane's 32 exponentials of one tile sum to less than this, or
   constexpr float kSlack = 14.f;          // rows whose maximum exceeds the reference by 2^kSlack move it
-  constexpr float kNoScore = -0x1p64f;    // the reference of a row whose first tile holds scores of -inf only
+  constexpr float kMost = 0x1.fffffep127f;
   const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   f32x16 s[MB];              // S^T tile: BN keys x 32 q rows per wave
   u32x4 pw[2 * MB];          // P^T of the current tile as packed bf16 B operands, one per k-step
@@ -406,9 +406,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
         for (int j = 0; j < 16; ++j) o_acc[db][j] *= alpha;
       l_run *= alpha;
     }
-    // (with scores of -inf alone it stays below any other score, so that the first key that counts moves it)
-    if (move) m_ref = first ? fmaxf(mx, kNoScore) : mx;
-    nmsc = -m_ref * scale_log2;
+    // (with scores of -inf alone it stays at the lowest finite one, so that the first key that counts moves it; the product
+    // stays finite too, so that scores of -inf have exponentials of 0)
+    if (move) m_ref = first ? fmaxf(mx, -kMost) : mx;
+    nmsc = fminf(-m_ref * scale_log2, kMost);
   };
   // slot of the matrix phase after which early pair idx runs: k-step idx / 4 of the tile before is read by the
   // O^T slots kSlotsS + DB (idx / 4) .. + DB - 1, and the pairs are spread two slots apart behind that

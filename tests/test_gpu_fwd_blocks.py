@@ -311,6 +311,31 @@ def test_a_run_that_begins_with_hidden_chunks(fill, n, Sc, D):
         assert ((out[i].float().cpu() - ro).abs() - 2 ** -8 * ro.abs()).max().item() <= 2e-2, i
 
 
+@pytest.mark.parametrize("hidden", [0, 1, 2])
+@pytest.mark.parametrize("Sc,D", [(200, 128), (64, 64), (100, 96)])
+@pytest.mark.parametrize("score", [-2.0 ** 70, -2.0 ** 127])
+def test_rows_whose_every_score_is_very_low(score, hidden, Sc, D):
+    """Finite scores near fp32's lowest number, alone or behind chunks of -inf: they count where nothing else does.  All of
+    them are one power of two, whose product with the scale is exact, so P is 1 and the result the mean of V, rounded once."""
+    g = torch.Generator().manual_seed(Sc + hidden)
+    q = torch.zeros(1, 130, 2, D)
+    q[..., 0] = 1.0
+    chunks = [torch.randn(2, 1, Sc, 2, D, generator=g) for _ in range(hidden + 1)]
+    for i, c in enumerate(chunks):
+        c[0, ..., 0] = score if i == hidden else float("-inf")
+    scale = D ** -0.5
+    q, chunks = q.bfloat16().cuda(), [c.bfloat16() for c in chunks]
+    ro = chunks[-1][1].float().mean(1, keepdim=True).expand(1, 130, 2, D)
+    out, lse = torch.empty(2, 1, 130, 2, D, dtype=torch.bfloat16, device="cuda"), torch.empty(2, 1, 2, 130, device="cuda")
+    run = [c.cuda() for c in chunks]
+    assert N.host.fwd_blocks(q, run, len(run), scale, False, None, None, None, out, lse, 0) is True
+    assert N.host.fwd_blocks(q, [torch.cat(run, 2)], 1, scale, False, None, None, None, out, lse, 1) is True
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert (lse[i].cpu() / (score * scale) - 1).abs().max().item() <= 1e-6, i
+        assert ((out[i].float().cpu() - ro).abs() - 2 ** -8 * ro.abs()).max().item() <= 1e-5, i
+
+
 def test_a_ring_whose_chunks_are_one_stacked_tensor():
     """The chunks of all ranks as the first dimension of one tensor, in a step with one result and in one with several."""
     import mercury_artifact_amd as M
