@@ -935,7 +935,9 @@ TileMap tile_map(int heads, int seq, int rows, int splits = 1, float* partial = 
 }
 
 // Estimated time (us) of n workgroups that visit `most` tiles at most and `mean` on average, one workgroup per CU at a
-// time: `fixed` per workgroup and `step` per tile, plus `busy` times the share of the CUs at work (clock and L2).
+// time: `fixed` per workgroup and `step` per tile, plus `busy` times the share of the CUs at work (clock and L2).  On 64
+// columns two workgroups of four wavefronts share a CU, so the estimate is too high there (causal 1500 x 1500 B2 H12: 50 us,
+// where the whole backward takes 41); what plan_block and group_chunks choose by it is measured beside the other choices.
 struct Cost { float fixed, step, busy; };
 float launch_time(float n, float mean, float most, const Cost& c) {
   const float full = floorf(n / 256.f), part = n / 256.f - full;
@@ -956,7 +958,13 @@ float launch_time(float n, float mean, float most, const Cost& c) {
 // where one workgroup's chain of tiles -- with grouped heads, all query heads of the group -- is what the launch waits for;
 // their sums meet in a third launch (one / with it):
 //     B1 H8/1 512 x 512      82.6 / 27.6     B1 H8/1 2048 x 2048    310 / 73.6     B1 H8/1 4096 x 4096   636 /  221
-//     B1 H2/2 4096 x 4096    85.2 / 69.8     B1 H32/4 2048 x 2048   338 /  220     causal, D 64: H8/1 2048 x 2048  249 / 45.3
+//     B1 H2/2 4096 x 4096    85.2 / 69.8     B1 H32/4 2048 x 2048   338 /  220
+// On 64 columns, where the costs are those of one workgroup per CU (two launches / one, * the form chosen):
+//     B1 H4   256 x 256     17.0 / 10.4*     B4 H5    512 x 512    24.5 / 15.0*     B1 H16 2048 x 2048  74.1 / 61.4*
+//     B2 H12 1500 x 1500    71.0 / 66.8*     B1 H32 2048 x 2048   117* / 121        B1 H32 4096 x 4096  442* / 448
+//     causal: B2 H12 1500 x 1500  60.7 / 40.8*                                      B1 H32 4096 x 4096  249* / 247
+// and one / shared by as many workgroups (sq, sk) as chosen: H8/1 2048 x 2048 226 / 46.0 (1, 8), H32/4 247 / 125 (1, 4), H2/2
+// 4096 x 4096 63.1 / 48.0 (2, 2), where 44.2 (4, 4) would be better.
 Cost joint_cost(int D) { return D <= 64 ? Cost{6.f, 0.75f, 0.12f} : Cost{7.f, 1.15f, 0.29f}; }
 struct Plan { bool joint; int sq, sk; float time; };       // time: estimated, without preparing delta and lse2
 constexpr int64_t kPartialMost = int64_t(32) << 20;     // bytes of sums a block may leave for bwd_reduce
@@ -996,7 +1004,11 @@ Plan plan_block(int B, int Sq, int Sc, int Hq, int Hkv, int D, bool causal) {
 // long.  Us a step, chunk by chunk / in launches of 2 / 4 / 8:
 //     8 chunks 512 x 512 B4 H5      162 /  117 / 95.8 / 89.5      1024 x 1024 H32                557 /  497 /  465 /  448
 //     256 x 256 H16                 104 / 67.2 / 56.8 / 52.3      512 x 512 H8/1                 201 /  337 /  174 / 90.2
-//     1237 x 1237 B2 H16/8 D80      632 /  605 /  510 /  499      700 x 700 H12 D64              135 / 99.0 / 90.5 / 80.6
+//     1237 x 1237 B2 H16/8 D80      632 /  605 /  510 /  499
+// D 64, * the number chosen:
+//     8 chunks 512 x 512 B4 H5      114 / 84.6 / 71.7 / 62.3*     1024 x 1024 H32                299 /  297 / 249* / 240
+//     256 x 256 H16                91.7 / 61.8 / 52.9 / 48.6*     512 x 512 H8/1                 154 /  248 /  128 / 65.4*
+//     1500 x 1500 B2 H12            558 /  446 / 405* / 392       700 x 700 H12                  136 / 98.6 / 88.0 / 77.9*
 int group_chunks(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks) {
   if (B == 0 || Sq == 0 || Sc == 0) return 1;
   const int64_t nq = tile_map(B * Hq, Sq, kRowsQ / 2).total, nk = tile_map(B * Hkv, Sc, kRowsKv).total;

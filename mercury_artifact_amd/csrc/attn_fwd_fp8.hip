@@ -22,8 +22,8 @@
 // What bounds it: the vector work of the softmax (64 fma, exponentials and adds and 32 conversions per 128 keys and lane,
 // about 1470 cycles beside 1024 of MFMA) and, with both units at work, the board's power.  A tile is therefore handled
 // as two halves, the MFMAs of the halves before and after threaded through the exponentials of the current one: at 16384 x
-// 16384 H32 4.07 M cycles instead of 4.86 M (vector unit 72 % busy instead of 62 %, matrix pipe 52 % instead of 43 %), of
-// which the clock gives a part back (1.88 GHz instead of 2.0): 2078 us instead of 2212.
+// 16384 H32 4.14 M cycles instead of 4.84 M (vector unit 71 % busy instead of 62 %, matrix pipe 51 % instead of 43 %), of
+// which the clock gives a part back (1.79 GHz instead of 1.94 on the box of the counters): 2078 us instead of 2212.
 #include "mhip_common.hpp"
 
 namespace mhip {

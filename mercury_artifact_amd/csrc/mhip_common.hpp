@@ -179,7 +179,7 @@ inline float fold_time(int results, int B, int Sq, int Hq, int D) {
   return results > 1 ? 4.f + (results + 1) * (2.f * B * Sq * Hq * D) / 5.3e6f : 0.f;
 }
 
-// The same for rows of 128 bytes (64 bf16), of which two share the 256 bytes that cover all banks: 16 consecutive rows x one
+// lds_row_swizzle for rows of 128 bytes (64 bf16), of which two share the 256 bytes that cover all banks: 16 consecutive rows x one
 // chunk take each of the 16 places once, and so do 4 rows x 4 consecutive chunks.
 __device__ __forceinline__ constexpr int lds_half_row_swizzle(int row) { return (((row >> 1) & 1) << 2) | ((row >> 2) & 3); }
 

@@ -254,7 +254,8 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
                       "(same result, one pass over the fp32 accumulator per block)", RuntimeWarning, stacklevel=3)
     done = 0
     places = [None] * n_blocks
-    # (a divided ring is one that wants to hold little of other ranks' keys at a time)
+    # (a divided ring goes sub-chunk by sub-chunk whether its chunks are all there or not: the option is for rings that want
+    # to hold little of other ranks' keys at a time)
     if defer and not two_streams and ring_divide == 1:
         together = _Together(n_blocks, q, kv, ring, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra)
         if together.size > 1:
