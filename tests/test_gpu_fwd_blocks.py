@@ -336,6 +336,18 @@ def test_rows_whose_every_score_is_very_low(score, hidden, Sc, D):
         assert ((out[i].float().cpu() - ro).abs() - 2 ** -8 * ro.abs()).max().item() <= 1e-5, i
 
 
+@pytest.mark.parametrize("Sc,D", [(100, 128), (70, 64)])
+def test_rows_that_see_no_key_at_a_very_large_scale(Sc, D):
+    """Rows above the causal diagonal have no score at any scale: out = 0 and LSE = -inf."""
+    import mercury_artifact_amd as M
+
+    g = torch.Generator().manual_seed(Sc)
+    q, k, v = (torch.randn(1, s, 2, D, generator=g).bfloat16().cuda() for s in (130, Sc, Sc))
+    out, lse = M.attn_fwd_block(q, k, v, 2.0 ** 100, True)
+    torch.cuda.synchronize()
+    assert (out[:, :130 - Sc] == 0).all() and (lse[:, :, :130 - Sc] == -math.inf).all()
+
+
 def test_a_ring_whose_chunks_are_one_stacked_tensor():
     """The chunks of all ranks as the first dimension of one tensor, in a step with one result and in one with several."""
     import mercury_artifact_amd as M
