@@ -293,3 +293,42 @@ def test_a_ring_of_another_class_sends_contiguous_chunks():
         ring = (M.LocalRing if key else Sender)((2,), 0, chunks)
         M.flash_attn_pack_kv(q, chunks[0], out[key], lse[key], 0.1, ring=ring)
     assert torch.equal(out[True], out[False]) and torch.equal(lse[True], lse[False])
+
+
+@pytest.mark.parametrize("mesh,S,Hq,Hkv,D,divide", [((4,), 512, 3, 3, 128, 4), ((2, 2), 300, 4, 2, 64, 3), ((8,), 1024, 8, 8, 96, 2)])
+def test_a_divided_ring_of_resident_chunks_takes_them_whole(mesh, S, Hq, Hkv, D, divide):
+    """Bit for bit the undivided step, the ring that was given stays where it was; a wrapper over the hops or the block
+    operator sees every part, and so does a ring whose hops copy."""
+    import mercury_artifact_amd as M
+    from mercury_artifact_amd import flash_attn_interface as FI
+
+    W = 4 if mesh != (8,) else 8
+    g = torch.Generator(device="cuda").manual_seed(divide)
+    q = torch.randn(1, S, Hq, D, generator=g, device="cuda").bfloat16()
+    kvs = [torch.randn(2, 1, S, Hkv, D, generator=g, device="cuda").bfloat16() for _ in range(W)]
+    step = M.flash_attn_pack_split_kv if len(mesh) == 2 else M.gqa_pack_kv
+
+    def run(divide, **kw):
+        o, lse = torch.empty_like(q), torch.empty(1, Hq, S, device="cuda")
+        ring = M.LocalRing(mesh, 1, kvs, **kw)
+        step(q, kvs[1], o, lse, D ** -0.5, ring=ring, ring_divide=divide)
+        return o, lse, ring.held
+
+    whole, parts, copied = run(1), run(divide), run(divide, copy=True)
+    assert torch.equal(whole[0], parts[0]) and torch.equal(whole[1], parts[1])
+    assert parts[2] == list(range(W)) == copied[2]
+    assert (copied[0].float() - whole[0].float()).abs().max().item() <= 2 * 2 ** -8 * whole[0].abs().max().item()
+    seen, real_hop, real_block = [], M.LocalRing.send_recv, FI.attn_fwd_block
+    M.LocalRing.send_recv = lambda self, to, source, x, *a: (seen.append(x.shape[2]), real_hop(self, to, source, x, *a))[1]
+    try:
+        run(divide)
+    finally:
+        M.LocalRing.send_recv = real_hop
+    assert seen == [S // divide] * ((W - 1) * divide)
+    seen.clear()
+    FI.attn_fwd_block = lambda q_, k_, *a, **kw: (seen.append(k_.shape[1]), real_block(q_, k_, *a, **kw))[1]
+    try:
+        run(divide)
+    finally:
+        FI.attn_fwd_block = real_block
+    assert seen == [S // divide] * (W * divide)
