@@ -12,6 +12,8 @@
 //   S^T = K Q^T  : v_mfma_f32_32x32x16_bf16 with A = K rows (LDS), B = Q (registers, loaded once).
 //                  The accumulator layout puts one Q row in each lane (lane % 32) and 32 of the
 //                  64 keys of the tile in that lane's registers, so the softmax is lane-local.
+//                  (Launches bound by the board's power use v_mfma_f32_16x16x32_bf16: two Q rows in
+//                  each lane, 16 keys of each, everything else alike.)
 //   O^T = V^T P^T: the same lane that produced P^T[key][q] feeds it back as the B operand; the
 //                  key order inside one MFMA k-step is whatever the accumulator registers hold, and
 //                  the V^T operand is gathered in exactly that order from the row-major V tile by
@@ -90,22 +92,33 @@ struct FwdChunks : FwdParams {
 // CHAIN: a workgroup visits p.per chunks one after the other, their tiles as one sequence: the ends of a workgroup's life
 // (arguments, Q, first tiles, O out) come once instead of once per chunk, and one result stands for all of them, which the
 // fold would otherwise write and read back as many times.
-template <bool CAUSAL, int KK, int KS, class P, bool CHAIN = false>
+//
+// M = rows and columns of an MFMA tile: v_mfma_f32_32x32x16_bf16 or v_mfma_f32_16x16x32_bf16, which does half as much work in
+// half the time and takes 12 % less energy for it (a register-only loop on random operands under the power cap: 1727 and
+// 1955 TFLOP/s).  Its twice as many instructions cost issue slots that the vector phase of the other wavefront wants, so it
+// pays where the clock is what gives: launches that keep every CU busy for long (small_tiles).
+template <bool CAUSAL, int KK, int KS, class P, bool CHAIN = false, int M = 32>
 __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) {
   constexpr bool kLone = std::is_same<P, FwdParams>::value;
   static_assert(!CHAIN || !kLone, "a run of chunks needs their addresses");
   static_assert(KK == 8 || KK == 6 || KK == 4, "128, 96 or 64 on-chip head-dim columns");
   static_assert(KS == 1 || KS == 2 || KS == 4, "key groups");
   static_assert(!CHAIN || (KS == 1 && !CAUSAL), "chunks are visited one after the other by workgroups of one key group");
-  constexpr int DB = KK / 2;        // blocks of 32 head-dim values in O^T
+  static_assert(M == 32 || (M == 16 && KS == 1), "32 x 32 or 16 x 16 MFMA tiles");
+  constexpr int R = 32 / M;         // row blocks of a wavefront
+  constexpr int NR = M * M / 64;    // registers of an accumulator tile
+  constexpr int KB = KK * M / 32;   // k-steps of 512 / M head-dim values in S^T
+  constexpr int DB = KK * 16 / M;   // blocks of M head-dim values in O^T
+  typedef typename std::conditional<M == 32, f32x16, f32x4>::type Acc;
   constexpr int RG = kWaves / KS;   // row groups of 32
   constexpr int kRows = 32 * RG;    // Q rows of the workgroup
   constexpr int BN = KS == 4 ? 32 : kBN;             // keys per tile
-  constexpr int MB = BN / 32;                        // 32-key blocks per tile
+  constexpr int MB = BN / M;                         // key blocks per tile
   constexpr int kTile = BN * kD * 2;                 // bytes of a tile
   constexpr int kGroupStages = KS == 1 ? kStages : 2;
-  constexpr int kSlotsS = MB * KK;      // matrix-phase slots of S^T
-  constexpr int kSlotsO = 2 * MB * DB;  // and of O^T (k-steps of 16 keys)
+  constexpr int kSlotsS = MB * KB;      // matrix-phase slots of S^T, an operand from LDS and R MFMAs each
+  constexpr int kSteps = BN * M / 512;  // k-steps of 512 / M keys of O^T
+  constexpr int kSlotsO = kSteps * DB;  // and of O^T
   static_assert(KS * kGroupStages * kTile == kStages * kTileBytes, "the K rings take 64 KB, and so do the V rings");
   constexpr int kQBase = 2 * kStages * kTileBytes;   // KS > 1: Q rows, later the O rows on their way out
   __shared__ __attribute__((aligned(16))) unsigned char smem[2 * kStages * kTileBytes + (KS > 1 ? kRows * kD * 2 : 0)];
@@ -151,8 +164,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // scalar: role branches stay uniform
   const int lane = tid & 63;
-  const int ln = lane & 31;
-  const int hf = lane >> 5;
+  const int ln = lane % M;
+  const int lg = lane / M;
   const bool group_b = wave >= 4;                 // second ping-pong group
   const int kg = KS == 1 ? 0 : wave / RG;         // key group
   const int rg = KS == 1 ? wave : wave % RG;      // row group
@@ -171,9 +184,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
     ntiles *= chunks_left + 1;
   }
 
-  // ---- Q fragment: B operand of S^T = K Q^T, lane (ln, hf) holds Q[row][16 ks + 8 hf .. +7] -----
+  // ---- Q fragment: B operand of S^T = K Q^T, lane (ln, lg) holds Q[row][512/M ks + 8 lg .. +7] of rows M r + ln ---
   const int my_q = q0 + rg * 32 + ln;
-  bf16x8 qf[KK];  // loaded in the prologue
+  bf16x8 qf[R][KB];  // loaded in the prologue
 
   // ---- global -> LDS copies of the K and V tiles ---------------------------------------------------
   // A tile is 64 rows of 256 bytes.  Chunk c (16 bytes) of row r lives at chunk position c ^ swz(r):
@@ -269,36 +282,34 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
       copy16_to_lds(vrs, lds_base + kVBase + stage * kTile + u * 1024, vvoff[u], soff);
   };
 
-  // K operand of S^T (A, 32 keys x 16 head-dim values): lane (ln, hf) reads chunk 2 kk + hf of row
-  // 32 mb + ln.
+  // K operand of S^T (A, M keys x 512/M head-dim values): lane (ln, lg) reads chunk 64/M ks + lg of row M mb + ln.
   // k_a and v_a hold the LDS addresses inside the stage that is read next and move on in place, each at a point of the
   // slot sequence where no read of its kind is due; everything else about an address is an immediate offset.
-  int k_a[KK];                                        // + mb * 8192
+  int k_a[KB];                                        // + mb * M rows
 #pragma unroll
-  for (int kk = 0; kk < KK; ++kk) k_a[kk] = (int)lds_ring + ln * 256 + (((2 * kk + hf) ^ swz(ln)) << 4);
-  // V^T operand of O^T (A, 32 head-dim values x 16 keys) for head-dim block db and k-step (mb, j2): the
-  // lane's 8 keys are rows R + {0..3} and R + 8 + {0..3}, R = 32 mb + 16 j2 + 4 hf -- the keys its P
-  // registers hold.  One ds_read_b64_tr_b16 per group of 4 rows: within 16 lanes, lane s supplies the
-  // address of row R + s/4, head-dim values 4 (s%4) .. +3 of the 16-column strip, and receives column s.
-  int v_a[DB][2];                                     // [db][second four rows]  + mb * 8192 + j2 * 4096
+  for (int ks = 0; ks < KB; ++ks) k_a[ks] = (int)lds_ring + ln * 256 + (((64 / M * ks + lg) ^ swz(ln)) << 4);
+  // V^T operand of O^T (A, M head-dim values x 512/M keys) for head-dim block db and k-step t: the lane's 8 keys are rows
+  // X + {0..3} and, 8 (M = 16: 16) rows on, four more, X = 512/M t + 4 lg -- the keys its P registers hold.  One
+  // ds_read_b64_tr_b16 per group of 4 rows: within 16 lanes, lane s supplies the address of row X + s/4, head-dim values 4 (s%4) .. +3 of the
+  // 16-column strip, and receives column s.
+  int v_a[KK];                                        // 32: [2 db + second four rows], 16: [db]; + t * 512/M rows
   {
-    const int s16 = lane & 15, strip = (lane >> 4) & 1;
+    const int s16 = lane & 15, strip = M == 32 ? (lane >> 4) & 1 : 0;
     const int cl = 2 * strip + ((s16 & 3) >> 1);
 #pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int row = 8 * h + 4 * hf + (s16 >> 2);
-        v_a[db][h] = (int)lds_ring + kVBase + row * 256 + (((4 * db + cl) ^ swz(row)) << 4) + (s16 & 1) * 8;
-      }
+    for (int i = 0; i < KK; ++i) {
+      const int db = M == 32 ? i / 2 : i, row = (M == 32 ? 8 * (i & 1) : 0) + 4 * lg + (s16 >> 2);
+      v_a[i] = (int)lds_ring + kVBase + row * 256 + (((M / 8 * db + cl) ^ swz(row)) << 4) + (s16 & 1) * 8;
+    }
   }
   typedef __attribute__((address_space(3))) bf16x4* lds_bf16x4;
   typedef __attribute__((address_space(3))) const bf16x8* lds_bf16x8;
-  auto read_k = [&](int mb, int kk) -> bf16x8 { return *(lds_bf16x8)(uintptr_t)(uint32_t)(k_a[kk] + mb * 8192); };
-  auto read_v = [&](int db, int kstep) -> bf16x8 {
-    const int off = (kstep >> 1) * 8192 + (kstep & 1) * 4096;
-    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(v_a[db][0] + off));
-    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(v_a[db][1] + off));
+  auto read_k = [&](int mb, int ks) -> bf16x8 { return *(lds_bf16x8)(uintptr_t)(uint32_t)(k_a[ks] + mb * M * 256); };
+  auto read_v = [&](int db, int t) -> bf16x8 {
+    const int at = t * (512 / M) * 256;
+    const int first = M == 32 ? v_a[2 * db % KK] : v_a[db], second = M == 32 ? v_a[(2 * db + 1) % KK] : v_a[db] + 4096;
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(first + at));
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(second + at));
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
   // byte distance from the stage of tile t to the stage of tile t + 1
@@ -306,44 +317,51 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
   const int causal_shift = p.Sc - p.Sq;
 
   // ---- accumulators -----------------------------------------------------------------------------
-  f32x16 o_acc[DB];
+  const Acc zero = {};
+  Acc o_acc[DB][R];          // O^T: head-dim values M db + 8 (j / 4) + 4 lg + j % 4 of rows M r + ln
 #pragma unroll
   for (int i = 0; i < DB; ++i)
 #pragma unroll
-    for (int j = 0; j < 16; ++j) o_acc[i][j] = 0.f;
+    for (int r = 0; r < R; ++r) o_acc[i][r] = zero;
   // m_ref: the raw (unscaled) score the exponentials of this lane's Q row are taken relative to.  It is
   // fixed by the first tile's row maximum and moves only when a later tile would overflow: the row sums are
   // watched, not the maxima, so the common path has no maximum, no cross-lane exchange and no rescale of O.
-  float m_ref = 0.f;
-  float nmsc = 0.f;          // -m_ref * scale * log2(e)
-  float l_run = 0.f;         // this lane's share of the running sum (the other 32 keys: lane ^ 32)
+  float m_ref[R] = {};
+  float nmsc[R] = {};        // -m_ref * scale * log2(e)
+  float l_run[R] = {};       // this lane's share of the running sums (the other keys: lanes ^ 32, with M = 16 ^ 16 and ^ 48 too)
+  auto row_sum = [](float x) { return M == 32 ? pair_sum(x) : quad_sum(x); };
   constexpr float kTrigger = 1048576.f;   // a lane's 32 exponentials of one tile sum to less than this, or
   constexpr float kSlack = 14.f;          // rows whose maximum exceeds the reference by 2^kSlack move it
   constexpr float kMost = 0x1.fffffep127f;
-  const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  f32x16 s[MB];              // S^T tile: BN keys x 32 q rows per wave
-  u32x4 pw[2 * MB];          // P^T of the current tile as packed bf16 B operands, one per k-step
+  Acc s[MB][R];              // S^T tile: BN keys x 32 q rows per wave, keys M mb + 8 (j / 4) + 4 lg + j % 4
+  u32x4 pw[kSteps][R];       // P^T of the current tile as packed bf16 B operands
 
+  auto mfma = [](const bf16x8& x, const bf16x8& y, const Acc& c) -> Acc {
+    if constexpr (M == 32) return __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0);
+  };
+  auto s_mfma = [&](int mb, int ks, const bf16x8& kf) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) s[mb][r] = mfma(kf, qf[r][ks], ks == 0 ? zero : s[mb][r]);
+  };
+  auto o_mfma = [&](int db, int t, const bf16x8& vf) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) o_acc[db][r] = mfma(vf, __builtin_bit_cast(bf16x8, pw[t][r]), o_acc[db][r]);
+  };
   auto qk = [&]() {                   // S^T(0); leaves k_a at K(1)
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
+    for (int ks = 0; ks < KB; ++ks) {
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        const bf16x8 kf = read_k(mb, kk);
-        s[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[kk], kk == 0 ? zero : s[mb], 0, 0, 0);
-      }
-      k_a[kk] += kTile;
+      for (int mb = 0; mb < MB; ++mb) s_mfma(mb, ks, read_k(mb, ks));
+      k_a[ks] += kTile;
     }
   };
 
   auto pv = [&]() {
 #pragma unroll
-    for (int kstep = 0; kstep < 2 * MB; ++kstep) {
+    for (int t = 0; t < kSteps; ++t) {
 #pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        const bf16x8 vf = read_v(db, kstep);
-        o_acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, __builtin_bit_cast(bf16x8, pw[kstep]), o_acc[db], 0, 0, 0);
-      }
+      for (int db = 0; db < DB; ++db) o_mfma(db, t, read_v(db, t));
     }
   };
 
@@ -355,82 +373,92 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
     bool need_mask = kv0 + BN > p.Sc;
     if (CAUSAL) need_mask = need_mask || (kv0 + BN - 1 > q0 + causal_shift);
     if (need_mask) {
-      int lim = p.Sc - 1;                                   // last visible key of this lane's row
-      if (CAUSAL) { const int c = my_q + causal_shift; lim = c < lim ? c : lim; }
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
+      for (int r = 0; r < R; ++r) {
+        int lim = p.Sc - 1;                                 // last visible key of this lane's row
+        if (CAUSAL) { const int c = my_q + r * M + causal_shift; lim = c < lim ? c : lim; }
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const int at = mb * 32 + (j >> 2) * 8 + (j & 3);
-          if (CHAIN ? at + hf * 4 > lim - kv0 : kv0 + at + hf * 4 > lim) s[mb][j] = -INFINITY;
-        }
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int j = 0; j < NR; ++j) {
+            const int at = mb * M + (j >> 2) * 8 + (j & 3);
+            if (CHAIN ? at + lg * 4 > lim - kv0 : kv0 + at + lg * 4 > lim) s[mb][r][j] = -INFINITY;
+          }
+      }
     }
   };
-  // Exponentials of the tile in 16 pairs: pair idx covers accumulator registers 2 idx, 2 idx + 1 (counted over
-  // both 32-key blocks) and gives one dword of the packed P^T operand of k-step idx / 4.  s stays intact.
+  // Exponentials of the tile in 16 pairs (eight of a 32-key tile): pair 4 (R t + r) + d gives dword d of the packed P^T operand of
+  // k-step t and row block r.  s stays intact.
   // The first kEarlyPairs pairs are computed inside the matrix phase, between the O^T MFMAs: measured with
   // cycle counters the vector phase is the longer of the two (1314 against 1265 ticks per 64-key tile), and
   // two pairs moved over make the step 3 % faster (four and more slow the matrix phase down by as much as
-  // they shorten the other; on 64 columns, where it has half the MFMAs, six do).  A pair may overwrite the P^T operand of k-step ks only after the last MFMA of
+  // they shorten the other; on 64 columns, where it has half the MFMAs, six do).  A pair may overwrite the P^T operand of k-step t only after the last MFMA of
   // that k-step has been issued.
-  float rs = 0.f;
+  float rs[R] = {};
   auto sm_pair = [&](int idx) {
-    const int mb = idx >> 3, r = (idx & 7) * 2;
-    float x0 = fast_exp2(__builtin_fmaf(s[mb][r], scale_log2, nmsc));
-    float x1 = fast_exp2(__builtin_fmaf(s[mb][r + 1], scale_log2, nmsc));
-    if (idx == 0) rs = x0 + x1; else rs += x0 + x1;
+    const int t = idx / (4 * R), r = (idx >> 2) % R, d = idx & 3, mb = (8 * t + 2 * d) / NR, e = (8 * t + 2 * d) % NR;
+    float x0 = fast_exp2(__builtin_fmaf(s[mb][r][e], scale_log2, nmsc[r]));
+    float x1 = fast_exp2(__builtin_fmaf(s[mb][r][e + 1], scale_log2, nmsc[r]));
+    if (t == 0 && d == 0) rs[r] = x0 + x1; else rs[r] += x0 + x1;
     uint32_t w = pack_bf16(x0, x1);
-    asm volatile("" : "+v"(w), "+v"(rs));          // keeps the pair where it is written
-    pw[idx >> 2][idx & 3] = w;
+    asm volatile("" : "+v"(w), "+v"(rs[r]));       // keeps the pair where it is written
+    pw[t][r][d] = w;
   };
   auto sm_exps = [&]() {
 #pragma unroll
-    for (int idx = 0; idx < 8 * MB; ++idx) sm_pair(idx);
+    for (int idx = 0; idx < BN / 4; ++idx) sm_pair(idx);
   };
   // Move the reference of the rows whose scores outgrew it (first tile: set it to the row maximum) and
   // rescale O and the running sum accordingly.
   auto sm_fix = [&](bool first) {
-    float mx = s[0][0];
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+    for (int r = 0; r < R; ++r) {
+      float mx = s[0][r][0];
 #pragma unroll
-      for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[mb][j]);
-    mx = pair_max(mx);
-    const float grown = (mx - m_ref) * scale_log2;
-    const bool move = first || grown > kSlack;                   // false for NaN
-    if (!first) {
-      const float alpha = move ? fast_exp2(-grown) : 1.f;
+      for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-      for (int db = 0; db < DB; ++db)
+        for (int j = 0; j < NR; ++j) mx = fmaxf(mx, s[mb][r][j]);
+      mx = M == 32 ? pair_max(mx) : quad_max(mx);
+      const float grown = (mx - m_ref[r]) * scale_log2;
+      const bool move = first || grown > kSlack;                 // false for NaN
+      if (!first) {
+        const float alpha = move ? fast_exp2(-grown) : 1.f;
 #pragma unroll
-        for (int j = 0; j < 16; ++j) o_acc[db][j] *= alpha;
-      l_run *= alpha;
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int j = 0; j < NR; ++j) o_acc[db][r][j] *= alpha;
+        l_run[r] *= alpha;
+      }
+      // (with scores of -inf alone it stays at the lowest finite one, so that the first key that counts moves it; the product
+      // stays finite too, so that scores of -inf have exponentials of 0)
+      if (move) m_ref[r] = first ? fmaxf(mx, -kMost) : mx;
+      nmsc[r] = fminf(-m_ref[r] * scale_log2, kMost);
     }
-    // (with scores of -inf alone it stays at the lowest finite one, so that the first key that counts moves it; the product
-    // stays finite too, so that scores of -inf have exponentials of 0)
-    if (move) m_ref = first ? fmaxf(mx, -kMost) : mx;
-    nmsc = fminf(-m_ref * scale_log2, kMost);
   };
-  // slot of the matrix phase after which early pair idx runs: k-step idx / 4 of the tile before is read by the
-  // O^T slots kSlotsS + DB (idx / 4) .. + DB - 1, and the pairs are spread two slots apart behind that
+  // slot of the matrix phase after which early pair idx runs: behind the DB slots of O^T that read k-step 0, whose first row
+  // block the pairs belong to (of 32 x 32 tiles with six pairs: and those of k-step 1), spread over the rest
   constexpr bool kShortMatrix = KS == 1 && KK < 8;
   constexpr int kEarlyPairs = KS == 1 && KK == 4 ? 6 : 2;
   constexpr int kEarlyGap = kEarlyPairs > 2 || MB * DB < 4 ? 1 : 2;
-  auto early_slot = [](int idx) { return kSlotsS + DB + kEarlyGap * idx; };
-  static_assert(DB + kEarlyGap * (kEarlyPairs - 1) < kSlotsO && (kEarlyPairs <= 4 || (DB + kEarlyGap * 4 >= 2 * DB && kEarlyPairs <= 8)),
+  auto early_slot = [](int idx) { return kSlotsS + DB + (M == 32 ? kEarlyGap * idx : idx * (kSlotsO - DB) / kEarlyPairs); };
+  static_assert(M == 16 || (DB + kEarlyGap * (kEarlyPairs - 1) < kSlotsO && (kEarlyPairs <= 4 || (DB + kEarlyGap * 4 >= 2 * DB && kEarlyPairs <= 8))),
                 "the early pairs have to fit behind the O^T slots of their k-steps");
   auto sm_tile = [&]() {
 #pragma unroll
-    for (int idx = kEarlyPairs; idx < 8 * MB; ++idx) sm_pair(idx);
-    if (__builtin_amdgcn_ballot_w64(!(rs < kTrigger)) != 0) {
+    for (int idx = kEarlyPairs; idx < BN / 4; ++idx) sm_pair(idx);
+    float sum = rs[0];
+    if (R == 2) sum += rs[R - 1];
+    if (__builtin_amdgcn_ballot_w64(!(sum < kTrigger)) != 0) {
       sm_fix(false);
       sm_exps();
     }
-    l_run += rs;
+#pragma unroll
+    for (int r = 0; r < R; ++r) l_run[r] += rs[r];
   };
 
-  // Matrix phase of tile t: S^T(t+1) and O^T += V^T(t) P^T(t), kSlotsS + kSlotsO MFMAs (32 on 128 columns and
-  // 64 keys) fed by as many LDS reads.  The reads run kFragDepth operands ahead of the MFMAs through a ring of registers, so the LDS latency is covered by the MFMAs in between.
+  // Matrix phase of tile t: S^T(t+1) and O^T += V^T(t) P^T(t), kSlotsS + kSlotsO operands (32 on 128 columns and 64 keys) from
+  // LDS with R MFMAs each.  The reads run kFragDepth operands ahead through a ring of registers, so the LDS latency is
+  // covered by the MFMAs in between.
   auto read_frag = [&](int i) -> bf16x8 {
     if (i < kSlotsS) return read_k(i % MB, i / MB);
     return read_v((i - kSlotsS) % DB, (i - kSlotsS) / DB);
@@ -442,28 +470,23 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
 #pragma unroll
     for (int i = 0; i < kFragDepth; ++i) frag[i] = read_frag(i);
   };
-  static_assert(kSlotsO >= KK / 2 && kFragDepth * 2 >= 2 * DB, "slots in which the operand addresses move on");
+  static_assert(kSlotsO >= KK / 2 && kFragDepth * 2 >= KK, "slots in which the operand addresses move on");
   auto matrix_phase = [&](int t) {
     const int k_step = stage_step(t + 1), v_step = stage_step(t);
 #pragma unroll
     for (int i = 0; i < kSlotsS + kSlotsO; ++i) {
-      if (i < kSlotsS) {
-        const int mb = i % MB, kk = i / MB;
-        s[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag[i % kFragDepth], qf[kk], kk == 0 ? zero : s[mb], 0, 0, 0);
-      } else {
-        const int db = (i - kSlotsS) % DB, kstep = (i - kSlotsS) / DB;
-        o_acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag[i % kFragDepth], __builtin_bit_cast(bf16x8, pw[kstep]), o_acc[db], 0, 0, 0);
-      }
+      if (i < kSlotsS) s_mfma(i % MB, i / MB, frag[i % kFragDepth]);
+      else o_mfma((i - kSlotsS) % DB, (i - kSlotsS) / DB, frag[i % kFragDepth]);
       if (i + kFragDepth < kSlotsS + kSlotsO) frag[i % kFragDepth] = read_frag(i + kFragDepth);
       // the last K read went out in slot kSlotsS - kFragDepth - 1, the last V read kFragDepth slots before the end
       if (i >= kSlotsS && i < kSlotsS + KK / 2) {
-        k_a[2 * (i - kSlotsS)] += k_step;
-        k_a[2 * (i - kSlotsS) + 1] += k_step;
+#pragma unroll
+        for (int e = 0; e < KB / (KK / 2); ++e) k_a[KB / (KK / 2) * (i - kSlotsS) + e] += k_step;
       }
-      if (i >= kSlotsS + kSlotsO - DB) {
-        const int db = i - (kSlotsS + kSlotsO - DB);
-        v_a[db][0] += v_step;
-        v_a[db][1] += v_step;
+      if (i >= kSlotsS + kSlotsO - KK / 2) {
+        const int at = 2 * (i - (kSlotsS + kSlotsO - KK / 2));
+        v_a[at] += v_step;
+        v_a[at + 1] += v_step;
       }
       // On fewer than 128 columns the vector phase, which is the same length, would hold up a matrix phase that is half or
       // three quarters as long: there the tile copies go out between the S^T MFMAs (K(t) and V(t-1) are read by then,
@@ -496,10 +519,12 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
   };
   auto read_q = [&](int lds_addr) {                // address of the first of the wavefront's 32 rows
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
-      qf[kk] = *(lds_bf16x8)(uintptr_t)(uint32_t)(k_a[kk] - (int)lds_ring + lds_addr);
-      if (kk * 16 + hf * 8 >= p.D) qf[kk] = bf16x8{};
-    }
+    for (int ks = 0; ks < KB; ++ks)
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        qf[r][ks] = *(lds_bf16x8)(uintptr_t)(uint32_t)(k_a[ks] - (int)lds_ring + lds_addr + r * M * 256);
+        if (ks * (512 / M) + lg * 8 >= p.D) qf[r][ks] = bf16x8{};
+      }
   };
 
   if constexpr (KS == 1) {
@@ -523,7 +548,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
       read_q(q_lds);
       // pinned here: otherwise the first use sits inside the main loop and so does the wait for the reads
 #pragma unroll
-      for (int kk = 0; kk < KK; ++kk) asm volatile("" : "+v"(qf[kk]));
+      for (int ks = 0; ks < KB; ++ks)
+#pragma unroll
+        for (int r = 0; r < R; ++r) asm volatile("" : "+v"(qf[r][ks]));
       __builtin_amdgcn_s_barrier();
       copy_k(2, 2);
       if (CHAIN) chain_k();
@@ -536,7 +563,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
       sm_mask(0);
       sm_fix(true);
       sm_exps();
-      l_run = rs;
+#pragma unroll
+      for (int r = 0; r < R; ++r) l_run[r] = rs[r];
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       if (ntiles > 1) first_frags();
@@ -556,7 +584,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
       __builtin_amdgcn_s_setprio(0);
       __builtin_amdgcn_s_barrier();
       // ---- vector phase: softmax(t+1), copies of the tiles ahead ---------------------------------------------
-      asm volatile("" : "+v"(s[0]), "+v"(s[MB - 1]));   // keeps the exponentials behind the barrier
+      for (int r = 0; r < R; ++r) asm volatile("" : "+v"(s[0][r]), "+v"(s[MB - 1][r]));   // keeps the exponentials behind the barrier
       sm_tile();
       if (!kShortMatrix) {
         copy_k(t + 4, t & 3);
@@ -573,11 +601,15 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
     if (!group_b) __builtin_amdgcn_s_barrier();
 
     // ---- epilogue -----------------------------------------------------------------------------------
-    const float l_tot = pair_sum(l_run);
-    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    if (hf == 0 && my_q < p.Sq) {
-      const float lse = l_tot > 0.f ? __builtin_fmaf(fast_log2(l_tot), kLn2, m_ref * p.scale) : -INFINITY;
-      p.lse[blk * p.l_sn + ((int64_t)b * p.Hq + hq) * p.Sq + my_q] = lse;
+    float inv[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const float l_tot = row_sum(l_run[r]);
+      inv[r] = l_tot > 0.f ? 1.f / l_tot : 0.f;
+      if (lg == 0 && my_q + r * M < p.Sq) {
+        const float lse = l_tot > 0.f ? __builtin_fmaf(fast_log2(l_tot), kLn2, m_ref[r] * p.scale) : -INFINITY;
+        p.lse[blk * p.l_sn + ((int64_t)b * p.Hq + hq) * p.Sq + my_q + r * M] = lse;
+      }
     }
 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // zero-filled copies of tiles past the end included
@@ -586,12 +618,14 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        u32x2 w;
-        w[0] = pack_bf16(o_acc[db][4 * g] * inv, o_acc[db][4 * g + 1] * inv);
-        w[1] = pack_bf16(o_acc[db][4 * g + 2] * inv, o_acc[db][4 * g + 3] * inv);
-        *reinterpret_cast<u32x2*>(os + ln * (kOStride * 2) + (db * 32 + g * 8 + hf * 4) * 2) = w;
-      }
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int g = 0; g < NR / 4; ++g) {
+          u32x2 w;
+          w[0] = pack_bf16(o_acc[db][r][4 * g] * inv[r], o_acc[db][r][4 * g + 1] * inv[r]);
+          w[1] = pack_bf16(o_acc[db][r][4 * g + 2] * inv[r], o_acc[db][r][4 * g + 3] * inv[r]);
+          *reinterpret_cast<u32x2*>(os + (r * M + ln) * (kOStride * 2) + (db * M + g * 8 + lg * 4) * 2) = w;
+        }
     __syncthreads();
     {
       const int chunk = lane & 15;
@@ -624,7 +658,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
       sm_mask(0);
       sm_fix(true);
       sm_exps();
-      l_run = rs;
+#pragma unroll
+      for (int r = 0; r < R; ++r) l_run[r] = rs[r];
       asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kCpy) : "memory");         // V(0) and K(1)
       __builtin_amdgcn_s_barrier();
       copy_k(2, 0);
@@ -640,7 +675,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
       __builtin_amdgcn_s_setprio(0);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
-      asm volatile("" : "+v"(s[0]), "+v"(s[MB - 1]));
+      for (int r = 0; r < R; ++r) asm volatile("" : "+v"(s[0][r]), "+v"(s[MB - 1][r]));
       copy_k(t + 3, (t + 1) & 1);
       copy_v(t + 2, t & 1);
       sm_tile();
@@ -657,8 +692,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
     // the head-dim columns it does not finish itself to the group that does (group g: chunks g * kShare .. of 8 columns).
     constexpr int kShare = DB * 4 / KS;                // chunks of 8 columns (4 registers of each lane half) per group
     f32x2* stats = reinterpret_cast<f32x2*>(smem + kQBase);              // [key group][row]
-    const float l_own = pair_sum(l_run);
-    if (hf == 0) stats[kg * kRows + rg * 32 + ln] = f32x2{m_ref, l_own};
+    const float l_own = pair_sum(l_run[0]);
+    if (lg == 0) stats[kg * kRows + rg * 32 + ln] = f32x2{m_ref[0], l_own};
     __syncthreads();
     float m_all = -INFINITY;
     f32x2 st[KS];
@@ -671,8 +706,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
 #pragma unroll
     for (int g = 0; g < KS; ++g)       // (a sum of NaN is no smaller than 0 and goes into the row's)
       l_tot += st[g][1] > 0.f ? st[g][1] * fast_exp2((st[g][0] - m_all) * scale_log2) : st[g][1];
-    const float weight = l_own > 0.f ? fast_exp2((m_ref - m_all) * scale_log2) / l_tot : 0.f;
-    if (kg == 0 && hf == 0 && my_q < p.Sq)
+    const float weight = l_own > 0.f ? fast_exp2((m_ref[0] - m_all) * scale_log2) / l_tot : 0.f;
+    if (kg == 0 && lg == 0 && my_q < p.Sq)
       p.lse[blk * p.l_sn + ((int64_t)b * p.Hq + hq) * p.Sq + my_q] =
           l_tot > 0.f ? __builtin_fmaf(fast_log2(l_tot), kLn2, m_all * p.scale) : -INFINITY;
     // slot (row group, finishing group, giving group): kShare vectors of 64 lanes x 16 bytes
@@ -688,7 +723,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
         const int unit = to * kShare + c;
         f32x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = o_acc[unit >> 2][(unit & 3) * 4 + e] * weight;
+        for (int e = 0; e < 4; ++e) v[e] = o_acc[unit >> 2][0][(unit & 3) * 4 + e] * weight;
         if (to == kg) keep[c] = v;
         else dst[c * 64] = v;
       }
@@ -707,7 +742,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
       u32x2 w;
       w[0] = pack_bf16(keep[c][0], keep[c][1]);
       w[1] = pack_bf16(keep[c][2], keep[c][3]);
-      *reinterpret_cast<u32x2*>(os + ln * 256 + (((kg * kShare + c) ^ swz(ln)) << 4) + hf * 8) = w;
+      *reinterpret_cast<u32x2*>(os + ln * 256 + (((kg * kShare + c) ^ swz(ln)) << 4) + lg * 8) = w;
     }
     __syncthreads();
     {
@@ -726,7 +761,21 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
   }
 }
 
-template <bool CAUSAL, int KK, int KS>
+// Whether the workgroups of a launch with one key group, of `tiles` key tiles each (causal: at most), use 16 x 16 MFMA tiles:
+// those that keep every CU busy, whose time is the board's power, and for long enough that their ends do not count.
+// Measured, us, 32 x 32 / 16 x 16 (workgroups x tiles):
+//     D 128  512 x 512  1644 / 1554   256 x 256   419 /  399   224 x 512   750 /  711   256 x 32  59.6 / 58.6   512 x 8  42.9 / 43.6
+//            160 x 512   595 /  597   288 x 512  1333 / 1344   160 x 20   29.1 / 32.0
+//     D 96   512 x 128   338 /  328   256 x 64   90.0 / 87.1   224 x 64   80.1 / 80.1   256 x 32  46.6 / 46.5   160 x 20  24.3 / 27.0
+//     D 64   512 x 128   257 /  250   256 x 64   68.9 / 66.4   224 x 512   477 /  498   256 x 32  34.8 / 35.7   160 x 20  19.9 / 22.9
+//     causal 4096 x 4096 H32: D 128  122.9 / 117.5   D 96  98.1 / 96.7   D 64  74.6 / 75.5
+bool small_tiles(const FwdParams& p, bool causal, int64_t tiles) {
+  const int64_t total = (int64_t)p.blocks * p.B * p.Hq * ((p.Sq + kBM - 1) / kBM), rounds = (total + 255) / 256;
+  if (causal) return p.D > 96 && tiles >= 64 && total >= 512;
+  return p.D > 96 ? tiles >= 32 && total * 20 >= rounds * 256 * 17 : tiles >= 64 && total * 20 >= rounds * 256 * 19;
+}
+
+template <bool CAUSAL, int KK, int KS, int M = 32>
 void launch_one(FwdChunks& p, hipStream_t stream) {
   const int rows = kBM / KS;
   p.nq_tiles = (p.Sq + rows - 1) / rows;
@@ -737,8 +786,8 @@ void launch_one(FwdChunks& p, hipStream_t stream) {
   p.by_order = Divisor(p.heads_per_xcd > 0 ? p.heads_per_xcd : p.blocks * p.heads);
   const dim3 grid(p.per_xcd * 8), block(kWaves * 64);
   const FwdParams& lone = p;
-  if (p.blocks > 1) hipLaunchKernelGGL((attn_fwd_bf16_d128<CAUSAL, KK, KS, FwdChunks>), grid, block, 0, stream, p);
-  else hipLaunchKernelGGL((attn_fwd_bf16_d128<CAUSAL, KK, KS, FwdParams>), grid, block, 0, stream, lone);
+  if (p.blocks > 1) hipLaunchKernelGGL((attn_fwd_bf16_d128<CAUSAL, KK, KS, FwdChunks, false, M>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((attn_fwd_bf16_d128<CAUSAL, KK, KS, FwdParams, false, M>), grid, block, 0, stream, lone);
 }
 template <int KK>
 void launch_chain(FwdChunks& p, hipStream_t stream) {
@@ -748,10 +797,17 @@ void launch_chain(FwdChunks& p, hipStream_t stream) {
   p.heads_per_xcd = 0;
   p.by_q_tiles = Divisor(p.nq_tiles);
   p.by_order = Divisor(1);
-  hipLaunchKernelGGL((attn_fwd_bf16_d128<false, KK, 1, FwdChunks, true>), dim3(p.per_xcd * 8), dim3(kWaves * 64), 0, stream, p);
+  const dim3 grid(p.per_xcd * 8), block(kWaves * 64);
+  if (small_tiles(p, false, (int64_t)p.per * ((p.Sc + kBN - 1) / kBN)))
+    hipLaunchKernelGGL((attn_fwd_bf16_d128<false, KK, 1, FwdChunks, true, 16>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((attn_fwd_bf16_d128<false, KK, 1, FwdChunks, true>), grid, block, 0, stream, p);
 }
 template <int KK>
 void launch_fwd(FwdChunks& p, bool causal, int groups, hipStream_t stream) {
+  if (groups == 1 && small_tiles(p, causal, (p.Sc + kBN - 1) / kBN)) {
+    if (!causal) return launch_one<false, KK, 1, 16>(p, stream);
+    if constexpr (KK == 8) return launch_one<true, KK, 1, 16>(p, stream);
+  }
   if (causal) {
     if (groups == 4) launch_one<true, KK, 4>(p, stream);
     else if (groups == 2) launch_one<true, KK, 2>(p, stream);

@@ -58,6 +58,20 @@ __device__ __forceinline__ float pair_sum(float x) {
   return a + b;
 }
 
+// the same over the lanes l, l ^ 16, l ^ 32 and l ^ 48
+__device__ __forceinline__ float quad_max(float x) {
+  x = pair_max(x);
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, x), false, false);
+  const unsigned a = r[0], b = r[1];
+  return fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+}
+__device__ __forceinline__ float quad_sum(float x) {
+  x = pair_sum(x);
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, x), false, false);
+  const unsigned a = r[0], b = r[1];
+  return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+}
+
 // sum of x over the lane's group of 16, in all of its lanes
 __device__ __forceinline__ float row16_sum(float x) {
   auto rotated = [](float v, auto n) {
