@@ -106,7 +106,7 @@ template <bool DQ, int WAVES, int KK>
 constexpr int kSmemBytesOf =
     WAVES == 8 ? 3 * kStageBytesOf<DQ, KK> + WAVES * 32 * kRowBytesOf<KK> : kStages * kStageBytesOf<DQ, KK>;
 
-// SPLIT: the workgroups of the pass may share their stationary tile (w.splits).
+// SPLIT: the workgroups of the pass may share their stationary tile (w.splits).  Of several chunks (dQ only) each takes whole ones.
 //
 // CHUNKS: several chunks of a step at once.  The dK / dV pass has a workgroup per key tile of every chunk; a workgroup of
 // the dQ pass visits the chunks one after the other, as the dK / dV pass visits the query heads of a group, so dQ meets the
@@ -115,7 +115,7 @@ template <bool DQ, bool CAUSAL, int KK, int WAVES, bool PREPARED, bool SPLIT, bo
 __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, const int block, unsigned char* smem,
                                          const Chunks* chunks = nullptr) {
   static_assert(DQ || WAVES == 4, "the dK / dV pass has no room for eight wavefronts in a workgroup");
-  static_assert(!CHUNKS || (!SPLIT && !CAUSAL), "launches of several chunks are not split further");
+  static_assert(!CHUNKS || (!(SPLIT && !DQ) && !CAUSAL), "launches of several chunks share the tiles of the dQ pass alone");
   static_assert(PREPARED || WAVES == 8, "the pass that prepares is the one with a launch of its own");
   constexpr int DB = KK / 2;                    // blocks of 32 head-dim values in the accumulators
   constexpr int kWavesWg = WAVES;
@@ -203,7 +203,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   // ---- streamed tiles ---------------------------------------------------------------------------------
   // DQ: K / V rows of kv head hs / group.  Otherwise: Q / dout rows of the `group` query heads that share
   // kv head hs, one head after the other.
-  const int heads_str = DQ ? (CHUNKS ? chunks->n : 1) : p.group;      // (DQ: chunks)
+  int heads_str = DQ ? (CHUNKS ? chunks->n : 1) : p.group;            // (DQ: chunks)
   int first_tile = 0, tiles_per_head = (n_str + kTile - 1) / kTile;
   if (CAUSAL) {
     if (DQ) {   // keys beyond the last row's diagonal are hidden
@@ -219,7 +219,13 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   const int span = tiles_per_head - first_tile;
   // this workgroup's part of the stream: tiles t0 .. t0 + ntiles - 1 of the pass's sequence
   int t0 = 0, ntiles = span * heads_str;
-  if (SPLIT && w.splits > 1) {
+  int first_chunk = 0;
+  if (SPLIT && CHUNKS) {
+    const int part = (chunks->n + w.splits - 1) >> w.log_splits;
+    first_chunk = split * part < chunks->n ? split * part : chunks->n;
+    heads_str = first_chunk + part < chunks->n ? first_chunk + part : chunks->n;
+    ntiles = span * (heads_str - first_chunk);
+  } else if (SPLIT && w.splits > 1) {
     const int all = ntiles, part = (all + w.splits - 1) >> w.log_splits;
     t0 = split * part < all ? split * part : all;
     ntiles = all - t0 < part ? all - t0 : part;
@@ -271,13 +277,13 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   // chunk) instead of a division per tile: every scalar instruction of the loop takes an issue slot of
   // the one wavefront a SIMD runs in the dK / dV pass.
   int cp_soff = 0, cp_ld_soff = 0, cp_ld_voff = 0;
-  int nx_h = SPLIT && !DQ && span > 0 ? t0 / span : 0, nx_t = 0;
-  int nx_r = t0 - nx_h * span;
+  int nx_h = SPLIT && !DQ && span > 0 ? t0 / span : first_chunk, nx_t = 0;
+  int nx_r = SPLIT && CHUNKS ? 0 : t0 - nx_h * span;
   int cur_r = nx_r;                                   // position of the tile being worked on
   const uint32_t ld_rows = (uint32_t)p.B * (uint32_t)p.Hq * (uint32_t)p.Sq;     // the host keeps this below 2^30
   const u32x4 ldrs = rsrc_words((wave & 1) ? p.delta : p.lse2, ld_rows * 4u);
   auto copy_setup = [&]() {
-    const bool live = SPLIT ? nx_t < ntiles : DQ && !CHUNKS ? nx_r < span : nx_h < heads_str;
+    const bool live = SPLIT && !CHUNKS ? nx_t < ntiles : DQ && !CHUNKS ? nx_r < span : nx_h < heads_str;
     const uint32_t hq = DQ ? 0u : (uint32_t)(hs * p.group + (live ? nx_h : 0));
     const uint32_t c0 = (uint32_t)((first_tile + (live ? nx_r : 0)) * kTile);
     // element offsets stay below 2^31 (checked by the host), so 32-bit arithmetic is exact
@@ -815,11 +821,11 @@ __global__ __launch_bounds__(256, KK == 4 ? 2 : 1) void bwd_joint(const BwdParam
 }
 
 // The same for several chunks of a step.  The dQ workgroups, whose chains are the longest, come first.
-template <int KK>
+template <int KK, bool SPLIT>
 __global__ __launch_bounds__(256, KK == 4 ? 2 : 1) void bwd_joint_chunks(const BwdParams p, const TileMap wq, const TileMap wk, const Chunks chunks) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<false, 4, KK>];
   const int first_k = wq.per_xcd * 8;
-  if ((int)blockIdx.x < first_k) bwd_pass<true, false, KK, 4, true, false, true>(p, wq, (int)blockIdx.x, smem, &chunks);
+  if ((int)blockIdx.x < first_k) bwd_pass<true, false, KK, 4, true, SPLIT, true>(p, wq, (int)blockIdx.x, smem, &chunks);
   else bwd_pass<false, false, KK, 4, true, false, true>(p, wk, (int)blockIdx.x - first_k, smem, &chunks);
 }
 
@@ -1029,6 +1035,32 @@ int group_chunks(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks) {
   return best;
 }
 
+// Workgroups that share a query tile of the dQ pass in a launch over n chunks, each with its part of them: the chain of tiles
+// over all chunks is what a launch waits for whose other workgroups leave CUs idle or are soon done.  Their sums meet in
+// bwd_reduce.  Us a step, one workgroup to a tile / as many as chosen:
+//     8 chunks 512 x 512 H4     67.1 / 31.4      200 x 200 H2   39.9 / 20.1      1024 x 1024 H8  141 / 121
+//     4 chunks 1024 x 1024 H4   68.3 / 42.7      256 x 256 H4   22.3 / 18.7
+//     D 64  8 chunks 1024 x 1024 H8  105 / 71.9  700 x 700 H12  77.1 / 61.4      256 x 256 H16  32.7 / 23.7
+// Not where the chip is full of other work (two to a tile): 8 chunks 512 x 512 B4 H5 91.2 / 96.9.
+int chunk_splits(int B, int Sq, int Sc, int Hq, int Hkv, int D, int n) {
+  const float nq = (float)tile_map(B * Hq, Sq, kRowsQ / 2).total, nk = (float)n * tile_map(B * Hkv, Sc, kRowsKv).total;
+  const float tq = (float)((Sc + kTile - 1) / kTile), tk = (float)((Sq + kTile - 1) / kTile) * (Hq / Hkv);
+  const Cost c = joint_cost(D);
+  const float turn = D <= 64 ? 1.f : 7.f;      // us between the workgroups of a CU (on 64 columns the other one runs on)
+  int best = 1;
+  float best_time = 0.f;
+  for (int s = 1; s <= n; s *= 2) {
+    const int64_t bytes = partial_bytes(B, Sq, Hq, D, 1, s);
+    if (bytes > kPartialMost) break;
+    const float share = nq * s + nk < 256.f ? (nq * s + nk) / 256.f : 1.f, step = c.step + share * c.busy;
+    const float chain = c.fixed + (n + s - 1) / s * tq * step, keys = c.fixed + tk * step;
+    const float longest = chain > keys ? chain : keys, spread = (nq * s * (chain + turn) + nk * (keys + turn)) / 256.f;
+    const float time = (longest > spread ? longest : spread) + (s > 1 ? 4.f + 2.f * (float)bytes / 4e6f : 0.f);
+    if (s == 1 || time < 0.95f * best_time) { best = s; best_time = time; }
+  }
+  return best;
+}
+
 template <bool CAUSAL, int KK>
 void launch_bwd(const BwdParams& p, const Plan& plan, float* partial, hipStream_t st) {
   if (plan.joint) {
@@ -1057,12 +1089,16 @@ void launch_bwd(const BwdParams& p, const Plan& plan, float* partial, hipStream_
 }
 
 template <int KK>
-void launch_chunks(const BwdParams& p, const Chunks& chunks, hipStream_t st) {
+void launch_chunks(const BwdParams& p, const Chunks& chunks, float* partial, hipStream_t st) {
   const int rows = p.B * p.Hq * p.Sq;
   if (!p.prepared) hipLaunchKernelGGL(bwd_prepare, dim3((rows + 15) / 16), dim3(256), 0, st, p, rows);
-  const TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ / 2);
+  const int splits = chunk_splits(p.B, p.Sq, p.Sc, p.Hq, p.Hkv, p.D, chunks.n);
+  const TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ / 2, splits, partial);
   const TileMap wk = tile_map(chunks.n * p.B * p.Hkv, p.Sc, kRowsKv);
-  hipLaunchKernelGGL((bwd_joint_chunks<KK>), dim3((wk.per_xcd + wq.per_xcd) * 8), dim3(256), 0, st, p, wq, wk, chunks);
+  const dim3 grid((wk.per_xcd + wq.per_xcd) * 8), block(256);
+  if (splits > 1) hipLaunchKernelGGL((bwd_joint_chunks<KK, true>), grid, block, 0, st, p, wq, wk, chunks);
+  else hipLaunchKernelGGL((bwd_joint_chunks<KK, false>), grid, block, 0, st, p, wq, wk, chunks);
+  if (splits > 1) hipLaunchKernelGGL(bwd_reduce, dim3((rows + 15) / 16), dim3(256), 0, st, p, wq, wk, rows, 0);
 }
 
 // -delta, lse2 and delta, (B, Hq, Sq) fp32 each, every one starting on a 16-byte boundary
@@ -1156,9 +1192,9 @@ int bwd_block(const void* dout, const void* q, const void* k, const void* v,
   const bool causal = mask == MHIP_MASK_CAUSAL;
 
   if (chunks) {
-    if (D <= 64) launch_chunks<4>(p, *chunks, st);
-    else if (D <= 96) launch_chunks<6>(p, *chunks, st);
-    else launch_chunks<8>(p, *chunks, st);
+    if (D <= 64) launch_chunks<4>(p, *chunks, partial, st);
+    else if (D <= 96) launch_chunks<6>(p, *chunks, partial, st);
+    else launch_chunks<8>(p, *chunks, partial, st);
     return launch_status();
   }
   const Plan plan = plan_block(B, Sq, Sc, Hq, Hkv, D, causal);

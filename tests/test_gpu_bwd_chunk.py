@@ -65,6 +65,37 @@ def test_backward_step_carries_the_sums(W, S, Hq, Hkv, D, dq_dtype, keep):
         _close(f"dkv {c}", got[c], torch.stack(tuple(rdkv[c])))
 
 
+@pytest.mark.parametrize("W,S,Hq,Hkv,D", [(8, 130, 2, 2, 128), (5, 200, 4, 2, 112), (7, 193, 3, 3, 96), (8, 65, 2, 1, 40), (3, 700, 2, 2, 64),
+                                          (6, 257, 1, 1, 72), (36, 64, 1, 1, 128)])
+@pytest.mark.parametrize("dq_dtype", [torch.bfloat16, torch.float32])
+def test_a_query_tile_shared_by_workgroups_of_a_step(W, S, Hq, Hkv, D, dq_dtype):
+    """Steps of a few heads, whose chain of tiles over all chunks is shared by several workgroups: chunk counts that do and do
+    not divide among them, ragged rows, and (36 chunks) launches that carry the sum on; twice the same bits."""
+    import mercury_artifact_amd as M
+
+    print(f"shared W{W} S{S} Hq{Hq} Hkv{Hkv} D{D} {dq_dtype}", flush=True)
+    B, rank, scale = 1, 1, D ** -0.5
+    assert N.lib().mhip_attn_bwd_group(B, S, S, Hq, Hkv, D, W) >= min(W, 12)
+    g = torch.Generator().manual_seed(W * 1000 + S)
+    q, dout = (torch.randn(B, S, Hq, D, generator=g).bfloat16() for _ in range(2))
+    kvs = [torch.randn(2, B, S, Hkv, D, generator=g).bfloat16() for _ in range(W)]
+    order = O.single_ring_order(rank, W)
+    o, lse = O.ring_forward(q.float(), [c.float() for c in kvs], order, scale)
+    rdq, rdkv = O.ring_backward(q.float(), [c.float() for c in kvs], order, o.bfloat16().float(), lse, dout.float(), scale)
+    dev, runs = [c.cuda() for c in kvs], []
+    for _ in range(2):
+        dq = torch.full(q.shape, float("nan"), dtype=dq_dtype, device="cuda")
+        dkv, got = torch.full_like(dev[rank], float("nan")), {}
+        M.flash_attn_backward(q.cuda(), dev[rank], o.bfloat16().cuda(), lse.cuda(), dout.cuda(), dq, dkv, scale,
+                              ring=M.LocalRing((W,), rank, dev), dkv_chunks=got)
+        torch.cuda.synchronize()
+        runs.append(dq)
+    assert torch.equal(*runs)
+    _close("dq", dq, rdq)
+    for c in range(W):
+        _close(f"dkv {c}", got[c], torch.stack(tuple(rdkv[c])))
+
+
 def _block(B, Sq, Sc, Hq, Hkv, D, causal, launches=1, shared=None):
     import mercury_artifact_amd as M
 
