@@ -111,13 +111,24 @@ constexpr int kSmemBytesOf =
 // CHUNKS: several chunks of a step at once.  The dK / dV pass has a workgroup per key tile of every chunk; a workgroup of
 // the dQ pass visits the chunks one after the other, as the dK / dV pass visits the query heads of a group, so dQ meets the
 // sum carried from launch to launch once per launch instead of once per chunk.
-template <bool DQ, bool CAUSAL, int KK, int WAVES, bool PREPARED, bool SPLIT, bool CHUNKS = false>
+//
+// M = rows and columns of an MFMA tile, as in the forward kernel: v_mfma_f32_32x32x16_bf16, or v_mfma_f32_16x16x32_bf16, which
+// takes less energy for the same work.  With it a lane holds two stationary rows (R), and an operand from LDS feeds an MFMA of each.
+// For the dQ pass of eight wavefronts alone, which runs against the board's power (small_tiles); the dK / dV pass has one
+// wavefront per SIMD to issue everything, takes 20 % more cycles with twice as many MFMAs and is no faster (4096 x 4096 H32 440 us / 444).
+template <bool DQ, bool CAUSAL, int KK, int WAVES, bool PREPARED, bool SPLIT, bool CHUNKS = false, int M = 32>
 __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, const int block, unsigned char* smem,
                                          const Chunks* chunks = nullptr) {
   static_assert(DQ || WAVES == 4, "the dK / dV pass has no room for eight wavefronts in a workgroup");
   static_assert(!CHUNKS || (!(SPLIT && !DQ) && !CAUSAL), "launches of several chunks share the tiles of the dQ pass alone");
   static_assert(PREPARED || WAVES == 8, "the pass that prepares is the one with a launch of its own");
-  constexpr int DB = KK / 2;                    // blocks of 32 head-dim values in the accumulators
+  static_assert(M == 32 || (M == 16 && DQ && WAVES == 8 && KK > 4), "32 x 32 or, in the dQ pass, 16 x 16 MFMA tiles");
+  constexpr int R = 32 / M;                     // blocks of M stationary rows of a wavefront
+  constexpr int NR = M * M / 64;                // registers of an accumulator tile
+  constexpr int MB = 32 / M;                    // blocks of M streamed rows in half a tile
+  constexpr int KB = KK * M / 32;               // k-steps of 512 / M head-dim values in T1 / T2
+  constexpr int DB = KK * 16 / M;               // blocks of M head-dim values in the accumulators
+  typedef typename std::conditional<M == 32, f32x16, f32x4>::type Acc;
   constexpr int kWavesWg = WAVES;
   constexpr int kRowsPerWg = kWavesWg * 32;
   constexpr int kRow = kRowBytesOf<KK>;
@@ -129,7 +140,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   constexpr int kStageBytes = kStageBytesOf<DQ, KK>;
   constexpr int kOffY = kTileBytes, kOffLse = 2 * kTileBytes, kOffDelta = kOffLse + kTile * 4;
   // chunk c (16 bytes) of row r of a tile is kept at chunk position c ^ swz(r)
-  auto swz = [](int row) { return kRow == 256 ? lds_row_swizzle(row) : lds_half_row_swizzle(row); };
+  auto swz = [](int row) { return M == 16 ? lds_row_swizzle_16(row) : kRow == 256 ? lds_row_swizzle(row) : lds_half_row_swizzle(row); };
   // The stationary rows pass through LDS on their way into registers, in one stage each; with eight wavefronts X takes
   // the last stage and 32 KB behind it and Y the two stages before.
   constexpr int kXRows = 3 * kStageBytes, kYRows = WAVES == 8 ? kStageBytes : 2 * kStageBytes;
@@ -190,15 +201,15 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
-  const int ln = lane & 31;
-  const int hf = lane >> 5;
-  const int my_r = r0 + wave * 32 + ln;             // this lane's stationary row
+  const int ln = lane % M;
+  const int lg = lane / M;
+  const int my_r = r0 + wave * 32 + ln;             // this lane's (first) stationary row; the other one is M further
 
-  // ---- stationary operands: B operands of T1 / T2, lane (ln, hf) holds row[16 ks + 8 hf .. +7]; for dQ the
+  // ---- stationary operands: B operands of T1 / T2, lane (ln, lg) holds row[512/M ks + 8 lg .. +7]; for dQ the
   // query is the stationary row and its lse2 / delta are per-lane scalars.  All loaded further down, behind
   // the first tile copies, so that one wait covers both latencies. ---------------------------------------
-  bf16x8 xf[KK], yf[KK];
-  float lse2_lane = 0.f, delta_lane = 0.f;
+  bf16x8 xf[R][KB], yf[R][KB];
+  float lse2_lane[R] = {}, delta_lane[R] = {};
 
   // ---- streamed tiles ---------------------------------------------------------------------------------
   // DQ: K / V rows of kv head hs / group.  Otherwise: Q / dout rows of the `group` query heads that share
@@ -316,34 +327,32 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     for (int piece = 0; piece < kCopiesPerTile; ++piece) copy_piece(piece, stage);
   };
 
-  // row-major operand reads (A of T1 / T2): lane (ln, hf) reads chunk 2 kk + hf of row 32 mb + ln
-  int rm_rd[KK];                                      // + mb * 32 rows
+  // row-major operand reads (A of T1 / T2): lane (ln, lg) reads chunk 64/M kk + lg of row M mb + ln
+  int rm_rd[KB];                                      // + mb * M rows
 #pragma unroll
-  for (int kk = 0; kk < KK; ++kk) rm_rd[kk] = ln * kRow + (((2 * kk + hf) ^ swz(ln)) << 4);
-  // transposed operand reads (A of the second MFMAs) for head-dim block db and k-step (mb, j2): the lane's
-  // 8 streamed rows are R + {0..3} and R + 8 + {0..3}, R = 32 mb + 16 j2 + 4 hf -- the rows its P / dS
+  for (int kk = 0; kk < KB; ++kk) rm_rd[kk] = ln * kRow + (((64 / M * kk + lg) ^ swz(ln)) << 4);
+  // transposed operand reads (A of the second MFMAs) for head-dim block db and k-step j2 of 512/M streamed rows of a half: the
+  // lane's 8 rows are X + {0..3} and, 8 (M = 16: 16) rows on, four more, X = 512/M j2 + 4 lg -- the rows its P / dS
   // registers hold.  One ds_read_b64_tr_b16 per group of 4 rows: within 16 lanes, lane s supplies the
-  // address of row R + s/4, head-dim values 4 (s%4) .. +3 of the 16-column strip, and receives column s.
-  int tr_rd[DB][2];                                   // [db][second four rows]  + mb * 32 rows + j2 * 16 rows
+  // address of row X + s/4, head-dim values 4 (s%4) .. +3 of the 16-column strip, and receives column s.
+  int tr_rd[KK];                                      // 32: [2 db + second four rows], 16: [db]; + j2 * 512/M rows
   {
-    const int s16 = lane & 15, strip = (lane >> 4) & 1;
+    const int s16 = lane & 15, strip = M == 32 ? (lane >> 4) & 1 : 0;
     const int cl = 2 * strip + ((s16 & 3) >> 1);
 #pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int row = 8 * h + 4 * hf + (s16 >> 2);
-        tr_rd[db][h] = row * kRow + (((4 * db + cl) ^ swz(row)) << 4) + (s16 & 1) * 8;
-      }
+    for (int i = 0; i < KK; ++i) {
+      const int db = M == 32 ? i / 2 : i, row = (M == 32 ? 8 * (i & 1) : 0) + 4 * lg + (s16 >> 2);
+      tr_rd[i] = row * kRow + (((M / 8 * db + cl) ^ swz(row)) << 4) + (s16 & 1) * 8;
+    }
   }
   typedef __attribute__((address_space(3))) bf16x4* lds_bf16x4;
   typedef __attribute__((address_space(3))) const bf16x8* lds_bf16x8;
-  f32x16 acc1[DB], acc2[DB];    // DQ: acc1 = dQ^T.  Otherwise acc1 = dK^T, acc2 = dV^T
+  const Acc zero = {};
+  Acc acc1[DB][R], acc2[DB][R];    // DQ: acc1 = dQ^T.  Otherwise acc1 = dK^T, acc2 = dV^T
 #pragma unroll
   for (int i = 0; i < DB; ++i)
 #pragma unroll
-    for (int j = 0; j < 16; ++j) { acc1[i][j] = 0.f; acc2[i][j] = 0.f; }
-  const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < R; ++r) acc1[i][r] = acc2[i][r] = zero;
 
   // Tile t lives in stage t % 4 and is processed as two halves of 32 streamed rows.  Per tile the matrix
   // pipe sees one unbroken sequence of MFMA slots in four phases (half as many slots in each on 64 columns, three quarters on 96):
@@ -359,8 +368,12 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   // stays the same.
   // operand reads in flight ahead of the MFMAs (2, 4 and 8 measure the same; 2 keeps eight wavefronts inside 256 registers)
   constexpr int kDepth = WAVES == 8 ? 2 : 4;
-  constexpr int kT = 2 * KK;                               // slots of a T1 / T2 phase
-  constexpr int kAcc = DQ ? 2 * DB : 4 * DB;               // slots of an accumulate phase
+  constexpr int kT = 2 * KK;                               // slots of a T1 / T2 phase, an operand from LDS and R MFMAs each
+  constexpr int kAcc = DQ ? KK : 2 * KK;                   // slots of an accumulate phase
+  // 16 x 16 tiles: P / dS of the second row block are due with the first operand of an accumulate phase, where 32 x 32 tiles
+  // need the second k-step's half a phase later.  Its MFMAs run kLag slots behind the first block's, those of the last
+  // kLag operands in the T1 / T2 phase that follows; the operands stay in the ring for as long.
+  constexpr int kLag = M == 16 ? kDepth : 0, kRing = kDepth + kLag;
   constexpr int kP1 = kT, kP2 = kT + kAcc, kP3 = 2 * kT + kAcc, kSlots = 2 * (kT + kAcc);
   // The 16 steps of the vector pipeline are spread over the slots of a T1 / T2 phase: slot i runs steps vec0(i) .. vec0(i + 1) - 1.
   auto vec0 = [](int i) -> int { return i * 16 / kT; };
@@ -372,63 +385,81 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   // those of the next tile start at slot kP2 - kDepth; tr_a in the last kDepth slots, after the last transposed read).
   // ld_cur / ld_next address lse2 / -delta of the current and the next tile.  Everything else about an address
   // is an immediate offset of the LDS instruction.
-  int rm_a[KK], tr_a[DB][2];
+  int rm_a[KB], tr_a[KK];
 #pragma unroll
-  for (int kk = 0; kk < KK; ++kk) rm_a[kk] = rm_rd[kk] + (int)lds_base;
+  for (int kk = 0; kk < KB; ++kk) rm_a[kk] = rm_rd[kk] + (int)lds_base;
 #pragma unroll
-  for (int db = 0; db < DB; ++db) { tr_a[db][0] = tr_rd[db][0] + (int)lds_base; tr_a[db][1] = tr_rd[db][1] + (int)lds_base; }
-  int ld_cur = (int)lds_base + hf * 16, ld_next = ld_cur + kStageBytes;
-  // slot i of the T1 / T2 sequence of one half: k-step i / 2, X (T1) on even and Y (T2) on odd slots
-  auto read_rm = [&](int mb, int i) -> bf16x8 {
-    return *(lds_bf16x8)(uintptr_t)(uint32_t)(rm_a[i >> 1] + mb * (32 * kRow) + ((i & 1) ? kOffY : 0));
+  for (int i = 0; i < KK; ++i) tr_a[i] = tr_rd[i] + (int)lds_base;
+  int ld_cur = (int)lds_base + lg * 16, ld_next = ld_cur + kStageBytes;
+  auto mfma = [](const bf16x8& x, const bf16x8& y, const Acc& c) -> Acc {
+    if constexpr (M == 32) return __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0);
   };
-  // T2 starts from -delta of the half's streamed rows (dQ pass: of this lane's stationary row), so that what
+  // slot i of the T1 / T2 sequence of one half: k-step i / (2 MB), X (T1) on even and Y (T2) on odd slots
+  auto read_rm = [&](int half, int i) -> bf16x8 {
+    return *(lds_bf16x8)(uintptr_t)(uint32_t)(rm_a[i / (2 * MB)] + (half * 32 + (i >> 1) % MB * M) * kRow + ((i & 1) ? kOffY : 0));
+  };
+  // T1 / T2 of a half: streamed rows M mb + 8 (j / 4) + 4 lg + j % 4 against stationary rows M r + ln
+  struct Scores {
+    Acc a[MB][R];
+    // the order of the vector work: elements 8 i .. 8 i + 7 make B operand i of the second MFMAs, k-step i (M = 16: row block i)
+    __device__ __forceinline__ static constexpr int r_of(int e) { return M == 32 ? 0 : e >> 3; }
+    __device__ __forceinline__ static constexpr int mb_of(int e) { return M == 32 ? 0 : (e >> 2) & 1; }
+    __device__ __forceinline__ static constexpr int j_of(int e) { return e % NR; }
+    __device__ __forceinline__ float get(int e) const { return a[mb_of(e)][r_of(e)][j_of(e)]; }
+    __device__ __forceinline__ void set(int e, float x) { a[mb_of(e)][r_of(e)][j_of(e)] = x; }
+  };
+  // T2 starts from -delta of the half's streamed rows (dQ pass: of this lane's stationary rows), so that what
   // the vector unit receives is dP - delta already
-  f32x16 nd;
-  auto t_mfma = [&](int i, const bf16x8& a, f32x16& n1, f32x16& n2) {
-    const int kk = i >> 1;
-    if (i & 1) n2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, yf[kk], kk == 0 ? nd : n2, 0, 0, 0);
-    else n1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, xf[kk], kk == 0 ? zero : n1, 0, 0, 0);
+  Acc nd[R];
+  auto t_mfma = [&](int i, int r, const bf16x8& a, Scores& n1, Scores& n2) {
+    const int kk = i / (2 * MB), mb = (i >> 1) % MB;
+    if (i & 1) n2.a[mb][r] = mfma(a, yf[r][kk], kk == 0 ? nd[r] : n2.a[mb][r]);
+    else n1.a[mb][r] = mfma(a, xf[r][kk], kk == 0 ? zero : n1.a[mb][r]);
   };
-  // slot i of an accumulate phase of half mb: head-dim block and k-step, X^T (dS) / Y^T (P) alternating for dK, dV
-  auto read_acc = [&](int mb, int i) -> bf16x8 {
+  // slot i of an accumulate phase of a half: head-dim block and k-step, X^T (dS) / Y^T (P) alternating for dK, dV
+  auto read_acc = [&](int half, int i) -> bf16x8 {
     const int m = DQ ? i : (i >> 1);
-    const int off = mb * (32 * kRow) + (m / DB) * (16 * kRow) + ((!DQ && (i & 1)) ? kOffY : 0);
-    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(tr_a[m % DB][0] + off));
-    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(tr_a[m % DB][1] + off));
+    const int off = half * (32 * kRow) + (m / DB) * (512 / M * kRow) + ((!DQ && (i & 1)) ? kOffY : 0);
+    const int first = M == 32 ? tr_a[2 * (m % DB) % KK] : tr_a[m % DB], second = M == 32 ? tr_a[(2 * (m % DB) + 1) % KK] : tr_a[m % DB] + 16 * kRow;
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(first + off));
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4)(uintptr_t)(uint32_t)(second + off));
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
 
-  bf16x8 pfrag[2], dsfrag[2];     // P and dS of the half being accumulated as B operands (two k-steps)
-  bf16x8 ring[kDepth];
-  f32x16 ta1, ta2, tb1, tb2;      // T1 / T2 of the two halves in flight: (t, first half), (t, second half)
+  bf16x8 pfrag[2] = {}, dsfrag[2] = {};     // P and dS of the half being accumulated as B operands (two k-steps or row blocks)
+  bf16x8 ring[kRing] = {};
+  Scores ta1, ta2, tb1, tb2;      // T1 / T2 of the two halves in flight: (t, first half), (t, second half)
   f32x4 lv[5];                    // lse2 of 4 streamed rows per entry (dK / dV pass), read one group ahead
 
   // Hidden elements (rows past the end of the streamed tensor, the causal mask) get a score of -inf,
   // hence P = dS = 0.  Only the last tile of a head and the tiles the diagonal crosses need it.
-  auto mask_half = [&](f32x16& c1, int cb) {
+  auto mask_half = [&](Scores& c1, int cb) {
     bool need_mask = cb + 32 > n_str;
     if (CAUSAL) need_mask = need_mask || (DQ ? (cb + 31 > r0 + shift) : (r0 + kRowsPerWg - 1 > cb + shift));
     if (need_mask) {
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int c = cb + (j >> 2) * 8 + hf * 4 + (j & 3);     // streamed row of this element
+      for (int e = 0; e < 16; ++e) {
+        const int j = c1.j_of(e), c = cb + c1.mb_of(e) * M + (j >> 2) * 8 + lg * 4 + (j & 3);     // streamed row of this element
         bool hidden = c >= n_str;
-        if (CAUSAL) hidden = hidden || (DQ ? (c > my_r + shift) : (my_r > c + shift));
-        if (hidden) c1[j] = -INFINITY;
+        if (CAUSAL) {
+          const int row = my_r + c1.r_of(e) * M;
+          hidden = hidden || (DQ ? (c > row + shift) : (row > c + shift));
+        }
+        if (hidden) c1.set(e, -INFINITY);
       }
     }
   };
-  // lse2 of rows 8 g + 4 hf .. + 3 of half mb of the current (next: of the following) tile
-  auto read_ld = [&](bool next, int mb, int g, f32x4& l) {
-    l = *(lds_f32x4)(uintptr_t)(uint32_t)((next ? ld_next : ld_cur) + kOffLse + (mb * 32 + g * 8) * 4);
+  // lse2 of rows 8 g + 4 lg .. + 3 of a half of the current (next: of the following) tile
+  auto read_ld = [&](bool next, int half, int g, f32x4& l) {
+    l = *(lds_f32x4)(uintptr_t)(uint32_t)((next ? ld_next : ld_cur) + kOffLse + (half * 32 + g * 8) * 4);
   };
-  // -delta of rows 8 g + 4 hf .. + 3 (g = 0..3) of half mb of the current / following tile, in the order of the
+  // -delta of rows 8 g + 4 lg .. + 3 (g = 0..3) of a half of the current / following tile, in the order of the
   // accumulator registers of T2 (dK / dV pass), one group per call
-  auto read_nd = [&](bool next, int mb, int g) {
-    const f32x4 d = *(lds_f32x4)(uintptr_t)(uint32_t)((next ? ld_next : ld_cur) + kOffDelta + (mb * 32 + g * 8) * 4);
+  auto read_nd = [&](bool next, int half, int g) {
+    const f32x4 d = *(lds_f32x4)(uintptr_t)(uint32_t)((next ? ld_next : ld_cur) + kOffDelta + (half * 32 + g * 8) * 4);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) nd[4 * g + e] = d[e];
+    for (int e = 0; e < 4; ++e) nd[0][(4 * g + e) % NR] = d[e];
   };
   // P / dS of the half in (c1, c2): 16 accumulator registers, spread over the 16 slots in which the next
   // half's T1 / T2 are issued AND the first slots of the accumulate phase that follows (a wavefront issues
@@ -438,50 +469,64 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   //   first_slot      argument of the exponential
   //   first_slot + 1  exponential
   //   first_slot + 2  dS = P (dP - delta)     (c2 arrives as dP - delta)
-  // Registers 0-7 (k-step 0 of the accumulate phase) are packed before that phase starts, registers 8-15
-  // before its second half does.
+  // Registers 0-7 (k-step or row block 0 of the accumulate phase) are packed before that phase starts, registers 8-15
+  // before its second half does (M = 16: before slot kLag of it).
+  // With 16 x 16 tiles a stage takes two half slots, one behind each of a slot's two MFMAs: behind both, its instructions
+  // leave the matrix unit less to do meanwhile (4.98 M cycles instead of 4.89 M for 4096 x 4096 H32).
   auto first_slot = [](int e) -> int {
+    if (M == 16) return e < 8 ? (e * 5) / 2 : 2 * e - 2;     // half slots: 0,2,5,..,17 | 14,16,..,28: packed up to 23 and 34
     if (DQ) return e < 8 ? (e * 3) / 2 : 1 + e;          // 0,1,3,4,6,7,9,10 | 9..16: packed at slots 13 and 19 (acc 16-19, 20-23)
     return e < 8 ? (e * 7) / 4 : 5 + e;                  // 0,1,3,5,7,8,10,12 | 13..20: packed at slots 15 and 23 (acc 16-23, 24-31)
   };
   float earg[16];
-  auto vector_slot = [&](int s, f32x16& c1, f32x16& c2, int mb) {
+  auto vector_slot = [&](int s, Scores& c1, Scores& c2, int half) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       const int f = first_slot(e);
       if (s == f) {
-        const float l = DQ ? lse2_lane : lv[e >> 2][e & 3];
-        earg[e] = __builtin_fmaf(c1[e], p.scale_log2, -l);
+        const float l = DQ ? lse2_lane[c1.r_of(e)] : lv[e >> 2][e & 3];
+        earg[e] = __builtin_fmaf(c1.get(e), p.scale_log2, -l);
         // lse2 of the next four rows, one group ahead
-        if (!DQ && (e & 3) == 0 && e < 12) read_ld(false, mb, (e >> 2) + 1, lv[(e >> 2) + 1]);
+        if (!DQ && (e & 3) == 0 && e < 12) read_ld(false, half, (e >> 2) + 1, lv[(e >> 2) + 1]);
       }
-      if (s == f + 1) c1[e] = fast_exp2(earg[e]);
-      if (s == f + 2) c2[e] = c1[e] * c2[e];
+      if (s == f + R) c1.set(e, fast_exp2(earg[e]));
+      if (s == f + 2 * R) c2.set(e, c1.get(e) * c2.get(e));
     }
+    // M = 32: the eight elements of an operand at once, M = 16: two at a time
 #pragma unroll
-    for (int j2 = 0; j2 < 2; ++j2)
-      if (s == first_slot(8 * j2 + 7) + 3) {
-        u32x4 wp, wd;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          wp[e] = pack_bf16(c1[8 * j2 + 2 * e], c1[8 * j2 + 2 * e + 1]);
-          wd[e] = pack_bf16(c2[8 * j2 + 2 * e], c2[8 * j2 + 2 * e + 1]);
-        }
-        pfrag[j2] = __builtin_bit_cast(bf16x8, wp);
-        dsfrag[j2] = __builtin_bit_cast(bf16x8, wd);
+    for (int e = 0; e < 16; e += 2)
+      if (s == first_slot(M == 32 ? e | 7 : e + 1) + 3 * R) {
+        u32x4 wp = __builtin_bit_cast(u32x4, pfrag[e >> 3]), wd = __builtin_bit_cast(u32x4, dsfrag[e >> 3]);
+        wp[(e >> 1) & 3] = pack_bf16(c1.get(e), c1.get(e + 1));
+        wd[(e >> 1) & 3] = pack_bf16(c2.get(e), c2.get(e + 1));
+        pfrag[e >> 3] = __builtin_bit_cast(bf16x8, wp);
+        dsfrag[e >> 3] = __builtin_bit_cast(bf16x8, wd);
       }
   };
-  // steps 16 .. of the vector pipeline, behind the T1 / T2 phase, run in the first slots of the accumulate phase
-  auto vector_tail = [&](int i, f32x16& c1, f32x16& c2, int mb) {
+  // the vector work behind MFMA r of slot i of a T1 / T2 phase, and of the accumulate phase that follows (steps 16 ..)
+  auto vector_t = [&](int i, int r, Scores& c1, Scores& c2, int half) {
+#pragma unroll
+    for (int v = vec0(i); v < vec0(i + 1); ++v) vector_slot(M == 32 ? v : 2 * v + r, c1, c2, half);
+  };
+  auto vector_tail = [&](int i, int r, Scores& c1, Scores& c2, int half) {
 #pragma unroll
     for (int v = vec0(i); v < vec0(i + 1); ++v)
-      if (v < (DQ ? 4 : 8)) vector_slot(16 + v, c1, c2, mb);
+      if (v < (DQ ? 4 : 8)) vector_slot(M == 32 ? 16 + v : 2 * (16 + v) + r, c1, c2, half);
   };
-  auto acc_mfma = [&](int i, const bf16x8& a) {
+  auto acc_one = [&](int i, int r, const bf16x8& a) {
     const int m = DQ ? i : (i >> 1);
-    const int db = m % DB, j2 = m / DB;
-    if (DQ || !(i & 1)) acc1[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, dsfrag[j2], acc1[db], 0, 0, 0);
-    else acc2[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pfrag[j2], acc2[db], 0, 0, 0);
+    const int db = m % DB, at = M == 32 ? m / DB : r;
+    if (DQ || !(i & 1)) acc1[db][r] = mfma(a, dsfrag[at], acc1[db][r]);
+    else acc2[db][r] = mfma(a, pfrag[at], acc2[db][r]);
+  };
+  // MFMA r of slot i of an accumulate phase that starts at slot `phase` of the tile
+  auto acc_mfma = [&](int i, int r, int phase) {
+    if (r == 0) acc_one(i, 0, ring[(phase + i) % kRing]);
+    else if (i >= kLag) acc_one(i - kLag, 1, ring[(phase + i - kLag) % kRing]);
+  };
+  // and the second row block's last MFMAs, in slot i of the T1 / T2 phase behind it
+  auto acc_rest = [&](int i, int phase) {
+    if (i < kLag) acc_one(kAcc - kLag + i, R - 1, ring[(phase + kAcc - kLag + i) % kRing]);
   };
   // LDS operand of slot s of the current tile's sequence; s >= kSlots continues into the next tile's P0.  The
   // T1 / T2 operands of slots kP2 .. kP3 - 1 and from kSlots on belong to the next tile: rm_a has moved on by then.
@@ -492,6 +537,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     if (s < kP3) return read_rm(0, s - kP2);
     return read_acc(1, s - kP3);
   };
+  auto refill = [&](int s) { ring[(s + kDepth) % kRing] = read_slot(s + kDepth); };
   static_assert(kP2 - kDepth >= kT && kAcc >= kDepth, "rm_a moves in the last kDepth slots of P0, tr_a in the last kDepth slots of P3");
 
   // Stationary rows: read straight into the fragment layout every load instruction would touch 32 rows (24 such loads
@@ -517,12 +563,14 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
         copy16_to_lds(src + (int64_t)row_of(u) * st_ss + (col < p.D ? col : 0), dst + u * 1024);
       }
     };
-    auto read_rows = [&](uint32_t src, bf16x8 (&f)[KK]) {
+    auto read_rows = [&](uint32_t src, bf16x8 (&f)[R][KB]) {
 #pragma unroll
-      for (int ks = 0; ks < KK; ++ks) {
-        f[ks] = *(lds_bf16x8)(uintptr_t)(src + rm_rd[ks]);
-        if (ks * 16 + hf * 8 >= p.D) f[ks] = bf16x8{};
-      }
+      for (int ks = 0; ks < KB; ++ks)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          f[r][ks] = *(lds_bf16x8)(uintptr_t)(src + rm_rd[ks] + r * M * kRow);
+          if (ks * (512 / M) + lg * 8 >= p.D) f[r][ks] = bf16x8{};
+        }
     };
     // Pin the fragments (the copies are invisible to the compiler's wait counting).  The dK / dV pass keeps these
     // MFMA operands in accumulation registers: its arithmetic registers are needed for the tiles of T1 / T2 that
@@ -530,11 +578,20 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     // at all (a kernel that does gets its 256 registers split 128 / 128).
     auto pin = [&]() {
 #pragma unroll
-      for (int ks = 0; ks < KK; ++ks) {
-        if (DQ || KK == 4) { asm volatile("" : "+v"(xf[ks])); asm volatile("" : "+v"(yf[ks])); }
-        else { asm volatile("" : "+a"(xf[ks])); asm volatile("" : "+a"(yf[ks])); }
-      }
+      for (int ks = 0; ks < KB; ++ks)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          if (DQ || KK == 4) { asm volatile("" : "+v"(xf[r][ks])); asm volatile("" : "+v"(yf[r][ks])); }
+          else { asm volatile("" : "+a"(xf[r][ks])); asm volatile("" : "+a"(yf[r][ks])); }
+        }
     };
+    // what row (lane % 32) of the wavefront has, handed to the lanes that hold the row
+    auto to_lanes = [&](float x, float (&y)[R]) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        y[r] = M == 32 ? x : __int_as_float(__builtin_amdgcn_ds_bpermute((r * M + ln) << 2, __float_as_int(x)));
+    };
+    const int half_row = r0 + wave * 32 + (lane & 31);
     if (!PREPARED) {
       // This pass runs first and prepares what both passes need per query row: delta = rowsum(dout * out), kept
       // negated (the dP products start from it), and lse2 = lse * log2(e) with -inf (a row that saw no key) turned
@@ -550,13 +607,13 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
         o8[u] = bf16x8{};
         if (col < p.D) o8[u] = *reinterpret_cast<const bf16x8*>(osrc + (int64_t)row_of(u) * p.o_ss + col);
       }
-      const int row = my_r < n_st ? my_r : n_st - 1;
+      const int row = half_row < n_st ? half_row : n_st - 1;
       const int64_t r = ((int64_t)b * p.Hq + hs) * p.Sq + row;
       const float l = p.lse[r];
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       // Lane (g, i) of four groups of 16 (64 columns: eight of 8) has columns of row 4 u + g (8 u + g) of out and dout in copy
       // u: the sum over the group is the row's delta, left in all of its lanes; lane i keeps the one of copy i % 8
-      // (i % 4), and lane ln fetches row ln's.
+      // (i % 4), and lane l fetches row l % 32's.
       float mine = 0.f;
 #pragma unroll
       for (int u = 0; u < kCopies; ++u) {
@@ -567,45 +624,53 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
         part = kLanes == 16 ? row16_sum(part) : row8_sum(part);
         mine = lane % kCopies == u ? part : mine;
       }
-      const int holder = ln % kRowsPerCopy * kLanes + ln / kRowsPerCopy;
+      const int holder = (lane & 31) % kRowsPerCopy * kLanes + (lane & 31) / kRowsPerCopy;
       const float delta = __int_as_float(__builtin_amdgcn_ds_bpermute(holder << 2, __float_as_int(mine)));
       read_rows(y_lds, yf);
       read_rows(x_lds, xf);
       pin();
-      lse2_lane = (l == -INFINITY) ? INFINITY : l * kLog2e;
-      delta_lane = -delta;
-      if (hf == 0 && my_r < n_st) {
-        p.delta[r] = delta_lane;
-        p.lse2[r] = lse2_lane;
+      const float lse2 = (l == -INFINITY) ? INFINITY : l * kLog2e;
+      to_lanes(lse2, lse2_lane);
+      to_lanes(-delta, delta_lane);
+      if (lane < 32 && half_row < n_st) {
+        p.delta[r] = -delta;
+        p.lse2[r] = lse2;
         if (p.softmax_d) p.softmax_d[r] = delta;     // for callers that want flash-attn's softmax_d back
       }
-      asm volatile("" : "+v"(lse2_lane), "+v"(delta_lane));
+#pragma unroll
+      for (int i = 0; i < R; ++i) asm volatile("" : "+v"(lse2_lane[i]), "+v"(delta_lane[i]));
       __builtin_amdgcn_s_barrier();                  // the rows' places are stages 1 .. 3 from here on
       if (ntiles > 0) { copy_tile(1); copy_tile(2); }
     } else if (ntiles > 0) {
       constexpr bool kEarly = WAVES == 4;            // stage 1 is not part of the rows' places
-      const int64_t r = DQ ? ((int64_t)b * p.Hq + hs) * p.Sq + (my_r < n_st ? my_r : n_st - 1) : 0;
+      const int64_t r = DQ ? ((int64_t)b * p.Hq + hs) * p.Sq + (half_row < n_st ? half_row : n_st - 1) : 0;
       const uint32_t ld_lds = lds_base + kSmemBytesOf<true, 4, KK> + wave * 256;     // 32 rows' lse2, then their delta
       if (DQ && !kEarly) {
-        lse2_lane = p.lse2[r];
-        delta_lane = p.delta[r];
-        asm volatile("" : "+v"(lse2_lane), "+v"(delta_lane));
+        to_lanes(p.lse2[r], lse2_lane);
+        to_lanes(p.delta[r], delta_lane);
+#pragma unroll
+        for (int i = 0; i < R; ++i) asm volatile("" : "+v"(lse2_lane[i]), "+v"(delta_lane[i]));
       }
       copy_tile(0);
       // (through LDS like the rows: loads into registers would be waited for before the first copy or with the last)
-      if (DQ && kEarly) copy4_to_lds((hf ? p.delta : p.lse2) + r, ld_lds);
+      if (DQ && kEarly) copy4_to_lds((lane >= 32 ? p.delta : p.lse2) + r, ld_lds);
       copy_rows(xsrc, x_lds);
       copy_rows(ysrc, y_lds);
       if (kEarly) copy_tile(1);
       asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kEarly ? kCopiesPerTile : 0) : "memory");
       if (DQ && kEarly) {
-        lse2_lane = *(lds_f32)(uintptr_t)(ld_lds + ln * 4);
-        delta_lane = *(lds_f32)(uintptr_t)(ld_lds + 128 + ln * 4);
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+          lse2_lane[i] = *(lds_f32)(uintptr_t)(ld_lds + (i * M + ln) * 4);
+          delta_lane[i] = *(lds_f32)(uintptr_t)(ld_lds + 128 + (i * M + ln) * 4);
+        }
       }
       read_rows(x_lds, xf);
       read_rows(y_lds, yf);
       pin();
-      if (DQ && kEarly) asm volatile("" : "+v"(lse2_lane), "+v"(delta_lane));
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+        if (DQ && kEarly) asm volatile("" : "+v"(lse2_lane[i]), "+v"(delta_lane[i]));
       __builtin_amdgcn_s_barrier();                  // tile 0 is there for everybody, the rows' places are free
       if (!kEarly) copy_tile(1);
       copy_tile(2);
@@ -614,7 +679,9 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   if (ntiles > 0) {
     if (DQ) {
 #pragma unroll
-      for (int j = 0; j < 16; ++j) nd[j] = delta_lane;
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int j = 0; j < NR; ++j) nd[r][j] = delta_lane[r];
     } else {
 #pragma unroll
       for (int g = 0; g < 4; ++g) read_nd(false, 0, g);
@@ -624,11 +691,12 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     for (int i = 0; i < kDepth; ++i) ring[i] = read_rm(0, i);
 #pragma unroll
     for (int i = 0; i < kT; ++i) {
-      t_mfma(i, ring[i % kDepth], ta1, ta2);
+#pragma unroll
+      for (int r = 0; r < R; ++r) t_mfma(i, r, ring[i % kDepth], ta1, ta2);
       if (i + kDepth < kT) ring[i % kDepth] = read_rm(0, i + kDepth);
     }
 #pragma unroll
-    for (int i = 0; i < kDepth; ++i) ring[i] = read_rm(1, i);            // slots 0 .. 3 of tile 0
+    for (int i = 0; i < kDepth; ++i) ring[i] = read_rm(1, i);            // slots 0 .. 3 of tile 0 (the places behind: zeros)
     if (!DQ) {
       read_ld(false, 0, 0, lv[0]);
 #pragma unroll
@@ -644,58 +712,76 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     // byte distance from this tile's stage to the next tile's, and from that one to the one after
     const int step1 = ((t + 1) & 3) == 0 ? -3 * kStageBytes : kStageBytes;
     const int step2 = ((t + 2) & 3) == 0 ? -3 * kStageBytes : kStageBytes;
-    static_assert(kSlots % kDepth == 0, "the ring position is the slot number modulo its depth");
+    static_assert(kSlots % kRing == 0 && kT >= kLag, "the ring position is the slot number modulo its depth");
     mask_half(ta1, c0);
 #pragma unroll
     for (int i = 0; i < kT; ++i) {                       // P0, carrying the copies of tile t+3
-      t_mfma(i, ring[i % kDepth], tb1, tb2);
 #pragma unroll
-      for (int v = vec0(i); v < vec0(i + 1); ++v) vector_slot(v, ta1, ta2, 0);
+      for (int r = 0; r < R; ++r) {
+        if (r > 0) __builtin_amdgcn_sched_barrier(0);
+        t_mfma(i, r, ring[i % kRing], tb1, tb2);
+        vector_t(i, r, ta1, ta2, 0);
+      }
+      acc_rest(i, kP3);                                  // of the tile before (the first tile: zeros)
 #pragma unroll
       for (int piece = i; piece < kCopiesPerTile; piece += kT) copy_piece(piece, (t + 3) & 3);
-      ring[i % kDepth] = read_slot(i + kDepth);
+      refill(i);
       if (i >= kT - kDepth) {                            // the last read of this tile's T1 / T2 operands is out: on to the next
 #pragma unroll
-        for (int a = (i - (kT - kDepth)) * KK / kDepth; a < (i + 1 - (kT - kDepth)) * KK / kDepth; ++a) rm_a[a] += step1;
+        for (int a = (i - (kT - kDepth)) * KB / kDepth; a < (i + 1 - (kT - kDepth)) * KB / kDepth; ++a) rm_a[a] += step1;
       }
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int i = 0; i < kAcc; ++i) {                     // P1
-      vector_tail(i, ta1, ta2, 0);
-      acc_mfma(i, ring[(kP1 + i) % kDepth]);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        if (r > 0) __builtin_amdgcn_sched_barrier(0);
+        vector_tail(i, r, ta1, ta2, 0);
+        acc_mfma(i, r, kP1);
+      }
       if (!DQ && i == kAcc - 2) read_ld(false, 1, 0, lv[0]);
       // -delta for T2 of (t+1, first half), which starts in P2: read once the vector work on this half's dP is
       // through (half of the slots), so that the values can land in the registers T2 accumulates in
       if (!DQ && i >= kAcc / 2 && i < kAcc / 2 + 4) read_nd(true, 0, i - kAcc / 2);
-      ring[(kP1 + i) % kDepth] = read_slot(kP1 + i + kDepth);
+      refill(kP1 + i);
       __builtin_amdgcn_sched_barrier(0);
     }
     mask_half(tb1, c0 + 32);
 #pragma unroll
     for (int i = 0; i < kT; ++i) {                       // P2
-      t_mfma(i, ring[(kP2 + i) % kDepth], ta1, ta2);
 #pragma unroll
-      for (int v = vec0(i); v < vec0(i + 1); ++v) vector_slot(v, tb1, tb2, 1);
-      ring[(kP2 + i) % kDepth] = read_slot(kP2 + i + kDepth);
+      for (int r = 0; r < R; ++r) {
+        if (r > 0) __builtin_amdgcn_sched_barrier(0);
+        t_mfma(i, r, ring[(kP2 + i) % kRing], ta1, ta2);
+        vector_t(i, r, tb1, tb2, 1);
+      }
+      acc_rest(i, kP1);
+      refill(kP2 + i);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int i = 0; i < kAcc; ++i) {                     // P3
-      vector_tail(i, tb1, tb2, 1);
-      acc_mfma(i, ring[(kP3 + i) % kDepth]);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        if (r > 0) __builtin_amdgcn_sched_barrier(0);
+        vector_tail(i, r, tb1, tb2, 1);
+        acc_mfma(i, r, kP3);
+      }
       if (!DQ && i == kAcc - 2) read_ld(true, 0, 0, lv[0]);
       if (!DQ && i >= kAcc / 2 && i < kAcc / 2 + 4) read_nd(true, 1, i - kAcc / 2);   // T2 of (t+1, second half): P0 of the next tile
-      ring[(kP3 + i) % kDepth] = read_slot(kP3 + i + kDepth);
+      refill(kP3 + i);
       if (i >= kAcc - kDepth) {                          // the last transposed read of this tile has been issued
 #pragma unroll
-        for (int a = (i - (kAcc - kDepth)) * 2 * DB / kDepth; a < (i + 1 - (kAcc - kDepth)) * 2 * DB / kDepth; ++a) tr_a[a >> 1][a & 1] += step1;
+        for (int a = (i - (kAcc - kDepth)) * KK / kDepth; a < (i + 1 - (kAcc - kDepth)) * KK / kDepth; ++a) tr_a[a] += step1;
       }
       __builtin_amdgcn_sched_barrier(0);
     }
     ld_cur = ld_next;
     ld_next += step2;
   }
+#pragma unroll
+  for (int i = 0; i < kLag; ++i) acc_rest(i, kP3);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the zero-filled copies of tiles past the end
 
   // ---- epilogue: acc^T[d][r] -> rows of the output through LDS --------------------------------------------
@@ -706,19 +792,25 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   };
-  auto write_out = [&](const f32x16 (&acc)[DB], float mul, uint16_t* dst, int64_t d_sb, int64_t d_ss,
+  // columns 4 c .. 4 c + 3 of a stationary row: lane (ln, lg) has every c = 64/M u + lg of rows M r + ln
+  auto unit = [](const Acc (&acc)[DB][R], int u, int r, float mul) {
+    f32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = acc[4 * u / NR][r][(4 * u + e) % NR] * mul;
+    return v;
+  };
+  constexpr int kUnits = DB * NR / 4;
+  auto write_out = [&](const Acc (&acc)[DB][R], float mul, uint16_t* dst, int64_t d_sb, int64_t d_ss,
                        int64_t d_sh, int head) {
     own_lds_order();
     constexpr int kOStride = kRow / 2 + 8;
     unsigned char* os = smem + wave * (32 * kOStride * 2);
 #pragma unroll
-    for (int db = 0; db < DB; ++db)
+    for (int u = 0; u < kUnits; ++u)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        u32x2 w;
-        w[0] = pack_bf16(acc[db][4 * g] * mul, acc[db][4 * g + 1] * mul);
-        w[1] = pack_bf16(acc[db][4 * g + 2] * mul, acc[db][4 * g + 3] * mul);
-        *reinterpret_cast<u32x2*>(os + ln * (kOStride * 2) + (db * 32 + g * 8 + hf * 4) * 2) = w;
+      for (int r = 0; r < R; ++r) {
+        const f32x4 v = unit(acc, u, r, mul);
+        *reinterpret_cast<u32x2*>(os + (r * M + ln) * (kOStride * 2) + (64 / M * u + lg) * 8) = u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
       }
     own_lds_order();
     const int chunk = lane & 15;
@@ -739,7 +831,7 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   // the way before the first store (a load cannot pass a store that may be to the same place, so that one row's after
   // the other cost a round trip each), and `finish` gets the lane's 4 columns of a row: a step of 8 chunks 4096 x 4096 H32,
   // dQ carried in fp32, 6838 us to 6790, causal 1500 x 1500 B2 H12 D 64 61.3 to 61.0.
-  auto write_out32 = [&](const f32x16 (&acc)[DB], float mul, auto&& fetch, auto&& finish) {
+  auto write_out32 = [&](const Acc (&acc)[DB][R], float mul, auto&& fetch, auto&& finish) {
     own_lds_order();
     constexpr int kRow32 = 2 * kRow, kPlaces = kRow32 / 16, kRowsAtOnce = 64 / kPlaces, kIts = 32 / kRowsAtOnce;
     unsigned char* os = smem + wave * (32 * kRow32);
@@ -751,13 +843,11 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
       if (first_row + it * kRowsAtOnce < n_st && col < p.D) old[it] = fetch(first_row + it * kRowsAtOnce, col);
     }
 #pragma unroll
-    for (int db = 0; db < DB; ++db)
+    for (int u = 0; u < kUnits; ++u)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        f32x4 v;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc[db][4 * g + e] * mul;
-        *reinterpret_cast<f32x4*>(os + ln * kRow32 + (((db * 8 + g * 2 + hf) ^ (ln % kPlaces)) << 4)) = v;
+      for (int r = 0; r < R; ++r) {
+        const int row = r * M + ln;
+        *reinterpret_cast<f32x4*>(os + row * kRow32 + (((64 / M * u + lg) ^ (row % kPlaces)) << 4)) = unit(acc, u, r, mul);
       }
     own_lds_order();
 #pragma unroll
@@ -811,11 +901,11 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   }
 }
 
-template <bool DQ, bool CAUSAL, int KK, bool PREPARED>
+template <bool DQ, bool CAUSAL, int KK, bool PREPARED, int M>
 __global__ __launch_bounds__(DQ ? 512 : 256, !DQ && KK == 4 ? 2 : 1) void bwd_main(const BwdParams p, const TileMap w) {
   constexpr int kWaves = DQ ? 8 : 4;
   __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<DQ, kWaves, KK>];
-  bwd_pass<DQ, CAUSAL, KK, kWaves, PREPARED, false>(p, w, (int)blockIdx.x, smem);
+  bwd_pass<DQ, CAUSAL, KK, kWaves, PREPARED, false, false, M>(p, w, (int)blockIdx.x, smem);
 }
 
 // Both passes side by side, for launches that leave CUs idle one after the other.
@@ -1069,6 +1159,26 @@ int chunk_splits(int B, int Sq, int Sc, int Hq, int Hkv, int D, int n) {
   return best;
 }
 
+// Whether the dQ pass of eight wavefronts, with workgroups of `tiles` key tiles each (causal: at most), uses 16 x 16 MFMA tiles: where
+// it keeps every CU busy for long enough, its time is the board's power.  The pass alone, us, 32 x 32 / 16 x 16 (workgroups x tiles):
+//     D 128  512 x 64  327 / 311    256 x 32  87.7 / 83.8    192 x 64  131 / 133      causal  512 x 64  183 / 174   1024 x 32  209 / 207
+//     D 96   512 x 64  255 / 247    256 x 32  65.4 / 63.7                             causal  512 x 64  144 / 141
+bool small_tiles(const TileMap& w, bool causal, int64_t tiles) {
+  const int64_t rounds = ((int64_t)w.total + 255) / 256;
+  return tiles >= 32 && (causal ? w.total >= 512 : (int64_t)w.total * 20 >= rounds * 256 * 17);
+}
+
+template <bool DQ, bool CAUSAL, int KK, bool PREPARED>
+void launch_pass(const BwdParams& p, const TileMap& w, int64_t tiles, hipStream_t st) {
+  const dim3 grid(w.per_xcd * 8), block(DQ ? 512 : 256);
+  if constexpr (DQ && KK > 4)
+    if (small_tiles(w, CAUSAL, tiles)) {
+      hipLaunchKernelGGL((bwd_main<DQ, CAUSAL, KK, PREPARED, 16>), grid, block, 0, st, p, w);
+      return;
+    }
+  hipLaunchKernelGGL((bwd_main<DQ, CAUSAL, KK, PREPARED, 32>), grid, block, 0, st, p, w);
+}
+
 template <bool CAUSAL, int KK>
 void launch_bwd(const BwdParams& p, const Plan& plan, float* partial, hipStream_t st) {
   if (plan.joint) {
@@ -1085,15 +1195,14 @@ void launch_bwd(const BwdParams& p, const Plan& plan, float* partial, hipStream_
       hipLaunchKernelGGL(bwd_reduce, dim3((q_rows + 2 * kv_rows + 15) / 16), dim3(256), 0, st, p, wq, wk, q_rows, kv_rows);
     return;
   }
-  const TileMap wk = tile_map(p.B * p.Hkv, p.Sc, kRowsKv);
   if (p.Sq > 0) {
     // dQ (and delta / lse2 for both passes): one workgroup per 256 query rows; has to run before the dK / dV pass
     const TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ);
-    if (p.prepared) hipLaunchKernelGGL((bwd_main<true, CAUSAL, KK, true>), dim3(wq.per_xcd * 8), dim3(512), 0, st, p, wq);
-    else hipLaunchKernelGGL((bwd_main<true, CAUSAL, KK, false>), dim3(wq.per_xcd * 8), dim3(512), 0, st, p, wq);
+    if (p.prepared) launch_pass<true, CAUSAL, KK, true>(p, wq, (p.Sc + kTile - 1) / kTile, st);
+    else launch_pass<true, CAUSAL, KK, false>(p, wq, (p.Sc + kTile - 1) / kTile, st);
   }
   // dK, dV: one workgroup per 128 keys of one kv head
-  if (p.Sc > 0) hipLaunchKernelGGL((bwd_main<false, CAUSAL, KK, true>), dim3(wk.per_xcd * 8), dim3(256), 0, st, p, wk);
+  if (p.Sc > 0) launch_pass<false, CAUSAL, KK, true>(p, tile_map(p.B * p.Hkv, p.Sc, kRowsKv), (int64_t)p.group * ((p.Sq + kTile - 1) / kTile), st);
 }
 
 template <int KK>

@@ -149,6 +149,15 @@ __device__ __forceinline__ void copy4_to_lds(const void* src, uint32_t lds_addr)
 // and 8 rows x 4 consecutive chunks (ds_read_b64_tr_b16 of a transposed operand).
 __device__ __forceinline__ constexpr int lds_row_swizzle(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
 
+// The same for 16 x 16 MFMA tiles, which read 16 rows x 4 chunks of a row-major operand and 16 rows x 2 consecutive chunks of a
+// transposed one.  ds_read_b128 serves lanes 0-3, 12-15 and 20-27 of a half-wave together, which are rows 0-3 and 12-15 of one chunk
+// and rows 4-11 of the next; ds_read_b64_tr_b16 half a wave, 8 consecutive rows.  With the map above both meet in the same banks.
+// (The dQ pass of 4096 x 4096 H32 loses 51 M LDS cycles of 103 M to conflicts with that one, 0.4 M with this.  The forward kernel is
+// no faster for it, 1572 us / 1570 a step of 8 such blocks, and keeps the map above.)
+__device__ __forceinline__ constexpr int lds_row_swizzle_16(int row) {
+  return ((row & 3) << 2) | (((row >> 1) ^ (row >> 2)) & 2) | ((row >> 3) & 1);
+}
+
 // Division of a number below 2^31 by a divisor the host knows: a multiplication and a shift on the scalar unit instead of
 // some twenty dependent instructions through the vector unit's reciprocal.  With s = ceil(log2 d) and
 // mul = floor(2^32 (2^s - d) / d) + 1 the quotient is (mulhi(n, mul) + n) >> s (Granlund and Montgomery, 1994).
