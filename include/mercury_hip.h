@@ -51,8 +51,9 @@ extern "C" {
  * 5: the workspace's size depends on B, Sq and Hq alone; mhip_attn_fwd_plan, mhip_attn_bwd_plan.
  * 6: mhip_attn_fwd_blocks, mhip_attn_fwd_group.
  * 7: mhip_attn_bwd_chunks, mhip_attn_bwd_group.
- * 8: mhip_attn_fwd_blocks takes the number of chunks of a result; mhip_attn_fwd_chain. */
-#define MHIP_ABI_VERSION 8
+ * 8: mhip_attn_fwd_blocks takes the number of chunks of a result; mhip_attn_fwd_chain.
+ * 9: mhip_attn_bwd_take. */
+#define MHIP_ABI_VERSION 9
 int         mhip_abi_version(void);   /* the MHIP_ABI_VERSION the library was built with */
 int         mhip_version(void);
 /* Optional: per-device set-up the entry points otherwise do on their first call on a device (today: the address
@@ -192,8 +193,9 @@ int mhip_attn_bwd_chunk(const void* dout, const void* q, const void* k, const vo
  * n chunks of a ring step in one launch, 1 <= n <= MHIP_MAX_GROUP: what n calls of mhip_attn_bwd_chunk without a mask do, with
  * T the sum over all of them.  ks, vs, dks, dvs, dk32s and dv32s are host arrays of n device pointers (entries of the
  * last four may be NULL, as there); all chunks have one Sc and one set of strides.
- * mhip_attn_bwd_group: how many chunks of a step of `chunks` chunks to put into one launch when all of them are there (host
- * function, launches nothing).
+ * mhip_attn_bwd_group: how many chunks of a step of `chunks` chunks to put into one launch of both passes when all of them are
+ * there; mhip_attn_bwd_take: how many to hand to one call, also where each pass has a launch of its own over them (host
+ * functions, nothing is launched).
  */
 int mhip_attn_bwd_chunks(const void* dout, const void* q, const void* const* ks, const void* const* vs, int n,
                          const void* out, const float* lse,
@@ -207,6 +209,7 @@ int mhip_attn_bwd_chunks(const void* dout, const void* q, const void* const* ks,
                          int64_t o_sb, int64_t o_ss, int64_t o_sh,     /* out      */
                          float softmax_scale, void* workspace, void* stream);
 int mhip_attn_bwd_group(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks);
+int mhip_attn_bwd_take(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks);
 
 /*
  * Which form of the kernels a call of the given sizes takes (host functions, nothing is launched; for tests and profiles,

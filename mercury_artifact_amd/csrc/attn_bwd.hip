@@ -908,6 +908,14 @@ __global__ __launch_bounds__(DQ ? 512 : 256, !DQ && KK == 4 ? 2 : 1) void bwd_ma
   bwd_pass<DQ, CAUSAL, KK, kWaves, PREPARED, false, false, M>(p, w, (int)blockIdx.x, smem);
 }
 
+// A pass over several chunks of a step: the same chains of tiles as in bwd_joint_chunks, where each pass alone fills the chip.
+template <bool DQ, int KK, bool PREPARED, int M>
+__global__ __launch_bounds__(DQ ? 512 : 256, !DQ && KK == 4 ? 2 : 1) void bwd_main_chunks(const BwdParams p, const TileMap w, const Chunks chunks) {
+  constexpr int kWaves = DQ ? 8 : 4;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<DQ, kWaves, KK>];
+  bwd_pass<DQ, false, KK, kWaves, PREPARED, false, true, M>(p, w, (int)blockIdx.x, smem, &chunks);
+}
+
 // Both passes side by side, for launches that leave CUs idle one after the other.
 template <bool CAUSAL, int KK, bool SPLIT>
 __global__ __launch_bounds__(256, KK == 4 ? 2 : 1) void bwd_joint(const BwdParams p, const TileMap wq, const TileMap wk) {
@@ -1069,6 +1077,8 @@ float launch_time(float n, float mean, float most, const Cost& c) {
 //     causal: B2 H12 1500 x 1500  60.7 / 40.8*                                      B1 H32 4096 x 4096  249* / 247
 // and one / shared by as many workgroups (sq, sk) as chosen: H8/1 2048 x 2048 226 / 46.0 (1, 8), H32/4 247 / 125 (1, 4), H2/2
 // 4096 x 4096 63.1 / 48.0 (2, 2), where 44.2 (4, 4) would be better.
+Cost dq_cost(int D) { return D <= 64 ? Cost{6.f, 0.95f, 0.45f} : Cost{7.f, 1.45f, 0.75f}; }       // 96 columns: the costs of
+Cost dkv_cost(int D) { return D <= 64 ? Cost{6.f, 0.75f, 0.25f} : Cost{7.f, 1.15f, 0.55f}; }      // 128, of which all save the same 12 %
 Cost joint_cost(int D) { return D <= 64 ? Cost{6.f, 0.75f, 0.12f} : Cost{7.f, 1.15f, 0.29f}; }
 struct Plan { bool joint; int sq, sk; float time; };       // time: estimated, without preparing delta and lse2
 constexpr int64_t kPartialMost = int64_t(32) << 20;     // bytes of sums a block may leave for bwd_reduce
@@ -1078,10 +1088,7 @@ int64_t partial_bytes(int B, int S, int H, int D, int tensors, int splits) {
 Plan plan_block(int B, int Sq, int Sc, int Hq, int Hkv, int D, bool causal) {
   Plan best = {false, 1, 1, 0.f};
   if (Sq == 0 || Sc == 0 || B == 0) return best;
-  const bool narrow = D <= 64;      // 96 columns: the costs of 128, of which both forms save the same 12 %
-  const Cost dq8 = narrow ? Cost{6.f, 0.95f, 0.45f} : Cost{7.f, 1.45f, 0.75f};
-  const Cost dkv = narrow ? Cost{6.f, 0.75f, 0.25f} : Cost{7.f, 1.15f, 0.55f};
-  const Cost both = joint_cost(D);
+  const Cost dq8 = dq_cost(D), dkv = dkv_cost(D), both = joint_cost(D);
   constexpr float kPrepare = 5.f, kReduce = 4.f, kBytesPerUs = 4e6f;
   const float tq = (float)((Sc + kTile - 1) / kTile), tk = (float)((Sq + kTile - 1) / kTile) * (Hq / Hkv);
   const float half = causal ? 0.53f : 1.f;          // mean share of the tiles under the diagonal
@@ -1113,21 +1120,43 @@ Plan plan_block(int B, int Sq, int Sc, int Hq, int Hkv, int D, bool causal) {
 //     8 chunks 512 x 512 B4 H5      114 / 84.6 / 71.7 / 62.3*     1024 x 1024 H32                299 /  297 / 249* / 240
 //     256 x 256 H16                91.7 / 61.8 / 52.9 / 48.6*     512 x 512 H8/1                 154 /  248 /  128 / 65.4*
 //     1500 x 1500 B2 H12            558 /  446 / 405* / 392       700 x 700 H12                  136 / 98.6 / 88.0 / 77.9*
-int group_chunks(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks) {
-  if (B == 0 || Sq == 0 || Sc == 0) return 1;
+float joint_chunks_time(int B, int Sq, int Sc, int Hq, int Hkv, int D, int n) {
   const int64_t nq = tile_map(B * Hq, Sq, kRowsQ / 2).total, nk = tile_map(B * Hkv, Sc, kRowsKv).total;
+  const int64_t workgroups = nq + n * nk;
+  if (n > kMaxGroup || workgroups > kGroupWorkgroups) return INFINITY;
   const float tq = (float)((Sc + kTile - 1) / kTile), tk = (float)((Sq + kTile - 1) / kTile) * (Hq / Hkv);
   const Cost c = joint_cost(D);
+  const float share = workgroups < 256 ? (float)workgroups / 256.f : 1.f, step = c.step + share * c.busy;
+  const float longest = c.fixed + (n * tq > tk ? n * tq : tk) * step;
+  const float spread = (nq * (c.fixed + n * tq * step) + n * nk * (c.fixed + tk * step)) / 256.f;
+  return longest > spread ? longest : spread;
+}
+// Where both passes fill the chip one after the other, each has a launch over the chunks (apart): the dQ pass keeps its eight
+// wavefronts, and its workgroups' ends and the carried sum come once here too.  Us a step, without / with:
+//     8 chunks 4096 x 4096 H32     6453 / 6175      2048 x 2048 H32     1820 / 1641      1024 x 1024 B2 H32    1118 /  931
+//     512 x 512 B4 H32              757 /  585      6000 x 600 H32      2016 / 1439      2048 x 2048 H32 D64   1004 /  891
+//     4 chunks 1024 x 1024 H64      560 /  474      4096 x 4096 H32/8   3121 / 2986      8192 x 8192 H8        3089 / 3013
+// and where the estimate expects more of other forms, what they take / both passes apart:
+//     8 chunks 1024 x 1024 H32      459 /  491      2048 x 2048 H16      821 /  874      4 chunks 3000 x 3000 H24 D96  1091 / 1202
+//     8 chunks 1536 x 1536 H32      953 /  934      2 chunks 7430 x 7430 H8/1  1689 / 1586
+float apart_chunks_time(int B, int Sq, int Sc, int Hq, int Hkv, int D, int n) {
+  if (n > kMaxGroup) return INFINITY;
+  const float tq = (float)((Sc + kTile - 1) / kTile), tk = (float)((Sq + kTile - 1) / kTile) * (Hq / Hkv);
+  const float nq = (float)tile_map(B * Hq, Sq, kRowsQ).total, nk = (float)tile_map(B * Hkv, Sc, kRowsKv).total;
+  return launch_time(nq, n * tq, n * tq, dq_cost(D)) + launch_time(n * nk, tk, tk, dkv_cost(D));
+}
+bool chunks_apart(int B, int Sq, int Sc, int Hq, int Hkv, int D, int n) {
+  return apart_chunks_time(B, Sq, Sc, Hq, Hkv, D, n) < joint_chunks_time(B, Sq, Sc, Hq, Hkv, D, n);
+}
+int group_chunks(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks, bool or_apart) {
+  if (B == 0 || Sq == 0 || Sc == 0) return 1;
   int best = 1;
   float best_time = plan_block(B, Sq, Sc, Hq, Hkv, D, false).time * chunks;
   for (int launches = chunks; launches >= 1; --launches) {
     const int n = (chunks + launches - 1) / launches;
-    const int64_t workgroups = nq + n * nk;
-    if (n > kMaxGroup || workgroups > kGroupWorkgroups) break;
-    const float share = workgroups < 256 ? (float)workgroups / 256.f : 1.f, step = c.step + share * c.busy;
-    const float longest = c.fixed + (n * tq > tk ? n * tq : tk) * step;
-    const float spread = (nq * (c.fixed + n * tq * step) + n * nk * (c.fixed + tk * step)) / 256.f;
-    const float time = ((chunks + n - 1) / n) * (longest > spread ? longest : spread);
+    if (n > kMaxGroup) break;
+    const float joint = joint_chunks_time(B, Sq, Sc, Hq, Hkv, D, n), apart = or_apart ? apart_chunks_time(B, Sq, Sc, Hq, Hkv, D, n) : INFINITY;
+    const float time = ((chunks + n - 1) / n) * (apart < joint ? apart : joint);
     if (n > 1 && time < best_time) { best_time = time; best = n; }
   }
   return best;
@@ -1205,8 +1234,27 @@ void launch_bwd(const BwdParams& p, const Plan& plan, float* partial, hipStream_
   if (p.Sc > 0) launch_pass<false, CAUSAL, KK, true>(p, tile_map(p.B * p.Hkv, p.Sc, kRowsKv), (int64_t)p.group * ((p.Sq + kTile - 1) / kTile), st);
 }
 
+template <bool DQ, int KK, bool PREPARED>
+void launch_pass_chunks(const BwdParams& p, const TileMap& w, int64_t tiles, const Chunks& chunks, hipStream_t st) {
+  const dim3 grid(w.per_xcd * 8), block(DQ ? 512 : 256);
+  if constexpr (DQ && KK > 4)
+    if (small_tiles(w, false, tiles)) {
+      hipLaunchKernelGGL((bwd_main_chunks<DQ, KK, PREPARED, 16>), grid, block, 0, st, p, w, chunks);
+      return;
+    }
+  hipLaunchKernelGGL((bwd_main_chunks<DQ, KK, PREPARED, 32>), grid, block, 0, st, p, w, chunks);
+}
+
 template <int KK>
 void launch_chunks(const BwdParams& p, const Chunks& chunks, float* partial, hipStream_t st) {
+  if (chunks_apart(p.B, p.Sq, p.Sc, p.Hq, p.Hkv, p.D, chunks.n)) {
+    const TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ);
+    const int64_t tiles = (int64_t)chunks.n * ((p.Sc + kTile - 1) / kTile);
+    if (p.prepared) launch_pass_chunks<true, KK, true>(p, wq, tiles, chunks, st);
+    else launch_pass_chunks<true, KK, false>(p, wq, tiles, chunks, st);
+    launch_pass_chunks<false, KK, true>(p, tile_map(chunks.n * p.B * p.Hkv, p.Sc, kRowsKv), 0, chunks, st);
+    return;
+  }
   const int rows = p.B * p.Hq * p.Sq;
   if (!p.prepared) hipLaunchKernelGGL(bwd_prepare, dim3((rows + 15) / 16), dim3(256), 0, st, p, rows);
   const int splits = chunk_splits(p.B, p.Sq, p.Sc, p.Hq, p.Hkv, p.D, chunks.n);
@@ -1387,7 +1435,12 @@ extern "C" int mhip_attn_bwd_chunk(const void* dout, const void* q, const void* 
 
 extern "C" int mhip_attn_bwd_group(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks) {
   if (B < 0 || Sq < 0 || Sc < 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || D <= 0 || D > kD || chunks < 1) return MHIP_EINVAL;
-  return group_chunks(B, Sq, Sc, Hq, Hkv, D, chunks);
+  return group_chunks(B, Sq, Sc, Hq, Hkv, D, chunks, false);
+}
+
+extern "C" int mhip_attn_bwd_take(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks) {
+  if (B < 0 || Sq < 0 || Sc < 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || D <= 0 || D > kD || chunks < 1) return MHIP_EINVAL;
+  return group_chunks(B, Sq, Sc, Hq, Hkv, D, chunks, true);
 }
 
 extern "C" int mhip_attn_bwd_chunks(const void* dout, const void* q, const void* const* ks, const void* const* vs, int n,

@@ -33,7 +33,7 @@ struct Entry {
   decltype(&mhip_attn_bwd_block) bwd = nullptr;
   decltype(&mhip_attn_bwd_chunk) chunk = nullptr;
   decltype(&mhip_attn_bwd_chunks) bwd_many = nullptr;
-  decltype(&mhip_attn_bwd_group) bwd_group = nullptr;
+  decltype(&mhip_attn_bwd_take) bwd_take = nullptr;
   decltype(&mhip_lse_merge) merge = nullptr;
   decltype(&mhip_lse_merge_many) many = nullptr;
   decltype(&mhip_pack_reduce) pack = nullptr;
@@ -468,7 +468,7 @@ PyObject* bwd_group(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   if (!q || !c || q->dim() != 4 || c->dim() != 5 || c->size(3) == 0 || q->size(2) % c->size(3) ||
       !fits({q->size(0), q->size(1), q->size(2), q->size(3), c->size(2), n}))
     SLOW;
-  const int most = entry.bwd_group(q->size(0), q->size(1), c->size(2), q->size(2), c->size(3), q->size(3), n);
+  const int most = entry.bwd_take(q->size(0), q->size(1), c->size(2), q->size(2), c->size(3), q->size(3), n);
   if (most < 1) SLOW;
   return PyLong_FromLong(most);
   END_HANDLE_TH_ERRORS
@@ -731,7 +731,7 @@ PyObject* bind(PyObject*, PyObject* table) {
                   take(entry.fwd_group, "mhip_attn_fwd_group") && take(entry.fwd_chain, "mhip_attn_fwd_chain") &&
                   take(entry.bwd_bytes, "mhip_attn_bwd_workspace_bytes") &&
                   take(entry.bwd, "mhip_attn_bwd_block") && take(entry.chunk, "mhip_attn_bwd_chunk") &&
-                  take(entry.bwd_many, "mhip_attn_bwd_chunks") && take(entry.bwd_group, "mhip_attn_bwd_group") &&
+                  take(entry.bwd_many, "mhip_attn_bwd_chunks") && take(entry.bwd_take, "mhip_attn_bwd_take") &&
                   take(entry.merge, "mhip_lse_merge") && take(entry.many, "mhip_lse_merge_many") &&
                   take(entry.pack, "mhip_pack_reduce") && take(entry.unpack, "mhip_unpack") &&
                   take(entry.quantize, "mhip_quantize_e4m3") && take(entry.error_string, "mhip_error_string");
