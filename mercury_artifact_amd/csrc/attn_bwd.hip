@@ -71,6 +71,7 @@ struct TileMap {
   int n_tiles;         // stationary tiles per (batch, head), times splits
   int total;
   int per_xcd;         // ceil(total / 8); the pass takes 8 * per_xcd workgroups
+  int first;           // the first of them in the launch: a multiple of 8, so that both halves of a joint one keep their XCDs
   int heads_per_xcd;   // (batch, stationary head) pairs per XCD when they divide evenly, else 0
   Divisor by_tiles;
   Divisor by_order;    // causal: by all (batch, stationary head) pairs, or by those of an XCD
@@ -921,18 +922,18 @@ template <bool CAUSAL, int KK, bool SPLIT>
 __global__ __launch_bounds__(256, KK == 4 ? 2 : 1) void bwd_joint(const BwdParams p, const TileMap wq, const TileMap wk) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<false, 4, KK>];
   static_assert(kSmemBytesOf<true, 4, KK> + 1024 <= kSmemBytesOf<false, 4, KK>, "one array for both, and lse2 and delta of the dQ rows");
-  const int first_q = wk.per_xcd * 8;         // a multiple of 8: both halves keep their XCDs
-  if ((int)blockIdx.x < first_q) bwd_pass<false, CAUSAL, KK, 4, true, SPLIT>(p, wk, (int)blockIdx.x, smem);
-  else bwd_pass<true, CAUSAL, KK, 4, true, SPLIT>(p, wq, (int)blockIdx.x - first_q, smem);
+  const int i = (int)blockIdx.x - wk.first;
+  if (i >= 0 && i < wk.per_xcd * 8) bwd_pass<false, CAUSAL, KK, 4, true, SPLIT>(p, wk, i, smem);
+  else bwd_pass<true, CAUSAL, KK, 4, true, SPLIT>(p, wq, (int)blockIdx.x - wq.first, smem);
 }
 
-// The same for several chunks of a step.  The dQ workgroups, whose chains are the longest, come first.
+// The same for several chunks of a step.
 template <int KK, bool SPLIT>
 __global__ __launch_bounds__(256, KK == 4 ? 2 : 1) void bwd_joint_chunks(const BwdParams p, const TileMap wq, const TileMap wk, const Chunks chunks) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytesOf<false, 4, KK>];
-  const int first_k = wq.per_xcd * 8;
-  if ((int)blockIdx.x < first_k) bwd_pass<true, false, KK, 4, true, SPLIT, true>(p, wq, (int)blockIdx.x, smem, &chunks);
-  else bwd_pass<false, false, KK, 4, true, false, true>(p, wk, (int)blockIdx.x - first_k, smem, &chunks);
+  const int i = (int)blockIdx.x - wq.first;
+  if (i >= 0 && i < wq.per_xcd * 8) bwd_pass<true, false, KK, 4, true, SPLIT, true>(p, wq, i, smem, &chunks);
+  else bwd_pass<false, false, KK, 4, true, false, true>(p, wk, (int)blockIdx.x - wk.first, smem, &chunks);
 }
 
 // lse2 and delta for bwd_joint: 16 lanes per query row.
@@ -1040,10 +1041,21 @@ TileMap tile_map(int heads, int seq, int rows, int splits = 1, float* partial = 
   w.n_tiles = (seq + rows - 1) / rows * splits;
   w.total = heads * w.n_tiles;
   w.per_xcd = (w.total + 7) / 8;
+  w.first = 0;
   w.heads_per_xcd = heads % 8 == 0 ? heads / 8 : 0;
   w.by_tiles = Divisor(w.n_tiles);
   w.by_order = Divisor(w.heads_per_xcd > 0 ? w.heads_per_xcd : heads);
   return w;
+}
+
+// The order of the passes in a joint launch: the one with the longer chains of tiles first (tq and tk tiles at most, of three and
+// four products each), so that the short ones fill the tail.  Us, where it is the other one than dK / dV for a block, dQ for
+// several, whose workgroups came first whatever their chains (before / this):
+//     1237 x 8192 B2 H16  590 / 510     700 x 6000 H24 D64  114 / 98.0    1024 x 16384 H16  430 / 421     512 x 8192 H8  77.0 / 75.5
+//     2 chunks  7430 x 7430 H8/1  1710 / 1417     12000 x 12000 H4/1  1970 / 1690     2048 x 2048 H32/4 D64  325 / 280
+void longest_first(TileMap& wq, TileMap& wk, float tq, float tk) {
+  if (4.f * tk >= 3.f * tq) wq.first = wk.per_xcd * 8;
+  else wk.first = wq.per_xcd * 8;
 }
 
 // Estimated time (us) of n workgroups that visit `most` tiles at most and `mean` on average, one workgroup per CU at a
@@ -1213,8 +1225,9 @@ void launch_bwd(const BwdParams& p, const Plan& plan, float* partial, hipStream_
   if (plan.joint) {
     const int rows = p.B * p.Hq * p.Sq;
     if (!p.prepared) hipLaunchKernelGGL(bwd_prepare, dim3((rows + 15) / 16), dim3(256), 0, st, p, rows);
-    const TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ / 2, plan.sq, partial);
-    const TileMap wk = tile_map(p.B * p.Hkv, p.Sc, kRowsKv, plan.sk, partial + partial_bytes(p.B, p.Sq, p.Hq, p.D, 1, plan.sq) / 4);
+    TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ / 2, plan.sq, partial);
+    TileMap wk = tile_map(p.B * p.Hkv, p.Sc, kRowsKv, plan.sk, partial + partial_bytes(p.B, p.Sq, p.Hq, p.D, 1, plan.sq) / 4);
+    longest_first(wq, wk, (float)((p.Sc + kTile - 1) / kTile) / plan.sq, (float)((p.Sq + kTile - 1) / kTile) * p.group / plan.sk);
     const dim3 grid((wk.per_xcd + wq.per_xcd) * 8), block(256);
     // (a kernel of its own: the bookkeeping of shared tiles costs 0.6 us where there are none)
     if (plan.sq > 1 || plan.sk > 1) hipLaunchKernelGGL((bwd_joint<CAUSAL, KK, true>), grid, block, 0, st, p, wq, wk);
@@ -1258,8 +1271,9 @@ void launch_chunks(const BwdParams& p, const Chunks& chunks, float* partial, hip
   const int rows = p.B * p.Hq * p.Sq;
   if (!p.prepared) hipLaunchKernelGGL(bwd_prepare, dim3((rows + 15) / 16), dim3(256), 0, st, p, rows);
   const int splits = chunk_splits(p.B, p.Sq, p.Sc, p.Hq, p.Hkv, p.D, chunks.n);
-  const TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ / 2, splits, partial);
-  const TileMap wk = tile_map(chunks.n * p.B * p.Hkv, p.Sc, kRowsKv);
+  TileMap wq = tile_map(p.B * p.Hq, p.Sq, kRowsQ / 2, splits, partial);
+  TileMap wk = tile_map(chunks.n * p.B * p.Hkv, p.Sc, kRowsKv);
+  longest_first(wq, wk, (float)((chunks.n + splits - 1) / splits) * ((p.Sc + kTile - 1) / kTile), (float)((p.Sq + kTile - 1) / kTile) * p.group);
   const dim3 grid((wk.per_xcd + wq.per_xcd) * 8), block(256);
   if (splits > 1) hipLaunchKernelGGL((bwd_joint_chunks<KK, true>), grid, block, 0, st, p, wq, wk, chunks);
   else hipLaunchKernelGGL((bwd_joint_chunks<KK, false>), grid, block, 0, st, p, wq, wk, chunks);
