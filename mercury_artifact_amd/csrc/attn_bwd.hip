@@ -1132,10 +1132,10 @@ Plan plan_block(int B, int Sq, int Sc, int Hq, int Hkv, int D, bool causal) {
 //     8 chunks 512 x 512 B4 H5      114 / 84.6 / 71.7 / 62.3*     1024 x 1024 H32                299 /  297 / 249* / 240
 //     256 x 256 H16                91.7 / 61.8 / 52.9 / 48.6*     512 x 512 H8/1                 154 /  248 /  128 / 65.4*
 //     1500 x 1500 B2 H12            558 /  446 / 405* / 392       700 x 700 H12                  136 / 98.6 / 88.0 / 77.9*
-float joint_chunks_time(int B, int Sq, int Sc, int Hq, int Hkv, int D, int n) {
+float joint_chunks_time(int B, int Sq, int Sc, int Hq, int Hkv, int D, int n, int most) {
   const int64_t nq = tile_map(B * Hq, Sq, kRowsQ / 2).total, nk = tile_map(B * Hkv, Sc, kRowsKv).total;
   const int64_t workgroups = nq + n * nk;
-  if (n > kMaxGroup || workgroups > kGroupWorkgroups) return INFINITY;
+  if (n > kMaxGroup || workgroups > most) return INFINITY;
   const float tq = (float)((Sc + kTile - 1) / kTile), tk = (float)((Sq + kTile - 1) / kTile) * (Hq / Hkv);
   const Cost c = joint_cost(D);
   const float share = workgroups < 256 ? (float)workgroups / 256.f : 1.f, step = c.step + share * c.busy;
@@ -1157,19 +1157,28 @@ float apart_chunks_time(int B, int Sq, int Sc, int Hq, int Hkv, int D, int n) {
   const float nq = (float)tile_map(B * Hq, Sq, kRowsQ).total, nk = (float)tile_map(B * Hkv, Sc, kRowsKv).total;
   return launch_time(nq, n * tq, n * tq, dq_cost(D)) + launch_time(n * nk, tk, tk, dkv_cost(D));
 }
+// Workgroups of a launch of both passes where those of each pass would leave CUs idle, which
+// has more to fill it with the more chunks there are.  Us a step, up to kGroupWorkgroups / this many:
+//     8 chunks 1024 x 1024 H32      480 /  455      2048 x 2048 H16   840 /  816     700 x 700 B2 H20    345 /  325
+//              1536 x 1536 H32      996 /  975      4096 x 4096 H8   1573 / 1562     6000 x 6000 H5     2172 / 2187 (not taken)
+//     4 chunks 3000 x 3000 H24 D96 1121 / 1099      3072 x 3072 H24  1390 / 1365     1500 x 1500 H48 D64  394 /  380
+constexpr int kStepWorkgroups = 4096;
+constexpr float kLongerLaunch = 0.996f;      // with less to gain by the estimate more chunks to a launch stay out
 bool chunks_apart(int B, int Sq, int Sc, int Hq, int Hkv, int D, int n) {
-  return apart_chunks_time(B, Sq, Sc, Hq, Hkv, D, n) < joint_chunks_time(B, Sq, Sc, Hq, Hkv, D, n);
+  return apart_chunks_time(B, Sq, Sc, Hq, Hkv, D, n) < joint_chunks_time(B, Sq, Sc, Hq, Hkv, D, n, kStepWorkgroups);
 }
-int group_chunks(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks, bool or_apart) {
+int group_chunks(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks, bool step) {
   if (B == 0 || Sq == 0 || Sc == 0) return 1;
   int best = 1;
   float best_time = plan_block(B, Sq, Sc, Hq, Hkv, D, false).time * chunks;
   for (int launches = chunks; launches >= 1; --launches) {
     const int n = (chunks + launches - 1) / launches;
     if (n > kMaxGroup) break;
-    const float joint = joint_chunks_time(B, Sq, Sc, Hq, Hkv, D, n), apart = or_apart ? apart_chunks_time(B, Sq, Sc, Hq, Hkv, D, n) : INFINITY;
+    const float joint = joint_chunks_time(B, Sq, Sc, Hq, Hkv, D, n, step ? kStepWorkgroups : kGroupWorkgroups);
+    const float apart = step ? apart_chunks_time(B, Sq, Sc, Hq, Hkv, D, n) : INFINITY;
+    const bool longer = joint < apart && joint_chunks_time(B, Sq, Sc, Hq, Hkv, D, n, kGroupWorkgroups) == INFINITY;
     const float time = ((chunks + n - 1) / n) * (apart < joint ? apart : joint);
-    if (n > 1 && time < best_time) { best_time = time; best = n; }
+    if (n > 1 && time < (longer ? kLongerLaunch : 1.f) * best_time) { best_time = time; best = n; }
   }
   return best;
 }
