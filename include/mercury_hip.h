@@ -190,7 +190,7 @@ int mhip_attn_bwd_chunk(const void* dout, const void* q, const void* k, const vo
                         float softmax_scale, int mask, void* workspace, void* stream);
 
 /*
- * n chunks of a ring step in one launch, 1 <= n <= MHIP_MAX_GROUP: what n calls of mhip_attn_bwd_chunk without a mask do, with
+ * n chunks of a ring step in one launch, or one of each pass, 1 <= n <= MHIP_MAX_GROUP: what n calls of mhip_attn_bwd_chunk without a mask do, with
  * T the sum over all of them.  ks, vs, dks, dvs, dk32s and dv32s are host arrays of n device pointers (entries of the
  * last four may be NULL, as there); all chunks have one Sc and one set of strides.
  * mhip_attn_bwd_group: how many chunks of a step of `chunks` chunks to put into one launch of both passes when all of them are

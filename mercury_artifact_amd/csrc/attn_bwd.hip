@@ -14,7 +14,7 @@
 // Launches that fill the chip run the passes one after the other (bwd_main): dQ first, with eight wavefronts per
 // workgroup, two per SIMD (it has half the accumulators of the other and fits 256 registers), and its prologue does
 // delta and lse2.  Smaller ones run both passes side by side in one launch (bwd_joint) behind a small one for delta and
-// lse2 (bwd_prepare).
+// lse2 (bwd_prepare).  Steps over several chunks have both forms too (bwd_main_chunks, bwd_joint_chunks).
 // All of them share one body (bwd_pass).  "Stationary" rows (32 per wavefront) sit in the lane index of every
 // MFMA accumulator, "streamed" rows in its registers, exactly as in the forward kernel:
 //     T1[c][r] = X_str[c] . X_st[r]      (scores)          T2[c][r] = Y_str[c] . Y_st[r]      (dP)
