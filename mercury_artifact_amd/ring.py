@@ -182,7 +182,6 @@ def _hop_methods():
 
 
 _HOP = _hop_methods()       # as this package defines them: a wrapper put over one, on a ring or on the class, sees every hop
-_BLOCK = _ops.attn_fwd_block
 
 
 def _resident_chunks(ring, kv):
@@ -245,6 +244,7 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
         raise ValueError("ring_divide must divide the chunk's rows")
     if ring_divide > 1 and ring.chunks is None:
         raise ValueError("ring_divide needs a LocalRing that holds the chunks")
+    sub = Sc // ring_divide
     n_blocks = len(steps) * ring_divide
     defer = (deferred_merge and n_blocks <= MAX_MERGE_MANY and o.dtype == torch.bfloat16
              and o.is_contiguous() and lse.is_contiguous())
@@ -252,24 +252,17 @@ def _ring_forward(q, kv, o, lse, softmax_scale, dropout_p, causal, window_size, 
         warnings.warn(f"ring step of {n_blocks} blocks into a {o.dtype} output: the one-pass fold takes at most "
                       f"{MAX_MERGE_MANY} blocks and writes contiguous bfloat16, so this step merges block by block "
                       "(same result, one pass over the fp32 accumulator per block)", RuntimeWarning, stacklevel=3)
-    # Dividing a ring is for those that want to hold little of other ranks' keys at a time.  Where every chunk lies in this
-    # GPU's memory anyway its parts are views and holding them costs nothing, but a block per part reads Q and leaves a result
-    # k times as often (4096 rows H32, 8 chunks of 4096 keys: 2415 us a step in four parts each, 1695 as whole chunks).  The
-    # ring that was given keeps its place, as it does part by part, and whoever wraps the hops or the block operator sees
-    # every part's.  (Under the causal mask a part of a chunk has a diagonal of its own.)
-    if (ring_divide > 1 and defer and not causal and _resident(ring) and _hop_methods() == _HOP and _ops.attn_fwd_block is _BLOCK
-            and all(c.shape == kv.shape for c in ring.chunks)):
-        ring, ring_divide, n_blocks = LocalRing(ring.mesh_shape, ring.rank, ring.chunks), 1, len(steps)
+    done = 0
+    places = [None] * n_blocks
+    # (a divided ring goes sub-chunk by sub-chunk whether its chunks are all there or not: the option is for rings that want
+    # to hold little of other ranks' keys at a time)
     if defer and not two_streams and ring_divide == 1:
         together = _Together(n_blocks, q, kv, ring, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra)
         if together.size > 1:
             together.step(_resident_chunks(ring, kv), o, lse)
             return
-    done = 0
-    places = [None] * n_blocks
     if defer:
         places = _block_results(n_blocks, q, kv, softmax_scale, dropout_p, causal, window_size, alibi_slopes, **extra)
-    sub = Sc // ring_divide
     main = side = None
     kv_ready = next_ready = None
     if two_streams and defer:

@@ -296,9 +296,9 @@ def test_a_ring_of_another_class_sends_contiguous_chunks():
 
 
 @pytest.mark.parametrize("mesh,S,Hq,Hkv,D,divide", [((4,), 512, 3, 3, 128, 4), ((2, 2), 300, 4, 2, 64, 3), ((8,), 1024, 8, 8, 96, 2)])
-def test_a_divided_ring_of_resident_chunks_takes_them_whole(mesh, S, Hq, Hkv, D, divide):
-    """Bit for bit the undivided step, the ring that was given stays where it was; a wrapper over the hops or the block
-    operator sees every part, and so does a ring whose hops copy."""
+def test_a_divided_ring_takes_its_chunks_in_parts(mesh, S, Hq, Hkv, D, divide):
+    """Wherever the chunks lie and whoever looks on: a ring that copies at every hop, a resident one, and one whose hops or
+    whose block operator are wrapped work on the same parts, bit for bit, and the wrappers see every one of them."""
     import mercury_artifact_amd as M
     from mercury_artifact_amd import flash_attn_interface as FI
 
@@ -314,21 +314,42 @@ def test_a_divided_ring_of_resident_chunks_takes_them_whole(mesh, S, Hq, Hkv, D,
         step(q, kvs[1], o, lse, D ** -0.5, ring=ring, ring_divide=divide)
         return o, lse, ring.held
 
-    whole, parts, copied = run(1), run(divide), run(divide, copy=True)
-    assert torch.equal(whole[0], parts[0]) and torch.equal(whole[1], parts[1])
-    assert parts[2] == list(range(W)) == copied[2]
-    assert (copied[0].float() - whole[0].float()).abs().max().item() <= 2 * 2 ** -8 * whole[0].abs().max().item()
-    seen, real_hop, real_block = [], M.LocalRing.send_recv, FI.attn_fwd_block
+    copied, runs, seen = run(divide, copy=True), [run(divide)], []
+    real_hop, real_block = M.LocalRing.send_recv, FI.attn_fwd_block
     M.LocalRing.send_recv = lambda self, to, source, x, *a: (seen.append(x.shape[2]), real_hop(self, to, source, x, *a))[1]
     try:
-        run(divide)
+        runs.append(run(divide))
     finally:
         M.LocalRing.send_recv = real_hop
     assert seen == [S // divide] * ((W - 1) * divide)
     seen.clear()
     FI.attn_fwd_block = lambda q_, k_, *a, **kw: (seen.append(k_.shape[1]), real_block(q_, k_, *a, **kw))[1]
     try:
-        run(divide)
+        runs.append(run(divide))
     finally:
         FI.attn_fwd_block = real_block
     assert seen == [S // divide] * (W * divide)
+    for o, lse, held in runs:
+        assert torch.equal(o, copied[0]) and torch.equal(lse, copied[1]) and held == list(range(W)) == copied[2]
+    whole = run(1)
+    assert (copied[0].float() - whole[0].float()).abs().max().item() <= 2 * 2 ** -8 * whole[0].abs().max().item()
+
+
+def test_parts_in_reach_of_chunks_that_are_not():
+    """Chunks whose rows lie too far apart for a block over all of them (2 GiB and more from the first to the last), divided into
+    parts that a block can address."""
+    import mercury_artifact_amd as M
+
+    W, S, H, D, apart = 2, 64, 2, 128, 1 << 24
+    q = torch.randn(1, S, H, D, generator=torch.Generator().manual_seed(6)).bfloat16().cuda()
+    memory = torch.empty(S * apart, dtype=torch.bfloat16, device="cuda")
+    wide = [memory.as_strided((2, 1, S, H, D), (H * D, S * apart, apart, D, 1), 2 * i * H * D) for i in range(W)]
+    g = torch.Generator(device="cuda").manual_seed(7)
+    for c in wide:
+        c.copy_(torch.randn(c.shape, generator=g, device="cuda"))
+    runs = []
+    for chunks in (wide, [c.contiguous() for c in wide]):
+        o, lse = torch.empty_like(q), torch.empty(1, H, S, device="cuda")
+        M.flash_attn_pack_kv(q, chunks[1], o, lse, 0.1, ring=M.LocalRing((W,), 1, chunks), ring_divide=2)
+        runs.append((o, lse))
+    assert torch.equal(runs[0][0], runs[1][0]) and torch.equal(runs[0][1], runs[1][1])
