@@ -320,3 +320,30 @@ def test_gradients_nobody_keeps_take_bounded_memory():
 
     one_by_one = peak(Hops((W,), 1, chunks))
     assert peak(M.LocalRing((W,), 1, chunks)) <= one_by_one + (32 << 20)
+
+
+@pytest.mark.parametrize("Hq,D,places,launches", [(64, 128, 2, []), (64, 128, 4, []), (64, 128, 8, [8]), (32, 64, 2, []), (32, 64, 5, [4, 4])])
+def test_gradients_nobody_keeps_are_planned_for_the_places_there_are(Hq, D, places, launches, monkeypatch):
+    """How many chunks share a launch is chosen among what there are places for, chunk by chunk included, and not cut down from
+    what the whole step would have taken, which was chosen for more chunks to fill a launch with."""
+    import mercury_artifact_amd as M
+    from mercury_artifact_amd import ring as R
+
+    W, S = 8, 64
+    assert N.lib().mhip_attn_bwd_take(1, S, S, Hq, 1, D, W) == 8
+    g = torch.Generator(device="cuda").manual_seed(6)
+    q, dout, o = (torch.randn(1, S, Hq, D, generator=g, device="cuda").bfloat16() for _ in range(3))
+    chunks = [torch.randn(2, 1, S, 1, D, generator=g, device="cuda").bfloat16() for _ in range(W)]
+    lse = torch.full((1, Hq, S), 6.0, device="cuda")
+    taken_together, real = [], N.host.bwd_chunks
+    monkeypatch.setattr(N.host, "bwd_chunks", lambda *a: (taken_together.append(len(a[2])), real(*a))[1])
+    monkeypatch.setattr(R, "UNKEPT_BYTES", places * chunks[0].numel() * 2)
+    grads = []
+    for kept in (None, {}):
+        dq, dkv = torch.empty_like(q), torch.empty_like(chunks[1])
+        M.flash_attn_backward(q, chunks[1], o, lse, dout, dq, dkv, D ** -0.5, ring=M.LocalRing((W,), 1, chunks), dkv_chunks=kept)
+        grads.append((dq, dkv))
+    assert taken_together == launches + [8]
+    # the same products summed in fp32 in another order, which can move a dS and a gradient to the next bf16 value
+    for a, b in zip(*grads):
+        assert (a.float() - b.float()).norm() <= 2 ** -8 * b.float().norm()
