@@ -52,8 +52,9 @@ extern "C" {
  * 6: mhip_attn_fwd_blocks, mhip_attn_fwd_group.
  * 7: mhip_attn_bwd_chunks, mhip_attn_bwd_group.
  * 8: mhip_attn_fwd_blocks takes the number of chunks of a result; mhip_attn_fwd_chain.
- * 9: mhip_attn_bwd_take. */
-#define MHIP_ABI_VERSION 9
+ * 9: mhip_attn_bwd_take.
+ * 10: mhip_attn_fwd_tile, mhip_attn_bwd_chunks_plan. */
+#define MHIP_ABI_VERSION 10
 int         mhip_abi_version(void);   /* the MHIP_ABI_VERSION the library was built with */
 int         mhip_version(void);
 /* Optional: per-device set-up the entry points otherwise do on their first call on a device (today: the address
@@ -190,12 +191,13 @@ int mhip_attn_bwd_chunk(const void* dout, const void* q, const void* k, const vo
                         float softmax_scale, int mask, void* workspace, void* stream);
 
 /*
- * n chunks of a ring step in one launch, or one of each pass, 1 <= n <= MHIP_MAX_GROUP: what n calls of mhip_attn_bwd_chunk without a mask do, with
- * T the sum over all of them.  ks, vs, dks, dvs, dk32s and dv32s are host arrays of n device pointers (entries of the
+ * n chunks of a ring step in one launch, or one of each pass, 1 <= n <= MHIP_MAX_GROUP: what n calls of mhip_attn_bwd_chunk without
+ * a mask do, with T the sum over all of them.  ks, vs, dks, dvs, dk32s and dv32s are host arrays of n device pointers (entries of the
  * last four may be NULL, as there); all chunks have one Sc and one set of strides.
- * mhip_attn_bwd_group: how many chunks of a step of `chunks` chunks to put into one launch of both passes when all of them are
- * there; mhip_attn_bwd_take: how many to hand to one call, also where each pass has a launch of its own over them (host
- * functions, nothing is launched).
+ * mhip_attn_bwd_take: how many chunks of a step of `chunks` chunks to hand to one call when all of them are there.
+ * mhip_attn_bwd_group: the same choice without the forms in which each pass has a launch of its own and without launches of more
+ * than 2048 workgroups.  Which form a call takes depends on its sizes and n alone, whichever function n came from
+ * (mhip_attn_bwd_chunks_plan).  Both are host functions, nothing is launched.
  */
 int mhip_attn_bwd_chunks(const void* dout, const void* q, const void* const* ks, const void* const* vs, int n,
                          const void* out, const float* lse,
@@ -218,10 +220,17 @@ int mhip_attn_bwd_take(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks
  * k_ss and v_ss are the row strides of k and v in elements.
  * mhip_attn_bwd_plan: 1 if both passes run side by side in one launch, 2 if one after the other; splits[0] and splits[1]
  * receive the number of workgroups that share a stationary tile of the dQ and of the dK / dV pass.
+ * mhip_attn_fwd_tile: rows and columns of the MFMA tiles (16 or 32) of a bf16 forward launch over n chunks, `per` of them to a
+ * result (mhip_attn_fwd_blocks; n = per = 1: mhip_attn_fwd_block).
+ * mhip_attn_bwd_chunks_plan: the launches, as from mhip_attn_bwd_plan, of a call over n chunks (mhip_attn_bwd_chunks; n = 1: a block,
+ * for which there may be a mask); form[0] receives the number of workgroups that share a stationary tile of the dQ pass, form[1]
+ * the rows and columns of its MFMA tiles.
  * Negative: an MHIP_E* code.
  */
 int mhip_attn_fwd_plan(int B, int Sq, int Sc, int Hq, int D, int64_t k_ss, int64_t v_ss, int mask, int dtype);
+int mhip_attn_fwd_tile(int n, int per, int B, int Sq, int Sc, int Hq, int D, int64_t k_ss, int64_t v_ss, int mask);
 int mhip_attn_bwd_plan(int B, int Sq, int Sc, int Hq, int Hkv, int D, int mask, int* splits);
+int mhip_attn_bwd_chunks_plan(int n, int B, int Sq, int Sc, int Hq, int Hkv, int D, int mask, int* form);
 
 /*
  * LSE-rescale merge.  Replaces the TorchScript `_update_out_and_lse`

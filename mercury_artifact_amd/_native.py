@@ -19,7 +19,7 @@ import torch
 # MERCURY_HIP_LIB is a deployment option: the path of the built library when it is not kept next to the package.
 _BUILT = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB_PATH = os.environ.get("MERCURY_HIP_LIB") or os.path.join(_BUILT, "libmercury_hip.so")
-ABI_VERSION = 9      # MHIP_ABI_VERSION of include/mercury_hip.h the signatures below were written against
+ABI_VERSION = 10     # MHIP_ABI_VERSION of include/mercury_hip.h the signatures below were written against
 
 
 class _NoHost:
@@ -73,7 +73,9 @@ _SIGNATURES = {
     "mhip_attn_bwd_group": (c_int, [_I] * 7),
     "mhip_attn_bwd_take": (c_int, [_I] * 7),
     "mhip_attn_fwd_plan": (c_int, [_I] * 5 + [_L] * 2 + [_I] * 2),
+    "mhip_attn_fwd_tile": (c_int, [_I] * 7 + [_L] * 2 + [_I]),
     "mhip_attn_bwd_plan": (c_int, [_I] * 7 + [ctypes.POINTER(c_int)]),
+    "mhip_attn_bwd_chunks_plan": (c_int, [_I] * 8 + [ctypes.POINTER(c_int)]),
     "mhip_lse_merge": (c_int, [_P] * 8 + [_I] * 4 + [_L] * 17 + [_P]),
     "mhip_lse_merge_many": (c_int, [_P, _P, _P, _P, _I, _P, _P] + [_I] * 4 + [_L] * 2 + [_P]),
     "mhip_flash_reduce": (c_int, [_P] * 3 + [_L, _I, _P]),

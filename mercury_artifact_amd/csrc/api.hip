@@ -11,6 +11,7 @@ int attn_fwd_fp8(const void* q, const void* const* ks, const void* const* vs, in
                  const float* q_descale, const float* k_descale, const float* v_descale, hipStream_t stream);
 int attn_fwd_bf16_chain(int n, int B, int Sq, int Sc, int Hq, int D);
 int attn_fwd_bf16_plan(int blocks, int B, int Sq, int Sc, int Hq, int D, int64_t k_ss, int64_t v_ss, int mask);
+int attn_fwd_bf16_tile(int n, int per, int B, int Sq, int Sc, int Hq, int D, int64_t k_ss, int64_t v_ss, int mask);
 int attn_fwd_fp8_chain(int n, int B, int Sq, int Sc, int Hq, int D);
 int attn_fwd_fp8_plan(int blocks, int B, int Sq, int Sc, int Hq, int mask);
 }  // namespace mhip
@@ -129,4 +130,11 @@ extern "C" int mhip_attn_fwd_plan(int B, int Sq, int Sc, int Hq, int D, int64_t 
   if (mask != MHIP_MASK_NONE && mask != MHIP_MASK_CAUSAL) return MHIP_EINVAL;
   if (dtype == MHIP_E4M3) return attn_fwd_fp8_plan(1, B, Sq, Sc, Hq, mask);
   return dtype == MHIP_BF16 ? attn_fwd_bf16_plan(1, B, Sq, Sc, Hq, D, k_ss, v_ss, mask) : MHIP_EDTYPE;
+}
+
+extern "C" int mhip_attn_fwd_tile(int n, int per, int B, int Sq, int Sc, int Hq, int D, int64_t k_ss, int64_t v_ss, int mask) {
+  if (n < 1 || n > kMaxGroup || per < 1 || per > n) return MHIP_EINVAL;
+  if (B < 0 || Sq < 0 || Sc < 0 || Hq <= 0 || D <= 0 || D > 128 || k_ss < 0 || v_ss < 0) return MHIP_EINVAL;
+  if (mask != MHIP_MASK_NONE && (mask != MHIP_MASK_CAUSAL || per > 1)) return MHIP_EINVAL;
+  return attn_fwd_bf16_tile(n, per, B, Sq, Sc, Hq, D, k_ss, v_ss, mask);
 }

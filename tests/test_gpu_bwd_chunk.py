@@ -22,6 +22,22 @@ def taken(B, Sq, Sc, Hq, Hkv, D, causal):
     return N.lib().mhip_attn_bwd_plan(B, Sq, Sc, Hq, Hkv, D, int(causal), splits), splits[0], splits[1]
 
 
+def form(n, B, Sq, Sc, Hq, Hkv, D):
+    """(launches, workgroups per query tile of the dQ pass, rows of its MFMA tiles) of a call over n chunks."""
+    what = (ctypes.c_int * 2)()
+    return N.lib().mhip_attn_bwd_chunks_plan(n, B, Sq, Sc, Hq, Hkv, D, 0, what), what[0], what[1]
+
+
+def by_hops(W, rank, chunks):
+    """A ring that makes no promise about its chunks: one launch (or one of each pass) for every chunk."""
+    import mercury_artifact_amd as M
+
+    class Hops(M.LocalRing):
+        pass
+
+    return Hops((W,), rank, chunks)
+
+
 def _close(name, got, ref):
     got, ref = got.float().cpu(), ref.float()
     rms = ref.square().mean().sqrt()
@@ -38,6 +54,7 @@ IN_TURN = [(3, 130, 128, 128, 64), (3, 130, 128, 64, 88), (3, 130, 128, 128, 128
 @pytest.mark.parametrize("W,S,Hq,Hkv,D", JOINT + IN_TURN)
 @pytest.mark.parametrize("dq_dtype,keep", [(torch.bfloat16, True), (torch.float32, True), (torch.bfloat16, False)])
 def test_backward_step_carries_the_sums(W, S, Hq, Hkv, D, dq_dtype, keep):
+    """Chunk by chunk, and on a ring whose chunks may go together."""
     import mercury_artifact_amd as M
 
     print(f"W{W} S{S} Hq{Hq} Hkv{Hkv} D{D} {dq_dtype} keep={keep}", flush=True)
@@ -50,19 +67,20 @@ def test_backward_step_carries_the_sums(W, S, Hq, Hkv, D, dq_dtype, keep):
     o, lse = O.ring_forward(q.float(), [c.float() for c in kvs], order, scale)
     rdq, rdkv = O.ring_backward(q.float(), [c.float() for c in kvs], order, o.bfloat16().float(), lse, dout.float(), scale)
     dev = [c.cuda() for c in kvs]
-    dq = torch.full(q.shape, float("nan"), dtype=dq_dtype, device="cuda")
-    dkv = torch.full_like(dev[rank], float("nan"))
-    got = {} if keep else None
-    M.flash_attn_backward(q.cuda(), dev[rank], o.bfloat16().cuda(), lse.cuda(), dout.cuda(), dq, dkv, scale,
-                          ring=M.LocalRing((W,), rank, dev), dkv_chunks=got)
-    torch.cuda.synchronize()
-    _close("dq", dq, rdq)
-    _close("own dkv", dkv, torch.stack(tuple(rdkv[rank])))
-    if keep:
-        assert torch.equal(got[rank], dkv.float())
-    for c in range(W) if keep else ():
-        assert got[c].dtype == torch.float32
-        _close(f"dkv {c}", got[c], torch.stack(tuple(rdkv[c])))
+    for ring in (by_hops(W, rank, dev), M.LocalRing((W,), rank, dev)):
+        dq = torch.full(q.shape, float("nan"), dtype=dq_dtype, device="cuda")
+        dkv = torch.full_like(dev[rank], float("nan"))
+        got = {} if keep else None
+        M.flash_attn_backward(q.cuda(), dev[rank], o.bfloat16().cuda(), lse.cuda(), dout.cuda(), dq, dkv, scale, ring=ring,
+                              dkv_chunks=got)
+        torch.cuda.synchronize()
+        _close("dq", dq, rdq)
+        _close("own dkv", dkv, torch.stack(tuple(rdkv[rank])))
+        if keep:
+            assert torch.equal(got[rank], dkv.float())
+        for c in range(W) if keep else ():
+            assert got[c].dtype == torch.float32
+            _close(f"dkv {c}", got[c], torch.stack(tuple(rdkv[c])))
 
 
 @pytest.mark.parametrize("W,S,Hq,Hkv,D", [(8, 130, 2, 2, 128), (5, 200, 4, 2, 112), (7, 193, 3, 3, 96), (8, 65, 2, 1, 40), (3, 700, 2, 2, 64),
@@ -75,7 +93,9 @@ def test_a_query_tile_shared_by_workgroups_of_a_step(W, S, Hq, Hkv, D, dq_dtype)
 
     print(f"shared W{W} S{S} Hq{Hq} Hkv{Hkv} D{D} {dq_dtype}", flush=True)
     B, rank, scale = 1, 1, D ** -0.5
-    assert N.lib().mhip_attn_bwd_group(B, S, S, Hq, Hkv, D, W) >= min(W, 12)
+    together = N.lib().mhip_attn_bwd_take(B, S, S, Hq, Hkv, D, W)
+    launches, shared_by, _ = form(together, B, S, S, Hq, Hkv, D)
+    assert together == min(W, 12) and launches == 1 and shared_by > 1
     g = torch.Generator().manual_seed(W * 1000 + S)
     q, dout = (torch.randn(B, S, Hq, D, generator=g).bfloat16() for _ in range(2))
     kvs = [torch.randn(2, B, S, Hkv, D, generator=g).bfloat16() for _ in range(W)]
@@ -214,7 +234,7 @@ def test_backward_step_in_grouped_launches(W, B, S, Hq, Hkv, D, group, dq_dtype,
     import mercury_artifact_amd as M
 
     print(f"grouped W{W} B{B} S{S} Hq{Hq} Hkv{Hkv} D{D} {dq_dtype} keep={keep}", flush=True)
-    assert N.lib().mhip_attn_bwd_group(B, S, S, Hq, Hkv, D, W) == group
+    assert N.lib().mhip_attn_bwd_take(B, S, S, Hq, Hkv, D, W) == group and form(group, B, S, S, Hq, Hkv, D)[0] == 1
     rank, scale = W // 2, D ** -0.5
     g = torch.Generator().manual_seed(W * 1000 + S)
     q, dout = (torch.randn(B, S, Hq, D, generator=g).bfloat16() for _ in range(2))
@@ -235,12 +255,9 @@ def test_backward_step_in_grouped_launches(W, B, S, Hq, Hkv, D, group, dq_dtype,
         assert got[c].dtype == torch.float32
         _close(f"dkv {c}", got[c], torch.stack(tuple(rdkv[c])))
 
-    class Other(M.LocalRing):            # makes no promise about its chunks: one launch each, the same gradients
-        pass
-
     dq1, dkv1, got1 = torch.empty_like(dq), torch.empty_like(dkv), {} if keep else None
     M.flash_attn_backward(q.cuda(), dev[rank], o.bfloat16().cuda(), lse.cuda(), dout.cuda(), dq1, dkv1, scale,
-                          ring=Other((W,), rank, dev), dkv_chunks=got1)
+                          ring=by_hops(W, rank, dev), dkv_chunks=got1)
     _close("dq, chunk by chunk", dq1, rdq)
     _close("dkv, chunk by chunk", dkv1, torch.stack(tuple(rdkv[rank])))
 
@@ -251,7 +268,7 @@ def test_grouped_gradients_over_operands(over):
     import mercury_artifact_amd as M
 
     W, B, S, H, D = 4, 1, 200, 4, 64
-    assert N.lib().mhip_attn_bwd_group(B, S, S, H, H, D, W) == 4
+    assert N.lib().mhip_attn_bwd_take(B, S, S, H, H, D, W) == 4
     g = torch.Generator().manual_seed(3)
 
     def fresh():
@@ -301,15 +318,12 @@ def test_gradients_nobody_keeps_take_bounded_memory():
     import mercury_artifact_amd as M
 
     W, S, H, D = 8, 2048, 8, 128
-    assert N.lib().mhip_attn_bwd_group(1, S, S, H, H, D, W) * 2 * S * H * D * 2 > 60 << 20
+    assert N.lib().mhip_attn_bwd_take(1, S, S, H, H, D, W) * 2 * S * H * D * 2 > 60 << 20
     g = torch.Generator(device="cuda").manual_seed(2)
     q, dout, o = (torch.randn(1, S, H, D, generator=g, device="cuda").bfloat16() for _ in range(3))
     chunks = [torch.randn(2, 1, S, H, D, generator=g, device="cuda").bfloat16() for _ in range(W)]
     lse = torch.full((1, H, S), 9.0, device="cuda")
     dq, dkv = torch.empty_like(q), torch.empty_like(chunks[0])
-
-    class Hops(M.LocalRing):             # a launch per chunk: one such gradient at a time
-        pass
 
     def peak(ring):
         torch.cuda.synchronize()
@@ -318,7 +332,7 @@ def test_gradients_nobody_keeps_take_bounded_memory():
         M.flash_attn_backward(q, chunks[1], o, lse, dout, dq, dkv, D ** -0.5, ring=ring)
         return torch.cuda.max_memory_allocated() - before
 
-    one_by_one = peak(Hops((W,), 1, chunks))
+    one_by_one = peak(by_hops(W, 1, chunks))         # one such gradient at a time
     assert peak(M.LocalRing((W,), 1, chunks)) <= one_by_one + (32 << 20)
 
 

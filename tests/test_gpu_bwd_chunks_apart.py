@@ -7,6 +7,7 @@ import torch
 import oracle as O
 from mercury_artifact_amd import _native as N
 from test_gpu_bwd import _check_grad
+from test_gpu_bwd_chunk import by_hops, form
 
 pytestmark = pytest.mark.gpu
 
@@ -24,6 +25,8 @@ def test_a_step_with_a_launch_for_each_pass(B, Sq, Sc, Hq, Hkv, D, W, dq_dtype, 
     together = N.lib().mhip_attn_bwd_take(B, Sq, Sc, Hq, Hkv, D, W)
     workgroups = B * Hq * -(-Sq // 128) + together * B * Hkv * -(-Sc // 128)
     assert together == min(W, 10 if W > 16 else 16) and workgroups > 4096         # more than both passes share a launch with
+    small = D > 64 and together * -(-Sc // 64) >= 32                              # the dQ pass on 16 x 16 MFMA tiles
+    assert form(together, B, Sq, Sc, Hq, Hkv, D) == (2, 1, 16 if small else 32)
     rank, scale = W // 2, D ** -0.5
     g = torch.Generator(device="cuda").manual_seed(W * 1000 + Sq)
     q, dout = (torch.randn(B, Sq, Hq, D, generator=g, device="cuda").bfloat16() for _ in range(2))
@@ -32,14 +35,11 @@ def test_a_step_with_a_launch_for_each_pass(B, Sq, Sc, Hq, Hkv, D, W, dq_dtype, 
     heads, group = [(0, 0), (B - 1, Hq - 1)], Hq // Hkv
     out, lse = M.attn_fwd_block(q, torch.cat([c[0] for c in chunks], 1), torch.cat([c[1] for c in chunks], 1), scale)
 
-    class Other(M.LocalRing):            # makes no promise about its chunks: one launch each
-        pass
-
     runs = []
-    for ring in (M.LocalRing, M.LocalRing, Other):
+    for ring in (M.LocalRing((W,), rank, chunks), M.LocalRing((W,), rank, chunks), by_hops(W, rank, chunks)):
         dq, dkv = torch.full(q.shape, float("nan"), dtype=dq_dtype, device="cuda"), torch.full_like(chunks[rank], float("nan"))
         kept = {} if keep else None
-        M.flash_attn_backward(q, chunks[rank], out, lse, dout, dq, dkv, scale, ring=ring((W,), rank, chunks), dkv_chunks=kept)
+        M.flash_attn_backward(q, chunks[rank], out, lse, dout, dq, dkv, scale, ring=ring, dkv_chunks=kept)
         torch.cuda.synchronize()
         runs.append((dq, dkv, kept))
     assert torch.equal(runs[0][0], runs[1][0])

@@ -9,16 +9,22 @@ import torch
 import oracle as O
 from mercury_artifact_amd import _native as N
 from test_gpu_bwd import _check_grad
+from test_gpu_bwd_chunk import by_hops
 
 pytestmark = pytest.mark.gpu
 H = 32
 
 
+def _form(Sq, Sc, D, causal):
+    """(launches, workgroups per query tile, rows of the dQ pass's MFMA tiles) of a block."""
+    what = (ctypes.c_int * 2)()
+    return N.lib().mhip_attn_bwd_chunks_plan(1, 1, Sq, Sc, H, H, D, int(causal), what), what[0], what[1]
+
+
 def _run(Sq, Sc, D, causal, heads=(0, 31)):
     import mercury_artifact_amd as M
 
-    splits = (ctypes.c_int * 2)()
-    assert N.lib().mhip_attn_bwd_plan(1, Sq, Sc, H, H, D, int(causal), splits) == 2
+    assert _form(Sq, Sc, D, causal) == (2, 1, 16)
     print(f"small tiles, backward Sq{Sq} Sc{Sc} D{D} causal={causal}", flush=True)
     g = torch.Generator().manual_seed(Sq * 1009 + Sc + D)
     q, dout = (torch.randn(1, Sq, H, D, generator=g).bfloat16() for _ in range(2))
@@ -53,6 +59,68 @@ def test_a_block_at_tile_edges(Sq, Sc, D):
 def test_under_the_causal_mask(Sq, Sc, D):
     """Rows that see every key, none, and keys up to a diagonal inside a 16-key block."""
     _run(Sq, Sc, D, True, heads=(0, 17))
+
+
+@pytest.mark.parametrize("Sq,Sc,D,causal", [(1793, 1985, 128, False), (1793, 2048, 96, False), (4081, 4081, 128, True), (4090, 4225, 96, True)])
+def test_rows_prepared_by_an_earlier_chunk(Sq, Sc, D, causal):
+    """lse2 and delta as an earlier chunk's call left them: a later call on them computes what one computes that works them out
+    itself, bit for bit, alone, and as the first, a middle and the last chunk of a carried sum."""
+    import mercury_artifact_amd as M
+
+    assert _form(Sq, Sc, D, causal) == (2, 1, 16)
+    print(f"prepared Sq{Sq} Sc{Sc} D{D} causal={causal}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(Sq + Sc + D)
+    mk = lambda rows: torch.randn(1, rows, H, D, generator=g, device="cuda").bfloat16()
+    q, dout, k, v, scale = mk(Sq), mk(Sq), mk(Sc), mk(Sc), D ** -0.5
+    out, lse = M.attn_fwd_block(q, k, v, scale, causal=causal)
+    want = [torch.empty_like(t) for t in (q, k, v)]
+    M.attn_bwd_block(dout, q, k, v, out, lse, *want, scale, causal=causal)
+    workspace = torch.empty(N.lib().mhip_attn_bwd_workspace_bytes(1, Sq, Sc, H, H, D), dtype=torch.uint8, device="cuda")
+    acc = torch.full(q.shape, float("nan"), device="cuda")
+
+    def call(first, last, prepared):
+        dq, dk, dv = (torch.full_like(t, float("nan")) for t in (q, k, v))
+        strides = [st for t in (q, k, dk, dq, out) for st in t.stride()[:3]]
+        N.check(N.lib().mhip_attn_bwd_chunk(*map(N.ptr, (dout, q, k, v, out, lse)), N.ptr(dq), N.ptr(acc), first, last, prepared, N.ptr(dk),
+                                            N.ptr(dv), None, None, 1, Sq, Sc, H, H, D, *strides, scale, int(causal), N.ptr(workspace),
+                                            N.stream_of(q)), "mhip_attn_bwd_chunk")
+        torch.cuda.synchronize()
+        assert torch.equal(dk, want[1]) and torch.equal(dv, want[2])
+        return dq
+
+    for prepared in (0, 1):
+        assert torch.equal(call(1, 1, prepared), want[0])
+    call(1, 0, 1)
+    once = acc.clone()
+    assert torch.equal(once.bfloat16(), want[0])
+    call(0, 0, 1)
+    assert torch.equal(acc, once + once)
+    assert torch.equal(call(0, 1, 1), (once + once + once).bfloat16())
+
+
+@pytest.mark.parametrize("Sq,Sc,D", [(1793, 1985, 128), (1809, 2047, 96)])
+def test_a_ring_that_hands_over_chunk_by_chunk(Sq, Sc, D):
+    """The block's kernels from the second chunk on: prepared rows, a carried dQ, fp32 gradients of the chunks."""
+    import mercury_artifact_amd as M
+
+    W, rank, scale, heads = 3, 1, D ** -0.5, (0, 31)
+    assert _form(Sq, Sc, D, False) == (2, 1, 16)
+    print(f"small tiles, by hops Sq{Sq} Sc{Sc} D{D}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(Sq * 7 + Sc + D)
+    q, dout = (torch.randn(1, Sq, H, D, generator=g, device="cuda").bfloat16() for _ in range(2))
+    chunks = [torch.randn(2, 1, Sc, H, D, generator=g, device="cuda").bfloat16() for _ in range(W)]
+    out, lse = M.attn_fwd_block(q, torch.cat([c[0] for c in chunks], 1), torch.cat([c[1] for c in chunks], 1), scale)
+    dq, dkv, kept = torch.full_like(q, float("nan")), torch.full_like(chunks[rank], float("nan")), {}
+    M.flash_attn_backward(q, chunks[rank], out, lse, dout, dq, dkv, scale, ring=by_hops(W, rank, chunks), dkv_chunks=kept)
+    torch.cuda.synchronize()
+    assert torch.equal(kept[rank], dkv.float())
+    for h in heads:
+        one = lambda t: t[..., h:h + 1, :].float().cpu()
+        rdq, rdkv = O.ring_backward(one(q), [one(c) for c in chunks], O.single_ring_order(rank, W), one(out), lse[:, h:h + 1].cpu(),
+                                    one(dout), scale)
+        _check_grad(f"dq head {h}", one(dq), rdq)
+        for c in range(W):
+            _check_grad(f"dkv {c} head {h}", one(kept[c]), torch.stack(tuple(rdkv[c])))
 
 
 def test_the_same_bits_every_time():

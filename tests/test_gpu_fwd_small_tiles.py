@@ -28,7 +28,7 @@ def _check(q, kv, out, lse, scale, causal, tag, heads):
 def _run(Sq, Sc, D, n, causal, ramp, tag):
     """n chunks as one result (n = 1: a lone block)."""
     B, H, Hkv, heads = (1, 32, 8, [(0, 0), (0, 31)]) if causal else (2, HEADS, 8, [(0, 0), (0, 77), (1, 127)])
-    assert N.lib().mhip_attn_fwd_plan(B, Sq, Sc, H, D, Hkv * D, Hkv * D, int(causal), N.MHIP_BF16) == 1 or n > 1
+    assert N.lib().mhip_attn_fwd_tile(n, n, B, Sq, Sc, H, D, Hkv * D, Hkv * D, int(causal)) == 16
     print(tag, flush=True)
     g = torch.Generator().manual_seed(Sq * 1009 + Sc + D)
     q = torch.randn(B, Sq, H, D, generator=g)
@@ -78,6 +78,7 @@ def test_a_moving_reference(Sq, Sc, D, n, causal, ramp):
 def test_rows_move_their_references_on_their_own():
     """Only one row in 16 outgrows its reference, and only in one tile: the other rows of its lane keep theirs."""
     B, Sq, Sc, H, D = 2, 256, 2048, HEADS, 128
+    assert N.lib().mhip_attn_fwd_tile(1, 1, B, Sq, Sc, H, D, 8 * D, 8 * D, 0) == 16
     g = torch.Generator().manual_seed(3)
     q, kv = torch.randn(B, Sq, H, D, generator=g), torch.randn(2, B, Sc, 8, D, generator=g)
     q[..., 0] = 0.0
@@ -94,6 +95,7 @@ def test_rows_move_their_references_on_their_own():
 def test_a_key_of_nan_reaches_the_rows_that_see_it():
     import mercury_artifact_amd as M
 
+    assert N.lib().mhip_attn_fwd_tile(1, 1, 1, 4100, 4100, 32, 128, 1024, 1024, 1) == 16
     g = torch.Generator().manual_seed(11)
     q = torch.randn(1, 4100, 32, 128, generator=g).bfloat16().cuda()
     kv = torch.randn(2, 1, 4100, 8, 128, generator=g).bfloat16().cuda()

@@ -2,7 +2,7 @@
 it is for; when a rule moves, these assertions say which kernels have been left without one."""
 import pytest
 import test_gpu_fwd_key_groups as G
-from test_gpu_bwd_chunk import IN_TURN, JOINT, taken as bwd_plan
+from test_gpu_bwd_chunk import GROUPED, IN_TURN, JOINT, form, taken as bwd_plan
 
 from mercury_artifact_amd import _native as N
 
@@ -60,6 +60,36 @@ def test_blocks_of_a_step_share_a_launch_of_up_to_eight_rounds():
     assert group(1, 16, 1, 64) == 16                                          # what an argument list holds
     assert group(1, 256, 4, 1) == 1 and group(1, 0, 4, 8) == group(0, 64, 4, 8) == 1
     assert group(1, 64, 0, 8) < 0 and group(1, 64, 4, 0) < 0 and group(-1, 64, 4, 1) < 0
+
+
+def test_chunks_of_a_backward_step_go_together():
+    """What the ring driver asks for, and the form of the call it then makes."""
+    take = N.lib().mhip_attn_bwd_take
+    assert take(1, 4096, 4096, 32, 32, 128, 8) == 8 and form(8, 1, 4096, 4096, 32, 32, 128) == (2, 1, 16)
+    assert take(1, 1024, 1024, 32, 32, 128, 8) == 8 and form(8, 1, 1024, 1024, 32, 32, 128) == (1, 1, 32)
+    assert take(1, 6000, 6000, 5, 5, 128, 8) == 4                             # 8 would be expected to gain 0.3 %
+    assert take(4, 512, 512, 5, 5, 128, 8) == 8 and form(8, 4, 512, 512, 5, 5, 128) == (1, 1, 32)
+    assert take(1, 512, 512, 4, 4, 128, 8) == 8 and form(8, 1, 512, 512, 4, 4, 128) == (1, 4, 32)
+    assert take(1, 64, 64, 1, 1, 64, 40) == 14 and form(14, 1, 64, 64, 1, 1, 64)[1] == 8
+    assert form(2, 4, 319, 319, 32, 32, 64) == (2, 1, 32)                     # also where mhip_attn_bwd_group says 2
+    assert form(8, 1, 2048, 2048, 32, 32, 64) == (2, 1, 32)                   # 64 columns keep the larger MFMA tiles
+    assert take(1, 256, 256, 4, 4, 64, 1) == take(0, 64, 64, 4, 4, 64, 8) == take(1, 0, 64, 4, 4, 64, 8) == 1
+    assert take(1, 64, 64, 4, 3, 64, 8) < 0 and take(1, 64, 64, 4, 4, 136, 8) < 0 and take(1, 64, 64, 4, 4, 64, 0) < 0
+    assert form(17, 1, 64, 64, 4, 4, 64)[0] < 0 and form(0, 1, 64, 64, 4, 4, 64)[0] < 0 and form(1, 1, 64, 64, 4, 3, 64)[0] < 0
+    for W, B, S, Hq, Hkv, D, group in GROUPED:
+        assert take(B, S, S, Hq, Hkv, D, W) == group and form(group, B, S, S, Hq, Hkv, D)[0] == 1
+
+
+def test_mfma_tiles_of_the_forward():
+    tile = N.lib().mhip_attn_fwd_tile
+    rows = [4096, 4096]
+    assert [tile(8, 8, 1, 4096, 4096, 32, D, *rows, 0) for D in (64, 96, 128)] == [16, 16, 16]
+    assert [tile(1, 1, 1, 4096, 4096, 32, D, *rows, 1) for D in (64, 96, 128)] == [32, 32, 16]
+    assert tile(8, 8, 1, 256, 256, 32, 128, *rows, 0) == 32 and tile(1, 1, 2, 256, 2048, 128, 128, *rows, 0) == 16
+    assert tile(1, 1, 2, 256, 2048, 128, 96, *rows, 0) == 32                  # 32 key tiles: 64 from here on
+    assert tile(1, 1, 1, 256, 256, 4, 128, *rows, 0) == 32                    # four key groups
+    assert tile(0, 1, 1, 64, 64, 4, 128, *rows, 0) < 0 and tile(2, 3, 1, 64, 64, 4, 128, *rows, 0) < 0
+    assert tile(2, 2, 1, 64, 64, 4, 128, *rows, 1) < 0 and tile(1, 1, 1, 64, 64, 4, 136, *rows, 0) < 0
 
 
 def test_chunks_of_a_backward_step_share_a_launch():
