@@ -826,17 +826,19 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
       }
     }
   };
-  // The same with fp32 rows on the way (512 or 256 bytes, their chunks of 4 columns swizzled by the row).  An instruction
-  // covers whole rows without a gap: a lane's own accumulator columns are 16 bytes of 32 different rows, and 8 columns per
-  // lane in two stores leave every other 16 bytes to the second one.  `fetch` gives what is there already, all of it on
-  // the way before the first store (a load cannot pass a store that may be to the same place, so that one row's after
-  // the other cost a round trip each), and `finish` gets the lane's 4 columns of a row: a step of 8 chunks 4096 x 4096 H32,
-  // dQ carried in fp32, 6838 us to 6790, causal 1500 x 1500 B2 H12 D 64 61.3 to 61.0.
-  auto write_out32 = [&](const Acc (&acc)[DB][R], float mul, auto&& fetch, auto&& finish) {
+  // The same with fp32 rows on the way (512 or 256 bytes, their chunks of 4 columns swizzled by the row).  A lane has 4 or 8
+  // columns of a row: a lane's own accumulator columns are 16 bytes of 32 different rows.  `fetch` gives what is there already, all
+  // of it on the way before the first store (a load cannot pass a store that may be to the same place, so that one row's after
+  // the other cost a round trip each), and `finish` gets the sums and that.  Rows that are fetched go with 4 columns to a lane, so
+  // that an instruction covers whole rows without a gap: a step of 8 chunks 4096 x 4096 H32, dQ carried in fp32, 6838 us to 6790.
+  // Rows that are only written go with 8, half as many of them with twice the work: 8 chunks 512 x 512 B4 H5, both passes in one
+  // launch, 85.5 us / 87.6 with 4.
+  auto write_out32 = [&](const Acc (&acc)[DB][R], float mul, auto columns, auto&& fetch, auto&& finish) {
     own_lds_order();
-    constexpr int kRow32 = 2 * kRow, kPlaces = kRow32 / 16, kRowsAtOnce = 64 / kPlaces, kIts = 32 / kRowsAtOnce;
+    constexpr int kH = decltype(columns)::value / 4, kRow32 = 2 * kRow, kPlaces = kRow32 / 16, kLanes = kPlaces / kH;
+    constexpr int kRowsAtOnce = 64 / kLanes, kIts = 32 / kRowsAtOnce;
     unsigned char* os = smem + wave * (32 * kRow32);
-    const int col = lane % kPlaces * 4, first_row = r0 + wave * 32 + lane / kPlaces;
+    const int place = lane % kLanes * kH, col = place * 4, first_row = r0 + wave * 32 + lane / kLanes;
     f32x4 old[kIts];
 #pragma unroll
     for (int it = 0; it < kIts; ++it) {
@@ -853,34 +855,42 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     own_lds_order();
 #pragma unroll
     for (int it = 0; it < kIts; ++it) {
-      const int r = lane / kPlaces + kRowsAtOnce * it;
-      if (first_row + it * kRowsAtOnce < n_st && col < p.D)
-        finish(*reinterpret_cast<const f32x4*>(os + r * kRow32 + (((col >> 2) ^ (r % kPlaces)) << 4)), old[it], first_row + it * kRowsAtOnce, col);
+      const int r = lane / kLanes + kRowsAtOnce * it;
+      if (first_row + it * kRowsAtOnce < n_st && col < p.D) {
+        f32x4 v[kH];
+#pragma unroll
+        for (int h = 0; h < kH; ++h) v[h] = *reinterpret_cast<const f32x4*>(os + r * kRow32 + (((place + h) ^ (r % kPlaces)) << 4));
+        finish(v, old[it], first_row + it * kRowsAtOnce, col);
+      }
     }
   };
+  const std::integral_constant<int, 4> four;
+  const std::integral_constant<int, 8> eight;
   auto pack4 = [](const f32x4& v) { return u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])}; };
   auto nothing = [](int, int) { return f32x4{}; };
   if (SPLIT && w.splits > 1) {
     // fp32 sums for bwd_reduce, (b, row, head, column) like the gradient itself
     const int64_t size = (int64_t)p.B * n_st * (DQ ? p.Hq : p.Hkv) * p.D;
     auto part = [&](float* base) {
-      return [=](const f32x4& v, const f32x4&, int row, int col) {
-        *reinterpret_cast<f32x4*>(base + split * size + (((int64_t)b * n_st + row) * (DQ ? p.Hq : p.Hkv) + hs) * p.D + col) = v;
+      return [=](const f32x4 (&v)[2], const f32x4&, int row, int col) {
+        f32x4* op = reinterpret_cast<f32x4*>(base + split * size + (((int64_t)b * n_st + row) * (DQ ? p.Hq : p.Hkv) + hs) * p.D + col);
+        op[0] = v[0];
+        op[1] = v[1];
       };
     };
-    write_out32(acc1, p.scale, nothing, part(w.partial));
-    if (!DQ) write_out32(acc2, 1.f, nothing, part(w.partial + w.splits * size));
+    write_out32(acc1, p.scale, eight, nothing, part(w.partial));
+    if (!DQ) write_out32(acc2, 1.f, eight, nothing, part(w.partial + w.splits * size));
   } else if (DQ) {
     if (p.dq_acc == nullptr) {
       write_out(acc1, p.scale, p.dq, p.dq_sb, p.dq_ss, p.dq_sh, hs);
     } else {
       uint16_t* dq = p.dq ? p.dq + b * p.dq_sb + hs * p.dq_sh : nullptr;
       auto at = [&](int row, int col) { return reinterpret_cast<f32x4*>(p.dq_acc + (((int64_t)b * p.Sq + row) * p.Hq + hs) * p.D + col); };
-      write_out32(acc1, p.scale, [&](int row, int col) { return p.dq_mode != kDqFirst ? *at(row, col) : f32x4{}; },
-                  [&](const f32x4& v, const f32x4& old, int row, int col) {
+      write_out32(acc1, p.scale, four, [&](int row, int col) { return p.dq_mode != kDqFirst ? *at(row, col) : f32x4{}; },
+                  [&](const f32x4 (&v)[1], const f32x4& old, int row, int col) {
         u32x2* qp = reinterpret_cast<u32x2*>(dq + (int64_t)row * p.dq_ss + col);
-        if (p.dq_mode == kDqAdd && dq) *qp = pack4(v);
-        const f32x4 sum = p.dq_mode != kDqFirst ? v + old : v;
+        if (p.dq_mode == kDqAdd && dq) *qp = pack4(v[0]);
+        const f32x4 sum = p.dq_mode != kDqFirst ? v[0] + old : v[0];
         if (p.dq_mode != kDqLast) *at(row, col) = sum;
         else *qp = pack4(sum);
       });
@@ -890,15 +900,16 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     write_out(acc2, 1.f, CHUNKS ? chunks->dv[chunk] : p.dv, p.dk_sb, p.dk_ss, p.dk_sh, hs);
   } else {
     auto store = [&](float* out32, uint16_t* out16) {
-      return [=](const f32x4& v, const f32x4&, int row, int col) {
-        const u32x2 w = pack4(v);
-        *reinterpret_cast<f32x4*>(out32 + (((int64_t)b * p.Sc + row) * p.Hkv + hs) * p.D + col) =
-            f32x4{bf16_lo(w[0]), bf16_hi(w[0]), bf16_lo(w[1]), bf16_hi(w[1])};
-        if (out16) *reinterpret_cast<u32x2*>(out16 + b * p.dk_sb + (int64_t)row * p.dk_ss + hs * p.dk_sh + col) = w;
+      return [=](const f32x4 (&v)[2], const f32x4&, int row, int col) {
+        const u32x2 lo = pack4(v[0]), hi = pack4(v[1]);
+        f32x4* op = reinterpret_cast<f32x4*>(out32 + (((int64_t)b * p.Sc + row) * p.Hkv + hs) * p.D + col);
+        op[0] = f32x4{bf16_lo(lo[0]), bf16_hi(lo[0]), bf16_lo(lo[1]), bf16_hi(lo[1])};
+        op[1] = f32x4{bf16_lo(hi[0]), bf16_hi(hi[0]), bf16_lo(hi[1]), bf16_hi(hi[1])};
+        if (out16) *reinterpret_cast<u32x4*>(out16 + b * p.dk_sb + (int64_t)row * p.dk_ss + hs * p.dk_sh + col) = u32x4{lo[0], lo[1], hi[0], hi[1]};
       };
     };
-    write_out32(acc1, p.scale, nothing, store(CHUNKS ? chunks->dk32[chunk] : p.dk32, CHUNKS ? chunks->dk[chunk] : p.dk));
-    write_out32(acc2, 1.f, nothing, store(CHUNKS ? chunks->dv32[chunk] : p.dv32, CHUNKS ? chunks->dv[chunk] : p.dv));
+    write_out32(acc1, p.scale, eight, nothing, store(CHUNKS ? chunks->dk32[chunk] : p.dk32, CHUNKS ? chunks->dk[chunk] : p.dk));
+    write_out32(acc2, 1.f, eight, nothing, store(CHUNKS ? chunks->dv32[chunk] : p.dv32, CHUNKS ? chunks->dv[chunk] : p.dv));
   }
 }
 
