@@ -767,13 +767,18 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_fwd_bf16_d128(const P p) 
 //     D 128  512 x 512  1644 / 1554   256 x 256   419 /  399   224 x 512   750 /  711   256 x 32  59.6 / 58.6   512 x 8  42.9 / 43.6
 //            160 x 512   595 /  597   288 x 512  1333 / 1344   160 x 20   29.1 / 32.0
 //     D 96   512 x 128   338 /  328   256 x 64   90.0 / 87.1   224 x 64   80.1 / 80.1   256 x 32  46.6 / 46.5   160 x 20  24.3 / 27.0
-//     D 64   512 x 128   257 /  250   256 x 64   68.9 / 66.4   224 x 512   477 /  498   256 x 32  34.8 / 35.7   160 x 20  19.9 / 22.9
+//     D 64   runs of chunks: 8 chunks 4096 x 4096 H32 1018 / 1002, H32/8 1020 / 979, 4 chunks 8192 x 8192 H32 2047 / 1973,
+//            8 chunks 2048 x 2048 H32 262 / 249, B2 H32/4 524 / 490        224 x 512   477 /  498
 //     causal 4096 x 4096 H32: D 128  122.9 / 117.5   D 96  98.1 / 96.7   D 64  74.6 / 75.5
-// (on 96 columns 1.4 % at the one causal size measured was not taken for enough).  All on N(0,1) operands.  The fewer bits the
+// (on 96 columns 1.4 % at the one causal size measured was not taken for enough).  Chunk by chunk launches up to 64 columns, whose
+// vector work is the larger part, gain and lose by turns and more often lose: D 64 4096 x 4096 H32 139 / 134, H32/8 132 / 134,
+// 7900 x 7900 H8 122 / 125, 8192 x 8192 H16/2 258 / 264, 16384 x 8192 B2 H8 516 / 527, 4096 x 16384 H64/8 1013 / 1041, B4 H32/4 6000 x 6000
+// 1140 / 1156, H32 1181 / 1183; D 40 4000 x 4500 B4 H16 278 / 284.  All on N(0,1) operands.  The fewer bits the
 // operands toggle the less there is to save: 4096 x 4096 H32 of N(0,1) values 218 / 213, of integers from -2 to 2 198 / 192, of zeros,
-// which no clock has to give way to, 146 / 175 (D 96 120 / 145, D 64 113 / 124).
+// which no clock has to give way to, 146 / 175 (D 96 120 / 145).
 bool small_tiles(const FwdParams& p, bool causal, int64_t tiles) {
   const int64_t total = (int64_t)p.blocks * p.B * p.Hq * ((p.Sq + kBM - 1) / kBM), rounds = (total + 255) / 256;
+  if (p.D <= 64 && p.per == 1) return false;
   if (causal) return p.D > 96 && tiles >= 64 && total >= 512;
   return p.D > 96 ? tiles >= 32 && total * 20 >= rounds * 256 * 17 : tiles >= 64 && total * 20 >= rounds * 256 * 19;
 }
@@ -807,10 +812,11 @@ void launch_chain(FwdChunks& p, hipStream_t stream) {
 }
 template <int KK>
 void launch_fwd(FwdChunks& p, bool causal, int groups, hipStream_t stream) {
-  if (groups == 1 && small_tiles(p, causal, (p.Sc + kBN - 1) / kBN)) {
-    if (!causal) return launch_one<false, KK, 1, 16>(p, stream);
-    if constexpr (KK == 8) return launch_one<true, KK, 1, 16>(p, stream);
-  }
+  if constexpr (KK > 4)
+    if (groups == 1 && small_tiles(p, causal, (p.Sc + kBN - 1) / kBN)) {
+      if (!causal) return launch_one<false, KK, 1, 16>(p, stream);
+      if constexpr (KK == 8) return launch_one<true, KK, 1, 16>(p, stream);
+    }
   if (causal) {
     if (groups == 4) launch_one<true, KK, 4>(p, stream);
     else if (groups == 2) launch_one<true, KK, 2>(p, stream);
@@ -882,7 +888,7 @@ int attn_fwd_bf16_plan(int blocks, int B, int Sq, int Sc, int Hq, int D, int64_t
 
 int attn_fwd_bf16_tile(int n, int per, int B, int Sq, int Sc, int Hq, int D, int64_t k_ss, int64_t v_ss, int mask) {
   FwdParams p{};
-  p.blocks = (n + per - 1) / per;
+  p.blocks = (n + per - 1) / per; p.per = per;
   p.B = B; p.Sq = Sq; p.Sc = Sc; p.Hq = Hq; p.D = D;
   p.k_ss = k_ss; p.v_ss = v_ss;
   const bool causal = mask == MHIP_MASK_CAUSAL;

@@ -1,5 +1,5 @@
 """The bf16 forward on 16 x 16 MFMA tiles, which launches take that keep every CU busy for long: 256 workgroups of at least 32
-key tiles (64 up to 96 columns), runs of chunks as long, causal launches of 512 and more.  Against the oracle on some of the
+key tiles (64 up to 96 columns; none but runs of chunks up to 64), causal launches of 512 and more.  Against the oracle on some of the
 heads, with the bound of test_gpu_fwd_key_groups.py."""
 import pytest
 import torch
@@ -28,7 +28,7 @@ def _check(q, kv, out, lse, scale, causal, tag, heads):
 def _run(Sq, Sc, D, n, causal, ramp, tag):
     """n chunks as one result (n = 1: a lone block)."""
     B, H, Hkv, heads = (1, 32, 8, [(0, 0), (0, 31)]) if causal else (2, HEADS, 8, [(0, 0), (0, 77), (1, 127)])
-    assert N.lib().mhip_attn_fwd_tile(n, n, B, Sq, Sc, H, D, Hkv * D, Hkv * D, int(causal)) == 16
+    assert N.lib().mhip_attn_fwd_tile(n, n, B, Sq, Sc, H, D, Hkv * D, Hkv * D, int(causal)) == (16 if D > 64 or n > 1 else 32)
     print(tag, flush=True)
     g = torch.Generator().manual_seed(Sq * 1009 + Sc + D)
     q = torch.randn(B, Sq, H, D, generator=g)

@@ -85,6 +85,8 @@ def test_mfma_tiles_of_the_forward():
     rows = [4096, 4096]
     assert [tile(8, 8, 1, 4096, 4096, 32, D, *rows, 0) for D in (64, 96, 128)] == [16, 16, 16]
     assert [tile(1, 1, 1, 4096, 4096, 32, D, *rows, 1) for D in (64, 96, 128)] == [32, 32, 16]
+    assert [tile(1, 1, 1, 4096, 4096, 32, D, *rows, 0) for D in (64, 72, 96, 128)] == [32, 16, 16, 16]
+    assert [tile(8, 1, 1, 4096, 4096, 32, D, *rows, 0) for D in (64, 96, 128)] == [32, 16, 16]       # chunk by chunk in one launch
     assert tile(8, 8, 1, 256, 256, 32, 128, *rows, 0) == 32 and tile(1, 1, 2, 256, 2048, 128, 128, *rows, 0) == 16
     assert tile(1, 1, 2, 256, 2048, 128, 96, *rows, 0) == 32                  # 32 key tiles: 64 from here on
     assert tile(1, 1, 1, 256, 256, 4, 128, *rows, 0) == 32                    # four key groups
