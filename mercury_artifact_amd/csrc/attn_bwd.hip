@@ -1206,22 +1206,30 @@ int group_chunks(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks, bool
 //     8 chunks 512 x 512 H4     67.1 / 31.4      200 x 200 H2   39.9 / 20.1      1024 x 1024 H8  141 / 121
 //     4 chunks 1024 x 1024 H4   68.3 / 42.7      256 x 256 H4   22.3 / 18.7
 //     D 64  8 chunks 1024 x 1024 H8  105 / 71.9  700 x 700 H12  77.1 / 61.4      256 x 256 H16  32.7 / 23.7
-// Not where the chip is full of other work (two to a tile): 8 chunks 512 x 512 B4 H5 91.2 / 96.9.
+// Not where the chip is full of other work (two to a tile): 8 chunks 512 x 512 B4 H5 91.2 / 96.9, or where the keys' workgroups
+// take as long: 3 chunks 997 x 997 B2 H4/2 60.5 / 62.5 (a tile of the dQ pass is three products to the other's four; the two
+// workgroups of a CU on 64 columns take turns, which costs it as much), 2 chunks 564 x 564 H8 D 80 30.0 / 30.8.
+// The third launch costs the host 3.5 us.  A step that the GPU is done with before the host has launched the next one (which takes it
+// 20 us and 3.5 for each chunk) is so much longer among others, so there it has to save the GPU twice that: 8 chunks 128 x 128
+// H16, one workgroup / four, replayed as a graph 32.0 / 28.0, alone 77 / 73, among others 48 / 51.2.
 int chunk_splits(int B, int Sq, int Sc, int Hq, int Hkv, int D, int n) {
   const float nq = (float)tile_map(B * Hq, Sq, kRowsQ / 2).total, nk = (float)n * tile_map(B * Hkv, Sc, kRowsKv).total;
   const float tq = (float)((Sc + kTile - 1) / kTile), tk = (float)((Sq + kTile - 1) / kTile) * (Hq / Hkv);
   const Cost c = joint_cost(D);
   const float turn = D <= 64 ? 1.f : 7.f;      // us between the workgroups of a CU (on 64 columns the other one runs on)
+  const float products = D <= 64 ? 1.f : 0.75f;
+  const float host = 20.f + 3.5f * n;
   int best = 1;
   float best_time = 0.f;
   for (int s = 1; s <= n; s *= 2) {
     const int64_t bytes = partial_bytes(B, Sq, Hq, D, 1, s);
     if (bytes > kPartialMost) break;
     const float share = nq * s + nk < 256.f ? (nq * s + nk) / 256.f : 1.f, step = c.step + share * c.busy;
-    const float chain = c.fixed + (n + s - 1) / s * tq * step, keys = c.fixed + tk * step;
+    const float chain = c.fixed + (n + s - 1) / s * tq * step * products, keys = c.fixed + tk * step;
     const float longest = chain > keys ? chain : keys, spread = (nq * s * (chain + turn) + nk * (keys + turn)) / 256.f;
     const float time = (longest > spread ? longest : spread) + (s > 1 ? 4.f + 2.f * (float)bytes / 4e6f : 0.f);
-    if (s == 1 || time < 0.95f * best_time) { best = s; best_time = time; }
+    const float less = best == 1 && best_time < host ? 7.f : 0.f;
+    if (s == 1 || (time < 0.95f * best_time && time < best_time - less)) { best = s; best_time = time; }
   }
   return best;
 }

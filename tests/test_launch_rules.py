@@ -70,7 +70,10 @@ def test_chunks_of_a_backward_step_go_together():
     assert take(1, 6000, 6000, 5, 5, 128, 8) == 4                             # 8 would be expected to gain 0.3 %
     assert take(4, 512, 512, 5, 5, 128, 8) == 8 and form(8, 4, 512, 512, 5, 5, 128) == (1, 1, 32)
     assert take(1, 512, 512, 4, 4, 128, 8) == 8 and form(8, 1, 512, 512, 4, 4, 128) == (1, 4, 32)
-    assert take(1, 64, 64, 1, 1, 64, 40) == 14 and form(14, 1, 64, 64, 1, 1, 64)[1] == 8
+    assert take(1, 64, 64, 1, 1, 64, 40) == 14 and form(14, 1, 64, 64, 1, 1, 64) == (1, 1, 32)
+    # shared query tiles: not for 4 us of a step that the host takes longer over, nor where the keys' workgroups take as long
+    assert form(8, 1, 256, 256, 4, 4, 64) == (1, 8, 32) and form(3, 1, 700, 700, 8, 8, 128) == (1, 2, 32)
+    assert form(8, 1, 128, 128, 16, 16, 128) == form(3, 2, 997, 997, 4, 2, 128) == form(2, 1, 564, 564, 8, 8, 80) == (1, 1, 32)
     assert form(2, 4, 319, 319, 32, 32, 64) == (2, 1, 32)                     # also where mhip_attn_bwd_group says 2
     assert form(8, 1, 2048, 2048, 32, 32, 64) == (2, 1, 32)                   # 64 columns keep the larger MFMA tiles
     assert take(1, 256, 256, 4, 4, 64, 1) == take(0, 64, 64, 4, 4, 64, 8) == take(1, 0, 64, 4, 4, 64, 8) == 1
