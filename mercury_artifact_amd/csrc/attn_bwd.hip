@@ -829,21 +829,24 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
   // The same with fp32 rows on the way (512 or 256 bytes, their chunks of 4 columns swizzled by the row).  A lane has 4 or 8
   // columns of a row: a lane's own accumulator columns are 16 bytes of 32 different rows.  `fetch` gives what is there already, all
   // of it on the way before the first store (a load cannot pass a store that may be to the same place, so that one row's after
-  // the other cost a round trip each), and `finish` gets the sums and that.  Rows that are fetched go with 4 columns to a lane, so
-  // that an instruction covers whole rows without a gap: a step of 8 chunks 4096 x 4096 H32, dQ carried in fp32, 6838 us to 6790.
-  // Rows that are only written go with 8, half as many of them with twice the work: 8 chunks 512 x 512 B4 H5, both passes in one
-  // launch, 85.5 us / 87.6 with 4.
+  // the other cost a round trip each), and `finish` gets the sums and that.  With 4 columns to a lane an instruction covers whole rows
+  // without a gap, which the carried dQ of a pass by itself gains from: a step of 8 chunks 4096 x 4096 H32 6838 us to 6790.  Elsewhere
+  // half as many rows with twice the work are better: 8 chunks 512 x 512 B4 H5, both passes in one launch, 85.5 us / 87.6 with 4; 8
+  // chunks 3131 x 3131 B4 H16 D 80, one launch each, dQ carried 6313 / 6435.
   auto write_out32 = [&](const Acc (&acc)[DB][R], float mul, auto columns, auto&& fetch, auto&& finish) {
     own_lds_order();
     constexpr int kH = decltype(columns)::value / 4, kRow32 = 2 * kRow, kPlaces = kRow32 / 16, kLanes = kPlaces / kH;
     constexpr int kRowsAtOnce = 64 / kLanes, kIts = 32 / kRowsAtOnce;
     unsigned char* os = smem + wave * (32 * kRow32);
     const int place = lane % kLanes * kH, col = place * 4, first_row = r0 + wave * 32 + lane / kLanes;
-    f32x4 old[kIts];
+    f32x4 old[kIts][kH];
 #pragma unroll
     for (int it = 0; it < kIts; ++it) {
-      old[it] = f32x4{};
-      if (first_row + it * kRowsAtOnce < n_st && col < p.D) old[it] = fetch(first_row + it * kRowsAtOnce, col);
+#pragma unroll
+      for (int h = 0; h < kH; ++h) old[it][h] = f32x4{};
+      if (first_row + it * kRowsAtOnce < n_st && col < p.D)
+#pragma unroll
+        for (int h = 0; h < kH; ++h) old[it][h] = fetch(first_row + it * kRowsAtOnce, col + 4 * h);
     }
 #pragma unroll
     for (int u = 0; u < kUnits; ++u)
@@ -864,15 +867,18 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
       }
     }
   };
-  const std::integral_constant<int, 4> four;
   const std::integral_constant<int, 8> eight;
   auto pack4 = [](const f32x4& v) { return u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])}; };
+  auto pack8 = [=](const f32x4 (&v)[2]) {
+    const u32x2 lo = pack4(v[0]), hi = pack4(v[1]);
+    return u32x4{lo[0], lo[1], hi[0], hi[1]};
+  };
   auto nothing = [](int, int) { return f32x4{}; };
   if (SPLIT && w.splits > 1) {
     // fp32 sums for bwd_reduce, (b, row, head, column) like the gradient itself
     const int64_t size = (int64_t)p.B * n_st * (DQ ? p.Hq : p.Hkv) * p.D;
     auto part = [&](float* base) {
-      return [=](const f32x4 (&v)[2], const f32x4&, int row, int col) {
+      return [=](const f32x4 (&v)[2], const f32x4 (&)[2], int row, int col) {
         f32x4* op = reinterpret_cast<f32x4*>(base + split * size + (((int64_t)b * n_st + row) * (DQ ? p.Hq : p.Hkv) + hs) * p.D + col);
         op[0] = v[0];
         op[1] = v[1];
@@ -886,13 +892,22 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     } else {
       uint16_t* dq = p.dq ? p.dq + b * p.dq_sb + hs * p.dq_sh : nullptr;
       auto at = [&](int row, int col) { return reinterpret_cast<f32x4*>(p.dq_acc + (((int64_t)b * p.Sq + row) * p.Hq + hs) * p.D + col); };
-      write_out32(acc1, p.scale, four, [&](int row, int col) { return p.dq_mode != kDqFirst ? *at(row, col) : f32x4{}; },
-                  [&](const f32x4 (&v)[1], const f32x4& old, int row, int col) {
-        u32x2* qp = reinterpret_cast<u32x2*>(dq + (int64_t)row * p.dq_ss + col);
-        if (p.dq_mode == kDqAdd && dq) *qp = pack4(v[0]);
-        const f32x4 sum = p.dq_mode != kDqFirst ? v[0] + old : v[0];
-        if (p.dq_mode != kDqLast) *at(row, col) = sum;
-        else *qp = pack4(sum);
+      constexpr int kH = WAVES == 8 ? 1 : 2;
+      auto put16 = [=](int row, int col, const f32x4 (&v)[kH]) {
+        uint16_t* to = dq + (int64_t)row * p.dq_ss + col;
+        if constexpr (kH == 1) *reinterpret_cast<u32x2*>(to) = pack4(v[0]);
+        else *reinterpret_cast<u32x4*>(to) = pack8(v);
+      };
+      write_out32(acc1, p.scale, std::integral_constant<int, 4 * kH>(),
+                  [&](int row, int col) { return p.dq_mode != kDqFirst ? *at(row, col) : f32x4{}; },
+                  [&](const f32x4 (&v)[kH], const f32x4 (&old)[kH], int row, int col) {
+        if (p.dq_mode == kDqAdd && dq) put16(row, col, v);
+        f32x4 sum[kH];
+#pragma unroll
+        for (int h = 0; h < kH; ++h) sum[h] = p.dq_mode != kDqFirst ? v[h] + old[h] : v[h];
+        if (p.dq_mode == kDqLast) return put16(row, col, sum);
+#pragma unroll
+        for (int h = 0; h < kH; ++h) *at(row, col + 4 * h) = sum[h];
       });
     }
   } else if ((CHUNKS ? chunks->dk32[chunk] : p.dk32) == nullptr) {
@@ -900,12 +915,12 @@ __device__ __forceinline__ void bwd_pass(const BwdParams& p, const TileMap& w, c
     write_out(acc2, 1.f, CHUNKS ? chunks->dv[chunk] : p.dv, p.dk_sb, p.dk_ss, p.dk_sh, hs);
   } else {
     auto store = [&](float* out32, uint16_t* out16) {
-      return [=](const f32x4 (&v)[2], const f32x4&, int row, int col) {
-        const u32x2 lo = pack4(v[0]), hi = pack4(v[1]);
+      return [=](const f32x4 (&v)[2], const f32x4 (&)[2], int row, int col) {
+        const u32x4 w = pack8(v);
         f32x4* op = reinterpret_cast<f32x4*>(out32 + (((int64_t)b * p.Sc + row) * p.Hkv + hs) * p.D + col);
-        op[0] = f32x4{bf16_lo(lo[0]), bf16_hi(lo[0]), bf16_lo(lo[1]), bf16_hi(lo[1])};
-        op[1] = f32x4{bf16_lo(hi[0]), bf16_hi(hi[0]), bf16_lo(hi[1]), bf16_hi(hi[1])};
-        if (out16) *reinterpret_cast<u32x4*>(out16 + b * p.dk_sb + (int64_t)row * p.dk_ss + hs * p.dk_sh + col) = u32x4{lo[0], lo[1], hi[0], hi[1]};
+        op[0] = f32x4{bf16_lo(w[0]), bf16_hi(w[0]), bf16_lo(w[1]), bf16_hi(w[1])};
+        op[1] = f32x4{bf16_lo(w[2]), bf16_hi(w[2]), bf16_lo(w[3]), bf16_hi(w[3])};
+        if (out16) *reinterpret_cast<u32x4*>(out16 + b * p.dk_sb + (int64_t)row * p.dk_ss + hs * p.dk_sh + col) = w;
       };
     };
     write_out32(acc1, p.scale, eight, nothing, store(CHUNKS ? chunks->dk32[chunk] : p.dk32, CHUNKS ? chunks->dk[chunk] : p.dk));
