@@ -1219,7 +1219,7 @@ int group_chunks(int B, int Sq, int Sc, int Hq, int Hkv, int D, int chunks, bool
 // over all chunks is what a launch waits for whose other workgroups leave CUs idle or are soon done.  Their sums meet in
 // bwd_reduce.  Us a step, one workgroup to a tile / as many as chosen:
 //     8 chunks 512 x 512 H4     67.1 / 31.4      200 x 200 H2   39.9 / 20.1      1024 x 1024 H8  141 / 121
-//     4 chunks 1024 x 1024 H4   68.3 / 42.7      256 x 256 H4   22.3 / 18.7
+//     4 chunks 1024 x 1024 H4   68.3 / 42.7      256 x 256 H4   22.3 / 18.7 (not taken, see below)
 //     D 64  8 chunks 1024 x 1024 H8  105 / 71.9  700 x 700 H12  77.1 / 61.4      256 x 256 H16  32.7 / 23.7
 // Not where the chip is full of other work (two to a tile): 8 chunks 512 x 512 B4 H5 91.2 / 96.9, or where the keys' workgroups
 // take as long: 3 chunks 997 x 997 B2 H4/2 60.5 / 62.5 (a tile of the dQ pass is three products to the other's four; the two
